@@ -473,6 +473,109 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(TO* __restrict__ C, const
   }
 }
 
+// The same product for fp32 operands whose rows are 16-byte aligned (k and every stride a multiple of 4 elements) on the
+// matrix cores' fp32 instruction (v_mfma_f32_32x32x2_f32: fp32 products and sums, nothing rounded in between).  A workgroup
+// of 8 waves owns a 32 x (32 NN) output tile, in the swapped orientation C^T = W A^T; its waves share k instead of the tile:
+// of every 64-deep step, staged through two LDS buffers, wave w multiplies the elements [8 w, 8 w + 8), so small tiles still
+// give every SIMD two waves.  A lane reads 4 consecutive k of its row and spends one on each of 4 instructions.  PF steps'
+// loads are in flight.  The waves' sums meet in LDS in wave order: an output's accumulation order depends on K alone, not on
+// the tile or the rows that share it.  Same three forms.
+// Bound by the fp32 matrix rate (157 TFLOP/s; a 32 x 32 x 2048 tile is 7 us of a CU's four pipes).  333 rows: 2048 x 2048
+// (N x K) 40 us (503 us with gemm_any_kernel; 70 TFLOP/s now), 16384 x 2048 270 us (434), 128 x 2048 16 us with the launch
+// (276).  Tiles of 64 x 64 with a wave per 32 x 32 part took 62, 265 and 56 us: one wave per SIMD and a chain of loads.
+template <typename TO, int NN>
+__global__ __launch_bounds__(512) void gemm_f32_kernel(TO* __restrict__ C, const float* __restrict__ A,
+                                                       const float* __restrict__ Wt, int M, int N, int K, long lda,
+                                                       long ldw, long ldc, long sA, long sW, long sC,
+                                                       const int* __restrict__ a_rows, const int* __restrict__ tiles) {
+  typedef float f32x16 __attribute__((ext_vector_type(16)));
+  constexpr int BM = 32, BN = 32 * NN, BK = 64, LD = BK + 4, PF = 4, PER = 64 / BM;
+  constexpr int STAGE = (BM + BN) * LD;            // floats of one LDS buffer: A rows, then W rows
+  constexpr int LDS = 2 * STAGE > 8 * 16 * 64 ? 2 * STAGE : 8 * 16 * 64;
+  __shared__ __attribute__((aligned(16))) float sm[LDS];
+  int row0, rows;
+  if (tiles != nullptr) {                          // PER blocks per listed tile of at most 64 rows
+    const int y = blockIdx.y / PER, sub = (blockIdx.y - y * PER) * BM;
+    const int g = tiles[3 * y];
+    if (g < 0) return;
+    row0 = tiles[3 * y + 1] + sub;
+    rows = min(BM, tiles[3 * y + 2] - sub);
+    if (rows <= 0) return;
+    Wt += (size_t)g * sW;
+  } else {
+    row0 = blockIdx.y * BM;
+    rows = min(BM, M - row0);
+    A += (size_t)blockIdx.z * sA;
+    Wt += (size_t)blockIdx.z * sW;
+    C += (size_t)blockIdx.z * sC;
+  }
+  const int col0 = blockIdx.x * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 31, h = lane >> 5;
+  const int lr = tid >> 4, lc = 4 * (tid & 15);    // loader: row lr (W: + 32 b), 4 elements from lc of the step
+  // rows and columns past the end repeat the last one (they are not stored)
+  const int ar = row0 + min(lr, rows - 1);
+  const float* ap = A + (size_t)(a_rows != nullptr ? a_rows[ar] : ar) * lda;
+  const float* wp[NN];
+#pragma unroll
+  for (int b = 0; b < NN; ++b) wp[b] = Wt + (size_t)min(col0 + 32 * b + lr, N - 1) * ldw;
+  f32x4 ra[PF], rw[PF][NN];
+  auto fetch = [&](f32x4& fa, f32x4 (&fw)[NN], int k0) {     // past the end: the row's last elements, staged as zeros
+    const int k = min(k0 + lc, K - 4);
+    fa = *reinterpret_cast<const f32x4*>(ap + k);
+#pragma unroll
+    for (int b = 0; b < NN; ++b) fw[b] = *reinterpret_cast<const f32x4*>(wp[b] + k);
+  };
+  f32x16 acc[NN];
+#pragma unroll
+  for (int n = 0; n < NN; ++n)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[n][i] = 0.f;
+  const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int p = 0; p < PF; ++p) fetch(ra[p], rw[p], BK * p);
+  for (int k0 = 0; k0 < K; k0 += BK * PF) {
+#pragma unroll
+    for (int p = 0; p < PF; ++p) {
+      const int k = k0 + BK * p;
+      if (k >= K) break;                           // uniform
+      float* st = sm + (p & 1) * STAGE;
+      const bool in = k + lc < K;
+      *reinterpret_cast<f32x4*>(st + lr * LD + lc) = in ? ra[p] : zero;
+#pragma unroll
+      for (int b = 0; b < NN; ++b) *reinterpret_cast<f32x4*>(st + (BM + 32 * b + lr) * LD + lc) = in ? rw[p][b] : zero;
+      lds_barrier();         // this buffer is written; the other one was read before every wave came here
+      fetch(ra[p], rw[p], k + BK * PF);
+      const f32x4 fa = *reinterpret_cast<const f32x4*>(st + li * LD + 8 * wave + 4 * h);
+      f32x4 fw[NN];
+#pragma unroll
+      for (int b = 0; b < NN; ++b) fw[b] = *reinterpret_cast<const f32x4*>(st + (BM + 32 * b + li) * LD + 8 * wave + 4 * h);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int n = 0; n < NN; ++n) acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(fw[n][i], fa[i], acc[n], 0, 0, 0);
+    }
+  }
+  // acc[n][4 q + i] = C[row li][col 32 n + 8 q + 4 h + i], this wave's share of k
+  float(*red)[16][64] = reinterpret_cast<float(*)[16][64]>(sm);
+#pragma unroll
+  for (int n = 0; n < NN; ++n) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) red[wave][i][lane] = acc[n][i];
+    __syncthreads();
+    float y[2] = {0.f, 0.f};                       // thread (wave, lane) finishes the elements 2 wave, 2 wave + 1
+#pragma unroll
+    for (int v = 0; v < 8; ++v)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) y[e] += red[v][2 * wave + e][lane];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int x = 2 * wave + e, c = col0 + 32 * n + 8 * (x >> 2) + 4 * h + (x & 3);
+      if (li < rows && c < N) stf(C, (size_t)(row0 + li) * ldc + c, y[e]);
+    }
+  }
+}
+
 // The same product for bf16 operands whose rows are 16-byte aligned (k and every stride a multiple of 8 elements) on
 // the matrix cores: 64 x 64 or (many rows and columns) 64 x 128 output tile, 32-deep k steps, 4 waves of 32 x 32 or
 // 32 x 64 (2 x NF v_mfma_f32_16x16x32_bf16) in the swapped orientation C^T = W A^T, so a lane ends with 4 consecutive
@@ -832,6 +935,22 @@ extern "C" int k8s_gemm_any(void* C, const void* A, const void* W, int M, int N,
     return (int)hipGetLastError();
   }
   const dim3 grid((N + 63) / 64, gy, batch);
+  const int gm = tiles != nullptr ? gy * 2 : (M + 31) / 32;     // fp32 tiles are 32 rows high
+  if (in_f32 && K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && sA % 4 == 0 && sW % 4 == 0 && ((uintptr_t)A & 15) == 0 &&
+      ((uintptr_t)W & 15) == 0 && gm <= 65535) {
+    // 32 x 64 tiles take about 1.8 times a 32 x 32 one (333 x 2048 x 2048: 50 us and 40 us; 512 rows: 49 and 52; 1 x 16384 x
+    // 2048: 32 and 39): the shape whose tiles fill the last round over the CUs better
+    const long t1 = (long)gm * ((N + 31) / 32) * batch, t2 = (long)gm * ((N + 63) / 64) * batch;
+    const bool wide = 2.0 * (double)((t2 + 255) / 256) < 1.1 * (double)((t1 + 255) / 256);
+    const dim3 gf((N + (wide ? 63 : 31)) / (wide ? 64 : 32), gm, batch);
+#define K8S_GF(TO, NN) \
+  gemm_f32_kernel<TO, NN><<<gf, 512, 0, s>>>((TO*)C, (const float*)A, (const float*)W, M, N, K, lda, ldw, ldc, sA, sW, sC, \
+                                             a_rows, tiles)
+    if (out_f32) { if (wide) K8S_GF(float, 2); else K8S_GF(float, 1); }
+    else { if (wide) K8S_GF(bf16_t, 2); else K8S_GF(bf16_t, 1); }
+#undef K8S_GF
+    return (int)hipGetLastError();
+  }
 #define K8S_GA(TI, TO) \
   gemm_any_kernel<TI, TO><<<grid, 256, 0, s>>>((TO*)C, (const TI*)A, (const TI*)W, M, N, K, lda, ldw, ldc, sA, sW, sC, \
                                                a_rows, tiles)
