@@ -171,6 +171,12 @@ int k8s_latent_attention_mfma(void* out, float* pacc, float* pml, const void* q_
                               const int* block_tables, int max_blocks, const int* tok_seq, const int* positions, int T,
                               int C, int R, int H, int Dn, int window, float scale, int bs, int nsplit, const int* cu_q,
                               int nseq, int max_qlen, const float* sinks, const void* gate, long ldg, hipStream_t s);
+int k8s_latent_prompt_ok(int C, int R, int Dn, int V);
+int k8s_latent_keys(int* rows, int* kbase, int* tiles, const int* cu_q, const int* positions, const int* block_tables,
+                    int max_blocks, int nseq, int window, int bs, int cap, int ntiles, hipStream_t s);
+int k8s_latent_prompt(void* out, const void* kv, const int* rows, const int* kbase, const void* q, const void* cache, int C,
+                      int R, int Dn, int V, const int* cu_q, const int* positions, int nseq, int max_qlen, int H, int window,
+                      float scale, const float* sinks, const void* gate, long ldg, int f32, hipStream_t s);
 int k8s_moe_route(int* idx, float* w, const float* logits, int ld, int T, int E, int top, float scale, int mode,
                   hipStream_t s);
 int k8s_window_kv_write(void* kcache, void* vcache, void* qkv, long ld, int koff, int voff, const void* qb,
@@ -597,6 +603,19 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
                                     max_blocks, P<int>(tok_seq), P<int>(positions), T, C, R, H, Dn, window, scale, bs,
                                     nsplit, P<int>(cu_q), nseq, max_qlen, P<float>(sinks), P(gate), ldg, S(s)),
           "latent_attention_mfma");
+  });
+  m.def("latent_prompt_ok", [](int C, int R, int Dn, int V) { return k8s_latent_prompt_ok(C, R, Dn, V) != 0; });
+  m.def("latent_keys", [](uintptr_t rows, uintptr_t kbase, uintptr_t tiles, uintptr_t cu_q, uintptr_t positions,
+                          uintptr_t bt, int max_blocks, int nseq, int window, int bs, int cap, int ntiles, int64_t s) {
+    check(k8s_latent_keys(P<int>(rows), P<int>(kbase), P<int>(tiles), P<int>(cu_q), P<int>(positions), P<int>(bt), max_blocks,
+                          nseq, window, bs, cap, ntiles, S(s)), "latent_keys");
+  });
+  m.def("latent_prompt", [](uintptr_t out, uintptr_t kv, uintptr_t rows, uintptr_t kbase, uintptr_t q, uintptr_t cache, int C,
+                            int R, int Dn, int V, uintptr_t cu_q, uintptr_t positions, int nseq, int max_qlen, int H,
+                            int window, float scale, uintptr_t sinks, uintptr_t gate, long ldg, int f32, int64_t s) {
+    check(k8s_latent_prompt(P(out), P(kv), P<int>(rows), P<int>(kbase), P(q), P(cache), C, R, Dn, V, P<int>(cu_q),
+                            P<int>(positions), nseq, max_qlen, H, window, scale, P<float>(sinks), P(gate), ldg, f32, S(s)),
+          "latent_prompt");
   });
   m.def("moe_route", [](uintptr_t idx, uintptr_t w, uintptr_t logits, int ld, int T, int E, int top, float scale,
                         int mode, int64_t s) {

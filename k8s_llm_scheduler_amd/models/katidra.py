@@ -264,6 +264,7 @@ class _Latent:
     uv: torch.Tensor                    # [H, V, kv_rank]
     o: torch.Tensor                     # [W, H V]
     cos_sin: torch.Tensor               # [positions, rot_dims] fp32
+    ukv: Optional[torch.Tensor]         # [H (Dn + V), kv_rank]: both up-projections as one product (sm.latent_expand)
 
 
 @dataclass
@@ -320,7 +321,7 @@ class KatidraModel(StreamModel):
         w_in, cols = stack_rows(tuple((s, get(p + s).cpu()) for s in ("dq", "dkv", "g")))
         return _Latent(m, t(w_in), cols, t(get(p + "dq.norm")), t(get(p + "uq")), t(get(p + "dkv.norm")),
                        t(get(p + "uk").view(H, Dn, C).transpose(1, 2)), t(get(p + "uv").view(H, V, C)), t(get(p + "o")),
-                       self._rope_table(m))
+                       self._rope_table(m), self._expand(get, p, H, R))
 
     def _build(self, get) -> None:
         c, t = self.cfg, self._t
@@ -395,14 +396,9 @@ class KatidraModel(StreamModel):
         q = sm.linear(cq, w.uq)                                            # [T, H (Dn + R)]
         sm.latent_kv_write(kv, proj[:, w.cols["dkv"]:w.cols["dkv"] + C + R], w.dkv_norm, q, w.cos_sin, b["positions"],
                            b["slot_mapping"], C, R, H, Dn, m.rot_dims, eps, interleaved=True)
-        q_abs = torch.empty(T, H, C, dtype=self.dtype, device=h.device)
-        sm.gemm(q.view(T, H, Dn + R)[:, :, :Dn].permute(1, 0, 2), w.uk_t, out=q_abs.permute(1, 0, 2))
-        lat = sm.latent_attention(q_abs, q, kv, b["block_tables"], b["tok_seq"], b["positions"], C, R, H, Dn, m.window,
-                                  m.scale, self.block_size, b.get("max_keys", 0), b["cu_q"], b.get("max_qlen", 0),
-                                  gate=proj[:, w.cols["g"]:w.cols["g"] + H])                # [T, H, C]
-        a = torch.empty(T, H, V, dtype=self.dtype, device=h.device)
-        sm.gemm(lat.permute(1, 0, 2), w.uv, out=a.permute(1, 0, 2))
-        return sm.linear(a.view(T, H * V), w.o)
+        a = sm.latent_mix(q, kv, w.uk_t, w.uv, w.ukv, b, C, R, H, Dn, V, m.window, m.scale, self.block_size,
+                          gate=proj[:, w.cols["g"]:w.cols["g"] + H])
+        return sm.linear(a, w.o)
 
     def _blocks(self, ids, b, after=None) -> torch.Tensor:
         """The residual stream after the last layer."""

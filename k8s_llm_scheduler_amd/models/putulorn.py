@@ -300,6 +300,7 @@ class _Latent:
     uv: torch.Tensor        # [H, V, C]
     o: torch.Tensor         # [W, H V]
     cos_sin: torch.Tensor   # [positions, rot_dims] fp32
+    ukv: Optional[torch.Tensor]   # [H (Dn + V), C]: both up-projections as one product (sm.latent_expand)
 
 
 @dataclass
@@ -379,7 +380,8 @@ class PutulornModel(StreamModel):
                     raise ValueError(f"layer {i}: rot.dims {m.rot_dims} must be even and at most rot_dim {m.rot_dim}")
                 mixer = _Latent(m, t(get(p + "q")), t(get(p + "dkv")), t(get(p + "dkv.norm")),
                                 t(get(p + "uk").reshape(H, Dn, C).transpose(1, 2)), t(get(p + "uv").reshape(H, V, C)),
-                                t(get(p + "o")), self._rope_table(m.rot_dims, m.rot_base))
+                                t(get(p + "o")), self._rope_table(m.rot_dims, m.rot_base),
+                                self._expand(get, p, H, m.rot_dim))
             f, mlp, n2 = L.mlp, None, None
             if f is not None:
                 q = f"l{i}.mlp."
@@ -459,14 +461,8 @@ class PutulornModel(StreamModel):
         dkv = sm.linear(h, w.dkv)                                          # [T, C + R]
         sm.latent_kv_write(cache, dkv, w.dkv_norm, q, w.cos_sin, b["positions"], b["slot_mapping"], C, R, H, Dn,
                            m.rot_dims, self.cfg.rms_eps)
-        q_abs = torch.empty(T, H, C, dtype=self.dtype, device=h.device)
-        sm.gemm(q.view(T, H, Dn + R)[:, :, :Dn].permute(1, 0, 2), w.uk_t, out=q_abs.permute(1, 0, 2))
-        lat = sm.latent_attention(q_abs, q, cache, b["block_tables"], b["tok_seq"], b["positions"], C, R, H, Dn,
-                                  m.window, m.scale, self.block_size, b.get("max_keys", 0), b["cu_q"],
-                                  b.get("max_qlen", 0))                   # [T, H, C]
-        a = torch.empty(T, H, V, dtype=self.dtype, device=h.device)
-        sm.gemm(lat.permute(1, 0, 2), w.uv, out=a.permute(1, 0, 2))
-        return sm.linear(a.view(T, H * V), w.o)
+        a = sm.latent_mix(q, cache, w.uk_t, w.uv, w.ukv, b, C, R, H, Dn, V, m.window, m.scale, self.block_size)
+        return sm.linear(a, w.o)
 
     def _mlp(self, w: _Mlp, h) -> torch.Tensor:
         f = w.cfg

@@ -290,6 +290,7 @@ class _Latent:
     sinks: torch.Tensor                 # fp32 [H]
     o: torch.Tensor                     # [W, H V]
     cos_sin: torch.Tensor               # [positions, rot_dim] fp32
+    ukv: Optional[torch.Tensor]         # [H (Dn + V), kv_rank]: both up-projections as one product (sm.latent_expand)
     cache: int = -1                     # index into kv_cache
 
 
@@ -372,7 +373,8 @@ class SemanexModel(StreamModel):
         w_in, cols = stack_rows((("dq", get(p + "dq").cpu()), ("dkv", get(p + "dkv").cpu()), ("g", get(p + "g").cpu())))
         return _Latent(m, t(w_in), cols, t(get(p + "dq.norm")), t(get(p + "uq")), t(get(p + "dkv.norm")),
                        t(get(p + "uk").view(H, Dn, C).transpose(1, 2)), t(get(p + "uv").view(H, V, C)),
-                       self._f(get(p + "sink")), t(get(p + "o")), self._rope_table(m.rot_dims, m.rot_base))
+                       self._f(get(p + "sink")), t(get(p + "o")), self._rope_table(m.rot_dims, m.rot_base),
+                       self._expand(get, p, H, R))
 
     def _build_side(self, get, p: str, m: ParallelConfig, where: str) -> _Side:
         t, f = self._t, self._f
@@ -480,14 +482,8 @@ class SemanexModel(StreamModel):
         q = sm.linear(cq, w.uq)                                            # [T, H (Dn + R)]
         sm.latent_kv_write(cache, proj[:, w.cols["dkv"]:w.cols["dkv"] + C + R], w.dkv_norm, q, w.cos_sin,
                            b["positions"], b["slot_mapping"], C, R, H, Dn, m.rot_dims, eps, interleaved=True)
-        q_abs = torch.empty(T, H, C, dtype=self.dtype, device=h.device)
-        sm.gemm(q.view(T, H, Dn + R)[:, :, :Dn].permute(1, 0, 2), w.uk_t, out=q_abs.permute(1, 0, 2))
-        lat = sm.latent_attention(q_abs, q, cache, b["block_tables"], b["tok_seq"], b["positions"], C, R, H, Dn, 0,
-                                  m.scale, self.block_size, b.get("max_keys", 0), b["cu_q"], b.get("max_qlen", 0),
-                                  sinks=w.sinks)                           # [T, H, C]
-        a = torch.empty(T, H, V, dtype=self.dtype, device=h.device)
-        sm.gemm(lat.permute(1, 0, 2), w.uv, out=a.permute(1, 0, 2))
-        y = sm.gate_mul(a.view(T, H * V), proj[:, w.cols["g"]:w.cols["g"] + H * V], sm.GATE_SIGMOID)
+        a = sm.latent_mix(q, cache, w.uk_t, w.uv, w.ukv, b, C, R, H, Dn, V, 0, m.scale, self.block_size, sinks=w.sinks)
+        y = sm.gate_mul(a, proj[:, w.cols["g"]:w.cols["g"] + H * V], sm.GATE_SIGMOID)
         return sm.linear(y, w.o)
 
     def _capped_attention(self, w: _Capped, h, b) -> torch.Tensor:

@@ -13,6 +13,7 @@ from typing import Callable, Dict, Optional
 
 import torch
 
+from ..ops import seqmix as sm
 from ..parallel import TPGroup
 
 
@@ -82,6 +83,11 @@ class StreamModel:
 
     def _t(self, t: torch.Tensor) -> torch.Tensor:
         return t.to(self.dtype).to(self.device).contiguous()
+
+    def _expand(self, get, p: str, H: int, R: int) -> Optional[torch.Tensor]:
+        """A latent attention's ``uk`` and ``uv`` stacked per head, for the sizes whose prompts write keys and values out."""
+        w = sm.latent_expand(get(p + "uk"), get(p + "uv"), H, R)
+        return None if w is None else self._t(w)
 
     def _weight_roots(self) -> tuple:
         raise NotImplementedError

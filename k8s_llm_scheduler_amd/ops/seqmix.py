@@ -1,7 +1,7 @@
 """Ops of models with an fp32 residual stream, recurrent / windowed- or latent-attention mixers and mixtures of experts.
 
 Same dispatch rule as the rest of :mod:`..ops`: CUDA (= HIP) tensors always run the gfx950 kernels
-(``stream32.hip``, ``mixers.hip``, ``window_attn.hip``, ``gated_scan.hip``, ``decay_scan.hip``, ``delta_scan.hip``, ``moe.hip``) and raise when the extension is missing; CPU tensors run the fp32
+(``stream32.hip``, ``mixers.hip``, ``latent_prompt.hip``, ``window_attn.hip``, ``gated_scan.hip``, ``decay_scan.hip``, ``delta_scan.hip``, ``moe.hip``) and raise when the extension is missing; CPU tensors run the fp32
 reference in :mod:`.reference` (the CPU test-suite).  Every op takes bf16 or true-fp32 activations / weights (the
 ``f32`` flag of the kernels); what a design computes in fp32 regardless (residual sum, recurrent state, decays, router,
 attention scores) is fp32 in both.
@@ -446,6 +446,79 @@ def latent_attention(q_abs: torch.Tensor, q: torch.Tensor, cache: torch.Tensor, 
     else:
         nat.latent_attention(out.data_ptr(), *args, _f32(dt), _p(sinks), gp, ldg, -1)
     return out
+
+
+# A batch of prompts writes its visible keys and values out (latent_prompt.hip) when its sequences bring at least
+# LATENT_EXPAND_MIN tokens on average: a portion that sees K rows then spends K C (Dn + V) multiply-adds per head on them
+# instead of n C (Dn + V) on its own queries and outputs, and saves n K (2 C - Dn - V) in the attention, which breaks even
+# at n = 170 for C = 512, Dn = V = 128 where everything in sight is cached already, and at any n where nothing is.  2048
+# tokens, 16 heads, window 1024: 383 us absorbed, 85 us written out; 512 tokens, 32 heads: 139 us and 42 us; fp32, 333
+# tokens, 16 heads: 1290 us and 70 us.
+LATENT_EXPAND_MIN = int(os.environ.get("K8S_LATENT_EXPAND_MIN", "160"))
+LATENT_EXPAND_BYTES = 1 << 30     # of keys and values
+
+
+def latent_expand(uk: torch.Tensor, uv: torch.Tensor, H: int, R: int) -> Optional[torch.Tensor]:
+    """W_uk [H Dn, C] and W_uv [H V, C] as one product per latent row, [H (Dn + V), C] (per head: key rows, value rows), or
+    None for sizes whose keys and values are never written out."""
+    C, Dn, V = uk.shape[1], uk.shape[0] // H, uv.shape[0] // H
+    if not (C % 8 == 0 and Dn == 128 and R == 64 and V == 128):
+        return None
+    return torch.cat([uk.view(H, Dn, C), uv.view(H, V, C)], 1).reshape(H * (Dn + V), C)
+
+
+def _latent_keys(b: dict, window: int, block_size: int, cap: int) -> tuple:
+    """(cache slots of the rows the batch's tokens see, first row of every sequence, row tiles): made once per batch."""
+    made = b.setdefault("latent_keys", {})
+    if window not in made:
+        dev, nseq = b["positions"].device, b["cu_q"].shape[0] - 1
+        ntiles = cap // 64 + nseq
+        rows = torch.empty(cap, dtype=I32, device=dev)
+        kbase = torch.empty(nseq, dtype=I32, device=dev)
+        tiles = torch.empty(ntiles, 3, dtype=I32, device=dev)
+        _native().latent_keys(rows.data_ptr(), kbase.data_ptr(), tiles.data_ptr(), _p(b["cu_q"], I32),
+                              _p(b["positions"], I32), _p(b["block_tables"], I32), b["block_tables"].shape[1], nseq, window,
+                              block_size, cap, ntiles, -1)
+        made[window] = (rows, kbase, tiles)
+    return made[window]
+
+
+def latent_mix(q: torch.Tensor, cache: torch.Tensor, uk_t: torch.Tensor, uv: torch.Tensor, ukv: Optional[torch.Tensor],
+               b: dict, C: int, R: int, H: int, Dn: int, V: int, window: int, scale: float, block_size: int, *,
+               sinks: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Latent attention with its up-projections, [T, H V]: queries q [T, H (Dn + R)] (rotated) over the batch ``b``'s cached
+    rows, ``uk_t`` [H, C, Dn], ``uv`` [H, V, C], ``ukv`` from :func:`latent_expand`; ``sinks`` and ``gate`` as for
+    :func:`latent_attention`.  Decoding and short portions absorb the queries (q W_uk), attend the cache as it is stored and
+    take the result through W_uv; batches of longer portions write the visible rows' keys and values out first."""
+    T = q.shape[0]
+    dt = q.dtype
+    nseq, max_qlen = b["cu_q"].shape[0] - 1, b.get("max_qlen", 0)
+    ctx = b["block_tables"].shape[1] * block_size
+    cap = min(T + nseq * (window - 1), nseq * ctx) if window else nseq * ctx
+    if (ukv is not None and _gpu(q, cache) and max_qlen > 0 and 0 < LATENT_EXPAND_MIN * nseq <= T and cap < 1 << 24
+            and cap * H * (Dn + V) * q.element_size() <= LATENT_EXPAND_BYTES and _native().latent_prompt_ok(C, R, Dn, V)):
+        if sinks is not None and (sinks.dtype != F32 or sinks.numel() != H):
+            raise ValueError("latent_mix: sinks are fp32 [H]")
+        if gate is not None and (gate.shape != (T, H) or gate.dtype != dt or gate.stride(1) != 1):
+            raise ValueError("latent_mix: the gate is [T, H] of the queries' type with contiguous rows")
+        rows, kbase, tiles = _latent_keys(b, int(window), block_size, cap)
+        kv = torch.empty(cap, H * (Dn + V), dtype=dt, device=q.device)
+        nat = _native()
+        nat.gemm_any(kv.data_ptr(), _p(cache, dt, "cache"), _p(ukv, dt, "ukv"), cap, H * (Dn + V), C, C + R, C, H * (Dn + V),
+                     1, 0, 0, 0, rows.data_ptr(), tiles.data_ptr(), tiles.shape[0], _f32(dt), _f32(dt), -1)
+        out = torch.empty(T, H * V, dtype=dt, device=q.device)
+        nat.latent_prompt(out.data_ptr(), kv.data_ptr(), rows.data_ptr(), kbase.data_ptr(), _p(q), cache.data_ptr(), C, R, Dn,
+                          V, _p(b["cu_q"], I32), _p(b["positions"], I32), nseq, int(max_qlen), H, int(window), float(scale),
+                          _p(sinks), gate.data_ptr() if gate is not None else 0, gate.stride(0) if gate is not None else 0,
+                          _f32(dt), -1)
+        return out
+    q_abs = torch.empty(T, H, C, dtype=dt, device=q.device)
+    gemm(q.view(T, H, Dn + R)[:, :, :Dn].permute(1, 0, 2), uk_t, out=q_abs.permute(1, 0, 2))
+    lat = latent_attention(q_abs, q, cache, b["block_tables"], b["tok_seq"], b["positions"], C, R, H, Dn, window, scale,
+                           block_size, b.get("max_keys", 0), b["cu_q"], max_qlen, sinks=sinks, gate=gate)     # [T, H, C]
+    a = torch.empty(T, H, V, dtype=dt, device=q.device)
+    gemm(lat.permute(1, 0, 2), uv, out=a.permute(1, 0, 2))
+    return a.view(T, H * V)
 
 
 # ----------------------------------------------------------------------------- mixture of experts

@@ -45,3 +45,65 @@ def test_fp32_grouped_products(tokens, top, E):
             e = int(idx[t, c])
             y = got.view(tokens, top, N)[t, c]
             assert ((y - h[t].double() @ w[e].double().T).abs() <= sum_bound(h[t:t + 1], w[e])[0]).all()
+
+
+# ----------------------------------------------------------------------------- latent attention of prompts
+# (tokens cached already, tokens brought) of every sequence; window.  Portions at the edges of the 64- and 128-token tiles,
+# windows cutting inside a step, a window of one, sequences without tokens, single tokens riding along behind long contexts,
+# many heads (the two tile heights of the bf16 kernel)
+LATENT = [([(0, 200)], 0, 3), ([(0, 64), (0, 449)], 100, 2), ([(37, 191), (0, 0), (5, 129)], 64, 2),
+          ([(700, 1), (0, 640), (333, 1), (16, 2)], 300, 16), ([(0, 513)], 1, 1), ([(0, 1153)], 513, 32),
+          ([(48, 400), (2, 300)], 0, 8)]
+
+
+@pytest.mark.parametrize("dt,tol", [(torch.float32, 2e-5), (torch.bfloat16, 2e-2)])
+@pytest.mark.parametrize("seqs,window,H", LATENT)
+@pytest.mark.parametrize("extra", ["", "gate", "sinks"])
+def test_latent_prompt(dt, tol, seqs, window, H, extra, monkeypatch):
+    """Written-out keys and values against 64 bits and against the absorbed form.  Tolerance: the type's rounding of keys,
+    values, weights and result, as for the absorbed kernels."""
+    C, R, Dn, V, bs = 512, 64, 128, 128, 16
+    g = torch.Generator().manual_seed(len(seqs) + window + H)
+    ends = [a + n for a, n in seqs]
+    pages = -(-max(ends) // bs)
+    bt = torch.randperm(len(seqs) * pages, generator=g).view(len(seqs), pages).to(torch.int32)
+    cache = torch.randn(len(seqs) * pages * bs, C + R, generator=g).to(dt)
+    T = sum(n for _, n in seqs)
+    q = torch.randn(T, H * (Dn + R), generator=g).to(dt)
+    uk, uv = ((torch.randn(H * d, C, generator=g) / C ** 0.5).to(dt) for d in (Dn, V))
+    gate = torch.randn(T, H + 3, generator=g).to(dt)[:, 1:H + 1] if extra == "gate" else None
+    sinks = torch.randn(H, generator=g) * 3.0 if extra == "sinks" else None
+    cu = torch.tensor([0] + [n for _, n in seqs]).cumsum(0).to(torch.int32)
+    pos = torch.cat([torch.arange(a, a + n) for a, n in seqs]).to(torch.int32)
+    tok_seq = torch.repeat_interleave(torch.arange(len(seqs)), torch.tensor([n for _, n in seqs])).to(torch.int32)
+    d = lambda t: None if t is None else t.to(DEV)
+    b = {"positions": d(pos), "cu_q": d(cu), "tok_seq": d(tok_seq), "block_tables": d(bt), "max_qlen": max(n for _, n in seqs)}
+    ukv = sm.latent_expand(d(uk), d(uv), H, R)
+    args = (d(uk.view(H, Dn, C).transpose(1, 2).contiguous()), d(uv.view(H, V, C)), ukv, b, C, R, H, Dn, V, window, 0.07, bs)
+    gd = torch.randn(T, H + 3, generator=g).to(dt).to(DEV)[:, 1:H + 1].copy_(gate) if gate is not None else None
+    monkeypatch.setattr(sm, "LATENT_EXPAND_MIN", 1)
+    got = sm.latent_mix(d(q), d(cache), *args, sinks=d(sinks), gate=gd)
+    assert "latent_keys" in b
+    monkeypatch.setattr(sm, "LATENT_EXPAND_MIN", 0)
+    absorbed = sm.latent_mix(d(q), d(cache), *args, sinks=d(sinks), gate=gd)
+    want = torch.zeros(T, H, V, dtype=torch.float64, device=DEV)
+    for s, (a, n) in enumerate(seqs):
+        if not n:
+            continue
+        key = torch.arange(a + n)
+        rows = d(cache)[(bt[s].long()[key // bs] * bs + key % bs).to(DEV)].double()
+        k = torch.cat([(rows[:, :C] @ d(uk).double().T).view(-1, H, Dn), rows[:, None, C:].expand(-1, H, R)], 2)
+        v = (rows[:, :C] @ d(uv).double().T).view(-1, H, V)
+        r = slice(int(cu[s]), int(cu[s + 1]))
+        sc = torch.einsum("thd,khd->htk", d(q).double().view(T, H, -1)[r], k) * 0.07
+        age = (torch.arange(a, a + n)[:, None] - key[None, :]).to(DEV)
+        sc = sc.masked_fill((age < 0) | ((age >= window) if window else (age < 0)), -float("inf"))
+        if sinks is not None:
+            sc = torch.cat([sc, d(sinks).double()[:, None, None].expand(H, n, 1)], 2)
+        y = torch.einsum("htk,khv->thv", torch.softmax(sc, -1)[..., :a + n], v)
+        want[r] = y * (torch.sigmoid(gd[r].double())[:, :, None] if gate is not None else 1.0)
+    want = want.view(T, H * V)
+    scale = want.abs().max()
+    assert (got.double() - want).abs().max() <= tol * scale
+    err = lambda y: float((y.double() - want).norm() / want.norm())
+    assert err(got) <= 1.1 * err(absorbed) + 1e-7      # no less exact than the absorbed form
