@@ -171,6 +171,11 @@ int k8s_latent_attention_mfma(void* out, float* pacc, float* pml, const void* q_
                               const int* block_tables, int max_blocks, const int* tok_seq, const int* positions, int T,
                               int C, int R, int H, int Dn, int window, float scale, int bs, int nsplit, const int* cu_q,
                               int nseq, int max_qlen, const float* sinks, const void* gate, long ldg, hipStream_t s);
+int k8s_latent_token_ok(int C, int R, int Dn, int V);
+int k8s_latent_token(void* out, float* pacc, float* pml, const void* q_abs, const void* q, const void* cache, const void* uv,
+                     const int* block_tables, int max_blocks, const int* tok_seq, const int* positions, int T, int C, int R,
+                     int H, int Dn, int V, int window, float scale, int bs, int nsplit, const float* sinks, const void* gate,
+                     long ldg, hipStream_t s);
 int k8s_latent_prompt_ok(int C, int R, int Dn, int V);
 int k8s_latent_keys(int* rows, int* kbase, int* tiles, const int* cu_q, const int* positions, const int* block_tables,
                     int max_blocks, int nseq, int window, int bs, int cap, int ntiles, hipStream_t s);
@@ -603,6 +608,15 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
                                     max_blocks, P<int>(tok_seq), P<int>(positions), T, C, R, H, Dn, window, scale, bs,
                                     nsplit, P<int>(cu_q), nseq, max_qlen, P<float>(sinks), P(gate), ldg, S(s)),
           "latent_attention_mfma");
+  });
+  m.def("latent_token_ok", [](int C, int R, int Dn, int V) { return k8s_latent_token_ok(C, R, Dn, V) != 0; });
+  m.def("latent_token", [](uintptr_t out, uintptr_t pacc, uintptr_t pml, uintptr_t q_abs, uintptr_t q, uintptr_t cache,
+                           uintptr_t uv, uintptr_t bt, int max_blocks, uintptr_t tok_seq, uintptr_t positions, int T, int C,
+                           int R, int H, int Dn, int V, int window, float scale, int bs, int nsplit, uintptr_t sinks,
+                           uintptr_t gate, long ldg, int64_t s) {
+    check(k8s_latent_token(P(out), P<float>(pacc), P<float>(pml), P(q_abs), P(q), P(cache), P(uv), P<int>(bt), max_blocks,
+                           P<int>(tok_seq), P<int>(positions), T, C, R, H, Dn, V, window, scale, bs, nsplit,
+                           P<float>(sinks), P(gate), ldg, S(s)), "latent_token");
   });
   m.def("latent_prompt_ok", [](int C, int R, int Dn, int V) { return k8s_latent_prompt_ok(C, R, Dn, V) != 0; });
   m.def("latent_keys", [](uintptr_t rows, uintptr_t kbase, uintptr_t tiles, uintptr_t cu_q, uintptr_t positions,

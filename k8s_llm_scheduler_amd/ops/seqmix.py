@@ -1,7 +1,8 @@
 """Ops of models with an fp32 residual stream, recurrent / windowed- or latent-attention mixers and mixtures of experts.
 
 Same dispatch rule as the rest of :mod:`..ops`: CUDA (= HIP) tensors always run the gfx950 kernels
-(``stream32.hip``, ``mixers.hip``, ``latent_prompt.hip``, ``window_attn.hip``, ``gated_scan.hip``, ``decay_scan.hip``, ``delta_scan.hip``, ``moe.hip``) and raise when the extension is missing; CPU tensors run the fp32
+(``stream32.hip``, ``mixers.hip``, ``latent_prompt.hip``,
+``latent_token.hip``, ``window_attn.hip``, ``gated_scan.hip``, ``decay_scan.hip``, ``delta_scan.hip``, ``moe.hip``) and raise when the extension is missing; CPU tensors run the fp32
 reference in :mod:`.reference` (the CPU test-suite).  Every op takes bf16 or true-fp32 activations / weights (the
 ``f32`` flag of the kernels); what a design computes in fp32 regardless (residual sum, recurrent state, decays, router,
 attention scores) is fp32 in both.
@@ -492,15 +493,15 @@ def latent_mix(q: torch.Tensor, cache: torch.Tensor, uk_t: torch.Tensor, uv: tor
     take the result through W_uv; batches of longer portions write the visible rows' keys and values out first."""
     T = q.shape[0]
     dt = q.dtype
+    if sinks is not None and (sinks.dtype != F32 or sinks.numel() != H):
+        raise ValueError("latent_mix: sinks are fp32 [H]")
+    if gate is not None and (gate.shape != (T, H) or gate.dtype != dt or gate.stride(1) != 1):
+        raise ValueError("latent_mix: the gate is [T, H] of the queries' type with contiguous rows")
     nseq, max_qlen = b["cu_q"].shape[0] - 1, b.get("max_qlen", 0)
     ctx = b["block_tables"].shape[1] * block_size
     cap = min(T + nseq * (window - 1), nseq * ctx) if window else nseq * ctx
     if (ukv is not None and _gpu(q, cache) and max_qlen > 0 and 0 < LATENT_EXPAND_MIN * nseq <= T and cap < 1 << 24
             and cap * H * (Dn + V) * q.element_size() <= LATENT_EXPAND_BYTES and _native().latent_prompt_ok(C, R, Dn, V)):
-        if sinks is not None and (sinks.dtype != F32 or sinks.numel() != H):
-            raise ValueError("latent_mix: sinks are fp32 [H]")
-        if gate is not None and (gate.shape != (T, H) or gate.dtype != dt or gate.stride(1) != 1):
-            raise ValueError("latent_mix: the gate is [T, H] of the queries' type with contiguous rows")
         rows, kbase, tiles = _latent_keys(b, int(window), block_size, cap)
         kv = torch.empty(cap, H * (Dn + V), dtype=dt, device=q.device)
         nat = _native()
@@ -514,6 +515,21 @@ def latent_mix(q: torch.Tensor, cache: torch.Tensor, uk_t: torch.Tensor, uv: tor
         return out
     q_abs = torch.empty(T, H, C, dtype=dt, device=q.device)
     gemm(q.view(T, H, Dn + R)[:, :, :Dn].permute(1, 0, 2), uk_t, out=q_abs.permute(1, 0, 2))
+    if max_qlen == 0 and dt == BF16 and _gpu(q, cache, sinks, gate) and _native().latent_token_ok(C, R, Dn, V):
+        # decoding: key splits of at least one 64-key step for about one workgroup per CU, joined by the kernel that takes
+        # the sums through W_uv
+        HP = (H + 15) // 16 * 16
+        seen = min(b.get("max_keys", 0) or ctx, window or ctx, ctx)
+        ns = max(1, min(256 // (T * (HP // 16)), (seen + 63) // 64, 32))
+        pacc = torch.empty(T * HP * ns * C, dtype=F32, device=q.device)
+        pml = torch.empty(T * HP * ns * 2, dtype=F32, device=q.device)
+        out = torch.empty(T, H * V, dtype=dt, device=q.device)
+        _native().latent_token(out.data_ptr(), pacc.data_ptr(), pml.data_ptr(), q_abs.data_ptr(), _p(q),
+                               _p(cache, dt, "cache"), _p(uv, dt, "uv"), _p(b["block_tables"], I32),
+                               b["block_tables"].shape[1], _p(b["tok_seq"], I32), _p(b["positions"], I32), T, C, R, H, Dn, V,
+                               int(window), float(scale), block_size, ns, _p(sinks),
+                               gate.data_ptr() if gate is not None else 0, gate.stride(0) if gate is not None else 0, -1)
+        return out
     lat = latent_attention(q_abs, q, cache, b["block_tables"], b["tok_seq"], b["positions"], C, R, H, Dn, window, scale,
                            block_size, b.get("max_keys", 0), b["cu_q"], max_qlen, sinks=sinks, gate=gate)     # [T, H, C]
     a = torch.empty(T, H, V, dtype=dt, device=q.device)

@@ -107,3 +107,48 @@ def test_latent_prompt(dt, tol, seqs, window, H, extra, monkeypatch):
     assert (got.double() - want).abs().max() <= tol * scale
     err = lambda y: float((y.double() - want).norm() / want.norm())
     assert err(got) <= 1.1 * err(absorbed) + 1e-7      # no less exact than the absorbed form
+
+
+# contexts of the rows (0: idle), window: around one 64-key step, one split per step and several steps per split, windows that
+# start inside a page, one row, more rows than a group of four
+@pytest.mark.parametrize("ctx,window,H", [([1, 63, 64, 65, 0, 129], 0, 3), ([530], 1024, 16), ([700, 2, 333], 100, 32),
+                                          ([0], 0, 16), ([1025] * 18, 0, 16), ([600, 17, 0, 900, 64], 513, 20)])
+@pytest.mark.parametrize("extra", ["", "gate", "sinks"])
+def test_latent_token(ctx, window, H, extra):
+    """Decoding in the latent space against 64 bits; tolerance as for the kernels it replaces, and no less exact than them."""
+    C, R, Dn, V, bs, dt = 512, 64, 128, 128, 16, torch.bfloat16
+    g = torch.Generator().manual_seed(sum(ctx) + window + H)
+    T, pages = len(ctx), -(-max(max(ctx), 1) // bs) + 2
+    bt = torch.randperm(T * pages, generator=g).view(T, pages).to(torch.int32)
+    r = lambda *s: torch.randn(*s, generator=g)
+    cache, q = r(T * pages * bs, C + R).to(dt).to(DEV), r(T, H * (Dn + R)).to(dt).to(DEV)
+    uk, uv = ((r(H * d, C) / C ** 0.5).to(dt).to(DEV) for d in (Dn, V))
+    gate = r(T, H + 3).to(dt).to(DEV)[:, 1:H + 1] if extra == "gate" else None
+    sinks = (r(H) * 3.0).to(DEV) if extra == "sinks" else None
+    pos = torch.tensor(ctx, dtype=torch.int32) - 1
+    ar = torch.arange(T + 1, dtype=torch.int32, device=DEV)
+    b = {"positions": pos.to(DEV), "cu_q": ar, "tok_seq": ar[:T], "block_tables": bt.to(DEV), "max_keys": pages * bs}
+    uk_t, uv3 = uk.view(H, Dn, C).transpose(1, 2).contiguous(), uv.view(H, V, C)
+    got = sm.latent_mix(q, cache, uk_t, uv3, None, b, C, R, H, Dn, V, window, 0.07, bs, sinks=sinks, gate=gate)
+    qa = torch.empty(T, H, C, dtype=dt, device=DEV)
+    sm.gemm(q.view(T, H, Dn + R)[:, :, :Dn].permute(1, 0, 2), uk_t, out=qa.permute(1, 0, 2))
+    lat = sm.latent_attention(qa, q, cache, b["block_tables"], b["tok_seq"], b["positions"], C, R, H, Dn, window, 0.07, bs,
+                              sinks=sinks, gate=gate)
+    old = torch.empty(T, H, V, dtype=dt, device=DEV)
+    sm.gemm(lat.permute(1, 0, 2), uv3, out=old.permute(1, 0, 2))
+    want = torch.zeros(T, H, V, dtype=torch.float64, device=DEV)
+    for t, n in enumerate(ctx):
+        if not n:
+            continue
+        key = torch.arange(max(0, n - window) if window else 0, n)
+        rows = cache[(bt[t].long()[key // bs] * bs + key % bs).to(DEV)].double()
+        k = torch.cat([(rows[:, :C] @ uk.double().T).view(-1, H, Dn), rows[:, None, C:].expand(-1, H, R)], 2)
+        sc = torch.einsum("hd,khd->hk", q[t].double().view(H, -1), k) * 0.07
+        if sinks is not None:
+            sc = torch.cat([sc, sinks.double()[:, None]], 1)
+        y = torch.einsum("hk,khv->hv", torch.softmax(sc, -1)[:, :len(key)], (rows[:, :C] @ uv.double().T).view(-1, H, V))
+        want[t] = y * (torch.sigmoid(gate[t].double())[:, None] if gate is not None else 1.0)
+    want = want.view(T, H * V)
+    assert (got.double() - want).abs().max() <= 2e-2 * want.abs().max()
+    err = lambda y: float((y.double() - want).norm() / want.norm().clamp(min=1e-30))
+    assert err(got) <= 1.1 * err(old.view(T, H * V)) + 1e-7
