@@ -149,8 +149,8 @@ int k8s_act(void* out, const void* x, int T, int F, int kind, float limit, float
 int k8s_gemm_any(void* C, const void* A, const void* W, int M, int N, int K, long lda, long ldw, long ldc, int batch,
                  long sA, long sW, long sC, const int* a_rows, const int* tiles, int ntiles, int in_f32, int out_f32,
                  hipStream_t s);
-int k8s_token_shift(void* out, const void* h, const void* mu, const void* state, const int* cu_q, const int* tok_seq,
-                    const int* seq_slots, const int* positions, int n, int T, int W, int f32, hipStream_t s);
+int k8s_token_shift(void* out, const void* h, const void* mu, void* state, const int* cu_q, const int* tok_seq,
+                    const int* seq_slots, const int* positions, int n, int T, int W, int save, int f32, hipStream_t s);
 int k8s_shift_save(void* state, const void* h, const int* cu_q, const int* seq_slots, const int* positions, int nseq,
                    int W, int f32, hipStream_t s);
 int k8s_wkv_max_dim();
@@ -564,9 +564,9 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
                        ntiles, in_f32, out_f32, S(s)), "gemm_any");
   });
   m.def("token_shift", [](uintptr_t out, uintptr_t h, uintptr_t mu, uintptr_t state, uintptr_t cu_q, uintptr_t tok_seq,
-                          uintptr_t seq_slots, uintptr_t positions, int n, int T, int W, int f32, int64_t s) {
+                          uintptr_t seq_slots, uintptr_t positions, int n, int T, int W, int save, int f32, int64_t s) {
     check(k8s_token_shift(P(out), P(h), P(mu), P(state), P<int>(cu_q), P<int>(tok_seq), P<int>(seq_slots),
-                          P<int>(positions), n, T, W, f32, S(s)), "token_shift");
+                          P<int>(positions), n, T, W, save, f32, S(s)), "token_shift");
   });
   m.def("shift_save", [](uintptr_t state, uintptr_t h, uintptr_t cu_q, uintptr_t seq_slots, uintptr_t positions,
                          int nseq, int W, int f32, int64_t s) {

@@ -59,6 +59,55 @@ __global__ __launch_bounds__(256) void resnorm_kernel(float* __restrict__ x, con
   }
 }
 
+// The form without groups for rows of whole vectors (W % 4 == 0, W <= 1024 NV, aligned pointers), w given: all loads ahead of
+// the reduction, the row in registers.  Bound by memory for prompts and by latency for single rows: 2048 rows of 2048, bf16
+// branch, 15.4 -> 10.4 us (50 MB: 6.3 us at 8 TB/s); 8 rows 7.7 -> 4.6 us.
+template <typename TA, int NV>
+__global__ __launch_bounds__(256) void resnorm_row_kernel(float* __restrict__ x, const TA* __restrict__ branch,
+                                                          const TA* __restrict__ branch2, float mult,
+                                                          const TA* __restrict__ rowvec, const TA* __restrict__ w,
+                                                          float offset, float eps, TA* __restrict__ out, int W) {
+  __shared__ float red[16];
+  const size_t base = (size_t)blockIdx.x * W;
+  const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 xv[NV], bv[NV], cv[NV], rv[NV], wv[NV];
+#pragma unroll
+  for (int n = 0; n < NV; ++n) {
+    const int i = 4 * (threadIdx.x + 256 * n);
+    const bool in = i < W;
+    xv[n] = in ? ldf4(x + base + i) : zero;
+    bv[n] = in && branch != nullptr ? ldf4(branch + base + i) : zero;
+    cv[n] = in && branch2 != nullptr ? ldf4(branch2 + base + i) : zero;
+    rv[n] = in && rowvec != nullptr ? ldf4(rowvec + i) : zero;
+    wv[n] = in ? ldf4(w + i) : zero;
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int n = 0; n < NV; ++n) {
+    const int i = 4 * (threadIdx.x + 256 * n);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float v = xv[n][e];
+      if (branch != nullptr) v += mult * (bv[n][e] + cv[n][e]);
+      if (rowvec != nullptr) v += rv[n][e];
+      xv[n][e] = v;
+      ss += v * v;
+    }
+    if (i < W && (branch != nullptr || rowvec != nullptr)) stf4(x + base + i, xv[n]);
+  }
+  ss = block_sum(ss, red);
+  const float inv = 1.0f / sqrtf(ss / (float)W + eps);
+#pragma unroll
+  for (int n = 0; n < NV; ++n) {
+    const int i = 4 * (threadIdx.x + 256 * n);
+    if (i >= W) continue;
+    f32x4 y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = xv[n][e] * inv * (offset + wv[n][e]);
+    stf4(out + base + i, y);
+  }
+}
+
 // Norm after the sum: x[t] <- (alpha x[t] + c1 branch[t] + c2 branch2[t]) / sqrt(mean(.^2) + eps) * gain, stored back
 // in fp32 (the stream stays normed); `out` (optional) receives the same row in the activation type, for the sublayer
 // that reads it next.  `gain` is one number for the whole row.  One workgroup per row; the row is held in registers
@@ -766,13 +815,26 @@ extern "C" int k8s_resnorm(float* x, const void* branch, const void* branch2, fl
   if (T <= 0) return 0;
   if (W <= 0 || (w != nullptr && out == nullptr) || groups < 1 || W % groups || (branch2 != nullptr && branch == nullptr))
     return -1;
-  if (f32)
-    resnorm_kernel<float><<<T, 256, 0, s>>>(x, (const float*)branch, (const float*)branch2, mult, (const float*)rowvec,
-                                            (const float*)w, offset, eps, (float*)out, W, groups);
-  else
-    resnorm_kernel<bf16_t><<<T, 256, 0, s>>>(x, (const bf16_t*)branch, (const bf16_t*)branch2, mult,
-                                             (const bf16_t*)rowvec, (const bf16_t*)w, offset, eps, (bf16_t*)out, W,
-                                             groups);
+#define K8S_RN(TA, NV)                                                                                              \
+  resnorm_row_kernel<TA, NV><<<T, 256, 0, s>>>(x, (const TA*)branch, (const TA*)branch2, mult, (const TA*)rowvec,     \
+                                               (const TA*)w, offset, eps, (TA*)out, W)
+#define K8S_RN_T(TA)                                                                                                \
+  do {                                                                                                              \
+    const bool vec = w != nullptr && groups == 1 && W % 4 == 0 && W <= 8192 && (uintptr_t)x % 16 == 0 &&             \
+                     ((uintptr_t)branch | (uintptr_t)branch2 | (uintptr_t)rowvec | (uintptr_t)w | (uintptr_t)out) %  \
+                             (4 * sizeof(TA)) == 0;                                                                 \
+    if (!vec)                                                                                                       \
+      resnorm_kernel<TA><<<T, 256, 0, s>>>(x, (const TA*)branch, (const TA*)branch2, mult, (const TA*)rowvec,        \
+                                           (const TA*)w, offset, eps, (TA*)out, W, groups);                         \
+    else if (W <= 1024) K8S_RN(TA, 1);                                                                              \
+    else if (W <= 2048) K8S_RN(TA, 2);                                                                              \
+    else if (W <= 4096) K8S_RN(TA, 4);                                                                              \
+    else K8S_RN(TA, 8);                                                                                             \
+  } while (0)
+  if (f32) K8S_RN_T(float);
+  else K8S_RN_T(bf16_t);
+#undef K8S_RN_T
+#undef K8S_RN
   return (int)hipGetLastError();
 }
 

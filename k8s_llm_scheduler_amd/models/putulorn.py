@@ -440,8 +440,7 @@ class PutulornModel(StreamModel):
     def _wkv(self, w: _Wkv, run: _Run, h, b) -> torch.Tensor:
         m = w.cfg
         S, shift = self.states[run.cache]
-        mix = sm.token_shift(h, w.mu, shift, b["cu_q"], b["tok_seq"], b["seq_slots"], b["positions"])   # [5, T, W]
-        sm.shift_save(shift, h, b["cu_q"], b["seq_slots"], b["positions"])
+        mix = sm.token_shift(h, w.mu, shift, b["cu_q"], b["tok_seq"], b["seq_slots"], b["positions"], save=True)   # [5, T, W]
         if sm.FAST_GEMM and h.is_cuda and sm._route_fast(mix[0], w.w_rkvg[0], self.dtype):
             r, k, v, g = (sm.linear(mix[i], w.w_rkvg[i]) for i in range(4))
         else:

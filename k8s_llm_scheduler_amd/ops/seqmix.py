@@ -311,17 +311,20 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out_dtype=None, *, a_rows: Optional[t
 
 # ----------------------------------------------------------------------------- recurrent mixer
 def token_shift(h: torch.Tensor, mu: torch.Tensor, state: torch.Tensor, cu_q: torch.Tensor, tok_seq: torch.Tensor,
-                seq_slots: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
+                seq_slots: torch.Tensor, positions: torch.Tensor, save: bool = False) -> torch.Tensor:
     """[n, T, W]: h + (previous token's h - h) * mu[s]; the previous token of a portion's first token is the slot's
-    row of ``state`` (zeros at position 0)."""
+    row of ``state`` (zeros at position 0).  ``save``: then, as :func:`shift_save`, state[slot] = the portion's last h."""
     if not _gpu(h, mu, state):
-        return ref.token_shift(h, mu, state, cu_q, seq_slots, positions)
+        out = ref.token_shift(h, mu, state, cu_q, seq_slots, positions)
+        if save:
+            ref.shift_save(state, h, cu_q, seq_slots, positions)
+        return out
     T, W = h.shape
     n = mu.shape[0]
     out = torch.empty(n, T, W, dtype=h.dtype, device=h.device)
     _native().token_shift(out.data_ptr(), _p(h), _p(mu, h.dtype, "mu"), _p(state, h.dtype, "state"),
                           _p(cu_q, I32, "cu_q"), _p(tok_seq, I32, "tok_seq"), _p(seq_slots, I32, "seq_slots"),
-                          _p(positions, I32, "positions"), n, T, W, _f32(h.dtype), -1)
+                          _p(positions, I32, "positions"), n, T, W, int(save), _f32(h.dtype), -1)
     return out
 
 

@@ -152,3 +152,32 @@ def test_latent_token(ctx, window, H, extra):
     assert (got.double() - want).abs().max() <= 2e-2 * want.abs().max()
     err = lambda y: float((y.double() - want).norm() / want.norm().clamp(min=1e-30))
     assert err(got) <= 1.1 * err(old.view(T, H * V)) + 1e-7
+
+
+@pytest.mark.parametrize("dt,tol", [(torch.float32, 2e-6), (torch.bfloat16, 1e-2)])
+@pytest.mark.parametrize("W", [4, 1023, 1024, 1028, 2052, 8192, 8196])
+def test_row_norm_and_token_shift_widths(dt, tol, W):
+    """Widths around the vector forms' register counts and the scalar forms beyond them, every optional operand, idle rows."""
+    from k8s_llm_scheduler_amd.ops import reference as ref
+    g = torch.Generator().manual_seed(W)
+    r = lambda *s: torch.randn(*s, generator=g)
+    T = 7
+    x, b1, b2, rv, w = r(T, W), r(T, W).to(dt), r(T, W).to(dt), r(W).to(dt), r(W).to(dt)
+    for branch, branch2, rowvec in ((b1, b2, rv), (b1, None, None), (None, None, rv), (None, None, None)):
+        xg, xc = x.to(DEV), x.clone()
+        d = lambda t: None if t is None else t.to(DEV)
+        got = sm.resnorm(xg, d(w), 1e-6, branch=d(branch), branch2=d(branch2), mult=0.3, rowvec=d(rowvec), offset=1.0, out_dtype=dt)
+        want = sm.resnorm(xc, w, 1e-6, branch=branch, branch2=branch2, mult=0.3, rowvec=rowvec, offset=1.0, out_dtype=dt)
+        assert (got.cpu().float() - want.float()).abs().max() <= tol * want.float().abs().max()
+        assert (xg.cpu() - xc).abs().max() <= 1e-6 * xc.abs().max()
+    cu = torch.tensor([0, 3, 3, 4, 5, 7], dtype=torch.int32)
+    pos = torch.tensor([0, 1, 2, -1, 9, 4, 5], dtype=torch.int32)
+    slots, tok_seq = torch.tensor([4, 0, 1, 2, 3], dtype=torch.int32), torch.tensor([0, 0, 0, 2, 3, 4, 4], dtype=torch.int32)
+    h, mu, st = r(T, W).to(dt), torch.rand(5, W, generator=g).to(dt), r(5, W).to(dt)
+    sg, sc = st.to(DEV), st.clone()
+    got = sm.token_shift(h.to(DEV), mu.to(DEV), sg, *(t.to(DEV) for t in (cu, tok_seq, slots, pos)), save=True).cpu()
+    want = ref.token_shift(h, mu, sc, cu, slots, pos)
+    ref.shift_save(sc, h, cu, slots, pos)
+    live = pos >= 0
+    assert (got[:, live].float() - want[:, live].float()).abs().max() <= tol * want.float().abs().max()
+    assert (got[:, ~live] == 0).all() and torch.equal(sg.cpu(), sc)
