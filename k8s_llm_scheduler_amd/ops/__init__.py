@@ -908,9 +908,51 @@ def _pg_load_table() -> dict:
     return _PG_TABLE
 
 
+# Time of a bf16 plan in us, (kernel, configuration) -> (fixed, per 64-deep k-step, per round, split, per MB of slab, per MB of
+# weights, per MB of output): a launch; per round of tiles over the CUs a fill and the tile's k-steps; with split-K the combine
+# launch and the slabs it moves; the weights and the output.  Fitted to 22 weight shapes (1152 x 2048 .. 28672 x 4096) at 8 row
+# counts (160 .. 2048), weights cold: rms error 5-8 % per configuration, the pick within 2 % of the best plan on average and
+# 24 % at most.  256 x 256 pgemm tiles with split-K until the grid is full (the rule before, and still the one of fp8 and
+# SwiGLU, which these figures do not cover) take 1.43 times as long on average: 2048 x 2048 x 2048 41.5 us, 24.6 us on 128 x
+# 128 tiles without a combine.  Past 64 k-steps the 128 x 128 tiles' operands fall out of an XCD's L2 between other kernels
+# (2048 x 2048 x 8192 inside a prompt: 91 us, alone 77; 72-80 us on split 256 x 256 tiles): _P4_LONG_K us more per step.
+_P4_COST = {("pgemm4", 1): (1.34, 0.754, 3.48, 4.66, 0.236, 0.0945, 0.485),
+            ("pgemm4", 2): (1.53, 0.738, 2.97, 4.19, 0.283, 0.0636, 0.555),
+            ("pgemm4", 3): (3.32, 0.440, 0.0, 3.82, 0.273, 0.0996, 0.480),
+            ("pgemm4", 4): (2.70, 1.158, 7.51, 3.61, 0.224, 0.0581, 0.248),
+            ("pgemm", 0): (5.50, 1.147, 11.06, 0.0, 0.163, 0.0143, 0.575)}
+_P4_LONG_K = 0.15
+
+
+@functools.lru_cache(maxsize=4096)
+def _pgemm_cheapest(M: int, N: int, K: int, num_cus: int) -> Tuple[str, int, int]:
+    """(kernel, configuration, splits) of the cheapest bf16 plan by _P4_COST."""
+    kt, best = K // 64, None
+    for (kern, cfg), (t0, step, rnd, sp, slab, wmb, omb) in _P4_COST.items():
+        bp, bq, _ = (pgemm4_configs() if kern == "pgemm4" else pgemm_configs())[cfg]
+        tiles = -(-N // bp) * -(-M // bq)
+        base = t0 + wmb * N * K * 2e-6 + omb * M * N * 2e-6
+        for s in (1, 2, 3, 4, 6, 8, 12, 16):
+            if s > 1 and (tiles * s > 2 * num_cus or kt // s < 4):
+                break
+            rounds, per = -(-tiles * s // num_cus), -(-kt // s)
+            us = base + rounds * (rnd + step * per) + (sp + slab * M * N * s * 4e-6 if s > 1 else 0.0)
+            if bp * bq <= 128 * 128:
+                us += _P4_LONG_K * max(0, per - 64) * rounds
+            if best is None or us < best[0]:
+                best = (us, kern, cfg, s)
+    return best[1:]
+
+
 def pgemm_heuristic(M: int, N: int, K: int, epi: int, fp8: bool, num_cus: int = 256) -> Tuple[str, int, int, int]:
-    """Big-tile plan of a shape the table has never seen: 256 x 256 tiles (pgemm.hip), split-K until the grid
-    covers the CUs."""
+    """Big-tile plan of a shape the table has never seen.  bf16 with a plain epilogue: the cheapest plan by _P4_COST at the
+    row count rounded up to 64.  Else 256 x 256 tiles (pgemm.hip), split-K until the grid covers the CUs."""
+    if not fp8 and epi in (EPI_BF16, EPI_F32) and K % 64 == 0:
+        return _pgemm_cheapest(-(-M // 64) * 64, N, K, num_cus) + (4,)
+    return _pgemm_big_tiles(M, N, K, epi, fp8, num_cus)
+
+
+def _pgemm_big_tiles(M: int, N: int, K: int, epi: int, fp8: bool, num_cus: int = 256) -> Tuple[str, int, int, int]:
     cfg = 0
     tiles = pgemm_tiles(cfg, M, N, epi)
     kt = K * (1 if fp8 else 2) // 128
@@ -949,7 +991,7 @@ def gemm_route(M: int, N: int, K: int, epi: int, fp8: bool) -> Tuple[str, Option
     plan, pg_us = pgemm_plan_for(M, N, K, epi, fp8)
     if GEMM_BACKEND == "pgemm":
         if plan[0] == "mgemm":
-            plan = pgemm_heuristic(M, N, K, epi, fp8)
+            plan = _pgemm_big_tiles(M, N, K, epi, fp8)
         return plan[0], plan[1:]
     if M < PG_MIN_M or plan[0] == "mgemm":   # (the tuner records "mgemm" where its tuned plan was faster)
         return "mgemm", None

@@ -68,6 +68,23 @@ def test_pgemm_table_picks_nearest_bucket_at_or_above(monkeypatch):
     assert ops.pgemm_plan_for(200, 100, 256, 0, True)[0][0] == "pgemm"
 
 
+def test_untuned_shapes_take_a_plan_that_runs(monkeypatch):
+    """Row counts around the tile heights and odd ones, weights of any aligned size: the cost rule's plan is one that the
+    kernel's own planner accepts, and it depends on the row count rounded up to 64 only."""
+    monkeypatch.setattr(ops, "_PG_TABLE", {})
+    for M in (129, 191, 192, 257, 333, 1000, 2048, 4097, 70000):
+        for N, K in ((16, 128), (100, 64), (576, 2048), (2048, 192), (16384, 4096), (128, 28672)):
+            for epi in (ops.EPI_BF16, ops.EPI_F32):
+                kern, cfg, sp, gm = ops.pgemm_heuristic(M, N, K, epi, False)
+                assert kern in ("pgemm", "pgemm4") and sp <= max(1, K // 64 // 4)
+                plan = ops.native().pgemm4_plan(M, N, K, epi, cfg, sp) if kern == "pgemm4" else \
+                    ops.native().pgemm_plan(M, N, K, epi, 0, cfg, sp)
+                assert plan[0] > 0
+                assert ops.pgemm_heuristic(-(-M // 64) * 64, N, K, epi, False) == (kern, cfg, sp, gm)
+    assert ops.pgemm_heuristic(2048, 2048, 2048, ops.EPI_BF16, True)[0] == "pgemm"
+    assert ops.pgemm_heuristic(2048, 2048, 2048, ops.EPI_SWIGLU, False)[0] == "pgemm"
+
+
 def test_auto_follows_the_tuned_winner(monkeypatch):
     monkeypatch.setattr(ops, "GEMM_BACKEND", "auto")
     monkeypatch.setattr(ops, "_PG_TABLE", {(1024, 1024, 0, 0): [(256, "mgemm", 0, 0, 0, 25.0),
