@@ -110,6 +110,11 @@ int k8s_mgemm(void* out, float* ws, unsigned* tickets, const void* x, const void
 int k8s_pgemm4_num_configs();
 int k8s_pgemm4_config(int cfg, int* bp, int* bq, int* lds_bytes);
 int k8s_pgemm4_plan(int M, int N_out, int K, int epi, int cfg, int splits, int* nwg, long long* slab_elems);
+int k8s_pgemm4_act(void* out, const void* x, const void* W, int M, int N_out, int K, int cfg, int group_m, int kind,
+                   float limit, float alpha, const void* bias, hipStream_t stream);
+int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M, int rows, int N_out, int K, int groups, const int* seg,
+                       const int* a_rows, long ldx, int cfg, int group_m, int kind, float limit, float alpha,
+                       hipStream_t stream);
 int k8s_pgemm4(void* out, float* slab, const void* x, const void* W, int M, int N_out, int K, int epi, int cfg,
                int splits, int group_m, const void* res, int rms, float eps, hipStream_t s);
 int k8s_embed_rows(float* out, const int* ids, const void* table, int T, int W, int vocab, float scale, int f32,
@@ -177,7 +182,7 @@ int k8s_latent_token(void* out, float* pacc, float* pml, const void* q_abs, cons
                      int H, int Dn, int V, int window, float scale, int bs, int nsplit, const float* sinks, const void* gate,
                      long ldg, hipStream_t s);
 int k8s_latent_prompt_ok(int C, int R, int Dn, int V);
-int k8s_latent_keys(int* rows, int* kbase, int* tiles, const int* cu_q, const int* positions, const int* block_tables,
+int k8s_latent_keys(int* rows, int* kbase, int* tiles, int* seg, const int* cu_q, const int* positions, const int* block_tables,
                     int max_blocks, int nseq, int window, int bs, int cap, int ntiles, hipStream_t s);
 int k8s_latent_prompt(void* out, const void* kv, const int* rows, const int* kbase, const void* q, const void* cache, int C,
                       int R, int Dn, int V, const int* cu_q, const int* positions, int nseq, int max_qlen, int H, int window,
@@ -619,10 +624,10 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
                            P<float>(sinks), P(gate), ldg, S(s)), "latent_token");
   });
   m.def("latent_prompt_ok", [](int C, int R, int Dn, int V) { return k8s_latent_prompt_ok(C, R, Dn, V) != 0; });
-  m.def("latent_keys", [](uintptr_t rows, uintptr_t kbase, uintptr_t tiles, uintptr_t cu_q, uintptr_t positions,
+  m.def("latent_keys", [](uintptr_t rows, uintptr_t kbase, uintptr_t tiles, uintptr_t seg, uintptr_t cu_q, uintptr_t positions,
                           uintptr_t bt, int max_blocks, int nseq, int window, int bs, int cap, int ntiles, int64_t s) {
-    check(k8s_latent_keys(P<int>(rows), P<int>(kbase), P<int>(tiles), P<int>(cu_q), P<int>(positions), P<int>(bt), max_blocks,
-                          nseq, window, bs, cap, ntiles, S(s)), "latent_keys");
+    check(k8s_latent_keys(P<int>(rows), P<int>(kbase), P<int>(tiles), P<int>(seg), P<int>(cu_q), P<int>(positions), P<int>(bt),
+                          max_blocks, nseq, window, bs, cap, ntiles, S(s)), "latent_keys");
   });
   m.def("latent_prompt", [](uintptr_t out, uintptr_t kv, uintptr_t rows, uintptr_t kbase, uintptr_t q, uintptr_t cache, int C,
                             int R, int Dn, int V, uintptr_t cu_q, uintptr_t positions, int nseq, int max_qlen, int H,
@@ -770,6 +775,15 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
     if (k8s_pgemm4_plan(M, N, K, epi, cfg, splits, &nwg, &slab) != 0)
       throw std::invalid_argument("pgemm4_plan: invalid plan");
     return py::make_tuple(nwg, slab);
+  });
+  m.def("pgemm4_act", [](uintptr_t out, uintptr_t x, uintptr_t W, int M, int N, int K, int cfg, int group_m, int kind,
+                         float limit, float alpha, uintptr_t bias, int64_t s) {
+    check(k8s_pgemm4_act(P(out), P(x), P(W), M, N, K, cfg, group_m, kind, limit, alpha, P(bias), S(s)), "pgemm4_act");
+  });
+  m.def("pgemm4_grouped", [](uintptr_t out, uintptr_t x, uintptr_t W, int M, int rows, int N, int K, int groups, uintptr_t seg,
+                             uintptr_t a_rows, long ldx, int cfg, int group_m, int kind, float limit, float alpha, int64_t s) {
+    check(k8s_pgemm4_grouped(P(out), P(x), P(W), M, rows, N, K, groups, P<int>(seg), P<int>(a_rows), ldx, cfg, group_m, kind,
+                             limit, alpha, S(s)), "pgemm4_grouped");
   });
   m.def("pgemm4", [](uintptr_t out, uintptr_t slab, uintptr_t x, uintptr_t W, int M, int N, int K, int epi, int cfg,
                      int splits, int group_m, uintptr_t res, int rms, float eps, int64_t s) {

@@ -27,9 +27,10 @@ __device__ __forceinline__ int latent_span(const int* cu_q, const int* positions
 }
 
 // One workgroup per sequence: rows[kbase[s] + i] = cache slot of the sequence's key lo + i; tiles (0, first row, rows) of at
-// most 64 rows each, the entries behind the last one (-1, 0, 0).
+// most 64 rows each, the entries behind the last one (-1, 0, 0); seg = (0, rows of all sequences).
 __global__ __launch_bounds__(256) void latent_keys_kernel(int* __restrict__ rows, int* __restrict__ kbase,
-                                                          int* __restrict__ tiles, const int* __restrict__ cu_q,
+                                                          int* __restrict__ tiles, int* __restrict__ seg,
+                                                          const int* __restrict__ cu_q,
                                                           const int* __restrict__ positions,
                                                           const int* __restrict__ block_tables, int max_blocks, int nseq,
                                                           int window, int bs, int cap, int ntiles) {
@@ -44,7 +45,13 @@ __global__ __launch_bounds__(256) void latent_keys_kernel(int* __restrict__ rows
   }
   const int base = (int)block_sum(nr, red), tile0 = (int)block_sum(nt, red);
   const int n = min(latent_span(cu_q, positions, s, window, lo), cap - base);
-  if (threadIdx.x == 0) kbase[s] = base;
+  if (threadIdx.x == 0) {
+    kbase[s] = base;
+    if (s == nseq - 1) {
+      seg[0] = 0;
+      seg[1] = base + max(n, 0);
+    }
+  }
   const int* btr = block_tables + (size_t)s * max_blocks;
   for (int i = threadIdx.x; i < n; i += blockDim.x) {
     const int key = lo + i, page = key / bs;
@@ -443,13 +450,13 @@ using namespace k8sllm;
 // Whether the kernels take these sizes.
 extern "C" int k8s_latent_prompt_ok(int C, int R, int Dn, int V) { return C % 8 == 0 && Dn == 128 && R == 64 && V == 128; }
 
-// rows [cap], kbase [nseq], tiles [ntiles][3]; cap and ntiles bound the batch's visible rows and their tiles.
-extern "C" int k8s_latent_keys(int* rows, int* kbase, int* tiles, const int* cu_q, const int* positions,
+// rows [cap], kbase [nseq], tiles [ntiles][3], seg [2]; cap and ntiles bound the batch's visible rows and their tiles.
+extern "C" int k8s_latent_keys(int* rows, int* kbase, int* tiles, int* seg, const int* cu_q, const int* positions,
                                const int* block_tables, int max_blocks, int nseq, int window, int bs, int cap, int ntiles,
                                hipStream_t s) {
   if (nseq <= 0) return 0;
   if (bs <= 0 || cap <= 0 || cap >= (1 << 24) || ntiles < cap / 64 + nseq) return -1;
-  latent_keys_kernel<<<nseq, 256, 0, s>>>(rows, kbase, tiles, cu_q, positions, block_tables, max_blocks, nseq, window, bs, cap,
+  latent_keys_kernel<<<nseq, 256, 0, s>>>(rows, kbase, tiles, seg, cu_q, positions, block_tables, max_blocks, nseq, window, bs, cap,
                                           ntiles);
   return (int)hipGetLastError();
 }

@@ -1,6 +1,7 @@
 // K3 / K8 / K9(+K10) / K11 / K12 at prefill row counts, bf16: the 4-wave big-tile MFMA GEMM.
 //
-//     out[M, N_out] = epi( x[M, K] . W[N, K]^T )      epi: bf16 (+ residual) | fp32 | SwiGLU, optional RMS prologue
+//     out[M, N_out] = epi( x[M, K] . W[N, K]^T )      epi: bf16 (+ residual) | fp32 | SwiGLU, optional RMS prologue;
+//                                                     an activation (elementwise, or gated with W = [gate; up])
 //
 // Why 4 waves (and not pgemm.hip's 8-wave ping-pong): PMC on the 2048 x 8192 x 8192 projection showed the
 // 8-wave 128 x 64-per-wave schedule parked 31 % of its wave cycles at barriers (SQ_WAIT_ANY) and issued 1.5x
@@ -30,7 +31,7 @@
 namespace k8sllm {
 
 namespace {
-enum { P4_BF16 = 0, P4_F32 = 1, P4_SWIGLU = 2 };
+enum { P4_BF16 = 0, P4_F32 = 1, P4_SWIGLU = 2, P4_GLU = 3, P4_ACT = 4 };   // GLU, ACT: bf16 out, activation KIND
 typedef __attribute__((ext_vector_type(2))) uint32_t p4_u32x2;
 
 template <int N>
@@ -43,6 +44,20 @@ __device__ __forceinline__ void p4_sync() {
   asm volatile("" ::: "memory");
 }
 __device__ __forceinline__ float p4_silu(float g) { return g / (1.f + __expf(-g)); }
+// Activations of the epilogues (kinds as in stream32.hip), on the hardware's exponential and reciprocal: 2^-21 relative, the
+// result is rounded to bf16.  The kind is a template argument: 128 unrolled elements per lane with every kind's branches
+// took 775 us where the product takes 64.
+__device__ __forceinline__ float p4_sigmoid(float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
+template <int KIND>
+__device__ __forceinline__ float p4_pair(float g, float u, float limit, float alpha) {
+  if constexpr (KIND == 0) return g * p4_sigmoid(1.5957691216057308f * (g + 0.044715f * g * g * g)) * u;
+  if constexpr (KIND == 5) return fmaxf(g, 0.f) * u;
+  if (limit > 0.f) {
+    g = fminf(g, limit);
+    u = fminf(fmaxf(u, -limit), limit);
+  }
+  return g * p4_sigmoid(alpha * g) * (u + 1.f);
+}
 }  // namespace
 
 struct P4Args {
@@ -52,14 +67,26 @@ struct P4Args {
   const uint8_t* x;      // [M][K] bf16
   const uint8_t* W;      // [rows][K] bf16
   uint32_t kbytes;       // bytes per row of x and W
+  uint32_t xbytes;       // grouped form: bytes per row of x
   int M, N_out, half_rows, wrows, K;
   int m_tiles, n_tiles, ks, splits, group_m, nwg;
   float eps;
+  float limit, alpha;    // P4_GLU: of the gated kind
+  const bf16_t* bias;    // P4_GLU, optional: [gate; up] biases
+  // grouped form: group g's rows are [seg[g], seg[g + 1]) of a compact row space (row r of x: a_rows[r], or r) and its
+  // weights W + g wstride bytes; m_tiles bounds the groups' row tiles.  8 experts, 3068 rows, K = 2048: gate / up with its
+  // activation (N = 2 x 2048) 94 us, down (N = 2048) 47 us; 140 and 10 us, and 78 us on the 64-row tiles of stream32.hip
+  const int* seg;
+  const int* a_rows;
+  long long wstride;
+  int groups;
 };
 
-template <int FP, int FQ, int EPI, bool RMS, bool K64 = false>
+template <int FP, int FQ, int EPI, bool RMS, bool K64 = false, bool GRP = false, int KIND = -1>
 __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
   constexpr int BP = 32 * FP, BQ = 32 * FQ;          // weight rows, tokens per tile (2 x 2 waves)
+  constexpr bool PAIR = EPI == P4_SWIGLU || EPI == P4_GLU;   // gate and up rows of one feature in one wave
+  static_assert(!GRP || (!RMS && !K64), "the grouped form has no prologue and 32-deep stages");
   constexpr int ROWS = BP + BQ;
   constexpr int SUB = ROWS * 64;                     // one 32-deep k-step of both operands
   constexpr int G = ROWS / 64;                       // 16-byte DMA instructions per thread per k-step
@@ -78,16 +105,42 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
   const int li = lane & 15, g = lane >> 4;
 
   // ---- block -> (tile, k-slice)
-  const int bid = blockIdx.x, q8 = a.nwg >> 3, r8 = a.nwg & 7, xcd = bid & 7, loc = bid >> 3;
+  int nwg = a.nwg, m_tiles = a.m_tiles;
+  if constexpr (GRP) {     // the launch covers an upper bound: spread the tiles there are over the XCDs
+    m_tiles = 0;
+    for (int e = 0; e < a.groups; ++e) m_tiles += (a.seg[e + 1] - a.seg[e] + BQ - 1) / BQ;
+    nwg = m_tiles * a.n_tiles;
+    if ((int)blockIdx.x >= nwg) return;
+  }
+  const int bid = blockIdx.x, q8 = nwg >> 3, r8 = nwg & 7, xcd = bid & 7, loc = bid >> 3;
   const int lid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + loc;
   const int tile = lid / a.splits, slice = lid - tile * a.splits;
   int mt, nt;
   {
-    const int per = a.group_m * a.n_tiles, gi = tile / per, m0 = gi * a.group_m;
-    const int gm = min(a.m_tiles - m0, a.group_m), in = tile - gi * per;
-    mt = m0 + in % gm;
+    const int per = a.group_m * a.n_tiles, gi = tile / per, mg = gi * a.group_m;
+    const int gm = min(m_tiles - mg, a.group_m), in = tile - gi * per;
+    mt = mg + in % gm;
     nt = in / gm;
   }
+  // tokens of the tile: rows [m0, m_end) of the compact row space
+  const uint8_t* Wb = a.W;
+  int m0 = mt * BQ, m_end = a.M;
+  if constexpr (GRP) {
+    int gi = 0, left = mt;                           // mt < m_tiles: a group is found
+    for (;; ++gi) {
+      const int nt_g = (a.seg[gi + 1] - a.seg[gi] + BQ - 1) / BQ;
+      if (left < nt_g) break;
+      left -= nt_g;
+    }
+    m0 = a.seg[gi] + left * BQ;
+    m_end = a.seg[gi + 1];
+    Wb += (long long)gi * a.wstride;
+  }
+  auto xrow = [&](int r) -> uint32_t {               // row r of the tile, past the end its last one
+    const int m = min(m0 + r, m_end - 1);
+    if constexpr (GRP) return (uint32_t)(a.a_rows != nullptr ? a.a_rows[m] : m);
+    return (uint32_t)m;
+  };
   const int ks0 = 2 * (int)((long long)slice * (a.ks / 2) / a.splits);
   const int n = 2 * (int)((long long)(slice + 1) * (a.ks / 2) / a.splits) - ks0;   // even, >= 2
 
@@ -102,7 +155,7 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
     if (j < GW) {
       const int w = r / (BP / 2), q = r % (BP / 2);
       int row;
-      if constexpr (EPI == P4_SWIGLU) {   // wave rows: BP/4 gate rows then the matching BP/4 up rows
+      if constexpr (PAIR) {   // wave rows: BP/4 gate rows then the matching BP/4 up rows
         const int f = min(nt * (BP / 2) + w * (BP / 4) + (q % (BP / 4)), a.N_out - 1);
         row = q < BP / 4 ? f : a.half_rows + f;
       } else {
@@ -110,7 +163,7 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
       }
       off[j] = (uint32_t)row * a.kbytes + col;
     } else {
-      off[j] = (uint32_t)min(mt * BQ + (r - BP), a.M - 1) * a.kbytes + col;
+      off[j] = xrow(r - BP) * (GRP ? a.xbytes : a.kbytes) + col;
     }
   }
   auto issue = [&](int u) {   // k-step u of this slice into slot u % 4
@@ -118,7 +171,7 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
     const uint32_t kb = (uint32_t)u * 64u;
 #pragma unroll
     for (int j = 0; j < G; ++j)
-      __builtin_amdgcn_global_load_lds((j < GW ? a.W : a.x) + (off[j] + kb),
+      __builtin_amdgcn_global_load_lds((j < GW ? Wb : a.x) + (off[j] + kb),
                                        (__attribute__((address_space(3))) void*)(dst + j * 4096), 16, 0, 0);
   };
 
@@ -196,7 +249,7 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
 #pragma unroll
       for (int d = 0; d < G; ++d)
         if (k == d * MF / G)
-          __builtin_amdgcn_global_load_lds((d < GW ? a.W : a.x) + (off[d] + kb),
+          __builtin_amdgcn_global_load_lds((d < GW ? Wb : a.x) + (off[d] + kb),
                                            (__attribute__((address_space(3))) void*)(dst + d * 4096), 16, 0, 0);
       asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(Ac[i]), "v"(Bc[j]));
 #pragma unroll
@@ -247,7 +300,7 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
       if (j < GW2) {
         const int w = r / (BP / 2), q = r % (BP / 2);
         int row;
-        if constexpr (EPI == P4_SWIGLU) {
+        if constexpr (PAIR) {
           const int f = min(nt * (BP / 2) + w * (BP / 4) + (q % (BP / 4)), a.N_out - 1);
           row = q < BP / 4 ? f : a.half_rows + f;
         } else {
@@ -255,11 +308,11 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
         }
         off2[j] = (uint32_t)row * a.kbytes + col;
       } else {
-        off2[j] = (uint32_t)min(mt * BQ + (r - BP), a.M - 1) * a.kbytes + col;
+        off2[j] = xrow(r - BP) * a.kbytes + col;
       }
     }
     auto dma2 = [&](int u, int d) {   // instruction d of stage u
-      __builtin_amdgcn_global_load_lds((d < GW2 ? a.W : a.x) + (off2[d] + (uint32_t)u * 128u),
+      __builtin_amdgcn_global_load_lds((d < GW2 ? Wb : a.x) + (off2[d] + (uint32_t)u * 128u),
                                        (__attribute__((address_space(3))) void*)(lds + (u & 1) * SUB2 + wid * 1024 +
                                                                                  d * 4096),
                                        16, 0, 0);
@@ -386,7 +439,7 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
 #pragma unroll
       for (int i = 0; i < FP; ++i) {
         int r0;
-        if constexpr (EPI == P4_SWIGLU) {
+        if constexpr (PAIR) {
           const int hf = i / (FP / 2), f = nt * (BP / 2) + wr * (BP / 4) + (i % (FP / 2)) * 16 + 4 * g;
           if (f >= a.N_out) continue;
           r0 = hf ? a.half_rows + f : f;
@@ -406,18 +459,29 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
 #pragma unroll
   for (int j = 0; j < FQ; ++j) {
     const int mloc = wc * (BQ / 2) + j * 16 + li;
-    const int m = mt * BQ + mloc;
-    if (m >= a.M) continue;
+    const int m = m0 + mloc;
+    if (m >= m_end) continue;
     float sx = 1.f;
     if constexpr (RMS) sx = rsqrtf(rss[mloc] / (float)a.K + a.eps);
-    if constexpr (EPI == P4_SWIGLU) {
+    if constexpr (PAIR) {
 #pragma unroll
       for (int i = 0; i < FP / 2; ++i) {
         const int f0 = nt * (BP / 2) + wr * (BP / 4) + i * 16 + 4 * g;
         if (f0 >= a.N_out) continue;
         float v[4];
+        if constexpr (EPI == P4_GLU) {
+          f32x4 bg = {0.f, 0.f, 0.f, 0.f}, bu = bg;
+          if (a.bias != nullptr) {
+            bg = ldf4(a.bias + f0);
+            bu = ldf4(a.bias + a.half_rows + f0);
+          }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = p4_silu(acc[i][j][e] * sx) * (acc[FP / 2 + i][j][e] * sx);
+          for (int e = 0; e < 4; ++e)
+            v[e] = p4_pair<KIND>(acc[i][j][e] + bg[e], acc[FP / 2 + i][j][e] + bu[e], a.limit, a.alpha);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = p4_silu(acc[i][j][e] * sx) * (acc[FP / 2 + i][j][e] * sx);
+        }
         const p4_u32x2 o = {pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
         *reinterpret_cast<p4_u32x2*>(reinterpret_cast<bf16_t*>(a.out) + (size_t)m * a.N_out + f0) = o;
       }
@@ -429,6 +493,10 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] * sx;
+        if constexpr (EPI == P4_ACT) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = v[e] > 0.f ? v[e] * v[e] : 0.f;      // kind 7
+        }
         if constexpr (EPI == P4_F32) {
           *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + (size_t)m * a.N_out + n0) =
               f32x4{v[0], v[1], v[2], v[3]};
@@ -620,6 +688,49 @@ extern "C" int k8s_pgemm_reduce(void* out, const void* res, const float* slab, i
   return -2;
 }
 
+// The forms with an activation (gated kinds 0, 1, 5; elementwise 7): configurations 1 - 4; the grouped ones: 1 and 3.
+template <int C, int EPI, bool GRP, int KIND>
+int p4_act_launch(const P4Args& a, hipStream_t s) {
+  hipLaunchKernelGGL((pgemm4_kernel<kP4Cfgs[C].fp, kP4Cfgs[C].fq, EPI, false, kP4Cfgs[C].k64, GRP, KIND>), dim3(a.nwg),
+                     dim3(256), 0, s, a);
+  return (int)hipGetLastError();
+}
+template <int C, bool GRP>
+int p4_act_kind(const P4Args& a, int kind, hipStream_t s) {
+  switch (kind) {
+    case 0: return p4_act_launch<C, P4_GLU, GRP, 0>(a, s);
+    case 1: return p4_act_launch<C, P4_GLU, GRP, 1>(a, s);
+    case 5: return p4_act_launch<C, P4_GLU, GRP, 5>(a, s);
+    case 7:
+      if constexpr (!GRP) return p4_act_launch<C, P4_ACT, false, 7>(a, s);
+      break;
+    case -1:
+      if constexpr (GRP) return p4_act_launch<C, P4_BF16, true, -1>(a, s);
+      break;
+  }
+  return -1;
+}
+P4Args p4_args(void* out, const void* x, const void* W, int M, int N_out, int K, bool pair, int cfg, int group_m) {
+  const int bp = 32 * kP4Cfgs[cfg].fp, bq = 32 * kP4Cfgs[cfg].fq, feat = pair ? bp / 2 : bp;
+  P4Args a = {};
+  a.out = out;
+  a.x = static_cast<const uint8_t*>(x);
+  a.W = static_cast<const uint8_t*>(W);
+  a.kbytes = (uint32_t)K * 2u;
+  a.M = M;
+  a.N_out = N_out;
+  a.half_rows = pair ? N_out : 0;
+  a.wrows = pair ? 2 * N_out : N_out;
+  a.K = K;
+  a.m_tiles = (M + bq - 1) / bq;
+  a.n_tiles = (N_out + feat - 1) / feat;
+  a.ks = K / 32;
+  a.splits = 1;
+  a.group_m = group_m > 0 ? group_m : 1;
+  a.nwg = a.m_tiles * a.n_tiles;
+  return a;
+}
+
 extern "C" int k8s_pgemm4_num_configs() { return kP4NumCfgs; }
 
 extern "C" int k8s_pgemm4_config(int cfg, int* bp, int* bq, int* lds_bytes) {
@@ -681,4 +792,55 @@ extern "C" int k8s_pgemm4(void* out, float* slab, const void* x, const void* W, 
   if (rc != 0 || splits == 1) return rc;
   return k8s_pgemm_reduce(out, res, slab, splits, M, N_out, K, epi, rms, eps, nullptr, nullptr, nullptr, nullptr,
                           stream);
+}
+
+// act(x W^T (+ bias)) in bf16: `kind` gated (0, 1, 5; W = [gate; up] rows, bias [2 N_out] optional) or 7 (elementwise).
+extern "C" int k8s_pgemm4_act(void* out, const void* x, const void* W, int M, int N_out, int K, int cfg, int group_m, int kind,
+                              float limit, float alpha, const void* bias, hipStream_t stream) {
+  const bool pair = kind != 7;
+  int nwg;
+  long long nsl;
+  if ((kind != 0 && kind != 1 && kind != 5 && kind != 7) || (!pair && bias != nullptr)) return -1;
+  if (k8s_pgemm4_plan(M, N_out, K, pair ? P4_SWIGLU : P4_BF16, cfg, 1, &nwg, &nsl) != 0) return -1;
+  const long long kbytes = (long long)K * 2;
+  if ((pair ? 2LL : 1LL) * N_out * kbytes >= (1LL << 32) || (long long)M * kbytes >= (1LL << 32)) return -5;
+  if (bias != nullptr && ((uintptr_t)bias & 7)) return -1;
+  P4Args a = p4_args(out, x, W, M, N_out, K, pair, cfg, group_m);
+  a.limit = limit;
+  a.alpha = alpha;
+  a.bias = static_cast<const bf16_t*>(bias);
+  switch (cfg) {
+    case 1: return p4_act_kind<1, false>(a, kind, stream);
+    case 2: return p4_act_kind<2, false>(a, kind, stream);
+    case 3: return p4_act_kind<3, false>(a, kind, stream);
+    case 4: return p4_act_kind<4, false>(a, kind, stream);
+  }
+  return -4;
+}
+
+// Grouped product over at most `rows` compact rows (x: M rows in memory, ldx elements apart): kind < 0 plain, or a gated kind
+// with [groups][2 N_out][K] weights.
+extern "C" int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M, int rows, int N_out, int K, int groups,
+                                  const int* seg, const int* a_rows, long ldx, int cfg, int group_m, int kind, float limit,
+                                  float alpha, hipStream_t stream) {
+  const bool pair = kind >= 0;
+  if (kind < -1 || (pair && kind > 1 && kind != 5)) return -1;
+  if (rows <= 0) return 0;
+  if (M <= 0 || N_out <= 0 || N_out % 4 || K <= 0 || K % 64 || groups <= 0 || seg == nullptr || (cfg != 1 && cfg != 3)) return -1;
+  if (ldx < K || ldx % 8 || (((uintptr_t)x | (uintptr_t)W) & 15) || ((uintptr_t)out & 7)) return -1;
+  const long long kbytes = (long long)K * 2, wrows = (pair ? 2LL : 1LL) * N_out;
+  if (wrows * kbytes >= (1LL << 32) || (long long)M * ldx * 2 >= (1LL << 32)) return -5;   // 32-bit DMA offsets
+  P4Args a = p4_args(out, x, W, rows, N_out, K, pair, cfg, group_m);
+  const int bq = 32 * kP4Cfgs[cfg].fq;
+  a.m_tiles = rows / bq + groups;        // whole tiles, and a partial one per group
+  if ((long long)a.m_tiles * a.n_tiles > (1LL << 30)) return -1;
+  a.nwg = a.m_tiles * a.n_tiles;
+  a.xbytes = (uint32_t)(ldx * 2);
+  a.seg = seg;
+  a.a_rows = a_rows;
+  a.wstride = wrows * kbytes;
+  a.groups = groups;
+  a.limit = limit;
+  a.alpha = alpha;
+  return cfg == 1 ? p4_act_kind<1, true>(a, kind, stream) : p4_act_kind<3, true>(a, kind, stream);
 }

@@ -520,15 +520,16 @@ class FavizenModel(StreamModel):
 
     @staticmethod
     def _glu(w: _Glu, h) -> torch.Tensor:
-        return sm.linear(sm.act(sm.linear(h, w.w_gu), sm.ACT_SWISH_CLAMP, w.limit, SWISH_ALPHA, bias=w.b_gu), w.w_down)
+        return sm.linear(sm.linear_act(h, w.w_gu, sm.ACT_SWISH_CLAMP, w.limit, SWISH_ALPHA, bias=w.b_gu), w.w_down)
 
     def _moe(self, w: _Moe, h, sg, b) -> torch.Tensor:
         f = w.cfg
         P = h.shape[0] * f.top
         key, l = w.route
         sorted_tok, pos, seg, tiles = b["routes"][key][l]
-        gu = sm.gemm(h, w.experts.w_gu, a_rows=sorted_tok, tiles=tiles, rows=P, seg=seg)
-        d = sm.gemm(sm.act(gu, sm.ACT_SWISH_CLAMP, f.limit, SWISH_ALPHA), w.experts.w_down, tiles=tiles, rows=P, seg=seg)
+        g = sm.gemm_act(h, w.experts.w_gu, sm.ACT_SWISH_CLAMP, f.limit, SWISH_ALPHA, a_rows=sorted_tok, tiles=tiles, rows=P,
+                        seg=seg)
+        d = sm.gemm(g, w.experts.w_down, tiles=tiles, rows=P, seg=seg)
         shared = self._glu(w.shared, h) if w.shared is not None else None
         return sm.moe_combine(d, pos, None, shared, sg, 0 if sg is not None else -1, top=f.top, scale=1.0 / f.top)
 

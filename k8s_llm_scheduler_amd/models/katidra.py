@@ -410,7 +410,7 @@ class KatidraModel(StreamModel):
             run = self._lightning if isinstance(w.mixer, _Lightning) else self._latent
             h = sm.branchnorm(x, run(w.mixer, L.cache, h, b), w.n1, c.rms_eps, out_dtype=dt)
             if w.w_up is not None:
-                f = sm.linear(sm.act(sm.linear(h, w.w_up), sm.ACT_RELU2), w.w_down)
+                f = sm.linear(sm.linear_act(h, w.w_up, sm.ACT_RELU2), w.w_down)
                 h = sm.branchnorm(x, f, w.n2, c.rms_eps, out_dtype=dt)
             if after is not None:
                 after.append(x.clone())

@@ -599,7 +599,7 @@ class NukizenModel(StreamModel):
         for L in self.layers:
             h = sm.resnorm(x, L.n1, c.rms_eps, branch=mix, branch2=ff, out_dtype=dt)
             mix = self._mixer(L, h, b)
-            ff = sm.linear(sm.act(sm.linear(h, L.w_gu), sm.ACT_RELU), L.w_down) if L.w_gu is not None else None
+            ff = sm.linear(sm.linear_act(h, L.w_gu, sm.ACT_RELU), L.w_down) if L.w_gu is not None else None
             if after is not None:
                 sm.resnorm(x, None, c.rms_eps, branch=mix, branch2=ff, out_dtype=dt)
                 mix = ff = None

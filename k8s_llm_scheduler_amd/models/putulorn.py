@@ -445,7 +445,7 @@ class PutulornModel(StreamModel):
             r, k, v, g = (sm.linear(mix[i], w.w_rkvg[i]) for i in range(4))
         else:
             r, k, v, g = sm.gemm(mix[:4], w.w_rkvg).unbind(0)
-        lo = sm.act(sm.linear(mix[4], w.w1), sm.ACT_TANH)
+        lo = sm.linear_act(mix[4], w.w1, sm.ACT_TANH)
         z = sm.linear(lo, w.w2, out_dtype=torch.float32)                  # decay logits stay fp32
         y = sm.wkv_scan(r, k, v, g, z, w.w0, w.u, w.lnw, S, b["cu_q"], b["seq_slots"], b["positions"], m.heads, m.dim,
                         self.cfg.rms_eps)
@@ -466,17 +466,18 @@ class PutulornModel(StreamModel):
     def _mlp(self, w: _Mlp, h) -> torch.Tensor:
         f = w.cfg
         if f.kind == "dense":
-            return sm.linear(sm.act(sm.linear(h, w.wgu), sm.ACT_GELU_TANH), w.down)
+            return sm.linear(sm.linear_act(h, w.wgu, sm.ACT_GELU_TANH), w.down)
         T = h.shape[0]
         logits = sm.linear(h, w.router, out_dtype=torch.float32)          # router (and shared gate) in fp32
         idx, wts = sm.moe_route(logits, f.experts, f.top, f.router_scale)
         sorted_tok, pos, seg, tiles = sm.moe_align(idx, f.experts)
         P = T * f.top
-        gu = sm.gemm(h, w.wgu, a_rows=sorted_tok, tiles=tiles, rows=P, seg=seg)          # [P, 2 F]
-        D = sm.gemm(sm.act(gu, sm.ACT_SWISH_CLAMP, f.limit, SWISH_ALPHA), w.down, tiles=tiles, rows=P, seg=seg)
+        g = sm.gemm_act(h, w.wgu, sm.ACT_SWISH_CLAMP, f.limit, SWISH_ALPHA, a_rows=sorted_tok, tiles=tiles, rows=P,
+                        seg=seg)                                          # [P, F]
+        D = sm.gemm(g, w.down, tiles=tiles, rows=P, seg=seg)
         shared = None
         if w.s_wgu is not None:
-            shared = sm.linear(sm.act(sm.linear(h, w.s_wgu), sm.ACT_SWISH_CLAMP, f.shared_limit, SWISH_ALPHA), w.s_down)
+            shared = sm.linear(sm.linear_act(h, w.s_wgu, sm.ACT_SWISH_CLAMP, f.shared_limit, SWISH_ALPHA), w.s_down)
         return sm.moe_combine(D, pos, wts, shared, logits, w.sg_col)
 
     def _forward(self, ids, b, rows) -> torch.Tensor:

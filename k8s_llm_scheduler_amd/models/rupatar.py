@@ -468,7 +468,7 @@ class RupatarModel(StreamModel):
         d = sm.gemm(a, w.down, tiles=tiles, rows=P, seg=seg)
         shared = None
         if w.s_up is not None:
-            shared = sm.linear(sm.act(sm.linear(h, w.s_up), sm.ACT_GELU_ERF), w.s_down)
+            shared = sm.linear(sm.linear_act(h, w.s_up, sm.ACT_GELU_ERF), w.s_down)
         return sm.moe_combine(d, pos, None, shared, None, -1, top=f.top)
 
     def _blocks(self, ids, b, after=None):

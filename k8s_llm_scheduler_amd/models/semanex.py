@@ -530,7 +530,7 @@ class SemanexModel(StreamModel):
                                  branch2=self._ssd(w.right, h, b), c1=w.cfg.left_scale, c2=w.cfg.right_scale,
                                  out_dtype=dt)
             if L.post2:
-                f = sm.linear(sm.act(sm.linear(h2, L.w_up), sm.ACT_GELU_ERF), L.w_down) if L.w_up is not None else None
+                f = sm.linear(sm.linear_act(h2, L.w_up, sm.ACT_GELU_ERF), L.w_down) if L.w_up is not None else None
                 sm.postnorm(x, f, c.alpha, L.gain2, c.rms_eps)
             if after is not None:
                 after.append(x.clone())

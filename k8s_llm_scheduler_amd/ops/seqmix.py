@@ -10,6 +10,7 @@ attention scores) is fp32 in both.
 
 from __future__ import annotations
 
+import math
 import os
 from typing import Optional
 
@@ -278,6 +279,8 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out_dtype=None, *, a_rows: Optional[t
             raise ValueError("gemm: k mismatch")
         if not _gpu(a, w):
             return ref.gemm_any(a, w, out_dtype, a_rows, tiles, seg)
+        if out_dtype == BF16 and _grouped_big(a, w, seg, rows, N):
+            return _pgemm4_grouped(a, w, a_rows, rows, seg, N)
         out = torch.empty(rows, N, dtype=out_dtype, device=a.device)
         _native().gemm_any(out.data_ptr(), a.data_ptr(), _p(w), rows, N, K, a.stride(0), K, N, 1, 0, N * K, 0,
                            _p(a_rows, I32, "a_rows"), _p(tiles, I32, "tiles"), tiles.shape[0], _f32(a.dtype),
@@ -307,6 +310,78 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out_dtype=None, *, a_rows: Optional[t
     _native().gemm_any(out.data_ptr(), a.data_ptr(), w.data_ptr(), M, N, K, a.stride(1), w.stride(1), out.stride(1), G,
                        a.stride(0), w.stride(0), out.stride(0), 0, 0, 0, _f32(a.dtype), _f32(out_dtype), -1)
     return out
+
+
+# Grouped bf16 products of at least GROUP_BIG_MIN rows per group on average (whole rows of at least 64 elements) run on the
+# big-tile kernel (pgemm4.hip, 128 tokens per tile).  8 groups, N = K = 2048, 16 / 32 / 96 / 192 / 512 rows per group: 27 / 27
+# / 29 / 30 / 64 us, on the 64-row tiles of stream32.hip 22 / 29 / 44 / 50 / 87 us; gate / up with the activation in its
+# epilogue (N = 2 x 2048) 38 / 39 / 41 / 55 / 117 us, 47 / 63 / 62 / 85 / 173 us as two launches.  Fewer rows stream the
+# weights past the LDS (gemm_group_kernel).
+GROUP_BIG_MIN = 16
+GROUP_BIG_MAX_GROUPS = 64        # every workgroup walks the groups' offsets
+
+
+def _grouped_big(a: torch.Tensor, w: torch.Tensor, seg: Optional[torch.Tensor], rows: int, N: int) -> bool:
+    from . import LEAN
+
+    E, _, K = w.shape
+    return (not LEAN and FAST_GEMM and a.dtype == BF16 and seg is not None and seg.is_cuda and E <= GROUP_BIG_MAX_GROUPS
+            and rows >= GROUP_BIG_MIN * E and K % 64 == 0 and N % 4 == 0 and N >= 128 and a.stride(0) % 8 == 0
+            and a.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0
+            and w.shape[1] * K * 2 < 1 << 32 and a.shape[0] * a.stride(0) * 2 < 1 << 32)
+
+
+def _grouped_cfg(rows: int, E: int, N: int, K: int, pair: bool) -> int:
+    """Configuration of the grouped big-tile product: 256 (1) or 128 (3) weight rows per tile by the time its rounds of tiles
+    over the CUs take (us, fitted to the products above and to N = 3584 / 4096, K = 3584 / 4096), groups of about equal
+    size drawn at random."""
+    r = rows / E
+    tiles = E * sum(0.5 + 0.5 * math.erf((r - 128 * k) / math.sqrt(2.0 * max(r, 1.0))) for k in range(1, int(r / 128) + 2)) + E
+    n, kt = (2 * N if pair else N), K / 64
+    big = 10.0 + math.ceil(tiles * -(-n // 256) / 256) * (kt + (12.0 if pair else 0.0))
+    small = 20.0 + math.ceil(tiles * -(-n // 128) / 256) * 0.56 * kt
+    return 1 if big < small else 3
+
+
+def _pgemm4_grouped(a, w, a_rows, rows: int, seg, N: int, kind: int = -1, limit: float = 0.0, alpha: float = 1.0):
+    E, _, K = w.shape
+    out = torch.empty(rows, N, dtype=BF16, device=a.device)
+    _native().pgemm4_grouped(out.data_ptr(), a.data_ptr(), w.data_ptr(), a.shape[0], rows, N, K, E, _p(seg, I32, "seg"),
+                             _p(a_rows, I32, "a_rows"), a.stride(0), _grouped_cfg(rows, E, N, K, kind >= 0), 4, kind,
+                             float(limit), float(alpha), -1)
+    return out
+
+
+def gemm_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, alpha: float = 1.0, *,
+             a_rows: Optional[torch.Tensor] = None, tiles: Optional[torch.Tensor] = None, rows: int = 0,
+             seg: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """act(gemm(a, w)) of a grouped product and a gated kind, w [E, 2 N, K] = gate | up: in the product's epilogue where
+    it runs on the big-tile kernel (the sums are then not rounded ahead of the activation)."""
+    N = w.shape[1] // 2
+    if a.shape[-1] == w.shape[-1] and w.shape[1] % 2 == 0 and a.dtype == w.dtype and _gpu(a, w) and \
+            _grouped_big(a, w, seg, rows, N):
+        return _pgemm4_grouped(a, w, a_rows, rows, seg, N, kind, limit, alpha)
+    return act(gemm(a, w, a_rows=a_rows, tiles=tiles, rows=rows, seg=seg), kind, limit, alpha)
+
+
+def linear_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, alpha: float = 1.0, *,
+               bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """act(linear(a, w), kind, bias=bias): in the product's epilogue where its plan is an unsplit big-tile one, which saves a
+    pass over the product (2048 x 2 x 8192, gated: 22 us; 2048 x 8192 elementwise: 15 us) and its rounding."""
+    pair = kind in (ACT_GELU_TANH, ACT_SWISH_CLAMP, ACT_RELU)
+    if (pair or kind == ACT_RELU2) and FAST_GEMM and _gpu(a, w, bias) and _route_fast(a, w, BF16) and a.dtype == BF16 and (not pair or w.shape[0] % 8 == 0):
+        from . import EPI_BF16, gemm_route
+
+        M, K = a.shape
+        kern, plan = gemm_route(M, w.shape[0], K, EPI_BF16, False) if M >= 129 else ("", None)
+        if kern == "pgemm4" and plan[1] == 1 and plan[0] in (1, 2, 3, 4) and a.data_ptr() % 16 == 0 and \
+                (bias is None or (pair and bias.dtype == BF16 and bias.numel() == w.shape[0] and bias.data_ptr() % 8 == 0)):
+            N = w.shape[0] // 2 if pair else w.shape[0]
+            out = torch.empty(M, N, dtype=BF16, device=a.device)
+            _native().pgemm4_act(out.data_ptr(), _p(a), _p(w), M, N, K, plan[0], plan[2], kind, float(limit), float(alpha),
+                                 _p(bias), -1)
+            return out
+    return act(linear(a, w), kind, limit, alpha, bias=bias)
 
 
 # ----------------------------------------------------------------------------- recurrent mixer
@@ -472,7 +547,8 @@ def latent_expand(uk: torch.Tensor, uv: torch.Tensor, H: int, R: int) -> Optiona
 
 
 def _latent_keys(b: dict, window: int, block_size: int, cap: int) -> tuple:
-    """(cache slots of the rows the batch's tokens see, first row of every sequence, row tiles): made once per batch."""
+    """(cache slots of the rows the batch's tokens see, first row of every sequence, row tiles, (0, rows)): made once per
+    batch."""
     made = b.setdefault("latent_keys", {})
     if window not in made:
         dev, nseq = b["positions"].device, b["cu_q"].shape[0] - 1
@@ -480,10 +556,11 @@ def _latent_keys(b: dict, window: int, block_size: int, cap: int) -> tuple:
         rows = torch.empty(cap, dtype=I32, device=dev)
         kbase = torch.empty(nseq, dtype=I32, device=dev)
         tiles = torch.empty(ntiles, 3, dtype=I32, device=dev)
-        _native().latent_keys(rows.data_ptr(), kbase.data_ptr(), tiles.data_ptr(), _p(b["cu_q"], I32),
+        seg = torch.empty(2, dtype=I32, device=dev)
+        _native().latent_keys(rows.data_ptr(), kbase.data_ptr(), tiles.data_ptr(), seg.data_ptr(), _p(b["cu_q"], I32),
                               _p(b["positions"], I32), _p(b["block_tables"], I32), b["block_tables"].shape[1], nseq, window,
                               block_size, cap, ntiles, -1)
-        made[window] = (rows, kbase, tiles)
+        made[window] = (rows, kbase, tiles, seg)
     return made[window]
 
 
@@ -505,11 +582,12 @@ def latent_mix(q: torch.Tensor, cache: torch.Tensor, uk_t: torch.Tensor, uv: tor
     cap = min(T + nseq * (window - 1), nseq * ctx) if window else nseq * ctx
     if (ukv is not None and _gpu(q, cache) and max_qlen > 0 and 0 < LATENT_EXPAND_MIN * nseq <= T and cap < 1 << 24
             and cap * H * (Dn + V) * q.element_size() <= LATENT_EXPAND_BYTES and _native().latent_prompt_ok(C, R, Dn, V)):
-        rows, kbase, tiles = _latent_keys(b, int(window), block_size, cap)
-        kv = torch.empty(cap, H * (Dn + V), dtype=dt, device=q.device)
+        rows, kbase, tiles, seg = _latent_keys(b, int(window), block_size, cap)
         nat = _native()
-        nat.gemm_any(kv.data_ptr(), _p(cache, dt, "cache"), _p(ukv, dt, "ukv"), cap, H * (Dn + V), C, C + R, C, H * (Dn + V),
-                     1, 0, 0, 0, rows.data_ptr(), tiles.data_ptr(), tiles.shape[0], _f32(dt), _f32(dt), -1)
+        if cache.shape[1] != C + R or ukv.shape != (H * (Dn + V), C):
+            raise ValueError("latent_mix: the cache holds C + R columns, ukv is [H (Dn + V), C]")
+        _p(cache, dt, "cache"), _p(ukv, dt, "ukv")
+        kv = gemm(cache[:, :C], ukv.unsqueeze(0), a_rows=rows, tiles=tiles, rows=cap, seg=seg)
         out = torch.empty(T, H * V, dtype=dt, device=q.device)
         nat.latent_prompt(out.data_ptr(), kv.data_ptr(), rows.data_ptr(), kbase.data_ptr(), _p(q), cache.data_ptr(), C, R, Dn,
                           V, _p(b["cu_q"], I32), _p(b["positions"], I32), nseq, int(max_qlen), H, int(window), float(scale),

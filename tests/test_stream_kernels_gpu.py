@@ -181,3 +181,75 @@ def test_row_norm_and_token_shift_widths(dt, tol, W):
     live = pos >= 0
     assert (got[:, live].float() - want[:, live].float()).abs().max() <= tol * want.float().abs().max()
     assert (got[:, ~live] == 0).all() and torch.equal(sg.cpu(), sc)
+
+
+# ----------------------------------------------------------------------------- grouped products on big tiles, activations in the epilogue
+KINDS = [sm.ACT_GELU_TANH, sm.ACT_SWISH_CLAMP, sm.ACT_RELU]
+ELEMENTWISE = [sm.ACT_TANH, sm.ACT_SILU, sm.ACT_GELU_ERF, sm.ACT_RELU2, sm.ACT_SOFTCAP]
+
+
+def act64(z, kind, limit, alpha):
+    if kind in KINDS:
+        g, u = z.chunk(2, -1)
+        if kind == sm.ACT_GELU_TANH:
+            return torch.nn.functional.gelu(g, approximate="tanh") * u
+        if kind == sm.ACT_RELU:
+            return g.clamp(min=0) * u
+        if limit:
+            g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+        return g * torch.sigmoid(alpha * g) * (u + 1.0)
+    return {sm.ACT_TANH: torch.tanh, sm.ACT_SILU: torch.nn.functional.silu, sm.ACT_GELU_ERF: torch.nn.functional.gelu,
+            sm.ACT_RELU2: lambda v: v.clamp(min=0) ** 2, sm.ACT_SOFTCAP: lambda v: limit * torch.tanh(v / limit)}[kind](z)
+
+
+@pytest.mark.parametrize("sizes", [(1, 127, 0, 128, 129), (40, 40, 40), (0, 0, 300), (257,), tuple([17] * 63 + [1])])
+@pytest.mark.parametrize("N,K", [(128, 64), (392, 192), (1024, 256)])
+@pytest.mark.parametrize("kind", [None] + KINDS)
+def test_grouped_big_tiles(sizes, N, K, kind):
+    """Groups at the edges of the 128-token tile, empty ones, more than fit a wave; gathered rows with a row stride."""
+    g = torch.Generator().manual_seed(sum(sizes) + N + K)
+    E, P = len(sizes), sum(sizes)
+    seg = torch.tensor((0,) + sizes).cumsum(0).to(torch.int32)
+    if P < sm.GROUP_BIG_MIN * E:
+        pytest.skip("too few rows for this path")
+    x = torch.randn(90, K + 8, generator=g).to(torch.bfloat16).to(DEV)[:, :K]
+    rows = torch.randint(0, 90, (P,), generator=g).to(torch.int32).to(DEV)
+    w = (torch.randn(E, N * (1 if kind is None else 2), K, generator=g) * 2 / K ** 0.5).to(torch.bfloat16).to(DEV)
+    tiles = torch.full((1, 3), -1, dtype=torch.int32, device=DEV)      # the big tiles come from seg
+    assert sm._grouped_big(x, w, seg.to(DEV), P, N)
+    kw = dict(a_rows=rows, tiles=tiles, rows=P, seg=seg.to(DEV))
+    for cfg in (1, 3):
+        sm_cfg, sm._grouped_cfg = sm._grouped_cfg, lambda *a: cfg
+        try:
+            got = sm.gemm(x, w, **kw) if kind is None else sm.gemm_act(x, w, kind, 1.5, 1.702, **kw)
+        finally:
+            sm._grouped_cfg = sm_cfg
+        for e in range(E):
+            r = slice(int(seg[e]), int(seg[e + 1]))
+            z = x[rows[r].long()].double() @ w[e].double().T
+            want = z if kind is None else act64(z, kind, 1.5, 1.702)
+            if want.numel():      # one rounding to bf16, and the fp32 sums'
+                assert ((got[r].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all(), (cfg, e)
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 1024, 512), (200, 520, 1024), (1031, 2048, 256), (2048, 2064, 320)])
+@pytest.mark.parametrize("kind", KINDS + ELEMENTWISE)
+@pytest.mark.parametrize("bias", [False, True])
+def test_linear_act(M, N, K, kind, bias):
+    """The activation in the epilogue, every tile configuration's edges, against 64 bits: one rounding."""
+    if bias and kind not in KINDS:
+        pytest.skip("elementwise kinds take no bias")
+    g = torch.Generator().manual_seed(M + N + K + kind)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(2 * N if kind in KINDS else N, K, generator=g) * 2 / K ** 0.5).to(torch.bfloat16).to(DEV)
+    b = torch.randn(2 * N, generator=g).to(torch.bfloat16).to(DEV) if bias else None
+    z = x.double() @ w.double().T + (b.double() if bias else 0.0)
+    want = act64(z, kind, 1.5, 1.702)
+    nat = sm._native()
+    for cfg in (1, 2, 3, 4) if kind in KINDS + [sm.ACT_RELU2] else ():
+        out = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=DEV)
+        nat.pgemm4_act(out.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K, cfg, 4, kind, 1.5, 1.702,
+                       b.data_ptr() if bias else 0, -1)
+        assert ((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all(), cfg
+    got = sm.linear_act(x, w, kind, 1.5, 1.702, bias=b)
+    assert ((got.double() - want).abs() <= 2.0 ** -6 * want.abs() + 4e-2).all()
