@@ -253,3 +253,40 @@ def test_linear_act(M, N, K, kind, bias):
         assert ((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all(), cfg
     got = sm.linear_act(x, w, kind, 1.5, 1.702, bias=b)
     assert ((got.double() - want).abs() <= 2.0 ** -6 * want.abs() + 4e-2).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16, 64), (16, 130, 128), (17, 100, 64), (64, 15, 1024), (65, 128, 2048), (200, 33, 320),
+                                   (2048, 128, 192)])
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
+def test_narrow_products(M, N, K, out):
+    """Few tiles: k shared by a workgroup's waves; rows and columns at the 16s and 64s, a row stride, a batch."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randn(2, M, K + 8, generator=g).to(torch.bfloat16).to(DEV)[:, :, 8:]
+    w = torch.randn(2, N, K, generator=g).to(torch.bfloat16).to(DEV)
+    bound = lambda a, w, y: sum_bound(a.cpu(), w.cpu()) + (2.0 ** -8 * y.abs().cpu() if out == torch.bfloat16 else 0.0)
+    got, exact = sm.gemm(a, w, out).cpu().double(), a.double() @ w.double().transpose(1, 2)
+    assert ((got - exact.cpu()).abs() <= bound(a, w, exact)).all()
+    one = sm.gemm(a[0], w[0], out).cpu().double()
+    assert ((one - exact[0].cpu()).abs() <= bound(a[0], w[0], exact[0])).all()
+
+
+def test_recurrence_prefix_over_many_chunks():
+    """More chunks than the prefix keeps in flight, head sizes that do not fill its workgroups, a resumed sequence beside a
+    new one: chunked against one workgroup per sequence."""
+    g = torch.Generator().manual_seed(5)
+    for H, D, lens, first in ((2, 64, (700, 129), (0, 33)), (1, 40, (1, 900), (7, 0))):
+        T = sum(lens)
+        r, k, v, gate = (torch.randn(T, H * D, generator=g).to(DEV) for _ in range(4))
+        z, w0, u, lnw = (torch.randn(T, H * D, generator=g).to(DEV), *(torch.randn(H * D, generator=g).to(DEV) for _ in range(3)))
+        st = torch.randn(2, H, D, D, generator=g).to(DEV)
+        cu = torch.tensor([0, lens[0], T], dtype=torch.int32, device=DEV)
+        pos = torch.cat([torch.arange(p, p + n) for p, n in zip(first, lens)]).to(torch.int32).to(DEV)
+        slots = torch.tensor([1, 0], dtype=torch.int32, device=DEV)
+        outs = []
+        for chunk in (0, 16, 64):
+            s = st.clone()
+            y = sm.wkv_scan(r, k, v, gate, z, w0, u, lnw, s, cu, slots, pos, H, D, 1e-6, chunk=chunk)
+            outs.append((y, s))
+        for y, s in outs[1:]:
+            assert (y - outs[0][0]).abs().max() <= 1e-4 * outs[0][0].abs().max()
+            assert (s - outs[0][1]).abs().max() <= 1e-5 * outs[0][1].abs().max()
