@@ -117,8 +117,10 @@ int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M, int rows,
                        hipStream_t stream);
 int k8s_pgemm4(void* out, float* slab, const void* x, const void* W, int M, int N_out, int K, int epi, int cfg,
                int splits, int group_m, const void* res, int rms, float eps, hipStream_t s);
-int k8s_embed_rows(float* out, const int* ids, const void* table, int T, int W, int vocab, float scale, int f32,
-                   hipStream_t s);
+int k8s_embed_rows(float* out, void* copy, const int* ids, const void* table, int T, int W, int vocab, float scale,
+                   int f32, hipStream_t s);
+int k8s_decode_meta(int* pos, int* slots, int* ar, const int* ctx, const int* block_tables, int max_blocks, int B, int bs,
+                    hipStream_t s);
 int k8s_resnorm(float* x, const void* branch, const void* branch2, float mult, const void* rowvec, const void* w,
                 float offset, float eps, void* out, int T, int W, int groups, int f32, hipStream_t s);
 int k8s_norm_mix(void* out, const void* a, long lda, const void* wa, const void* b, const void* wb, float eps, float ca,
@@ -490,9 +492,14 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
   });
 
   // fp32 residual stream, recurrent / latent mixers, mixture of experts (stream32.hip, mixers.hip, moe.hip)
-  m.def("embed_rows", [](uintptr_t out, uintptr_t ids, uintptr_t table, int T, int W, int vocab, float scale, int f32,
-                         int64_t s) {
-    check(k8s_embed_rows(P<float>(out), P<int>(ids), P(table), T, W, vocab, scale, f32, S(s)), "embed_rows");
+  m.def("embed_rows", [](uintptr_t out, uintptr_t copy, uintptr_t ids, uintptr_t table, int T, int W, int vocab,
+                         float scale, int f32, int64_t s) {
+    check(k8s_embed_rows(P<float>(out), P(copy), P<int>(ids), P(table), T, W, vocab, scale, f32, S(s)), "embed_rows");
+  });
+  m.def("decode_meta", [](uintptr_t pos, uintptr_t slots, uintptr_t ar, uintptr_t ctx, uintptr_t block_tables,
+                          int max_blocks, int B, int bs, int64_t s) {
+    check(k8s_decode_meta(P<int>(pos), P<int>(slots), P<int>(ar), P<int>(ctx), P<int>(block_tables), max_blocks, B, bs,
+                          S(s)), "decode_meta");
   });
   m.def("resnorm", [](uintptr_t x, uintptr_t branch, uintptr_t branch2, float mult, uintptr_t rowvec, uintptr_t w,
                       float offset, float eps, uintptr_t out, int T, int W, int groups, int f32, int64_t s) {

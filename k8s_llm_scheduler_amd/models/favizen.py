@@ -38,7 +38,7 @@ from ..ops import reference as ref
 from ..ops import seqmix as sm
 from ..parallel import TPGroup
 from . import stream
-from .stream import StreamModel
+from .stream import StreamModel, pick_rows
 
 ARCHITECTURE = "Favizen"
 MIXERS = ("attention", "attention_2")
@@ -561,7 +561,7 @@ class FavizenModel(StreamModel):
         c = self.cfg
         x, branch, w, bias = self._blocks(ids, b)
         # the logits' factor rides on the final norm
-        hf = sm.branchnorm(x.index_select(0, rows), branch.index_select(0, rows), w, c.rms_eps, out_dtype=self.dtype,
+        hf = sm.branchnorm(pick_rows(x, rows), pick_rows(branch, rows), w, c.rms_eps, out_dtype=self.dtype,
                            bias=bias, next_w=self.final_norm, gain=c.logit_scale)
         return sm.linear(hf, self.lm_head, out_dtype=F32).unsqueeze(0)     # [1, S, vocab]
 

@@ -34,7 +34,7 @@ from ..ops import reference as ref
 from ..ops import seqmix as sm
 from ..parallel import TPGroup
 from . import stream
-from .stream import StreamModel, stack_rows
+from .stream import StreamModel, pick_rows, stack_rows
 
 ARCHITECTURE = "Katidra"
 MIXERS = ("lightning", "latent_attention")
@@ -309,7 +309,7 @@ class KatidraModel(StreamModel):
     def _build_lightning(self, get, p: str, m: LightningConfig, where: str) -> _Lightning:
         if max(m.dim, m.vdim) > sm.gated_scan_max_dim():
             raise ValueError(f"{where}: head sizes {m.dim} x {m.vdim} exceed the kernels' {sm.gated_scan_max_dim()}")
-        w_in, cols = stack_rows(tuple((s, get(p + s).cpu()) for s in ("q", "k", "v", "g")))
+        w_in, cols = stack_rows(tuple((s, get(p + s)) for s in ("q", "k", "v", "g")))
         return _Lightning(m, self._t(w_in), cols, self._f(torch.tensor(m.decay, dtype=torch.float64)),
                           self._f(get(p + "norm")), self._t(get(p + "o")))
 
@@ -318,7 +318,7 @@ class KatidraModel(StreamModel):
         H, Dn, R, V, C = m.heads, m.dim, m.rot_dim, m.vdim, m.kv_rank
         if m.rot_dims % 2 or not 0 < m.rot_dims <= R:
             raise ValueError(f"{where}: rot.dims {m.rot_dims} must be even, positive and at most rot_dim {R}")
-        w_in, cols = stack_rows(tuple((s, get(p + s).cpu()) for s in ("dq", "dkv", "g")))
+        w_in, cols = stack_rows(tuple((s, get(p + s)) for s in ("dq", "dkv", "g")))
         return _Latent(m, t(w_in), cols, t(get(p + "dq.norm")), t(get(p + "uq")), t(get(p + "dkv.norm")),
                        t(get(p + "uk").view(H, Dn, C).transpose(1, 2)), t(get(p + "uv").view(H, V, C)), t(get(p + "o")),
                        self._rope_table(m), self._expand(get, p, H, R))
@@ -403,8 +403,7 @@ class KatidraModel(StreamModel):
     def _blocks(self, ids, b, after=None) -> torch.Tensor:
         """The residual stream after the last layer."""
         c, dt = self.cfg, self.dtype
-        x = sm.embed_rows(ids, self.embed, c.embed_scale)
-        h = x.to(dt)                      # the stream as the next sublayer reads it
+        x, h = sm.embed_rows(ids, self.embed, c.embed_scale, copy=True)    # h: the stream as the next sublayer reads it
         for L in self.layers:
             w = L.w
             run = self._lightning if isinstance(w.mixer, _Lightning) else self._latent
@@ -418,7 +417,7 @@ class KatidraModel(StreamModel):
 
     def _forward(self, ids, b, rows) -> torch.Tensor:
         x = self._blocks(ids, b)
-        hf = sm.resnorm(x.index_select(0, rows), self.final_norm, self.cfg.rms_eps, out_dtype=self.dtype)
+        hf = sm.resnorm(pick_rows(x, rows), self.final_norm, self.cfg.rms_eps, out_dtype=self.dtype)
         return sm.linear(hf, self.lm_head, out_dtype=F32).unsqueeze(0)     # [1, S, vocab]
 
     def residual_after_runs(self, ids, b) -> List[torch.Tensor]:

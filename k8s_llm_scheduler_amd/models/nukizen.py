@@ -41,7 +41,7 @@ from ..ops import reference as ref
 from ..ops import seqmix as sm
 from ..parallel import TPGroup
 from . import stream
-from .stream import StreamModel
+from .stream import StreamModel, pick_rows
 
 ARCHITECTURE = "Nukizen"
 MIXERS = ("attention", "rglru", "parallel")
@@ -609,8 +609,7 @@ class NukizenModel(StreamModel):
     def _forward(self, ids, b, rows) -> torch.Tensor:
         c = self.cfg
         x, mix, ff = self._blocks(ids, b)
-        pick = lambda t: t.index_select(0, rows) if t is not None else None
-        hf = sm.resnorm(x.index_select(0, rows), self.final_norm, c.rms_eps, branch=pick(mix), branch2=pick(ff),
+        hf = sm.resnorm(pick_rows(x, rows), self.final_norm, c.rms_eps, branch=pick_rows(mix, rows), branch2=pick_rows(ff, rows),
                         out_dtype=self.dtype)
         z = sm.linear(hf, self.lm_head, out_dtype=F32)
         if c.logit_softcap > 0:

@@ -33,7 +33,7 @@ from ..ops import reference as ref
 from ..ops import seqmix as sm
 from ..parallel import TPGroup
 from . import stream
-from .stream import StreamModel
+from .stream import StreamModel, pick_rows
 
 ARCHITECTURE = "Putulorn"
 SWISH_ALPHA = 1.702          # the experts' sigmoid slope
@@ -495,8 +495,8 @@ class PutulornModel(StreamModel):
                 pend = self._mlp(L.mlp, h)
             else:
                 pend = y
-        xs = x.index_select(0, rows)
-        hf = sm.resnorm(xs, self.final_norm, eps, branch=pend.index_select(0, rows) if pend is not None else None,
+        xs = pick_rows(x, rows)
+        hf = sm.resnorm(xs, self.final_norm, eps, branch=pick_rows(pend, rows),
                         mult=mult, offset=1.0, out_dtype=dt)
         return sm.linear(hf, self.lm_head, out_dtype=torch.float32).unsqueeze(0)      # [1, S, vocab]
 

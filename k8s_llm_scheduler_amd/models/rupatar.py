@@ -38,7 +38,7 @@ from ..ops import reference as ref
 from ..ops import seqmix as sm
 from ..parallel import TPGroup
 from . import stream
-from .stream import StreamModel
+from .stream import StreamModel, pick_rows
 
 ARCHITECTURE = "Rupatar"
 MIXERS = ("attention", "hgrn2", "mlstm")
@@ -494,8 +494,8 @@ class RupatarModel(StreamModel):
     def _forward(self, ids, b, rows) -> torch.Tensor:
         c = self.cfg
         x, pend, bias = self._blocks(ids, b)
-        xs = x.index_select(0, rows)
-        hf = sm.resnorm(xs, self.final_norm, c.rms_eps, branch=pend.index_select(0, rows) if pend is not None else None,
+        xs = pick_rows(x, rows)
+        hf = sm.resnorm(xs, self.final_norm, c.rms_eps, branch=pick_rows(pend, rows),
                         rowvec=bias, out_dtype=self.dtype, groups=c.norm_groups)
         return sm.linear(hf, self.lm_head, out_dtype=F32).unsqueeze(0)                    # [1, S, vocab]
 

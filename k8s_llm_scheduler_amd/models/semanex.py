@@ -38,7 +38,7 @@ from ..ops import reference as ref
 from ..ops import seqmix as sm
 from ..parallel import TPGroup
 from . import stream
-from .stream import StreamModel, stack_rows
+from .stream import StreamModel, pick_rows, stack_rows
 
 ARCHITECTURE = "Semanex"
 MIXERS = ("latent_attention", "parallel")
@@ -370,7 +370,7 @@ class SemanexModel(StreamModel):
         H, Dn, R, V, C = m.heads, m.dim, m.rot_dim, m.vdim, m.kv_rank
         if m.rot_dims % 2 or not 0 < m.rot_dims <= R:
             raise ValueError(f"{where}: rot.dims {m.rot_dims} must be even, positive and at most rot_dim {R}")
-        w_in, cols = stack_rows((("dq", get(p + "dq").cpu()), ("dkv", get(p + "dkv").cpu()), ("g", get(p + "g").cpu())))
+        w_in, cols = stack_rows((("dq", get(p + "dq")), ("dkv", get(p + "dkv")), ("g", get(p + "g"))))
         return _Latent(m, t(w_in), cols, t(get(p + "dq.norm")), t(get(p + "uq")), t(get(p + "dkv.norm")),
                        t(get(p + "uk").view(H, Dn, C).transpose(1, 2)), t(get(p + "uv").view(H, V, C)),
                        self._f(get(p + "sink")), t(get(p + "o")), self._rope_table(m.rot_dims, m.rot_base),
@@ -386,7 +386,7 @@ class SemanexModel(StreamModel):
         if max(r.state, r.vdim) > sm.gated_scan_max_dim():
             raise ValueError(f"{where}: state {r.state} x {r.vdim} exceeds the kernels' {sm.gated_scan_max_dim()}")
         q = p + "left."
-        w_in, cols = stack_rows(tuple((s, get(q + s).cpu()) for s in ("q", "k", "v", "g")))
+        w_in, cols = stack_rows(tuple((s, get(q + s)) for s in ("q", "k", "v", "g")))
         left = _Capped(a, t(w_in), cols, t(get(q + "q.norm")), t(get(q + "k.norm")), t(get(q + "o")))
         q = p + "right."
         r.conv = int(get(q + "conv").shape[1])                 # the taps are what the checkpoint holds
@@ -539,7 +539,7 @@ class SemanexModel(StreamModel):
     def _forward(self, ids, b, rows) -> torch.Tensor:
         c = self.cfg
         x = self._blocks(ids, b)
-        hf = sm.postnorm(x.index_select(0, rows), None, 1.0, self.final_gain, c.rms_eps, out_dtype=self.dtype)
+        hf = sm.postnorm(pick_rows(x, rows), None, 1.0, self.final_gain, c.rms_eps, out_dtype=self.dtype)
         return sm.linear(hf, self.lm_head, out_dtype=F32).unsqueeze(0)     # [1, S, vocab]
 
     def residual_after_runs(self, ids, b) -> List[torch.Tensor]:

@@ -33,12 +33,17 @@ def stack_rows(parts, align: int = 16):
     rows, cols, at = [], {}, 0
     for key, w in parts:
         cols[key] = at
-        rows.append(w)
+        rows.append(w if not rows else w.to(rows[0].device))
         pad = (-w.shape[0]) % align
         if pad:
-            rows.append(torch.zeros(pad, w.shape[1], dtype=w.dtype))
+            rows.append(torch.zeros(pad, w.shape[1], dtype=w.dtype, device=w.device))
         at += w.shape[0] + pad
     return torch.cat(rows), cols
+
+
+def pick_rows(t: Optional[torch.Tensor], rows: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """The rows whose logits are wanted (None: all of them)."""
+    return t if t is None or rows is None else t.index_select(0, rows)
 
 
 class StreamModel:
@@ -142,16 +147,11 @@ class StreamModel:
         touch neither cache nor state."""
         self._check_ready()
         B = tokens.shape[0]
-        dev = tokens.device
-        bs = self.block_size
-        pos = (context_lens - 1).clamp(min=0).long()
-        blk = block_tables.long().gather(1, (pos // bs).unsqueeze(1)).squeeze(1)
-        slots = torch.where(context_lens > 0, blk * bs + pos % bs, torch.full_like(blk, -1)).to(torch.int32)
-        ar = torch.arange(B + 1, dtype=torch.int32, device=dev)
-        b = {"positions": (context_lens - 1).to(torch.int32), "slot_mapping": slots.contiguous(), "cu_q": ar,
-             "tok_seq": ar[:B], "block_tables": block_tables.contiguous(), "seq_slots": ar[:B],
-             "max_keys": int(max_context)}
-        return self._forward(tokens, b, ar[:B].long())
+        tables = block_tables.contiguous()
+        pos, slots, ar = sm.decode_meta(context_lens.to(torch.int32).contiguous(), tables, self.block_size)
+        b = {"positions": pos, "slot_mapping": slots, "cu_q": ar, "tok_seq": ar[:B], "block_tables": tables,
+             "seq_slots": ar[:B], "max_keys": int(max_context)}
+        return self._forward(tokens, b, None)
 
     def warm(self) -> None:
         pass

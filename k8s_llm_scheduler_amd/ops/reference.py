@@ -506,6 +506,15 @@ def embed_rows(ids: torch.Tensor, table: torch.Tensor, scale: float = 1.0) -> to
     return table.index_select(0, ids.long()).float() * scale
 
 
+def decode_meta(context_lens: torch.Tensor, block_tables: torch.Tensor, block_size: int):
+    """int32 (positions, cache slots (-1: idle), 0 .. B) of a step of single tokens."""
+    pos = (context_lens - 1).clamp(min=0).long()
+    blk = block_tables.long().gather(1, (pos // block_size).unsqueeze(1)).squeeze(1)
+    slots = torch.where(context_lens > 0, blk * block_size + pos % block_size, torch.full_like(blk, -1)).to(torch.int32)
+    ar = torch.arange(context_lens.shape[0] + 1, dtype=torch.int32, device=context_lens.device)
+    return (context_lens - 1).to(torch.int32), slots.contiguous(), ar
+
+
 def resnorm(x: torch.Tensor, branch, mult: float, rowvec, w, offset: float, eps: float, out_dtype, groups: int = 1,
             branch2=None):
     """x (fp32, in place) += mult * (branch + branch2) + rowvec; returns x / sqrt(mean(x^2) + eps) * (offset + w) or

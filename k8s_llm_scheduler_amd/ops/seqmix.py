@@ -59,15 +59,33 @@ def _f32(dtype) -> int:
 
 
 # ----------------------------------------------------------------------------- residual stream
-def embed_rows(ids: torch.Tensor, table: torch.Tensor, scale: float = 1.0) -> torch.Tensor:
-    """fp32 [T, W] rows of ``table`` (bf16 or fp32) times ``scale``."""
+def embed_rows(ids: torch.Tensor, table: torch.Tensor, scale: float = 1.0, copy: bool = False):
+    """fp32 [T, W] rows of ``table`` (bf16 or fp32) times ``scale``; ``copy``: (rows, the same in the table's type)."""
     if not _gpu(ids, table):
-        return ref.embed_rows(ids, table, scale)
+        x = ref.embed_rows(ids, table, scale)
+        return (x, x.to(table.dtype, copy=True)) if copy else x
     T, W = ids.shape[0], table.shape[1]
     out = torch.empty(T, W, dtype=F32, device=table.device)
-    _native().embed_rows(out.data_ptr(), _p(ids, I32, "ids"), _p(table), T, W, table.shape[0], float(scale),
+    same = torch.empty(T, W, dtype=table.dtype, device=table.device) if copy else None
+    _native().embed_rows(out.data_ptr(), _p(same), _p(ids, I32, "ids"), _p(table), T, W, table.shape[0], float(scale),
                          _f32(table.dtype), -1)
-    return out
+    return (out, same) if copy else out
+
+
+def decode_meta(context_lens: torch.Tensor, block_tables: torch.Tensor, block_size: int):
+    """Of a step of single tokens, row i = state slot i with ``context_lens[i]`` tokens (0: idle): int32 (positions,
+    cache slots (-1: idle), 0 .. B)."""
+    if not _gpu(context_lens, block_tables):
+        return ref.decode_meta(context_lens, block_tables, block_size)
+    B = context_lens.shape[0]
+    if block_tables.dim() != 2 or block_tables.shape[0] < B:
+        raise ValueError("decode_meta: a row of the block table for every context length")
+    n = (B + 4) // 4 * 4
+    meta = torch.empty(3, n, dtype=I32, device=context_lens.device)      # rows 16 bytes aligned
+    pos, slots, ar = meta[0, :B], meta[1, :B], meta[2, :B + 1]
+    _native().decode_meta(pos.data_ptr(), slots.data_ptr(), ar.data_ptr(), _p(context_lens, I32, "context_lens"),
+                          _p(block_tables, I32, "block_tables"), block_tables.shape[1], B, int(block_size), -1)
+    return pos, slots, ar
 
 
 def resnorm(x: torch.Tensor, w: Optional[torch.Tensor], eps: float, *, branch: Optional[torch.Tensor] = None,

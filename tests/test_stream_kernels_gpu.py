@@ -290,3 +290,25 @@ def test_recurrence_prefix_over_many_chunks():
         for y, s in outs[1:]:
             assert (y - outs[0][0]).abs().max() <= 1e-4 * outs[0][0].abs().max()
             assert (s - outs[0][1]).abs().max() <= 1e-5 * outs[0][1].abs().max()
+
+
+@pytest.mark.parametrize("bs", [1, 16])
+@pytest.mark.parametrize("B", [1, 5, 255, 256, 300])
+def test_decode_meta(B, bs):
+    """Against the reference ops: idle rows, first and last position of a page, of the table; beyond it a row idles."""
+    nb = 7
+    ctx = torch.tensor([(0, 1, bs, bs + 1, nb * bs, nb * bs - 1, 3)[i % 7] for i in range(B)], dtype=torch.int32)
+    bt = torch.randperm(B * nb).int().view(B, nb)
+    want, got = sm.decode_meta(ctx, bt, bs), sm.decode_meta(ctx.to(DEV), bt.to(DEV), bs)
+    for w, g in zip(want, got):
+        assert torch.equal(w, g.cpu())
+    pos, slots, _ = sm.decode_meta(torch.full((B,), nb * bs + 1, dtype=torch.int32, device=DEV), bt.to(DEV), bs)
+    assert (pos == -1).all() and (slots == -1).all()
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_embedding_copy(dt):
+    ids, table = torch.tensor([3, 0, 6, 3], dtype=torch.int32), torch.randn(7, 1030).to(dt)
+    want, got = sm.embed_rows(ids, table, 1.7, copy=True), sm.embed_rows(ids.to(DEV), table.to(DEV), 1.7, copy=True)
+    assert all(torch.equal(w, g.cpu()) for w, g in zip(want, got))
+    assert torch.equal(got[0], sm.embed_rows(ids.to(DEV), table.to(DEV), 1.7))
