@@ -730,14 +730,18 @@ __global__ __launch_bounds__(256) void window_attention_mfma_kernel(
 //   * two LDS buffers, one barrier per step: while a step is computed the next one is stored and the one after next is
 //     loaded into registers, its page numbers a step earlier still; a thread always moves one row's pieces;
 //   * scores in base 2 (scale and slopes carry log2 e), no mask arithmetic on slices that every column of the wave sees,
-//     accumulators rescaled only when some column's maximum moved, sums kept per lane until the end.
-template <int DK, int DV, int NCB>
+//     accumulators rescaled only when some column's maximum moved, sums kept per lane until the end;
+//   * where the tiles are few (a short portion behind a long cached one), nsplit workgroups share a tile's steps and leave
+//     (max, sum, unnormalised sum) for window_merge_kernel: a step is a chain of LDS and shuffle latencies of about 2.5 us
+//     however few workgroups run.  16 query heads over 4 of 128, 97 tokens behind 1000: 46.6 us in
+//     one piece, 23.3 us in 8 with the merge.  (A template flag: the arithmetic of the splits costs the whole walk 8%.)
+template <int DK, int DV, int NCB, bool SPLIT>
 __global__ __launch_bounds__(512) void window_prompt_kernel(
-    bf16_t* __restrict__ out, const bf16_t* __restrict__ q, long ldq, const bf16_t* __restrict__ gate, long ldg,
-    const bf16_t* __restrict__ kcache, const bf16_t* __restrict__ vcache, const int* __restrict__ block_tables,
-    int max_blocks, const int* __restrict__ cu_q, const int* __restrict__ positions, int H, int G, int window, float scale,
-    int sink, int bshift, int R, int chunk, float softcap, const float* __restrict__ sinkv, int gate_ph,
-    const float* __restrict__ slopes) {
+    bf16_t* __restrict__ out, float* __restrict__ pacc, float* __restrict__ pml, const bf16_t* __restrict__ q, long ldq,
+    const bf16_t* __restrict__ gate, long ldg, const bf16_t* __restrict__ kcache, const bf16_t* __restrict__ vcache,
+    const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ cu_q, const int* __restrict__ positions,
+    int H, int G, int window, float scale, int sink, int bshift, int nsplit, int R, int chunk, float softcap,
+    const float* __restrict__ sinkv, int gate_ph, const float* __restrict__ slopes) {
   constexpr int NKK = DK / 32, NVB = DV / 16, KT = 64;
   constexpr int ROWK = (DK + 8) * 2, ROWV = (DV + 8) * 2, BUF = KT * (ROWK + ROWV);   // LDS bytes
   constexpr int CK = DK / 8, CV = DV / 8, NST = (CK + CV + 7) / 8;                   // 16-byte pieces; per thread
@@ -746,11 +750,13 @@ __global__ __launch_bounds__(512) void window_prompt_kernel(
   const int seq = blockIdx.z, g = blockIdx.y;
   const int tid = threadIdx.x, wave = (tid >> 6) & 3, grp = tid >> 8, lane = tid & 63, li = lane & 15, g4 = lane >> 4;
   const int TPC = 16 / R, TPB = 4 * NCB * TPC;
-  const int tq0 = cu_q[seq] + blockIdx.x * TPB, tend = cu_q[seq + 1];
+  const int split = SPLIT ? blockIdx.x % nsplit : 0;
+  const int tq0 = cu_q[seq] + (SPLIT ? blockIdx.x / nsplit : blockIdx.x) * TPB, tend = cu_q[seq + 1];
   if (tq0 >= tend) return;
   const int p_first = positions[tq0];
   const int nval = min(TPB, tend - tq0);
   if (p_first < 0) {   // idle rows: defined output
+    if (SPLIT) return;          // (the merge's business)
     for (int i = tid; i < nval * R * DV; i += 512) {
       const int tt = i / (R * DV), r = i - tt * (R * DV);
       out[(size_t)(tq0 + tt) * H * DV + (size_t)g * R * DV + r] = 0;
@@ -761,7 +767,17 @@ __global__ __launch_bounds__(512) void window_prompt_kernel(
   auto lo_of = [&](int p) { return chunk > 0 ? p - p % chunk : (window > 0 ? max(0, p - window + 1) : 0); };
   const int lo_min = lo_of(p_first);
   const int nkeys = p_last + 1 - lo_min;
-  const int nsteps = (nkeys + KT - 1) / KT;
+  const int ntot = (nkeys + KT - 1) / KT, per = SPLIT ? max(2, (ntot + nsplit - 1) / nsplit) : ntot;
+  const int step0 = split * per, nsteps = min(ntot, step0 + per);      // this split's steps
+  if (SPLIT && step0 >= ntot) {   // none (split 0 always has one)
+    for (int i = tid; i < nval * R; i += 512) {
+      const int tt = i / R;
+      const size_t rec = ((size_t)(tq0 + tt) * H + g * R + (i - tt * R)) * nsplit + split;
+      pml[rec * 2] = -INFINITY;
+      pml[rec * 2 + 1] = 0.f;
+    }
+    return;
+  }
   const int* btr = block_tables + (size_t)seq * max_blocks;
   const int GD = G * DK, GV = G * DV, bmask = (1 << bshift) - 1;
   const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
@@ -790,7 +806,7 @@ __global__ __launch_bounds__(512) void window_prompt_kernel(
   }
   const bool w_any = w_pmax >= 0;
   const int w_lo = w_any ? lo_of(w_pmin) : 0, w_hi_lo = w_any ? lo_of(w_pmax) : 0;   // first key any / every column sees
-  const bool with_sink = sink && grp == 0;
+  const bool with_sink = sink && grp == 0 && split == 0;
   const float sc2 = scale * LOG2E;
   const float slope2 = slopes != nullptr ? slopes[hd] * LOG2E : 0.f;
   f32x4 o[NCB][NVB];
@@ -830,13 +846,13 @@ __global__ __launch_bounds__(512) void window_prompt_kernel(
       else if (c < CK + CV) *reinterpret_cast<u32x4*>(buf + KT * ROWK + sr * ROWV + 16 * (c - CK)) = pre[i];
     }
   };
-  stage_load(0, page_of(0));
-  stage_store(smem_p);
-  int page = nsteps > 1 ? page_of(1) : -1;
-  if (nsteps > 1) stage_load(1, page);
-  page = nsteps > 2 ? page_of(2) : -1;
+  stage_load(step0, page_of(step0));
+  stage_store(smem_p + (step0 & 1) * BUF);
+  int page = step0 + 1 < nsteps ? page_of(step0 + 1) : -1;
+  if (step0 + 1 < nsteps) stage_load(step0 + 1, page);
+  page = step0 + 2 < nsteps ? page_of(step0 + 2) : -1;
   __syncthreads();
-  for (int step = 0; step < nsteps; ++step) {
+  for (int step = step0; step < nsteps; ++step) {
     char* buf = smem_p + (step & 1) * BUF;
     if (step + 1 < nsteps) {
       stage_store(smem_p + ((step + 1) & 1) * BUF);
@@ -972,14 +988,26 @@ __global__ __launch_bounds__(512) void window_prompt_kernel(
     const float m1 = b[4 * NVB * 64], M = fmaxf(m_run[cb], m1);
     const float f0 = m_run[cb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[cb] - M);
     const float f1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - M);
-    const float inv = 1.f / (l_run[cb] * f0 + b[(4 * NVB + 1) * 64] * f1);
+    const float lsum = l_run[cb] * f0 + b[(4 * NVB + 1) * 64] * f1, inv = SPLIT ? 1.f : 1.f / lsum;
+    const float m2 = M * 0.6931471805599453f;       // -inf and sum 0: no key of this split is seen
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int c = 4 * g4 + i;
       const float w0 = __shfl(f0 * inv, c, WAVE), w1 = __shfl(f1 * inv, c, WAVE);
+      const float mt = SPLIT ? __shfl(m2, c, WAVE) : 0.f, lt = SPLIT ? __shfl(lsum, c, WAVE) : 0.f;
       const int toff = (wave * NCB + cb) * TPC + c / R;
       if (toff >= nval) continue;
       const int t = tq0 + toff, h = g * R + c % R;
+      if constexpr (SPLIT) {
+        const size_t rec = ((size_t)t * H + h) * nsplit + split;
+#pragma unroll
+        for (int n = 0; n < NVB; ++n) pacc[rec * DV + 16 * n + li] = o[cb][n][i] * w0 + b[(4 * n + i) * 64] * w1;
+        if (li == 0) {
+          pml[rec * 2] = mt;
+          pml[rec * 2 + 1] = lt;
+        }
+        continue;
+      }
       float s = 1.f;
       if (gate != nullptr && gate_ph) s = 1.f / (1.f + expf(-bf2f(gate[(size_t)t * ldg + h])));
 #pragma unroll
@@ -1321,46 +1349,65 @@ extern "C" int k8s_window_mfma_ok(int H, int G, int D, int V) {
   return (R == 1 || R == 2 || R == 4 || R == 8 || R == 16) && D % 8 == 0 && V % 16 == 0 && D <= 256 && V <= 256;
 }
 
-// Prompt portions in bf16: nseq sequences of at most max_qlen tokens, cu_q their query offsets.
-extern "C" int k8s_window_attention_mfma(void* out, const void* q, long ldq, const void* gate, long ldg,
-                                         const void* kcache, const void* vcache, const float* kpool, const float* vpool,
+// Tokens that one workgroup of window_prompt_kernel takes (0: it does not take these sizes).
+extern "C" int k8s_window_prompt_tile(int H, int G, int D, int V, int P, int bs) {
+  if (!k8s_window_mfma_ok(H, G, D, V) || P > 0 || D != V || (D != 64 && D != 96 && D != 128) || bs <= 0 || (bs & (bs - 1)))
+    return 0;
+  return 4 * 2 * (16 / (H / G));
+}
+
+// Prompt portions in bf16: nseq sequences of at most max_qlen tokens (T in all), cu_q their query offsets.  nsplit > 1 (only
+// where k8s_window_prompt_tile > 0): pacc [T, H, nsplit, V] and pml [T, H, nsplit, 2] fp32 workspaces.
+extern "C" int k8s_window_attention_mfma(void* out, float* pacc, float* pml, const void* q, long ldq, const void* gate,
+                                         long ldg, const void* kcache, const void* vcache, const float* kpool, const float* vpool,
                                          const int* block_tables, int max_blocks, const int* cu_q, const int* positions,
-                                         int nseq, int max_qlen, int H, int G, int D, int V, int window, int P,
-                                         float scale, int sink, int bs, int chunk, float softcap,
+                                         int nseq, int max_qlen, int T, int H, int G, int D, int V, int window, int P,
+                                         float scale, int sink, int bs, int nsplit, int chunk, float softcap,
                                          const float* sinkv, int gate_ph, const float* slopes, hipStream_t s) {
   if (nseq <= 0 || max_qlen <= 0) return 0;
+  if (nsplit < 1 || nsplit > 64 || (nsplit > 1 && (pacc == nullptr || pml == nullptr || T <= 0))) return -1;
   if (!k8s_window_mfma_ok(H, G, D, V) || bs <= 0 || nseq > 65535 || G > 65535 || ldq % 8 || ((uintptr_t)q & 15)) return -1;
   if (window > 0 && P > 0 && (kpool == nullptr || vpool == nullptr || slopes != nullptr)) return -1;
   const int R = H / G, ppb = P > 0 ? (bs + P - 1) / P : 1;
   constexpr int NCB = 2;
-  if (P <= 0 && D == V && (D == 64 || D == 96 || D == 128) && (bs & (bs - 1)) == 0) {
-    const int tpb = 4 * NCB * (16 / R);
-    const dim3 grid((max_qlen + tpb - 1) / tpb, G, nseq);
+  if (k8s_window_prompt_tile(H, G, D, V, P, bs) > 0) {
+    const int tpb = k8s_window_prompt_tile(H, G, D, V, P, bs);
+    const dim3 grid((max_qlen + tpb - 1) / tpb * nsplit, G, nseq);
     int bshift = 0;
     while ((1 << bshift) < bs) ++bshift;
     const size_t stage = (size_t)2 * 64 * (D + 8 + V + 8) * 2;                     // two buffers of 64 rows
     const size_t merge = (size_t)4 * 64 * NCB * (4 * (V / 16) + 2) * sizeof(float);   // one group's results
     const size_t lds = stage > merge ? stage : merge;
-#define K8S_WP(DK)                                                                                                      \
+#define K8S_WP(DK, SPLIT)                                                                                               \
   do {                                                                                                                  \
     static bool grown = false;   /* more LDS than a launch gets by default */                                           \
     if (!grown) {                                                                                                       \
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_prompt_kernel<DK, DK, NCB>),        \
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_prompt_kernel<DK, DK, NCB, SPLIT>), \
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                   \
       if (e != hipSuccess) return (int)e;                                                                               \
       grown = true;                                                                                                     \
     }                                                                                                                   \
-    window_prompt_kernel<DK, DK, NCB><<<grid, 512, lds, s>>>(                                                           \
-        (bf16_t*)out, (const bf16_t*)q, ldq, (const bf16_t*)gate, ldg, (const bf16_t*)kcache, (const bf16_t*)vcache,    \
-        block_tables, max_blocks, cu_q, positions, H, G, window, scale, sink, bshift, R, chunk, softcap, sinkv, gate_ph, \
-        slopes);                                                                                                        \
+    window_prompt_kernel<DK, DK, NCB, SPLIT><<<grid, 512, lds, s>>>(                                                    \
+        (bf16_t*)out, pacc, pml, (const bf16_t*)q, ldq, (const bf16_t*)gate, ldg, (const bf16_t*)kcache,                \
+        (const bf16_t*)vcache, block_tables, max_blocks, cu_q, positions, H, G, window, scale, sink, bshift, nsplit, R, \
+        chunk, softcap, sinkv, gate_ph, slopes);                                                                        \
   } while (0)
-    if (D == 64) K8S_WP(64);
-    else if (D == 96) K8S_WP(96);
-    else K8S_WP(128);
+#define K8S_WP_D(SPLIT)                \
+  do {                                 \
+    if (D == 64) K8S_WP(64, SPLIT);    \
+    else if (D == 96) K8S_WP(96, SPLIT); \
+    else K8S_WP(128, SPLIT);           \
+  } while (0)
+    if (nsplit > 1) K8S_WP_D(true);
+    else K8S_WP_D(false);
+#undef K8S_WP_D
 #undef K8S_WP
+    if (nsplit > 1)
+      window_merge_kernel<bf16_t><<<dim3(T, H), 64, 0, s>>>((bf16_t*)out, pacc, pml, (const bf16_t*)gate, ldg, positions, H,
+                                                            V, nsplit, gate_ph);
     return (int)hipGetLastError();
   }
+  if (nsplit > 1) return -1;
   const size_t lds = (size_t)32 * ((D + 8) + (V + 8)) * 2;
   const int TPB = 4 * NCB * (16 / R);
   const dim3 grid((max_qlen + TPB - 1) / TPB, G, nseq);

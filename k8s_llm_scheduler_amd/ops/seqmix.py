@@ -798,6 +798,13 @@ def token_splits(T: int, G: int, keys: int) -> int:
     return max(1, min(-(-512 // max(1, T * G)), -(-max(1, keys) // 128), 16))
 
 
+def prompt_splits(groups: int, keys: int) -> int:
+    """Key splits of the prompt kernel's ``groups`` workgroups: up to 256 (one per CU: 40 workgroups, 300 tokens behind 1000,
+    6 splits 30 us, 8 splits 40 us), of two 64-key steps at least, at most 8 (1000 keys, 16 workgroups: 8 splits 23 us, 16
+    splits 26 us, the more the merge reads)."""
+    return max(1, min(256 // max(1, groups), -(-max(1, keys) // 128), 8))
+
+
 def window_attention(q: torch.Tensor, gate: Optional[torch.Tensor], kcache: torch.Tensor, vcache: torch.Tensor,
                      kpool: Optional[torch.Tensor], vpool: Optional[torch.Tensor], block_tables: torch.Tensor,
                      tok_seq: torch.Tensor, positions: torch.Tensor, H: int, window: int, P: int, scale: float,
@@ -841,12 +848,21 @@ def window_attention(q: torch.Tensor, gate: Optional[torch.Tensor], kcache: torc
     nat = _native()
     if (WINDOW_MFMA and dt == BF16 and cu_q is not None and max_qlen > 1 and nat.window_mfma_ok(H, G, D, V)
             and q.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0):
-        nat.window_attention_mfma(out.data_ptr(), q.data_ptr(), q.stride(0), gate.data_ptr() if gate is not None else 0,
+        tile = nat.window_prompt_tile(H, G, D, V, int(P), block_size)
+        ns, pacc, pml = 1, None, None
+        if tile > 0:
+            max_pos = max_keys or block_tables.shape[1] * block_size
+            ns = prompt_splits(-(-int(max_qlen) // tile) * G * (cu_q.shape[0] - 1),
+                               min(max_pos, (chunk or window + tile) if chunk > 0 or window > 0 else max_pos))
+        if ns > 1:
+            pacc = torch.empty(T * H * ns * V, dtype=F32, device=q.device)
+            pml = torch.empty(T * H * ns * 2, dtype=F32, device=q.device)
+        nat.window_attention_mfma(out.data_ptr(), _p(pacc), _p(pml), q.data_ptr(), q.stride(0), gate.data_ptr() if gate is not None else 0,
                                   gate.stride(0) if gate is not None else 0, _p(kcache, dt, "kcache"),
                                   _p(vcache, dt, "vcache"), _p(kpool, F32, "kpool"), _p(vpool, F32, "vpool"),
                                   _p(block_tables, I32, "block_tables"), block_tables.shape[1], _p(cu_q, I32, "cu_q"),
-                                  _p(positions, I32), cu_q.shape[0] - 1, int(max_qlen), H, G, D, V, int(window), int(P),
-                                  float(scale), int(bool(sink)), block_size, int(chunk), float(softcap), _p(sinks),
+                                  _p(positions, I32), cu_q.shape[0] - 1, int(max_qlen), T, H, G, D, V, int(window), int(P),
+                                  float(scale), int(bool(sink)), block_size, ns, int(chunk), float(softcap), _p(sinks),
                                   int(bool(gate_per_head)), _p(slopes), -1)
         return out
     max_pos = max_keys or block_tables.shape[1] * block_size

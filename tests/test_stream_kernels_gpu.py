@@ -312,3 +312,34 @@ def test_embedding_copy(dt):
     want, got = sm.embed_rows(ids, table, 1.7, copy=True), sm.embed_rows(ids.to(DEV), table.to(DEV), 1.7, copy=True)
     assert all(torch.equal(w, g.cpu()) for w, g in zip(want, got))
     assert torch.equal(got[0], sm.embed_rows(ids.to(DEV), table.to(DEV), 1.7))
+
+
+@pytest.mark.parametrize("H,G,D,kw", [
+    (16, 4, 128, dict(window=0)), (8, 2, 64, dict(window=150, slopes=True)), (6, 6, 96, dict(chunk=200, softcap=3.0)),
+    (4, 2, 96, dict(window=1)), (8, 4, 128, dict(chunk=96, slopes=True, gate=False)),
+])
+@pytest.mark.parametrize("ns", [2, 3, 16])
+def test_prompt_attention_key_splits(H, G, D, kw, ns, monkeypatch):
+    """Splits of several steps, of one, without any (short sequences, windows) and the sink in split 0 only, against one
+    workgroup per tile: the same fp32 sums in another order, rounded once to bf16 (2^-9 of a value, both sides), and the
+    weights' second bf16 term (2^-16) of every key."""
+    torch.manual_seed(3)
+    bs, dt = 16, torch.bfloat16
+    lens = [(0, 133), (290, 70), (40, 1), (-1, 1), (500, 35)]
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    cu = i32([0] + [n for _, n in lens]).cumsum(0).int()
+    pos = i32([p for a, n in lens for p in (range(a, a + n) if a >= 0 else [-1])])
+    tok_seq = i32([s for s, (_, n) in enumerate(lens) for _ in range(n)])
+    bt = torch.randperm(5 * 36, device=DEV).int().view(5, 36)
+    kc, vc = (torch.randn(5 * 36 * bs, G, D, device=DEV).to(dt) for _ in range(2))
+    q = torch.randn(pos.shape[0], H * D + 16, device=DEV).to(dt)
+    gate = torch.randn(pos.shape[0], H * D, device=DEV).to(dt) if kw.get("gate", True) else None
+    slopes = torch.linspace(0.003, 1.0, H, device=DEV) if kw.get("slopes") else None
+    outs = []
+    for n in (1, ns):
+        monkeypatch.setattr(sm, "prompt_splits", lambda groups, keys: n)
+        outs.append(sm.window_attention(q, gate, kc, vc, None, None, bt, tok_seq, pos, H, kw.get("window", 0), 0, D ** -0.5,
+                                        True, bs, cu, 133, chunk=kw.get("chunk", 0), softcap=kw.get("softcap", 0.0),
+                                        sinks=torch.linspace(-3, 3, H, device=DEV), slopes=slopes).float())
+    assert (outs[1][pos < 0] == 0).all()
+    assert ((outs[1] - outs[0]).abs() <= 2.0 ** -7 * outs[0].abs() + 2.0 ** -13 * outs[0].abs().max()).all()
