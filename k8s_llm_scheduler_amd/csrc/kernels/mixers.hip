@@ -85,9 +85,10 @@ __global__ void shift_save_kernel(TA* __restrict__ state, const TA* __restrict__
 //
 // MODE 0: a whole sequence per workgroup, from the slot's state (zero at position 0) to the slot's state.
 // Long prompts run as three passes over chunks of Lc tokens, so the recurrence is parallel over chunks:
-// MODE 1: a chunk from a zero state, no outputs: its state contribution and the product of its decays -> cs_loc, cs_dec;
-//         wkv_prefix_kernel then walks a sequence's chunks: start[c + 1] = dec[c] * start[c] + loc[c];
-// MODE 2: a chunk from its start state with outputs; a sequence's last chunk leaves the slot's state.
+// wkv_chunk_state_kernel: a chunk's state contribution and the product of its decays -> cs_loc, cs_dec;
+// wkv_prefix_kernel then walks a sequence's chunks: start[c + 1] = dec[c] * start[c] + loc[c];
+// MODE 2 (heads of more than 64 channels; wkv_chunk_out_kernel for the others): a chunk from its start state with outputs;
+//         a sequence's last chunk leaves the slot's state.
 template <typename TA, int CH, int MODE>
 __global__ __launch_bounds__(1024) void wkv_scan_kernel(TA* __restrict__ out, const TA* __restrict__ r,
                                                         const TA* __restrict__ k, const TA* __restrict__ v,
@@ -96,15 +97,14 @@ __global__ __launch_bounds__(1024) void wkv_scan_kernel(TA* __restrict__ out, co
                                                         const TA* __restrict__ lnw, float* __restrict__ state,
                                                         const int* __restrict__ cu_q, const int* __restrict__ seq_slots,
                                                         const int* __restrict__ positions, int H, int D, float eps,
-                                                        int nseq, int Lc, float* __restrict__ cs_loc,
-                                                        float* __restrict__ cs_dec, const float* __restrict__ cs_start) {
+                                                        int nseq, int Lc, const float* __restrict__ cs_start) {
   constexpr int DMAX = 128;
   __shared__ __attribute__((aligned(16))) float sr[DMAX], sk[DMAX], sw[DMAX], su[DMAX];
   __shared__ float po[DMAX / CH][DMAX];
   __shared__ float red[4];
   const int hd = blockIdx.y;
   int s, a, b, p0;
-  bool from_zero, last = true;
+  bool from_zero, last = true, many = false;
   if (MODE == 0) {
     s = blockIdx.x;
     a = cu_q[s];
@@ -118,23 +118,21 @@ __global__ __launch_bounds__(1024) void wkv_scan_kernel(TA* __restrict__ out, co
     if (ck.s < 0) return;
     s = ck.s;
     last = ck.c == ck.n - 1;
-    if (MODE == 1 && last) return;          // nothing follows a sequence's last chunk
     a = cu_q[s] + ck.c * Lc;
     b = min(cu_q[s + 1], a + Lc);
     p0 = positions[a];
-    from_zero = MODE == 1 || p0 == 0;
+    from_zero = p0 == 0;
+    many = ck.n > 1;
   }
   const int j = threadIdx.x, c = threadIdx.y, NS = blockDim.y, DV = blockDim.x;
   const bool on = j < D;
   const int HD = H * D, i0 = c * CH;
   float* st = state + ((size_t)seq_slots[s] * H + hd) * D * D;
-  const size_t crec = ((size_t)blockIdx.x * H + hd) * D * D;     // this chunk's record in cs_loc / cs_start
-  const float* src = (MODE == 2 && a != cu_q[s]) ? cs_start + crec : st;
-  float S[CH], decp[CH];
+  const float* src = many ? cs_start + ((size_t)blockIdx.x * H + hd) * D * D : st;
+  float S[CH];
 #pragma unroll
   for (int e = 0; e < CH; ++e) {
     S[e] = (on && i0 + e < D && !from_zero) ? src[(size_t)(i0 + e) * D + j] : 0.f;
-    decp[e] = 1.f;
   }
   float w0j = 0.f, lnj = 0.f;
   if (c == 0) {                       // group 0 stages the token's r, k, w (and u once); channels >= D stay zero
@@ -153,10 +151,8 @@ __global__ __launch_bounds__(1024) void wkv_scan_kernel(TA* __restrict__ out, co
       const size_t base = (size_t)t * ld + (size_t)hd * D + j;
       nv = ldf(v, base);
       if (c == 0) {
-        if (MODE != 1) {
-          nr = ldf(r, base);
-          ng = ldf(g, base);
-        }
+        nr = ldf(r, base);
+        ng = ldf(g, base);
         nk = ldf(k, base);
         nz = z[(size_t)t * HD + (size_t)hd * D + j];
       }
@@ -182,14 +178,9 @@ __global__ __launch_bounds__(1024) void wkv_scan_kernel(TA* __restrict__ out, co
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float kv = k4[e] * cv;
-        if (MODE != 1) o4[e] = fmaf(r4[e], fmaf(u4[e], kv, S[e0 + e]), o4[e]);
+        o4[e] = fmaf(r4[e], fmaf(u4[e], kv, S[e0 + e]), o4[e]);
         S[e0 + e] = fmaf(w4[e], S[e0 + e], kv);
-        if (MODE == 1) decp[e0 + e] *= w4[e];
       }
-    }
-    if (MODE == 1) {
-      lds_barrier();                   // the LDS rows are free for the next token
-      continue;
     }
     if (on) po[c][j] = (o4[0] + o4[1]) + (o4[2] + o4[3]);
     lds_barrier();
@@ -209,25 +200,241 @@ __global__ __launch_bounds__(1024) void wkv_scan_kernel(TA* __restrict__ out, co
       stf(out, (size_t)t * HD + (size_t)hd * D + j, y);
     }
   }
-  if (on) {
-    float* dst = MODE == 1 ? cs_loc + crec : st;
-    if (MODE != 2 || last) {
+  if (on && last) {
 #pragma unroll
-      for (int e = 0; e < CH; ++e)
-        if (i0 + e < D) dst[(size_t)(i0 + e) * D + j] = S[e];
-    }
-    if (MODE == 1 && j == 0) {
+    for (int e = 0; e < CH; ++e)
+      if (i0 + e < D) st[(size_t)(i0 + e) * D + j] = S[e];
+  }
+}
+
+// MODE 1 on the matrix cores: a chunk's state contribution is the product
+//   loc[i][j] = sum_s (k_s[i] prod_{t > s} w_t[i]) v_s[j],     dec[i] = prod_t w_t[i],
+// fp32 in and out (v_mfma_f32_16x16x4_f32); the decay products are of numbers <= 1, so nothing overflows whatever the
+// decays.  Workgroups (chunk, head, 64 x 64 block of the state) of 4 waves: the chunk's tokens from the last to the first
+// in blocks of 64, a wave multiplies up the decays behind 16 tokens (lane = key channel) and the waves' totals meet in LDS;
+// then a wave takes 16 key channels.  Walking the tokens one by one took 55 us for 2048 tokens of 32 heads of 64, this 22 us
+// (33 MB read, 17 MB written: 8 us; the rest is the chain of the decays and the three barriers of a chunk).
+template <typename TA>
+__global__ __launch_bounds__(256) void wkv_chunk_state_kernel(const TA* __restrict__ k, const TA* __restrict__ v, long ld,
+                                                              const float* __restrict__ z, const TA* __restrict__ w0,
+                                                              const int* __restrict__ cu_q,
+                                                              const int* __restrict__ positions, int H, int D, int nseq,
+                                                              int Lc, float* __restrict__ cs_loc,
+                                                              float* __restrict__ cs_dec) {
+  constexpr int TB = 64, LD = 80;                 // tokens of a block; a row: four of them fall into different banks
+  __shared__ float kk[TB][LD], vv[TB][LD], tot[4][64];
+  const int hd = blockIdx.y, nb = (D + 63) / 64, ib = blockIdx.z / nb, jb = blockIdx.z % nb;
+  const WkvChunk ck = wkv_find_chunk(blockIdx.x, cu_q, positions, nseq, Lc);
+  if (ck.s < 0 || ck.c == ck.n - 1) return;       // nothing follows a sequence's last chunk
+  const int a = cu_q[ck.s] + ck.c * Lc, b = a + Lc;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, g4 = lane >> 4;
+  const int i = 64 * ib + lane, j = 64 * jb + lane, HD = H * D;
+  const bool oni = i < D, onj = j < D;
+  const int ic = min(i, D - 1), jc = min(j, D - 1);
+  const float w0i = ldf(w0, (size_t)hd * D + ic);
+  float after = 1.f;                              // the decays behind this block
+  f32x4 acc[4];
 #pragma unroll
-      for (int e = 0; e < CH; ++e)
-        if (i0 + e < D) cs_dec[((size_t)blockIdx.x * H + hd) * D + i0 + e] = decp[e];
+  for (int n = 0; n < 4; ++n) acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int top = b; top > a; top -= TB) {
+    const int t0 = top - TB + 16 * wave;          // this wave's 16 tokens; those before the chunk count as nothing
+    float kx[16], wx[16], vx[16];
+    TA kr[16], vr[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {                // (loads at clamped places, all in flight; what is not there is dropped)
+      const int t = max(t0 + u, a);
+      kr[u] = k[(size_t)t * ld + (size_t)hd * D + ic];
+      vr[u] = v[(size_t)t * ld + (size_t)hd * D + jc];
+      wx[u] = z[(size_t)t * HD + (size_t)hd * D + ic];
     }
+    float run = 1.f;
+#pragma unroll
+    for (int u = 15; u >= 0; --u) {
+      const bool in = t0 + u >= a;
+      kx[u] = in && oni ? ldf(kr, u) * run : 0.f;
+      vx[u] = in && onj ? ldf(vr, u) : 0.f;
+      run *= in ? expf(-expf(wx[u] + w0i)) : 1.f;
+    }
+    __syncthreads();                              // the block before has been read
+    tot[wave][lane] = run;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) vv[16 * wave + u][lane] = vx[u];
+    __syncthreads();
+    float f = after;
+    for (int w = 3; w > wave; --w) f *= tot[w][lane];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) kk[16 * wave + u][lane] = kx[u] * f;
+    after *= (tot[3][lane] * tot[2][lane]) * (tot[1][lane] * tot[0][lane]);
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < TB / 4; ++s) {
+      const float x = kk[4 * s + g4][16 * wave + li];
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+        acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, vv[4 * s + g4][16 * n + li], acc[n], 0, 0, 0);
+    }
+  }   // acc[n][e] = loc[64 ib + 16 wave + 4 g4 + e][64 jb + 16 n + li]
+  const size_t rec = (size_t)blockIdx.x * H + hd;
+#pragma unroll
+  for (int n = 0; n < 4; ++n)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int x = 64 * ib + 16 * wave + 4 * g4 + e, y = 64 * jb + 16 * n + li;
+      if (x < D && y < D) cs_loc[rec * D * D + (size_t)x * D + y] = acc[n][e];
+    }
+  if (wave == 0 && jb == 0 && oni) cs_dec[rec * D + i] = after;
+}
+
+// Sums over the 4 lanes of a quad and the 64 of a wave, in all of them; up to 16 lanes by register moves, without LDS.
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float quad_sum(float v) { return dpp_add<0x4E>(dpp_add<0xB1>(v)); }   // lanes ^ 1, ^ 2
+__device__ __forceinline__ float row_sum(float v) { return dpp_add<0x140>(dpp_add<0x141>(quad_sum(v))); }   // mirrored
+
+// MODE 2 for heads of at most 64 channels: two waves per (chunk, head).  Lane 4 jg + ig of a wave holds the state's 16 x 2
+// block of key channels 16 ig .. and value channels 32 wave + 2 jg .., so a token's r, k and w come from LDS once per 32
+// elements (a column per lane, as above, reads them once per 16, waits for them and for two barriers in every token: 129 us
+// for 2048 tokens of 32 heads of 64, this 52 us).  8 tokens are staged at a time, 4 by each wave (lane = channel) and their
+// outputs finished by the same one; the next 8 load meanwhile.  Bound by the vector units: 200 multiply-adds per token and
+// head in the walk and about 100 instructions for the decays, gates and norm.  The bonus term is a scalar per token:
+// sum_i r_i u_i k_i v_j = (sum_i r_i u_i k_i) v_j.
+template <typename TA>
+__global__ __launch_bounds__(128, 2) void wkv_chunk_out_kernel(TA* __restrict__ out, const TA* __restrict__ r,
+                                                               const TA* __restrict__ k, const TA* __restrict__ v,
+                                                               const TA* __restrict__ g, long ld,
+                                                               const float* __restrict__ z, const TA* __restrict__ w0,
+                                                               const TA* __restrict__ u, const TA* __restrict__ lnw,
+                                                               float* __restrict__ state, const int* __restrict__ cu_q,
+                                                               const int* __restrict__ seq_slots,
+                                                               const int* __restrict__ positions, int H, int D, float eps,
+                                                               int nseq, int Lc, const float* __restrict__ cs_start) {
+  constexpr int TB = 8, TW = TB / 2;
+  __shared__ __attribute__((aligned(16))) float sr[TB][64], sk[TB][64], sw[TB][64], sv[TB][64], so[TB][64];
+  const int hd = blockIdx.y;
+  const WkvChunk ck = wkv_find_chunk(blockIdx.x, cu_q, positions, nseq, Lc);
+  if (ck.s < 0) return;
+  const int a = __builtin_amdgcn_readfirstlane(cu_q[ck.s] + ck.c * Lc);
+  const int b = __builtin_amdgcn_readfirstlane(min(cu_q[ck.s + 1], a + Lc));
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int ig = lane & 3, j0 = 32 * wave + 2 * (lane >> 2), HD = H * D;
+  const bool on = lane < D;
+  float* st = state + ((size_t)seq_slots[ck.s] * H + hd) * D * D;
+  const float* src = ck.n > 1 ? cs_start + ((size_t)blockIdx.x * H + hd) * D * D : st;
+  const bool from_zero = positions[a] == 0;
+  float S[16][2];
+#pragma unroll
+  for (int e = 0; e < 16; ++e)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int x = 16 * ig + e, y = j0 + q;
+      const float f = src[min(x, D - 1) * D + min(y, D - 1)];
+      S[e][q] = !from_zero && x < D && y < D ? f : 0.f;
+    }
+  const size_t h0 = (size_t)hd * D;
+  const unsigned lc = min(lane, D - 1);
+  const float uj = ldf(u + h0, lc), w0j = ldf(w0 + h0, lc), lnj = ldf(lnw + h0, lc);
+  TA nr[TW], nk[TW], nv[TW], ng[TW];              // the next tokens as they come: converted only once they are staged
+  float nz[TW];
+  auto fetch = [&](int t0) {
+#pragma unroll
+    for (int x = 0; x < TW; ++x) {                // (at clamped places: every load in flight)
+      const int t = min(t0 + TW * wave + x, b - 1);
+      const size_t base = (size_t)t * ld + h0;
+      nr[x] = (r + base)[lc];
+      nk[x] = (k + base)[lc];
+      nv[x] = (v + base)[lc];
+      ng[x] = (g + base)[lc];
+      nz[x] = (z + (size_t)t * HD + h0)[lc];
+    }
+  };
+  fetch(a);
+  for (int t0 = a; t0 < b; t0 += TB) {
+    const int tw = t0 + TW * wave;                // this wave's first token
+    float bonus[TW], cv[TW], cg[TW];
+#pragma unroll
+    for (int x = 0; x < TW; ++x) {                // a token or channel that is not there: k = r = 0, w = 1
+      const bool in = on && tw + x < b;
+      const float rx = in ? ldf(nr, x) : 0.f, kx = in ? ldf(nk, x) : 0.f, w = expf(-expf(nz[x] + w0j));
+      cv[x] = in ? ldf(nv, x) : 0.f;
+      cg[x] = ldf(ng, x);
+      bonus[x] = row_sum(rx * (uj * kx));
+      sr[TW * wave + x][lane] = rx;
+      sk[TW * wave + x][lane] = kx;
+      sv[TW * wave + x][lane] = cv[x];
+      sw[TW * wave + x][lane] = in ? w : 1.f;
+    }
+    if (t0 + TB < b) fetch(t0 + TB);
+    lds_barrier();
+    // a step: 4 of the 16 key channels of a token; its rows are read two steps ahead
+    f32x4 r4[3], k4[3], w4[3];
+    typedef __attribute__((ext_vector_type(2))) float f32x2;
+    f32x2 v2[2];
+    auto rows = [&](int step) {
+      const int x = step >> 2, c = 16 * ig + 4 * (step & 3);
+      if ((step & 3) == 0) v2[x & 1] = *reinterpret_cast<const f32x2*>(&sv[x][j0]);
+      r4[step % 3] = *reinterpret_cast<const f32x4*>(&sr[x][c]);
+      k4[step % 3] = *reinterpret_cast<const f32x4*>(&sk[x][c]);
+      w4[step % 3] = *reinterpret_cast<const f32x4*>(&sw[x][c]);
+    };
+    rows(0);
+    rows(1);
+    float o[2][2];                                // even and odd key channels: two chains per value channel
+#pragma unroll
+    for (int step = 0; step < 4 * TB; ++step) {
+      const int x = step >> 2, e0 = 4 * (step & 3), n = step % 3;
+      if (step + 2 < 4 * TB) rows(step + 2);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          float& acc = o[e & 1][q];
+          acc = e0 + e < 2 ? r4[n][e] * S[e][q] : fmaf(r4[n][e], S[e0 + e][q], acc);
+          S[e0 + e][q] = fmaf(w4[n][e], S[e0 + e][q], k4[n][e] * v2[x & 1][q]);
+        }
+      if (e0 == 12) {
+        const float y0 = quad_sum(o[0][0] + o[1][0]), y1 = quad_sum(o[0][1] + o[1][1]);
+        if (ig < 2) so[x][j0 + ig] = ig == 0 ? y0 : y1;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int m = 32; m > 8; m >>= 1)
+#pragma unroll
+      for (int x = 0; x < TW; ++x) bonus[x] += __shfl_xor(bonus[x], m, WAVE);
+    lds_barrier();
+    float y[TW], ss[TW];
+#pragma unroll
+    for (int x = 0; x < TW; ++x) {
+      y[x] = on ? fmaf(bonus[x], cv[x], so[TW * wave + x][lane]) : 0.f;
+      ss[x] = row_sum(y[x] * y[x]);
+    }
+#pragma unroll
+    for (int m = 32; m > 8; m >>= 1)
+#pragma unroll
+      for (int x = 0; x < TW; ++x) ss[x] += __shfl_xor(ss[x], m, WAVE);
+#pragma unroll
+    for (int x = 0; x < TW; ++x) {                // o / rms * lnw * silu(g), one division
+      y[x] = y[x] * lnj * cg[x] / (sqrtf(ss[x] / (float)D + eps) * (1.f + expf(-cg[x])));
+      if (on && tw + x < b) stf(out + (size_t)(tw + x) * HD + h0, lane, y[x]);
+    }
+  }
+  if (ck.c == ck.n - 1) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int x = 16 * ig + e, y = j0 + q;
+        if (x < D && y < D) st[(size_t)x * D + y] = S[e][q];
+      }
   }
 }
 
 // start[first chunk + c + 1] = dec[c] * start[c] + loc[c] along a sequence's chunks; start of chunk 0 is the slot's state
-// (or zero at position 0) and is read by the MODE 2 pass directly.  Workgroups (sequence, head, 256 state elements), a
+// (or zero at position 0), copied here: the pass that reads it runs beside the one that replaces the slot's.  Workgroups (sequence, head, 256 state elements), a
 // thread per element with 8 chunks' records in flight: 2048 tokens, 32 heads of 64 x 64, 131 us with one workgroup per head
-// and a load waited for in every step, 17 us now (33 MB read and written: 4 us at 8 TB/s each way, the rest latency).
+// and a load waited for in every step, 15 us now (33 MB read and written: 4 us at 8 TB/s each way, the rest latency).
 __global__ __launch_bounds__(256) void wkv_prefix_kernel(float* __restrict__ cs_start, const float* __restrict__ cs_loc,
                                                          const float* __restrict__ cs_dec, const float* __restrict__ state,
                                                          const int* __restrict__ cu_q, const int* __restrict__ seq_slots,
@@ -244,6 +451,7 @@ __global__ __launch_bounds__(256) void wkv_prefix_kernel(float* __restrict__ cs_
   if (n < 1) return;
   const int i = e / D;
   float S = positions[a] == 0 ? 0.f : state[((size_t)seq_slots[s] * H + hd) * D * D + e];
+  cs_start[((size_t)first * H + hd) * D * D + e] = S;
   constexpr int PF = 8;
   for (int c0 = 0; c0 < n; c0 += PF) {
     float dec[PF], loc[PF];
@@ -728,25 +936,43 @@ extern "C" int k8s_wkv_scan(void* out, const void* r, const void* k, const void*
   if (H <= 0 || D <= 0 || D > 128 || H > 65535) return -1;
   constexpr int CH = 16;
   const dim3 block((D + 63) / 64 * 64, (D + CH - 1) / CH);
-#define K8S_WKV(TA, MODE, GX, LOC, DEC, START)                                                                        \
+#define K8S_WKV(TA, MODE, GX, START)                                                                                  \
   wkv_scan_kernel<TA, CH, MODE><<<dim3(GX, H), block, 0, s>>>((TA*)out, (const TA*)r, (const TA*)k, (const TA*)v,      \
                                                               (const TA*)g, ld, z, (const TA*)w0, (const TA*)u,        \
                                                               (const TA*)lnw, state, cu_q, seq_slots, positions, H, D, \
-                                                              eps, nseq, Lc, LOC, DEC, START)
+                                                              eps, nseq, Lc, START)
   if (Lc <= 0 || ws == nullptr) {
-    if (f32) K8S_WKV(float, 0, nseq, nullptr, nullptr, nullptr);
-    else K8S_WKV(bf16_t, 0, nseq, nullptr, nullptr, nullptr);
+    if (f32) K8S_WKV(float, 0, nseq, nullptr);
+    else K8S_WKV(bf16_t, 0, nseq, nullptr);
     return (int)hipGetLastError();
   }
-  const int chunks = (T + Lc - 1) / Lc + nseq;
+  const int chunks = (T + Lc - 1) / Lc + nseq, nb = (D + 63) / 64;
   float* loc = ws;
   float* start = ws + (size_t)chunks * H * D * D;
   float* dec = start + (size_t)chunks * H * D * D;
-  if (f32) K8S_WKV(float, 1, chunks, loc, dec, nullptr);
-  else K8S_WKV(bf16_t, 1, chunks, loc, dec, nullptr);
+  if (f32)
+    wkv_chunk_state_kernel<float><<<dim3(chunks, H, nb * nb), 256, 0, s>>>((const float*)k, (const float*)v, ld, z,
+                                                                           (const float*)w0, cu_q, positions, H, D, nseq,
+                                                                           Lc, loc, dec);
+  else
+    wkv_chunk_state_kernel<bf16_t><<<dim3(chunks, H, nb * nb), 256, 0, s>>>((const bf16_t*)k, (const bf16_t*)v, ld, z,
+                                                                            (const bf16_t*)w0, cu_q, positions, H, D,
+                                                                            nseq, Lc, loc, dec);
   wkv_prefix_kernel<<<dim3(nseq, H, (D * D + 255) / 256), 256, 0, s>>>(start, loc, dec, state, cu_q, seq_slots, positions, H, D, Lc);
-  if (f32) K8S_WKV(float, 2, chunks, nullptr, nullptr, start);
-  else K8S_WKV(bf16_t, 2, chunks, nullptr, nullptr, start);
+#define K8S_WKVO(TA)                                                                                                   \
+  wkv_chunk_out_kernel<TA><<<dim3(chunks, H), 128, 0, s>>>((TA*)out, (const TA*)r, (const TA*)k, (const TA*)v,           \
+                                                          (const TA*)g, ld, z, (const TA*)w0, (const TA*)u,             \
+                                                          (const TA*)lnw, state, cu_q, seq_slots, positions, H, D, eps, \
+                                                          nseq, Lc, start)
+  if (D <= 64) {
+    if (f32) K8S_WKVO(float);
+    else K8S_WKVO(bf16_t);
+  } else if (f32) {
+    K8S_WKV(float, 2, chunks, start);
+  } else {
+    K8S_WKV(bf16_t, 2, chunks, start);
+  }
+#undef K8S_WKVO
 #undef K8S_WKV
   return (int)hipGetLastError();
 }

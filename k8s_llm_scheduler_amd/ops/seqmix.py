@@ -434,10 +434,19 @@ def wkv_max_dim() -> int:
     return 128
 
 
-# Batches of at least WKV_CHUNK_MIN tokens run the recurrence as three passes over chunks of WKV_CHUNK tokens (parallel
-# over chunks); shorter ones (decoding, short portions) as one workgroup per sequence.
-WKV_CHUNK = int(os.environ.get("K8S_WKV_CHUNK", "64"))
-WKV_CHUNK_MIN = int(os.environ.get("K8S_WKV_CHUNK_MIN", "256"))
+WKV_CHUNK = int(os.environ.get("K8S_WKV_CHUNK", "0"))            # > 0: chunks of that many tokens
+WKV_CHUNK_MIN = int(os.environ.get("K8S_WKV_CHUNK_MIN", "0"))    # > 0: from that many tokens on
+
+
+def wkv_chunk(T: int, nseq: int, H: int) -> int:
+    """Tokens of a chunk where the recurrence runs as three passes over chunks (parallel over them), 0 where a workgroup walks
+    each sequence alone (decoding, very short portions).  The walk takes 1.4 us a token of the longest sequence, the passes
+    about 20 us and more with the batch: (heads of 64) one sequence of 32 tokens 48 / 22 us, 8 of 32 49 / 37 us, 16 of 32
+    52 / 65 us, 16 of 64 102 / 91 us -- from 256 tokens or 32 a sequence on.  Chunks of 64, of 32 while those would leave
+    CUs without two workgroups (512 tokens of 32 heads: 46 / 56 us; 2048: 109 / 78 us)."""
+    if T < (WKV_CHUNK_MIN or min(256, 32 * nseq)):
+        return 0
+    return WKV_CHUNK or (64 if (-(-T // 64) + nseq) * H >= 512 else 32)
 
 
 def wkv_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, z: torch.Tensor, w0: torch.Tensor,
@@ -458,7 +467,7 @@ def wkv_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
             raise ValueError("wkv_scan: r, k, v, g must share dtype and row stride")
     out = torch.empty(T, H * D, dtype=r.dtype, device=r.device)
     nseq = cu_q.shape[0] - 1
-    Lc = (WKV_CHUNK if T >= WKV_CHUNK_MIN else 0) if chunk is None else int(chunk)
+    Lc = wkv_chunk(T, nseq, H) if chunk is None else int(chunk)
     ws = torch.empty(_native().wkv_workspace(T, nseq, H, D, Lc), dtype=F32, device=r.device) if Lc > 0 else None
     _native().wkv_scan(out.data_ptr(), r.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), ld, _p(z),
                        _p(w0, r.dtype, "w0"), _p(u, r.dtype, "u"), _p(lnw, r.dtype, "lnw"), _p(state),

@@ -274,7 +274,8 @@ def test_recurrence_prefix_over_many_chunks():
     """More chunks than the prefix keeps in flight, head sizes that do not fill its workgroups, a resumed sequence beside a
     new one: chunked against one workgroup per sequence."""
     g = torch.Generator().manual_seed(5)
-    for H, D, lens, first in ((2, 64, (700, 129), (0, 33)), (1, 40, (1, 900), (7, 0))):
+    for H, D, lens, first in ((2, 64, (700, 129), (0, 33)), (1, 40, (1, 900), (7, 0)), (1, 128, (65, 300), (9, 1)),
+                              (3, 17, (64, 128), (2, 0))):
         T = sum(lens)
         r, k, v, gate = (torch.randn(T, H * D, generator=g).to(DEV) for _ in range(4))
         z, w0, u, lnw = (torch.randn(T, H * D, generator=g).to(DEV), *(torch.randn(H * D, generator=g).to(DEV) for _ in range(3)))
@@ -283,7 +284,7 @@ def test_recurrence_prefix_over_many_chunks():
         pos = torch.cat([torch.arange(p, p + n) for p, n in zip(first, lens)]).to(torch.int32).to(DEV)
         slots = torch.tensor([1, 0], dtype=torch.int32, device=DEV)
         outs = []
-        for chunk in (0, 16, 64):
+        for chunk in (0, 16, 64, 67, 150):
             s = st.clone()
             y = sm.wkv_scan(r, k, v, gate, z, w0, u, lnw, s, cu, slots, pos, H, D, 1e-6, chunk=chunk)
             outs.append((y, s))
