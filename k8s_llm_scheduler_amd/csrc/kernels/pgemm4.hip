@@ -75,8 +75,10 @@ struct P4Args {
   const bf16_t* bias;    // P4_GLU, optional: [gate; up] biases
   // grouped form: group g's rows are [seg[g], seg[g + 1]) of a compact row space (row r of x: a_rows[r], or r) and its
   // weights W + g wstride bytes; m_tiles bounds the groups' row tiles.  8 experts, 3068 rows, K = 2048: gate / up with its
-  // activation (N = 2 x 2048) 94 us, down (N = 2048) 47 us; 140 and 10 us, and 78 us on the 64-row tiles of stream32.hip
+  // activation (N = 2 x 2048) 94 us, down (N = 2048) 47 us; 140 and 10 us, and 78 us on the 64-row tiles of stream32.hip.
+  // seg == nullptr: groups of gsize rows (products of several inputs with a weight each in one launch)
   const int* seg;
+  int gsize;
   const int* a_rows;
   long long wstride;
   int groups;
@@ -106,9 +108,10 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
 
   // ---- block -> (tile, k-slice)
   int nwg = a.nwg, m_tiles = a.m_tiles;
+  auto first = [&](int e) { return a.seg != nullptr ? a.seg[e] : e * a.gsize; };   // group e's first row
   if constexpr (GRP) {     // the launch covers an upper bound: spread the tiles there are over the XCDs
     m_tiles = 0;
-    for (int e = 0; e < a.groups; ++e) m_tiles += (a.seg[e + 1] - a.seg[e] + BQ - 1) / BQ;
+    for (int e = 0; e < a.groups; ++e) m_tiles += (first(e + 1) - first(e) + BQ - 1) / BQ;
     nwg = m_tiles * a.n_tiles;
     if ((int)blockIdx.x >= nwg) return;
   }
@@ -128,12 +131,12 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
   if constexpr (GRP) {
     int gi = 0, left = mt;                           // mt < m_tiles: a group is found
     for (;; ++gi) {
-      const int nt_g = (a.seg[gi + 1] - a.seg[gi] + BQ - 1) / BQ;
+      const int nt_g = (first(gi + 1) - first(gi) + BQ - 1) / BQ;
       if (left < nt_g) break;
       left -= nt_g;
     }
-    m0 = a.seg[gi] + left * BQ;
-    m_end = a.seg[gi + 1];
+    m0 = first(gi) + left * BQ;
+    m_end = first(gi + 1);
     Wb += (long long)gi * a.wstride;
   }
   auto xrow = [&](int r) -> uint32_t {               // row r of the tile, past the end its last one
@@ -826,7 +829,7 @@ extern "C" int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M
   const bool pair = kind >= 0;
   if (kind < -1 || (pair && kind > 1 && kind != 5)) return -1;
   if (rows <= 0) return 0;
-  if (M <= 0 || N_out <= 0 || N_out % 4 || K <= 0 || K % 64 || groups <= 0 || seg == nullptr || (cfg != 1 && cfg != 3)) return -1;
+  if (M <= 0 || N_out <= 0 || N_out % 4 || K <= 0 || K % 64 || groups <= 0 || (seg == nullptr && rows % groups) || (cfg != 1 && cfg != 3)) return -1;
   if (ldx < K || ldx % 8 || (((uintptr_t)x | (uintptr_t)W) & 15) || ((uintptr_t)out & 7)) return -1;
   const long long kbytes = (long long)K * 2, wrows = (pair ? 2LL : 1LL) * N_out;
   if (wrows * kbytes >= (1LL << 32) || (long long)M * ldx * 2 >= (1LL << 32)) return -5;   // 32-bit DMA offsets
@@ -837,6 +840,7 @@ extern "C" int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M
   a.nwg = a.m_tiles * a.n_tiles;
   a.xbytes = (uint32_t)(ldx * 2);
   a.seg = seg;
+  a.gsize = rows / groups;
   a.a_rows = a_rows;
   a.wstride = wrows * kbytes;
   a.groups = groups;

@@ -441,10 +441,7 @@ class PutulornModel(StreamModel):
         m = w.cfg
         S, shift = self.states[run.cache]
         mix = sm.token_shift(h, w.mu, shift, b["cu_q"], b["tok_seq"], b["seq_slots"], b["positions"], save=True)   # [5, T, W]
-        if sm.FAST_GEMM and h.is_cuda and sm._route_fast(mix[0], w.w_rkvg[0], self.dtype):
-            r, k, v, g = (sm.linear(mix[i], w.w_rkvg[i]) for i in range(4))
-        else:
-            r, k, v, g = sm.gemm(mix[:4], w.w_rkvg).unbind(0)
+        r, k, v, g = sm.linear_each(mix[:4], w.w_rkvg)
         lo = sm.linear_act(mix[4], w.w1, sm.ACT_TANH)
         z = sm.linear(lo, w.w2, out_dtype=torch.float32)                  # decay logits stay fp32
         y = sm.wkv_scan(r, k, v, g, z, w.w0, w.u, w.lnw, S, b["cu_q"], b["seq_slots"], b["positions"], m.heads, m.dim,

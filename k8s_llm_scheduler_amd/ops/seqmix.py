@@ -349,12 +349,13 @@ def _grouped_big(a: torch.Tensor, w: torch.Tensor, seg: Optional[torch.Tensor], 
             and w.shape[1] * K * 2 < 1 << 32 and a.shape[0] * a.stride(0) * 2 < 1 << 32)
 
 
-def _grouped_cfg(rows: int, E: int, N: int, K: int, pair: bool) -> int:
+def _grouped_cfg(rows: int, E: int, N: int, K: int, pair: bool, even: bool = False) -> int:
     """Configuration of the grouped big-tile product: 256 (1) or 128 (3) weight rows per tile by the time its rounds of tiles
-    over the CUs take (us, fitted to the products above and to N = 3584 / 4096, K = 3584 / 4096), groups of about equal
-    size drawn at random."""
+    over the CUs take (us, fitted to the products above and to N = 3584 / 4096, K = 3584 / 4096), groups of the same size
+    (``even``) or of about equal size drawn at random."""
     r = rows / E
-    tiles = E * sum(0.5 + 0.5 * math.erf((r - 128 * k) / math.sqrt(2.0 * max(r, 1.0))) for k in range(1, int(r / 128) + 2)) + E
+    tiles = E * -(-rows // E // 128) if even else E + E * sum(
+        0.5 + 0.5 * math.erf((r - 128 * k) / math.sqrt(2.0 * max(r, 1.0))) for k in range(1, int(r / 128) + 2))
     n, kt = (2 * N if pair else N), K / 64
     big = 10.0 + math.ceil(tiles * -(-n // 256) / 256) * (kt + (12.0 if pair else 0.0))
     small = 20.0 + math.ceil(tiles * -(-n // 128) / 256) * 0.56 * kt
@@ -365,9 +366,37 @@ def _pgemm4_grouped(a, w, a_rows, rows: int, seg, N: int, kind: int = -1, limit:
     E, _, K = w.shape
     out = torch.empty(rows, N, dtype=BF16, device=a.device)
     _native().pgemm4_grouped(out.data_ptr(), a.data_ptr(), w.data_ptr(), a.shape[0], rows, N, K, E, _p(seg, I32, "seg"),
-                             _p(a_rows, I32, "a_rows"), a.stride(0), _grouped_cfg(rows, E, N, K, kind >= 0), 4, kind,
+                             _p(a_rows, I32, "a_rows"), a.stride(0), _grouped_cfg(rows, E, N, K, kind >= 0, seg is None), 4, kind,
                              float(limit), float(alpha), -1)
     return out
+
+
+def linear_each(a: torch.Tensor, w: torch.Tensor):
+    """[a[i] @ w[i].T]: several inputs, a weight each (a [G, M, K], w [G, N, K]) -> G tensors [M, N] of one row stride.  One
+    launch where that is faster than G of :func:`linear`.  4 weights of 2048 x 2048, M = 8 / 64 / 128 / 512 / 1024 / 2048: the
+    any-shape kernel (k shared by the waves while its tiles are few) 11 / 24 / 38 / 52 / 77 / 139 us, the grouped big tiles
+    27 / 29 / 30 / 31 / 45 / 80, four launches 22 / 39 / 47 / 76 / 109 / 114; of 4096 x 4096, M = 16 / 32 / 64 / 512 / 2048:
+    70 / 71 / 73 / 136 / 472, 53 / 54 / 55 / 81 / 288, 39 / 54 / 71 / 135 / 300 (beyond, a launch's own tiles fill the card
+    and its deeper stages win)."""
+    G, M, K = a.shape
+    N = w.shape[1]
+    if not (FAST_GEMM and _gpu(a, w) and _route_fast(a[0], w[0], a.dtype)):
+        return gemm(a, w).unbind(0)
+    if _each_once(a, w):
+        if G * (-(-M // 64)) * (-(-N // 64)) <= 128:
+            return gemm(a, w).unbind(0)
+        if 32 < M <= 2048:
+            return _pgemm4_grouped(a.view(G * M, K), w, None, G * M, None, N).view(G, M, N).unbind(0)
+    return tuple(linear(a[i], w[i]) for i in range(G))
+
+
+def _each_once(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether products of several inputs may share a launch: the routing is free, sizes and places fit the big tiles."""
+    from . import GEMM_BACKEND
+
+    G, M, K = a.shape
+    return (GEMM_BACKEND == "auto" and a.is_contiguous() and w.is_contiguous() and G <= GROUP_BIG_MAX_GROUPS
+            and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.shape[1] * K * 2 < 1 << 32 and G * M * K * 2 < 1 << 32)
 
 
 def gemm_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, alpha: float = 1.0, *,

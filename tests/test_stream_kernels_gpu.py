@@ -344,3 +344,16 @@ def test_prompt_attention_key_splits(H, G, D, kw, ns, monkeypatch):
                                         sinks=torch.linspace(-3, 3, H, device=DEV), slopes=slopes).float())
     assert (outs[1][pos < 0] == 0).all()
     assert ((outs[1] - outs[0]).abs() <= 2.0 ** -7 * outs[0].abs() + 2.0 ** -13 * outs[0].abs().max()).all()
+
+
+@pytest.mark.parametrize("M", [1, 32, 33, 64, 127, 129, 1031, 2048, 2049])
+@pytest.mark.parametrize("N,K", [(2048, 256), (1040, 512), (4096, 192)])
+def test_products_of_several_inputs(M, N, K):
+    """Every way a launch is shared: few tiles, even groups of the big tiles with remainders, one launch per input."""
+    g = torch.Generator().manual_seed(M + N)
+    a, w = (torch.randn(3, n, K, generator=g).to(torch.bfloat16) for n in (M, N))
+    got = sm.linear_each(a.to(DEV), w.to(DEV))
+    assert len({t.stride(0) for t in got}) == 1
+    for x, y, z in zip(a, w, got):
+        exact = x.double() @ y.double().T
+        assert ((z.cpu().double() - exact).abs() <= sum_bound(x, y) + 2.0 ** -8 * exact.abs()).all()
