@@ -255,6 +255,32 @@ def test_linear_act(M, N, K, kind, bias):
     assert ((got.double() - want).abs() <= 2.0 ** -6 * want.abs() + 4e-2).all()
 
 
+@pytest.mark.parametrize("tokens,top,E,N,K", [(1, 1, 3, 130, 64), (5, 2, 3, 15, 128), (48, 2, 8, 72, 320), (100, 1, 2, 33, 2048)])
+@pytest.mark.parametrize("kind", KINDS)
+def test_few_rows_gated(tokens, top, E, N, K, kind):
+    """Tiles of at most 16 and of up to 64 rows, columns that do not fill 16, gathered rows with a stride: one rounding."""
+    g = torch.Generator().manual_seed(tokens + N + K)
+    idx = torch.rand(tokens, E, generator=g).argsort(1)[:, :top].to(torch.int32)
+    rows, pos, seg, tiles = sm.moe_align(idx.to(DEV), E)
+    h = torch.randn(tokens, K + 8, generator=g).to(torch.bfloat16).to(DEV)[:, :K]
+    w = (torch.randn(E, 2 * N, K, generator=g) * 2 / K ** 0.5).to(torch.bfloat16).to(DEV)
+    got = sm.gemm_act(h, w, kind, 1.5, 1.702, a_rows=rows, tiles=tiles, rows=tokens * top).double()[pos.long()]
+    for c in range(top):
+        z = (h.double().unsqueeze(1) @ w.double()[idx[:, c].long().to(DEV)].transpose(1, 2)).squeeze(1)
+        want = act64(z, kind, 1.5, 1.702)
+        assert ((got.view(tokens, top, N)[:, c] - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16, 64), (16, 130, 128), (17, 100, 64), (200, 33, 320)])
+@pytest.mark.parametrize("kind", [k for k in ELEMENTWISE if k != sm.ACT_SOFTCAP])
+def test_few_tiles_elementwise(M, N, K, kind):
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K + 8, generator=g).to(torch.bfloat16).to(DEV)[:, 8:]
+    w = (torch.randn(N, K, generator=g) * 2 / K ** 0.5).to(torch.bfloat16).to(DEV)
+    want = act64(x.double() @ w.double().T, kind, 0.0, 1.0)
+    assert ((sm.linear_act(x, w, kind).double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 64), (16, 130, 128), (17, 100, 64), (64, 15, 1024), (65, 128, 2048), (200, 33, 320),
                                    (2048, 128, 192)])
 @pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
