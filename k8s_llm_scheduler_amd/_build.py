@@ -33,9 +33,9 @@ CSRC = PKG / "csrc"
 BUILD = PKG.parent / "build" / "native"
 ARCH = os.environ.get("K8S_HIP_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-# Kernels added since the packed-fp32 rule are built without the packed fp32 instructions (v_pk_add/mul/fma_f32), which
-# -O3 otherwise forms from ordinary float code.  The older kernel files keep the flags they were validated with: with
-# the option on every file, the two-rank fused GEMV all-reduce check of tests/test_multigpu.py reported a wrong sum.
+# Kernels added since the packed-fp32 rule, and pgemm4.hip with its activation epilogues, are built without the packed fp32
+# instructions (v_pk_add/mul/fma_f32), which -O3 otherwise forms from ordinary float code.  The other kernel files keep the
+# flags they were validated with: with the option on every file, the two-rank fused GEMV all-reduce check of tests/test_multigpu.py reported a wrong sum.
 NO_PACKED_FP32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 NO_PACKED_FP32_FILES = {"stream32.hip", "mixers.hip", "latent_prompt.hip", "latent_token.hip", "moe.hip",
                         "window_attn.hip", "gated_scan.hip", "delta_scan.hip", "decay_scan.hip", "pgemm4.hip"}

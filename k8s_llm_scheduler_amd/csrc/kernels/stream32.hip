@@ -1097,7 +1097,7 @@ extern "C" int k8s_gemm_any(void* C, const void* A, const void* W, int M, int N,
     return (int)hipGetLastError();
   }
   // at most 128 tiles of 64 x 64: 16 columns per workgroup and k shared by its waves (8 x 128 x 2048: 26.8 us on two tiles,
-  // 4.5 us; 2048 x 128 x 2048: 36 us on 64 tiles, 12 us; from 256 tiles on the tiles are faster)
+  // 4.8 us; 2048 x 128 x 2048: 36 us on 64 tiles, 14.3 us; at 256 tiles both take the same)
   if (vec && tiles == nullptr && K % 64 == 0 && (long)gy * ((N + 63) / 64) * batch <= 128) {
     const dim3 gn((N + 15) / 16, gy, batch);
     if (out_f32) gemm_narrow_kernel<float, FEW_NONE><<<gn, 256, 0, s>>>((float*)C, (const bf16_t*)A, (const bf16_t*)W, M, N, K, lda,
