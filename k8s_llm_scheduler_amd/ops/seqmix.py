@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import math
 import os
+import sys
 from typing import Optional
 
 import torch
@@ -27,17 +28,23 @@ BF16, F32, I32 = torch.bfloat16, torch.float32, torch.int32
 GROUP_BM = 64   # row-tile height of the grouped GEMM (gemm_any_kernel's BM)
 
 
-def _native():
-    from . import native
+# Short prompts are bound by their launches' preparation here: an import statement in a function costs about 1 us of every
+# call (97 tokens, 104 launches: 1475 us of preparation with them, 1396 us).
+_ops = sys.modules[__package__]
 
-    return native()
+
+def _native():
+    return _ops.native()
 
 
 def _gpu(*ts) -> bool:
-    cuda = [t.is_cuda for t in ts if t is not None]
-    if any(cuda) and not all(cuda):
-        raise ValueError("mixed CPU/GPU tensors")
-    return bool(cuda) and cuda[0]
+    cuda = None
+    for t in ts:
+        if t is not None and t.is_cuda is not cuda:
+            if cuda is not None:
+                raise ValueError("mixed CPU/GPU tensors")
+            cuda = t.is_cuda
+    return bool(cuda)
 
 
 def _p(t: Optional[torch.Tensor], dtype=None, name: str = "tensor") -> int:
@@ -246,13 +253,11 @@ def _route_fast(a: torch.Tensor, w: torch.Tensor, out_dtype) -> bool:
     """bf16 products of production size whose shape the framework's tuned GEMV / MFMA GEMM kernels take (128-byte
     k steps, N % 16 == 0, at least 1024 x 512 weights: the sizes their plan tables and heuristics were tuned and
     tested on).  Smaller products are launch-bound and stay on the any-shape kernel."""
-    from . import GEMM_BACKEND, LEAN
-
-    if LEAN:
+    if _ops.LEAN:
         return False
     if a.dtype != BF16 or w.dtype != BF16 or out_dtype not in (BF16, F32) or a.dim() != 2 or w.dim() != 2:
         return False
-    if GEMM_BACKEND == "library" or not a.is_contiguous() or not w.is_contiguous():
+    if _ops.GEMM_BACKEND == "library" or not a.is_contiguous() or not w.is_contiguous():
         return False
     N, K = w.shape
     return K % 64 == 0 and N % 16 == 0 and K * N >= 512 * 1024 and K >= 128 and N >= 128
@@ -269,11 +274,9 @@ def linear(a: torch.Tensor, w: torch.Tensor, out_dtype=None) -> torch.Tensor:
     if not _gpu(a, w):
         return ref.gemm_any(a, w, out_dtype)
     if FAST_GEMM and _route_fast(a, w, out_dtype):
-        from . import NoKernelForShape, linear as tuned
-
         try:
-            return tuned(a, w, out_dtype=F32 if out_dtype == F32 else None)
-        except NoKernelForShape:
+            return _ops.linear(a, w, out_dtype=F32 if out_dtype == F32 else None)
+        except _ops.NoKernelForShape:
             pass
     return gemm(a, w, out_dtype)
 
@@ -340,10 +343,8 @@ GROUP_BIG_MAX_GROUPS = 64        # every workgroup walks the groups' offsets
 
 
 def _grouped_big(a: torch.Tensor, w: torch.Tensor, seg: Optional[torch.Tensor], rows: int, N: int) -> bool:
-    from . import LEAN
-
     E, _, K = w.shape
-    return (not LEAN and FAST_GEMM and a.dtype == BF16 and seg is not None and seg.is_cuda and E <= GROUP_BIG_MAX_GROUPS
+    return (not _ops.LEAN and FAST_GEMM and a.dtype == BF16 and seg is not None and seg.is_cuda and E <= GROUP_BIG_MAX_GROUPS
             and rows >= GROUP_BIG_MIN * E and K % 64 == 0 and N % 4 == 0 and N >= 128 and a.stride(0) % 8 == 0
             and a.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0
             and w.shape[1] * K * 2 < 1 << 32 and a.shape[0] * a.stride(0) * 2 < 1 << 32)
@@ -399,10 +400,8 @@ def linear_each(a: torch.Tensor, w: torch.Tensor):
 
 def _each_once(a: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether products of several inputs may share a launch: the routing is free, sizes and places fit the big tiles."""
-    from . import GEMM_BACKEND
-
     G, M, K = a.shape
-    return (GEMM_BACKEND == "auto" and a.is_contiguous() and w.is_contiguous() and G <= GROUP_BIG_MAX_GROUPS
+    return (_ops.GEMM_BACKEND == "auto" and a.is_contiguous() and w.is_contiguous() and G <= GROUP_BIG_MAX_GROUPS
             and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.shape[1] * K * 2 < 1 << 32 and G * M * K * 2 < 1 << 32)
 
 
@@ -433,10 +432,8 @@ def linear_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, 
     pass over the product (2048 x 2 x 8192, gated: 22 us; 2048 x 8192 elementwise: 15 us) and its rounding."""
     pair = kind in (ACT_GELU_TANH, ACT_SWISH_CLAMP, ACT_RELU)
     if (pair or kind == ACT_RELU2) and FAST_GEMM and _gpu(a, w, bias) and _route_fast(a, w, BF16) and a.dtype == BF16 and (not pair or w.shape[0] % 8 == 0):
-        from . import EPI_BF16, gemm_route
-
         M, K = a.shape
-        kern, plan = gemm_route(M, w.shape[0], K, EPI_BF16, False) if M >= 129 else ("", None)
+        kern, plan = _ops.gemm_route(M, w.shape[0], K, _ops.EPI_BF16, False) if M >= 129 else ("", None)
         if kern == "pgemm4" and plan[1] == 1 and plan[0] in (1, 2, 3, 4) and a.data_ptr() % 16 == 0 and \
                 (bias is None or (pair and bias.dtype == BF16 and bias.numel() == w.shape[0] and bias.data_ptr() % 8 == 0)):
             N = w.shape[0] // 2 if pair else w.shape[0]
