@@ -734,7 +734,7 @@ __global__ __launch_bounds__(256) void window_attention_mfma_kernel(
 //   * where the tiles are few (a short portion behind a long cached one), nsplit workgroups share a tile's steps and leave
 //     (max, sum, unnormalised sum) for window_merge_kernel: a step is a chain of LDS and shuffle latencies of about 2.5 us
 //     however few workgroups run.  16 query heads over 4 of 128, 97 tokens behind 1000: 46.6 us in
-//     one piece, 23.3 us in 8 with the merge.  (A template flag: the arithmetic of the splits costs the whole walk 8%.)
+//     one piece, 22.9 us in 6 with the merge.  (A template flag: the arithmetic of the splits costs the whole walk 8%.)
 template <int DK, int DV, int NCB, bool SPLIT>
 __global__ __launch_bounds__(512) void window_prompt_kernel(
     bf16_t* __restrict__ out, float* __restrict__ pacc, float* __restrict__ pml, const bf16_t* __restrict__ q, long ldq,

@@ -858,9 +858,10 @@ def token_splits(T: int, G: int, keys: int) -> int:
 
 def prompt_splits(groups: int, keys: int) -> int:
     """Key splits of the prompt kernel's ``groups`` workgroups: up to 256 (one per CU: 40 workgroups, 300 tokens behind 1000,
-    6 splits 30 us, 8 splits 40 us), of two 64-key steps at least, at most 8 (1000 keys, 16 workgroups: 8 splits 23 us, 16
-    splits 26 us, the more the merge reads)."""
-    return max(1, min(256 // max(1, groups), -(-max(1, keys) // 128), 8))
+    6 splits 30 us, 8 splits 40 us), of two 64-key steps at least, at most 6 (16 workgroups, 97 tokens behind 1000: 1 split 46.2
+    us, 4 24.8, 6 22.9, 8 23.3, 16 25.6, the more the merge reads).  How many keys there are is only known on the device: 97
+    tokens behind none pay 2.5 us for the merge (13.4 us in one piece), 300 tokens nothing (20 us)."""
+    return max(1, min(256 // max(1, groups), -(-max(1, keys) // 128), 6))
 
 
 def window_attention(q: torch.Tensor, gate: Optional[torch.Tensor], kcache: torch.Tensor, vcache: torch.Tensor,
