@@ -383,8 +383,8 @@ def linear_each(a: torch.Tensor, w: torch.Tensor):
     """[a[i] @ w[i].T]: several inputs, a weight each (a [G, M, K], w [G, N, K]) -> G tensors [M, N] of one row stride.  One
     launch where that is faster than G of :func:`linear`.  4 weights of 2048 x 2048, M = 8 / 64 / 128 / 512 / 1024 / 2048: the
     any-shape kernel (k shared by the waves while its tiles are few) 11 / 24 / 38 / 52 / 77 / 139 us, the grouped big tiles
-    27 / 29 / 30 / 31 / 45 / 80, four launches 22 / 39 / 47 / 76 / 109 / 114; of 4096 x 4096, M = 16 / 32 / 64 / 512 / 2048:
-    70 / 71 / 73 / 136 / 472, 53 / 54 / 55 / 81 / 288, 39 / 54 / 71 / 135 / 300 (beyond, a launch's own tiles fill the card
+    27 / 29 / 30 / 31 / 45 / 80, four launches 22 / 27 / 33 / 76 / 109 / 114; of 4096 x 4096, M = 16 / 32 / 64 / 512 / 2048:
+    70 / 71 / 73 / 136 / 472, 53 / 54 / 55 / 81 / 288, 39 / 47 / 55 / 135 / 300 (beyond, a launch's own tiles fill the card
     and its deeper stages win)."""
     G, M, K = a.shape
     N = w.shape[1]

@@ -178,3 +178,21 @@ def test_mx_plans_are_tuned_for_every_tp_shard():
         for N, K, epi in _llama70b_decode_shapes(tp):
             key = (N, K, epi, 4 if epi == ops.EPI_SWIGLU else 3)
             assert sorted(r[0] for r in table.get(key, [])) == [32, 64, 128, 256], (tp, key)
+
+
+@pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 97, 128])
+def test_untuned_batched_decode_plans_run(M):
+    """The one-round plans of 17 - 128 rows over sizes and k: valid, at most one round of small tiles, split k only with steps
+    left; other k keep the general rule."""
+    for N in (16, 100, 576, 1024, 2048, 3104, 4096, 8192, 16384, 32768, 151936):
+        for K in (64, 128, 192, 256, 768, 1024, 1408, 2048, 3584, 4096, 8192, 14336):
+            for epi in (ops.EPI_BF16, ops.EPI_F32):
+                cfg, split = ops.mgemm_heuristic(M, N, K, epi, False)
+                assert ops.mgemm_valid(cfg, M, N, K, epi, False, split), (M, N, K, cfg, split)
+                one = ops._mgemm_one_round(M, N, K, epi, 256)
+                assert (one is None) == (K % 256 != 0)
+                if one is not None:
+                    assert one == (cfg, split)
+                    tiles = ops._mg_tiles(cfg, M, N, epi) * split
+                    assert tiles <= 256 or cfg in (22, 31), (M, N, K, cfg, split)
+                    assert split == 1 or K * 2 // ops.mgemm_configs()[cfg][5] // split >= 8

@@ -383,3 +383,20 @@ def test_products_of_several_inputs(M, N, K):
     for x, y, z in zip(a, w, got):
         exact = x.double() @ y.double().T
         assert ((z.cpu().double() - exact).abs() <= sum_bound(x, y) + 2.0 ** -8 * exact.abs()).all()
+
+
+@pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 128])
+@pytest.mark.parametrize("N,K", [(16, 256), (1028, 512), (2592, 2048), (4096, 3072), (8192, 512), (16400, 256), (40000, 256),
+                                 (520, 8192), (2048, 8192)])
+@pytest.mark.parametrize("epi", [0, 1])
+def test_untuned_products_of_17_to_128_rows(M, N, K, epi):
+    """Every tile and split that the one-round rule picks, columns and rows that do not fill the tile, both outputs."""
+    from k8s_llm_scheduler_amd import ops
+
+    g = torch.Generator().manual_seed(M + N + K)
+    x, w = torch.randn(M, K, generator=g).to(torch.bfloat16), torch.randn(N, K, generator=g).to(torch.bfloat16)
+    cfg, split = ops.mgemm_heuristic(M, N, K, epi, False)
+    got = ops.mgemm(x.to(DEV), w.to(DEV), epi, cfg=cfg, grid=split)
+    a, b = x.to(DEV).double(), w.to(DEV).double()
+    exact, bound = a @ b.T, 2.0 * K * 2.0 ** -24 * (a.abs() @ b.abs().T) + 1e-30
+    assert ((got.double() - exact).abs() <= bound + (2.0 ** -8 * exact.abs() if epi == 0 else 0.0)).all()
