@@ -183,7 +183,8 @@ __global__ __launch_bounds__(4 * V) void latent_out_kernel(bf16_t* __restrict__ 
     float den = wave_sum(e * l);
     if (sinks != nullptr) den += expf(sinks[hd] - M);
     const float gh = gate != nullptr ? 1.f / (1.f + expf(-bf2f(gate[(size_t)(t0 + wave) * ldg + hd]))) : 1.f;
-    if (lane < 32) ws[wave][lane] = e > 0.f ? e / den * gh : 0.f;
+    // weight 0 is for records that were not written (maximum -inf, sum 0); a NaN or infinite score makes the sum NaN
+    if (lane < 32) ws[wave][lane] = m == -INFINITY && l == 0.f ? 0.f : e / den * gh;
   }
   __syncthreads();
   const int k = tid >> 7, c = 4 * (tid & 127);
@@ -198,7 +199,7 @@ __global__ __launch_bounds__(4 * V) void latent_out_kernel(bf16_t* __restrict__ 
       for (int u = 0; u < 8; ++u) {
         const float w = s + u < nsplit ? ws[k][s + u] : 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) y[i] += w != 0.f ? w * x[u][i] : 0.f;     // an empty split's record is not written
+        for (int i = 0; i < 4; ++i) y[i] += w != 0.f ? w * x[u][i] : 0.f;     // (w 0: nothing, or nothing written)
       }
     }
     stf4(&lat[k][c], y);

@@ -154,6 +154,38 @@ def test_latent_token(ctx, window, H, extra):
     assert err(got) <= 1.1 * err(old.view(T, H * V)) + 1e-7
 
 
+@pytest.mark.parametrize("keys", [40, 700])
+@pytest.mark.parametrize("sink", [False, True])
+def test_latent_token_lets_non_finite_scores_through(keys, sink):
+    """A NaN query head and a key of infinite score, in one split and in many: NaN where 64 bits give NaN (score +inf, or all
+    scores NaN), finite where the infinite score is -inf (weight 0), idle rows zero."""
+    C, R, Dn, V, H, bs, dt = 512, 64, 128, 128, 16, 16, torch.bfloat16
+    g = torch.Generator().manual_seed(keys)
+    r = lambda *s: torch.randn(*s, generator=g)
+    pages = -(-keys // bs)
+    q, cache = r(3, H, Dn + R), r(3 * pages * bs, C + R)
+    q[0, 5, Dn + 3] = float("nan")
+    cache[pages * bs + keys // 2, C + 7] = float("inf")      # (a rotated part: no value)
+    q, cache = q.to(dt).to(DEV), cache.to(dt).to(DEV)
+    uk, uv = ((r(H * d, C) / C ** 0.5).to(dt).to(DEV) for d in (Dn, V))
+    sinks = torch.zeros(H, device=DEV) if sink else None
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    b = {"positions": i32([keys - 1, keys - 1, -1]), "cu_q": i32([0, 1, 2, 3]), "tok_seq": i32([0, 1, 2]),
+         "block_tables": torch.arange(3 * pages, dtype=torch.int32, device=DEV).view(3, pages), "max_keys": pages * bs}
+    got = sm.latent_mix(q.view(3, -1), cache, uk.view(H, Dn, C).transpose(1, 2).contiguous(), uv.view(H, V, C), None, b, C, R, H,
+                        Dn, V, 0, 0.07, bs, sinks=sinks).view(3, H, V)
+    assert (got[2] == 0).all()
+    for t in range(2):
+        rows = cache.view(3, pages * bs, -1)[t, :keys].double()
+        k = torch.cat([(rows[:, :C] @ uk.double().T).view(-1, H, Dn), rows[:, None, C:].expand(-1, H, R)], 2)
+        sc = (q[t].double()[None] * k).sum(2) * 0.07                                  # [keys, H]
+        p = torch.softmax(sc if sinks is None else torch.cat([sc, sinks.double()[None]]), 0)[:keys]
+        want = torch.einsum("kh,khv->hv", p, (rows[:, :C] @ uv.double().T).view(-1, H, V))
+        bad = torch.isnan(want)
+        assert bad.any() and not bad.all() and torch.equal(bad, torch.isnan(got[t]))
+        assert (got[t].double() - want)[~bad].abs().max() <= 2e-2 * want[~bad].abs().max()
+
+
 @pytest.mark.parametrize("dt,tol", [(torch.float32, 2e-6), (torch.bfloat16, 1e-2)])
 @pytest.mark.parametrize("W", [4, 1023, 1024, 1028, 2052, 8192, 8196])
 def test_row_norm_and_token_shift_widths(dt, tol, W):
