@@ -260,7 +260,7 @@ def _route_fast(a: torch.Tensor, w: torch.Tensor, out_dtype) -> bool:
     if _ops.GEMM_BACKEND == "library" or not a.is_contiguous() or not w.is_contiguous():
         return False
     N, K = w.shape
-    return K % 64 == 0 and N % 16 == 0 and K * N >= 512 * 1024 and K >= 128 and N >= 128
+    return a.shape[1] == K and K % 64 == 0 and N % 16 == 0 and K * N >= 512 * 1024 and K >= 128 and N >= 128
 
 
 # route fitting bf16 shapes to ops.linear (K8S_SEQMIX_FAST_GEMM=0: every product on the any-shape kernel)
@@ -388,6 +388,8 @@ def linear_each(a: torch.Tensor, w: torch.Tensor):
     and its deeper stages win)."""
     G, M, K = a.shape
     N = w.shape[1]
+    if w.shape != (G, N, K):
+        raise ValueError(f"linear_each: inputs {tuple(a.shape)} and weights {tuple(w.shape)}")
     if not (FAST_GEMM and _gpu(a, w) and _route_fast(a[0], w[0], a.dtype)):
         return gemm(a, w).unbind(0)
     if _each_once(a, w):

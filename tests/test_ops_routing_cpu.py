@@ -4,8 +4,10 @@
 import json
 
 import pytest
+import torch
 
 from k8s_llm_scheduler_amd import ops
+from k8s_llm_scheduler_amd.ops import seqmix as sm
 
 
 def test_row_buckets():
@@ -196,3 +198,40 @@ def test_untuned_batched_decode_plans_run(M):
                     tiles = ops._mg_tiles(cfg, M, N, epi) * split
                     assert tiles <= 256 or cfg in (22, 31), (M, N, K, cfg, split)
                     assert split == 1 or K * 2 // ops.mgemm_configs()[cfg][5] // split >= 8
+
+
+# ----------------------------------------------------------------------------- stream designs: routing without a GPU
+class Recorder:
+    """Stands for the extension: notes the entry points that a call reaches, answers every size question with yes."""
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        def entry(*args):
+            self.calls.append(name)
+            return True
+
+        return entry
+
+
+@pytest.fixture
+def recorder(monkeypatch):
+    nat = Recorder()
+    monkeypatch.setattr(sm, "_gpu", lambda *ts: True)
+    monkeypatch.setattr(ops, "_gpu", lambda *ts: True)
+    monkeypatch.setattr(ops, "native", lambda: nat)
+    return nat
+
+
+@pytest.mark.parametrize("M", [1, 8, 40, 200, 1024])
+def test_products_refuse_operands_of_unequal_k(M, recorder):
+    """Sizes of the tuned kernels, which take k from one operand: an error ahead of any launch, also for more inputs than
+    weights."""
+    a, w = torch.zeros(M, 1024, dtype=torch.bfloat16), torch.zeros(2048, 512, dtype=torch.bfloat16)
+    for call in (lambda: sm.linear(a, w), lambda: sm.linear_act(a, w, sm.ACT_RELU2), lambda: sm.linear_act(a, w, sm.ACT_RELU),
+                 lambda: sm.linear_each(a.expand(2, M, 1024), w.expand(2, 2048, 512)),
+                 lambda: sm.linear_each(a.expand(3, M, 1024), torch.zeros(2, 2048, 1024, dtype=torch.bfloat16))):
+        with pytest.raises(ValueError):
+            call()
+    assert recorder.calls == []
