@@ -287,8 +287,8 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out_dtype=None, *, a_rows: Optional[t
     """The any-shape GEMM.  2-D: a [M, K] (row stride free) @ w [N, K]^T.  3-D: batched over dim 0 (a [G, M, K] with
     any strides whose last is 1, w [G, N, K]) -> [G, M, N]; ``out``: a [G, M, N] view with any batch / row strides.
     Grouped (``tiles`` [n, 3] from :func:`moe_align`, w [G, N, K]): ``rows`` compact rows, row r = a[a_rows[r]] (or
-    a[r]), the rows of tile (g, r0, n) use w[g] -> [rows, N] (``seg``: the groups' row offsets, read by the CPU
-    reference only)."""
+    a[r]), the rows of tile (g, r0, n) use w[g] -> [rows, N].  ``seg`` int32 [G + 1]: the groups' row offsets, the same
+    rows as ``tiles`` lists; the CPU reference and the big-tile kernel (:func:`_grouped_big`) go by them."""
     out_dtype = out_dtype or a.dtype
     if a.dtype != w.dtype:
         raise TypeError(f"gemm operands differ in dtype: {a.dtype} and {w.dtype}")
@@ -344,10 +344,11 @@ GROUP_BIG_MAX_GROUPS = 64        # every workgroup walks the groups' offsets
 
 def _grouped_big(a: torch.Tensor, w: torch.Tensor, seg: Optional[torch.Tensor], rows: int, N: int) -> bool:
     E, _, K = w.shape
-    return (not _ops.LEAN and FAST_GEMM and a.dtype == BF16 and seg is not None and seg.is_cuda and E <= GROUP_BIG_MAX_GROUPS
-            and rows >= GROUP_BIG_MIN * E and K % 64 == 0 and N % 4 == 0 and N >= 128 and a.stride(0) % 8 == 0
-            and a.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0
-            and w.shape[1] * K * 2 < 1 << 32 and a.shape[0] * a.stride(0) * 2 < 1 << 32)
+    return (not _ops.LEAN and FAST_GEMM and a.dtype == BF16 and seg is not None and seg.is_cuda and seg.dtype == I32
+            and seg.is_contiguous() and seg.numel() == E + 1 and E <= GROUP_BIG_MAX_GROUPS
+            and rows >= GROUP_BIG_MIN * E and K % 64 == 0 and N % 4 == 0 and N >= 128 and a.dim() == 2 and a.stride(1) == 1
+            and a.stride(0) >= K and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.is_contiguous()
+            and w.data_ptr() % 16 == 0 and w.shape[1] * K * 2 < 1 << 32 and a.shape[0] * a.stride(0) * 2 < 1 << 32)
 
 
 def _grouped_cfg(rows: int, E: int, N: int, K: int, pair: bool, even: bool = False) -> int:

@@ -235,3 +235,35 @@ def test_products_refuse_operands_of_unequal_k(M, recorder):
         with pytest.raises(ValueError):
             call()
     assert recorder.calls == []
+
+
+def test_grouped_products_on_big_tiles_take_what_the_kernel_reads(recorder, monkeypatch):
+    """Row offsets of another length, type or layout, gathered rows that share memory or are strided in k: the route that goes
+    by the tiles alone, or its refusal."""
+    monkeypatch.setattr(ops, "LEAN", False)
+    E, N, K, rows = 4, 256, 128, 300
+    w, tiles = torch.zeros(E, 2 * N, K, dtype=torch.bfloat16), torch.zeros(9, 3, dtype=torch.int32)
+    a = torch.zeros(rows, K, dtype=torch.bfloat16)
+
+    class Seg(torch.Tensor):
+        is_cuda = True
+
+    seg = lambda n=E + 1, dt=torch.int32, step=1: torch.zeros(n * step, dtype=dt)[::step].as_subclass(Seg)
+
+    def reached(a, seg, kind=None):
+        recorder.calls.clear()
+        try:
+            if kind is None:
+                sm.gemm(a, w, tiles=tiles, rows=rows, seg=seg)
+            else:
+                sm.gemm_act(a, w, kind, tiles=tiles, rows=rows, seg=seg)
+        except ValueError:
+            return "refused"
+        return recorder.calls[0]
+
+    for kind in (None, sm.ACT_RELU):
+        assert reached(a, seg(), kind) == "pgemm4_grouped"
+        for s in (None, seg(E), seg(E + 2), seg(dt=torch.int64), seg(step=2), torch.zeros(E + 1, dtype=torch.int32)):
+            assert reached(a, s, kind) in ("gemm_any", "gemm_few_act")
+        assert reached(a[:1].expand(rows, K), seg(), kind) in ("gemm_any", "gemm_few_act")       # one row for all: stride 0
+        assert reached(a.T.contiguous().T, seg(), kind) == "refused"
