@@ -267,3 +267,27 @@ def test_grouped_products_on_big_tiles_take_what_the_kernel_reads(recorder, monk
             assert reached(a, s, kind) in ("gemm_any", "gemm_few_act")
         assert reached(a[:1].expand(rows, K), seg(), kind) in ("gemm_any", "gemm_few_act")       # one row for all: stride 0
         assert reached(a.T.contiguous().T, seg(), kind) == "refused"
+
+
+def latent_calls(recorder, T, *, seqs=1, decode=False, dt=torch.bfloat16, q=None, gate=None, uv=None, window=0, blocks=64, H=4):
+    """Entry points that latent_mix reaches for a batch of T tokens of ``seqs`` sequences, sizes of the matrix-core kernels."""
+    C, R, D, bs = 512, 64, 128, 16
+    i32 = lambda *s: torch.zeros(*s, dtype=torch.int32)
+    z = lambda *s: torch.zeros(*s, dtype=dt)
+    b = {"positions": i32(T), "cu_q": i32(seqs + 1), "tok_seq": i32(T), "block_tables": i32(seqs, blocks),
+         "max_qlen": 0 if decode else T}
+    recorder.calls.clear()
+    sm.latent_mix(z(T, H * (D + R)) if q is None else q, z(2 * bs, C + R), z(H, C, D), z(H, D, C) if uv is None else uv,
+                  z(2 * H * D, C), b, C, R, H, D, D, window, 0.1, bs, gate=gate)
+    return [c for c in recorder.calls if c.startswith("latent") and not c.endswith("_ok")]
+
+
+def test_latent_attention_on_plain_fmas_when_told_so(recorder, monkeypatch):
+    for dt in (torch.bfloat16, torch.float32):
+        assert latent_calls(recorder, 200, dt=dt) == ["latent_keys", "latent_prompt"]
+        assert latent_calls(recorder, 2, seqs=2, decode=True, dt=dt) == [
+            "latent_token" if dt == torch.bfloat16 else "latent_attention"]
+        monkeypatch.setattr(sm, "LATENT_MFMA", False)
+        assert latent_calls(recorder, 200, dt=dt) == ["latent_attention"]
+        assert latent_calls(recorder, 2, seqs=2, decode=True, dt=dt) == ["latent_attention"]
+        monkeypatch.setattr(sm, "LATENT_MFMA", True)
