@@ -659,7 +659,8 @@ def latent_mix(q: torch.Tensor, cache: torch.Tensor, uk_t: torch.Tensor, uv: tor
     nseq, max_qlen = b["cu_q"].shape[0] - 1, b.get("max_qlen", 0)
     ctx = b["block_tables"].shape[1] * block_size
     cap = min(T + nseq * (window - 1), nseq * ctx) if window else nseq * ctx
-    if (LATENT_MFMA and ukv is not None and _gpu(q, cache) and max_qlen > 0 and 0 < LATENT_EXPAND_MIN * nseq <= T
+    aligned = (q.data_ptr() | cache.data_ptr()) % 16 == 0          # the two newer forms move whole vectors only
+    if (LATENT_MFMA and ukv is not None and _gpu(q, cache) and aligned and max_qlen > 0 and 0 < LATENT_EXPAND_MIN * nseq <= T
             and cap < 1 << 24 and cap * H * (Dn + V) * q.element_size() <= LATENT_EXPAND_BYTES
             and _native().latent_prompt_ok(C, R, Dn, V)):
         rows, kbase, tiles, seg = _latent_keys(b, int(window), block_size, cap)
@@ -676,8 +677,8 @@ def latent_mix(q: torch.Tensor, cache: torch.Tensor, uk_t: torch.Tensor, uv: tor
         return out
     q_abs = torch.empty(T, H, C, dtype=dt, device=q.device)
     gemm(q.view(T, H, Dn + R)[:, :, :Dn].permute(1, 0, 2), uk_t, out=q_abs.permute(1, 0, 2))
-    if LATENT_MFMA and max_qlen == 0 and dt == BF16 and _gpu(q, cache, sinks, gate) and \
-            _native().latent_token_ok(C, R, Dn, V):
+    if LATENT_MFMA and max_qlen == 0 and dt == BF16 and _gpu(q, cache, sinks, gate) and aligned and \
+            uv.data_ptr() % 16 == 0 and _native().latent_token_ok(C, R, Dn, V):
         # decoding: key splits of at least one 64-key step for about one workgroup per CU, joined by the kernel that takes
         # the sums through W_uv
         HP = (H + 15) // 16 * 16

@@ -2,6 +2,7 @@
 (hand-written kernels always; the library only as the K8S_GEMM=library oracle), and the GEMV row threshold."""
 
 import json
+import math
 
 import pytest
 import torch
@@ -291,3 +292,14 @@ def test_latent_attention_on_plain_fmas_when_told_so(recorder, monkeypatch):
         assert latent_calls(recorder, 200, dt=dt) == ["latent_attention"]
         assert latent_calls(recorder, 2, seqs=2, decode=True, dt=dt) == ["latent_attention"]
         monkeypatch.setattr(sm, "LATENT_MFMA", True)
+
+
+def test_latent_attention_of_unaligned_operands_is_absorbed(recorder):
+    """Queries (both forms) or value weights (single tokens) that do not start at a whole vector: the kernels without that
+    demand, as ever."""
+    odd = lambda *s: torch.zeros(1 + math.prod(s), dtype=torch.bfloat16)[1:].view(*s)
+    attend = ["latent_attention_mfma"]
+    assert latent_calls(recorder, 200, q=odd(200, 4 * 192)) == attend
+    assert latent_calls(recorder, 200, uv=odd(4, 128, 512)) == ["latent_keys", "latent_prompt"]      # (not read)
+    assert latent_calls(recorder, 2, seqs=2, decode=True, q=odd(2, 4 * 192)) == attend
+    assert latent_calls(recorder, 2, seqs=2, decode=True, uv=odd(4, 128, 512)) == attend
