@@ -656,6 +656,8 @@ def latent_mix(q: torch.Tensor, cache: torch.Tensor, uk_t: torch.Tensor, uv: tor
         raise ValueError("latent_mix: sinks are fp32 [H]")
     if gate is not None and (gate.shape != (T, H) or gate.dtype != dt or gate.stride(1) != 1):
         raise ValueError("latent_mix: the gate is [T, H] of the queries' type with contiguous rows")
+    if q.shape != (T, H * (Dn + R)) or cache.dim() != 2 or cache.shape[1] != C + R or uv.shape != (H, V, C):
+        raise ValueError("latent_mix: queries [T, H (Dn + R)], a cache of C + R columns, uv [H, V, C]")
     nseq, max_qlen = b["cu_q"].shape[0] - 1, b.get("max_qlen", 0)
     ctx = b["block_tables"].shape[1] * block_size
     cap = min(T + nseq * (window - 1), nseq * ctx) if window else nseq * ctx
@@ -665,8 +667,8 @@ def latent_mix(q: torch.Tensor, cache: torch.Tensor, uk_t: torch.Tensor, uv: tor
             and _native().latent_prompt_ok(C, R, Dn, V)):
         rows, kbase, tiles, seg = _latent_keys(b, int(window), block_size, cap)
         nat = _native()
-        if cache.shape[1] != C + R or ukv.shape != (H * (Dn + V), C):
-            raise ValueError("latent_mix: the cache holds C + R columns, ukv is [H (Dn + V), C]")
+        if ukv.shape != (H * (Dn + V), C):
+            raise ValueError("latent_mix: ukv is [H (Dn + V), C]")
         _p(cache, dt, "cache"), _p(ukv, dt, "ukv")
         kv = gemm(cache[:, :C], ukv.unsqueeze(0), a_rows=rows, tiles=tiles, rows=cap, seg=seg)
         out = torch.empty(T, H * V, dtype=dt, device=q.device)

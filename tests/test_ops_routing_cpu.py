@@ -270,7 +270,7 @@ def test_grouped_products_on_big_tiles_take_what_the_kernel_reads(recorder, monk
         assert reached(a.T.contiguous().T, seg(), kind) == "refused"
 
 
-def latent_calls(recorder, T, *, seqs=1, decode=False, dt=torch.bfloat16, q=None, gate=None, uv=None, window=0, blocks=64, H=4):
+def latent_calls(recorder, T, *, seqs=1, decode=False, dt=torch.bfloat16, q=None, cache=None, uv=None, blocks=64, H=4):
     """Entry points that latent_mix reaches for a batch of T tokens of ``seqs`` sequences, sizes of the matrix-core kernels."""
     C, R, D, bs = 512, 64, 128, 16
     i32 = lambda *s: torch.zeros(*s, dtype=torch.int32)
@@ -278,8 +278,9 @@ def latent_calls(recorder, T, *, seqs=1, decode=False, dt=torch.bfloat16, q=None
     b = {"positions": i32(T), "cu_q": i32(seqs + 1), "tok_seq": i32(T), "block_tables": i32(seqs, blocks),
          "max_qlen": 0 if decode else T}
     recorder.calls.clear()
-    sm.latent_mix(z(T, H * (D + R)) if q is None else q, z(2 * bs, C + R), z(H, C, D), z(H, D, C) if uv is None else uv,
-                  z(2 * H * D, C), b, C, R, H, D, D, window, 0.1, bs, gate=gate)
+    pick = lambda t, *s: z(*s) if t is None else t
+    sm.latent_mix(pick(q, T, H * (D + R)), pick(cache, 2 * bs, C + R), z(H, C, D), pick(uv, H, D, C), z(2 * H * D, C), b, C, R, H,
+                  D, D, 0, 0.1, bs)
     return [c for c in recorder.calls if c.startswith("latent") and not c.endswith("_ok")]
 
 
@@ -303,3 +304,13 @@ def test_latent_attention_of_unaligned_operands_is_absorbed(recorder):
     assert latent_calls(recorder, 200, uv=odd(4, 128, 512)) == ["latent_keys", "latent_prompt"]      # (not read)
     assert latent_calls(recorder, 2, seqs=2, decode=True, q=odd(2, 4 * 192)) == attend
     assert latent_calls(recorder, 2, seqs=2, decode=True, uv=odd(4, 128, 512)) == attend
+
+
+@pytest.mark.parametrize("T,decode", [(200, False), (2, True)])
+def test_latent_attention_refuses_operands_of_other_sizes(recorder, T, decode):
+    """Queries, cache rows and value weights of other sizes than the heads': an error ahead of the attention, on every route."""
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)
+    for kw in ({"q": z(T, 4 * 128)}, {"cache": z(32, 512)}, {"uv": z(4, 64, 512)}, {"uv": z(3, 128, 512)}):
+        with pytest.raises((ValueError, RuntimeError)):
+            latent_calls(recorder, T, seqs=1 if not decode else T, decode=decode, **kw)
+        assert not [c for c in recorder.calls if c in ("latent_prompt", "latent_token", "latent_attention_mfma")], kw
