@@ -663,20 +663,24 @@ def latent_mix(q: torch.Tensor, cache: torch.Tensor, uk_t: torch.Tensor, uv: tor
     cap = min(T + nseq * (window - 1), nseq * ctx) if window else nseq * ctx
     aligned = (q.data_ptr() | cache.data_ptr()) % 16 == 0          # the two newer forms move whole vectors only
     if (LATENT_MFMA and ukv is not None and _gpu(q, cache) and aligned and max_qlen > 0 and 0 < LATENT_EXPAND_MIN * nseq <= T
-            and cap < 1 << 24 and cap * H * (Dn + V) * q.element_size() <= LATENT_EXPAND_BYTES
+            and not b.get("latent_absorbed") and cap < 1 << 24 and cap * H * (Dn + V) * q.element_size() <= LATENT_EXPAND_BYTES
             and _native().latent_prompt_ok(C, R, Dn, V)):
         rows, kbase, tiles, seg = _latent_keys(b, int(window), block_size, cap)
         nat = _native()
         if ukv.shape != (H * (Dn + V), C):
             raise ValueError("latent_mix: ukv is [H (Dn + V), C]")
         _p(cache, dt, "cache"), _p(ukv, dt, "ukv")
-        kv = gemm(cache[:, :C], ukv.unsqueeze(0), a_rows=rows, tiles=tiles, rows=cap, seg=seg)
-        out = torch.empty(T, H * V, dtype=dt, device=q.device)
-        nat.latent_prompt(out.data_ptr(), kv.data_ptr(), rows.data_ptr(), kbase.data_ptr(), _p(q), cache.data_ptr(), C, R, Dn,
-                          V, _p(b["cu_q"], I32), _p(b["positions"], I32), nseq, int(max_qlen), H, int(window), float(scale),
-                          _p(sinks), gate.data_ptr() if gate is not None else 0, gate.stride(0) if gate is not None else 0,
-                          _f32(dt), -1)
-        return out
+        try:
+            kv = gemm(cache[:, :C], ukv.unsqueeze(0), a_rows=rows, tiles=tiles, rows=cap, seg=seg)
+        except torch.OutOfMemoryError:      # no room for the keys and values: this batch's layers run absorbed
+            b["latent_absorbed"] = True
+        else:
+            out = torch.empty(T, H * V, dtype=dt, device=q.device)
+            nat.latent_prompt(out.data_ptr(), kv.data_ptr(), rows.data_ptr(), kbase.data_ptr(), _p(q), cache.data_ptr(), C, R, Dn,
+                              V, _p(b["cu_q"], I32), _p(b["positions"], I32), nseq, int(max_qlen), H, int(window), float(scale),
+                              _p(sinks), gate.data_ptr() if gate is not None else 0,
+                              gate.stride(0) if gate is not None else 0, _f32(dt), -1)
+            return out
     q_abs = torch.empty(T, H, C, dtype=dt, device=q.device)
     gemm(q.view(T, H, Dn + R)[:, :, :Dn].permute(1, 0, 2), uk_t, out=q_abs.permute(1, 0, 2))
     if LATENT_MFMA and max_qlen == 0 and dt == BF16 and _gpu(q, cache, sinks, gate) and aligned and \

@@ -270,17 +270,19 @@ def test_grouped_products_on_big_tiles_take_what_the_kernel_reads(recorder, monk
         assert reached(a.T.contiguous().T, seg(), kind) == "refused"
 
 
-def latent_calls(recorder, T, *, seqs=1, decode=False, dt=torch.bfloat16, q=None, cache=None, uv=None, blocks=64, H=4):
+def latent_calls(recorder, T, *, seqs=1, decode=False, dt=torch.bfloat16, q=None, cache=None, uv=None, blocks=64, H=4, keep=None):
     """Entry points that latent_mix reaches for a batch of T tokens of ``seqs`` sequences, sizes of the matrix-core kernels."""
     C, R, D, bs = 512, 64, 128, 16
     i32 = lambda *s: torch.zeros(*s, dtype=torch.int32)
     z = lambda *s: torch.zeros(*s, dtype=dt)
     b = {"positions": i32(T), "cu_q": i32(seqs + 1), "tok_seq": i32(T), "block_tables": i32(seqs, blocks),
-         "max_qlen": 0 if decode else T}
+         "max_qlen": 0 if decode else T, **(keep or {})}
     recorder.calls.clear()
     pick = lambda t, *s: z(*s) if t is None else t
     sm.latent_mix(pick(q, T, H * (D + R)), pick(cache, 2 * bs, C + R), z(H, C, D), pick(uv, H, D, C), z(2 * H * D, C), b, C, R, H,
                   D, D, 0, 0.1, bs)
+    if keep is not None:
+        keep.update(b)
     return [c for c in recorder.calls if c.startswith("latent") and not c.endswith("_ok")]
 
 
@@ -314,3 +316,25 @@ def test_latent_attention_refuses_operands_of_other_sizes(recorder, T, decode):
         with pytest.raises((ValueError, RuntimeError)):
             latent_calls(recorder, T, seqs=1 if not decode else T, decode=decode, **kw)
         assert not [c for c in recorder.calls if c in ("latent_prompt", "latent_token", "latent_attention_mfma")], kw
+
+
+def test_latent_attention_without_room_for_keys_and_values(recorder, monkeypatch):
+    """The written-out keys and values are bounded by LATENT_EXPAND_BYTES; where the device has no room for them the batch
+    runs absorbed, and its other layers do not ask again."""
+    attend = ["latent_attention_mfma"]
+    bs, per_row = 16, 4 * 256 * 2
+    assert latent_calls(recorder, 200, blocks=sm.LATENT_EXPAND_BYTES // per_row // bs) == ["latent_keys", "latent_prompt"]
+    assert latent_calls(recorder, 200, blocks=sm.LATENT_EXPAND_BYTES // per_row // bs + 1) == attend
+    gemm, asked = sm.gemm, []
+
+    def full(a, w, *args, rows=None, **kw):
+        if rows is None:
+            return gemm(a, w, *args, **kw)
+        asked.append(rows)
+        raise torch.OutOfMemoryError("no room")
+
+    monkeypatch.setattr(sm, "gemm", full)
+    batch = {}
+    assert latent_calls(recorder, 200, keep=batch) == ["latent_keys"] + attend
+    assert latent_calls(recorder, 200, keep=batch) == attend
+    assert asked == [64 * bs]
