@@ -486,19 +486,27 @@ def wkv_max_dim() -> int:
     return 128
 
 
-WKV_CHUNK = int(os.environ.get("K8S_WKV_CHUNK", "0"))            # > 0: chunks of that many tokens
-WKV_CHUNK_MIN = int(os.environ.get("K8S_WKV_CHUNK_MIN", "0"))    # > 0: from that many tokens on
+def _env_int(name: str) -> Optional[int]:
+    return int(os.environ[name]) if name in os.environ else None
+
+
+WKV_CHUNK = _env_int("K8S_WKV_CHUNK")            # set: chunks of that many tokens (0: none, every sequence is walked)
+WKV_CHUNK_MIN = _env_int("K8S_WKV_CHUNK_MIN")    # set: chunks from that many tokens on
 
 
 def wkv_chunk(T: int, nseq: int, H: int) -> int:
     """Tokens of a chunk where the recurrence runs as three passes over chunks (parallel over them), 0 where a workgroup walks
-    each sequence alone (decoding, very short portions).  The walk takes 1.4 us a token of the longest sequence, the passes
-    about 20 us and more with the batch: (heads of 64) one sequence of 32 tokens 48 / 22 us, 8 of 32 49 / 37 us, 16 of 32
-    52 / 65 us, 16 of 64 102 / 91 us -- from 256 tokens or 32 a sequence on.  Chunks of 64, of 32 while those would leave
-    CUs without two workgroups (512 tokens of 32 heads: 46 / 56 us; 2048: 109 / 78 us)."""
-    if T < (WKV_CHUNK_MIN or min(256, 32 * nseq)):
+    each sequence alone.  The walk takes 1.4 us a token of the longest sequence, the passes about 20 us and more with the
+    batch: (heads of 64) one sequence of 32 tokens 48 / 22 us, 8 of 32 49 / 37 us.  Chunks from 32 tokens a sequence on, the
+    average standing for the longest, which is not known here, and from 256 tokens on whatever the sequences (one long one
+    beside many short ones is the costly case; 16 of 32 alone would walk faster, 52 / 65 us, 16 of 64 102 / 91 us).  Below
+    256 rows decoding walks.  Chunks of 64, of 32 while those would leave CUs without two workgroups (512 tokens of 32 heads:
+    46 / 56 us; 2048: 109 / 78 us)."""
+    if T < (min(256, 32 * nseq) if WKV_CHUNK_MIN is None else WKV_CHUNK_MIN):
         return 0
-    return WKV_CHUNK or (64 if (-(-T // 64) + nseq) * H >= 512 else 32)
+    if WKV_CHUNK is not None:
+        return max(0, WKV_CHUNK)
+    return 64 if (-(-T // 64) + nseq) * H >= 512 else 32
 
 
 def wkv_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, z: torch.Tensor, w0: torch.Tensor,

@@ -3,12 +3,18 @@
 
 import json
 import math
+import os
+import subprocess
+import sys
+from pathlib import Path
 
 import pytest
 import torch
 
 from k8s_llm_scheduler_amd import ops
 from k8s_llm_scheduler_amd.ops import seqmix as sm
+
+ROOT = Path(__file__).resolve().parent.parent
 
 
 def test_row_buckets():
@@ -338,3 +344,17 @@ def test_latent_attention_without_room_for_keys_and_values(recorder, monkeypatch
     assert latent_calls(recorder, 200, keep=batch) == ["latent_keys"] + attend
     assert latent_calls(recorder, 200, keep=batch) == attend
     assert asked == [64 * bs]
+
+
+@pytest.mark.parametrize("env,want", [
+    ({}, [0, 0, 32, 32, 64, 32]), ({"K8S_WKV_CHUNK": "0"}, [0] * 6), ({"K8S_WKV_CHUNK": "48"}, [0, 0, 48, 48, 48, 48]),
+    ({"K8S_WKV_CHUNK_MIN": "0"}, [32, 32, 32, 32, 64, 32]), ({"K8S_WKV_CHUNK_MIN": "300"}, [0, 0, 0, 0, 64, 32]),
+    ({"K8S_WKV_CHUNK": "16", "K8S_WKV_CHUNK_MIN": "1"}, [16] * 6)])
+def test_recurrence_chunks_follow_their_switches(env, want):
+    """(tokens, sequences, heads): decoding, below and at 32 tokens a sequence, from 256 tokens on, chunks that fill the CUs,
+    a batch of many rows.  0 in K8S_WKV_CHUNK turns the chunks off, in K8S_WKV_CHUNK_MIN always on."""
+    code = ("from k8s_llm_scheduler_amd.ops import seqmix as sm\n"
+            "print([sm.wkv_chunk(*a) for a in ((8, 8, 32), (63, 2, 32), (64, 2, 4), (255, 3, 2), (2048, 1, 32), (300, 300, 1))])")
+    clean = {k: v for k, v in os.environ.items() if not k.startswith("K8S_WKV")}
+    out = subprocess.run([sys.executable, "-c", code], env={**clean, **env}, cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert out.stdout.strip() == str(want), out.stderr
