@@ -148,7 +148,7 @@ class StreamModel:
         self._check_ready()
         B = tokens.shape[0]
         tables = block_tables.contiguous()
-        pos, slots, ar = sm.decode_meta(context_lens.to(torch.int32).contiguous(), tables, self.block_size)
+        pos, slots, ar = sm.decode_meta(context_lens.to(torch.int32).contiguous(), tables.to(torch.int32), self.block_size)
         b = {"positions": pos, "slot_mapping": slots, "cu_q": ar, "tok_seq": ar[:B], "block_tables": tables,
              "seq_slots": ar[:B], "max_keys": int(max_context)}
         return self._forward(tokens, b, None)

@@ -12,6 +12,7 @@ import pytest
 import torch
 
 from k8s_llm_scheduler_amd import ops
+from k8s_llm_scheduler_amd.models.stream import StreamModel
 from k8s_llm_scheduler_amd.ops import seqmix as sm
 
 ROOT = Path(__file__).resolve().parent.parent
@@ -358,3 +359,23 @@ def test_recurrence_chunks_follow_their_switches(env, want):
     clean = {k: v for k, v in os.environ.items() if not k.startswith("K8S_WKV")}
     out = subprocess.run([sys.executable, "-c", code], env={**clean, **env}, cwd=ROOT, capture_output=True, text=True, timeout=300)
     assert out.stdout.strip() == str(want), out.stderr
+
+
+@pytest.mark.parametrize("dt", [torch.int32, torch.int64])
+def test_decode_steps_take_block_tables_of_both_integer_types(recorder, dt):
+    """A design without attention reads its block table for the step's slots alone; layers that attend get it as it came."""
+    class Model(StreamModel):
+        block_size = 16
+
+        def __init__(self):
+            pass
+
+        def _check_ready(self):
+            pass
+
+        def _forward(self, ids, b, rows):
+            return b
+
+    tables = torch.zeros(3, 4, dtype=dt)
+    b = Model().forward_decode(torch.zeros(3, dtype=torch.int32), torch.ones(3, dtype=torch.int64), tables, 64)
+    assert recorder.calls == ["decode_meta"] and b["block_tables"].dtype == dt
