@@ -607,6 +607,7 @@ def _mg_plan_info(M: int, N: int, K: int, epi: int, fp8: bool, cfg: int, nwg: in
     return tuple(native().mgemm_plan_info(M, N, K, epi, int(fp8), cfg, nwg))
 
 
+@functools.lru_cache(maxsize=4096)
 def _mgemm_one_round(M: int, N: int, K: int, epi: int, num_cus: int) -> Optional[Tuple[int, int]]:
     """Tile + split of an untuned bf16 product of 17 - 128 rows: the smallest tile whose workgroups still fit the CUs once.
     A workgroup streams its weight rows over the whole of k, so the time is that of its own chain of loads: half the tile on

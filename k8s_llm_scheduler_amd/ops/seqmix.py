@@ -10,6 +10,7 @@ attention scores) is fp32 in both.
 
 from __future__ import annotations
 
+import functools
 import math
 import os
 import sys
@@ -351,13 +352,18 @@ def _grouped_big(a: torch.Tensor, w: torch.Tensor, seg: Optional[torch.Tensor], 
             and w.data_ptr() % 16 == 0 and w.shape[1] * K * 2 < 1 << 32 and a.shape[0] * a.stride(0) * 2 < 1 << 32)
 
 
+@functools.lru_cache(maxsize=4096)
 def _grouped_cfg(rows: int, E: int, N: int, K: int, pair: bool, even: bool = False) -> int:
     """Configuration of the grouped big-tile product: 256 (1) or 128 (3) weight rows per tile by the time its rounds of tiles
     over the CUs take (us, fitted to the products above and to N = 3584 / 4096, K = 3584 / 4096), groups of the same size
     (``even``) or of about equal size drawn at random."""
     r = rows / E
-    tiles = E * -(-rows // E // 128) if even else E + E * sum(
-        0.5 + 0.5 * math.erf((r - 128 * k) / math.sqrt(2.0 * max(r, 1.0))) for k in range(1, int(r / 128) + 2))
+    if even or E == 1:
+        tiles = E * -(-rows // E // 128)
+    else:       # a group's tiles beyond k: the chance that it has more than 128 k rows, 1 up to six deviations below the mean
+        sure = max(0, int((r - 6.0 * math.sqrt(max(r, 1.0))) // 128))
+        tiles = E * (1 + sure + sum(0.5 + 0.5 * math.erf((r - 128 * k) / math.sqrt(2.0 * max(r, 1.0)))
+                                    for k in range(sure + 1, int(r / 128) + 2)))
     n, kt = (2 * N if pair else N), K / 64
     big = 10.0 + math.ceil(tiles * -(-n // 256) / 256) * (kt + (12.0 if pair else 0.0))
     small = 20.0 + math.ceil(tiles * -(-n // 128) / 256) * 0.56 * kt

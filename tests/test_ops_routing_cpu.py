@@ -379,3 +379,25 @@ def test_decode_steps_take_block_tables_of_both_integer_types(recorder, dt):
     tables = torch.zeros(3, 4, dtype=dt)
     b = Model().forward_decode(torch.zeros(3, dtype=torch.int32), torch.ones(3, dtype=torch.int64), tables, 64)
     assert recorder.calls == ["decode_meta"] and b["block_tables"].dtype == dt
+
+
+def test_plans_are_worked_out_once_and_in_bounded_time(monkeypatch):
+    """Plans stand on every product's way to the device: a shape's second call looks its plan up, and the expected tiles of
+    large groups are not summed term by term (the same number: the terms left out are 0 or 1 to 1e-9)."""
+    valid, calls = ops.mgemm_valid, []
+    monkeypatch.setattr(ops, "mgemm_valid", lambda *a: calls.append(a) or valid(*a))
+    first = ops.mgemm_heuristic(71, 3104, 2048, ops.EPI_BF16, False)
+    asked = len(calls)
+    assert ops.mgemm_heuristic(71, 3104, 2048, ops.EPI_BF16, False) == first and len(calls) == asked
+    erf, terms = math.erf, []
+    monkeypatch.setattr(sm.math, "erf", lambda x: terms.append(x) or erf(x))
+    for rows, E, N, K, pair in ((131072, 1, 4096, 512, False), (131072, 2, 2048, 2048, True), (3068, 8, 2048, 2048, True),
+                                (194, 8, 2048, 2048, False), (90000, 8, 128, 64, False)):
+        r = rows / E
+        terms.clear()
+        got = sm._grouped_cfg.__wrapped__(rows, E, N, K, pair)
+        assert len(terms) <= 2 + 12.0 * r ** 0.5 / 128
+        tiles = E + E * sum(0.5 + 0.5 * erf((r - 128 * k) / (2.0 * r) ** 0.5) for k in range(1, int(r / 128) + 2))
+        per, kt = (2 if pair else 1) * N, K / 64
+        big = 10.0 + math.ceil(tiles * -(-per // 256) / 256) * (kt + (12.0 if pair else 0.0))
+        assert got == (1 if big < 20.0 + math.ceil(tiles * -(-per // 128) / 256) * 0.56 * kt else 3)
