@@ -154,7 +154,7 @@ int k8s_rglru_scan(void* out, const float* u, const float* gates, const float* g
 int k8s_act(void* out, const void* x, int T, int F, int kind, float limit, float alpha, const float* row_scale,
             const int* row_map, const void* bias, int f32, hipStream_t s);
 int k8s_gemm_few_act(void* C, const void* A, const void* W, int M, int N, int K, long lda, const int* a_rows,
-                     const int* tiles, int ntiles, int kind, float limit, float alpha, const void* bias, hipStream_t s);
+                     const int* tiles, int ntiles, int kind, float limit, float alpha, hipStream_t s);
 int k8s_gemm_any(void* C, const void* A, const void* W, int M, int N, int K, long lda, long ldw, long ldc, int batch,
                  long sA, long sW, long sC, const int* a_rows, const int* tiles, int ntiles, int in_f32, int out_f32,
                  hipStream_t s);
@@ -573,9 +573,9 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
     check(k8s_act(P(out), P(x), T, F, kind, limit, alpha, P<float>(row_scale), P<int>(row_map), P(bias), f32, S(s)), "act");
   });
   m.def("gemm_few_act", [](uintptr_t C, uintptr_t A, uintptr_t W, int M, int N, int K, long lda, uintptr_t a_rows,
-                           uintptr_t tiles, int ntiles, int kind, float limit, float alpha, uintptr_t bias, int64_t s) {
-    check(k8s_gemm_few_act(P(C), P(A), P(W), M, N, K, lda, P<int>(a_rows), P<int>(tiles), ntiles, kind, limit, alpha, P(bias),
-                           S(s)), "gemm_few_act");
+                           uintptr_t tiles, int ntiles, int kind, float limit, float alpha, int64_t s) {
+    check(k8s_gemm_few_act(P(C), P(A), P(W), M, N, K, lda, P<int>(a_rows), P<int>(tiles), ntiles, kind, limit, alpha, S(s)),
+          "gemm_few_act");
   });
   m.def("gemm_any", [](uintptr_t C, uintptr_t A, uintptr_t W, int M, int N, int K, long lda, long ldw, long ldc,
                        int batch, long sA, long sW, long sC, uintptr_t a_rows, uintptr_t tiles, int ntiles, int in_f32,

@@ -737,15 +737,13 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(TO* __restrict__ C, cons
   }
 }
 
-// An activation in the epilogue of the few-row products: elementwise, or gated (weight rows [0, N) gate, [N, 2 N) up, with
-// the [2 N] bias of both added first); the sums are not rounded ahead of it.  Gate / up of 8
-// experts of 2 x 2048 x 2048, 64 / 96 rows: 36.9 / 40.6 us with the launch behind it, 33.2 / 34.8 us; 8 x 128 x 2048 with tanh:
-// 7.1 us, 5.6 us.
+// An activation in the epilogue of the few-row products: elementwise (plain ones), or gated (grouped ones; weight rows [0, N)
+// gate, [N, 2 N) up); the sums are not rounded ahead of it.  Gate / up of 8 experts of 2 x 2048 x 2048, 64 / 96 rows: 36.9 /
+// 40.6 us with the launch behind it, 33.2 / 34.8 us; 8 x 128 x 2048 with tanh: 7.1 us, 5.6 us.
 enum { FEW_NONE = 0, FEW_ELEM = 1, FEW_PAIR = 2 };
 struct FewAct {
   int kind;
   float limit, alpha;
-  const bf16_t* bias;
 };
 // Grouped products of few rows (decoding with experts): a workgroup takes 16 columns of one row tile (at most 64 rows).  The
 // weights go from memory straight into MFMA operands, no LDS staging; its 4 waves share the k range in 64-deep pieces (wave w
@@ -829,14 +827,7 @@ __device__ __forceinline__ void gemm_group_tile(TO* C, const bf16_t* A, const bf
       if (c >= N) continue;
       float v = y[0][e];
       if constexpr (ACT == FEW_ELEM) v = act_elem(v, act.kind, act.limit);
-      if constexpr (ACT == FEW_PAIR) {
-        float u = y[NP - 1][e];
-        if (act.bias != nullptr) {
-          v += bf2f(act.bias[c]);
-          u += bf2f(act.bias[N + c]);
-        }
-        v = act_pair(v, u, act.kind, act.limit, act.alpha);
-      }
+      if constexpr (ACT == FEW_PAIR) v = act_pair(v, y[NP - 1][e], act.kind, act.limit, act.alpha);
       stf(C, (size_t)(row0 + r) * ldc + c, v);
     }
   }
@@ -861,7 +852,7 @@ template <typename TO, int ACT>
 __global__ __launch_bounds__(256) void gemm_narrow_kernel(TO* __restrict__ C, const bf16_t* __restrict__ A,
                                                           const bf16_t* __restrict__ Wt, int M, int N, int K, long lda,
                                                           long ldw, long ldc, long sA, long sW, long sC, FewAct act) {
-  __shared__ __attribute__((aligned(16))) float red[(ACT == FEW_PAIR ? 2 : 1) * 4 * 4 * 64 * 4];
+  __shared__ __attribute__((aligned(16))) float red[4 * 4 * 64 * 4];
   const int row0 = blockIdx.y * 64, rows = min(64, M - row0);
   A += (size_t)blockIdx.z * sA;
   Wt += (size_t)blockIdx.z * sW;
@@ -1042,32 +1033,24 @@ extern "C" int k8s_act(void* out, const void* x, int T, int F, int kind, float l
   return (int)hipGetLastError();
 }
 
-// act(A W^T) in bf16 of few rows: plain (tiles == nullptr; M rows) or grouped (tiles, w [groups, .., K]); a gated `kind` takes
-// W with 2 N rows.  K % 64 == 0, rows of whole 16-byte vectors.
+// act(A W^T) in bf16 of few rows: elementwise of a plain product (tiles == nullptr; M rows), or a gated `kind` of a grouped one
+// (tiles, W [groups, 2 N, K]).  K % 64 == 0, rows of whole 16-byte vectors.
 extern "C" int k8s_gemm_few_act(void* C, const void* A, const void* W, int M, int N, int K, long lda, const int* a_rows,
-                                const int* tiles, int ntiles, int kind, float limit, float alpha, const void* bias,
-                                hipStream_t s) {
+                                const int* tiles, int ntiles, int kind, float limit, float alpha, hipStream_t s) {
   const bool pair = kind == 0 || kind == 1 || kind == 5;
   if (N <= 0 || K <= 0 || K % 64 || lda % 8 || kind < 0 || kind > 7 || (((uintptr_t)A | (uintptr_t)W) & 15)) return -1;
-  if ((bias != nullptr && (!pair || tiles != nullptr)) || (kind == 6 && !(limit > 0.f))) return -1;
-  const int gy = tiles != nullptr ? ntiles : (M + 63) / 64;
+  if (pair != (tiles != nullptr) || (kind == 6 && !(limit > 0.f))) return -1;
+  const int gy = pair ? ntiles : (M + 63) / 64;
   if (M <= 0 || gy <= 0) return 0;
   if (gy > 65535) return -2;
   const dim3 grid((N + 15) / 16, gy);
-  const FewAct act{kind, limit, alpha, (const bf16_t*)bias};
-  const long sW = (pair ? 2L : 1L) * N * K;
-#define K8S_FA(ACT)                                                                                                       \
-  do {                                                                                                                    \
-    if (tiles != nullptr)                                                                                                 \
-      gemm_group_kernel<bf16_t, ACT><<<grid, 256, 0, s>>>((bf16_t*)C, (const bf16_t*)A, (const bf16_t*)W, N, K, lda, K,   \
-                                                          N, sW, a_rows, tiles, act);                                     \
-    else                                                                                                                  \
-      gemm_narrow_kernel<bf16_t, ACT><<<grid, 256, 0, s>>>((bf16_t*)C, (const bf16_t*)A, (const bf16_t*)W, M, N, K, lda,  \
-                                                           K, N, 0, 0, 0, act);                                           \
-  } while (0)
-  if (pair) K8S_FA(FEW_PAIR);
-  else K8S_FA(FEW_ELEM);
-#undef K8S_FA
+  const FewAct act{kind, limit, alpha};
+  if (pair)
+    gemm_group_kernel<bf16_t, FEW_PAIR><<<grid, 256, 0, s>>>((bf16_t*)C, (const bf16_t*)A, (const bf16_t*)W, N, K, lda, K, N,
+                                                             2L * N * K, a_rows, tiles, act);
+  else
+    gemm_narrow_kernel<bf16_t, FEW_ELEM><<<grid, 256, 0, s>>>((bf16_t*)C, (const bf16_t*)A, (const bf16_t*)W, M, N, K, lda, K,
+                                                              N, 0, 0, 0, act);
   return (int)hipGetLastError();
 }
 
@@ -1085,7 +1068,7 @@ extern "C" int k8s_gemm_any(void* C, const void* A, const void* W, int M, int N,
     gy = (M + 63) / 64;
   }
   if (gy > 65535 || batch > 65535) return -2;
-  // bf16 rows that can be moved as 16-byte vectors: the MFMA kernel; anything else (fp32, odd strides): plain FMAs
+  // bf16 rows that can be moved as 16-byte vectors: the bf16 MFMA kernels; fp32 ones: gemm_f32_kernel; anything else: plain FMAs
   const bool vec = !in_f32 && K % 8 == 0 && lda % 8 == 0 && ldw % 8 == 0 && sA % 8 == 0 && sW % 8 == 0 &&
                    ((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0;
   if (vec && tiles != nullptr && K % 64 == 0 && M <= 32 * ntiles && M <= 512) {   // few rows per group

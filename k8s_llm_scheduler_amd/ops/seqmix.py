@@ -430,7 +430,7 @@ def gemm_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, al
         out = torch.empty(rows, N, dtype=BF16, device=a.device)
         _native().gemm_few_act(out.data_ptr(), a.data_ptr(), w.data_ptr(), rows, N, w.shape[2], a.stride(0),
                                _p(a_rows, I32, "a_rows"), _p(tiles, I32, "tiles"), tiles.shape[0], kind, float(limit),
-                               float(alpha), 0, -1)
+                               float(alpha), -1)
         return out
     return act(gemm(a, w, a_rows=a_rows, tiles=tiles, rows=rows, seg=seg), kind, limit, alpha)
 
@@ -455,7 +455,7 @@ def linear_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, 
             not (FAST_GEMM and _route_fast(a, w, BF16)):
         out = torch.empty(a.shape[0], w.shape[0], dtype=BF16, device=a.device)     # few tiles: gemm() would take that kernel
         _native().gemm_few_act(out.data_ptr(), a.data_ptr(), w.data_ptr(), a.shape[0], w.shape[0], w.shape[1], a.stride(0), 0, 0,
-                               0, kind, float(limit), float(alpha), 0, -1)
+                               0, kind, float(limit), float(alpha), -1)
         return out
     return act(linear(a, w), kind, limit, alpha, bias=bias)
 
