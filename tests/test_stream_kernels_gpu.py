@@ -4,10 +4,25 @@ bits."""
 import pytest
 import torch
 
+from k8s_llm_scheduler_amd import ops
 from k8s_llm_scheduler_amd.ops import seqmix as sm
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
+
+
+@pytest.fixture
+def entries(monkeypatch):
+    """Names of the extension's entry points in the order of their calls."""
+    nat, calls = ops.native(), []
+
+    class Spy:
+        def __getattr__(self, name):
+            calls.append(name)
+            return getattr(nat, name)
+
+    monkeypatch.setattr(ops, "native", Spy)
+    return calls
 
 
 def sum_bound(a, w):
@@ -107,6 +122,58 @@ def test_latent_prompt(dt, tol, seqs, window, H, extra, monkeypatch):
     assert (got.double() - want).abs().max() <= tol * scale
     err = lambda y: float((y.double() - want).norm() / want.norm())
     assert err(got) <= 1.1 * err(absorbed) + 1e-7      # no less exact than the absorbed form
+
+
+def attend64(q, k, v, first, scale, window=0, chunk=0, sinks=None, slopes=None, softcap=0.0):
+    """q [n, H, D] of the tokens from position ``first`` on over k, v [first + n, G, ..]: softmax in 64 bits, [n, H, V]."""
+    n, H, R = q.shape[0], q.shape[1], q.shape[1] // k.shape[1]
+    at, key = torch.arange(first, first + n, device=q.device)[:, None], torch.arange(first + n, device=q.device)[None]
+    hide = (key > at) | ((at - key >= window) if window else key > at) | ((at // chunk != key // chunk) if chunk else key > at)
+    out = []
+    for h in range(H):
+        s = (q[:, h].double() @ k[:, h // R].double().T) * scale
+        if softcap:
+            s = softcap * torch.tanh(s / softcap)
+        if slopes is not None:
+            s = s - slopes[h].double() * (at - key)
+        s = s.masked_fill(hide, -float("inf"))
+        if sinks is not None:
+            s = torch.cat([s, sinks[h].double().expand(n, 1)], 1)
+        out.append(torch.softmax(s, 1)[:, :first + n] @ v[:, h // R].double())
+    return torch.stack(out, 1)
+
+
+@pytest.mark.parametrize("dt,tol", [(torch.float32, 2e-5), (torch.bfloat16, 2e-2)])
+@pytest.mark.parametrize("window", [0, 100])
+def test_latent_prompt_idle_rows_and_non_finite_scores(dt, tol, window, monkeypatch):
+    """An idle row between two portions is zero and changes nothing; a NaN query head and a key whose rotated part makes
+    infinite scores: NaN exactly where 64 bits give NaN, the tolerance of finite keys elsewhere."""
+    C, R, D, H, bs = 512, 64, 128, 3, 16
+    g = torch.Generator().manual_seed(window)
+    r = lambda *s: torch.randn(*s, generator=g)
+    seqs, pages = [(0, 200), (-1, 1), (30, 170)], 13
+    T = sum(n for _, n in seqs)
+    q, cache = r(T, H, D + R), r(3 * pages * bs, C + R)
+    q[50, 1, D + 5] = float("nan")
+    cache[2 * pages * bs + 60, C + 9] = float("inf")
+    q, cache = q.to(dt).to(DEV), cache.to(dt).to(DEV)
+    uk, uv = ((r(H * D, C) / C ** 0.5).to(dt).to(DEV) for _ in range(2))
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    b = {"positions": i32([a + i for a, n in seqs for i in range(n)]), "cu_q": i32([0, 200, 201, 371]),
+         "tok_seq": i32([s for s, (_, n) in enumerate(seqs) for _ in range(n)]), "max_qlen": 200,
+         "block_tables": torch.arange(3 * pages, dtype=torch.int32, device=DEV).view(3, pages)}
+    monkeypatch.setattr(sm, "LATENT_EXPAND_MIN", 1)
+    got = sm.latent_mix(q.view(T, -1), cache, uk.view(H, D, C).transpose(1, 2).contiguous(), uv.view(H, D, C),
+                        sm.latent_expand(uk, uv, H, R), b, C, R, H, D, D, window, 0.07, bs).view(T, H, D)
+    assert "latent_keys" in b and (got[200] == 0).all()
+    for s, at in ((0, 0), (2, 201)):
+        first, n = seqs[s]
+        rows = cache.view(3, pages * bs, -1)[s, :first + n].double()
+        k = torch.cat([(rows[:, :C] @ uk.double().T).view(-1, H, D), rows[:, None, C:].expand(-1, H, R)], 2)
+        want = attend64(q[at:at + n], k, (rows[:, :C] @ uv.double().T).view(-1, H, D), first, 0.07, window)
+        bad, y = torch.isnan(want), got[at:at + n]
+        assert bad.any() and not bad.all() and torch.equal(bad, torch.isnan(y))
+        assert (y.double() - want)[~bad].abs().max() <= tol * want[~bad].abs().max()
 
 
 # contexts of the rows (0: idle), window: around one 64-key step, one split per step and several steps per split, windows that
@@ -267,8 +334,10 @@ def test_grouped_big_tiles(sizes, N, K, kind):
 @pytest.mark.parametrize("M,N,K", [(129, 1024, 512), (200, 520, 1024), (1031, 2048, 256), (2048, 2064, 320)])
 @pytest.mark.parametrize("kind", KINDS + ELEMENTWISE)
 @pytest.mark.parametrize("bias", [False, True])
-def test_linear_act(M, N, K, kind, bias):
-    """The activation in the epilogue, every tile configuration's edges, against 64 bits: one rounding."""
+def test_linear_act(M, N, K, kind, bias, entries):
+    """The activation in the epilogue, every tile configuration's edges, against 64 bits: one rounding.  Two launches and two
+    roundings only for 200 x 1040, which runs in k slices, and for the elementwise kinds without an epilogue of the big tiles
+    (200 x 520 is few tiles, which have one for all but the cap)."""
     if bias and kind not in KINDS:
         pytest.skip("elementwise kinds take no bias")
     g = torch.Generator().manual_seed(M + N + K + kind)
@@ -283,13 +352,20 @@ def test_linear_act(M, N, K, kind, bias):
         nat.pgemm4_act(out.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K, cfg, 4, kind, 1.5, 1.702,
                        b.data_ptr() if bias else 0, -1)
         assert ((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all(), cfg
+    entries.clear()
     got = sm.linear_act(x, w, kind, 1.5, 1.702, bias=b)
-    assert ((got.double() - want).abs() <= 2.0 ** -6 * want.abs() + 4e-2).all()
+    few = M == 200 and kind not in KINDS + [sm.ACT_SOFTCAP]
+    fused = few or (M != 200 and kind in KINDS + [sm.ACT_RELU2])
+    assert ("act" in entries) != fused and ("gemm_few_act" if few else "pgemm4_act" if fused else "act") in entries
+    if fused:
+        assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all()
+    else:
+        assert ((got.double() - want).abs() <= 2.0 ** -6 * want.abs() + 4e-2).all()
 
 
 @pytest.mark.parametrize("tokens,top,E,N,K", [(1, 1, 3, 130, 64), (5, 2, 3, 15, 128), (48, 2, 8, 72, 320), (100, 1, 2, 33, 2048)])
 @pytest.mark.parametrize("kind", KINDS)
-def test_few_rows_gated(tokens, top, E, N, K, kind):
+def test_few_rows_gated(tokens, top, E, N, K, kind, entries):
     """Tiles of at most 16 and of up to 64 rows, columns that do not fill 16, gathered rows with a stride: one rounding."""
     g = torch.Generator().manual_seed(tokens + N + K)
     idx = torch.rand(tokens, E, generator=g).argsort(1)[:, :top].to(torch.int32)
@@ -297,6 +373,7 @@ def test_few_rows_gated(tokens, top, E, N, K, kind):
     h = torch.randn(tokens, K + 8, generator=g).to(torch.bfloat16).to(DEV)[:, :K]
     w = (torch.randn(E, 2 * N, K, generator=g) * 2 / K ** 0.5).to(torch.bfloat16).to(DEV)
     got = sm.gemm_act(h, w, kind, 1.5, 1.702, a_rows=rows, tiles=tiles, rows=tokens * top).double()[pos.long()]
+    assert entries[-1] == "gemm_few_act"
     for c in range(top):
         z = (h.double().unsqueeze(1) @ w.double()[idx[:, c].long().to(DEV)].transpose(1, 2)).squeeze(1)
         want = act64(z, kind, 1.5, 1.702)
@@ -305,12 +382,13 @@ def test_few_rows_gated(tokens, top, E, N, K, kind):
 
 @pytest.mark.parametrize("M,N,K", [(1, 16, 64), (16, 130, 128), (17, 100, 64), (200, 33, 320)])
 @pytest.mark.parametrize("kind", [k for k in ELEMENTWISE if k != sm.ACT_SOFTCAP])
-def test_few_tiles_elementwise(M, N, K, kind):
+def test_few_tiles_elementwise(M, N, K, kind, entries):
     g = torch.Generator().manual_seed(M + N + K)
     x = torch.randn(M, K + 8, generator=g).to(torch.bfloat16).to(DEV)[:, 8:]
     w = (torch.randn(N, K, generator=g) * 2 / K ** 0.5).to(torch.bfloat16).to(DEV)
     want = act64(x.double() @ w.double().T, kind, 0.0, 1.0)
     assert ((sm.linear_act(x, w, kind).double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all()
+    assert entries == ["gemm_few_act"]
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 16, 64), (16, 130, 128), (17, 100, 64), (64, 15, 1024), (65, 128, 2048), (200, 33, 320),
@@ -402,15 +480,56 @@ def test_prompt_attention_key_splits(H, G, D, kw, ns, monkeypatch):
                                         sinks=torch.linspace(-3, 3, H, device=DEV), slopes=slopes).float())
     assert (outs[1][pos < 0] == 0).all()
     assert ((outs[1] - outs[0]).abs() <= 2.0 ** -7 * outs[0].abs() + 2.0 ** -13 * outs[0].abs().max()).all()
+    for s, (a, n) in enumerate(lens):
+        if a < 0:
+            continue
+        r, rows = slice(int(cu[s]), int(cu[s + 1])), torch.arange(a + n, device=DEV)
+        rows = bt[s].long()[rows // bs] * bs + rows % bs
+        want = attend64(q[r, :H * D].reshape(n, H, D), kc[rows], vc[rows], a, D ** -0.5, kw.get("window", 0), kw.get("chunk", 0),
+                        torch.linspace(-3, 3, H, device=DEV), slopes, kw.get("softcap", 0.0)).view(n, H * D)
+        want = want * torch.sigmoid(gate[r].double()) if gate is not None else want
+        for y in outs:      # one rounding to bf16; weights of two bf16 terms and fp32 scores: 2^-13 of the largest value
+            assert ((y[r].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * want.abs().max()).all()
+
+
+@pytest.mark.parametrize("ns", [1, 2, 6])
+@pytest.mark.parametrize("sink", [False, True])
+def test_prompt_attention_lets_non_finite_scores_through(ns, sink, monkeypatch):
+    """A NaN query and a key that makes infinite scores, in one piece and in key splits: NaN where 64 bits give NaN."""
+    g = torch.Generator().manual_seed(ns)
+    H, G, D, bs, first, n = 8, 4, 128, 16, 400, 70
+    q, kc, vc = (torch.randn(*s, generator=g) for s in ((n, H, D), (512, G, D), (512, G, D)))
+    q[20, 3, 7] = float("nan")
+    kc[430, 1, 5] = float("inf")
+    q, kc, vc = (t.to(torch.bfloat16).to(DEV) for t in (q, kc, vc))
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    sinks = torch.linspace(-1, 1, H, device=DEV) if sink else None
+    monkeypatch.setattr(sm, "prompt_splits", lambda groups, keys: ns)
+    got = sm.window_attention(q.view(n, -1), None, kc, vc, None, None, torch.arange(32, dtype=torch.int32, device=DEV).view(1, 32),
+                              i32([0] * n), i32(list(range(first, first + n))), H, 0, 0, D ** -0.5, sink, bs, i32([0, n]), n,
+                              sinks=sinks).view(n, H, D)
+    want = attend64(q, kc[:first + n], vc[:first + n], first, D ** -0.5, sinks=sinks)
+    bad = torch.isnan(want)
+    assert bad.any() and not bad.all() and torch.equal(bad, torch.isnan(got))
+    assert (got.double() - want)[~bad].abs().max() <= 2.0 ** -7 * want[~bad].abs().max()
 
 
 @pytest.mark.parametrize("M", [1, 32, 33, 64, 127, 129, 1031, 2048, 2049])
 @pytest.mark.parametrize("N,K", [(2048, 256), (1040, 512), (4096, 192)])
-def test_products_of_several_inputs(M, N, K):
-    """Every way a launch is shared: few tiles, even groups of the big tiles with remainders, one launch per input."""
+def test_products_of_several_inputs(M, N, K, entries):
+    """Every way a launch is shared: few tiles (up to 64, 128 and no rows of these widths), even groups of the big tiles with
+    remainders, one launch per input."""
     g = torch.Generator().manual_seed(M + N)
     a, w = (torch.randn(3, n, K, generator=g).to(torch.bfloat16) for n in (M, N))
-    got = sm.linear_each(a.to(DEV), w.to(DEV))
+    a_dev, w_dev = a.to(DEV), w.to(DEV)
+    entries.clear()
+    got = sm.linear_each(a_dev, w_dev)
+    if M <= {2048: 64, 1040: 128, 4096: 0}[N]:
+        assert entries == ["gemm_any"]
+    elif 32 < M <= 2048:
+        assert entries == ["pgemm4_grouped"]
+    else:
+        assert len(entries) >= 3 and not {"gemm_any", "pgemm4_grouped"} & set(entries)
     assert len({t.stride(0) for t in got}) == 1
     for x, y, z in zip(a, w, got):
         exact = x.double() @ y.double().T
