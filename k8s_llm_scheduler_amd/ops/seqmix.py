@@ -269,8 +269,8 @@ FAST_GEMM = os.environ.get("K8S_SEQMIX_FAST_GEMM", "1") != "0"
 
 
 def linear(a: torch.Tensor, w: torch.Tensor, out_dtype=None) -> torch.Tensor:
-    """a [M, K] @ w [N, K]^T for any shape, bf16 or fp32 operands (fp32: plain fp32 FMAs, no reduced-precision
-    matrix mode), fp32 accumulation.  Shapes that fit the tuned bf16 kernels go there."""
+    """a [M, K] @ w [N, K]^T for any shape, bf16 or fp32 operands (fp32: fp32 products and sums, on the matrix cores' fp32
+    instruction or plain FMAs, no reduced-precision mode), fp32 accumulation.  Shapes that fit the tuned bf16 kernels go there."""
     out_dtype = out_dtype or a.dtype
     if not _gpu(a, w):
         return ref.gemm_any(a, w, out_dtype)
@@ -481,7 +481,7 @@ def token_shift(h: torch.Tensor, mu: torch.Tensor, state: torch.Tensor, cu_q: to
 
 def shift_save(state: torch.Tensor, h: torch.Tensor, cu_q: torch.Tensor, seq_slots: torch.Tensor,
                positions: torch.Tensor) -> None:
-    """state[slot of s] = h[last token of sequence s]."""
+    """state[slot of s] = h[last token of sequence s]: the save of :func:`token_shift` as a launch of its own."""
     if not _gpu(h, state):
         return ref.shift_save(state, h, cu_q, seq_slots, positions)
     _native().shift_save(_p(state, h.dtype, "state"), _p(h), _p(cu_q, I32), _p(seq_slots, I32), _p(positions, I32),
@@ -623,8 +623,10 @@ def latent_attention(q_abs: torch.Tensor, q: torch.Tensor, cache: torch.Tensor, 
 # A batch of prompts writes its visible keys and values out (latent_prompt.hip) when its sequences bring at least
 # LATENT_EXPAND_MIN tokens on average: a portion that sees K rows then spends K C (Dn + V) multiply-adds per head on them
 # instead of n C (Dn + V) on its own queries and outputs, and saves n K (2 C - Dn - V) in the attention, which breaks even
-# at n = 170 for C = 512, Dn = V = 128 where everything in sight is cached already, and at any n where nothing is.  2048
-# tokens, 16 heads, window 1024: 383 us absorbed, 85 us written out; 512 tokens, 32 heads: 139 us and 42 us; fp32, 333
+# at n = 170 for C = 512, Dn = V = 128 where everything in sight is cached already, and at any n where nothing is.  The
+# average, riding single tokens included, is what the host knows (a sequence's cached length is on the device): it is safe
+# for long cached parts and leaves fresh short prompts and prompts with many riders absorbed, as they ran before this form.
+# 2048 tokens, 16 heads, window 1024: 383 us absorbed, 85 us written out; 512 tokens, 32 heads: 139 us and 42 us; fp32, 333
 # tokens, 16 heads: 1290 us and 70 us.
 LATENT_EXPAND_MIN = int(os.environ.get("K8S_LATENT_EXPAND_MIN", "160"))
 LATENT_EXPAND_BYTES = 1 << 30     # of keys and values
