@@ -30,7 +30,7 @@ GROUP_BM = 64   # row-tile height of the grouped GEMM (gemm_any_kernel's BM)
 
 
 # Short prompts are bound by their launches' preparation here: an import statement in a function costs about 1 us of every
-# call (97 tokens, 104 launches: 1475 us of preparation with them, 1396 us).
+# call (97 tokens, 118 launches: 1475 us of preparation with them, 1396 us).
 _ops = sys.modules[__package__]
 
 
