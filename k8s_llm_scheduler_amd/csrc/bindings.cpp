@@ -155,6 +155,9 @@ int k8s_act(void* out, const void* x, int T, int F, int kind, float limit, float
             const int* row_map, const void* bias, int f32, hipStream_t s);
 int k8s_gemm_few_act(void* C, const void* A, const void* W, int M, int N, int K, long lda, const int* a_rows,
                      const int* tiles, int ntiles, int kind, float limit, float alpha, hipStream_t s);
+int k8s_gemm_f32_tiles(void* C, const float* A, const float* W, int M, int N, int K, long lda, long ldw, long ldc, int batch,
+                       long sA, long sW, long sC, const int* a_rows, const int* tiles, int ntiles, int out_f32, int fq,
+                       hipStream_t s);
 int k8s_gemm_any(void* C, const void* A, const void* W, int M, int N, int K, long lda, long ldw, long ldc, int batch,
                  long sA, long sW, long sC, const int* a_rows, const int* tiles, int ntiles, int in_f32, int out_f32,
                  hipStream_t s);
@@ -576,6 +579,12 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
                            uintptr_t tiles, int ntiles, int kind, float limit, float alpha, int64_t s) {
     check(k8s_gemm_few_act(P(C), P(A), P(W), M, N, K, lda, P<int>(a_rows), P<int>(tiles), ntiles, kind, limit, alpha, S(s)),
           "gemm_few_act");
+  });
+  m.def("gemm_f32_tiles", [](uintptr_t C, uintptr_t A, uintptr_t W, int M, int N, int K, long lda, long ldw, long ldc,
+                             int batch, long sA, long sW, long sC, uintptr_t a_rows, uintptr_t tiles, int ntiles,
+                             int out_f32, int fq, intptr_t s) {
+    check(k8s_gemm_f32_tiles(P(C), P<float>(A), P<float>(W), M, N, K, lda, ldw, ldc, batch, sA, sW, sC, P<int>(a_rows),
+                             P<int>(tiles), ntiles, out_f32, fq, S(s)), "gemm_f32_tiles");
   });
   m.def("gemm_any", [](uintptr_t C, uintptr_t A, uintptr_t W, int M, int N, int K, long lda, long ldw, long ldc,
                        int batch, long sA, long sW, long sC, uintptr_t a_rows, uintptr_t tiles, int ntiles, int in_f32,

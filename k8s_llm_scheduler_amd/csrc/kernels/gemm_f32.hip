@@ -1,0 +1,229 @@
+// fp32 products of many tiles: C[M, N] = A[M, K] W[N, K]^T on v_mfma_f32_16x16x4_f32 (fp32 products and sums), K % 32 == 0.
+//
+// A workgroup of 4 waves owns 64 columns x 16 FQ rows (swapped orientation C^T = W A^T; a wave 16 columns x all rows), so the
+// row count is padded to 16 and FQ is chosen for the tiles to fill the CUs' last round.  k in 32-deep stages of 128-byte rows
+// through a ring of NS LDS slots filled by LDS-DMA (XOR swizzle on the source: conflict-free 16-byte fragment reads), one
+// barrier a stage; the fragments of the next 16 k are read between the products of the current ones.
+// Every 32, 64 (K >= 1024) or 128 (K >= 2048) k the products' registers are added to a second set: chains of that many terms
+// and then of their number, whatever the tile.  Error against 64 bits, 2-norm: K = 2048 2.2e-7, 8192 2.5e-7 (2.9e-7 and 5.8e-7
+// with the eight shares of gemm_f32_kernel).
+//
+// Bound by the matrix rate (157 TFLOP/s at 2.4 GHz; the clock holds 2.25 here): 85 % of a busy CU's cycles with two workgroups
+// on it, 75 - 80 % with one (a stage's barrier and waits cost about 350 cycles).  333 rows (N x K), with the launch: 16384 x
+// 2048 258 -> 175 us (three rounds of 112-row tiles), 2048 x 2048 42 -> 36, 2048 x 8192 154 -> 130; 200 x 16384 x 2048 165 ->
+// 116, 512 x 4096 x 4096 174 -> 137.
+#include <type_traits>
+
+#include "common.h"
+
+namespace k8sllm {
+
+template <int N>
+__device__ __forceinline__ void f32_vmcnt() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+struct F32Args {
+  void* C;
+  const float *A, *W;
+  int M, N, K, mt, nt, batch;       // mt row tiles; listed tiles: PER blocks for each
+  long lda, ldw, ldc, sA, sW, sC;
+  const int *a_rows, *tiles;
+  int vec;                          // 4 consecutive columns can be stored as one vector
+  int chain;                        // stages of a chain - 1 (a power of two less one)
+};
+
+template <typename TO, int FQ>
+__global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(F32Args a) {
+  constexpr int BP = 64, BQ = 16 * FQ, GW = BP / 32, GX = (FQ + 1) / 2, G = GW + GX, STAGE = 32 * G * 128;
+  constexpr int NS = FQ > 4 ? 3 : 4;                       // 72 KB at most: two workgroups on a CU
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ __attribute__((aligned(16))) char lds[NS * STAGE];
+  // blocks of one XCD (id % 8) take consecutive tiles, rows fastest: a column's weights are read from one L2
+  const int tot = a.mt * a.nt * a.batch, q8 = tot >> 3, r8 = tot & 7, xcd = blockIdx.x & 7;
+  int t = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (int)(blockIdx.x >> 3);
+  const int ti = t % a.mt;
+  t /= a.mt;
+  const int tj = t % a.nt, tb = t / a.nt;
+  const float *A = a.A + (size_t)tb * a.sA, *W = a.W + (size_t)tb * a.sW;
+  int row0 = ti * BQ, rows = min(BQ, a.M - row0);
+  if (a.tiles != nullptr) {
+    constexpr int PER = 64 / BQ > 0 ? 64 / BQ : 1;
+    const int y = ti / PER, sub = (ti - y * PER) * BQ, g = a.tiles[3 * y];
+    if (g < 0) return;
+    row0 = a.tiles[3 * y + 1] + sub;
+    rows = min(BQ, a.tiles[3 * y + 2] - sub);
+    if (rows <= 0) return;
+    W += (size_t)g * a.sW;
+  }
+  const int col0 = tj * BP;
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, g = lane >> 4;
+  // loader: instruction j moves the stage's rows 32 j .. 32 j + 31 (weights first), 16 bytes a thread; rows past the end
+  // repeat the last one
+  const float* src[G];
+  const int lr = tid >> 3, lc = ((tid & 7) ^ (lr & 7)) * 4;
+#pragma unroll
+  for (int j = 0; j < G; ++j) {
+    if (j < GW) {
+      src[j] = W + (size_t)min(col0 + 32 * j + lr, a.N - 1) * a.ldw + lc;
+    } else {
+      const int r = row0 + min(32 * (j - GW) + lr, rows - 1);
+      src[j] = A + (size_t)(a.a_rows != nullptr ? a.a_rows[r] : r) * a.lda + lc;
+    }
+  }
+  auto dma = [&](int u, int slot, int j) {
+    __builtin_amdgcn_global_load_lds(src[j] + (size_t)u * 32,
+                                     (__attribute__((address_space(3))) void*)(lds + slot * STAGE + wid * 1024 + j * 4096),
+                                     16, 0, 0);
+  };
+  const uint32_t base = (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)lds);
+  const uint32_t pw = base + (wid * 16 + li) * 128, px = base + (BP + li) * 128;
+  const uint32_t ch[2] = {(uint32_t)(g ^ (li & 7)) << 4, (uint32_t)((4 + g) ^ (li & 7)) << 4};
+  f32x4 w0, w1, x0[FQ], x1[FQ], acc[FQ], sum[FQ];
+#pragma unroll
+  for (int j = 0; j < FQ; ++j) sum[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Reads and products are volatile asm in program order (as in pgemm4.hip): the compiler does not drain the LDS counter
+  // ahead of every product.  Nothing touches a fragment before the lgkmcnt(0) that ends the phase of its read.
+  auto read = [&](uint32_t o, int r, f32x4& w, f32x4* x) {
+    if (r == 0) asm volatile("ds_read_b128 %0, %1" : "=v"(w) : "v"(pw + o));
+    else asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(x[r - 1]) : "v"(px + o), "i"((r - 1) * 2048));
+  };
+  // products of (wc, xc) -- `fresh`: onto zero -- with the reads at o into (wn, xn) in their first half, and in the second
+  // (u >= 0) the loads of stage u into slot us
+  auto phase = [&](auto fresh, const f32x4& wc, const f32x4* xc, f32x4& wn, f32x4* xn, uint32_t o, int u, int us) {
+    constexpr int MF = 4 * FQ;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int j = 0; j < FQ; ++j) {
+        const int k = e * FQ + j;
+        if (decltype(fresh)::value && e == 0)
+          asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, 0" : "=&v"(acc[j]) : "v"(wc[e]), "v"(xc[j][e]));
+        else
+          asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+v"(acc[j]) : "v"(wc[e]), "v"(xc[j][e]));
+#pragma unroll
+        for (int r = 0; r <= FQ; ++r)
+          if (k == r * (MF / 2) / (FQ + 1)) read(o, r, wn, xn);
+#pragma unroll
+        for (int d = 0; d < G; ++d)
+          if (k == MF / 2 + d * (MF / 2) / G && u >= 0) dma(u, us, d);
+      }
+  };
+  auto landed = [&]() {       // every wave's part of the next stage is in LDS, and every read of the current one has retired
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    f32_vmcnt<(NS - 2) * G>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto flush = [&]() {        // the products are opaque to the hazard recogniser: their results wait out the latency first
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < FQ; ++j) {
+      asm volatile("" : "+v"(acc[j]));
+      sum[j] += acc[j];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  const int S = a.K / 32;
+#pragma unroll
+  for (int q = 0; q < NS - 1; ++q)
+#pragma unroll
+    for (int d = 0; d < G; ++d) dma(min(q, S - 1), q, d);
+  landed();
+#pragma unroll
+  for (int r = 0; r <= FQ; ++r) read(ch[0], r, w0, x0);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  int slot = 0;
+  for (int s = 0; s < S; ++s) {
+    // stage s + NS - 1 (past the end: the last one again) goes into the slot of s - 1, whose reads every wave has retired
+    const int us = slot == 0 ? NS - 1 : slot - 1, u = min(s + NS - 1, S - 1);
+    const uint32_t o1 = (uint32_t)(slot * STAGE) + ch[1];
+    if ((s & a.chain) == 0) phase(std::true_type{}, w0, x0, w1, x1, o1, u, us);
+    else phase(std::false_type{}, w0, x0, w1, x1, o1, u, us);
+    slot = slot + 1 == NS ? 0 : slot + 1;
+    landed();
+    phase(std::false_type{}, w1, x1, w0, x0, (uint32_t)(slot * STAGE) + ch[0], -1, 0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    if ((s & a.chain) == a.chain || s == S - 1) flush();
+  }
+  f32_vmcnt<0>();             // no load into LDS is left behind
+  // sum[j][e] = C[row 16 j + li][column 16 wid + 4 g + e]
+  TO* C = reinterpret_cast<TO*>(a.C) + (size_t)tb * a.sC;
+  const int c = col0 + 16 * wid + 4 * g;
+#pragma unroll
+  for (int j = 0; j < FQ; ++j) {
+    const int r = 16 * j + li;
+    if (r >= rows || c >= a.N) continue;
+    const size_t at = (size_t)(row0 + r) * a.ldc + c;
+    if (a.vec) {
+      stf4(C + at, sum[j]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < a.N) stf(C, at + e, sum[j][e]);
+    }
+  }
+#endif
+}
+
+}  // namespace k8sllm
+
+using namespace k8sllm;
+
+// The tile for a product, and whether it is expected to beat gemm_f32_kernel's tiles (0: it is not): both in us per 32 k, one
+// constant part and one per round of tiles over the CUs, fitted to M 24 - 512, N 128 - 16384, K 512 - 8192 (where the two
+// models are within 5 % of each other, so are the kernels).  K < 512: shares of K / 8 leave the smaller error.
+extern "C" int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles) {
+  if (K < 512 || K % 32 || M <= 0 || N <= 0) return 0;
+  const auto rounds = [&](long rows, long cols) { return (double)((rows * cols * batch + 255) / 256); };
+  const long gm = ntiles > 0 ? 2L * ntiles : (M + 31) / 32;
+  const double r1 = rounds(gm, (N + 31) / 32), r2 = rounds(gm, (N + 63) / 64);
+  double best = 2.0 * r2 < 1.1 * r1 ? 0.365 * r2 + 0.03 : 0.16 * r1 + 0.1;
+  int pick = 0;
+  for (int fq = 8; fq >= 1; --fq) {
+    if (ntiles > 0 && 64 % (16 * fq)) continue;
+    const double t = rounds(ntiles > 0 ? 4L / fq * ntiles : (M + 16 * fq - 1) / (16 * fq), (N + 63) / 64) * (0.125 * fq + 0.04) + 0.1;
+    if (t < best) {
+      best = t;
+      pick = fq;
+    }
+  }
+  return pick;
+}
+
+// fq: rows of a tile / 16 (1 - 8; listed tiles of at most 64 rows: 1, 2, 4).
+extern "C" int k8s_gemm_f32_tiles(void* C, const float* A, const float* W, int M, int N, int K, long lda, long ldw, long ldc,
+                                  int batch, long sA, long sW, long sC, const int* a_rows, const int* tiles, int ntiles,
+                                  int out_f32, int fq, hipStream_t s) {
+  if (M <= 0 || N <= 0 || K < 32 || K % 32 || batch <= 0 || fq < 1 || fq > 8 || (lda | ldw | sA | sW) % 4 ||
+      (((uintptr_t)A | (uintptr_t)W) & 15))
+    return -1;
+  if (tiles != nullptr && (64 % (16 * fq) || ntiles <= 0)) return -1;
+  F32Args a = {C, A, W, M, N, K, 0, 0, 0, lda, ldw, ldc, sA, sW, sC, a_rows, tiles, 0};
+  a.mt = tiles != nullptr ? ntiles * (4 / fq) : (M + 16 * fq - 1) / (16 * fq);
+  a.nt = (N + 63) / 64;
+  a.batch = tiles != nullptr ? 1 : batch;
+  const long long blocks = (long long)a.mt * a.nt * a.batch;
+  if (blocks > (1LL << 30)) return -2;
+  a.vec = N % 4 == 0 && ldc % 4 == 0 && sC % 4 == 0 && ((uintptr_t)C & 15) == 0;
+  a.chain = K >= 2048 ? 3 : K >= 1024 ? 1 : 0;
+  auto go = [&](auto n) {
+    constexpr int FQ = decltype(n)::value;
+    if (out_f32) gemm_f32_tile_kernel<float, FQ><<<dim3((unsigned)blocks), 256, 0, s>>>(a);
+    else gemm_f32_tile_kernel<bf16_t, FQ><<<dim3((unsigned)blocks), 256, 0, s>>>(a);
+  };
+  switch (fq) {
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 3: go(std::integral_constant<int, 3>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    case 5: go(std::integral_constant<int, 5>{}); break;
+    case 6: go(std::integral_constant<int, 6>{}); break;
+    case 7: go(std::integral_constant<int, 7>{}); break;
+    case 8: go(std::integral_constant<int, 8>{}); break;
+  }
+  return (int)hipGetLastError();
+}

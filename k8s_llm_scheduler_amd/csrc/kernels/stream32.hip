@@ -552,7 +552,7 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(TO* __restrict__ C, const
 // the tile or the rows that share it.  Same three forms.
 // Bound by the fp32 matrix rate (157 TFLOP/s; a 32 x 32 x 2048 tile is 7 us of a CU's four pipes).  333 rows: 2048 x 2048
 // (N x K) 40 us (503 us with gemm_any_kernel; 70 TFLOP/s now), 16384 x 2048 270 us (434), 128 x 2048 16 us with the launch
-// (276).  Tiles of 64 x 64 with a wave per 32 x 32 part took 62, 265 and 56 us: one wave per SIMD and a chain of loads.
+// (276).  What fills the chip in tiles of 64 columns runs on gemm_f32.hip's.
 template <typename TO, int NN>
 __global__ __launch_bounds__(512) void gemm_f32_kernel(TO* __restrict__ C, const float* __restrict__ A,
                                                        const float* __restrict__ Wt, int M, int N, int K, long lda,
@@ -1054,6 +1054,11 @@ extern "C" int k8s_gemm_few_act(void* C, const void* A, const void* W, int M, in
   return (int)hipGetLastError();
 }
 
+extern "C" int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles);
+extern "C" int k8s_gemm_f32_tiles(void* C, const float* A, const float* W, int M, int N, int K, long lda, long ldw, long ldc,
+                                  int batch, long sA, long sW, long sC, const int* a_rows, const int* tiles, int ntiles,
+                                  int out_f32, int fq, hipStream_t s);
+
 extern "C" int k8s_gemm_any(void* C, const void* A, const void* W, int M, int N, int K, long lda, long ldw, long ldc,
                             int batch, long sA, long sW, long sC, const int* a_rows, const int* tiles, int ntiles,
                             int in_f32, int out_f32, hipStream_t s) {
@@ -1104,6 +1109,12 @@ extern "C" int k8s_gemm_any(void* C, const void* A, const void* W, int M, int N,
   const int gm = tiles != nullptr ? gy * 2 : (M + 31) / 32;     // fp32 tiles are 32 rows high
   if (in_f32 && K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && sA % 4 == 0 && sW % 4 == 0 && ((uintptr_t)A & 15) == 0 &&
       ((uintptr_t)W & 15) == 0 && gm <= 65535) {
+    const int fq = k8s_gemm_f32_rule(M, N, K, batch, tiles != nullptr ? ntiles : 0);
+    if (fq > 0) {
+      const int rc = k8s_gemm_f32_tiles(C, (const float*)A, (const float*)W, M, N, K, lda, ldw, ldc, batch, sA, sW, sC, a_rows,
+                                        tiles, ntiles, out_f32, fq, s);
+      if (rc != -2) return rc;
+    }
     // 32 x 64 tiles take about 1.8 times a 32 x 32 one (333 x 2048 x 2048: 50 us and 40 us; 512 rows: 49 and 52; 1 x 16384 x
     // 2048: 32 and 39): the shape whose tiles fill the last round over the CUs better
     const long t1 = (long)gm * ((N + 31) / 32) * batch, t2 = (long)gm * ((N + 63) / 64) * batch;
