@@ -8,22 +8,27 @@
 // the LDS instructions of the library's 256 x 256 kernel, which runs 4 waves of 128 x 128
 // (profiles/pmc_pgemm_vs_hipblaslt_M2048_oproj_tp1.txt).  Here every wave owns a 128 x 128 output (64
 // fragments of v_mfma_f32_16x16x32_bf16, 256 accumulator registers: the AGPR half of the unified file at one
-// wave per SIMD), so per 32-deep k-step a wave issues 16 fragment reads for 64 MFMAs.
+// wave per SIMD), so per 32 k a wave issues 16 fragment reads for 64 MFMAs.
 //
-//  * ring of 4 LDS k-steps (BP + BQ rows x 64 bytes each, 128 KiB at 256 x 256) filled by LDS-DMA
-//    (global_load_lds_dwordx4); k-step s+3 is issued right after the barrier of iteration s into the slot
-//    k-step s-1 vacated, so three k-steps (two MFMA blocks, ~2k cycles) of DMA are in flight across the raw
-//    s_barriers; the one wait per k-step is a counted `s_waitcnt vmcnt` (never 0 in the steady state).
-//  * register double buffer: the fragments of k-step s+1 are read (ds_read_b128) before the 64 MFMAs of
-//    k-step s, so the LDS latency hides under the matrix pipe of the same wave.
-//  * DMA image lane-linear, XOR swizzle on the per-lane global source (16-byte chunk c of row r in slot
-//    c ^ ((r >> 2) & 3)): the 16-row fragment reads are conflict-free on 64-byte rows.
+//  * 64-deep LDS stages of 128-byte rows (every LDS-DMA instruction moves 8 whole rows): three of weights, two of x -- all of
+//    the CU's 160 KB at 256 x 256, two workgroups on a CU at 128 x 128.  x comes from L2; the weights, from memory, are two
+//    stages (about 2 us) in flight across the raw s_barriers, of which there is one per 2 x FP x FQ MFMAs.
+//  * register double buffer: the fragments of the next 32 k are read (ds_read_b128) under the MFMAs of the current ones, in
+//    the first half of them: spread over all of them, the wait at the end stood 100 - 150 of 1024 matrix cycles a step.
+//  * DMA image lane-linear, XOR swizzle on the per-lane global source: the 16-row fragment reads are conflict-free.
+//  * bf16 output through LDS, in 64 - 256-byte runs of a row a store instead of 32-byte pieces of 16 rows.
 //  * swapped orientation C^T = W . x^T: every lane ends with 4 consecutive features of one token (gate/up
 //    rows of one feature sit in the same lane for the SwiGLU epilogue).
 //  * XCD-aware bijective block remap, group_m m-tiles per n-column group, k-slices of a tile adjacent.
 //  * split-K: every slice stores fp32 partial sums into its own slab [M][W rows] (plus the RMS row sums) and
 //    pgemm_reduce_kernel sums the slabs in slice order (deterministic) and applies the epilogue -- a
 //    parallel reduction over the whole chip instead of one last-arriving workgroup reading every slab.
+//
+// us, weights from memory (rows x N x K), with 32-deep stages, reads and stores spread as they fell -> now, and hipBLASLt:
+// 256 x 256 tiles 2048 x 8192 x 2048 64 -> 56 (52), x 8192 208 -> 188 (188), 3413 x 8192 x 8192 364 -> 342 (333); 128 x 256
+// 2048 x 8192 x 2048 82 -> 64; 128 x 128 2048 x 2048 x 2048 25 -> 22 (22), x 8192 94 -> 73 (78).  Bound by the matrix rate at
+// the clock that the power allows (1.7 - 2.0 GHz in long launches; operands all zero take 25 % less time): 89 % of a stage's
+// cycles are the matrix cores', and at K = 2048 a fifth of the launch is its start, first loads and stores.
 #include <type_traits>
 
 #include "common.h"
@@ -43,10 +48,16 @@ __device__ __forceinline__ void p4_sync() {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 }
+// LDS-DMA of 16 bytes a lane, from a uniform base and the lane's 32-bit offset to LDS byte `lds` + 16 lane.  In asm: from the
+// builtin the compiler hoists base + offset, or the widened offset, into 64-bit lane addresses and adds the step to each of
+// them, an instruction and two registers per load.
+__device__ __forceinline__ void p4_dma(const uint8_t* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
+}
 __device__ __forceinline__ float p4_silu(float g) { return g / (1.f + __expf(-g)); }
 // Activations of the epilogues (kinds as in stream32.hip), on the hardware's exponential and reciprocal: a sigmoid of x is
-// off by about (|x| + 4) 2^-24 relative (the exponent x log2 e is rounded to fp32), the result is then rounded to bf16.  The kind is a template argument: 128 unrolled elements per lane with every kind's branches
-// took 775 us where the product takes 64.
+// off by about (|x| + 4) 2^-24 relative (the exponent x log2 e is rounded to fp32), the result is then rounded to bf16.  The
+// kind is a template argument: 128 unrolled elements per lane with every kind's branches took 775 us where the product takes 56.
 __device__ __forceinline__ float p4_sigmoid(float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 template <int KIND>
 __device__ __forceinline__ float p4_pair(float g, float u, float limit, float alpha) {
@@ -71,6 +82,7 @@ struct P4Args {
   int M, N_out, half_rows, wrows, K;
   int m_tiles, n_tiles, ks, splits, group_m, nwg;
   float eps;
+  int wide;              // the output's rows can be stored in 16-byte pieces
   float limit, alpha;    // P4_GLU: of the gated kind
   const bf16_t* bias;    // P4_GLU, optional: [gate; up] biases
   // grouped form: group g's rows are [seg[g], seg[g + 1]) of a compact row space (row r of x: a_rows[r], or r) and its
@@ -84,22 +96,18 @@ struct P4Args {
   int groups;
 };
 
-template <int FP, int FQ, int EPI, bool RMS, bool K64 = false, bool GRP = false, int KIND = -1>
+template <int FP, int FQ, int EPI, bool RMS, bool GRP = false, int KIND = -1>
 __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
   constexpr int BP = 32 * FP, BQ = 32 * FQ;          // weight rows, tokens per tile (2 x 2 waves)
   constexpr bool PAIR = EPI == P4_SWIGLU || EPI == P4_GLU;   // gate and up rows of one feature in one wave
-  static_assert(!GRP || (!RMS && !K64), "the grouped form has no prologue and 32-deep stages");
-  constexpr int ROWS = BP + BQ;
-  constexpr int SUB = ROWS * 64;                     // one 32-deep k-step of both operands
-  constexpr int G = ROWS / 64;                       // 16-byte DMA instructions per thread per k-step
-  constexpr int NSLOT = 4;
-  static_assert(ROWS % 64 == 0 && G >= 1, "tile shape");
-  // K64: 64-deep LDS stages of 128-byte rows, two of them (the same 4 x 32-deep bytes): every LDS-DMA instruction
-  // moves 8 whole 128-byte rows instead of 16 half rows, and one barrier covers 2 x FP x FQ MFMAs
-  constexpr int RING = K64 ? 2 * ROWS * 128 : NSLOT * SUB;
+  static_assert(!GRP || !RMS, "the grouped form has no prologue");
+  constexpr int SUBW = BP * 128, SUBX = BQ * 128;    // a 64-deep stage of either operand
+  constexpr int GW = BP / 32, GX = BQ / 32;          // 16-byte DMA instructions per thread and stage
+  constexpr int X0 = 3 * SUBW, RING = X0 + 2 * SUBX;
+  constexpr int RSS = RING - BQ * 8;                 // in the last stage's memory, once it has been read
 #if defined(__HIP_DEVICE_COMPILE__)
-  __shared__ __attribute__((aligned(16))) char lds[RING + BQ * 8];
-  float* rss = reinterpret_cast<float*>(lds + RING);   // [2][BQ] row sums of squares (wave rows)
+  __shared__ __attribute__((aligned(16))) char lds[RING];
+  float* rss = reinterpret_cast<float*>(lds + RSS);   // [2][BQ] row sums of squares (wave rows)
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -145,76 +153,42 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
     return (uint32_t)m;
   };
   const int ks0 = 2 * (int)((long long)slice * (a.ks / 2) / a.splits);
-  const int n = 2 * (int)((long long)(slice + 1) * (a.ks / 2) / a.splits) - ks0;   // even, >= 2
+  const int n2 = (int)((long long)(slice + 1) * (a.ks / 2) / a.splits) - ks0 / 2;   // 64-deep stages, >= 1
 
-  // ---- per-thread DMA sources: chunk p = j * 256 + tid of the k-step image (rows 0..BP-1 weights, then x);
-  // instructions j < GW cover weight rows only, the rest x rows only
-  constexpr int GW = BP / 64;
-  uint32_t off[G];
+  // ---- per-thread DMA sources: chunk p = j * 256 + tid of the stage image, 8 chunks of 16 bytes a row
+  const uint32_t col0 = (uint32_t)(ks0 * 64);
+  uint32_t wo[GW], xo[GX];
 #pragma unroll
-  for (int j = 0; j < G; ++j) {
-    const int p = j * 256 + tid, r = p >> 2, c = (p & 3) ^ ((r >> 2) & 3);
-    const uint32_t col = (uint32_t)(c * 16 + ks0 * 64);
-    if (j < GW) {
-      const int w = r / (BP / 2), q = r % (BP / 2);
-      int row;
-      if constexpr (PAIR) {   // wave rows: BP/4 gate rows then the matching BP/4 up rows
-        const int f = min(nt * (BP / 2) + w * (BP / 4) + (q % (BP / 4)), a.N_out - 1);
-        row = q < BP / 4 ? f : a.half_rows + f;
-      } else {
-        row = min(nt * BP + r, a.N_out - 1);
-      }
-      off[j] = (uint32_t)row * a.kbytes + col;
+  for (int j = 0; j < GW; ++j) {
+    const int p = j * 256 + tid, r = p >> 3, c = (p & 7) ^ ((r >> 1) & 7);
+    const int w = r / (BP / 2), q = r % (BP / 2);
+    int row;
+    if constexpr (PAIR) {   // wave rows: BP/4 gate rows then the matching BP/4 up rows
+      const int f = min(nt * (BP / 2) + w * (BP / 4) + (q % (BP / 4)), a.N_out - 1);
+      row = q < BP / 4 ? f : a.half_rows + f;
     } else {
-      off[j] = xrow(r - BP) * (GRP ? a.xbytes : a.kbytes) + col;
+      row = min(nt * BP + r, a.N_out - 1);
     }
+    wo[j] = (uint32_t)row * a.kbytes + (uint32_t)(c * 16) + col0;
   }
-  auto issue = [&](int u) {   // k-step u of this slice into slot u % 4
-    char* dst = lds + (u & (NSLOT - 1)) * SUB + wid * 1024;
-    const uint32_t kb = (uint32_t)u * 64u;
 #pragma unroll
-    for (int j = 0; j < G; ++j)
-      __builtin_amdgcn_global_load_lds((j < GW ? Wb : a.x) + (off[j] + kb),
-                                       (__attribute__((address_space(3))) void*)(dst + j * 4096), 16, 0, 0);
+  for (int j = 0; j < GX; ++j) {
+    const int p = j * 256 + tid, r = p >> 3, c = (p & 7) ^ ((r >> 1) & 7);
+    xo[j] = xrow(r) * (GRP ? a.xbytes : a.kbytes) + (uint32_t)(c * 16) + col0;
+  }
+  // this wave's 1 KB of the first 4 KB of LDS
+  const uint32_t lds0 = (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)lds) + wid * 1024;
+  auto dma_w = [&](int u, int slot, int d) {   // instruction d of stage u's weights (slot u % 3), of its x
+    p4_dma(Wb + (size_t)u * 128, wo[d], lds0 + slot * SUBW + d * 4096);
   };
+  auto dma_x = [&](int u, int d) { p4_dma(a.x + (size_t)u * 128, xo[d], lds0 + X0 + (u & 1) * SUBX + d * 4096); };
 
-  // ---- fragment reads: row li of a 16-row fragment, chunk g (k 8g .. 8g+7), swizzled
-  const int lo = li * 64 + ((g ^ (li >> 2)) << 4);
-  const int pb = (wr * (BP / 2)) * 64 + lo, qb = (BP + wc * (BQ / 2)) * 64 + lo;
   bf16x8 A0[FP], B0[FQ], A1[FP], B1[FQ];
-  // The fragment reads are inline asm as well: a compiler-visible LDS read ahead of the (opaque) asm MFMAs made the
-  // compiler drain lgkmcnt(0) before the first MFMA, exposing the whole read latency every k-step.  Nothing reads
-  // An / Bn before the next k-step's p4_sync, whose lgkmcnt(0) retires these reads.
-  auto rd = [&](int u, bf16x8* A, bf16x8* B) {
-    const char* sb = lds + (u & (NSLOT - 1)) * SUB;
-    const uint32_t la = (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)(sb + pb));
-    const uint32_t lb = (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)(sb + qb));
-#pragma unroll
-    for (int f = 0; f < FP; ++f) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(A[f]) : "v"(la), "i"(f * 1024));
-#pragma unroll
-    for (int f = 0; f < FQ; ++f) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(B[f]) : "v"(lb), "i"(f * 1024));
-  };
-
   f32x4 acc[FP][FQ];
-#pragma unroll
-  for (int i = 0; i < FP; ++i)
-#pragma unroll
-    for (int j = 0; j < FQ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   float ss[FQ];
 #pragma unroll
   for (int f = 0; f < FQ; ++f) ss[f] = 0.f;
 
-  // MFMAs of fragment rows [i0, i1) on one k-step's registers (+ the RMS squares of the x fragments)
-  auto mma = [&](const bf16x8* A, const bf16x8* B, int i0, int i1) {
-#pragma unroll
-    for (int i = 0; i < FP; ++i)
-      if (i >= i0 && i < i1)
-#pragma unroll
-        for (int j = 0; j < FQ; ++j)
-          // in place, in inline asm: the AGPR tile stays put (with the builtin the register allocator rotated the
-          // accumulators through AGPR <-> VGPR copies, 2.2-3.7 per MFMA in every configuration; 11-13 % slower)
-          asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(A[i]), "v"(B[j]));
-  };
   auto squares = [&](const bf16x8* B, bool sq) {
     if constexpr (RMS) {
       if (sq) {   // the two wave rows hold the same x fragments: each squares every other k-step
@@ -228,185 +202,121 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
       }
     }
   };
-  // One k-step s: make s+1 visible (counted vmcnt + barrier), refill the slot of s-1 with s+3 (LDS-DMA), read
-  // s+1 into the other register set, then the 64 MFMAs on s (registers read one k-step earlier).
-  // One k-step s: make s+1 visible (counted vmcnt + barrier), then the 64 MFMAs on s (registers read one k-step
-  // earlier) with the LDS-DMA refill of s-1's slot by s+3 and the fragment reads of s+1 spread between them: one wave
-  // per SIMD, so nothing else would hide a DMA issue or an LDS read (all three are volatile asm or side-effecting
-  // builtins, so this program order is the issue order).
-  auto step_full = [&](int s, bf16x8* Ac, bf16x8* Bc, bf16x8* An, bf16x8* Bn) {
-    p4_vmcnt<G>();
-    p4_sync();
-    __builtin_amdgcn_sched_barrier(0);
-    constexpr int MF = FP * FQ, DR = FP + FQ;
-    char* dst = lds + ((s + 3) & (NSLOT - 1)) * SUB + wid * 1024;
-    const uint32_t kb = (uint32_t)(s + 3) * 64u;
-    const char* sb = lds + ((s + 1) & (NSLOT - 1)) * SUB;
-    const uint32_t la = (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)(sb + pb));
-    const uint32_t lb = (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)(sb + qb));
+  // Called with the first k-steps' loads in flight (the zero comes out of an asm behind them, 256 register writes would
+  // otherwise go first).  The inline-asm MFMAs are opaque to the hazard recognizer: every zeroed accumulator passes through
+  // an asm tied to it after its write, all before the first MFMA (volatile asm keeps its order).
+  auto clear = [&]() {
+    float z;
+    asm volatile("v_mov_b32 %0, 0" : "=v"(z));
 #pragma unroll
     for (int i = 0; i < FP; ++i)
 #pragma unroll
-    for (int j = 0; j < FQ; ++j) {
-      const int k = i * FQ + j;
-#pragma unroll
-      for (int d = 0; d < G; ++d)
-        if (k == d * MF / G)
-          __builtin_amdgcn_global_load_lds((d < GW ? Wb : a.x) + (off[d] + kb),
-                                           (__attribute__((address_space(3))) void*)(dst + d * 4096), 16, 0, 0);
-      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(Ac[i]), "v"(Bc[j]));
-#pragma unroll
-      for (int r = 0; r < DR; ++r)
-        if (k == r * MF / DR + MF / (2 * DR)) {
-          if (r < FP)
-            asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(An[r]) : "v"(la), "i"(r * 1024));
-          else
-            asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(Bn[r - FP]) : "v"(lb), "i"((r - FP) * 1024));
-        }
-    }
-    squares(Bc, (s & 1) == wr);
-  };
-  auto step_tail = [&](int s, bf16x8* Ac, bf16x8* Bc, bf16x8* An, bf16x8* Bn) {
-    if (s + 1 < n) {
-      if (s + 2 < n) p4_vmcnt<G>(); else p4_vmcnt<0>();
-      p4_sync();
-      if (s + 3 < n) issue(s + 3);
-      rd(s + 1, An, Bn);
-    }
-    mma(Ac, Bc, 0, FP);
-    squares(Bc, (s & 1) == wr);
-  };
-
-  {   // the inline-asm MFMAs are opaque to the hazard recognizer: every zeroed accumulator passes through an asm
-    // tied to it after its write, all before the first MFMA (volatile asm keeps its order)
+      for (int j = 0; j < FQ; ++j) acc[i][j] = f32x4{z, z, z, z};
     asm volatile("s_nop 1" ::: "memory");
 #pragma unroll
     for (int i = 0; i < FP; ++i)
 #pragma unroll
       for (int j = 0; j < FQ; ++j) asm volatile("s_nop 0" : "+a"(acc[i][j]));
-  }
-  if constexpr (K64) {
-    // ---- 64-deep stages: stage u in slot u & 1, row r at r * 128 bytes, 16-byte chunk c of row r at slot
-    // c ^ ((r >> 1) & 7) (the swizzle is applied on the per-lane global source, the DMA image is lane-linear).
-    // Sub-step h (k 32 h .. 32 h + 31) of a fragment row li = chunks 4 h + g.  Register sets: R0 = (A0, B0) holds
-    // sub-step 0, R1 = (A1, B1) sub-step 1.  Per stage s after the barrier: phase A = the MFMAs of (s - 1, 1) on R1
-    // with the reads of (s, 0) into R0 and the LDS-DMA of stage s + 1 (into the slot of s - 1, whose reads every
-    // wave retired before the barrier) spread between them; phase P = the MFMAs of (s, 0) on R0 with the reads of
-    // (s, 1) into R1.
-    constexpr int SUB2 = ROWS * 128, G2 = ROWS / 32, GW2 = BP / 32;
-    const int n2 = n / 2;
-    uint32_t off2[G2];
+  };
+  // ---- 64-deep stages: weights of stage u in slot u % 3, x in slot u & 1; row r at r * 128 bytes, 16-byte chunk c of row
+  // r at slot c ^ ((r >> 1) & 7) (the swizzle is applied on the per-lane global source, the DMA image is lane-linear).
+  // Sub-step h (k 32 h .. 32 h + 31) of a fragment row li = chunks 4 h + g.  Register sets: R0 = (A0, B0) holds
+  // sub-step 0, R1 = (A1, B1) sub-step 1.  Per stage s after the barrier: phase A = the MFMAs of (s - 1, 1) on R1
+  // with the reads of (s, 0) into R0, the LDS-DMA of x of stage s + 1 and then of the weights of stage s + 2 (into the
+  // slots of s - 1, whose reads every wave retired before the barrier) spread between them; phase P = the MFMAs of (s, 0)
+  // on R0 with the reads of (s, 1) into R1.  x comes from L2; the weights, from memory, are two stages (about 2 us) in
+  // flight, and the wait of a stage leaves the next one's weights outstanding.
+  // The fragment reads go out in the first half of a phase: at its end, where they had been spread to, the wait for them
+  // stood 100 - 150 of 1024 matrix cycles per phase (8192 columns, 2048 rows, all operands zero: K = 8192 160 -> 140 us).
+  const int lo0 = li * 128 + ((g ^ (li >> 1)) << 4), lo1 = li * 128 + (((4 + g) ^ (li >> 1)) << 4);
+  const int pb2 = wr * (BP / 2) * 128, qb2 = X0 + wc * (BQ / 2) * 128;
+  auto laddr = [&](int off) {
+    return (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)(lds + off));
+  };
+  auto rd2 = [&](bf16x8* A, bf16x8* B) {   // (0, 0), not interleaved
+    const uint32_t la = laddr(pb2 + lo0), lb = laddr(qb2 + lo0);
 #pragma unroll
-    for (int j = 0; j < G2; ++j) {
-      const int p = j * 256 + tid, r = p >> 3, c = (p & 7) ^ ((r >> 1) & 7);
-      const uint32_t col = (uint32_t)(c * 16 + ks0 * 64);
-      if (j < GW2) {
-        const int w = r / (BP / 2), q = r % (BP / 2);
-        int row;
-        if constexpr (PAIR) {
-          const int f = min(nt * (BP / 2) + w * (BP / 4) + (q % (BP / 4)), a.N_out - 1);
-          row = q < BP / 4 ? f : a.half_rows + f;
-        } else {
-          row = min(nt * BP + r, a.N_out - 1);
-        }
-        off2[j] = (uint32_t)row * a.kbytes + col;
-      } else {
-        off2[j] = xrow(r - BP) * a.kbytes + col;
+    for (int f = 0; f < FP; ++f) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(A[f]) : "v"(la), "i"(f * 2048));
+#pragma unroll
+    for (int f = 0; f < FQ; ++f) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(B[f]) : "v"(lb), "i"(f * 2048));
+  };
+  // 64 MFMAs on (Ac, Bc) with (rd) the reads of sub-step h of stage u into (An, Bn), (dx) the loads of x of stage u + 1 and
+  // (dw) of the weights of stage u + 2 spread between them
+  auto phase = [&](const bf16x8* Ac, const bf16x8* Bc, int u, int ws, int h, bf16x8* An, bf16x8* Bn, auto rdc, auto dxc,
+                   auto dwc) {   // ws = u % 3
+    constexpr int MF = FP * FQ, DR = FP + FQ;
+    constexpr bool rd = decltype(rdc)::value, dx = decltype(dxc)::value, dw = decltype(dwc)::value;
+    const uint32_t la = laddr(ws * SUBW + pb2 + (h ? lo1 : lo0)), lb = laddr((u & 1) * SUBX + qb2 + (h ? lo1 : lo0));
+    const int wt = ws == 0 ? 2 : ws - 1;               // the slot of stage u + 2
+#pragma unroll
+    for (int i = 0; i < FP; ++i)
+#pragma unroll
+      for (int j = 0; j < FQ; ++j) {
+        const int k = i * FQ + j;
+#pragma unroll
+        for (int d = 0; d < (GW + GX); ++d)
+          if (k == d * MF / (GW + GX)) {
+            if (d < GX && dx) dma_x(u + 1, d);
+            if (d >= GX && dw) dma_w(u + 2, wt, d - GX);
+          }
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(Ac[i]), "v"(Bc[j]));
+#pragma unroll
+        for (int r = 0; r < DR; ++r)
+          if (k == 1 + r * (MF / 2) / DR && rd) {
+            if (r < FP)
+              asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(An[r]) : "v"(la), "i"(r * 2048));
+            else
+              asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(Bn[r - FP]) : "v"(lb), "i"((r - FP) * 2048));
+          }
       }
-    }
-    auto dma2 = [&](int u, int d) {   // instruction d of stage u
-      __builtin_amdgcn_global_load_lds((d < GW2 ? Wb : a.x) + (off2[d] + (uint32_t)u * 128u),
-                                       (__attribute__((address_space(3))) void*)(lds + (u & 1) * SUB2 + wid * 1024 +
-                                                                                 d * 4096),
-                                       16, 0, 0);
-    };
-    const int lo0 = li * 128 + ((g ^ (li >> 1)) << 4), lo1 = li * 128 + (((4 + g) ^ (li >> 1)) << 4);
-    const int pb2 = wr * (BP / 2) * 128, qb2 = (BP + wc * (BQ / 2)) * 128;
-    auto laddr = [&](int u, int off) {
-      return (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)(lds + (u & 1) * SUB2 + off));
-    };
-    auto rd2 = [&](int u, int h, bf16x8* A, bf16x8* B) {   // whole sub-step, not interleaved (prologue / tail)
-      const uint32_t la = laddr(u, pb2 + (h ? lo1 : lo0)), lb = laddr(u, qb2 + (h ? lo1 : lo0));
+  };
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  // prologue: weights of stages 0 - 2 and x of stages 0 and 1 in flight, stage 0 visible, (0, 0) read
+  auto all_w = [&](int u) {
 #pragma unroll
-      for (int f = 0; f < FP; ++f) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(A[f]) : "v"(la), "i"(f * 2048));
+    for (int d = 0; d < GW; ++d) dma_w(u, u, d);
+  };
+  auto all_x = [&](int u) {
 #pragma unroll
-      for (int f = 0; f < FQ; ++f) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(B[f]) : "v"(lb), "i"(f * 2048));
-    };
-    // 64 MFMAs on (Ac, Bc) with the reads of sub-step h of stage u into (An, Bn) and (dma) the G2 instructions of
-    // stage u + 1 spread between them
-    auto phase = [&](const bf16x8* Ac, const bf16x8* Bc, int u, int h, bf16x8* An, bf16x8* Bn, bool rd, bool dma) {
-      constexpr int MF = FP * FQ, DR = FP + FQ;
-      const uint32_t la = laddr(u, pb2 + (h ? lo1 : lo0)), lb = laddr(u, qb2 + (h ? lo1 : lo0));
-#pragma unroll
-      for (int i = 0; i < FP; ++i)
-#pragma unroll
-        for (int j = 0; j < FQ; ++j) {
-          const int k = i * FQ + j;
-#pragma unroll
-          for (int d = 0; d < G2; ++d)
-            if (k == d * MF / G2 && dma) dma2(u + 1, d);
-          asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(Ac[i]), "v"(Bc[j]));
-#pragma unroll
-          for (int r = 0; r < DR; ++r)
-            if (k == 4 + r * (MF - 8) / DR && rd) {   // the first read 4 MFMAs in: the previous phase's
-                                                       // MFMAs on these registers are long issued
-              if (r < FP)
-                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(An[r]) : "v"(la), "i"(r * 2048));
-              else
-                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(Bn[r - FP]) : "v"(lb), "i"((r - FP) * 2048));
-            }
-        }
-    };
-    // prologue: stages 0 (and 1) in flight, stage 0 visible, (0, 0) read
-#pragma unroll
-    for (int d = 0; d < G2; ++d) dma2(0, d);
-    p4_vmcnt<0>();
-    p4_sync();
-    rd2(0, 0, A0, B0);
-    if (n2 > 1) {
-#pragma unroll
-      for (int d = 0; d < G2; ++d) dma2(1, d);
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    phase(A0, B0, 0, 1, A1, B1, true, false);           // P_0: (0, 0) on R0, read (0, 1)
-    squares(B0, wr == 0);
-    for (int s2 = 1; s2 < n2; ++s2) {
-      p4_vmcnt<0>();                                     // stage s2 landed (this wave's DMA)
-      p4_sync();                                         // ... for every wave; (s2 - 1, 1) reads retired
-      __builtin_amdgcn_sched_barrier(0);
-      phase(A1, B1, s2, 0, A0, B0, true, s2 + 1 < n2);   // A: (s2 - 1, 1) on R1, read (s2, 0), DMA stage s2 + 1
-      squares(B1, wr == 1);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-      phase(A0, B0, s2, 1, A1, B1, true, false);         // P: (s2, 0) on R0, read (s2, 1)
-      squares(B0, wr == 0);
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    phase(A1, B1, 0, 0, A0, B0, false, false);           // the last sub-step, (n2 - 1, 1), on R1
-    squares(B1, wr == 1);
-  } else {
-  // n is even (the host splits K in 64-deep units): the loop body is two k-steps with fixed register sets
-  issue(0);
-  issue(1);
-  if (n > 2) issue(2);
-  if (n > 2) p4_vmcnt<2 * G>(); else p4_vmcnt<G>();
+    for (int d = 0; d < GX; ++d) dma_x(u, d);
+  };
+  all_w(0);
+  all_x(0);
+  if (n2 > 1) {
+    all_w(1);
+    all_x(1);
+  }
+  if (n2 > 2) all_w(2);
+  clear();
+  if (n2 > 2) p4_vmcnt<(GW + GX) + GW>(); else if (n2 > 1) p4_vmcnt<(GW + GX)>(); else p4_vmcnt<0>();
   p4_sync();
-  rd(0, A0, B0);
-  int s = 0;
-  for (; s + 4 < n; s += 2) {
-    step_full(s, A0, B0, A1, B1);
-    step_full(s + 1, A1, B1, A0, B0);
-  }
-  if (s + 2 < n) {
-    step_tail(s, A0, B0, A1, B1);
-    step_tail(s + 1, A1, B1, A0, B0);
-    s += 2;
-  }
-  step_tail(s, A0, B0, A1, B1);
-  step_tail(s + 1, A1, B1, A0, B0);
-  }
+  rd2(A0, B0);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  phase(A0, B0, 0, 0, 1, A1, B1, yes, no, no);           // P_0: (0, 0) on R0, read (0, 1)
+  squares(B0, wr == 0);
+  int ws = 1;                                          // s2 % 3
+  auto stage = [&](int s2, auto dx, auto dw) {
+    // stage s2 landed (this wave's DMA), the weights of s2 + 1 may be under way
+    if constexpr (decltype(dx)::value) p4_vmcnt<GW>(); else p4_vmcnt<0>();
+    p4_sync();                                         // ... for every wave; (s2 - 1, 1) reads retired
+    __builtin_amdgcn_sched_barrier(0);
+    phase(A1, B1, s2, ws, 0, A0, B0, yes, dx, dw);     // A: (s2 - 1, 1) on R1, read (s2, 0), DMA
+    squares(B1, wr == 1);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    phase(A0, B0, s2, ws, 1, A1, B1, yes, no, no);     // P: (s2, 0) on R0, read (s2, 1)
+    squares(B0, wr == 0);
+    ws = ws == 2 ? 0 : ws + 1;
+  };
+  for (int s2 = 1; s2 < n2 - 2; ++s2) stage(s2, yes, yes);
+  if (n2 > 2) stage(n2 - 2, yes, no);
+  if (n2 > 1) stage(n2 - 1, no, no);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  phase(A1, B1, 0, 0, 0, A0, B0, no, no, no);          // the last sub-step, (n2 - 1, 1), on R1
+  squares(B1, wr == 1);
   p4_vmcnt<0>();
   {   // ... and the last MFMAs' results wait out the MFMA latency before the epilogue reads them:
     // the padding, then one tied empty asm per accumulator (so no read is hoisted above the padding)
@@ -418,6 +328,7 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
   }
 
   if constexpr (RMS) {
+    __syncthreads();                                     // rss lies in the last stage's memory
 #pragma unroll
     for (int f = 0; f < FQ; ++f) {
       ss[f] += __shfl_xor(ss[f], 16, WAVE);
@@ -459,51 +370,86 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
   }
 
   // ---- epilogue: lane holds out[token li of fragment j][features 4 g .. 4 g + 3 of fragment i]
+  constexpr int OF = PAIR ? FP / 2 : FP;             // fragments of output features
+  auto rms = [&](int mloc) -> float {
+    if constexpr (RMS) return rsqrtf(rss[mloc] / (float)a.K + a.eps);
+    else return 1.f;
+  };
+  // the 4 features of fragments (i, j): the sums with their scale, bias and activation
+  auto value = [&](int i, int j, int n0, float sx, float* v) {
+    if constexpr (EPI == P4_GLU) {
+      f32x4 bg = {0.f, 0.f, 0.f, 0.f}, bu = bg;
+      if (a.bias != nullptr) {
+        bg = ldf4(a.bias + n0);
+        bu = ldf4(a.bias + a.half_rows + n0);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[e] = p4_pair<KIND>(acc[i][j][e] + bg[e], acc[FP / 2 + i][j][e] + bu[e], a.limit, a.alpha);
+    } else if constexpr (EPI == P4_SWIGLU) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = p4_silu(acc[i][j][e] * sx) * (acc[FP / 2 + i][j][e] * sx);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] * sx;
+      if constexpr (EPI == P4_ACT) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = v[e] > 0.f ? v[e] * v[e] : 0.f;      // kind 7
+      }
+    }
+  };
+  const int nw = nt * (32 * OF) + wr * (16 * OF);    // the wave's first feature
+  if constexpr (EPI != P4_F32) {
+    if (a.wide) {
+      // bf16 rows through LDS: the wave's 16 FQ tokens x 16 OF features in the ring's memory (16-byte chunk c of a row in slot
+      // c ^ row), then 16 bytes a lane in row order -- whole 64 - 256-byte runs of a row a store, where the registers' order
+      // gives 32-byte pieces of 16 rows
+      constexpr int NC = 2 * OF, ROW = 32 * OF, SH = NC == 4 ? 1 : 0;
+      static_assert(4 * 16 * FQ * ROW <= RING, "the tile's rows fit the ring");
+      __syncthreads();                               // every wave has read its last fragments
+      char* mine = lds + wid * (16 * FQ * ROW);
+#pragma unroll
+      for (int j = 0; j < FQ; ++j) {
+        const int row = j * 16 + li;
+        const float sx = rms(wc * (BQ / 2) + row);
+#pragma unroll
+        for (int i = 0; i < OF; ++i) {
+          float v[4];
+          value(i, j, min(nw + i * 16 + 4 * g, a.N_out - 4), sx, v);
+          *reinterpret_cast<p4_u32x2*>(mine + row * ROW + (((2 * i + (g >> 1)) ^ ((row >> SH) & (NC - 1))) << 4) + (g & 1) * 8) =
+              p4_u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+        }
+      }
+      asm volatile("" ::: "memory");                 // the wave's own LDS operations run in order
+      __builtin_amdgcn_wave_barrier();
+      const int c = lane % NC;
+#pragma unroll
+      for (int p = 0; p < 16 * FQ * NC / 64; ++p) {
+        const int row = p * (64 / NC) + lane / NC, m = m0 + wc * (BQ / 2) + row, n0 = nw + c * 8;
+        const u32x4 o = *reinterpret_cast<const u32x4*>(mine + row * ROW + ((c ^ ((row >> SH) & (NC - 1))) << 4));
+        if (m < m_end && n0 < a.N_out)
+          *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(a.out) + (size_t)m * a.N_out + n0) = o;
+      }
+      return;
+    }
+  }
 #pragma unroll
   for (int j = 0; j < FQ; ++j) {
     const int mloc = wc * (BQ / 2) + j * 16 + li;
     const int m = m0 + mloc;
     if (m >= m_end) continue;
-    float sx = 1.f;
-    if constexpr (RMS) sx = rsqrtf(rss[mloc] / (float)a.K + a.eps);
-    if constexpr (PAIR) {
+    const float sx = rms(mloc);
 #pragma unroll
-      for (int i = 0; i < FP / 2; ++i) {
-        const int f0 = nt * (BP / 2) + wr * (BP / 4) + i * 16 + 4 * g;
-        if (f0 >= a.N_out) continue;
-        float v[4];
-        if constexpr (EPI == P4_GLU) {
-          f32x4 bg = {0.f, 0.f, 0.f, 0.f}, bu = bg;
-          if (a.bias != nullptr) {
-            bg = ldf4(a.bias + f0);
-            bu = ldf4(a.bias + a.half_rows + f0);
-          }
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            v[e] = p4_pair<KIND>(acc[i][j][e] + bg[e], acc[FP / 2 + i][j][e] + bu[e], a.limit, a.alpha);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = p4_silu(acc[i][j][e] * sx) * (acc[FP / 2 + i][j][e] * sx);
-        }
-        const p4_u32x2 o = {pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
-        *reinterpret_cast<p4_u32x2*>(reinterpret_cast<bf16_t*>(a.out) + (size_t)m * a.N_out + f0) = o;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < FP; ++i) {
-        const int n0 = nt * BP + wr * (BP / 2) + i * 16 + 4 * g;
-        if (n0 >= a.N_out) continue;
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] * sx;
-        if constexpr (EPI == P4_ACT) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = v[e] > 0.f ? v[e] * v[e] : 0.f;      // kind 7
-        }
-        if constexpr (EPI == P4_F32) {
-          *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + (size_t)m * a.N_out + n0) =
-              f32x4{v[0], v[1], v[2], v[3]};
-        } else {
+    for (int i = 0; i < OF; ++i) {
+      const int n0 = nw + i * 16 + 4 * g;
+      if (n0 >= a.N_out) continue;
+      float v[4];
+      value(i, j, n0, sx, v);
+      if constexpr (EPI == P4_F32) {
+        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + (size_t)m * a.N_out + n0) =
+            f32x4{v[0], v[1], v[2], v[3]};
+      } else {
+        if constexpr (EPI == P4_BF16) {
           if (a.res != nullptr) {
             const p4_u32x2 rr = *reinterpret_cast<const p4_u32x2*>(a.res + (size_t)m * a.N_out + n0);
             v[0] += lo_bf(rr[0]);
@@ -511,9 +457,9 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
             v[2] += lo_bf(rr[1]);
             v[3] += hi_bf(rr[1]);
           }
-          const p4_u32x2 o = {pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
-          *reinterpret_cast<p4_u32x2*>(reinterpret_cast<bf16_t*>(a.out) + (size_t)m * a.N_out + n0) = o;
         }
+        const p4_u32x2 o = {pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+        *reinterpret_cast<p4_u32x2*>(reinterpret_cast<bf16_t*>(a.out) + (size_t)m * a.N_out + n0) = o;
       }
     }
   }
@@ -594,7 +540,6 @@ using namespace k8sllm;
 namespace {
 struct P4Cfg {
   int fp, fq;
-  bool k64 = false;
 };
 // tile configurations: BP = 32 FP weight rows x BQ = 32 FQ tokens, 4 waves of (BP / 2) x (BQ / 2)
 constexpr P4Cfg kP4Cfgs[] = {
@@ -602,15 +547,13 @@ constexpr P4Cfg kP4Cfgs[] = {
     {8, 4},   // 1: 256 x 128
     {4, 8},   // 2: 128 x 256
     {4, 4},   // 3: 128 x 128
-    {8, 8, true},   // 4: 256 x 256, 64-deep LDS stages (128-byte rows): 1.01-1.10x of config 0 on 29 of 30 70B
-                    // TP=1 / TP=8 shapes; the 64-deep forms of configs 1 and 2 were within 2 % of them and were dropped
-                    // (profiles/pgemm4_asm_r6.txt)
+    {8, 8},   // 4: as 0 (saved plans name it)
 };
 constexpr int kP4NumCfgs = sizeof(kP4Cfgs) / sizeof(kP4Cfgs[0]);
 
 template <int C, int EPI, bool RMS>
 int p4_launch(const P4Args& a, hipStream_t s) {
-  hipLaunchKernelGGL((pgemm4_kernel<kP4Cfgs[C].fp, kP4Cfgs[C].fq, EPI, RMS, kP4Cfgs[C].k64>), dim3(a.nwg),
+  hipLaunchKernelGGL((pgemm4_kernel<kP4Cfgs[C].fp, kP4Cfgs[C].fq, EPI, RMS>), dim3(a.nwg),
                      dim3(256), 0, s, a);
   return (int)hipGetLastError();
 }
@@ -694,7 +637,7 @@ extern "C" int k8s_pgemm_reduce(void* out, const void* res, const float* slab, i
 // The forms with an activation (gated kinds 0, 1, 5; elementwise 7): configurations 1 - 4; the grouped ones: 1 and 3.
 template <int C, int EPI, bool GRP, int KIND>
 int p4_act_launch(const P4Args& a, hipStream_t s) {
-  hipLaunchKernelGGL((pgemm4_kernel<kP4Cfgs[C].fp, kP4Cfgs[C].fq, EPI, false, kP4Cfgs[C].k64, GRP, KIND>), dim3(a.nwg),
+  hipLaunchKernelGGL((pgemm4_kernel<kP4Cfgs[C].fp, kP4Cfgs[C].fq, EPI, false, GRP, KIND>), dim3(a.nwg),
                      dim3(256), 0, s, a);
   return (int)hipGetLastError();
 }
@@ -731,6 +674,7 @@ P4Args p4_args(void* out, const void* x, const void* W, int M, int N_out, int K,
   a.splits = 1;
   a.group_m = group_m > 0 ? group_m : 1;
   a.nwg = a.m_tiles * a.n_tiles;
+  a.wide = N_out % 8 == 0 && ((uintptr_t)out & 15) == 0;
   return a;
 }
 
@@ -740,7 +684,7 @@ extern "C" int k8s_pgemm4_config(int cfg, int* bp, int* bq, int* lds_bytes) {
   if (cfg < 0 || cfg >= kP4NumCfgs) return -1;
   *bp = 32 * kP4Cfgs[cfg].fp;
   *bq = 32 * kP4Cfgs[cfg].fq;
-  *lds_bytes = 4 * (*bp + *bq) * 64 + *bq * 8;
+  *lds_bytes = (3 * *bp + 2 * *bq) * 128;
   return 0;
 }
 
@@ -791,6 +735,7 @@ extern "C" int k8s_pgemm4(void* out, float* slab, const void* x, const void* W, 
   a.group_m = group_m > 0 ? group_m : 1;
   a.nwg = nwg;
   a.eps = eps;
+  a.wide = res == nullptr && N_out % 8 == 0 && ((uintptr_t)out & 15) == 0;
   int rc = p4_cfg(a, cfg, epi, rms, stream);
   if (rc != 0 || splits == 1) return rc;
   return k8s_pgemm_reduce(out, res, slab, splits, M, N_out, K, epi, rms, eps, nullptr, nullptr, nullptr, nullptr,
