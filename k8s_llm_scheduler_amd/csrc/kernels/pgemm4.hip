@@ -548,6 +548,8 @@ constexpr P4Cfg kP4Cfgs[] = {
     {4, 8},   // 2: 128 x 256
     {4, 4},   // 3: 128 x 128
     {8, 8},   // 4: as 0 (saved plans name it)
+    {4, 2},   // 5: 128 x 64
+    {2, 2},   // 6: 64 x 64
 };
 constexpr int kP4NumCfgs = sizeof(kP4Cfgs) / sizeof(kP4Cfgs[0]);
 
@@ -634,7 +636,7 @@ extern "C" int k8s_pgemm_reduce(void* out, const void* res, const float* slab, i
   return -2;
 }
 
-// The forms with an activation (gated kinds 0, 1, 5; elementwise 7): configurations 1 - 4; the grouped ones: 1 and 3.
+// The forms with an activation (gated kinds 0, 1, 5; elementwise 7) and the grouped ones.
 template <int C, int EPI, bool GRP, int KIND>
 int p4_act_launch(const P4Args& a, hipStream_t s) {
   hipLaunchKernelGGL((pgemm4_kernel<kP4Cfgs[C].fp, kP4Cfgs[C].fq, EPI, false, GRP, KIND>), dim3(a.nwg),
@@ -761,7 +763,10 @@ extern "C" int k8s_pgemm4_act(void* out, const void* x, const void* W, int M, in
     case 1: return p4_act_kind<1, false>(a, kind, stream);
     case 2: return p4_act_kind<2, false>(a, kind, stream);
     case 3: return p4_act_kind<3, false>(a, kind, stream);
+    case 0:
     case 4: return p4_act_kind<4, false>(a, kind, stream);
+    case 5: return p4_act_kind<5, false>(a, kind, stream);
+    case 6: return p4_act_kind<6, false>(a, kind, stream);
   }
   return -4;
 }
@@ -774,7 +779,7 @@ extern "C" int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M
   const bool pair = kind >= 0;
   if (kind < -1 || (pair && kind > 1 && kind != 5)) return -1;
   if (rows <= 0) return 0;
-  if (M <= 0 || N_out <= 0 || N_out % 4 || K <= 0 || K % 64 || groups <= 0 || (seg == nullptr && rows % groups) || (cfg != 1 && cfg != 3)) return -1;
+  if (M <= 0 || N_out <= 0 || N_out % 4 || K <= 0 || K % 64 || groups <= 0 || (seg == nullptr && rows % groups) || cfg < 0 || cfg >= kP4NumCfgs) return -1;
   if (ldx < K || ldx % 8 || (((uintptr_t)x | (uintptr_t)W) & 15) || ((uintptr_t)out & 7)) return -1;
   const long long kbytes = (long long)K * 2, wrows = (pair ? 2LL : 1LL) * N_out;
   if (wrows * kbytes >= (1LL << 32) || (long long)M * ldx * 2 >= (1LL << 32)) return -5;   // 32-bit DMA offsets
@@ -791,5 +796,12 @@ extern "C" int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M
   a.groups = groups;
   a.limit = limit;
   a.alpha = alpha;
-  return cfg == 1 ? p4_act_kind<1, true>(a, kind, stream) : p4_act_kind<3, true>(a, kind, stream);
+  switch (cfg) {
+    case 1: return p4_act_kind<1, true>(a, kind, stream);
+    case 2: return p4_act_kind<2, true>(a, kind, stream);
+    case 3: return p4_act_kind<3, true>(a, kind, stream);
+    case 5: return p4_act_kind<5, true>(a, kind, stream);
+    case 6: return p4_act_kind<6, true>(a, kind, stream);
+  }
+  return p4_act_kind<4, true>(a, kind, stream);
 }

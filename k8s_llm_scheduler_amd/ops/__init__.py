@@ -943,40 +943,37 @@ def _pg_load_table() -> dict:
     return _PG_TABLE
 
 
-# Time of a bf16 plan in us, (kernel, configuration) -> (fixed, per 64-deep k-step, per round, split, per MB of slab, per MB of
-# weights, per MB of output): a launch; per round of tiles over the CUs a fill and the tile's k-steps; with split-K the combine
-# launch and the slabs it moves; the weights and the output.  Fitted to 22 weight shapes (1152 x 2048 .. 28672 x 4096) at 8 row
-# counts (160 .. 2048), weights cold: rms error 5-8 % per configuration, the pick within 2 % of the best plan on average and
-# 24 % at most.  256 x 256 pgemm tiles with split-K until the grid is full (the rule before, and still the one of fp8 and
-# SwiGLU, which these figures do not cover) take 1.43 times as long on average: 2048 x 2048 x 2048 41.5 us, 24.6 us on 128 x
-# 128 tiles without a combine.  Past 64 k-steps the 128 x 128 tiles' operands fall out of an XCD's L2 between other kernels
-# (2048 x 2048 x 8192 inside a prompt: 91 us, alone 77; 72-80 us on split 256 x 256 tiles): _P4_LONG_K us more per step.
-_P4_COST = {("pgemm4", 1): (1.34, 0.754, 3.48, 4.66, 0.236, 0.0945, 0.485),
-            ("pgemm4", 2): (1.53, 0.738, 2.97, 4.19, 0.283, 0.0636, 0.555),
-            ("pgemm4", 3): (3.32, 0.440, 0.0, 3.82, 0.273, 0.0996, 0.480),
-            ("pgemm4", 4): (2.70, 1.158, 7.51, 3.61, 0.224, 0.0581, 0.248),
-            ("pgemm", 0): (5.50, 1.147, 11.06, 0.0, 0.163, 0.0143, 0.575)}
-_P4_LONG_K = 0.15
+# Time of a bf16 plan on pgemm4.hip in us, configuration -> (per round of tiles over the CUs and 64-deep k-step, per round, per
+# k-step, split, per MB of slab, per MB of weights, per MB of output): the tiles' k-steps, of which workgroups that share a CU
+# hide part from each other; with split-K the combine launch and the slabs it moves; the weights and the output.  Fitted to 22
+# weight shapes (576 x 2048 .. 28672 x 4096) at 12 row counts (40 .. 2048), weights cold: rms error 6 - 10 % per configuration,
+# the pick within 2 % of the best plan on average and 21 % at most, the same as hipBLASLt on average (0.92 - 1.09 of its time
+# by row count).  pgemm.hip's 8-wave tiles were the best plan of none.
+_P4_COST = {1: (0.657, 2.23, 0.0, 5.7, 0.302, 0.0684, 0.367),
+            2: (0.599, 2.19, 0.0, 4.12, 0.34, 0.0527, 0.514),
+            3: (0.297, 0.0, 0.155, 5.46, 0.348, 0.0739, 0.635),
+            4: (1.01, 5.43, 0.0, 4.18, 0.304, 0.0306, 0.436),
+            5: (0.234, 0.173, 0.137, 4.94, 0.298, 0.0902, 0.687),
+            6: (0.152, 0.231, 0.173, 4.37, 0.203, 0.0883, 0.245)}
+_P4_COST_T0 = {1: 0.0, 2: 1.09, 3: 0.218, 4: 1.5, 5: 0.0, 6: 0.599}
 
 
 @functools.lru_cache(maxsize=4096)
 def _pgemm_cheapest(M: int, N: int, K: int, num_cus: int) -> Tuple[str, int, int]:
     """(kernel, configuration, splits) of the cheapest bf16 plan by _P4_COST."""
     kt, best = K // 64, None
-    for (kern, cfg), (t0, step, rnd, sp, slab, wmb, omb) in _P4_COST.items():
-        bp, bq, _ = (pgemm4_configs() if kern == "pgemm4" else pgemm_configs())[cfg]
+    for cfg, (tile, rnd, step, sp, slab, wmb, omb) in _P4_COST.items():
+        bp, bq, _ = pgemm4_configs()[cfg]
         tiles = -(-N // bp) * -(-M // bq)
-        base = t0 + wmb * N * K * 2e-6 + omb * M * N * 2e-6
-        for s in (1, 2, 3, 4, 6, 8, 12, 16):
+        base = _P4_COST_T0[cfg] + wmb * N * K * 2e-6 + omb * M * N * 2e-6
+        for s in (1, 2, 3, 4, 6, 8):
             if s > 1 and (tiles * s > 2 * num_cus or kt // s < 4):
                 break
             rounds, per = -(-tiles * s // num_cus), -(-kt // s)
-            us = base + rounds * (rnd + step * per) + (sp + slab * M * N * s * 4e-6 if s > 1 else 0.0)
-            if bp * bq <= 128 * 128:
-                us += _P4_LONG_K * max(0, per - 64) * rounds
+            us = base + rounds * (rnd + tile * per) + step * per + (sp + slab * M * N * s * 4e-6 if s > 1 else 0.0)
             if best is None or us < best[0]:
-                best = (us, kern, cfg, s)
-    return best[1:]
+                best = (us, cfg, s)
+    return ("pgemm4",) + best[1:]
 
 
 def pgemm_heuristic(M: int, N: int, K: int, epi: int, fp8: bool, num_cus: int = 256) -> Tuple[str, int, int, int]:

@@ -335,10 +335,9 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out_dtype=None, *, a_rows: Optional[t
 
 
 # Grouped bf16 products of at least GROUP_BIG_MIN rows per group on average (whole rows of at least 64 elements) run on the
-# big-tile kernel (pgemm4.hip, 128 tokens per tile).  8 groups, N = K = 2048, 16 / 32 / 96 / 192 / 512 rows per group: 27 / 27
-# / 29 / 30 / 64 us, on the 64-row tiles of stream32.hip 22 / 29 / 44 / 50 / 87 us; gate / up with the activation in its
-# epilogue (N = 2 x 2048) 38 / 39 / 41 / 55 / 117 us, 47 / 63 / 62 / 85 / 173 us as two launches.  Fewer rows stream the
-# weights past the LDS (gemm_group_kernel).
+# big-tile kernel (pgemm4.hip).  8 groups, N = K = 2048, 8 / 16 / 32 / 96 / 192 / 512 rows per group, weights from memory: 20 /
+# 20 / 20 / 22 / 24 / 46 us, past the LDS (gemm_group_kernel) 18 / 22 / 31 us; gate / up with the activation in its epilogue
+# (N = 2 x 2048), 16 / 32 / 96 / 192 / 512 rows: 33 / 33 / 36 / 41 / 89 us, 37 / 44 us.  Fewer rows stream the weights past the LDS.
 GROUP_BIG_MIN = 16
 GROUP_BIG_MAX_GROUPS = 64        # every workgroup walks the groups' offsets
 
@@ -354,9 +353,8 @@ def _grouped_big(a: torch.Tensor, w: torch.Tensor, seg: Optional[torch.Tensor], 
 
 @functools.lru_cache(maxsize=4096)
 def _grouped_cfg(rows: int, E: int, N: int, K: int, pair: bool, even: bool = False) -> int:
-    """Configuration of the grouped big-tile product: 256 (1) or 128 (3) weight rows per tile by the time its rounds of tiles
-    over the CUs take (us, fitted to the products above and to N = 3584 / 4096, K = 3584 / 4096), groups of the same size
-    (``even``) or of about equal size drawn at random."""
+    """The better of the 128-token tiles of the grouped big-tile product: 256 (1) or 128 (3) weight rows by the time its rounds
+    of tiles over the CUs take, groups of the same size (``even``) or of about equal size drawn at random."""
     r = rows / E
     if even or E == 1:
         tiles = E * -(-rows // E // 128)
@@ -370,11 +368,45 @@ def _grouped_cfg(rows: int, E: int, N: int, K: int, pair: bool, even: bool = Fal
     return 1 if big < small else 3
 
 
+# Time of a grouped product in us, configuration -> (fixed, per round of tiles over the CUs and 64-deep k-step, per round, per
+# k-step, per MB of weights, per MB of output, per round and 65536 outputs of a gated activation).  Fitted to 8 products of 1 -
+# 16 groups, 512 x 4096 .. 2 x 3584 x 4096, 2 - 2048 rows per group, weights cold: rms error 5 - 11 % per configuration, the
+# pick within 2 % of the best configuration on average, 41 % at most.  _GROUP_TILE: weight rows and tokens of a tile.
+_GROUP_TILE = {1: (256, 128), 2: (128, 256), 3: (128, 128), 4: (256, 256), 5: (128, 64), 6: (64, 64)}
+_GROUP_COST = {1: (0.0, 0.524, 4.92, 0.0, 0.11, 0.424, 6.72), 2: (0.0, 0.542, 4.91, 0.0, 0.0696, 0.486, 9.86),
+               3: (3.28, 0.379, 0.0, 0.0254, 0.0878, 0.27, 11.6), 4: (0.0, 0.864, 8.67, 0.0, 0.0913, 0.323, 8.6),
+               5: (2.67, 0.304, 0.0, 0.0345, 0.0953, 0.174, 16.3), 6: (2.29, 0.176, 0.0, 0.16, 0.0834, 0.076, 15.8)}
+
+
+@functools.lru_cache(maxsize=4096)
+def _grouped_tile(base: int, rows: int, E: int, N: int, K: int, pair: bool, even: bool = False) -> int:
+    """Configuration of the grouped big-tile product: ``base`` (:func:`_grouped_cfg`'s), or what is cheaper by _GROUP_COST of
+    the tiles of 256 and 64 tokens and of 128 x 256.  Groups as there."""
+    r, n, kt, best = rows / E, (2 * N if pair else N), K / 64, None
+    for cfg in (base, 2, 4, 5, 6):
+        t0, tile, rnd, step, wmb, omb, act_us = _GROUP_COST[cfg]
+        bp, bq = _GROUP_TILE[cfg]
+        if even or E == 1:
+            tiles = E * -(-rows // E // bq)
+        else:   # a group's tiles beyond k: the chance that it has more than bq k rows, 1 up to six deviations below the mean
+            d = 6.0 * math.sqrt(max(r, 1.0))
+            sure = max(0, int((r - d) // bq))
+            tiles = E * (1 + sure + sum(0.5 + 0.5 * math.erf((r - bq * k) / math.sqrt(2.0 * max(r, 1.0)))
+                                        for k in range(sure + 1, int((r + d) / bq) + 2)))
+        rounds = math.ceil(tiles * -(-n // bp) / 256 - 1e-9)
+        us = t0 + rounds * (tile * kt + rnd + (act_us * bp * bq / 65536 if pair else 0.0)) + step * kt + \
+            wmb * E * n * K * 2e-6 + omb * rows * N * 2e-6
+        if best is None or us < best[0]:
+            best = (us, cfg)
+    return best[1]
+
+
 def _pgemm4_grouped(a, w, a_rows, rows: int, seg, N: int, kind: int = -1, limit: float = 0.0, alpha: float = 1.0):
     E, _, K = w.shape
     out = torch.empty(rows, N, dtype=BF16, device=a.device)
+    shape = (rows, E, N, K, kind >= 0, seg is None)
     _native().pgemm4_grouped(out.data_ptr(), a.data_ptr(), w.data_ptr(), a.shape[0], rows, N, K, E, _p(seg, I32, "seg"),
-                             _p(a_rows, I32, "a_rows"), a.stride(0), _grouped_cfg(rows, E, N, K, kind >= 0, seg is None), 4, kind,
+                             _p(a_rows, I32, "a_rows"), a.stride(0), _grouped_tile(_grouped_cfg(*shape), *shape), 4, kind,
                              float(limit), float(alpha), -1)
     return out
 
@@ -388,11 +420,10 @@ def _few_fits(a: torch.Tensor, w: torch.Tensor) -> bool:
 
 def linear_each(a: torch.Tensor, w: torch.Tensor):
     """[a[i] @ w[i].T]: several inputs, a weight each (a [G, M, K], w [G, N, K]) -> G tensors [M, N] of one row stride.  One
-    launch where that is faster than G of :func:`linear`.  4 weights of 2048 x 2048, M = 8 / 64 / 128 / 512 / 1024 / 2048: the
-    any-shape kernel (k shared by the waves while its tiles are few) 11 / 24 / 38 / 52 / 77 / 139 us, the grouped big tiles
-    27 / 29 / 30 / 31 / 45 / 80, four launches 22 / 27 / 33 / 76 / 109 / 114; of 4096 x 4096, M = 16 / 32 / 64 / 512 / 2048:
-    70 / 71 / 73 / 136 / 472, 53 / 54 / 55 / 81 / 288, 39 / 47 / 55 / 135 / 300 (beyond, a launch's own tiles fill the card
-    and its deeper stages win)."""
+    launch where that is faster than G of :func:`linear`.  4 weights of 2048 x 2048, M = 8 / 32 / 64 / 128 / 512 / 1024 / 2048:
+    the any-shape kernel (k shared by the waves while its tiles are few) 11 / 16 / 23 / 33 us, the grouped big tiles 16 / 16 /
+    17 / 17 / 22 / 33 / 56, four launches 21 / 22 / 27 / 32 / 59 / 66 / 86; of 4096 x 4096, M = 8 / 16 / 32 / 64 / 512 / 2048: 31 /
+    37 / 54 / 84 us, 35 / 35 / 36 / 37 / 61 / 194, 33 / 41 / 45 / 54 / 117 / 235."""
     G, M, K = a.shape
     N = w.shape[1]
     if w.shape != (G, N, K):
@@ -438,12 +469,14 @@ def gemm_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, al
 def linear_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, alpha: float = 1.0, *,
                bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """act(linear(a, w), kind, bias=bias): in the product's epilogue where its plan is an unsplit big-tile one, which saves a
-    pass over the product (2048 x 2 x 8192, gated: 22 us; 2048 x 8192 elementwise: 15 us) and its rounding."""
+    pass over the product (2048 x 2 x 8192, gated: 22 us; 2048 x 8192 elementwise: 15 us) and its rounding.  Deep products of
+    few tiles keep the launch of their own, as when they ran in k slices: the pass that it saves there is 1 - 2 us."""
     pair = kind in (ACT_GELU_TANH, ACT_SWISH_CLAMP, ACT_RELU)
     if (pair or kind == ACT_RELU2) and FAST_GEMM and _gpu(a, w, bias) and _route_fast(a, w, BF16) and a.dtype == BF16 and (not pair or w.shape[0] % 8 == 0):
         M, K = a.shape
         kern, plan = _ops.gemm_route(M, w.shape[0], K, _ops.EPI_BF16, False) if M >= 129 else ("", None)
-        if kern == "pgemm4" and plan[1] == 1 and plan[0] in (1, 2, 3, 4) and a.data_ptr() % 16 == 0 and \
+        if kern == "pgemm4" and plan[1] == 1 and (K < 1024 or _ops.pgemm4_tiles(plan[0], M, w.shape[0], _ops.EPI_BF16) >= 96) and \
+                a.data_ptr() % 16 == 0 and \
                 (bias is None or (pair and bias.dtype == BF16 and bias.numel() == w.shape[0] and bias.data_ptr() % 8 == 0)):
             N = w.shape[0] // 2 if pair else w.shape[0]
             out = torch.empty(M, N, dtype=BF16, device=a.device)

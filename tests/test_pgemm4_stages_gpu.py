@@ -7,7 +7,7 @@ from k8s_llm_scheduler_amd import ops
 from k8s_llm_scheduler_amd.ops import seqmix as sm
 
 pytestmark = pytest.mark.gpu
-TILES = {0: (256, 256), 1: (256, 128), 2: (128, 256), 3: (128, 128), 4: (256, 256)}
+TILES = {0: (256, 256), 1: (256, 128), 2: (128, 256), 3: (128, 128), 4: (256, 256), 5: (128, 64), 6: (64, 64)}
 
 
 def whole(n, K, seed):
@@ -24,7 +24,7 @@ def untouched(buf, M, N, shift=0):
     return bool((buf[:shift] == 7).all() and (buf[shift + M * N:] == 7).all())
 
 
-@pytest.mark.parametrize("cfg", range(5))
+@pytest.mark.parametrize("cfg", range(7))
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 320])
 def test_stages_and_row_stores(cfg, K):
     bp, bq = TILES[cfg]
@@ -40,7 +40,7 @@ def test_stages_and_row_stores(cfg, K):
             assert torch.equal(ops.pgemm4(x, w, ops.EPI_BF16, cfg=cfg, splits=2).float(), want), (M, N, "split")
 
 
-@pytest.mark.parametrize("cfg", [1, 2, 3, 4])
+@pytest.mark.parametrize("cfg", range(7))
 @pytest.mark.parametrize("K", [64, 192])
 def test_activations_and_rms(cfg, K):
     bp, bq = TILES[cfg]
@@ -64,7 +64,7 @@ def test_activations_and_rms(cfg, K):
         assert ((got - ref).abs() <= ref.abs() * (2.0**-8 + (y[:, :N].abs() + 16) * 2.0**-23) + 1e-30).all(), (M, N)
 
 
-@pytest.mark.parametrize("cfg", [1, 3])
+@pytest.mark.parametrize("cfg", range(7))
 def test_grouped(cfg):
     counts, N, K = [130, 0, 1, 257], 264, 192
     seg = torch.tensor([0] + counts).cumsum(0).int().cuda()

@@ -42,7 +42,7 @@ def candidates(M, N, K, epi, fp8, num_cus=256, kernels=("pgemm", "pgemm4")):
         cfgs = ops.pgemm_configs() if kern == "pgemm" else ops.pgemm4_configs()
         tiles_fn = ops.pgemm_tiles if kern == "pgemm" else ops.pgemm4_tiles
         for c, (bp, bq, _lds) in enumerate(cfgs):
-            if bq > 2 * max(M, 128):
+            if bq > 2 * max(M, 128) or (kern == "pgemm4" and c == 4):     # (configuration 4 is 0 again)
                 continue
             tiles = tiles_fn(c, M, N, epi)
             for s in SPLITS:
