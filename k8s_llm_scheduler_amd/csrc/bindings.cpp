@@ -155,6 +155,12 @@ int k8s_act(void* out, const void* x, int T, int F, int kind, float limit, float
             const int* row_map, const void* bias, int f32, hipStream_t s);
 int k8s_gemm_few_act(void* C, const void* A, const void* W, int M, int N, int K, long lda, const int* a_rows,
                      const int* tiles, int ntiles, int kind, float limit, float alpha, hipStream_t s);
+int k8s_gemv_act(void* out, void* partial, const void* x, const void* W, int M, int N_out, int K, int kind, float limit, float alpha,
+                 hipStream_t stream);
+int k8s_sgemv_act(void* out, void* partial, const void* x, const void* W, int M, int N, int K, int kind, float limit, float alpha,
+                  hipStream_t stream);
+int k8s_mgemm_act(void* out, float* ws, unsigned* tickets, const void* x, const void* W, int M, int N_out, int K, int cfg, int nwg,
+                  int cmax, int kind, float limit, float alpha, int fenced, hipStream_t stream);
 int k8s_gemm_f32_tiles(void* C, const float* A, const float* W, int M, int N, int K, long lda, long ldw, long ldc, int batch,
                        long sA, long sW, long sC, const int* a_rows, const int* tiles, int ntiles, int out_f32, int fq,
                        hipStream_t s);
@@ -347,6 +353,22 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
   m.def("pgemm_set_prio", [](int mode) { return k8s_pgemm_set_prio(mode); });
   m.def("pgemm_set_row_slabs", [](int on) { return k8s_pgemm_set_row_slabs(on); });
   m.def("gemv_set_wide", [](int on) { return k8s_gemv_set_wide(on); });
+  m.def("gemv_act", [](uintptr_t out, uintptr_t partial, uintptr_t x, uintptr_t W, int M, int N, int K, int kind, float limit,
+                       float alpha, int64_t s) {
+    check(k8s_gemv_act(P(out), P(partial), P(x), P(W), M, N, K, kind, limit, alpha, S(s)), "gemv_act");
+  });
+  m.def("sgemv_act", [](uintptr_t out, uintptr_t partial, uintptr_t x, uintptr_t W, int M, int N, int K, int kind, float limit,
+                        float alpha, int64_t s) {
+    const int rc = k8s_sgemv_act(P(out), P(partial), P(x), P(W), M, N, K, kind, limit, alpha, S(s));
+    if (rc != -5) check(rc, "sgemv_act");
+    return rc;
+  });
+  m.def("mgemm_act", [](uintptr_t out, uintptr_t ws, uintptr_t tickets, uintptr_t x, uintptr_t W, int M, int N, int K, int cfg,
+                        int nwg, int cmax, int kind, float limit, float alpha, int fenced, int64_t s) {
+    check(k8s_mgemm_act(P(out), P<float>(ws), P<unsigned>(tickets), P(x), P(W), M, N, K, cfg, nwg, cmax, kind, limit, alpha, fenced,
+                        S(s)),
+          "mgemm_act");
+  });
   m.def("gemv_set_loop", [](int wg) { return k8s_gemv_set_loop(wg); });
   m.def("gemv_plan", [](int M, int N, int K, int epi, int mode) {
     int ks, sp;

@@ -31,6 +31,7 @@
 // cycles are the matrix cores', and at K = 2048 a fifth of the launch is its start, first loads and stores.
 #include <type_traits>
 
+#include "act.h"
 #include "common.h"
 
 namespace k8sllm {
@@ -55,20 +56,8 @@ __device__ __forceinline__ void p4_dma(const uint8_t* base, uint32_t off, uint32
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }
 __device__ __forceinline__ float p4_silu(float g) { return g / (1.f + __expf(-g)); }
-// Activations of the epilogues (kinds as in stream32.hip), on the hardware's exponential and reciprocal: a sigmoid of x is
-// off by about (|x| + 4) 2^-24 relative (the exponent x log2 e is rounded to fp32), the result is then rounded to bf16.  The
-// kind is a template argument: 128 unrolled elements per lane with every kind's branches took 775 us where the product takes 56.
-__device__ __forceinline__ float p4_sigmoid(float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
-template <int KIND>
-__device__ __forceinline__ float p4_pair(float g, float u, float limit, float alpha) {
-  if constexpr (KIND == 0) return g * p4_sigmoid(1.5957691216057308f * (g + 0.044715f * g * g * g)) * u;
-  if constexpr (KIND == 5) return fmaxf(g, 0.f) * u;
-  if (limit > 0.f) {
-    g = fminf(g, limit);
-    u = fminf(fmaxf(u, -limit), limit);
-  }
-  return g * p4_sigmoid(alpha * g) * (u + 1.f);
-}
+// The kind of an activation (act.h) is a template argument: 128 unrolled elements per lane with every kind's branches took 775
+// us where the product takes 56.
 }  // namespace
 
 struct P4Args {
@@ -385,7 +374,7 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        v[e] = p4_pair<KIND>(acc[i][j][e] + bg[e], acc[FP / 2 + i][j][e] + bu[e], a.limit, a.alpha);
+        v[e] = epi_pair<KIND>(acc[i][j][e] + bg[e], acc[FP / 2 + i][j][e] + bu[e], a.limit, a.alpha);
     } else if constexpr (EPI == P4_SWIGLU) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = p4_silu(acc[i][j][e] * sx) * (acc[FP / 2 + i][j][e] * sx);

@@ -800,6 +800,40 @@ def mgemm(x: torch.Tensor, w, epi: int = EPI_BF16, cfg: Optional[int] = None,
     return out
 
 
+def linear_act_rows(x: torch.Tensor, w: torch.Tensor, pair: bool, kind: int, limit: float, alpha: float) -> Optional[torch.Tensor]:
+    """act(x[M, K] @ w.T) of M <= 128 bf16 rows with the activation in the epilogue (``pair``: w = [gate; up]), on the kernel that
+    :func:`linear` takes for M rows with the plan of its SwiGLU or plain form; None where that is another one (the library,
+    a forced family) or does not take the shape.  It saves the activation's launch, 2 us of a captured step, and one rounding."""
+    M, K = x.shape
+    N = w.shape[0] // 2 if pair else w.shape[0]
+    if GEMM_BACKEND != "auto" or M > 128 or M < 1 or K % 64 or N % 4:
+        return None
+    epi = EPI_SWIGLU if pair else EPI_BF16
+    out = torch.empty(M, N, dtype=BF16, device=x.device)
+    if M <= min(GEMV_MAX_M, 2):
+        _, splits = native().gemv_plan(M, N, K, epi, 0)
+        part = torch.empty(splits * M * w.shape[0], dtype=F32, device=x.device) if splits > 1 else None
+        native().gemv_act(out.data_ptr(), part.data_ptr() if part is not None else 0, _chk(x, BF16, "x"), _chk(w, BF16, "w"), M, N,
+                          K, kind, limit, alpha, -1)
+        return out
+    if M <= SGEMV_MAX_M:
+        n = native().sgemv_workspace(M, N, K, epi, 0)
+        part = torch.empty(n, dtype=F32, device=x.device) if n > 0 else None
+        rc = native().sgemv_act(out.data_ptr(), part.data_ptr() if part is not None else 0, _chk(x, BF16, "x"), _chk(w, BF16, "w"),
+                                M, N, K, kind, limit, alpha, -1)
+        return None if rc == -5 else out
+    cfg, grid = mgemm_plan(M, N, K, epi, False)
+    if not mgemm_valid(cfg, M, N, K, epi, False, grid):
+        return None
+    nwg = mgemm_nwg(cfg, M, N, K, epi, False, grid)
+    tiles, cmax, n = _mg_plan_info(M, N, K, epi, 0, cfg, nwg)
+    ws = torch.empty(n, dtype=F32, device=x.device) if n > 0 else None
+    native().mgemm_act(out.data_ptr(), ws.data_ptr() if ws is not None else 0,
+                       _zeroed_scratch(x.device, "mgemm", 4 * tiles, 64 * 1024) if cmax > 1 else 0, _chk(x, BF16, "x"),
+                       _chk(w, BF16, "w"), M, N, K, cfg, nwg, cmax, kind, limit, alpha, int(MGEMM_FENCED), -1)
+    return out
+
+
 # ----------------------------------------------------------------------------- big-tile MFMA GEMM (prefill rows)
 _PG_CFGS: Optional[list] = None
 
