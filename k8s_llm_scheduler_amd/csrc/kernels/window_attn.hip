@@ -724,25 +724,29 @@ __global__ __launch_bounds__(256) void window_attention_mfma_kernel(
 
 // The prompt kernel without pooled blocks, for exact sizes (DK key, DV value dimensions) and pages of a power of two.  The
 // orientation of the products is the one above; what differs:
-//   * 8 waves in two groups: both groups own the same tokens (a wave NCB blocks of 16 columns), group k takes the keys
-//     [32 k, 32 k + 32) of every 64-key step with a running softmax of its own, and the two are merged at the end -- two
-//     independent waves per SIMD hide each other's latencies, and a staged fragment still serves NCB column blocks;
+//   * 8 waves in two groups: both groups own the same tokens (a wave one block of 16 columns), group k takes the keys
+//     [32 k, 32 k + 32) of every 64-key step with a running softmax of its own, and the two are merged at the end;
+//   * one column block a wave is at most 128 registers, so two workgroups share a CU: a step is a chain of LDS reads, shuffles
+//     and about 350 vector instructions a block (2 us for a lone workgroup), and four waves per SIMD hide each other's.
+//     With two blocks a wave (210 registers, one workgroup on a CU, each staged key used twice) a step is no shorter and the
+//     longest sequence of a batch decides: 16 query heads over 4 of 128, five prompts of 153 - 459 tokens and three single
+//     tokens behind 640 - 700 39.6 -> 27.8 us, 512 fresh tokens 23.9 -> 22.0, 1024 38.6 -> 32.1, 97 behind 1000 23.4 ->
+//     20.6, 2048 47.4 -> 47.2 (with the merge where there is one);
 //   * two LDS buffers, one barrier per step: while a step is computed the next one is stored and the one after next is
 //     loaded into registers, its page numbers a step earlier still; a thread always moves one row's pieces;
 //   * scores in base 2 (scale and slopes carry log2 e), no mask arithmetic on slices that every column of the wave sees,
 //     accumulators rescaled only when some column's maximum moved, sums kept per lane until the end;
 //   * where the tiles are few (a short portion behind a long cached one), nsplit workgroups share a tile's steps and leave
-//     (max, sum, unnormalised sum) for window_merge_kernel: a step is a chain of LDS and shuffle latencies of about 2.5 us
-//     however few workgroups run.  16 query heads over 4 of 128, 97 tokens behind 1000: 46.6 us in
-//     one piece, 22.9 us in 6 with the merge.  (A template flag: the arithmetic of the splits costs the whole walk 8%.)
-template <int DK, int DV, int NCB, bool SPLIT>
-__global__ __launch_bounds__(512) void window_prompt_kernel(
+//     (max, sum, unnormalised sum) for window_merge_kernel: 97 tokens behind 1000 33.0 us in one piece, 20.6 us in 6 with the
+//     merge.  (A template flag: the arithmetic of the splits costs the whole walk 8%.)
+template <int DK, int DV, bool SPLIT>
+__global__ __launch_bounds__(512, 4) void window_prompt_kernel(
     bf16_t* __restrict__ out, float* __restrict__ pacc, float* __restrict__ pml, const bf16_t* __restrict__ q, long ldq,
     const bf16_t* __restrict__ gate, long ldg, const bf16_t* __restrict__ kcache, const bf16_t* __restrict__ vcache,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ cu_q, const int* __restrict__ positions,
     int H, int G, int window, float scale, int sink, int bshift, int nsplit, int R, int chunk, float softcap,
     const float* __restrict__ sinkv, int gate_ph, const float* __restrict__ slopes) {
-  constexpr int NKK = DK / 32, NVB = DV / 16, KT = 64;
+  constexpr int NCB = 1, NKK = DK / 32, NVB = DV / 16, KT = 64;      // NCB: column blocks of a wave
   constexpr int ROWK = (DK + 8) * 2, ROWV = (DV + 8) * 2, BUF = KT * (ROWK + ROWV);   // LDS bytes
   constexpr int CK = DK / 8, CV = DV / 8, NST = (CK + CV + 7) / 8;                   // 16-byte pieces; per thread
   constexpr float LOG2E = 1.4426950408889634f;
@@ -1353,7 +1357,7 @@ extern "C" int k8s_window_mfma_ok(int H, int G, int D, int V) {
 extern "C" int k8s_window_prompt_tile(int H, int G, int D, int V, int P, int bs) {
   if (!k8s_window_mfma_ok(H, G, D, V) || P > 0 || D != V || (D != 64 && D != 96 && D != 128) || bs <= 0 || (bs & (bs - 1)))
     return 0;
-  return 4 * 2 * (16 / (H / G));
+  return 4 * (16 / (H / G));
 }
 
 // Prompt portions in bf16: nseq sequences of at most max_qlen tokens (T in all), cu_q their query offsets.  nsplit > 1 (only
@@ -1369,25 +1373,24 @@ extern "C" int k8s_window_attention_mfma(void* out, float* pacc, float* pml, con
   if (!k8s_window_mfma_ok(H, G, D, V) || bs <= 0 || nseq > 65535 || G > 65535 || ldq % 8 || ((uintptr_t)q & 15)) return -1;
   if (window > 0 && P > 0 && (kpool == nullptr || vpool == nullptr || slopes != nullptr)) return -1;
   const int R = H / G, ppb = P > 0 ? (bs + P - 1) / P : 1;
-  constexpr int NCB = 2;
   if (k8s_window_prompt_tile(H, G, D, V, P, bs) > 0) {
     const int tpb = k8s_window_prompt_tile(H, G, D, V, P, bs);
     const dim3 grid((max_qlen + tpb - 1) / tpb * nsplit, G, nseq);
     int bshift = 0;
     while ((1 << bshift) < bs) ++bshift;
     const size_t stage = (size_t)2 * 64 * (D + 8 + V + 8) * 2;                     // two buffers of 64 rows
-    const size_t merge = (size_t)4 * 64 * NCB * (4 * (V / 16) + 2) * sizeof(float);   // one group's results
+    const size_t merge = (size_t)4 * 64 * (4 * (V / 16) + 2) * sizeof(float);   // one group's results
     const size_t lds = stage > merge ? stage : merge;
 #define K8S_WP(DK, SPLIT)                                                                                               \
   do {                                                                                                                  \
     static bool grown = false;   /* more LDS than a launch gets by default */                                           \
     if (!grown) {                                                                                                       \
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_prompt_kernel<DK, DK, NCB, SPLIT>), \
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(window_prompt_kernel<DK, DK, SPLIT>), \
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                   \
       if (e != hipSuccess) return (int)e;                                                                               \
       grown = true;                                                                                                     \
     }                                                                                                                   \
-    window_prompt_kernel<DK, DK, NCB, SPLIT><<<grid, 512, lds, s>>>(                                                    \
+    window_prompt_kernel<DK, DK, SPLIT><<<grid, 512, lds, s>>>(                                                    \
         (bf16_t*)out, pacc, pml, (const bf16_t*)q, ldq, (const bf16_t*)gate, ldg, (const bf16_t*)kcache,                \
         (const bf16_t*)vcache, block_tables, max_blocks, cu_q, positions, H, G, window, scale, sink, bshift, nsplit, R, \
         chunk, softcap, sinkv, gate_ph, slopes);                                                                        \
@@ -1409,6 +1412,7 @@ extern "C" int k8s_window_attention_mfma(void* out, float* pacc, float* pml, con
   }
   if (nsplit > 1) return -1;
   const size_t lds = (size_t)32 * ((D + 8) + (V + 8)) * 2;
+  constexpr int NCB = 2;
   const int TPB = 4 * NCB * (16 / R);
   const dim3 grid((max_qlen + TPB - 1) / TPB, G, nseq);
   static int cus = 0;

@@ -923,10 +923,10 @@ def token_splits(T: int, G: int, keys: int) -> int:
 
 
 def prompt_splits(groups: int, keys: int) -> int:
-    """Key splits of the prompt kernel's ``groups`` workgroups: up to 256 (one per CU: 40 workgroups, 300 tokens behind 1000,
-    6 splits 30 us, 8 splits 40 us), of two 64-key steps at least, at most 6 (16 workgroups, 97 tokens behind 1000: 1 split 46.2
-    us, 4 24.8, 6 22.9, 8 23.3, 16 25.6, the more the merge reads).  How many keys there are is only known on the device: 97
-    tokens behind none pay 2.5 us for the merge (13.4 us in one piece), 300 tokens nothing (20 us)."""
+    """Key splits of the prompt kernel's ``groups`` workgroups: up to 256 of them (76 workgroups, 300 tokens behind 1000: 1 split
+    33.4 us, 3 25.7, 6 26.7, 8 34.2; 128, 512 fresh tokens: 1 20.0, 2 22.0, 4 23.2), of two 64-key steps at least, at most 6 (28
+    workgroups, 97 tokens behind 1000: 1 split 33.0 us, 2 25.1, 4 20.7, 6 20.6, 8 21.1, the more the merge reads).  How many
+    keys there are is only known on the device: 97 tokens behind none pay 3.6 us for the splits and their merge (9.8 in one piece)."""
     return max(1, min(256 // max(1, groups), -(-max(1, keys) // 128), 6))
 
 
@@ -977,7 +977,8 @@ def window_attention(q: torch.Tensor, gate: Optional[torch.Tensor], kcache: torc
         ns, pacc, pml = 1, None, None
         if tile > 0:
             max_pos = max_keys or block_tables.shape[1] * block_size
-            ns = prompt_splits(-(-int(max_qlen) // tile) * G * (cu_q.shape[0] - 1),
+            nseq = cu_q.shape[0] - 1     # (a batch of unequal portions has fewer tiles than its launch has workgroups)
+            ns = prompt_splits(G * min(-(-int(max_qlen) // tile) * nseq, T // tile + nseq),
                                min(max_pos, (chunk or window + tile) if chunk > 0 or window > 0 else max_pos))
         if ns > 1:
             pacc = torch.empty(T * H * ns * V, dtype=F32, device=q.device)
