@@ -43,7 +43,7 @@ SgPlan sg_plan(int K) {
 // The same plan k8s_sgemv takes for these operands (fp8: e4m3 weights), so the slabs always fit.
 extern "C" long long k8s_sgemv_workspace(int M, int N, int K, int epi, int fp8) {
   SmPlan sp;
-  const int g = sm_take(M, K, fp8 != 0, sp) ? sp.g : sg_plan(K).g;
+  const int g = sm_take(M, N, K, fp8 != 0, false, sp) ? sp.g : sg_plan(K).g;
   if (g <= 1) return 0;
   return (long long)g * M * (epi == SG_SWIGLU ? 2 : 1) * N;
 }
@@ -73,7 +73,7 @@ extern "C" int k8s_sgemv(void* out, void* partial, const void* x, const void* W,
   const bf16_t* xx = (const bf16_t*)x;
   const bf16_t* rr = (const bf16_t*)res;
   SmPlan sp;
-  if (sm_take(M, K, fp8, sp)) {
+  if (sm_take(M, N, K, fp8, norm != 0, sp)) {
     if (norm && sp.g > 1) return -5;
     if (sp.g > 1 && partial == nullptr) return -3;
 #define SMK(MT, JT, EE, NN, RR, F8) \

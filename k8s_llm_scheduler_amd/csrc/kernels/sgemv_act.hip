@@ -12,7 +12,7 @@ extern "C" int k8s_sgemv_act(void* out, void* partial, const void* x, const void
   const bool pair = kind == 0 || kind == 1 || kind == 5;
   if (M < 1 || M > 16 || N <= 0 || K <= 0 || (!pair && kind != 7)) return -1;
   SmPlan sp;
-  if (!sm_take(M, K, false, sp)) return -5;
+  if (!sm_take(M, N, K, false, false, sp)) return -5;
   if (sp.g > 1 && partial == nullptr) return -3;
   const EpiAct act{kind, limit, alpha};
   bool whole = false;      // the launch reduces its k-groups itself

@@ -595,15 +595,21 @@ __global__ void sgemv_finalize_kernel(void* __restrict__ out, const float* __res
 
 // MFMA plan (smfma_kernel): JT register steps per wave (1, 2, 4, 8; a step = 16 chunks of every row of a quad),
 // jw live steps, G k-groups.  Needs whole steps (K % 128 bf16, K % 256 fp8); one k-group covers 8 waves x 8 steps
-// (8192 k) -- fp8 4 steps (8192 k: an fp8 step holds twice the x of a bf16 one).
+// (8192 k) -- fp8 4 steps (8192 k: an fp8 step holds twice the x of a bf16 one).  Bands of 16 rows (the least) that leave
+// CUs idle take more groups, as long as a wave keeps two steps and the depth pays for the reduction (2.3 us).  us, one group
+// -> the rule's: 8 x 2048 x 8192 12.8 -> 11.2, x 6144 11.1 -> 9.2, 8 x 1024 x 8192 12.6 -> 8.9, 16 x 2048 x 8192 16.5 -> 12.8;
+// K = 4096 stays in one (8 x 2048 7.8, two groups 8.1).  The norm prologue needs all of K in one group.
 struct SmPlan {
   int jt, jw, g;
 };
-static bool sm_plan(int K, bool fp8, SmPlan& p) {
+static int sm_cus();
+static bool sm_plan(int N, int K, bool fp8, bool norm, SmPlan& p) {
   const int epc = fp8 ? 16 : 8;
   if (K % (16 * epc) != 0) return false;
   const int c16 = K / (16 * epc), jmax = fp8 ? 4 : 8;
-  const int g = (c16 + SM_KW * jmax - 1) / (SM_KW * jmax);
+  int g = (c16 + SM_KW * jmax - 1) / (SM_KW * jmax);
+  if (!norm && c16 >= 48)
+    while ((N + 15) / 16 * g * 2 <= sm_cus() && c16 >= 4 * SM_KW * g) g *= 2;
   const int jw = (c16 + SM_KW * g - 1) / (SM_KW * g);
   p = {jw <= 1 ? 1 : (jw <= 2 ? 2 : (jw <= 4 ? 4 : 8)), jw, g};
   return true;
@@ -626,7 +632,9 @@ static int sm_cus() {
   }();
   return v;
 }
-static bool sm_take(int M, int K, bool fp8, SmPlan& p) { return M >= sm_min_m() && M <= 16 && sm_plan(K, fp8, p); }
+static bool sm_take(int M, int N, int K, bool fp8, bool norm, SmPlan& p) {
+  return M >= sm_min_m() && M <= 16 && sm_plan(N, K, fp8, norm, p);
+}
 
 // Workgroups of the MFMA form per CU the band is sized for: what the kernel's registers allow (one for every form
 // since the epilogue prefetch took the 8-row kernels past 128 VGPRs), capped by K8S_SGEMV_WG_PER_CU (default 1: at 2 the 70B QKV / gate/up / down ran 9 / 3 / 3 %

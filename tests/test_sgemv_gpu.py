@@ -105,6 +105,15 @@ def test_llama70b_shapes(name, N, K, epi, norm, with_res, fp8):
         _run(M, N, K, epi, fp8, norm, with_res, seed=M)
 
 
+@pytest.mark.parametrize("M", [3, 8, 16])
+@pytest.mark.parametrize("N,K", [(2048, 6144), (2049, 6144), (2048, 8192), (1024, 8192), (1030, 8192), (5, 6016), (40, 14336)])
+def test_k_groups_of_few_bands(M, N, K):
+    """k-groups taken because the 16-row bands leave CUs idle: either side of one band per CU and group, of the least depth and
+    of two steps a wave, with every epilogue."""
+    for epi, res in ((ops.EPI_BF16, False), (ops.EPI_BF16, True), (ops.EPI_F32, False), (ops.EPI_SWIGLU, False)):
+        _run(M, N, K, epi, False, False, res, seed=N + K)
+
+
 def test_deterministic():
     w = _weights(8192, 28672, False, 3)
     x = (torch.rand(6, 28672, device=DEV) * 2 - 1).to(torch.bfloat16)
