@@ -293,15 +293,21 @@ __device__ __forceinline__ float dpp_add(float v) {
 __device__ __forceinline__ float quad_sum(float v) { return dpp_add<0x4E>(dpp_add<0xB1>(v)); }   // lanes ^ 1, ^ 2
 __device__ __forceinline__ float row_sum(float v) { return dpp_add<0x140>(dpp_add<0x141>(quad_sum(v))); }   // mirrored
 
-// MODE 2 for heads of at most 64 channels: two waves per (chunk, head).  Lane 4 jg + ig of a wave holds the state's 16 x 2
-// block of key channels 16 ig .. and value channels 32 wave + 2 jg .., so a token's r, k and w come from LDS once per 32
-// elements (a column per lane, as above, reads them once per 16, waits for them and for two barriers in every token: 129 us
-// for 2048 tokens of 32 heads of 64, this 52 us).  8 tokens are staged at a time, 4 by each wave (lane = channel) and their
-// outputs finished by the same one; the next 8 load meanwhile.  Bound by the vector units: 200 multiply-adds per token and
-// head in the walk and about 100 instructions for the decays, gates and norm.  The bonus term is a scalar per token:
-// sum_i r_i u_i k_i v_j = (sum_i r_i u_i k_i) v_j.
+// MODE 2 for heads of at most 64 channels on the matrix cores (v_mfma_f32_16x16x4_f32: fp32 in, fp32 sums), by 16 tokens t:
+//   o_t[j] = sum_i r_t[i] P_t[i] S[i][j] + sum_(s < t) A_ts v_s[j] + A_tt v_t[j],   A_ts = sum_i r_t[i] k_s[i] prod_(s < x < t) w_x[i],
+//   S'[i][j] = P[i] S[i][j] + sum_s (k_s[i] prod_(x > s) w_x[i]) v_s[j],            A_tt = sum_i r_t[i] u[i] k_t[i],
+// P_t the decays ahead of t, P those of all 16: products of numbers <= 1, multiplied up and never divided, so nothing overflows
+// whatever the decays.  A workgroup of 4 waves per (chunk, head), a wave 16 value columns of the state in 4 accumulators,
+// whose layout (row 4 g4 + e, column li) is the B operand of the first sum with the key channels taken in the order 16 m +
+// 4 g4 + e.  Staging: a wave 4 tokens, lane = channel, the next 16 tokens' loads in flight.
+// A without a division: the highest bit in which s and t differ cuts the tokens between them at a multiple of 2^bit, r_t takes the
+// decays from there on and k_s those up to there.  For every bit one 16 x 64 matrix M holds the rows r of the tokens with
+// the bit and the rows k of those without, and wave `bit` takes its part of A from M M^T (one fragment for both operands).
+// 2048 tokens of 32 heads of 64: 44 us, 333 in fp32 13.5 (walking the state token by token in registers, 200 vector multiply-adds
+// per token, head and wave: 54 and 22.6; A by a walk over t: 45 and 15.4).  About 850 vector instructions a wave for 16
+// tokens (24 us of the 44: the decays' and gates' exponentials, staging, the norm) and 52 products (11 us), four waves on a SIMD.
 template <typename TA>
-__global__ __launch_bounds__(128, 2) void wkv_chunk_out_kernel(TA* __restrict__ out, const TA* __restrict__ r,
+__global__ __launch_bounds__(256, 4) void wkv_chunk_out_kernel(TA* __restrict__ out, const TA* __restrict__ r,
                                                                const TA* __restrict__ k, const TA* __restrict__ v,
                                                                const TA* __restrict__ g, long ld,
                                                                const float* __restrict__ z, const TA* __restrict__ w0,
@@ -310,32 +316,35 @@ __global__ __launch_bounds__(128, 2) void wkv_chunk_out_kernel(TA* __restrict__ 
                                                                const int* __restrict__ seq_slots,
                                                                const int* __restrict__ positions, int H, int D, float eps,
                                                                int nseq, int Lc, const float* __restrict__ cs_start) {
-  constexpr int TB = 8, TW = TB / 2;
-  __shared__ __attribute__((aligned(16))) float sr[TB][64], sk[TB][64], sw[TB][64], sv[TB][64], so[TB][64];
+  constexpr int TB = 16, TW = TB / 4, LR = 68, LC = 80;   // row strides: conflict-free 16-byte rows, 4-byte columns
+  __shared__ __attribute__((aligned(16))) float lv[4][TB][LR], rp[TB][LR], kp[TB][LC], sv[TB][LC];
+  __shared__ __attribute__((aligned(16))) float sa[TB][20], tot[4][64], dec[64], ssq[4][TB];
+  __shared__ int odd[4];
   const int hd = blockIdx.y;
   const WkvChunk ck = wkv_find_chunk(blockIdx.x, cu_q, positions, nseq, Lc);
   if (ck.s < 0) return;
   const int a = __builtin_amdgcn_readfirstlane(cu_q[ck.s] + ck.c * Lc);
   const int b = __builtin_amdgcn_readfirstlane(min(cu_q[ck.s + 1], a + Lc));
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int ig = lane & 3, j0 = 32 * wave + 2 * (lane >> 2), HD = H * D;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, li = lane & 15, g4 = lane >> 4;
+  const int j = 16 * wave + li, jc = min(j, D - 1), HD = H * D;      // this lane's value column
   const bool on = lane < D;
   float* st = state + ((size_t)seq_slots[ck.s] * H + hd) * D * D;
   const float* src = ck.n > 1 ? cs_start + ((size_t)blockIdx.x * H + hd) * D * D : st;
   const bool from_zero = positions[a] == 0;
-  float S[16][2];
+  f32x4 S[4];                                     // S[m][e]: key channel 16 m + 4 g4 + e, value column j
 #pragma unroll
-  for (int e = 0; e < 16; ++e)
+  for (int m = 0; m < 4; ++m)
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int x = 16 * ig + e, y = j0 + q;
-      const float f = src[min(x, D - 1) * D + min(y, D - 1)];
-      S[e][q] = !from_zero && x < D && y < D ? f : 0.f;
+    for (int e = 0; e < 4; ++e) {
+      const int i = 16 * m + 4 * g4 + e;
+      const float f = src[min(i, D - 1) * D + jc];
+      S[m][e] = !from_zero && i < D && j < D ? f : 0.f;
     }
   const size_t h0 = (size_t)hd * D;
   const unsigned lc = min(lane, D - 1);
-  const float uj = ldf(u + h0, lc), w0j = ldf(w0 + h0, lc), lnj = ldf(lnw + h0, lc);
-  TA nr[TW], nk[TW], nv[TW], ng[TW];              // the next tokens as they come: converted only once they are staged
+  const float w0i = ldf(w0 + h0, lc), lnj = ldf(lnw + h0, jc), ui = ldf(u + h0, lc);
+  if (threadIdx.x < TB * TB) sa[threadIdx.x >> 4][threadIdx.x & 15] = 0.f;     // (t < s stays 0)
+  TA nr[TW], nk[TW], nv[TW];                      // the next tokens as they come: converted only once they are staged
   float nz[TW];
   auto fetch = [&](int t0) {
 #pragma unroll
@@ -345,96 +354,147 @@ __global__ __launch_bounds__(128, 2) void wkv_chunk_out_kernel(TA* __restrict__ 
       nr[x] = (r + base)[lc];
       nk[x] = (k + base)[lc];
       nv[x] = (v + base)[lc];
-      ng[x] = (g + base)[lc];
       nz[x] = (z + (size_t)t * HD + h0)[lc];
     }
   };
   fetch(a);
   for (int t0 = a; t0 < b; t0 += TB) {
-    const int tw = t0 + TW * wave;                // this wave's first token
-    float bonus[TW], cv[TW], cg[TW];
+    float rx[TW], kx[TW], wx[TW];
+    bool fin = true;
 #pragma unroll
-    for (int x = 0; x < TW; ++x) {                // a token or channel that is not there: k = r = 0, w = 1
-      const bool in = on && tw + x < b;
-      const float rx = in ? ldf(nr, x) : 0.f, kx = in ? ldf(nk, x) : 0.f, w = expf(-expf(nz[x] + w0j));
-      cv[x] = in ? ldf(nv, x) : 0.f;
-      cg[x] = ldf(ng, x);
-      bonus[x] = row_sum(rx * (uj * kx));
-      sr[TW * wave + x][lane] = rx;
-      sk[TW * wave + x][lane] = kx;
-      sv[TW * wave + x][lane] = cv[x];
-      sw[TW * wave + x][lane] = in ? w : 1.f;
+    for (int x = 0; x < TW; ++x) {                // a token or channel that is not there: r = k = v = 0, w = 1
+      const int t = TW * wave + x;
+      const bool in = on && t0 + t < b;
+      const float w = expf(-expf(nz[x] + w0i)), vx = in ? ldf(nv, x) : 0.f;
+      rx[x] = in ? ldf(nr, x) : 0.f;
+      kx[x] = in ? ldf(nk, x) : 0.f;
+      wx[x] = in ? w : 1.f;
+      fin = fin && fabsf(vx) < INFINITY;
+      sv[t][lane] = vx;
     }
-    if (t0 + TB < b) fetch(t0 + TB);
-    lds_barrier();
-    // a step: 4 of the 16 key channels of a token; its rows are read two steps ahead
-    f32x4 r4[3], k4[3], w4[3];
-    typedef __attribute__((ext_vector_type(2))) float f32x2;
-    f32x2 v2[2];
-    auto rows = [&](int step) {
-      const int x = step >> 2, c = 16 * ig + 4 * (step & 3);
-      if ((step & 3) == 0) v2[x & 1] = *reinterpret_cast<const f32x2*>(&sv[x][j0]);
-      r4[step % 3] = *reinterpret_cast<const f32x4*>(&sr[x][c]);
-      k4[step % 3] = *reinterpret_cast<const f32x4*>(&sk[x][c]);
-      w4[step % 3] = *reinterpret_cast<const f32x4*>(&sw[x][c]);
-    };
-    rows(0);
-    rows(1);
-    float o[2][2];                                // even and odd key channels: two chains per value channel
+    const float w01 = wx[0] * wx[1], w23 = wx[2] * wx[3];
+    const float before[4] = {1.f, wx[0], w01, w01 * wx[2]}, after[4] = {wx[1] * w23, w23, wx[3], 1.f};    // in these 4 tokens
+    tot[wave][lane] = w01 * w23;
 #pragma unroll
-    for (int step = 0; step < 4 * TB; ++step) {
-      const int x = step >> 2, e0 = 4 * (step & 3), n = step % 3;
-      if (step + 2 < 4 * TB) rows(step + 2);
+    for (int x = 0; x < TW; ++x) {                // bits 0 - 2 lie within the 4 tokens
+      const int t = TW * wave + x;
+      lv[0][t][lane] = x & 1 ? rx[x] : kx[x];
+      lv[1][t][lane] = x == 0 ? kx[0] * wx[1] : x == 1 ? kx[1] : x == 2 ? rx[2] : rx[3] * wx[2];
+      lv[2][t][lane] = wave & 1 ? rx[x] * before[x] : kx[x] * after[x];
+    }
+    float own[TW];                                // A_tt
+#pragma unroll
+    for (int x = 0; x < TW; ++x) own[x] = row_sum(rx[x] * (ui * kx[x]));
+#pragma unroll
+    for (int m = 32; m > 8; m >>= 1)
+#pragma unroll
+      for (int x = 0; x < TW; ++x) own[x] += __shfl_xor(own[x], m, WAVE);
+    const bool all = __all(fin);
+    if (lane == 0) odd[wave] = !all;
+    if (t0 + TB < b) fetch(t0 + TB);
+    TA ng[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ng[e] = (g + (size_t)min(t0 + 4 * g4 + e, b - 1) * ld + h0)[jc];
+    lds_barrier();
+    {
+      float ahead = 1.f, behind = 1.f;
+      const float q0 = tot[0][lane], q1 = tot[1][lane], q2 = tot[2][lane], q3 = tot[3][lane];
+      if (wave > 0) ahead = q0;
+      if (wave > 1) ahead *= q1;
+      if (wave > 2) ahead *= q2;
+      if (wave < 3) behind = q3;
+      if (wave < 2) behind *= q2;
+      if (wave < 1) behind *= q1;
+      if (wave == 0) dec[lane] = (q0 * q1) * (q2 * q3);
+      const float near = wave == 3 ? q2 : wave == 0 ? q1 : 1.f;    // bit 3: the other 4 tokens of this half, if between
+#pragma unroll
+      for (int x = 0; x < TW; ++x) {
+        const int t = TW * wave + x;
+        const float f = rx[x] * before[x], l = kx[x] * after[x];
+        rp[t][lane] = f * ahead;
+        kp[t][lane] = l * behind;
+        lv[3][t][lane] = (wave > 1 ? f : l) * near;
+        if (lane == 0) sa[t][t] = own[x];
+      }
+    }
+    lds_barrier();
+    {
+      f32x4 y = f32x4{0.f, 0.f, 0.f, 0.f};        // y[e]: t = 4 g4 + e, s = li
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(&lv[wave][li][16 * m + 4 * g4]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], x[e], y, 0, 0, 0);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int t = 4 * g4 + e;
+        if (((t ^ li) >> wave) == 1 && t > li) sa[t][li] = y[e];
+      }
+    }
+    f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};          // o[e]: token 4 g4 + e, value column j
+    float vs[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) vs[q] = sv[4 * q + g4][j];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(&rp[li][16 * m + 4 * g4]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], S[m][e], o, 0, 0, 0);
+    }
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const f32x4 f = *reinterpret_cast<const f32x4*>(&dec[16 * m + 4 * g4]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[m][e] *= f[e];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) S[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(kp[4 * q + g4][16 * m + li], vs[q], S[m], 0, 0, 0);
+    lds_barrier();
+    if ((odd[0] | odd[1]) | (odd[2] | odd[3])) {  // an infinite or NaN value: it does not reach the tokens ahead of it
 #pragma unroll
       for (int e = 0; e < 4; ++e)
+        for (int s = 0; s <= 4 * g4 + e; ++s) o[e] = fmaf(sa[4 * g4 + e][s], sv[s][j], o[e]);
+    } else {
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          float& acc = o[e & 1][q];
-          acc = e0 + e < 2 ? r4[n][e] * S[e][q] : fmaf(r4[n][e], S[e0 + e][q], acc);
-          S[e0 + e][q] = fmaf(w4[n][e], S[e0 + e][q], k4[n][e] * v2[x & 1][q]);
-        }
-      if (e0 == 12) {
-        const float y0 = quad_sum(o[0][0] + o[1][0]), y1 = quad_sum(o[0][1] + o[1][1]);
-        if (ig < 2) so[x][j0 + ig] = ig == 0 ? y0 : y1;
-      }
-      __builtin_amdgcn_sched_barrier(0);
+      for (int q = 0; q < 4; ++q) o = __builtin_amdgcn_mfma_f32_16x16x4f32(sa[li][4 * q + g4], vs[q], o, 0, 0, 0);
     }
+    f32x4 ss;
 #pragma unroll
-    for (int m = 32; m > 8; m >>= 1)
-#pragma unroll
-      for (int x = 0; x < TW; ++x) bonus[x] += __shfl_xor(bonus[x], m, WAVE);
+    for (int e = 0; e < 4; ++e) ss[e] = row_sum(o[e] * o[e]);
+    if (li == 0) *reinterpret_cast<f32x4*>(&ssq[wave][4 * g4]) = ss;
     lds_barrier();
-    float y[TW], ss[TW];
 #pragma unroll
-    for (int x = 0; x < TW; ++x) {
-      y[x] = on ? fmaf(bonus[x], cv[x], so[TW * wave + x][lane]) : 0.f;
-      ss[x] = row_sum(y[x] * y[x]);
+    for (int w = 0; w < 4; ++w) {
+      const f32x4 y = *reinterpret_cast<const f32x4*>(&ssq[w][4 * g4]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ss[e] = w == 0 ? y[e] : ss[e] + y[e];
     }
 #pragma unroll
-    for (int m = 32; m > 8; m >>= 1)
-#pragma unroll
-      for (int x = 0; x < TW; ++x) ss[x] += __shfl_xor(ss[x], m, WAVE);
-#pragma unroll
-    for (int x = 0; x < TW; ++x) {                // o / rms * lnw * silu(g), one division
-      y[x] = y[x] * lnj * cg[x] / (sqrtf(ss[x] / (float)D + eps) * (1.f + expf(-cg[x])));
-      if (on && tw + x < b) stf(out + (size_t)(tw + x) * HD + h0, lane, y[x]);
+    for (int e = 0; e < 4; ++e) {                 // o / rms * lnw * silu(g), one division
+      const int t = t0 + 4 * g4 + e;
+      const float c = ldf(ng, e), y = o[e] * lnj * c * rsqrtf(ss[e] / (float)D + eps) / (1.f + expf(-c));
+      if (t < b && j < D) stf(out + (size_t)t * HD + h0, j, y);
     }
   }
   if (ck.c == ck.n - 1) {
 #pragma unroll
-    for (int e = 0; e < 16; ++e)
+    for (int m = 0; m < 4; ++m)
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int x = 16 * ig + e, y = j0 + q;
-        if (x < D && y < D) st[(size_t)x * D + y] = S[e][q];
+      for (int e = 0; e < 4; ++e) {
+        const int i = 16 * m + 4 * g4 + e;
+        if (i < D && j < D) st[(size_t)i * D + j] = S[m][e];
       }
   }
 }
 
 // start[first chunk + c + 1] = dec[c] * start[c] + loc[c] along a sequence's chunks; start of chunk 0 is the slot's state
 // (or zero at position 0), copied here: the pass that reads it runs beside the one that replaces the slot's.  Workgroups (sequence, head, 256 state elements), a
-// thread per element with 8 chunks' records in flight: 2048 tokens, 32 heads of 64 x 64, 131 us with one workgroup per head
-// and a load waited for in every step, 15 us now (33 MB read and written: 4 us at 8 TB/s each way, the rest latency).
+// thread per element with 16 chunks' records in flight: 2048 tokens, 32 heads of 64 x 64, 131 us with one workgroup per head
+// and a load waited for in every step, 14.8 us with 8 records in flight, 11 with 16 (33 MB read and written: 4 us at 8 TB/s each way, the
+// rest latency).
 __global__ __launch_bounds__(256) void wkv_prefix_kernel(float* __restrict__ cs_start, const float* __restrict__ cs_loc,
                                                          const float* __restrict__ cs_dec, const float* __restrict__ state,
                                                          const int* __restrict__ cu_q, const int* __restrict__ seq_slots,
@@ -452,7 +512,7 @@ __global__ __launch_bounds__(256) void wkv_prefix_kernel(float* __restrict__ cs_
   const int i = e / D;
   float S = positions[a] == 0 ? 0.f : state[((size_t)seq_slots[s] * H + hd) * D * D + e];
   cs_start[((size_t)first * H + hd) * D * D + e] = S;
-  constexpr int PF = 8;
+  constexpr int PF = 16;
   for (int c0 = 0; c0 < n; c0 += PF) {
     float dec[PF], loc[PF];
 #pragma unroll
@@ -960,7 +1020,7 @@ extern "C" int k8s_wkv_scan(void* out, const void* r, const void* k, const void*
                                                                             nseq, Lc, loc, dec);
   wkv_prefix_kernel<<<dim3(nseq, H, (D * D + 255) / 256), 256, 0, s>>>(start, loc, dec, state, cu_q, seq_slots, positions, H, D, Lc);
 #define K8S_WKVO(TA)                                                                                                   \
-  wkv_chunk_out_kernel<TA><<<dim3(chunks, H), 128, 0, s>>>((TA*)out, (const TA*)r, (const TA*)k, (const TA*)v,           \
+  wkv_chunk_out_kernel<TA><<<dim3(chunks, H), 256, 0, s>>>((TA*)out, (const TA*)r, (const TA*)k, (const TA*)v,           \
                                                           (const TA*)g, ld, z, (const TA*)w0, (const TA*)u,             \
                                                           (const TA*)lnw, state, cu_q, seq_slots, positions, H, D, eps, \
                                                           nseq, Lc, start)

@@ -551,3 +551,46 @@ def test_untuned_products_of_17_to_128_rows(M, N, K, epi):
     a, b = x.to(DEV).double(), w.to(DEV).double()
     exact, bound = a @ b.T, 2.0 * K * 2.0 ** -24 * (a.abs() @ b.abs().T) + 1e-30
     assert ((got.double() - exact).abs() <= bound + (2.0 ** -8 * exact.abs() if epi == 0 else 0.0)).all()
+
+
+def wkv64(r, k, v, g, z, w0, u, lnw, S, eps):
+    """The recurrence of one sequence in 64 bits, token by token: r .. z [T, H, D], S [H, D, D]; outputs and end state."""
+    w, out = torch.exp(-torch.exp(z + w0)), []
+    for t in range(r.shape[0]):
+        kv = k[t][:, :, None] * v[t][:, None, :]
+        out.append((r[t][:, :, None] * (S + u[:, :, None] * kv)).sum(1))
+        S = w[t][:, :, None] * S + kv
+    o = torch.stack(out)
+    return o / torch.sqrt((o * o).mean(-1, keepdim=True) + eps) * lnw * g * torch.sigmoid(g), S
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,D", [(3, 64), (2, 20), (5, 48)])
+@pytest.mark.parametrize("T,chunk", [(15, 64), (16, 64), (17, 16), (64, 64), (65, 64), (129, 48), (200, 25)])
+@pytest.mark.parametrize("value", [None, float("inf"), float("nan")])
+def test_wkv_outputs_by_16_tokens(dt, H, D, T, chunk, value):
+    """Ends of 16 tokens and of chunks, decays from none to all of the state within a token, and a value that is not finite:
+    it reaches its column from its own token on and nothing before it."""
+    gen = torch.Generator().manual_seed(T + D)
+    rnd = lambda *s: torch.randn(*s, generator=gen)
+    r, k, v, g = (rnd(T, H, D).to(dt) for _ in range(4))
+    z, w0, u, lnw = 3.0 * rnd(T, H, D), rnd(H, D).to(dt), (0.5 * rnd(H, D)).to(dt), (1 + 0.1 * rnd(H, D)).to(dt)
+    at = T - T // 3
+    if value is not None:
+        v[at, 1, 3] = value
+    S0 = rnd(1, H, D, D)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    S = S0.to(DEV).clone()
+    got = sm.wkv_scan(*(x.reshape(T, -1).to(DEV) for x in (r, k, v, g, z)), *(x.reshape(-1).to(DEV) for x in (w0, u, lnw)), S,
+                      i32([0, T]), i32([0]), i32(range(7, 7 + T)), H, D, 1e-6, chunk=chunk).view(T, H, D).double().cpu()
+    want, end = wkv64(*(x.double() for x in (r, k, v, g, z, w0, u, lnw, S0[0])), 1e-6)
+    head = torch.ones(T, H, dtype=torch.bool)
+    if value is not None:
+        head[at:, 1] = False
+        assert not torch.isfinite(got[at, 1]).all()
+    # chains of at most 64 + 16 + 64 fp32 terms and the decays' products: 2^-24 times their number at most, then the norm
+    # (outputs are of the order of one) and one rounding
+    ulp = 2.0 ** -24 if dt == torch.float32 else 2.0 ** -8
+    assert ((got - want)[head].abs() <= ulp * want[head].abs() + 2.0 ** -15 * (1 + want[head].abs())).all()
+    if value is None:
+        assert ((S[0].double().cpu() - end).abs() <= 2.0 ** -17 * (1 + end.abs().max())).all()
