@@ -595,20 +595,20 @@ __global__ void sgemv_finalize_kernel(void* __restrict__ out, const float* __res
 
 // MFMA plan (smfma_kernel): JT register steps per wave (1, 2, 4, 8; a step = 16 chunks of every row of a quad),
 // jw live steps, G k-groups.  Needs whole steps (K % 128 bf16, K % 256 fp8); one k-group covers 8 waves x 8 steps
-// (8192 k) -- fp8 4 steps (8192 k: an fp8 step holds twice the x of a bf16 one).  Bands of 16 rows (the least) that leave
-// CUs idle take more groups, as long as a wave keeps two steps and the depth pays for the reduction (2.3 us).  us, one group
-// -> the rule's: 8 x 2048 x 8192 12.8 -> 11.2, x 6144 11.1 -> 9.2, 8 x 1024 x 8192 12.6 -> 8.9, 16 x 2048 x 8192 16.5 -> 12.8;
-// K = 4096 stays in one (8 x 2048 7.8, two groups 8.1).  The norm prologue needs all of K in one group.
+// (8192 k) -- fp8 4 steps (8192 k: an fp8 step holds twice the x of a bf16 one).  9 - 16 rows take more groups where bands of
+// 16 output rows leave CUs idle, as long as a wave keeps two steps and the depth pays for the reduction (2.3 us): us, 16 rows,
+// one group -> the rule's: 2048 x 8192 16.5 -> 12.7, x 6144 14.1 -> 10.9, 1024 x 8192 16.3 -> 10.0.  Up to 8 rows narrower
+// bands do better (sm_launch).  The norm prologue needs all of K in one group.
 struct SmPlan {
   int jt, jw, g;
 };
 static int sm_cus();
-static bool sm_plan(int N, int K, bool fp8, bool norm, SmPlan& p) {
+static bool sm_plan(int M, int N, int K, bool fp8, bool norm, SmPlan& p) {
   const int epc = fp8 ? 16 : 8;
   if (K % (16 * epc) != 0) return false;
   const int c16 = K / (16 * epc), jmax = fp8 ? 4 : 8;
   int g = (c16 + SM_KW * jmax - 1) / (SM_KW * jmax);
-  if (!norm && c16 >= 48)
+  if (M > 8 && !fp8 && !norm && c16 >= 48)
     while ((N + 15) / 16 * g * 2 <= sm_cus() && c16 >= 4 * SM_KW * g) g *= 2;
   const int jw = (c16 + SM_KW * g - 1) / (SM_KW * g);
   p = {jw <= 1 ? 1 : (jw <= 2 ? 2 : (jw <= 4 ? 4 : 8)), jw, g};
@@ -633,7 +633,7 @@ static int sm_cus() {
   return v;
 }
 static bool sm_take(int M, int N, int K, bool fp8, bool norm, SmPlan& p) {
-  return M >= sm_min_m() && M <= 16 && sm_plan(N, K, fp8, norm, p);
+  return M >= sm_min_m() && M <= 16 && sm_plan(M, N, K, fp8, norm, p);
 }
 
 // Workgroups of the MFMA form per CU the band is sized for: what the kernel's registers allow (one for every form
@@ -655,12 +655,14 @@ static bool sm_launch(void* out, void* partial, const bf16_t* x, const void* W, 
       n = 1;
     return max(1, min(n, sm_wg_cap()));
   }();
-  // ~occ workgroups per CU and k-group, at least 16 rows (x is re-read per workgroup), at most the LDS partials'
-  // quads (SwiGLU: gate + up quads, with the phantom rounding)
+  // ~occ workgroups per CU and k-group, at least 8 rows (x is re-read per workgroup), at most the LDS partials'
+  // quads (SwiGLU: gate + up quads, with the phantom rounding).  us with at least 16 rows -> 8 (8 x 2048 x 8192: in two k-groups
+  // 11.2): 8 x 2048 x 8192 12.8 -> 9.5, x 4096 7.7 -> 6.1, x 2048 5.2 -> 4.8; 4 x 2048 x 8192 11.4 -> 8.8; 16 x 2048 x 4096 9.5 ->
+  // 7.5, x 2048 6.4 -> 5.9
   constexpr int qmax = 512 / MT;
   const int bandmax = 4 * qmax / (sg_paired(EE) ? 2 : 1);
   const int per = max(1, sm_cus() * occ / sp.g);
-  int band = max(min(16, N), (N + per - 1) / per);
+  int band = max(min(8, N), (N + per - 1) / per);
   if (band > bandmax) {
     int nb = (N + bandmax - 1) / bandmax;
     nb = (nb + per - 1) / per * per;   // whole rounds of workgroups
