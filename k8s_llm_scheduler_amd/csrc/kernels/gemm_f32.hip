@@ -9,9 +9,8 @@
 // with the eight shares of gemm_f32_kernel).
 //
 // Bound by the matrix rate (157 TFLOP/s at 2.4 GHz; the clock holds 2.25 here): 85 % of a busy CU's cycles with two workgroups
-// on it, 75 - 80 % with one (a stage's barrier and waits cost about 350 cycles).  333 rows (N x K), with the launch: 16384 x
-// 2048 258 -> 175 us (three rounds of 112-row tiles), 2048 x 2048 42 -> 36, 2048 x 8192 154 -> 130; 200 x 16384 x 2048 165 ->
-// 116, 512 x 4096 x 4096 174 -> 137.
+// on it, 70 - 80 % with one (a stage's barrier and waits cost about 350 cycles; a ring of 8 slots changes nothing).  us with the
+// launch: 333 x 16384 x 2048 258 -> 175 (three rounds of 112-row tiles), 200 x 16384 x 2048 165 -> 116.
 #include <type_traits>
 
 #include "common.h"
@@ -169,13 +168,184 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(F32Args a) {
 #endif
 }
 
+// The same product with k shared by the waves instead of the columns: a wave owns all 64 columns x 16 FQ rows of the tile for a
+// quarter of k, stages its own weights and rows (16-deep, 64-byte rows, a ring of 4 slots) and meets the others once, at the
+// end, in LDS -- no barrier and no other wave's loads to wait for while k lasts.  85 - 90 % of the matrix rate on a CU with one
+// workgroup (all that the rings leave room for).  us, columns shared -> k shared: 333 x 2048 x 2048 35.0 -> 31.4, x 8192 129 ->
+// 109, 200 x 2048 x 8192 97 -> 79, 200 x 4096 x 4096 81 -> 73, 100 x 4096 x 14336 170 -> 144, 64 x 16384 x 2048 50 -> 45; in three
+// rounds and more it is behind (333 x 16384 x 2048 180 and 203).  Ahead of gemm_f32_kernel's eight shares too: 333 x 576 x 2048
+// 18.0 -> 14.4, 64 x 2048 x 8192 68 -> 58.  Error against 64 bits, 2-norm: 2.1e-7 - 2.3e-7.
+template <typename TO, int FQ>
+__global__ __launch_bounds__(256, 1) void gemm_f32_kwave_kernel(F32Args a) {
+  constexpr int BP = 64, BQ = 16 * FQ, G = 4 + FQ, STAGE = G * 1024, NS = 4, RING = NS * STAGE;
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ __attribute__((aligned(16))) char lds[4 * RING];
+  static_assert(4 * RING >= 4 * BP * BQ * 4, "the waves' sums fit the rings");
+  const int tot = a.mt * a.nt * a.batch, q8 = tot >> 3, r8 = tot & 7, xcd = blockIdx.x & 7;
+  int t = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (int)(blockIdx.x >> 3);
+  const int ti = t % a.mt;
+  t /= a.mt;
+  const int tj = t % a.nt, tb = t / a.nt;
+  const float *A = a.A + (size_t)tb * a.sA, *W = a.W + (size_t)tb * a.sW;
+  int row0 = ti * BQ, rows = min(BQ, a.M - row0);
+  if (a.tiles != nullptr) {
+    constexpr int PER = 64 / BQ > 0 ? 64 / BQ : 1;
+    const int y = ti / PER, sub = (ti - y * PER) * BQ, g = a.tiles[3 * y];
+    if (g < 0) return;
+    row0 = a.tiles[3 * y + 1] + sub;
+    rows = min(BQ, a.tiles[3 * y + 2] - sub);
+    if (rows <= 0) return;
+    W += (size_t)g * a.sW;
+  }
+  const int col0 = tj * BP;
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, g = lane >> 4;
+  const int S = a.K / 16, first = wid * S / 4, last = (wid + 1) * S / 4 - 1;     // this wave's 16-deep stages (K >= 64)
+  // loader: instruction j moves 16 rows of the stage (weights first), 16 bytes a lane; rows past the end repeat the last one
+  const float* src[G];
+  const int lr = lane >> 2, lc = ((lane & 3) ^ (lr >> 2)) * 4;
+#pragma unroll
+  for (int j = 0; j < G; ++j) {
+    if (j < 4) {
+      src[j] = W + (size_t)min(col0 + 16 * j + lr, a.N - 1) * a.ldw + lc;
+    } else {
+      const int r = row0 + min(16 * (j - 4) + lr, rows - 1);
+      src[j] = A + (size_t)(a.a_rows != nullptr ? a.a_rows[r] : r) * a.lda + lc;
+    }
+  }
+  char* mine = lds + wid * RING;
+  auto dma = [&](int u, int slot, int j) {
+    __builtin_amdgcn_global_load_lds(src[j] + (size_t)u * 16,
+                                     (__attribute__((address_space(3))) void*)(mine + slot * STAGE + j * 1024), 16, 0, 0);
+  };
+  const uint32_t base = (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)mine);
+  const uint32_t pl = base + li * 64 + ((g ^ (li >> 2)) << 4);
+  f32x4 f0[G], f1[G], acc[4][FQ], sum[4][FQ];      // fragments: 4 of weights, FQ of rows
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < FQ; ++j) sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto read = [&](uint32_t o, int r, f32x4* f) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f[r]) : "v"(pl + o), "i"(r * 1024));
+  };
+  // Products of f with (more) the reads of the next stage at o into n in their first half and the loads of stage u into slot us,
+  // whose fragments are those of f, in the second.  A read's output is always used by the next phase, and nothing touches it
+  // before the wait at the end; the products are opaque to the hazard recogniser, so the phase also waits out their latency
+  // (the matrix unit is busy with the last one that long anyway).
+  auto phase = [&](auto more, const f32x4* f, f32x4* n, uint32_t o, int u, int us) {
+    constexpr int MF = 16 * FQ;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < FQ; ++j) {
+          const int k = (e * 4 + i) * FQ + j;
+          asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+v"(acc[i][j]) : "v"(f[i][e]), "v"(f[4 + j][e]));
+          if constexpr (decltype(more)::value) {
+#pragma unroll
+            for (int r = 0; r < G; ++r)
+              if (k == r * (MF / 2) / G) read(o, r, n);
+#pragma unroll
+            for (int d = 0; d < G; ++d)
+              if (k == MF / 2 + d * (MF / 2) / G) dma(u, us, d);
+          }
+        }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
+    if constexpr (decltype(more)::value) f32_vmcnt<(NS - 2) * G>();        // the stage after the next has landed
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto clear = [&]() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < FQ; ++j) {
+        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        asm volatile("" : "+v"(acc[i][j]));
+      }
+    asm volatile("s_nop 7" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto flush = [&]() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < FQ; ++j) {
+        asm volatile("" : "+v"(acc[i][j]));
+        sum[i][j] += acc[i][j];
+      }
+    clear();
+  };
+#pragma unroll
+  for (int q = 0; q < NS; ++q)
+#pragma unroll
+    for (int d = 0; d < G; ++d) dma(min(first + q, last), q, d);
+  clear();
+  f32_vmcnt<(NS - 1) * G>();
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int r = 0; r < G; ++r) read(0, r, f0);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  f32_vmcnt<(NS - 2) * G>();
+  __builtin_amdgcn_sched_barrier(0);
+  const int n = last - first + 1, chain = 2 * a.chain + 1;        // a chain's stages - 1
+  int slot = 0, s = 0;
+  auto step = [&](auto more, const f32x4* f, f32x4* nx) {
+    const int next = slot + 1 == NS ? 0 : slot + 1;
+    phase(more, f, nx, (uint32_t)(next * STAGE), min(first + s + NS, last), slot);
+    slot = next;
+    if ((s & chain) == chain || !decltype(more)::value) flush();
+    ++s;
+  };
+  constexpr std::true_type yes{};
+  while (s + 2 < n) {
+    step(yes, f0, f1);
+    step(yes, f1, f0);
+  }
+  if (s + 2 == n) {
+    step(yes, f0, f1);
+    step(std::false_type{}, f1, f0);
+  } else {
+    step(std::false_type{}, f0, f1);
+  }
+  f32_vmcnt<0>();             // no load into LDS is left behind
+  __syncthreads();
+  float* red = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < FQ; ++j) *reinterpret_cast<f32x4*>(red + (((wid * 4 + i) * FQ + j) * 64 + lane) * 4) = sum[i][j];
+  __syncthreads();
+  // C[row 16 j + li][column 16 wid + 4 g + e]
+  TO* C = reinterpret_cast<TO*>(a.C) + (size_t)tb * a.sC;
+  const int c = col0 + 16 * wid + 4 * g;
+#pragma unroll
+  for (int j = 0; j < FQ; ++j) {
+    const int r = 16 * j + li;
+    f32x4 y = *reinterpret_cast<const f32x4*>(red + ((wid * FQ + j) * 64 + lane) * 4);
+#pragma unroll
+    for (int w = 1; w < 4; ++w) y += *reinterpret_cast<const f32x4*>(red + (((w * 4 + wid) * FQ + j) * 64 + lane) * 4);
+    if (r >= rows || c >= a.N) continue;
+    const size_t at = (size_t)(row0 + r) * a.ldc + c;
+    if (a.vec) {
+      stf4(C + at, y);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < a.N) stf(C, at + e, y[e]);
+    }
+  }
+#endif
+}
+
 }  // namespace k8sllm
 
 using namespace k8sllm;
 
 // The tile for a product, and whether it is expected to beat gemm_f32_kernel's tiles (0: it is not): both in us per 32 k, one
 // constant part and one per round of tiles over the CUs, fitted to M 24 - 512, N 128 - 16384, K 512 - 8192 (where the two
-// models are within 5 % of each other, so are the kernels).  K < 512: shares of K / 8 leave the smaller error.
+// models are within 5 % of each other, so are the kernels).  16 more: k shared by the waves; a round of one workgroup per CU
+// also pays its start and its sum (4.5 us, of which nothing overlaps), so it is the choice for one or two rounds.  K < 512:
+// shares of K / 8 leave the smaller error.
 extern "C" int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles) {
   if (K < 512 || K % 32 || M <= 0 || N <= 0) return 0;
   const auto rounds = [&](long rows, long cols) { return (double)((rows * cols * batch + 255) / 256); };
@@ -185,20 +355,28 @@ extern "C" int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles) {
   int pick = 0;
   for (int fq = 8; fq >= 1; --fq) {
     if (ntiles > 0 && 64 % (16 * fq)) continue;
-    const double t = rounds(ntiles > 0 ? 4L / fq * ntiles : (M + 16 * fq - 1) / (16 * fq), (N + 63) / 64) * (0.125 * fq + 0.04) + 0.1;
+    const double r = rounds(ntiles > 0 ? 4L / fq * ntiles : (M + 16 * fq - 1) / (16 * fq), (N + 63) / 64);
+    const double t = r * (0.125 * fq + 0.04) + 0.1;
     if (t < best) {
       best = t;
       pick = fq;
+    }
+    const double tk = r * (0.12 * fq + 0.03 + 4.5 * 32 / K);
+    if (fq <= 4 && tk < 0.96 * best) {
+      best = tk;
+      pick = 16 + fq;
     }
   }
   return pick;
 }
 
-// fq: rows of a tile / 16 (1 - 8; listed tiles of at most 64 rows: 1, 2, 4).
+// fq: rows of a tile / 16 (1 - 8; listed tiles of at most 64 rows: 1, 2, 4), or 16 + that (1 - 4): k shared by the waves.
 extern "C" int k8s_gemm_f32_tiles(void* C, const float* A, const float* W, int M, int N, int K, long lda, long ldw, long ldc,
                                   int batch, long sA, long sW, long sC, const int* a_rows, const int* tiles, int ntiles,
                                   int out_f32, int fq, hipStream_t s) {
-  if (M <= 0 || N <= 0 || K < 32 || K % 32 || batch <= 0 || fq < 1 || fq > 8 || (lda | ldw | sA | sW) % 4 ||
+  const bool kwave = fq > 16;
+  if (kwave) fq -= 16;
+  if (M <= 0 || N <= 0 || K < (kwave ? 64 : 32) || K % 32 || batch <= 0 || fq < 1 || fq > (kwave ? 4 : 8) || (lda | ldw | sA | sW) % 4 ||
       (((uintptr_t)A | (uintptr_t)W) & 15))
     return -1;
   if (tiles != nullptr && (64 % (16 * fq) || ntiles <= 0)) return -1;
@@ -212,6 +390,13 @@ extern "C" int k8s_gemm_f32_tiles(void* C, const float* A, const float* W, int M
   a.chain = K >= 2048 ? 3 : K >= 1024 ? 1 : 0;
   auto go = [&](auto n) {
     constexpr int FQ = decltype(n)::value;
+    if constexpr (FQ <= 4) {
+      if (kwave) {
+        if (out_f32) gemm_f32_kwave_kernel<float, FQ><<<dim3((unsigned)blocks), 256, 0, s>>>(a);
+        else gemm_f32_kwave_kernel<bf16_t, FQ><<<dim3((unsigned)blocks), 256, 0, s>>>(a);
+        return;
+      }
+    }
     if (out_f32) gemm_f32_tile_kernel<float, FQ><<<dim3((unsigned)blocks), 256, 0, s>>>(a);
     else gemm_f32_tile_kernel<bf16_t, FQ><<<dim3((unsigned)blocks), 256, 0, s>>>(a);
   };

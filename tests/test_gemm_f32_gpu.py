@@ -79,3 +79,39 @@ def test_batched_and_grouped():
             x = a[pick[seg[e]:seg[e + 1]].long()]
             d = (out[seg[e]:seg[e + 1]].double() - x.double() @ w[e].double().T).abs()
             assert (d <= bound(x, w[e], 1024)).all(), (fq, e)
+
+
+@pytest.mark.parametrize("fq", range(1, 5))
+@pytest.mark.parametrize("rows,N,K", [(0, 64, 64), (1, 130, 96), (-1, 67, 160), (5, 200, 1056), (0, 63, 2208), (1, 64, 544)])
+def test_k_shared_by_the_waves(fq, rows, N, K):
+    """As above for the tiles whose waves share k: one stage a wave and more, uneven shares, an odd number of them, and infinities
+    and NaN in the last and the first k."""
+    M = 16 * fq * (2 if rows == 5 else 1) + rows
+    g = torch.Generator().manual_seed(fq * 1000 + N)
+    a, w = (torch.randint(-8, 9, (n, K), generator=g).float().cuda() for n in (M, N))
+    assert torch.equal(tiles_call(a, w, 16 + fq).double(), a.double() @ w.double().T)      # |sums| < 2^24
+    a = torch.randn(M, K + 4, generator=g).cuda()[:, :K]
+    w = torch.randn(N, K, generator=g).cuda()
+    ref = a.double() @ w.double().T
+    assert ((tiles_call(a, w, 16 + fq, ldc=N + 1).double() - ref).abs() <= bound(a, w, K)).all()
+    assert ((tiles_call(a, w, 16 + fq, torch.bfloat16).double() - ref).abs() <= bound(a, w, K) + 2.0**-8 * ref.abs()).all()
+    a[M // 2, K - 1], w[N // 3, 0] = float("inf"), float("nan")
+    bad = ~tiles_call(a, w, 16 + fq).isfinite()
+    assert bad[M // 2].all() and bad[:, N // 3].all() and int(bad.sum()) == M + N - 1
+
+
+@pytest.mark.parametrize("fq", [1, 2, 4])
+def test_listed_tiles_with_k_shared(fq):
+    g = torch.Generator().manual_seed(fq)
+    counts = [70, 0, 64, 1]
+    seg = torch.tensor([0] + counts).cumsum(0).int()
+    listed = [(e, int(seg[e]) + r, min(64, n - r)) for e, n in enumerate(counts) for r in range(0, n, 64)] + [(-1, 0, 0)]
+    tiles = torch.tensor(listed, dtype=torch.int32).cuda()
+    a, w = torch.randn(50, 576, generator=g).cuda(), torch.randn(4, 130, 576, generator=g).cuda()
+    pick = torch.randint(0, 50, (int(seg[-1]),), generator=g).int().cuda()
+    out = torch.empty(int(seg[-1]), 130, device="cuda")
+    ops.native().gemm_f32_tiles(out.data_ptr(), a.data_ptr(), w.data_ptr(), out.shape[0], 130, 576, 576, 576, 130, 1, 0, 130 * 576, 0,
+                                pick.data_ptr(), tiles.data_ptr(), len(listed), 1, 16 + fq, -1)
+    for e in range(4):
+        x = a[pick[seg[e]:seg[e + 1]].long()]
+        assert ((out[seg[e]:seg[e + 1]].double() - x.double() @ w[e].double().T).abs() <= bound(x, w[e], 576)).all(), e
