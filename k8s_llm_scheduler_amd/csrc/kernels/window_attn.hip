@@ -1026,12 +1026,16 @@ __global__ __launch_bounds__(512, 4) void window_prompt_kernel(
 }
 
 // Single tokens on the matrix cores (no pooled blocks, DK key and value dimensions, pages of a power of two, at most 16 query
-// heads per key head): workgroups (token, key head, key split) of 4 waves.  A wave walks its own 32-key tiles without a
+// heads per key head): workgroups (token, key head, key split) of NW waves.  A wave walks its own 32-key tiles without a
 // workgroup barrier: keys go from the cache straight into MFMA operands (a lane loads 8 dimensions of one key), values
 // through the wave's LDS rows for the transposing read; the 16 columns of the products are the group's heads (padded).  The
 // waves merge in LDS; one split writes the result, several leave (max, sum, unnormalised sum) for window_merge_kernel.
-template <int DK>
-__global__ __launch_bounds__(256) void window_token_kernel(
+// A tile is a chain of loads and LDS of 2.5 us, the merge's launch 4 us: 8 waves take the tiles of 512 keys in two rounds and
+// need no splits.  16 heads over 4 of 128, us, 4 waves with splits and their merge -> 8 waves: 32 tokens behind up to 545 keys
+// 17.5 -> 13.9, behind 100 10.0 -> 6.2, 64 behind 545 20.4 -> 14.8; with half the splits one token behind 1024 14.6 -> 12.5, 8
+// behind 1500 without a window 21.3 -> 15.3.  16 waves (no splits at all) do not fit 128 registers at 128 dimensions: 19.1.
+template <int DK, int NW>
+__global__ __launch_bounds__(64 * NW) void window_token_kernel(
     bf16_t* __restrict__ out, float* __restrict__ pacc, float* __restrict__ pml, const bf16_t* __restrict__ q, long ldq,
     const bf16_t* __restrict__ gate, long ldg, const bf16_t* __restrict__ kcache, const bf16_t* __restrict__ vcache,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ tok_seq,
@@ -1039,14 +1043,14 @@ __global__ __launch_bounds__(256) void window_token_kernel(
     float softcap, const float* __restrict__ sinkv, int gate_ph, const float* __restrict__ slopes) {
   constexpr int NKK = DK / 32, NVB = DK / 16, C8 = DK / 8, ROWV = (DK + 8) * 2, NV = 32 * C8 / 64;
   constexpr float LOG2E = 1.4426950408889634f, LN2 = 0.6931471805599453f;
-  __shared__ __attribute__((aligned(16))) char vrows[4][32 * ROWV];   // a wave's values; later its sums [R][DK] fp32
-  __shared__ float ml[4][16][2];
+  __shared__ __attribute__((aligned(16))) char vrows[NW][32 * ROWV];   // a wave's values; later its sums [R][DK] fp32
+  __shared__ float ml[NW][16][2];
   const int t = blockIdx.x, g = blockIdx.y, split = blockIdx.z, R = H / G;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, g4 = lane >> 4;
   const int p = positions[t];
   if (p < 0) {   // idle row: defined output, nothing read
     if (nsplit == 1)
-      for (int i = tid; i < R * DK; i += 256) out[(size_t)t * H * DK + (size_t)g * R * DK + i] = 0;
+      for (int i = tid; i < R * DK; i += 64 * NW) out[(size_t)t * H * DK + (size_t)g * R * DK + i] = 0;
     return;
   }
   const int lo = chunk > 0 ? p - p % chunk : (window > 0 ? max(0, p - window + 1) : 0);
@@ -1069,7 +1073,7 @@ __global__ __launch_bounds__(256) void window_token_kernel(
   for (int n = 0; n < NVB; ++n) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
   char* vl = vrows[wave];
   const int qd = li >> 2, pd = li & 3;
-  for (int tile = tile0 + wave; tile < tile1; tile += 4) {
+  for (int tile = tile0 + wave; tile < tile1; tile += NW) {
     const int j0 = lo + tile * 32;
     int slot[2];                                  // cache slots of keys j0 + li and j0 + 16 + li
 #pragma unroll
@@ -1166,14 +1170,14 @@ __global__ __launch_bounds__(256) void window_token_kernel(
       for (int n = 0; n < NVB; ++n) mine[(4 * g4 + i) * DK + 16 * n + li] = o[n][i];
     }
   __syncthreads();
-  for (int idx = tid; idx < R * DK; idx += 256) {
+  for (int idx = tid; idx < R * DK; idx += 64 * NW) {
     const int r = idx / DK, d = idx - r * DK, h = g * R + r;
     float M = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) M = fmaxf(M, ml[w][r][0]);
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, ml[w][r][0]);
     float a = 0.f, l = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < NW; ++w) {
       const float f = ml[w][r][0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[w][r][0] - M);
       a += f * reinterpret_cast<const float*>(vrows[w])[idx];
       l += f * ml[w][r][1];
@@ -1331,14 +1335,20 @@ extern "C" int k8s_window_token(void* out, float* pacc, float* pml, const void* 
   if (nsplit < 1 || nsplit > 64 || (nsplit > 1 && (pacc == nullptr || pml == nullptr))) return -1;
   int bshift = 0;
   while ((1 << bshift) < bs) ++bshift;
-#define K8S_WT(DK)                                                                                                        \
-  window_token_kernel<DK><<<dim3(T, G, nsplit), 256, 0, s>>>(                                                             \
+#define K8S_WT(DK, NW)                                                                                                    \
+  window_token_kernel<DK, NW><<<dim3(T, G, nsplit), 64 * NW, 0, s>>>(                                                     \
       (bf16_t*)out, pacc, pml, (const bf16_t*)q, ldq, (const bf16_t*)gate, ldg, (const bf16_t*)kcache,                    \
       (const bf16_t*)vcache, block_tables, max_blocks, tok_seq, positions, H, G, window, scale, sink, bshift, nsplit, chunk, \
       softcap, sinkv, gate_ph, slopes)
-  if (D == 64) K8S_WT(64);
-  else if (D == 96) K8S_WT(96);
-  else K8S_WT(128);
+#define K8S_WT_D(NW)                \
+  do {                              \
+    if (D == 64) K8S_WT(64, NW);    \
+    else if (D == 96) K8S_WT(96, NW); \
+    else K8S_WT(128, NW);           \
+  } while (0)
+  if ((long)T * G <= 512) K8S_WT_D(8);      // (more fill the chip with 4 waves each)
+  else K8S_WT_D(4);
+#undef K8S_WT_D
 #undef K8S_WT
   if (nsplit > 1)
     window_merge_kernel<bf16_t><<<dim3(T, H), 64, 0, s>>>((bf16_t*)out, pacc, pml, (const bf16_t*)gate, ldg, positions, H, D,

@@ -918,8 +918,13 @@ def window_splits(T: int, G: int, window: int, P: int, max_pos: int, tile_rows: 
 
 
 def token_splits(T: int, G: int, keys: int) -> int:
-    """Key splits of the one-token kernel: about 512 workgroups, each with at least one 32-key tile for its four waves."""
-    return max(1, min(-(-512 // max(1, T * G)), -(-max(1, keys) // 128), 16))
+    """Key splits of the one-token kernel (workgroups of 8 waves up to 512 tokens x key heads): one for each 256 keys, a 32-key tile
+    a wave, up to 256 workgroups; none for up to 1024 keys of at least 128 tokens x key heads, where two tiles a wave cost less
+    than the merge's launch."""
+    n = max(1, T * G)
+    if n >= 128 and keys <= 1024:
+        return 1
+    return max(1, min(256 // n, -(-max(1, keys) // 256), 16))
 
 
 def prompt_splits(groups: int, keys: int) -> int:

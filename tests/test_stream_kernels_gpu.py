@@ -594,3 +594,21 @@ def test_wkv_outputs_by_16_tokens(dt, H, D, T, chunk, value):
     assert ((got - want)[head].abs() <= ulp * want[head].abs() + 2.0 ** -15 * (1 + want[head].abs())).all()
     if value is None:
         assert ((S[0].double().cpu() - end).abs() <= 2.0 ** -17 * (1 + end.abs().max())).all()
+
+
+@pytest.mark.parametrize("H,G,D,kw", [(16, 4, 128, dict(window=0)), (8, 4, 64, dict(window=150)), (6, 3, 96, dict(chunk=100))])
+@pytest.mark.parametrize("T,max_keys", [(1, 1024), (3, 4096), (32, 1024), (43, 0), (172, 1024)])
+def test_token_attention_by_waves(H, G, D, kw, T, max_keys):
+    """8 waves with and without key splits and 4 waves (more than 512 tokens x key heads), waves with two tiles, one and none."""
+    gen = torch.Generator().manual_seed(T)
+    bs, n, i32 = 16, 40, lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    ctx = [(1, 32, 33, 600, 257, 513)[i % 6] + (i // 6) % 7 for i in range(T)]
+    kc, vc, q = (torch.randn(*s, generator=gen).to(torch.bfloat16).to(DEV) for s in ((T * n * bs, G, D),) * 2 + ((T, H * D),))
+    bt = torch.randperm(T * n, generator=gen).int().view(T, n).to(DEV)
+    got = sm.window_attention(q, None, kc, vc, None, None, bt, i32(range(T)), i32([c - 1 for c in ctx]), H, kw.get("window", 0), 0,
+                              D ** -0.5, False, bs, max_keys=max_keys, chunk=kw.get("chunk", 0))
+    for t, c in enumerate(ctx):
+        rows = torch.arange(c, device=DEV)
+        rows = bt[t].long()[rows // bs] * bs + rows % bs
+        want = attend64(q[t:t + 1].view(1, H, D), kc[rows], vc[rows], c - 1, D ** -0.5, kw.get("window", 0), kw.get("chunk", 0)).view(-1)
+        assert ((got[t].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * want.abs().max()).all(), t
