@@ -108,8 +108,8 @@ def test_llama70b_shapes(name, N, K, epi, norm, with_res, fp8):
 @pytest.mark.parametrize("M", [3, 8, 16])
 @pytest.mark.parametrize("N,K", [(2048, 6144), (2049, 6144), (2048, 8192), (1024, 8192), (1030, 8192), (5, 6016), (40, 14336)])
 def test_k_groups_of_few_bands(M, N, K):
-    """k-groups taken because the 16-row bands leave CUs idle: either side of one band per CU and group, of the least depth and
-    of two steps a wave, with every epilogue."""
+    """Bands of 8 rows, and the k-groups that 9 - 16 rows take because 16-row bands leave CUs idle: either side of one band per CU
+    and group, of the least depth and of two steps a wave, with every epilogue."""
     for epi, res in ((ops.EPI_BF16, False), (ops.EPI_BF16, True), (ops.EPI_F32, False), (ops.EPI_SWIGLU, False)):
         _run(M, N, K, epi, False, False, res, seed=N + K)
 
