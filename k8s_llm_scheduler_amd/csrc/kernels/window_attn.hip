@@ -400,7 +400,8 @@ __global__ void window_attention_kernel(TA* __restrict__ out, float* __restrict_
 }
 
 // out[t][head] = sum_s e^(m_s - M) acc_s / sum_s e^(m_s - M) l_s over the key splits (at most 64), times sigmoid(gate) if
-// given.  One wave per (token, head): lane s weighs split s, then every lane sums its value dimensions.
+// given.  One wave per (token, head): lane s weighs split s, then every lane sums its value dimensions, 8 splits' loads in
+// flight (a load under the weight's branch waited for each split: 97 tokens, 16 heads of 128, 6 splits 7.4 -> 4.3 us).
 template <typename TA>
 __global__ __launch_bounds__(64) void window_merge_kernel(TA* __restrict__ out, const float* __restrict__ pacc,
                                                           const float* __restrict__ pml, const TA* __restrict__ gate,
@@ -421,12 +422,17 @@ __global__ __launch_bounds__(64) void window_merge_kernel(TA* __restrict__ out, 
   float wt = ms == -INFINITY ? 0.f : expf(ms - M);
   wt /= wave_sum(wt * ls);
   for (int d0 = 0; d0 < V; d0 += 64) {            // every lane stays in the loop: the shuffles read all of them
-    const int d = d0 + lane;
+    const int d = d0 + lane, dc = min(d, V - 1);
     float a = 0.f;
-#pragma unroll 4
-    for (int s = 0; s < nsplit; ++s) {
-      const float w = __shfl(wt, s, WAVE);
-      if (w != 0.f && d < V) a = fmaf(w, pacc[(rec0 + s) * V + d], a);     // (a split without keys left nothing)
+    for (int s0 = 0; s0 < nsplit; s0 += 8) {      // 8 splits' loads in flight, at clamped places
+      float x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) x[u] = pacc[(rec0 + min(s0 + u, nsplit - 1)) * V + dc];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float w = __shfl(wt, s0 + u, WAVE);       // (0 past the last split, and for a split without keys, which left nothing)
+        a = w != 0.f ? fmaf(w, x[u], a) : a;
+      }
     }
     if (d >= V) continue;
     if (gate != nullptr)
@@ -731,13 +737,13 @@ __global__ __launch_bounds__(256) void window_attention_mfma_kernel(
 //     With two blocks a wave (210 registers, one workgroup on a CU, each staged key used twice) a step is no shorter and the
 //     longest sequence of a batch decides: 16 query heads over 4 of 128, five prompts of 153 - 459 tokens and three single
 //     tokens behind 640 - 700 39.6 -> 27.8 us, 512 fresh tokens 23.9 -> 22.0, 1024 38.6 -> 32.1, 97 behind 1000 23.4 ->
-//     20.6, 2048 47.4 -> 47.2 (with the merge where there is one);
+//     20.6 (17.3 with the merge as it is now), 2048 47.4 -> 47.2 (with the merge where there is one);
 //   * two LDS buffers, one barrier per step: while a step is computed the next one is stored and the one after next is
 //     loaded into registers, its page numbers a step earlier still; a thread always moves one row's pieces;
 //   * scores in base 2 (scale and slopes carry log2 e), no mask arithmetic on slices that every column of the wave sees,
 //     accumulators rescaled only when some column's maximum moved, sums kept per lane until the end;
 //   * where the tiles are few (a short portion behind a long cached one), nsplit workgroups share a tile's steps and leave
-//     (max, sum, unnormalised sum) for window_merge_kernel: 97 tokens behind 1000 33.0 us in one piece, 20.6 us in 6 with the
+//     (max, sum, unnormalised sum) for window_merge_kernel: 97 tokens behind 1000 32.7 us in one piece, 17.3 us in 6 with the
 //     merge.  (A template flag: the arithmetic of the splits costs the whole walk 8%.)
 template <int DK, int DV, bool SPLIT>
 __global__ __launch_bounds__(512, 4) void window_prompt_kernel(

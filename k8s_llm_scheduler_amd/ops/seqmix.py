@@ -929,9 +929,9 @@ def token_splits(T: int, G: int, keys: int) -> int:
 
 def prompt_splits(groups: int, keys: int) -> int:
     """Key splits of the prompt kernel's ``groups`` workgroups: up to 256 of them (76 workgroups, 300 tokens behind 1000: 1 split
-    33.4 us, 3 25.7, 6 26.7, 8 34.2; 128, 512 fresh tokens: 1 20.0, 2 22.0, 4 23.2), of two 64-key steps at least, at most 6 (28
-    workgroups, 97 tokens behind 1000: 1 split 33.0 us, 2 25.1, 4 20.7, 6 20.6, 8 21.1, the more the merge reads).  How many
-    keys there are is only known on the device: 97 tokens behind none pay 3.6 us for the splits and their merge (9.8 in one piece)."""
+    33.3 us, 3 24.9, 6 23.9, 8 30.5; 128, 512 fresh tokens: 1 20.0, 2 22.6, 4 22.6), of two 64-key steps at least, at most 6 (28
+    workgroups, 97 tokens behind 1000: 1 split 32.7 us, 2 24.5, 4 18.7, 6 17.3, 8 16.6; 40, 150 behind 2000: 6 19.4, 8 21.5).  How
+    many keys there are is only known on the device: 97 tokens behind none pay 3 us for the splits and their merge (9.7 in one piece)."""
     return max(1, min(256 // max(1, groups), -(-max(1, keys) // 128), 6))
 
 
