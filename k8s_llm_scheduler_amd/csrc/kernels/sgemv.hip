@@ -1,5 +1,5 @@
 // K3/K8/K9/K11/K12 for SMALL decode batches (3..8 rows): out[M, N] = epi(x[M, K] . W[N, K]^T), the weights
-// streamed from HBM exactly once (VERDICT r3 item 5; the decode GEMV of gemv.hip stages x in LDS, 64-128 KiB per
+// streamed from HBM exactly once (the decode GEMV of gemv.hip stages x in LDS, 64-128 KiB per
 // workgroup at 4-8 rows, and re-stages it for every 8 output rows; mgemm's MFMA tiles waste 3/4 of a 16-row tile).
 //
 // Structure (one 256-thread workgroup = 4 waves; KW of them split K, 4 / KW row groups split the rows):
