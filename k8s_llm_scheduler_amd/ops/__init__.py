@@ -800,6 +800,18 @@ def mgemm(x: torch.Tensor, w, epi: int = EPI_BF16, cfg: Optional[int] = None,
     return out
 
 
+def _mgemm_act_plan(M: int, N: int, K: int, epi: int) -> Tuple[int, int]:
+    """mgemm's plan of a product with an activation.  Gated ones without a tuned plan go by the one-round rule, as the product of
+    their 2 N weight rows alone does: in one launch they are then faster than the product and the activation in two, which one
+    tile shape per row count is not.  us, that shape / two launches / the rule: 2 x 8192 x 2048, M = 64 25.3 / 21.5 / 18.8, 128
+    30.1 / 26.5 / 22.6; 2 x 14336 x 4096, M = 32 58 / 53 / 50, 128 95 / 63 / 59; 2 x 2048 x 14336, M = 64 54 / 32 / 30."""
+    if epi == EPI_SWIGLU and 16 < M <= 128 and _mg_table_row(M, N, K, epi, False) is None:
+        plan = _mgemm_one_round(M, N, K, epi, 256)
+        if plan is not None:
+            return plan
+    return mgemm_plan(M, N, K, epi, False)
+
+
 def linear_act_rows(x: torch.Tensor, w: torch.Tensor, pair: bool, kind: int, limit: float, alpha: float) -> Optional[torch.Tensor]:
     """act(x[M, K] @ w.T) of M <= 128 bf16 rows with the activation in the epilogue (``pair``: w = [gate; up]), on the kernel that
     :func:`linear` takes for M rows with the plan of its SwiGLU or plain form; None where that is another one (the library,
@@ -822,7 +834,7 @@ def linear_act_rows(x: torch.Tensor, w: torch.Tensor, pair: bool, kind: int, lim
         rc = native().sgemv_act(out.data_ptr(), part.data_ptr() if part is not None else 0, _chk(x, BF16, "x"), _chk(w, BF16, "w"),
                                 M, N, K, kind, limit, alpha, -1)
         return None if rc == -5 else out
-    cfg, grid = mgemm_plan(M, N, K, epi, False)
+    cfg, grid = _mgemm_act_plan(M, N, K, epi)
     if not mgemm_valid(cfg, M, N, K, epi, False, grid):
         return None
     nwg = mgemm_nwg(cfg, M, N, K, epi, False, grid)
