@@ -351,6 +351,14 @@ extern "C" int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles) {
   const auto rounds = [&](long rows, long cols) { return (double)((rows * cols * batch + 255) / 256); };
   const long gm = ntiles > 0 ? 2L * ntiles : (M + 31) / 32;
   const double r1 = rounds(gm, (N + 31) / 32), r2 = rounds(gm, (N + 63) / 64);
+  // Few rows in one round of gemm_f32_kernel's tiles wait for weights that none but their own workgroup reads, which the fitted
+  // parts leave out; the tiles of 64 columns keep fewer CUs loading.  us, k shared by the waves / gemm_f32_kernel, weights from
+  // memory: 1 row, 2048 x 2048 19.3 / 19.2, 4096 x 14336 135 / 120; 16 rows 22.8 / 19.6, 155 / 120; narrow ones, 128 x 2048, 1 row
+  // 17.7 / 18.5, 4 rows 19.0 / 18.6, 16 rows 21.8 / 19.0 (from the cache 13.5 / 16.7).  From 17 rows on two row tiles share them:
+  // 17 rows 18.5 / 19.6, 2048 x 8192 61.5 / 68.7, 4096 x 14336 124 / 120; 24 rows 20.0 / 19.7, 67.1 / 68.7, 129 / 121; 32 rows
+  // 20.8 / 19.8, 70.1 / 68.7.
+  const long cols = (long)N * batch;
+  if (ntiles == 0 && r1 == 1.0 && M <= 32 && (M <= 4 ? cols > 256 : M <= 16 || M > 24 || cols > 2048)) return 0;
   double best = 2.0 * r2 < 1.1 * r1 ? 0.365 * r2 + 0.03 : 0.16 * r1 + 0.1;
   int pick = 0;
   for (int fq = 8; fq >= 1; --fq) {

@@ -53,3 +53,24 @@ def test_gated_products_of_17_to_128_rows_take_the_plan_of_their_weight_rows(M, 
     if ops.mgemm_configs()[plain][4]:      # gate / up pairs
         assert (cfg, nwg) == (plain, ops.mgemm_nwg(plain, M, rows, K, ops.EPI_BF16, False, split))
     assert nwg <= 256 or ops.mgemm_configs()[cfg][1] >= 64       # small tiles only where one round holds them
+
+
+@pytest.mark.parametrize("N,K", [(64, 2048), (576, 2048), (2048, 2048), (8192, 2048), (4096, 4096), (1024, 8192), (4096, 14336)])
+def test_fp32_products_of_few_rows_keep_the_tiles_that_fill_the_chip(N, K):
+    """Up to 32 rows in one round of 32 x 32 tiles: those, but for up to 4 rows of very narrow weights and 17 - 24 of narrow ones,
+    where k is shared by the waves; with more rows or rounds one of the wider tiles."""
+    rule = ops.native().gemm_f32_rule
+    for M in (5, 8, 16, 25, 32):
+        assert rule(M, N, K, 1, 0) == 0, M
+    for M in (1, 2, 4):
+        assert rule(M, N, K, 1, 0) == (17 if N <= 256 else 0), M
+    for M in (17, 24):
+        assert rule(M, N, K, 1, 0) == (17 if N <= 2048 else 0), M
+    assert rule(33, N, K, 1, 0) > 0
+    for M in (1, 16, 32):
+        assert rule(M, 16384, 2048, 1, 0) > 0 and rule(M, 2048, 2048, 8, 0) > 0, M
+
+
+def test_fp32_products_of_other_depths_are_not_asked():
+    rule = ops.native().gemm_f32_rule
+    assert [rule(333, 2048, K, 1, 0) for K in (480, 500, 2056)] == [0, 0, 0]
