@@ -348,8 +348,19 @@ using namespace k8sllm;
 // shares of K / 8 leave the smaller error.
 extern "C" int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles) {
   if (K < 512 || K % 32 || M <= 0 || N <= 0) return 0;
+  // Listed tiles: most of the list is short of 64 rows or empty, and where its blocks meet on a CU is left to chance, so the parts
+  // below do not hold.  From 32 rows a group on (the list has one tile a group more than the rows fill) 32-row tiles, where the
+  // 64-row ones would be 280 and more, and from 1000 of 64 rows and more a group on those.  us, gemm_f32_kernel / 32 / 64 rows,
+  // weights from memory, groups x columns x k, rows a group: 8 x 4096 x 2048, 24 63 / 87 / 81, 40 100 / 86 / 80, 96 162 / 149 /
+  // 142; 8 x 2048 x 2048, 24 54 / 60 / 72, 40 61 / 58 / 71, 130 115 / 103 / 109; 16 x 1024 x 2048, 40 61 / 46 / 72, 500 352 / 303 / 307;
+  // 4 x 2048 x 2048 (144 tiles), 40 32 / 42 / 43.
+  if (ntiles > 0) {
+    const long groups = ntiles - (M + 63) / 64 > 1 ? ntiles - (M + 63) / 64 : 1;
+    const double t = (M / 64.0 + groups / 2.0) * ((N + 63) / 64);
+    return M < 32 * groups || t < 280.0 ? 0 : M >= 64 * groups && t >= 1000.0 ? 4 : 2;
+  }
   const auto rounds = [&](long rows, long cols) { return (double)((rows * cols * batch + 255) / 256); };
-  const long gm = ntiles > 0 ? 2L * ntiles : (M + 31) / 32;
+  const long gm = (M + 31) / 32;
   const double r1 = rounds(gm, (N + 31) / 32), r2 = rounds(gm, (N + 63) / 64);
   // Few rows in one round of gemm_f32_kernel's tiles wait for weights that none but their own workgroup reads, which the fitted
   // parts leave out; the tiles of 64 columns keep fewer CUs loading.  us, k shared by the waves / gemm_f32_kernel, weights from
@@ -358,12 +369,11 @@ extern "C" int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles) {
   // 17 rows 18.5 / 19.6, 2048 x 8192 61.5 / 68.7, 4096 x 14336 124 / 120; 24 rows 20.0 / 19.7, 67.1 / 68.7, 129 / 121; 32 rows
   // 20.8 / 19.8, 70.1 / 68.7.
   const long cols = (long)N * batch;
-  if (ntiles == 0 && r1 == 1.0 && M <= 32 && (M <= 4 ? cols > 256 : M <= 16 || M > 24 || cols > 2048)) return 0;
+  if (r1 == 1.0 && M <= 32 && (M <= 4 ? cols > 256 : M <= 16 || M > 24 || cols > 2048)) return 0;
   double best = 2.0 * r2 < 1.1 * r1 ? 0.365 * r2 + 0.03 : 0.16 * r1 + 0.1;
   int pick = 0;
   for (int fq = 8; fq >= 1; --fq) {
-    if (ntiles > 0 && 64 % (16 * fq)) continue;
-    const double r = rounds(ntiles > 0 ? 4L / fq * ntiles : (M + 16 * fq - 1) / (16 * fq), (N + 63) / 64);
+    const double r = rounds((M + 16 * fq - 1) / (16 * fq), (N + 63) / 64);
     const double t = r * (0.125 * fq + 0.04) + 0.1;
     if (t < best) {
       best = t;

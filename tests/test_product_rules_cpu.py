@@ -74,3 +74,18 @@ def test_fp32_products_of_few_rows_keep_the_tiles_that_fill_the_chip(N, K):
 def test_fp32_products_of_other_depths_are_not_asked():
     rule = ops.native().gemm_f32_rule
     assert [rule(333, 2048, K, 1, 0) for K in (480, 500, 2056)] == [0, 0, 0]
+
+
+@pytest.mark.parametrize("E,N,K", [(8, 2048, 2048), (8, 4096, 2048), (8, 7168, 4096), (16, 1024, 2048)])
+def test_fp32_products_of_listed_tiles_go_by_the_groups_rows(E, N, K):
+    """The list holds a tile a group more than the rows fill: groups of fewer than 32 rows keep the 32 x 32 tiles, as products do that
+    64-row tiles would not spread over the chip; the rest takes tiles of 32 rows, or of 64 where there are many."""
+    rule = ops.native().gemm_f32_rule
+    listed = lambda rows: (rows + 63) // 64 + E
+    for per in (1, 4, 16, 24, 31):
+        assert rule(per * E, N, K, 1, listed(per * E)) == 0, per
+    for per in (40, 63):
+        assert rule(per * E, N, K, 1, listed(per * E)) == 2, per
+    assert rule(500 * E, N, K, 1, listed(500 * E)) == 4 and rule(96 * E, 1024, K, 1, listed(96 * E)) in (0, 2)
+    assert rule(40 * E, 64, K, 1, listed(40 * E)) == 0 and rule(40 * 4, 2048, K, 1, 3 + 4) == 0
+    assert rule(500 * E, N, 480, 1, listed(500 * E)) == 0
