@@ -492,9 +492,11 @@ __global__ __launch_bounds__(256, 4) void wkv_chunk_out_kernel(TA* __restrict__ 
 
 // start[first chunk + c + 1] = dec[c] * start[c] + loc[c] along a sequence's chunks; start of chunk 0 is the slot's state
 // (or zero at position 0), copied here: the pass that reads it runs beside the one that replaces the slot's.  Workgroups (sequence, head, 256 state elements), a
-// thread per element with 16 chunks' records in flight: 2048 tokens, 32 heads of 64 x 64, 131 us with one workgroup per head
+// thread per element with PF chunks' records in flight: 2048 tokens, 32 heads of 64 x 64, 131 us with one workgroup per head
 // and a load waited for in every step, 14.8 us with 8 records in flight, 11 with 16 (33 MB read and written: 4 us at 8 TB/s each way, the
-// rest latency).
+// rest latency).  Loads past the last record repeat it and cost as much as the others: 8 x 100 tokens, 16 heads of 128 x 128, the
+// recurrence 196 us with 8, 214 with 16.
+template <int PF>
 __global__ __launch_bounds__(256) void wkv_prefix_kernel(float* __restrict__ cs_start, const float* __restrict__ cs_loc,
                                                          const float* __restrict__ cs_dec, const float* __restrict__ state,
                                                          const int* __restrict__ cu_q, const int* __restrict__ seq_slots,
@@ -512,7 +514,6 @@ __global__ __launch_bounds__(256) void wkv_prefix_kernel(float* __restrict__ cs_
   const int i = e / D;
   float S = positions[a] == 0 ? 0.f : state[((size_t)seq_slots[s] * H + hd) * D * D + e];
   cs_start[((size_t)first * H + hd) * D * D + e] = S;
-  constexpr int PF = 16;
   for (int c0 = 0; c0 < n; c0 += PF) {
     float dec[PF], loc[PF];
 #pragma unroll
@@ -1018,7 +1019,11 @@ extern "C" int k8s_wkv_scan(void* out, const void* r, const void* k, const void*
     wkv_chunk_state_kernel<bf16_t><<<dim3(chunks, H, nb * nb), 256, 0, s>>>((const bf16_t*)k, (const bf16_t*)v, ld, z,
                                                                             (const bf16_t*)w0, cu_q, positions, H, D,
                                                                             nseq, Lc, loc, dec);
-  wkv_prefix_kernel<<<dim3(nseq, H, (D * D + 255) / 256), 256, 0, s>>>(start, loc, dec, state, cu_q, seq_slots, positions, H, D, Lc);
+  const dim3 walks(nseq, H, (D * D + 255) / 256);
+  if ((long)T >= 8L * nseq * Lc || (long)nseq * H * D * D < 1L << 16)      // 8 chunks a sequence on average, or little traffic
+    wkv_prefix_kernel<16><<<walks, 256, 0, s>>>(start, loc, dec, state, cu_q, seq_slots, positions, H, D, Lc);
+  else
+    wkv_prefix_kernel<8><<<walks, 256, 0, s>>>(start, loc, dec, state, cu_q, seq_slots, positions, H, D, Lc);
 #define K8S_WKVO(TA)                                                                                                   \
   wkv_chunk_out_kernel<TA><<<dim3(chunks, H), 256, 0, s>>>((TA*)out, (const TA*)r, (const TA*)k, (const TA*)v,           \
                                                           (const TA*)g, ld, z, (const TA*)w0, (const TA*)u,             \

@@ -429,6 +429,27 @@ def test_recurrence_prefix_over_many_chunks():
             assert (s - outs[0][1]).abs().max() <= 1e-5 * outs[0][1].abs().max()
 
 
+@pytest.mark.parametrize("records", [1, 7, 8, 9, 15, 16, 17, 33])
+@pytest.mark.parametrize("empty", [0, 10])
+def test_recurrence_prefix_at_the_ends_of_its_groups(records, empty):
+    """Chunks whose records fill the prefix's groups, one more and one less, against 64 bits: 16 loads in flight, and 8
+    where the states are many (empty sequences beside the long one) and have few chunks on average."""
+    H, D, chunk = 2, 64, 16
+    T, n = chunk * (records + 1), 1 + empty
+    gen = torch.Generator().manual_seed(records)
+    r, k, v, g = (torch.randn(T, H, D, generator=gen) for _ in range(4))
+    z, w0, u, lnw = torch.randn(T, H, D, generator=gen) - 4.0, *(torch.randn(H, D, generator=gen) for _ in range(3))
+    S0 = torch.randn(n, H, D, D, generator=gen)
+    S, i32 = S0.to(DEV).clone(), lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    got = sm.wkv_scan(*(x.reshape(T, -1).to(DEV) for x in (r, k, v, g, z)), *(x.reshape(-1).to(DEV) for x in (w0, u, lnw)), S,
+                      i32([0] + [T] * n), i32(range(n)), i32(range(7, 7 + T)), H, D, 1e-6, chunk=chunk).view(T, H, D).double().cpu()
+    want, end = wkv64(*(x.double() for x in (r, k, v, g, z, w0, u, lnw, S0[0])), 1e-6)
+    # fp32 sums of at most 64 terms a product, the chunks' of at most their number: as the outputs by 16 tokens below
+    assert (got - want).abs().max() <= 2.0 ** -15 * (1 + want.abs().max())
+    assert (S[0].double().cpu() - end).abs().max() <= 2.0 ** -17 * (1 + end.abs().max())
+    assert torch.equal(S[1:].cpu(), S0[1:])
+
+
 @pytest.mark.parametrize("bs", [1, 16])
 @pytest.mark.parametrize("B", [1, 5, 255, 256, 300])
 def test_decode_meta(B, bs):
