@@ -1352,7 +1352,10 @@ extern "C" int k8s_window_token(void* out, float* pacc, float* pml, const void* 
     else if (D == 96) K8S_WT(96, NW); \
     else K8S_WT(128, NW);           \
   } while (0)
-  if ((long)T * G <= 512) K8S_WT_D(8);      // (more fill the chip with 4 waves each)
+  // 8 waves while every workgroup runs at once (two on a CU at 64 dimensions, one at more), else 4, of which two to four share a
+  // CU.  16 heads over 4 of 128, us, 8 / 4 waves: 64 tokens behind 40 6.2 / 6.6, behind 1000 29 / 36; 66 9.6 / 7.1, 39 / 40; 128 10.4 /
+  // 7.9, 53 / 50; of 64, 128 tokens 6.5 / 5.9, 28 / 31, 144 6.7 / 6.5, 35 / 34.  (T x G alone decides: the splits are made for it.)
+  if ((long)T * G <= (D == 64 ? 512 : 256)) K8S_WT_D(8);
   else K8S_WT_D(4);
 #undef K8S_WT_D
 #undef K8S_WT

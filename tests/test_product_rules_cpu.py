@@ -89,3 +89,16 @@ def test_fp32_products_of_listed_tiles_go_by_the_groups_rows(E, N, K):
     assert rule(500 * E, N, K, 1, listed(500 * E)) == 4 and rule(96 * E, 1024, K, 1, listed(96 * E)) in (0, 2)
     assert rule(40 * E, 64, K, 1, listed(40 * E)) == 0 and rule(40 * 4, 2048, K, 1, 3 + 4) == 0
     assert rule(500 * E, N, 480, 1, listed(500 * E)) == 0
+
+
+def test_key_splits_of_single_tokens():
+    """No splits where two tiles a wave cost less than the merge, nor where they would only add a round of workgroups; long contexts
+    of 65 - 512 tokens x key heads are split where that fills a round."""
+    s = sm.token_splits
+    assert [s(T, 4, 1024, 128) for T in (1, 8, 16, 31, 32, 64, 65, 80, 128, 200)] == [4, 4, 4, 2, 1, 1, 1, 1, 1, 1]
+    assert [s(T, 4, 4096, 128) for T in (1, 4, 16, 40, 48, 56, 64, 80, 128)] == [16, 16, 4, 3, 4, 1, 1, 3, 1]
+    assert [s(T, 4, 4096, 64) for T in (40, 48, 64, 128)] == [3, 2, 2, 1]
+    assert [s(T, 4, 4096, 96) for T in (64, 80, 96)] == [1, 2, 2] and [s(T, 4, 1024, 96) for T in (64, 80, 112)] == [1, 2, 1]
+    for D in (64, 96, 128):
+        assert all(1 <= s(T, G, keys, D) <= 16 for T in (1, 7, 33, 65, 300, 5000) for G in (1, 4, 8) for keys in (0, 1, 31, 2049, 8192))
+        assert s(300, 8, 40, D) == 1 and s(160, 4, 4096, D) == 1

@@ -633,3 +633,24 @@ def test_token_attention_by_waves(H, G, D, kw, T, max_keys):
         rows = bt[t].long()[rows // bs] * bs + rows % bs
         want = attend64(q[t:t + 1].view(1, H, D), kc[rows], vc[rows], c - 1, D ** -0.5, kw.get("window", 0), kw.get("chunk", 0)).view(-1)
         assert ((got[t].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * want.abs().max()).all(), t
+
+
+@pytest.mark.parametrize("H,G,D", [(16, 4, 128), (8, 4, 96), (4, 2, 64)])
+@pytest.mark.parametrize("groups,context", [(256, 40), (260, 90), (260, 1100), (320, 1100), (512, 33), (516, 65)])
+def test_token_attention_where_the_waves_change(H, G, D, groups, context):
+    """8 waves up to the workgroups that run at once, 4 beyond (256 tokens x key heads, at 64 dimensions 512), with and without key
+    splits: against 64 bits."""
+    T, bs, i32 = groups // G, 16, lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    n = -(-context // bs)
+    gen = torch.Generator().manual_seed(groups + context)
+    ctx = [1 + (i * 37) % context for i in range(T)]
+    kc, vc = (torch.randn(n * bs + 16 * bs, G, D, generator=gen).to(torch.bfloat16).to(DEV) for _ in range(2))
+    q = torch.randn(T, H * D, generator=gen).to(torch.bfloat16).to(DEV)
+    bt = torch.stack([(torch.arange(n) + i % 16) for i in range(T)]).int().to(DEV)      # (pages may be shared: nothing is written)
+    got = sm.window_attention(q, None, kc, vc, None, None, bt, i32(range(T)), i32([c - 1 for c in ctx]), H, 0, 0, D ** -0.5, False, bs,
+                              max_keys=max(context, 2100 if context > 1000 else 0))
+    for t, c in enumerate(ctx):
+        rows = torch.arange(c, device=DEV)
+        rows = bt[t].long()[rows // bs] * bs + rows % bs
+        want = attend64(q[t:t + 1].view(1, H, D), kc[rows], vc[rows], c - 1, D ** -0.5, 0, 0).view(-1)
+        assert ((got[t].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * want.abs().max()).all(), t
