@@ -922,16 +922,17 @@ _TOKEN_SLOTS = {64: (512, 1024), 96: (256, 768), 128: (256, 512)}
 
 
 @functools.lru_cache(maxsize=4096)
-def token_splits(T: int, G: int, keys: int, D: int) -> int:
+def token_splits(T: int, G: int, keys: int, D: int, known: bool = True) -> int:
     """Key splits of the one-token kernel, whose workgroups have 8 waves while all of them (T x G) run at once, else 4.  Few tokens: one
     split for each 256 keys, a 32-key tile a wave, up to 256 workgroups; none for up to 1024 keys of at least 128 tokens x key heads,
     where two tiles a wave cost less than the merge's launch, and none for more than 512.  Between, by the rounds that the workgroups take,
     each as long as its waves' tiles, and the merge (two tiles); us, 1 / 2 / 3 / 4 splits: 40 tokens of 4 key heads of 128
     behind 4000 88 / 84 / 72 / 76, 56 of them 94 / 97 / 98 / 99, 80 142 / 150 / 124 / 130; of 64 dimensions, 40 57 / 47 / 39 / 46; of 96, 80 132 /
-    100 / 114 / 102, behind 1000 36 / 32 / 36 / 35."""
+    100 / 114 / 102, behind 1000 36 / 32 / 36 / 35.  Not where ``keys`` is only what the block tables could hold (``known`` false: the
+    tokens of a prompt whose query groups make no tile, 97 fresh ones 10.3 / 14.7 with three splits)."""
     n = max(1, T * G)
-    if n <= 64 or n > 512 or (n <= 256 and keys <= 1024):
-        return 1 if n >= 128 else max(1, min(256 // n, -(-max(1, keys) // 256), 16))
+    if n <= 64 or n > 512 or not known or (n <= 256 and keys <= 1024):
+        return 1 if n >= 128 and keys <= 1024 else max(1, min(256 // n, -(-max(1, keys) // 256), 16))
     wide, narrow = _TOKEN_SLOTS[D]
     waves, slots = (8, wide) if n <= wide else (4, narrow)
     tiles = -(-max(1, keys) // 32)
@@ -1014,7 +1015,7 @@ def window_attention(q: torch.Tensor, gate: Optional[torch.Tensor], kcache: torc
     max_pos = max_keys or block_tables.shape[1] * block_size
     if (WINDOW_MFMA and dt == BF16 and P <= 0 and nat.window_token_ok(H, G, D, V, block_size) and q.stride(0) % 8 == 0
             and q.data_ptr() % 16 == 0):
-        ns = token_splits(T, G, min(max_pos, chunk or window or max_pos), D)
+        ns = token_splits(T, G, min(max_pos, chunk or window or max_pos), D, max_keys > 0)
         pacc = pml = None
         if ns > 1:
             pacc = torch.empty(T * H * ns * V, dtype=F32, device=q.device)

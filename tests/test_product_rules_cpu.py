@@ -102,3 +102,4 @@ def test_key_splits_of_single_tokens():
     for D in (64, 96, 128):
         assert all(1 <= s(T, G, keys, D) <= 16 for T in (1, 7, 33, 65, 300, 5000) for G in (1, 4, 8) for keys in (0, 1, 31, 2049, 8192))
         assert s(300, 8, 40, D) == 1 and s(160, 4, 4096, D) == 1
+        assert [s(T, 4, 8192, D, False) for T in (8, 32, 40, 97, 400)] == [8, 2, 1, 1, 1]      # how many keys there are is not known
