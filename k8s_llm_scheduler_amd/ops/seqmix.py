@@ -944,11 +944,14 @@ def token_splits(T: int, G: int, keys: int, D: int, known: bool = True) -> int:
 
 
 def prompt_splits(groups: int, keys: int) -> int:
-    """Key splits of the prompt kernel's ``groups`` workgroups: up to 256 of them (76 workgroups, 300 tokens behind 1000: 1 split
-    33.3 us, 3 24.9, 6 23.9, 8 30.5; 128, 512 fresh tokens: 1 20.0, 2 22.6, 4 22.6), of two 64-key steps at least, at most 6 (28
-    workgroups, 97 tokens behind 1000: 1 split 32.7 us, 2 24.5, 4 18.7, 6 17.3, 8 16.6; 40, 150 behind 2000: 6 19.4, 8 21.5).  How
-    many keys there are is only known on the device: 97 tokens behind none pay 3 us for the splits and their merge (9.7 in one piece)."""
-    return max(1, min(256 // max(1, groups), -(-max(1, keys) // 128), 6))
+    """Key splits of the prompt kernel's ``groups`` workgroups: up to 256 of them (128, 512 fresh tokens: 1 20.0, 2 22.6, 4 22.6), of
+    two 64-key steps at least, at most 6 (28 workgroups, 97 tokens behind 1000: 1 split 32.7 us, 2 24.5, 4 18.7, 6 17.3, 8 16.6; 52, 200
+    tokens: 4 22.2, 6 25.4).  65 - 170 workgroups that may see more than 2048 keys: up to 512, as many as run at once (76, 300 tokens
+    behind 4000: 1 split 107, 3 51.3, 6 42.9; behind 1000 40.1, 27.5, 26.9; 152: 1 108, 3 69.6, behind 1000 42.4, 36.7; 128, 500 behind
+    1000: 1 44.1, 2 35.6, 4 33.6).  How many keys there are is only known on the device: 97 tokens behind none pay 3 us for the
+    splits and their merge (9.7 in one piece)."""
+    most = 512 if keys > 2048 and 64 < groups <= 170 else 256
+    return max(1, min(most // max(1, groups), -(-max(1, keys) // 128), 6))
 
 
 def window_attention(q: torch.Tensor, gate: Optional[torch.Tensor], kcache: torch.Tensor, vcache: torch.Tensor,

@@ -103,3 +103,12 @@ def test_key_splits_of_single_tokens():
         assert all(1 <= s(T, G, keys, D) <= 16 for T in (1, 7, 33, 65, 300, 5000) for G in (1, 4, 8) for keys in (0, 1, 31, 2049, 8192))
         assert s(300, 8, 40, D) == 1 and s(160, 4, 4096, D) == 1
         assert [s(T, 4, 8192, D, False) for T in (8, 32, 40, 97, 400)] == [8, 2, 1, 1, 1]      # how many keys there are is not known
+
+
+def test_key_splits_of_prompts():
+    """Windows keep to 256 workgroups; where more than 2048 keys may be visible, 65 - 170 workgroups are split up to the 512 that run
+    at once."""
+    s = sm.prompt_splits
+    assert [s(g, 1040) for g in (1, 28, 52, 76, 128, 129, 512)] == [6, 6, 4, 3, 2, 1, 1]
+    assert [s(g, 8192) for g in (28, 52, 64, 65, 76, 100, 128, 152, 170, 171, 256, 512)] == [6, 4, 4, 6, 6, 5, 4, 3, 3, 1, 1, 1]
+    assert s(76, 100) == 1 and s(3, 300) == 3
