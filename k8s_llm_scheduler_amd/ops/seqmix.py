@@ -351,27 +351,11 @@ def _grouped_big(a: torch.Tensor, w: torch.Tensor, seg: Optional[torch.Tensor], 
             and w.data_ptr() % 16 == 0 and w.shape[1] * K * 2 < 1 << 32 and a.shape[0] * a.stride(0) * 2 < 1 << 32)
 
 
-@functools.lru_cache(maxsize=4096)
-def _grouped_cfg(rows: int, E: int, N: int, K: int, pair: bool, even: bool = False) -> int:
-    """The better of the 128-token tiles of the grouped big-tile product: 256 (1) or 128 (3) weight rows by the time its rounds
-    of tiles over the CUs take, groups of the same size (``even``) or of about equal size drawn at random."""
-    r = rows / E
-    if even or E == 1:
-        tiles = E * -(-rows // E // 128)
-    else:       # a group's tiles beyond k: the chance that it has more than 128 k rows, 1 up to six deviations below the mean
-        sure = max(0, int((r - 6.0 * math.sqrt(max(r, 1.0))) // 128))
-        tiles = E * (1 + sure + sum(0.5 + 0.5 * math.erf((r - 128 * k) / math.sqrt(2.0 * max(r, 1.0)))
-                                    for k in range(sure + 1, int(r / 128) + 2)))
-    n, kt = (2 * N if pair else N), K / 64
-    big = 10.0 + math.ceil(tiles * -(-n // 256) / 256) * (kt + (12.0 if pair else 0.0))
-    small = 20.0 + math.ceil(tiles * -(-n // 128) / 256) * 0.56 * kt
-    return 1 if big < small else 3
-
-
 # Time of a grouped product in us, configuration -> (fixed, per round of tiles over the CUs and 64-deep k-step, per round, per
 # k-step, per MB of weights, per MB of output, per round and 65536 outputs of a gated activation).  Fitted to 8 products of 1 -
-# 16 groups, 512 x 4096 .. 2 x 3584 x 4096, 2 - 2048 rows per group, weights cold: rms error 5 - 11 % per configuration, the
-# pick within 2 % of the best configuration on average, 41 % at most.  _GROUP_TILE: weight rows and tokens of a tile.
+# 16 groups, 512 x 4096 .. 2 x 3584 x 4096, 2 - 2048 rows per group, weights cold: rms error 5 - 11 % per configuration.  Over 8
+# other products (4 - 16 groups drawn at random, 1024 x 2048 .. 2 x 3584 x 4096, 18 row counts of 128 - 4096) the pick is within 1.5 % of the best configuration on
+# average, 35 % at most.  _GROUP_TILE: weight rows and tokens of a tile.
 _GROUP_TILE = {1: (256, 128), 2: (128, 256), 3: (128, 128), 4: (256, 256), 5: (128, 64), 6: (64, 64)}
 _GROUP_COST = {1: (0.0, 0.524, 4.92, 0.0, 0.11, 0.424, 6.72), 2: (0.0, 0.542, 4.91, 0.0, 0.0696, 0.486, 9.86),
                3: (3.28, 0.379, 0.0, 0.0254, 0.0878, 0.27, 11.6), 4: (0.0, 0.864, 8.67, 0.0, 0.0913, 0.323, 8.6),
@@ -379,21 +363,22 @@ _GROUP_COST = {1: (0.0, 0.524, 4.92, 0.0, 0.11, 0.424, 6.72), 2: (0.0, 0.542, 4.
 
 
 @functools.lru_cache(maxsize=4096)
-def _grouped_tile(base: int, rows: int, E: int, N: int, K: int, pair: bool, even: bool = False) -> int:
-    """Configuration of the grouped big-tile product: ``base`` (:func:`_grouped_cfg`'s), or what is cheaper by _GROUP_COST of
-    the tiles of 256 and 64 tokens and of 128 x 256.  Groups as there."""
+def _grouped_tile(rows: int, E: int, N: int, K: int, pair: bool, even: bool = False) -> int:
+    """Configuration of the grouped big-tile product: the cheapest of them all by _GROUP_COST, for groups of the same size (``even``)
+    or of about equal size drawn at random, whose tiles are expected ones: up to 5 that would begin another round most often are
+    not there (1700 rows of 16 experts, 2 x 2048 x 4096: 260.5 tiles expected, 136 us in one round, 152 the next best)."""
     r, n, kt, best = rows / E, (2 * N if pair else N), K / 64, None
-    for cfg in (base, 2, 4, 5, 6):
-        t0, tile, rnd, step, wmb, omb, act_us = _GROUP_COST[cfg]
+    for cfg, (t0, tile, rnd, step, wmb, omb, act_us) in _GROUP_COST.items():
         bp, bq = _GROUP_TILE[cfg]
         if even or E == 1:
-            tiles = E * -(-rows // E // bq)
+            tiles, spare = E * -(-rows // E // bq), 1e-9
         else:   # a group's tiles beyond k: the chance that it has more than bq k rows, 1 up to six deviations below the mean
             d = 6.0 * math.sqrt(max(r, 1.0))
             sure = max(0, int((r - d) // bq))
             tiles = E * (1 + sure + sum(0.5 + 0.5 * math.erf((r - bq * k) / math.sqrt(2.0 * max(r, 1.0)))
                                         for k in range(sure + 1, int((r + d) / bq) + 2)))
-        rounds = math.ceil(tiles * -(-n // bp) / 256 - 1e-9)
+            spare = 0.02
+        rounds = max(1, math.ceil(tiles * -(-n // bp) / 256 - spare))
         us = t0 + rounds * (tile * kt + rnd + (act_us * bp * bq / 65536 if pair else 0.0)) + step * kt + \
             wmb * E * n * K * 2e-6 + omb * rows * N * 2e-6
         if best is None or us < best[0]:
@@ -404,9 +389,8 @@ def _grouped_tile(base: int, rows: int, E: int, N: int, K: int, pair: bool, even
 def _pgemm4_grouped(a, w, a_rows, rows: int, seg, N: int, kind: int = -1, limit: float = 0.0, alpha: float = 1.0):
     E, _, K = w.shape
     out = torch.empty(rows, N, dtype=BF16, device=a.device)
-    shape = (rows, E, N, K, kind >= 0, seg is None)
     _native().pgemm4_grouped(out.data_ptr(), a.data_ptr(), w.data_ptr(), a.shape[0], rows, N, K, E, _p(seg, I32, "seg"),
-                             _p(a_rows, I32, "a_rows"), a.stride(0), _grouped_tile(_grouped_cfg(*shape), *shape), 4, kind,
+                             _p(a_rows, I32, "a_rows"), a.stride(0), _grouped_tile(rows, E, N, K, kind >= 0, seg is None), 4, kind,
                              float(limit), float(alpha), -1)
     return out
 

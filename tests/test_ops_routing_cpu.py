@@ -395,9 +395,22 @@ def test_plans_are_worked_out_once_and_in_bounded_time(monkeypatch):
                                 (194, 8, 2048, 2048, False), (90000, 8, 128, 64, False)):
         r = rows / E
         terms.clear()
-        got = sm._grouped_cfg.__wrapped__(rows, E, N, K, pair)
-        assert len(terms) <= 2 + 12.0 * r ** 0.5 / 128
-        tiles = E + E * sum(0.5 + 0.5 * erf((r - 128 * k) / (2.0 * r) ** 0.5) for k in range(1, int(r / 128) + 2))
-        per, kt = (2 if pair else 1) * N, K / 64
-        big = 10.0 + math.ceil(tiles * -(-per // 256) / 256) * (kt + (12.0 if pair else 0.0))
-        assert got == (1 if big < 20.0 + math.ceil(tiles * -(-per // 128) / 256) * 0.56 * kt else 3)
+        got = sm._grouped_tile.__wrapped__(rows, E, N, K, pair)
+        assert len(terms) <= sum(2 + 12.0 * r ** 0.5 / bq for _, bq in sm._GROUP_TILE.values())
+        cost = {}
+        for cfg, (bp, bq) in sm._GROUP_TILE.items():
+            start, tile, per_round, step, wmb, omb, act = sm._GROUP_COST[cfg]
+            more = sum(0.5 + 0.5 * erf((r - bq * k) / (2.0 * r) ** 0.5) for k in range(1, int((r + 6.0 * r ** 0.5) / bq) + 2))
+            tiles, spare = (E + E * more, 0.02) if E > 1 else (-(-rows // bq), 0.0)
+            per, kt = (2 if pair else 1) * N, K / 64
+            rounds = max(1, math.ceil(tiles * -(-per // bp) / 256 - spare))
+            cost[cfg] = start + rounds * (tile * kt + per_round + (act * bp * bq / 65536 if pair else 0.0)) + step * kt + \
+                2e-6 * (wmb * E * per * K + omb * rows * N)
+        assert got == min(cost, key=cost.get)
+
+
+@pytest.mark.parametrize("rows,E,N,K,pair,want", [(600, 8, 2048, 2048, True, 3), (1700, 8, 2048, 2048, False, 3), (1700, 16, 2048, 4096, True, 1),
+                                                  (160, 8, 2048, 2048, False, 6)])
+def test_grouped_products_take_the_cheapest_tile_of_all(rows, E, N, K, pair, want):
+    """Where one tile was left out of the choice, or a few expected tiles past a whole round priced the better one out of it."""
+    assert sm._grouped_tile(rows, E, N, K, pair) == want

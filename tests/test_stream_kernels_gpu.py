@@ -301,11 +301,35 @@ def act64(z, kind, limit, alpha):
             sm.ACT_RELU2: lambda v: v.clamp(min=0) ** 2, sm.ACT_SOFTCAP: lambda v: limit * torch.tanh(v / limit)}[kind](z)
 
 
-@pytest.mark.parametrize("sizes", [(1, 127, 0, 128, 129), (40, 40, 40), (0, 0, 300), (257,), tuple([17] * 63 + [1])])
+@pytest.fixture
+def grouped_tile(monkeypatch):
+    """Forces the tile configuration of grouped products: set ``cfg``; ``ran`` lists those that were launched."""
+    class Force:
+        cfg, ran = None, []
+
+    nat, force = ops.native(), Force()
+    force.ran = []
+
+    class Spy:
+        def __getattr__(self, name):
+            if name != "pgemm4_grouped":
+                return getattr(nat, name)
+            return lambda *args: (force.ran.append(args[11]), nat.pgemm4_grouped(*args))[1]
+
+    monkeypatch.setattr(ops, "native", Spy)
+    monkeypatch.setattr(sm, "_grouped_tile", lambda *args: force.cfg)
+    return force
+
+
+GROUPED_TILES = [1, 2, 3, 4, 5, 6]      # 256 x 128, 128 x 256, 128 x 128, 256 x 256, 128 x 64, 64 x 64 (weight rows x tokens)
+
+
+@pytest.mark.parametrize("sizes", [(1, 127, 0, 128, 129), (40, 40, 40), (0, 0, 300), (257,), tuple([17] * 63 + [1]), (63, 65, 0, 64, 255, 256)])
 @pytest.mark.parametrize("N,K", [(128, 64), (392, 192), (1024, 256)])
 @pytest.mark.parametrize("kind", [None] + KINDS)
-def test_grouped_big_tiles(sizes, N, K, kind):
-    """Groups at the edges of the 128-token tile, empty ones, more than fit a wave; gathered rows with a row stride."""
+def test_grouped_big_tiles(sizes, N, K, kind, grouped_tile):
+    """Every tile with groups at the edges of its 64, 128 or 256 tokens, empty ones, more than fit a wave; gathered rows with a row
+    stride."""
     g = torch.Generator().manual_seed(sum(sizes) + N + K)
     E, P = len(sizes), sum(sizes)
     seg = torch.tensor((0,) + sizes).cumsum(0).to(torch.int32)
@@ -317,18 +341,33 @@ def test_grouped_big_tiles(sizes, N, K, kind):
     tiles = torch.full((1, 3), -1, dtype=torch.int32, device=DEV)      # the big tiles come from seg
     assert sm._grouped_big(x, w, seg.to(DEV), P, N)
     kw = dict(a_rows=rows, tiles=tiles, rows=P, seg=seg.to(DEV))
-    for cfg in (1, 3):
-        sm_cfg, sm._grouped_cfg = sm._grouped_cfg, lambda *a: cfg
-        try:
-            got = sm.gemm(x, w, **kw) if kind is None else sm.gemm_act(x, w, kind, 1.5, 1.702, **kw)
-        finally:
-            sm._grouped_cfg = sm_cfg
-        for e in range(E):
-            r = slice(int(seg[e]), int(seg[e + 1]))
-            z = x[rows[r].long()].double() @ w[e].double().T
-            want = z if kind is None else act64(z, kind, 1.5, 1.702)
-            if want.numel():      # one rounding to bf16, and the fp32 sums'
-                assert ((got[r].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all(), (cfg, e)
+    want = []
+    for e in range(E):
+        z = x[rows[int(seg[e]):int(seg[e + 1])].long()].double() @ w[e].double().T
+        want.append(z if kind is None else act64(z, kind, 1.5, 1.702))
+    want = torch.cat(want)
+    for cfg in GROUPED_TILES:
+        grouped_tile.cfg = cfg
+        got = sm.gemm(x, w, **kw) if kind is None else sm.gemm_act(x, w, kind, 1.5, 1.702, **kw)
+        # one rounding to bf16, and the fp32 sums'
+        assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all(), cfg
+    assert grouped_tile.ran == GROUPED_TILES
+
+
+@pytest.mark.parametrize("M", [1, 63, 65, 128, 257])
+@pytest.mark.parametrize("N,K", [(128, 64), (392, 192)])
+def test_several_inputs_on_every_big_tile(M, N, K, grouped_tile):
+    """Groups of one size, without a list of their offsets: rows at the edges of every tile."""
+    g = torch.Generator().manual_seed(M + N)
+    a, w = (torch.randn(3, n, K, generator=g).to(torch.bfloat16).to(DEV) for n in (M, N))
+    for cfg in GROUPED_TILES:
+        grouped_tile.cfg = cfg
+        got = sm._pgemm4_grouped(a.view(3 * M, K), w, None, 3 * M, None, N).view(3, M, N)
+        for i in range(3):
+            exact = a[i].double() @ w[i].double().T
+            bound = sum_bound(a[i].cpu(), w[i].cpu()).to(DEV) + 2.0 ** -8 * exact.abs()
+            assert ((got[i].double() - exact).abs() <= bound).all(), (cfg, i)
+    assert grouped_tile.ran == GROUPED_TILES
 
 
 @pytest.mark.parametrize("M,N,K", [(129, 1024, 512), (200, 520, 1024), (1031, 2048, 256), (2048, 2064, 320)])
