@@ -453,9 +453,8 @@ def gemm_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, al
 def linear_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, alpha: float = 1.0, *,
                bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """act(linear(a, w), kind, bias=bias): in the product's epilogue where its plan is an unsplit big-tile one, which saves a
-    pass over the product (2048 x 2 x 8192, gated: 22 us; 2048 x 8192 elementwise: 15 us) and its rounding, and up to 128 rows
-    (a captured step of 1 row 477 -> 456 us, of 8 rows 655 -> 637, of 32 rows 1028 -> 1016).  Deep products of
-    few big tiles keep the launch of their own, as when they ran in k slices: the pass that it saves there is 1 - 2 us."""
+    pass over the product (2048 x 2 x 8192, gated: 22 us; 2048 x 8192 elementwise: 15 us; 200 x 1040 x 1024, few tiles: 9.8 -> 7.3)
+    and its rounding, and up to 128 rows (a captured step of 1 row 477 -> 456 us, of 8 rows 655 -> 637, of 32 rows 1028 -> 1016)."""
     pair = kind in (ACT_GELU_TANH, ACT_SWISH_CLAMP, ACT_RELU)
     if (pair or kind == ACT_RELU2) and FAST_GEMM and _gpu(a, w, bias) and _route_fast(a, w, BF16) and a.dtype == BF16 and (not pair or w.shape[0] % 8 == 0):
         M, K = a.shape
@@ -464,8 +463,7 @@ def linear_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, 
             if out is not None:
                 return out
         kern, plan = _ops.gemm_route(M, w.shape[0], K, _ops.EPI_BF16, False) if M >= 129 else ("", None)
-        if kern == "pgemm4" and plan[1] == 1 and (K < 1024 or _ops.pgemm4_tiles(plan[0], M, w.shape[0], _ops.EPI_BF16) >= 96) and \
-                a.data_ptr() % 16 == 0 and \
+        if kern == "pgemm4" and plan[1] == 1 and a.data_ptr() % 16 == 0 and \
                 (bias is None or (pair and bias.dtype == BF16 and bias.numel() == w.shape[0] and bias.data_ptr() % 8 == 0)):
             N = w.shape[0] // 2 if pair else w.shape[0]
             out = torch.empty(M, N, dtype=BF16, device=a.device)

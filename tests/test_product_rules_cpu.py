@@ -112,3 +112,13 @@ def test_key_splits_of_prompts():
     assert [s(g, 1040) for g in (1, 28, 52, 76, 128, 129, 512)] == [6, 6, 4, 3, 2, 1, 1]
     assert [s(g, 8192) for g in (28, 52, 64, 65, 76, 100, 128, 152, 170, 171, 256, 512)] == [6, 4, 4, 6, 6, 5, 4, 3, 3, 1, 1, 1]
     assert s(76, 100) == 1 and s(3, 300) == 3
+
+
+@pytest.mark.parametrize("M,N,K,kind", [(200, 1040, 1024, sm.ACT_RELU), (129, 1040, 1024, sm.ACT_RELU2), (333, 2048, 2048, sm.ACT_GELU_TANH),
+                                        (160, 1024, 4096, sm.ACT_GELU_TANH), (200, 1536, 4096, sm.ACT_RELU2)])
+def test_activations_join_every_unsplit_product_of_big_tiles(M, N, K, kind, launches):
+    """However few its tiles; products whose k is split get the activation as a launch of its own."""
+    kern, plan = ops.gemm_route(M, N, K, ops.EPI_BF16, False)
+    assert kern == "pgemm4"
+    sm.linear_act(torch.zeros(M, K, dtype=BF16), torch.zeros(N, K, dtype=BF16), kind)
+    assert launches.names() == (["pgemm4_act"] if plan[1] == 1 else ["pgemm4", "act"]) and (plan[1] > 1) == (K == 4096)

@@ -370,13 +370,13 @@ def test_several_inputs_on_every_big_tile(M, N, K, grouped_tile):
     assert grouped_tile.ran == GROUPED_TILES
 
 
-@pytest.mark.parametrize("M,N,K", [(129, 1024, 512), (200, 520, 1024), (1031, 2048, 256), (2048, 2064, 320)])
+@pytest.mark.parametrize("M,N,K", [(129, 1024, 512), (200, 520, 1024), (1031, 2048, 256), (2048, 2064, 320), (160, 512, 4096)])
 @pytest.mark.parametrize("kind", KINDS + ELEMENTWISE)
 @pytest.mark.parametrize("bias", [False, True])
 def test_linear_act(M, N, K, kind, bias, entries):
     """The activation in the epilogue, every tile configuration's edges, against 64 bits: one rounding.  Two launches and two
-    roundings only for 200 x 1040, which runs in k slices, and for the elementwise kinds without an epilogue of the big tiles
-    (200 x 520 is few tiles, which have one for all but the cap)."""
+    roundings only where the product's plan splits k (160 rows of depth 4096), and for the elementwise kinds without an epilogue of the
+    big tiles (200 x 520 is few tiles, which have one for all but the cap)."""
     if bias and kind not in KINDS:
         pytest.skip("elementwise kinds take no bias")
     g = torch.Generator().manual_seed(M + N + K + kind)
@@ -394,7 +394,9 @@ def test_linear_act(M, N, K, kind, bias, entries):
     entries.clear()
     got = sm.linear_act(x, w, kind, 1.5, 1.702, bias=b)
     few = M == 200 and kind not in KINDS + [sm.ACT_SOFTCAP]
-    fused = few or (M != 200 and kind in KINDS + [sm.ACT_RELU2])
+    kern, plan = ops.gemm_route(M, w.shape[0], K, ops.EPI_BF16, False)
+    assert kern == "pgemm4" and (plan[1] > 1) == (K == 4096)
+    fused = few or (plan[1] == 1 and kind in KINDS + [sm.ACT_RELU2])
     assert ("act" in entries) != fused and ("gemm_few_act" if few else "pgemm4_act" if fused else "act") in entries
     if fused:
         assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all()
