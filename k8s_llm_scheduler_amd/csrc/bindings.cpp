@@ -157,6 +157,7 @@ int k8s_gemm_few_act(void* C, const void* A, const void* W, int M, int N, int K,
                      const int* tiles, int ntiles, int kind, float limit, float alpha, hipStream_t s);
 int k8s_gemv_act(void* out, void* partial, const void* x, const void* W, int M, int N_out, int K, int kind, float limit, float alpha,
                  hipStream_t stream);
+int k8s_gemv_act_plan(int M, int N_out, int K, int pair, int* ks, int* splits, int* wgs, int* per);
 int k8s_sgemv_act(void* out, void* partial, const void* x, const void* W, int M, int N, int K, int kind, float limit, float alpha,
                   hipStream_t stream);
 int k8s_mgemm_act(void* out, float* ws, unsigned* tickets, const void* x, const void* W, int M, int N_out, int K, int cfg, int nwg,
@@ -356,7 +357,14 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
   m.def("gemv_set_wide", [](int on) { return k8s_gemv_set_wide(on); });
   m.def("gemv_act", [](uintptr_t out, uintptr_t partial, uintptr_t x, uintptr_t W, int M, int N, int K, int kind, float limit,
                        float alpha, int64_t s) {
-    check(k8s_gemv_act(P(out), P(partial), P(x), P(W), M, N, K, kind, limit, alpha, S(s)), "gemv_act");
+    const int rc = k8s_gemv_act(P(out), P(partial), P(x), P(W), M, N, K, kind, limit, alpha, S(s));
+    if (rc != -5) check(rc, "gemv_act");
+    return rc;
+  });
+  m.def("gemv_act_plan", [](int M, int N, int K, int pair) {      // (splits, workgroups, row sets a wave), or None: a form that gemv_act lacks
+    int ks = 0, splits = 0, wgs = 0, per = 0;
+    const int rc = k8s_gemv_act_plan(M, N, K, pair, &ks, &splits, &wgs, &per);
+    return rc == 0 ? py::object(py::make_tuple(splits, wgs, per)) : py::object(py::none());
   });
   m.def("sgemv_act", [](uintptr_t out, uintptr_t partial, uintptr_t x, uintptr_t W, int M, int N, int K, int kind, float limit,
                         float alpha, int64_t s) {

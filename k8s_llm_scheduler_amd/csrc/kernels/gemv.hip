@@ -92,6 +92,45 @@ extern "C" int k8s_gemv_set_loop(int wg_per_cu) {   // returns the previous sett
   return old;
 }
 
+// KW: waves per row set (K8S_GEMV_KW = 2 / 4 splits a row set's K over that many waves).  One wave per row
+// set is the default: the two-wave split the small-N projections (TP = 8 QKV, LM head) used to take measured
+// slower end to end (TP = 8 shapes 4.28 -> 4.26 ms/token with one wave, 8B and TP = 1 unchanged,
+// profiles/gemv_kw_ab.txt).
+static int gemv_kw() {
+  static const int env = [] { const char* e = getenv("K8S_GEMV_KW"); return e ? atoi(e) : 0; }();
+  return (env == 2 || env == 4) ? env : 1;
+}
+// Workgroups per CU of the row-set loop over a grid of `wgs` one-row-set workgroups; 0: no loop.
+static int gemv_loop_wg(bool fp8, int M, int N_out, int K, int epi, int mode, int splits, int wgs) {
+  const bool swiglu_loop = epi == EPI_SWIGLU && wgs <= g_gemv_loop_swiglu_max;
+  // the loop only on matrices of >= 64 Mi weights (the 70B's at TP = 1, gate/up at TP = 4): on the smaller ones
+  // (Llama-3-8B, fp8 at TP = 4) it measured slower
+  const bool big = (long long)(epi == EPI_SWIGLU ? 2 * N_out : N_out) * K >= ((long long)g_gemv_loop_min_mi << 20);
+  const bool plain_loop = epi == EPI_BF16 && big;
+  const int wg = g_gemv_loop >= 0 ? g_gemv_loop
+                                  : (fp8 ? (big ? 2 : 0) : (plain_loop ? g_gemv_loop_bf16 : (swiglu_loop ? 2 : 0)));
+  return wg > 0 && splits == 1 && gemv_kw() == 1 && mode != 1 && M <= 2 && wgs > 256 * wg ? wg : 0;
+}
+// wide: 8-wave workgroups for the looped plain bf16-epilogue projections whose x slice takes >= 32 KiB of LDS (the
+// down projection, K = 28672: 56 KiB): LDS, not waves, bounds those at 2 workgroups per CU, so twice the waves
+// per workgroup put twice the weight loads in flight per CU (K8S_GEMV_WIDE = 0 turns it off)
+static bool gemv_is_wide(int M, int K, int epi, int mode) {
+  return g_gemv_wide && mode == 0 && epi == EPI_BF16 && (long long)M * K * 2 >= 32768;
+}
+
+// The launch of gemv_act.hip's products, the one that k8s_gemv makes of epi 2 (gated) or 0 (elementwise) under the same switches:
+// k slice, splits, workgroups and (per > 1) row sets a wave.  -5: a form that is not built there.
+extern "C" int k8s_gemv_act_plan(int M, int N_out, int K, int pair, int* ks, int* splits, int* wgs, int* per) {
+  const int epi = pair ? EPI_SWIGLU : EPI_BF16;
+  k8s_gemv_plan(M, N_out, K, epi, 0, ks, splits);
+  const int rows = 4 * gemv_rpw(M, N_out, epi, 0), one = (N_out + rows - 1) / rows;
+  const int wg = gemv_loop_wg(false, M, N_out, K, epi, 0, *splits, one);
+  if (gemv_kw() != 1 || (wg > 0 && gemv_is_wide(M, K, epi, 0))) return -5;
+  *per = wg > 0 ? (one + 256 * wg - 1) / (256 * wg) : 1;
+  *wgs = (one + *per - 1) / *per;
+  return 0;
+}
+
 static int gemv_launch(int mode, void* out, void* partial, const void* x, const void* W, const float* wscale, int M,
                        int N_out, int K, int epi, const void* res_in, void* res_out, const void* nw, float eps,
                        hipStream_t stream) {
@@ -103,12 +142,7 @@ static int gemv_launch(int mode, void* out, void* partial, const void* x, const 
   if (splits > 1 && partial == nullptr) return -3;
   float* part = splits > 1 ? (float*)partial : nullptr;
   const int rpw = gemv_rpw(M, N_out, epi, mode);
-  // KW: waves per row set (K8S_GEMV_KW = 2 / 4 splits a row set's K over that many waves).  One wave per row
-  // set is the default: the two-wave split the small-N projections (TP = 8 QKV, LM head) used to take measured
-  // slower end to end (TP = 8 shapes 4.28 -> 4.26 ms/token with one wave, 8B and TP = 1 unchanged,
-  // profiles/gemv_kw_ab.txt).
-  static const int kw_env = [] { const char* e = getenv("K8S_GEMV_KW"); return e ? atoi(e) : 0; }();
-  const int kw = (kw_env == 2 || kw_env == 4) ? kw_env : 1;
+  const int kw = gemv_kw();
   // The norm variants keep 4 row sets per workgroup when they split K (8 waves, 512 threads):
   // the per-workgroup norm prologue is then shared by twice the waves instead of being repeated.
   const int nt = (mode != 0 && kw == 2 && M <= 4) ? 512 : 256;
@@ -121,18 +155,9 @@ static int gemv_launch(int mode, void* out, void* partial, const void* x, const 
   const bf16_t* ri = (const bf16_t*)res_in;
   bf16_t* ro = (bf16_t*)res_out;
   const bf16_t* gw = (const bf16_t*)nw;
-  const bool swiglu_loop = epi == EPI_SWIGLU && (int)grid.x <= g_gemv_loop_swiglu_max;
-  // the loop only on matrices of >= 64 Mi weights (the 70B's at TP = 1, gate/up at TP = 4): on the smaller ones
-  // (Llama-3-8B, fp8 at TP = 4) it measured slower
-  const bool big = (long long)(epi == EPI_SWIGLU ? 2 * N_out : N_out) * K >= ((long long)g_gemv_loop_min_mi << 20);
-  const bool plain_loop = epi == EPI_BF16 && big;
-  const int loop_wg = g_gemv_loop >= 0 ? g_gemv_loop
-                                       : (fp8 ? (big ? 2 : 0) : (plain_loop ? g_gemv_loop_bf16 : (swiglu_loop ? 2 : 0)));
-  if (loop_wg > 0 && splits == 1 && kw == 1 && mode != 1 && M <= 2 && (int)grid.x > 256 * loop_wg) {
-    // wide: 8-wave workgroups for the plain bf16-epilogue projections whose x slice takes >= 32 KiB of LDS (the
-    // down projection, K = 28672: 56 KiB): LDS, not waves, bounds those at 2 workgroups per CU, so twice the waves
-    // per workgroup put twice the weight loads in flight per CU (K8S_GEMV_WIDE = 0 turns it off)
-    const bool wide = g_gemv_wide && mode == 0 && epi == EPI_BF16 && (long long)M * K * 2 >= 32768;
+  const int loop_wg = gemv_loop_wg(fp8, M, N_out, K, epi, mode, splits, (int)grid.x);
+  if (loop_wg > 0) {
+    const bool wide = gemv_is_wide(M, K, epi, mode);
     if (wide) {
       const int wgs = (N_out + 8 * rpw - 1) / (8 * rpw);
       {

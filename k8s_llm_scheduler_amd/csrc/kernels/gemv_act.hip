@@ -7,27 +7,21 @@
 using namespace k8sllm;
 
 extern "C" int k8s_gemv_rpw(int M, int N_out, int epi);
-extern "C" void k8s_gemv_plan(int M, int N_out, int K, int epi, int mode, int* ks_out, int* splits_out);
-extern "C" int k8s_gemv_set_loop(int wg_per_cu);
+extern "C" int k8s_gemv_act_plan(int M, int N_out, int K, int pair, int* ks, int* splits, int* wgs, int* per);
 
-// kind: gated 0, 1, 5 (W [2 N_out][K] = gate | up) or 7; partial: as k8s_gemv_plan asks for with epi 2 (gated) or 0.
+// kind: gated 0, 1, 5 (W [2 N_out][K] = gate | up) or 7; partial: as k8s_gemv_plan asks for with epi 2 (gated) or 0.  -5: the
+// switches or the size ask for a form of the GEMV that is not built here.
 extern "C" int k8s_gemv_act(void* out, void* partial, const void* x, const void* W, int M, int N_out, int K, int kind,
                             float limit, float alpha, hipStream_t stream) {
   const bool pair = kind == 0 || kind == 1 || kind == 5;
   if (M < 1 || M > 2 || K <= 0 || K % 8 != 0 || N_out <= 0 || (!pair && kind != 7)) return -1;
-  const int plain = pair ? EPI_SWIGLU : EPI_BF16;
-  int ks, splits;
-  k8s_gemv_plan(M, N_out, K, plain, 0, &ks, &splits);
+  int ks, splits, wgs, per;
+  const int rc = k8s_gemv_act_plan(M, N_out, K, pair, &ks, &splits, &wgs, &per);
+  if (rc != 0) return rc;
   if (splits > 1 && partial == nullptr) return -3;
   float* part = splits > 1 ? (float*)partial : nullptr;
-  const int rpw = k8s_gemv_rpw(M, N_out, plain), half = pair ? N_out : 0;
-  dim3 grid((N_out + 4 * rpw - 1) / (4 * rpw), splits);
-  // row sets in a loop where the SwiGLU form takes it by default: two workgroups per CU
-  const bool loop = pair && splits == 1 && k8s_gemv_set_loop(-2) != 0 && grid.x > 512 && grid.x <= 2048;
-  if (loop) {
-    const int per = ((int)grid.x + 511) / 512;
-    grid.x = (grid.x + per - 1) / per;
-  }
+  const int rpw = k8s_gemv_rpw(M, N_out, pair ? EPI_SWIGLU : EPI_BF16), half = pair ? N_out : 0;
+  const dim3 grid(wgs, splits);
   const size_t lds = (size_t)M * ks * 2;
   const EpiAct act{kind, limit, alpha};
   auto go = [&](auto m, auto r) {
@@ -36,9 +30,8 @@ extern "C" int k8s_gemv_act(void* out, void* partial, const void* x, const void*
 #define GA(EE, LP) \
   gemv_kernel<MM, RR, EE, 0, false, 1, 256, false, LP><<<grid, 256, lds, stream>>>( \
       out, part, xx, W, N_out, K, ks, half, nullptr, nullptr, nullptr, 0.f, nullptr, GemvAr{}, act)
-    if (loop) GA(EPI_GLU, true);
-    else if (pair) GA(EPI_GLU, false);
-    else GA(EPI_ELEM, false);
+    if (pair) { if (per > 1) GA(EPI_GLU, true); else GA(EPI_GLU, false); }
+    else { if (per > 1) GA(EPI_ELEM, true); else GA(EPI_ELEM, false); }
 #undef GA
   };
   using std::integral_constant;

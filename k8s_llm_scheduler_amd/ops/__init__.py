@@ -822,12 +822,14 @@ def linear_act_rows(x: torch.Tensor, w: torch.Tensor, pair: bool, kind: int, lim
         return None
     epi = EPI_SWIGLU if pair else EPI_BF16
     out = torch.empty(M, N, dtype=BF16, device=x.device)
-    if M <= min(GEMV_MAX_M, 2):
+    if M <= GEMV_MAX_M:
+        if M > 2:      # (K8S_GEMV_MAX_M)
+            return None
         _, splits = native().gemv_plan(M, N, K, epi, 0)
         part = torch.empty(splits * M * w.shape[0], dtype=F32, device=x.device) if splits > 1 else None
-        native().gemv_act(out.data_ptr(), part.data_ptr() if part is not None else 0, _chk(x, BF16, "x"), _chk(w, BF16, "w"), M, N,
-                          K, kind, limit, alpha, -1)
-        return out
+        rc = native().gemv_act(out.data_ptr(), part.data_ptr() if part is not None else 0, _chk(x, BF16, "x"), _chk(w, BF16, "w"),
+                               M, N, K, kind, limit, alpha, -1)
+        return None if rc == -5 else out
     if M <= SGEMV_MAX_M:
         n = native().sgemv_workspace(M, N, K, epi, 0)
         part = torch.empty(n, dtype=F32, device=x.device) if n > 0 else None

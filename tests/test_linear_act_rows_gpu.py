@@ -62,3 +62,23 @@ def test_replays_equal_the_eager_result():
         again = run()
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(again, want))
+
+
+@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("kind", [sm.ACT_SWISH_CLAMP, sm.ACT_RELU2])
+def test_row_sets_in_a_loop(M, kind):
+    """One or two rows with the GEMV's row-set loop off and at 1 - 3 workgroups a CU, row sets that do not divide among the waves."""
+    pair, N, K = kind != sm.ACT_RELU2, 4104 if kind != sm.ACT_RELU2 else 8224, 1024
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(2 * N if pair else N, K, generator=g, device=DEV) * 2 / K ** 0.5).to(torch.bfloat16)
+    want = act64(x.double() @ w.double().T, kind, 1.5, 1.702)
+    before = ops.native().gemv_set_loop(-2)
+    try:
+        for loop in (0, 1, 2, 3):
+            ops.native().gemv_set_loop(loop)
+            got = ops.linear_act_rows(x, w, pair, kind, 1.5, 1.702)
+            assert ops.native().gemv_act_plan(M, N, K, pair)[2] == (1 if loop == 0 else -(-(1026 if pair else 1028) // (256 * loop)))
+            assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all(), loop
+    finally:
+        ops.native().gemv_set_loop(before)

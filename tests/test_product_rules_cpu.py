@@ -1,5 +1,10 @@
 """Which kernel and which plan a product takes, without a GPU: the launches are noted instead of made, every size question goes
 to the extension."""
+import os
+import subprocess
+import sys
+from pathlib import Path
+
 import pytest
 import torch
 
@@ -7,6 +12,7 @@ from k8s_llm_scheduler_amd import ops
 from k8s_llm_scheduler_amd.ops import seqmix as sm
 
 BF16 = torch.bfloat16
+ROOT = Path(__file__).resolve().parent.parent
 
 
 class Launches:
@@ -21,7 +27,7 @@ class Launches:
     def __getattr__(self, name):
         if name not in self.LAUNCH:
             return getattr(self.real, name)
-        return lambda *args: self.made.append((name, args))
+        return lambda *args: self.made.append((name, args)) or 0
 
     def names(self):
         return [n for n, _ in self.made]
@@ -122,3 +128,30 @@ def test_activations_join_every_unsplit_product_of_big_tiles(M, N, K, kind, laun
     assert kern == "pgemm4"
     sm.linear_act(torch.zeros(M, K, dtype=BF16), torch.zeros(N, K, dtype=BF16), kind)
     assert launches.names() == (["pgemm4_act"] if plan[1] == 1 else ["pgemm4", "act"]) and (plan[1] > 1) == (K == 4096)
+
+
+def test_activations_follow_the_switches_of_the_gemv(launches, monkeypatch):
+    """K8S_GEMV_MAX_M moves 3 - 8 rows to the GEMV, whose form with an activation takes two: then the product and the activation."""
+    for rows, kind in ((4096, sm.ACT_GELU_TANH), (2048, sm.ACT_RELU2)):
+        w = torch.zeros(rows, 2048, dtype=BF16)
+        for limit, M, want in ((2, 1, "gemv_act"), (2, 3, "sgemv_act"), (8, 2, "gemv_act"), (8, 3, "act"), (8, 8, "act"), (8, 9, "sgemv_act"),
+                               (1, 1, "gemv_act")):
+            monkeypatch.setattr(ops, "GEMV_MAX_M", limit)
+            launches.made.clear()
+            sm.linear_act(torch.zeros(M, 2048, dtype=BF16), w, kind)
+            assert launches.names()[-1] == want and len(launches.made) == (2 if want == "act" else 1), (limit, M)
+            assert want != "act" or launches.names()[0].startswith("gemv")
+
+
+@pytest.mark.parametrize("env,want", [
+    ({}, [(1, 342, 3), (1, 512, 2), (1, 3584, 1), (1, 1024, 1)]), ({"K8S_GEMV_LOOP": "0"}, [(1, 1026, 1), (1, 1024, 1), (1, 3584, 1), (1, 1024, 1)]),
+    ({"K8S_GEMV_LOOP": "1"}, [(1, 206, 5), (1, 256, 4), (1, 256, 14), (1, 256, 4)]), ({"K8S_GEMV_LOOP": "3"}, [(1, 513, 2), (1, 512, 2), (1, 717, 5), (1, 512, 2)]),
+    ({"K8S_GEMV_LOOP_SWIGLU_MAX": "1000"}, [(1, 1026, 1), (1, 1024, 1), (1, 3584, 1), (1, 1024, 1)]), ({"K8S_GEMV_KW": "2"}, [None] * 4),
+    ({"K8S_GEMV_RPW1": "2"}, [(1, 257, 2), (1, 512, 1), (1, 448, 4), (1, 1024, 1)])])
+def test_launches_with_an_activation_follow_the_gemv_switches(env, want):
+    """(k splits, workgroups, row sets a wave) of 2 x 4104 x 1024, 2 x 4096 x 2048, 2 x 14336 x 4096 and, elementwise, 8192 x 2048."""
+    code = ("from k8s_llm_scheduler_amd import ops\n"
+            "print([ops.native().gemv_act_plan(1, n, k, p) for n, k, p in ((4104, 1024, 1), (4096, 2048, 1), (14336, 4096, 1), (8192, 2048, 0))])")
+    clean = {k: v for k, v in os.environ.items() if not k.startswith("K8S_GEMV")}
+    out = subprocess.run([sys.executable, "-c", code], env={**clean, **env}, cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert out.stdout.strip() == str(want), out.stderr
