@@ -404,10 +404,11 @@ def _few_fits(a: torch.Tensor, w: torch.Tensor) -> bool:
 
 def linear_each(a: torch.Tensor, w: torch.Tensor):
     """[a[i] @ w[i].T]: several inputs, a weight each (a [G, M, K], w [G, N, K]) -> G tensors [M, N] of one row stride.  One
-    launch where that is faster than G of :func:`linear`.  4 weights of 2048 x 2048, M = 8 / 32 / 64 / 128 / 512 / 1024 / 2048:
-    the any-shape kernel (k shared by the waves while its tiles are few) 11 / 16 / 23 / 33 us, the grouped big tiles 16 / 16 /
-    17 / 17 / 22 / 33 / 56, four launches 21 / 22 / 27 / 32 / 59 / 66 / 86; of 4096 x 4096, M = 8 / 16 / 32 / 64 / 512 / 2048: 31 /
-    37 / 54 / 84 us, 35 / 35 / 36 / 37 / 61 / 194, 33 / 41 / 45 / 54 / 117 / 235."""
+    launch where that is faster than G of :func:`linear`: the any-shape kernel (k shared by the waves while its tiles are few) up to
+    32 rows, and as long as its workgroups of 16 columns run at once; else the grouped big tiles from 16 rows on, of small weights from
+    the first.  us, weights from memory, any-shape / big tiles / G launches: 4 weights of 2048 x 2048, M = 8 10.9 / 17.7 / 19.9, 32 17.2 /
+    17.8 / 24.2, 64 24.5 / 18.3 / 29.2, 512 51.7 / 23.8 / 60.3; of 512 x 2048, 128 13.3 / 15.6 / 23.3, 200 20.9 / 15.1 / 39.8; of 4096 x
+    4096, 8 71 / 37.2 / 33.1, 16 71 / 36.8 / 39.4, 64 73.6 / 38.6 / 54.6, 2048 - / 195 / 236; 8 of 2048 x 2048, 1 36.7 / 20.4 / 34.2."""
     G, M, K = a.shape
     N = w.shape[1]
     if w.shape != (G, N, K):
@@ -415,9 +416,10 @@ def linear_each(a: torch.Tensor, w: torch.Tensor):
     if not (FAST_GEMM and _gpu(a, w) and _route_fast(a[0], w[0], a.dtype)):
         return gemm(a, w).unbind(0)
     if _each_once(a, w):
-        if G * (-(-M // 64)) * (-(-N // 64)) <= 128:
+        rows = G * (-(-M // 64))
+        if rows * (-(-N // 64)) <= 128 and (M <= 32 or rows * (-(-N // 16)) <= 256):
             return gemm(a, w).unbind(0)
-        if 32 < M <= 2048:
+        if M <= 2048 and (M >= 16 or N * K <= 1 << 23):
             return _pgemm4_grouped(a.view(G * M, K), w, None, G * M, None, N).view(G, M, N).unbind(0)
     return tuple(linear(a[i], w[i]) for i in range(G))
 

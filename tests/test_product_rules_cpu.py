@@ -155,3 +155,15 @@ def test_launches_with_an_activation_follow_the_gemv_switches(env, want):
     clean = {k: v for k, v in os.environ.items() if not k.startswith("K8S_GEMV")}
     out = subprocess.run([sys.executable, "-c", code], env={**clean, **env}, cwd=ROOT, capture_output=True, text=True, timeout=300)
     assert out.stdout.strip() == str(want), out.stderr
+
+
+@pytest.mark.parametrize("G,N,K,any_to,grouped_from", [(4, 2048, 2048, 32, 33), (2, 2048, 2048, 64, 65), (4, 512, 2048, 128, 129), (4, 1024, 4096, 64, 65),
+                                                       (4, 4096, 4096, 0, 16), (8, 2048, 2048, 0, 1), (3, 6144, 2048, 0, 16)])
+def test_products_of_several_inputs_share_a_launch_where_that_is_faster(G, N, K, any_to, grouped_from, launches):
+    """Up to which rows the any-shape kernel takes them, from which the grouped big tiles do; else one launch each."""
+    w = torch.zeros(G, N, K, dtype=BF16)
+    for M in (1, 8, 15, 16, 32, 33, 64, 65, 128, 129, 512, 2048, 2049):
+        launches.made.clear()
+        sm.linear_each(torch.zeros(G, M, K, dtype=BF16), w)
+        want = ["gemm_any"] if M <= any_to else ["pgemm4_grouped"] if grouped_from <= M <= 2048 else None
+        assert launches.names() == want if want else len(launches.made) >= G, M

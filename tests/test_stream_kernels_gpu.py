@@ -579,16 +579,16 @@ def test_prompt_attention_lets_non_finite_scores_through(ns, sink, monkeypatch):
 @pytest.mark.parametrize("M", [1, 32, 33, 64, 127, 129, 1031, 2048, 2049])
 @pytest.mark.parametrize("N,K", [(2048, 256), (1040, 512), (4096, 192)])
 def test_products_of_several_inputs(M, N, K, entries):
-    """Every way a launch is shared: few tiles (up to 64, 128 and no rows of these widths), even groups of the big tiles with
+    """Every way a launch is shared: few tiles (up to 32, 64 and no rows of these widths), even groups of the big tiles with
     remainders, one launch per input."""
     g = torch.Generator().manual_seed(M + N)
     a, w = (torch.randn(3, n, K, generator=g).to(torch.bfloat16) for n in (M, N))
     a_dev, w_dev = a.to(DEV), w.to(DEV)
     entries.clear()
     got = sm.linear_each(a_dev, w_dev)
-    if M <= {2048: 64, 1040: 128, 4096: 0}[N]:
+    if M <= {2048: 32, 1040: 64, 4096: 0}[N]:
         assert entries == ["gemm_any"]
-    elif 32 < M <= 2048:
+    elif M <= 2048:
         assert entries == ["pgemm4_grouped"]
     else:
         assert len(entries) >= 3 and not {"gemm_any", "pgemm4_grouped"} & set(entries)
