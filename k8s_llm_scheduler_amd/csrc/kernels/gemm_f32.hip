@@ -171,9 +171,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(F32Args a) {
 // The same product with k shared by the waves instead of the columns: a wave owns all 64 columns x 16 FQ rows of the tile for a
 // quarter of k, stages its own weights and rows (16-deep, 64-byte rows, a ring of 4 slots) and meets the others once, at the
 // end, in LDS -- no barrier and no other wave's loads to wait for while k lasts.  85 - 90 % of the matrix rate on a CU with one
-// workgroup (all that the rings leave room for).  us, columns shared -> k shared: 333 x 2048 x 2048 35.0 -> 31.4, x 8192 129 ->
-// 109, 200 x 2048 x 8192 97 -> 79, 200 x 4096 x 4096 81 -> 73, 100 x 4096 x 14336 170 -> 144, 64 x 16384 x 2048 50 -> 45; in three
-// rounds and more it is behind (333 x 16384 x 2048 180 and 203).  Ahead of gemm_f32_kernel's eight shares too: 333 x 576 x 2048
+// workgroup (all that the rings leave room for, but at FQ = 1, where two fit).  us, columns shared -> k shared:
+// 333 x 2048 x 2048 35.0 -> 31.4, x 8192 129 -> 109, 200 x 2048 x 8192 97 -> 79, 200 x 4096 x 4096 81 -> 73,
+// 100 x 4096 x 14336 170 -> 144, 64 x 16384 x 2048 50 -> 45; in three rounds and more it is behind (333 x 16384 x 2048 180 and 203).  Ahead of gemm_f32_kernel's eight shares too: 333 x 576 x 2048
 // 18.0 -> 14.4, 64 x 2048 x 8192 68 -> 58.  Error against 64 bits, 2-norm: 2.1e-7 - 2.3e-7.
 template <typename TO, int FQ>
 __global__ __launch_bounds__(256, 1) void gemm_f32_kwave_kernel(F32Args a) {

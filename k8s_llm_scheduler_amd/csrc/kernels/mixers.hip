@@ -303,6 +303,7 @@ __device__ __forceinline__ float row_sum(float v) { return dpp_add<0x140>(dpp_ad
 // A without a division: the highest bit in which s and t differ cuts the tokens between them at a multiple of 2^bit, r_t takes the
 // decays from there on and k_s those up to there.  For every bit one 16 x 64 matrix M holds the rows r of the tokens with
 // the bit and the rows k of those without, and wave `bit` takes its part of A from M M^T (one fragment for both operands).
+// 128 registers (four waves a SIMD) are two fewer than it wants: two addresses of the end state wait in memory until then.
 // 2048 tokens of 32 heads of 64: 44 us, 333 in fp32 13.5 (walking the state token by token in registers, 200 vector multiply-adds
 // per token, head and wave: 54 and 22.6; A by a walk over t: 45 and 15.4).  About 850 vector instructions a wave for 16
 // tokens (24 us of the 44: the decays' and gates' exponentials, staging, the norm) and 52 products (11 us), four waves on a SIMD.

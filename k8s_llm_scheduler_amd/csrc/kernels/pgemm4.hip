@@ -28,7 +28,9 @@
 // 256 x 256 tiles 2048 x 8192 x 2048 64 -> 56 (52), x 8192 208 -> 188 (188), 3413 x 8192 x 8192 364 -> 342 (333); 128 x 256
 // 2048 x 8192 x 2048 82 -> 64; 128 x 128 2048 x 2048 x 2048 25 -> 22 (22), x 8192 94 -> 73 (78).  Bound by the matrix rate at
 // the clock that the power allows (1.7 - 2.0 GHz in long launches; operands all zero take 25 % less time): 89 % of a stage's
-// cycles are the matrix cores', and at K = 2048 a fifth of the launch is its start, first loads and stores.
+// cycles are the matrix cores', and at K = 2048 a fifth of the launch is its start, first loads and stores.  The 256 x 256 tiles
+// take all 512 registers, and by the compiler's report spill 16 - 38 of them between the k loop and the rows in LDS (bf16 20,
+// SwiGLU 31, fp32 output 0, with the RMS prologue 28, 24 and 12; the gated kinds 31 - 38, relu^2 16), none of it inside the loop.
 #include <type_traits>
 
 #include "act.h"
@@ -51,10 +53,15 @@ __device__ __forceinline__ void p4_sync() {
 }
 // LDS-DMA of 16 bytes a lane, from a uniform base and the lane's 32-bit offset to LDS byte `lds` + 16 lane.  In asm: from the
 // builtin the compiler hoists base + offset, or the widened offset, into 64-bit lane addresses and adds the step to each of
-// them, an instruction and two registers per load.
+// them, an instruction and two registers per load.  m0 is the compiler's own, which it need not keep for itself across an asm that
+// names it (the warning that is off here): nothing else in this file may want it -- no LDS-DMA builtin, no register indexed at run
+// time.  (In this file's assembly every m0 is the move of one of these.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void p4_dma(const uint8_t* base, uint32_t off, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 __device__ __forceinline__ float p4_silu(float g) { return g / (1.f + __expf(-g)); }
 // The kind of an activation (act.h) is a template argument: 128 unrolled elements per lane with every kind's branches took 775
 // us where the product takes 56.
@@ -75,8 +82,8 @@ struct P4Args {
   float limit, alpha;    // P4_GLU: of the gated kind
   const bf16_t* bias;    // P4_GLU, optional: [gate; up] biases
   // grouped form: group g's rows are [seg[g], seg[g + 1]) of a compact row space (row r of x: a_rows[r], or r) and its
-  // weights W + g wstride bytes; m_tiles bounds the groups' row tiles.  8 experts, 3068 rows, K = 2048: gate / up with its
-  // activation (N = 2 x 2048) 94 us, down (N = 2048) 47 us; 140 and 10 us, and 78 us on the 64-row tiles of stream32.hip.
+  // weights W + g wstride bytes; m_tiles bounds the groups' row tiles.  8 experts, 3068 rows, K = 2048, in a step: gate / up
+  // with its activation (N = 2 x 2048) 69 us, down (N = 2048) 34 us; 140 and 10 us, and 78 us on the 64-row tiles of stream32.hip.
   // seg == nullptr: groups of gsize rows (products of several inputs with a weight each in one launch)
   const int* seg;
   int gsize;

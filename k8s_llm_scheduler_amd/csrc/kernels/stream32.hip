@@ -568,9 +568,10 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(TO* __restrict__ C, const
 // give every SIMD two waves.  A lane reads 4 consecutive k of its row and spends one on each of 4 instructions.  PF steps'
 // loads are in flight.  The waves' sums meet in LDS in wave order: an output's accumulation order depends on K alone, not on
 // the tile or the rows that share it.  Same three forms.
-// Bound by the fp32 matrix rate (157 TFLOP/s; a 32 x 32 x 2048 tile is 7 us of a CU's four pipes).  333 rows: 2048 x 2048
-// (N x K) 40 us (503 us with gemm_any_kernel; 70 TFLOP/s now), 16384 x 2048 270 us (434), 128 x 2048 16 us with the launch
-// (276).  What fills the chip in tiles of 64 columns runs on gemm_f32.hip's.
+// It takes what k8s_gemm_f32_rule leaves it: few rows, few tiles, short listed groups, depths below 512 or no multiple of 32; the rest
+// runs on gemm_f32.hip's tiles.  Bound by the loads of weights that no other workgroup reads (16 rows, from memory: 2048 x 2048
+// (N x K) 19.6 us, 4096 x 14336 120 us), and with many rows by the fp32 matrix rate (157 TFLOP/s; a 32 x 32 x 2048 tile is 7 us of
+// a CU's four pipes).
 template <typename TO, int NN>
 __global__ __launch_bounds__(512) void gemm_f32_kernel(TO* __restrict__ C, const float* __restrict__ A,
                                                        const float* __restrict__ Wt, int M, int N, int K, long lda,
@@ -1091,7 +1092,8 @@ extern "C" int k8s_gemm_any(void* C, const void* A, const void* W, int M, int N,
     gy = (M + 63) / 64;
   }
   if (gy > 65535 || batch > 65535) return -2;
-  // bf16 rows that can be moved as 16-byte vectors: the bf16 MFMA kernels; fp32 ones: gemm_f32_kernel; anything else: plain FMAs
+  // bf16 rows that can be moved as 16-byte vectors: the bf16 MFMA kernels; fp32 ones: gemm_f32.hip's tiles or gemm_f32_kernel, by
+  // k8s_gemm_f32_rule; anything else: plain FMAs
   const bool vec = !in_f32 && K % 8 == 0 && lda % 8 == 0 && ldw % 8 == 0 && sA % 8 == 0 && sW % 8 == 0 &&
                    ((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0;
   if (vec && tiles != nullptr && K % 64 == 0 && M <= 32 * ntiles && M <= 512) {   // few rows per group

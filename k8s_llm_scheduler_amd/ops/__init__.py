@@ -996,7 +996,8 @@ def _pg_load_table() -> dict:
 # hide part from each other; with split-K the combine launch and the slabs it moves; the weights and the output.  Fitted to 22
 # weight shapes (576 x 2048 .. 28672 x 4096) at 12 row counts (40 .. 2048), weights cold: rms error 6 - 10 % per configuration,
 # the pick within 2 % of the best plan on average and 21 % at most, the same as hipBLASLt on average (0.92 - 1.09 of its time
-# by row count).  pgemm.hip's 8-wave tiles were the best plan of none.
+# by row count).  pgemm.hip's 8-wave tiles were the best plan of none of these; the tuned table names them for some of the 70B's
+# products of 192 - 8192 rows and its logits, and SwiGLU and fp8 products that it does not list take them (_pgemm_big_tiles).
 _P4_COST = {1: (0.657, 2.23, 0.0, 5.7, 0.302, 0.0684, 0.367),
             2: (0.599, 2.19, 0.0, 4.12, 0.34, 0.0527, 0.514),
             3: (0.297, 0.0, 0.155, 5.46, 0.348, 0.0739, 0.635),

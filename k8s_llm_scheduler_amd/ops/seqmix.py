@@ -289,7 +289,9 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out_dtype=None, *, a_rows: Optional[t
     any strides whose last is 1, w [G, N, K]) -> [G, M, N]; ``out``: a [G, M, N] view with any batch / row strides.
     Grouped (``tiles`` [n, 3] from :func:`moe_align`, w [G, N, K]): ``rows`` compact rows, row r = a[a_rows[r]] (or
     a[r]), the rows of tile (g, r0, n) use w[g] -> [rows, N].  ``seg`` int32 [G + 1]: the groups' row offsets, the same
-    rows as ``tiles`` lists; the CPU reference and the big-tile kernel (:func:`_grouped_big`) go by them."""
+    rows as ``tiles`` lists; the CPU reference and the big-tile kernel (:func:`_grouped_big`) go by them.  The order of an output's
+    sums depends on the kernel, and that on the sizes: in bf16, and in fp32 from a depth of 512 on, a row's result may differ in the last
+    bits with the rows beside it (fp32 of less depth or of rows that are not 16-byte aligned: not)."""
     out_dtype = out_dtype or a.dtype
     if a.dtype != w.dtype:
         raise TypeError(f"gemm operands differ in dtype: {a.dtype} and {w.dtype}")

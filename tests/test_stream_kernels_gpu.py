@@ -33,7 +33,8 @@ def sum_bound(a, w):
 @pytest.mark.parametrize("M,N,K", [(1, 1, 4), (31, 33, 60), (32, 32, 64), (33, 65, 68), (64, 64, 256), (97, 130, 260),
                                    (40, 16388, 8), (1031, 576, 132), (256, 2048, 320)])
 def test_fp32_products(M, N, K):
-    """Both tile shapes of the fp32 matrix-core product, remainders in every dimension, an odd row stride, a batch."""
+    """Both tile shapes of gemm_f32_kernel (every depth here is below 512), remainders in every dimension, an odd row stride, a
+    batch."""
     g = torch.Generator().manual_seed(M + N + K)
     a, w = torch.randn(M, K + 4, generator=g)[:, :K], torch.randn(N, K, generator=g)
     a[:, 0] *= 1e4
@@ -43,7 +44,7 @@ def test_fp32_products(M, N, K):
     b = torch.stack([a, 2.0 * a])
     got = sm.gemm(b.to(DEV), torch.stack([w, w]).to(DEV)).cpu()
     assert torch.equal(got[1], 2.0 * got[0])
-    assert torch.equal(got[0], sm.gemm(ag, w.to(DEV)).cpu())      # the order of the sums depends on K alone
+    assert torch.equal(got[0], sm.gemm(ag, w.to(DEV)).cpu())      # within this kernel the order of the sums depends on K alone
     assert torch.equal(got[0][M // 2:], sm.gemm(ag[M // 2:], w.to(DEV)).cpu())
 
 
