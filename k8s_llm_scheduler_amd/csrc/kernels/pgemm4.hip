@@ -10,9 +10,19 @@
 // fragments of v_mfma_f32_16x16x32_bf16, 256 accumulator registers: the AGPR half of the unified file at one
 // wave per SIMD), so per 32 k a wave issues 16 fragment reads for 64 MFMAs.
 //
-//  * 64-deep LDS stages of 128-byte rows (every LDS-DMA instruction moves 8 whole rows): three of weights, two of x -- all of
-//    the CU's 160 KB at 256 x 256, two workgroups on a CU at 128 x 128.  x comes from L2; the weights, from memory, are two
-//    stages (about 2 us) in flight across the raw s_barriers, of which there is one per 2 x FP x FQ MFMAs.
+//  * 64-deep LDS stages of 128-byte rows (every LDS-DMA instruction moves 8 whole rows), DW stages of weights and DX of x in
+//    flight across the raw s_barriers, of which there is one per 2 x FP x FQ MFMAs: two and one (three slots, two) from 128 x 64
+//    on -- all of the CU's 160 KB at 256 x 256, two workgroups on a CU at 128 x 128, where more of them measured 0 - 5 % -- and four of
+//    both at 64 x 64, whose stage is 0.1 us of matrix work against a load's 0.5 - 2 (200 x 2048 x 2048 12.6 -> 9.5 us, 333 x 2128 x 2048
+//    0.66 of its time; two workgroups on a CU still).  The least that a stage can take: 32 KB of the two operands in 0.26 us out of
+//    L2 (53 bytes a cycle and CU), what misses L2 at 6 - 7 TB/s whatever holds it.
+//  * one row tile (the weights are read once): XCD i starts its walk over k at stage i n / 8 and wraps.  In step with each other
+//    all of them ask for the same bytes of every row, whose strides of 16 KB meet on a part of the memory's channels, and for the
+//    same lines of x (loads alone, 32768 rows of 16 KB: 4.1 -> 6 TB/s).  241 x 57344 x 8192 251 -> 230 us, 8192 x 28672 136 -> 131,
+//    8192 x 8192 50 -> 47.  With more row tiles the walk in step is the better one (2048 x 16384 x 2048 106 -> 111): so not there; the
+//    grouped form by its rows (P4Args::spread).
+//  * tiles of 224 rows (a fragment then holds 8 gate and 8 up rows, a pair in a lane) and of 192 tokens, where they fill the last
+//    round: 241 x 57344 x 8192 on 256 CUs 230 -> 207 us, 3413 x 10240 x 8192 484 -> 412.
 //  * register double buffer: the fragments of the next 32 k are read (ds_read_b128) under the MFMAs of the current ones, in
 //    the first half of them: spread over all of them, the wait at the end stood 100 - 150 of 1024 matrix cycles a step.
 //  * DMA image lane-linear, XOR swizzle on the per-lane global source: the 16-row fragment reads are conflict-free.
@@ -24,7 +34,7 @@
 //    pgemm_reduce_kernel sums the slabs in slice order (deterministic) and applies the epilogue -- a
 //    parallel reduction over the whole chip instead of one last-arriving workgroup reading every slab.
 //
-// us, weights from memory (rows x N x K), with 32-deep stages, reads and stores spread as they fell -> now, and hipBLASLt:
+// us, weights from memory (rows x N x K), with 32-deep stages, reads and stores spread as they fell -> as above, and hipBLASLt:
 // 256 x 256 tiles 2048 x 8192 x 2048 64 -> 56 (52), x 8192 208 -> 188 (188), 3413 x 8192 x 8192 364 -> 342 (333); 128 x 256
 // 2048 x 8192 x 2048 82 -> 64; 128 x 128 2048 x 2048 x 2048 25 -> 22 (22), x 8192 94 -> 73 (78).  Bound by the matrix rate at
 // the clock that the power allows (1.7 - 2.0 GHz in long launches; operands all zero take 25 % less time): 89 % of a stage's
@@ -41,6 +51,7 @@ namespace k8sllm {
 namespace {
 enum { P4_BF16 = 0, P4_F32 = 1, P4_SWIGLU = 2, P4_GLU = 3, P4_ACT = 4 };   // GLU, ACT: bf16 out, activation KIND
 typedef __attribute__((ext_vector_type(2))) uint32_t p4_u32x2;
+typedef __attribute__((ext_vector_type(2))) float p4_f32x2;
 
 template <int N>
 __device__ __forceinline__ void p4_vmcnt() {
@@ -78,12 +89,15 @@ struct P4Args {
   int M, N_out, half_rows, wrows, K;
   int m_tiles, n_tiles, ks, splits, group_m, nwg;
   float eps;
+  int spread;            // the XCDs start their walk over k an eighth of it apart
   int wide;              // the output's rows can be stored in 16-byte pieces
   float limit, alpha;    // P4_GLU: of the gated kind
   const bf16_t* bias;    // P4_GLU, optional: [gate; up] biases
   // grouped form: group g's rows are [seg[g], seg[g + 1]) of a compact row space (row r of x: a_rows[r], or r) and its
   // weights W + g wstride bytes; m_tiles bounds the groups' row tiles.  8 experts, 3068 rows, K = 2048, in a step: gate / up
   // with its activation (N = 2 x 2048) 69 us, down (N = 2048) 34 us; 140 and 10 us, and 78 us on the 64-row tiles of stream32.hip.
+  // spread with 8 groups and more, an XCD's tiles then another group's, of up to 192 rows: gate / up of 8 experts, 4 - 192 rows
+  // each 29.4 -> 27.8 us (64 x 64), 16 of 2 x 2048 x 4096 139 -> 108 (256 x 128); 4 groups 30.0 -> 34.0, 320 rows 70 -> 71.
   // seg == nullptr: groups of gsize rows (products of several inputs with a weight each in one launch)
   const int* seg;
   int gsize;
@@ -92,14 +106,16 @@ struct P4Args {
   int groups;
 };
 
-template <int FP, int FQ, int EPI, bool RMS, bool GRP = false, int KIND = -1>
+template <int FP, int FQ, int DW, int DX, int EPI, bool RMS, bool GRP = false, int KIND = -1>
 __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
+  static_assert(DW == DX || DW == DX + 1, "a stage's last load is followed by whole stages of later ones");
   constexpr int BP = 32 * FP, BQ = 32 * FQ;          // weight rows, tokens per tile (2 x 2 waves)
   constexpr bool PAIR = EPI == P4_SWIGLU || EPI == P4_GLU;   // gate and up rows of one feature in one wave
+  constexpr bool MIX = PAIR && FP % 2 != 0;          // ... and in one fragment: a lane's four rows are gate, gate, up, up
   static_assert(!GRP || !RMS, "the grouped form has no prologue");
   constexpr int SUBW = BP * 128, SUBX = BQ * 128;    // a 64-deep stage of either operand
   constexpr int GW = BP / 32, GX = BQ / 32;          // 16-byte DMA instructions per thread and stage
-  constexpr int X0 = 3 * SUBW, RING = X0 + 2 * SUBX;
+  constexpr int X0 = (DW + 1) * SUBW, RING = X0 + (DX + 1) * SUBX;
   constexpr int RSS = RING - BQ * 8;                 // in the last stage's memory, once it has been read
 #if defined(__HIP_DEVICE_COMPILE__)
   __shared__ __attribute__((aligned(16))) char lds[RING];
@@ -159,7 +175,10 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
     const int p = j * 256 + tid, r = p >> 3, c = (p & 7) ^ ((r >> 1) & 7);
     const int w = r / (BP / 2), q = r % (BP / 2);
     int row;
-    if constexpr (PAIR) {   // wave rows: BP/4 gate rows then the matching BP/4 up rows
+    if constexpr (MIX) {
+      const int f = min(nt * (BP / 2) + w * (BP / 4) + (q >> 4) * 8 + ((q >> 1) & 6) + (q & 1), a.N_out - 1);
+      row = q & 2 ? a.half_rows + f : f;
+    } else if constexpr (PAIR) {   // wave rows: BP/4 gate rows then the matching BP/4 up rows
       const int f = min(nt * (BP / 2) + w * (BP / 4) + (q % (BP / 4)), a.N_out - 1);
       row = q < BP / 4 ? f : a.half_rows + f;
     } else {
@@ -174,10 +193,13 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
   }
   // this wave's 1 KB of the first 4 KB of LDS
   const uint32_t lds0 = (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)lds) + wid * 1024;
-  auto dma_w = [&](int u, int slot, int d) {   // instruction d of stage u's weights (slot u % 3), of its x
-    p4_dma(Wb + (size_t)u * 128, wo[d], lds0 + slot * SUBW + d * 4096);
-  };
-  auto dma_x = [&](int u, int d) { p4_dma(a.x + (size_t)u * 128, xo[d], lds0 + X0 + (u & 1) * SUBX + d * 4096); };
+  // the walk over k starts at stage `rot` and wraps: stage u reads bytes k0(u) .. k0(u) + 127 of the slice's rows
+  const int rot = a.spread ? (int)(((long long)xcd * n2) >> 3) : 0;
+  const uint32_t kend = (uint32_t)n2 * 128u;
+  auto next_k = [&](uint32_t k) -> uint32_t { return k + 128u == kend ? 0u : k + 128u; };
+  // instruction d of a stage's weights (k offset, byte offset of its slot), of its x
+  auto dma_w = [&](uint32_t k, int slot, int d) { p4_dma(Wb + k, wo[d], lds0 + slot + d * 4096); };
+  auto dma_x = [&](uint32_t k, int slot, int d) { p4_dma(a.x + k, xo[d], lds0 + X0 + slot + d * 4096); };
 
   bf16x8 A0[FP], B0[FQ], A1[FP], B1[FQ];
   f32x4 acc[FP][FQ];
@@ -214,14 +236,13 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
 #pragma unroll
       for (int j = 0; j < FQ; ++j) asm volatile("s_nop 0" : "+a"(acc[i][j]));
   };
-  // ---- 64-deep stages: weights of stage u in slot u % 3, x in slot u & 1; row r at r * 128 bytes, 16-byte chunk c of row
+  // ---- 64-deep stages: weights of stage u in slot u % (DW + 1), x in slot u % (DX + 1); row r at r * 128 bytes, 16-byte chunk c of row
   // r at slot c ^ ((r >> 1) & 7) (the swizzle is applied on the per-lane global source, the DMA image is lane-linear).
   // Sub-step h (k 32 h .. 32 h + 31) of a fragment row li = chunks 4 h + g.  Register sets: R0 = (A0, B0) holds
   // sub-step 0, R1 = (A1, B1) sub-step 1.  Per stage s after the barrier: phase A = the MFMAs of (s - 1, 1) on R1
-  // with the reads of (s, 0) into R0, the LDS-DMA of x of stage s + 1 and then of the weights of stage s + 2 (into the
+  // with the reads of (s, 0) into R0, the LDS-DMA of x of stage s + DX and then of the weights of stage s + DW (into the
   // slots of s - 1, whose reads every wave retired before the barrier) spread between them; phase P = the MFMAs of (s, 0)
-  // on R0 with the reads of (s, 1) into R1.  x comes from L2; the weights, from memory, are two stages (about 2 us) in
-  // flight, and the wait of a stage leaves the next one's weights outstanding.
+  // on R0 with the reads of (s, 1) into R1.  The wait of a stage leaves what was issued behind it outstanding.
   // The fragment reads go out in the first half of a phase: at its end, where they had been spread to, the wait for them
   // stood 100 - 150 of 1024 matrix cycles per phase (8192 columns, 2048 rows, all operands zero: K = 8192 160 -> 140 us).
   const int lo0 = li * 128 + ((g ^ (li >> 1)) << 4), lo1 = li * 128 + (((4 + g) ^ (li >> 1)) << 4);
@@ -236,14 +257,13 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
 #pragma unroll
     for (int f = 0; f < FQ; ++f) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(B[f]) : "v"(lb), "i"(f * 2048));
   };
-  // 64 MFMAs on (Ac, Bc) with (rd) the reads of sub-step h of stage u into (An, Bn), (dx) the loads of x of stage u + 1 and
-  // (dw) of the weights of stage u + 2 spread between them
-  auto phase = [&](const bf16x8* Ac, const bf16x8* Bc, int u, int ws, int h, bf16x8* An, bf16x8* Bn, auto rdc, auto dxc,
-                   auto dwc) {   // ws = u % 3
+  // the MFMAs on (Ac, Bc) with (rd) the reads of sub-step h of a stage (slots at lw, lx) into (An, Bn), (dx) the loads of x of
+  // the stage at kx into the slot at px and (dw) of the weights of the one at kw into pw spread between them
+  auto phase = [&](const bf16x8* Ac, const bf16x8* Bc, int lw, int lx, int h, bf16x8* An, bf16x8* Bn, uint32_t kw, int pw,
+                   uint32_t kx, int px, auto rdc, auto dxc, auto dwc) {
     constexpr int MF = FP * FQ, DR = FP + FQ;
     constexpr bool rd = decltype(rdc)::value, dx = decltype(dxc)::value, dw = decltype(dwc)::value;
-    const uint32_t la = laddr(ws * SUBW + pb2 + (h ? lo1 : lo0)), lb = laddr((u & 1) * SUBX + qb2 + (h ? lo1 : lo0));
-    const int wt = ws == 0 ? 2 : ws - 1;               // the slot of stage u + 2
+    const uint32_t la = laddr(lw + pb2 + (h ? lo1 : lo0)), lb = laddr(lx + qb2 + (h ? lo1 : lo0));
 #pragma unroll
     for (int i = 0; i < FP; ++i)
 #pragma unroll
@@ -252,8 +272,8 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
 #pragma unroll
         for (int d = 0; d < (GW + GX); ++d)
           if (k == d * MF / (GW + GX)) {
-            if (d < GX && dx) dma_x(u + 1, d);
-            if (d >= GX && dw) dma_w(u + 2, wt, d - GX);
+            if (d < GX && dx) dma_x(kx, px, d);
+            if (d >= GX && dw) dma_w(kw, pw, d - GX);
           }
         asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(Ac[i]), "v"(Bc[j]));
 #pragma unroll
@@ -268,50 +288,79 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
   };
   constexpr std::true_type yes{};
   constexpr std::false_type no{};
-  // prologue: weights of stages 0 - 2 and x of stages 0 and 1 in flight, stage 0 visible, (0, 0) read
-  auto all_w = [&](int u) {
+  // prologue: every slot's loads in flight, stage 0 visible, (0, 0) read
+  uint32_t kw = (uint32_t)rot * 128u, kx = kw;         // of the next stage to load
 #pragma unroll
-    for (int d = 0; d < GW; ++d) dma_w(u, u, d);
-  };
-  auto all_x = [&](int u) {
+  for (int u = 0; u <= DW; ++u)
+    if (u < n2) {
 #pragma unroll
-    for (int d = 0; d < GX; ++d) dma_x(u, d);
-  };
-  all_w(0);
-  all_x(0);
-  if (n2 > 1) {
-    all_w(1);
-    all_x(1);
-  }
-  if (n2 > 2) all_w(2);
+      for (int d = 0; d < GW; ++d) dma_w(kw, u * SUBW, d);
+      if (u <= DX) {
+#pragma unroll
+        for (int d = 0; d < GX; ++d) dma_x(kw, u * SUBX, d);
+        kx = kw = next_k(kw);
+      } else {
+        kx = kw;                                       // DW == DX + 1: x is one stage behind
+        kw = next_k(kw);
+      }
+    }
   clear();
-  if (n2 > 2) p4_vmcnt<(GW + GX) + GW>(); else if (n2 > 1) p4_vmcnt<(GW + GX)>(); else p4_vmcnt<0>();
+  // wait for stage 0: what may still be under way is what was issued behind it
+  auto behind = [](int w, int x) constexpr { return w * GW + x * GX; };
+  if (n2 > DW) p4_vmcnt<behind(DW, DX)>();
+  else if (DW > 4 && n2 == 5) p4_vmcnt<behind(4, DX < 4 ? DX : 4)>();
+  else if (DW > 3 && n2 == 4) p4_vmcnt<behind(3, DX < 3 ? DX : 3)>();
+  else if (DW > 2 && n2 == 3) p4_vmcnt<behind(2, DX < 2 ? DX : 2)>();
+  else if (DW > 1 && n2 == 2) p4_vmcnt<behind(1, 1)>();
+  else p4_vmcnt<0>();
   p4_sync();
   rd2(A0, B0);
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
-  phase(A0, B0, 0, 0, 1, A1, B1, yes, no, no);           // P_0: (0, 0) on R0, read (0, 1)
+  phase(A0, B0, 0, 0, 1, A1, B1, 0, 0, 0, 0, yes, no, no);   // P_0: (0, 0) on R0, read (0, 1)
   squares(B0, wr == 0);
-  int ws = 1;                                          // s2 % 3
-  auto stage = [&](int s2, auto dx, auto dw) {
-    // stage s2 landed (this wave's DMA), the weights of s2 + 1 may be under way
-    if constexpr (decltype(dx)::value) p4_vmcnt<GW>(); else p4_vmcnt<0>();
+  int lw = SUBW, lx = SUBX, pw = 0, px = 0;            // byte offsets of the slots of stage s2, and of the one before it
+  // stage s2, of which `left` follow (DW stands for DW and more)
+  auto stage = [&](auto leftc) {
+    constexpr int left = decltype(leftc)::value;
+    constexpr int ow = left < DW - 1 ? left : DW - 1, ox = left < DX - 1 ? left : DX - 1;
+    constexpr std::integral_constant<bool, (left >= DX)> dx{};
+    constexpr std::integral_constant<bool, (left >= DW)> dw{};
+    p4_vmcnt<behind(ow, ox)>();                        // stage s2 landed (this wave's DMA), later ones may be under way
     p4_sync();                                         // ... for every wave; (s2 - 1, 1) reads retired
     __builtin_amdgcn_sched_barrier(0);
-    phase(A1, B1, s2, ws, 0, A0, B0, yes, dx, dw);     // A: (s2 - 1, 1) on R1, read (s2, 0), DMA
+    phase(A1, B1, lw, lx, 0, A0, B0, kw, pw, kx, px, yes, dx, dw);   // A: (s2 - 1, 1) on R1, read (s2, 0), DMA
     squares(B1, wr == 1);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    phase(A0, B0, s2, ws, 1, A1, B1, yes, no, no);     // P: (s2, 0) on R0, read (s2, 1)
+    phase(A0, B0, lw, lx, 1, A1, B1, 0, 0, 0, 0, yes, no, no);       // P: (s2, 0) on R0, read (s2, 1)
     squares(B0, wr == 0);
-    ws = ws == 2 ? 0 : ws + 1;
+    pw = lw;
+    px = lx;
+    lw = lw == DW * SUBW ? 0 : lw + SUBW;
+    lx = DX == 1 ? SUBX - lx : lx == DX * SUBX ? 0 : lx + SUBX;
+    if constexpr (DW == DX) {
+      kx = kw = next_k(kw);
+    } else {
+      kx = kw;
+      kw = next_k(kw);
+    }
   };
-  for (int s2 = 1; s2 < n2 - 2; ++s2) stage(s2, yes, yes);
-  if (n2 > 2) stage(n2 - 2, yes, no);
-  if (n2 > 1) stage(n2 - 1, no, no);
+  for (int s2 = 1; s2 < n2 - DW; ++s2) stage(std::integral_constant<int, DW>{});
+  auto tail = [&](auto leftc) {
+    constexpr int left = decltype(leftc)::value;
+    if constexpr (left < DW)
+      if (n2 - 1 > left) stage(leftc);
+  };
+  static_assert(DW <= 5, "tail stages");
+  tail(std::integral_constant<int, 4>{});
+  tail(std::integral_constant<int, 3>{});
+  tail(std::integral_constant<int, 2>{});
+  tail(std::integral_constant<int, 1>{});
+  tail(std::integral_constant<int, 0>{});
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
-  phase(A1, B1, 0, 0, 0, A0, B0, no, no, no);          // the last sub-step, (n2 - 1, 1), on R1
+  phase(A1, B1, 0, 0, 0, A0, B0, 0, 0, 0, 0, no, no, no);   // the last sub-step, (n2 - 1, 1), on R1
   squares(B1, wr == 1);
   p4_vmcnt<0>();
   {   // ... and the last MFMAs' results wait out the MFMA latency before the epilogue reads them:
@@ -349,7 +398,14 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
 #pragma unroll
       for (int i = 0; i < FP; ++i) {
         int r0;
-        if constexpr (PAIR) {
+        if constexpr (MIX) {
+          const int f = nt * (BP / 2) + wr * (BP / 4) + i * 8 + 2 * g;
+          if (f >= a.N_out) continue;
+          float* row = sl + (size_t)m * a.wrows;
+          *reinterpret_cast<p4_f32x2*>(row + f) = p4_f32x2{acc[i][j][0], acc[i][j][1]};
+          *reinterpret_cast<p4_f32x2*>(row + a.half_rows + f) = p4_f32x2{acc[i][j][2], acc[i][j][3]};
+          continue;
+        } else if constexpr (PAIR) {
           const int hf = i / (FP / 2), f = nt * (BP / 2) + wr * (BP / 4) + (i % (FP / 2)) * 16 + 4 * g;
           if (f >= a.N_out) continue;
           r0 = hf ? a.half_rows + f : f;
@@ -365,26 +421,39 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
     return;
   }
 
-  // ---- epilogue: lane holds out[token li of fragment j][features 4 g .. 4 g + 3 of fragment i]
-  constexpr int OF = PAIR ? FP / 2 : FP;             // fragments of output features
+  // ---- epilogue: lane holds out[token li of fragment j][features 4 g .. 4 g + 3 of fragment i] (MIX: 2 g, 2 g + 1 of 8)
+  constexpr int OF = PAIR && !MIX ? FP / 2 : FP;     // fragments of output features
+  constexpr int FF = MIX ? 8 : 16, LF = FF / 4;      // features of one, and of a lane in it
   auto rms = [&](int mloc) -> float {
     if constexpr (RMS) return rsqrtf(rss[mloc] / (float)a.K + a.eps);
     else return 1.f;
   };
-  // the 4 features of fragments (i, j): the sums with their scale, bias and activation
+  // the LF features of fragments (i, j): the sums with their scale, bias and activation
   auto value = [&](int i, int j, int n0, float sx, float* v) {
     if constexpr (EPI == P4_GLU) {
       f32x4 bg = {0.f, 0.f, 0.f, 0.f}, bu = bg;
       if (a.bias != nullptr) {
-        bg = ldf4(a.bias + n0);
-        bu = ldf4(a.bias + a.half_rows + n0);
+        if constexpr (MIX) {                         // (n0 and N_out are even)
+          const uint32_t p = *reinterpret_cast<const uint32_t*>(a.bias + n0);
+          const uint32_t q = *reinterpret_cast<const uint32_t*>(a.bias + a.half_rows + n0);
+          bg = f32x4{lo_bf(p), hi_bf(p), 0.f, 0.f};
+          bu = f32x4{lo_bf(q), hi_bf(q), 0.f, 0.f};
+        } else {
+          bg = ldf4(a.bias + n0);
+          bu = ldf4(a.bias + a.half_rows + n0);
+        }
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        v[e] = epi_pair<KIND>(acc[i][j][e] + bg[e], acc[FP / 2 + i][j][e] + bu[e], a.limit, a.alpha);
+      for (int e = 0; e < LF; ++e) {
+        const float up = MIX ? acc[i][j][2 + e] : acc[FP / 2 + i][j][e];
+        v[e] = epi_pair<KIND>(acc[i][j][e] + bg[e], up + bu[e], a.limit, a.alpha);
+      }
     } else if constexpr (EPI == P4_SWIGLU) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = p4_silu(acc[i][j][e] * sx) * (acc[FP / 2 + i][j][e] * sx);
+      for (int e = 0; e < LF; ++e) {
+        const float up = MIX ? acc[i][j][2 + e] : acc[FP / 2 + i][j][e];
+        v[e] = p4_silu(acc[i][j][e] * sx) * (up * sx);
+      }
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] * sx;
@@ -394,26 +463,29 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
       }
     }
   };
-  const int nw = nt * (32 * OF) + wr * (16 * OF);    // the wave's first feature
+  const int nw = nt * (2 * FF * OF) + wr * (FF * OF);    // the wave's first feature
   if constexpr (EPI != P4_F32) {
     if (a.wide) {
-      // bf16 rows through LDS: the wave's 16 FQ tokens x 16 OF features in the ring's memory (16-byte chunk c of a row in slot
+      // bf16 rows through LDS: the wave's 16 FQ tokens x FF OF features in the ring's memory (16-byte chunk c of a row in slot
       // c ^ row), then 16 bytes a lane in row order -- whole 64 - 256-byte runs of a row a store, where the registers' order
       // gives 32-byte pieces of 16 rows
-      constexpr int NC = 2 * OF, ROW = 32 * OF, SH = NC == 4 ? 1 : 0;
-      static_assert(4 * 16 * FQ * ROW <= RING, "the tile's rows fit the ring");
+      constexpr int CH = FF * OF / 8, NC = CH <= 2 ? 2 : CH <= 4 ? 4 : CH <= 8 ? 8 : 16, ROW = 16 * NC, SH = NC == 4 ? 1 : 0;   // CH of NC chunks
+      static_assert(FF * OF % 8 == 0 && 4 * 16 * FQ * ROW <= RING, "the tile's rows fit the ring");
       __syncthreads();                               // every wave has read its last fragments
       char* mine = lds + wid * (16 * FQ * ROW);
 #pragma unroll
       for (int j = 0; j < FQ; ++j) {
-        const int row = j * 16 + li;
+        const int row = j * 16 + li, sw = (row >> SH) & (NC - 1);
         const float sx = rms(wc * (BQ / 2) + row);
 #pragma unroll
         for (int i = 0; i < OF; ++i) {
           float v[4];
-          value(i, j, min(nw + i * 16 + 4 * g, a.N_out - 4), sx, v);
-          *reinterpret_cast<p4_u32x2*>(mine + row * ROW + (((2 * i + (g >> 1)) ^ ((row >> SH) & (NC - 1))) << 4) + (g & 1) * 8) =
-              p4_u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+          value(i, j, min(nw + i * FF + LF * g, a.N_out - LF), sx, v);
+          if constexpr (MIX)
+            *reinterpret_cast<uint32_t*>(mine + row * ROW + ((i ^ sw) << 4) + g * 4) = pack_bf2(v[0], v[1]);
+          else
+            *reinterpret_cast<p4_u32x2*>(mine + row * ROW + (((2 * i + (g >> 1)) ^ sw) << 4) + (g & 1) * 8) =
+                p4_u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
         }
       }
       asm volatile("" ::: "memory");                 // the wave's own LDS operations run in order
@@ -423,7 +495,7 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
       for (int p = 0; p < 16 * FQ * NC / 64; ++p) {
         const int row = p * (64 / NC) + lane / NC, m = m0 + wc * (BQ / 2) + row, n0 = nw + c * 8;
         const u32x4 o = *reinterpret_cast<const u32x4*>(mine + row * ROW + ((c ^ ((row >> SH) & (NC - 1))) << 4));
-        if (m < m_end && n0 < a.N_out)
+        if (m < m_end && n0 < a.N_out && (CH == NC || c < CH))
           *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(a.out) + (size_t)m * a.N_out + n0) = o;
       }
       return;
@@ -437,11 +509,13 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
     const float sx = rms(mloc);
 #pragma unroll
     for (int i = 0; i < OF; ++i) {
-      const int n0 = nw + i * 16 + 4 * g;
+      const int n0 = nw + i * FF + LF * g;
       if (n0 >= a.N_out) continue;
       float v[4];
       value(i, j, n0, sx, v);
-      if constexpr (EPI == P4_F32) {
+      if constexpr (MIX) {
+        *reinterpret_cast<uint32_t*>(reinterpret_cast<bf16_t*>(a.out) + (size_t)m * a.N_out + n0) = pack_bf2(v[0], v[1]);
+      } else if constexpr (EPI == P4_F32) {
         *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + (size_t)m * a.N_out + n0) =
             f32x4{v[0], v[1], v[2], v[3]};
       } else {
@@ -535,23 +609,25 @@ using namespace k8sllm;
 
 namespace {
 struct P4Cfg {
-  int fp, fq;
+  int fp, fq, dw, dx;
 };
 // tile configurations: BP = 32 FP weight rows x BQ = 32 FQ tokens, 4 waves of (BP / 2) x (BQ / 2)
 constexpr P4Cfg kP4Cfgs[] = {
-    {8, 8},   // 0: 256 x 256
-    {8, 4},   // 1: 256 x 128
-    {4, 8},   // 2: 128 x 256
-    {4, 4},   // 3: 128 x 128
-    {8, 8},   // 4: as 0 (saved plans name it)
-    {4, 2},   // 5: 128 x 64
-    {2, 2},   // 6: 64 x 64
+    {8, 8, 2, 1},   // 0: 256 x 256
+    {8, 4, 2, 1},   // 1: 256 x 128
+    {4, 8, 2, 1},   // 2: 128 x 256
+    {4, 4, 2, 1},   // 3: 128 x 128
+    {8, 8, 2, 1},   // 4: as 0 (saved plans name it)
+    {4, 2, 2, 1},   // 5: 128 x 64
+    {2, 2, 4, 4},   // 6: 64 x 64
+    {7, 8, 2, 1},   // 7: 224 x 256
+    {8, 6, 2, 1},   // 8: 256 x 192
 };
 constexpr int kP4NumCfgs = sizeof(kP4Cfgs) / sizeof(kP4Cfgs[0]);
 
 template <int C, int EPI, bool RMS>
 int p4_launch(const P4Args& a, hipStream_t s) {
-  hipLaunchKernelGGL((pgemm4_kernel<kP4Cfgs[C].fp, kP4Cfgs[C].fq, EPI, RMS>), dim3(a.nwg),
+  hipLaunchKernelGGL((pgemm4_kernel<kP4Cfgs[C].fp, kP4Cfgs[C].fq, kP4Cfgs[C].dw, kP4Cfgs[C].dx, EPI, RMS>), dim3(a.nwg),
                      dim3(256), 0, s, a);
   return (int)hipGetLastError();
 }
@@ -635,7 +711,7 @@ extern "C" int k8s_pgemm_reduce(void* out, const void* res, const float* slab, i
 // The forms with an activation (gated kinds 0, 1, 5; elementwise 7) and the grouped ones.
 template <int C, int EPI, bool GRP, int KIND>
 int p4_act_launch(const P4Args& a, hipStream_t s) {
-  hipLaunchKernelGGL((pgemm4_kernel<kP4Cfgs[C].fp, kP4Cfgs[C].fq, EPI, false, GRP, KIND>), dim3(a.nwg),
+  hipLaunchKernelGGL((pgemm4_kernel<kP4Cfgs[C].fp, kP4Cfgs[C].fq, kP4Cfgs[C].dw, kP4Cfgs[C].dx, EPI, false, GRP, KIND>), dim3(a.nwg),
                      dim3(256), 0, s, a);
   return (int)hipGetLastError();
 }
@@ -672,6 +748,7 @@ P4Args p4_args(void* out, const void* x, const void* W, int M, int N_out, int K,
   a.splits = 1;
   a.group_m = group_m > 0 ? group_m : 1;
   a.nwg = a.m_tiles * a.n_tiles;
+  a.spread = a.m_tiles == 1;
   a.wide = N_out % 8 == 0 && ((uintptr_t)out & 15) == 0;
   return a;
 }
@@ -682,7 +759,7 @@ extern "C" int k8s_pgemm4_config(int cfg, int* bp, int* bq, int* lds_bytes) {
   if (cfg < 0 || cfg >= kP4NumCfgs) return -1;
   *bp = 32 * kP4Cfgs[cfg].fp;
   *bq = 32 * kP4Cfgs[cfg].fq;
-  *lds_bytes = (3 * *bp + 2 * *bq) * 128;
+  *lds_bytes = ((kP4Cfgs[cfg].dw + 1) * *bp + (kP4Cfgs[cfg].dx + 1) * *bq) * 128;
   return 0;
 }
 
@@ -714,7 +791,7 @@ extern "C" int k8s_pgemm4(void* out, float* slab, const void* x, const void* W, 
   if (res != nullptr && epi != P4_BF16) return -6;
   const int bp = 32 * kP4Cfgs[cfg].fp, bq = 32 * kP4Cfgs[cfg].fq;
   const int feat = epi == P4_SWIGLU ? bp / 2 : bp;
-  P4Args a;
+  P4Args a = {};
   a.out = out;
   a.res = static_cast<const bf16_t*>(res);
   a.slab = slab;
@@ -733,6 +810,7 @@ extern "C" int k8s_pgemm4(void* out, float* slab, const void* x, const void* W, 
   a.group_m = group_m > 0 ? group_m : 1;
   a.nwg = nwg;
   a.eps = eps;
+  a.spread = a.m_tiles == 1;
   a.wide = res == nullptr && N_out % 8 == 0 && ((uintptr_t)out & 15) == 0;
   int rc = p4_cfg(a, cfg, epi, rms, stream);
   if (rc != 0 || splits == 1) return rc;
@@ -763,6 +841,8 @@ extern "C" int k8s_pgemm4_act(void* out, const void* x, const void* W, int M, in
     case 4: return p4_act_kind<4, false>(a, kind, stream);
     case 5: return p4_act_kind<5, false>(a, kind, stream);
     case 6: return p4_act_kind<6, false>(a, kind, stream);
+    case 7: return p4_act_kind<7, false>(a, kind, stream);
+    case 8: return p4_act_kind<8, false>(a, kind, stream);
   }
   return -4;
 }
@@ -782,6 +862,7 @@ extern "C" int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M
   P4Args a = p4_args(out, x, W, rows, N_out, K, pair, cfg, group_m);
   const int bq = 32 * kP4Cfgs[cfg].fq;
   a.m_tiles = rows / bq + groups;        // whole tiles, and a partial one per group
+  a.spread = groups >= 8 && rows <= 192LL * groups;
   if ((long long)a.m_tiles * a.n_tiles > (1LL << 30)) return -1;
   a.nwg = a.m_tiles * a.n_tiles;
   a.xbytes = (uint32_t)(ldx * 2);
@@ -798,6 +879,8 @@ extern "C" int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M
     case 3: return p4_act_kind<3, true>(a, kind, stream);
     case 5: return p4_act_kind<5, true>(a, kind, stream);
     case 6: return p4_act_kind<6, true>(a, kind, stream);
+    case 7: return p4_act_kind<7, true>(a, kind, stream);
+    case 8: return p4_act_kind<8, true>(a, kind, stream);
   }
   return p4_act_kind<4, true>(a, kind, stream);
 }

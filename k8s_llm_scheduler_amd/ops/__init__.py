@@ -994,17 +994,19 @@ def _pg_load_table() -> dict:
 # Time of a bf16 plan on pgemm4.hip in us, configuration -> (per round of tiles over the CUs and 64-deep k-step, per round, per
 # k-step, split, per MB of slab, per MB of weights, per MB of output): the tiles' k-steps, of which workgroups that share a CU
 # hide part from each other; with split-K the combine launch and the slabs it moves; the weights and the output.  Fitted to 22
-# weight shapes (576 x 2048 .. 28672 x 4096) at 12 row counts (40 .. 2048), weights cold: rms error 6 - 10 % per configuration,
-# the pick within 2 % of the best plan on average and 21 % at most, the same as hipBLASLt on average (0.92 - 1.09 of its time
-# by row count).  pgemm.hip's 8-wave tiles were the best plan of none of these; the tuned table names them for some of the 70B's
-# products of 192 - 8192 rows and its logits, and SwiGLU and fp8 products that it does not list take them (_pgemm_big_tiles).
-_P4_COST = {1: (0.657, 2.23, 0.0, 5.7, 0.302, 0.0684, 0.367),
-            2: (0.599, 2.19, 0.0, 4.12, 0.34, 0.0527, 0.514),
-            3: (0.297, 0.0, 0.155, 5.46, 0.348, 0.0739, 0.635),
-            4: (1.01, 5.43, 0.0, 4.18, 0.304, 0.0306, 0.436),
-            5: (0.234, 0.173, 0.137, 4.94, 0.298, 0.0902, 0.687),
-            6: (0.152, 0.231, 0.173, 4.37, 0.203, 0.0883, 0.245)}
-_P4_COST_T0 = {1: 0.0, 2: 1.09, 3: 0.218, 4: 1.5, 5: 0.0, 6: 0.599}
+# weight shapes (576 x 2048 .. 28672 x 4096) at 12 row counts (130 .. 2048), weights cold: rms error 5 - 10 % per configuration,
+# the pick within 1 % of the best plan on average and 18 % at most, 6 % faster on average than the rule for the six tiles there
+# were (64 x 64 then two stages ahead), 7 % slower at most (256 x 6144 x 3072) but for 14 % at 256 x 2048 x 8192.  pgemm.hip's 8-wave tiles were the best plan of none of these; the tuned table names them for some of the 70B's
+# products of 256 - 8192 rows and its logits, and SwiGLU and fp8 products that it does not list take them (_pgemm_big_tiles).
+_P4_COST = {1: (0.652, 2.2, 0.0, 5.33, 0.24, 0.066, 0.305),
+            2: (0.652, 2.3, 0.0, 4.98, 0.273, 0.0316, 0.345),
+            3: (0.299, 0.0, 0.148, 4.36, 0.307, 0.0852, 0.37),
+            4: (1.06, 7.03, 0.0, 6.75, 0.223, 0.0147, 0.355),
+            5: (0.182, 0.22, 0.199, 4.3, 0.326, 0.0841, 0.735),
+            6: (0.177, 0.0, 0.0115, 2.41, 0.413, 0.0816, 0.257),
+            7: (0.943, 5.56, 0.0, 5.98, 0.238, 0.0159, 0.346),
+            8: (0.823, 4.47, 0.0, 6.41, 0.219, 0.0347, 0.326)}
+_P4_COST_T0 = {1: 2.16, 2: 1.46, 3: 2.25, 4: 0.0, 5: 0.34, 6: 2.9, 7: 0.298, 8: 1.16}
 
 
 @functools.lru_cache(maxsize=4096)

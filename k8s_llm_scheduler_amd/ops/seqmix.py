@@ -354,14 +354,15 @@ def _grouped_big(a: torch.Tensor, w: torch.Tensor, seg: Optional[torch.Tensor], 
 
 
 # Time of a grouped product in us, configuration -> (fixed, per round of tiles over the CUs and 64-deep k-step, per round, per
-# k-step, per MB of weights, per MB of output, per round and 65536 outputs of a gated activation).  Fitted to 8 products of 1 -
-# 16 groups, 512 x 4096 .. 2 x 3584 x 4096, 2 - 2048 rows per group, weights cold: rms error 5 - 11 % per configuration.  Over 8
-# other products (4 - 16 groups drawn at random, 1024 x 2048 .. 2 x 3584 x 4096, 18 row counts of 128 - 4096) the pick is within 1.5 % of the best configuration on
-# average, 35 % at most.  _GROUP_TILE: weight rows and tokens of a tile.
-_GROUP_TILE = {1: (256, 128), 2: (128, 256), 3: (128, 128), 4: (256, 256), 5: (128, 64), 6: (64, 64)}
-_GROUP_COST = {1: (0.0, 0.524, 4.92, 0.0, 0.11, 0.424, 6.72), 2: (0.0, 0.542, 4.91, 0.0, 0.0696, 0.486, 9.86),
-               3: (3.28, 0.379, 0.0, 0.0254, 0.0878, 0.27, 11.6), 4: (0.0, 0.864, 8.67, 0.0, 0.0913, 0.323, 8.6),
-               5: (2.67, 0.304, 0.0, 0.0345, 0.0953, 0.174, 16.3), 6: (2.29, 0.176, 0.0, 0.16, 0.0834, 0.076, 15.8)}
+# k-step, per MB of weights, per MB of output, per round and 65536 outputs of a gated activation).  Fitted to 10 products of 4 -
+# 16 groups, 2048 x 1024 .. 2 x 3584 x 4096, 4 - 768 rows per group drawn at random, weights cold: rms error 4 - 8 % per
+# configuration, the pick within 1 % of the best configuration on average, 23 % at most, and 7 % faster on average than the pick of
+# the six tiles there were.  _GROUP_TILE: weight rows and tokens of a tile.
+_GROUP_TILE = {1: (256, 128), 2: (128, 256), 3: (128, 128), 4: (256, 256), 5: (128, 64), 6: (64, 64), 7: (224, 256), 8: (256, 192)}
+_GROUP_COST = {1: (0.0, 0.632, 2.7, 0.0, 0.0957, 0.701, 3.45), 2: (1.58, 0.488, 5.91, 0.0, 0.0921, 0.574, 8.35),
+               3: (4.05, 0.397, 0.0, 0.0266, 0.0876, 0.397, 3.35), 4: (0.0, 0.897, 8.92, 0.0, 0.0896, 0.484, 5.54),
+               5: (2.99, 0.317, 0.0, 0.0184, 0.103, 0.324, 4.53), 6: (0.417, 0.164, 0.608, 0.0738, 0.105, 0.636, 1.43),
+               7: (0.0, 0.849, 7.16, 0.0, 0.0733, 0.465, 3.83), 8: (0.0, 0.762, 4.85, 0.0, 0.0828, 0.515, 2.92)}
 
 
 @functools.lru_cache(maxsize=4096)

@@ -1,0 +1,85 @@
+"""The 4-wave big-tile products with deeper rings, 224- and 192-wide tiles and the XCDs spread over k: whole numbers, so that every
+sum is exact in any order, and bf16 results where they are; rows that do not fill the tile, one stage to more than the ring holds."""
+import pytest
+import torch
+
+from k8s_llm_scheduler_amd import ops
+from k8s_llm_scheduler_amd.ops import seqmix as sm
+
+pytestmark = pytest.mark.gpu
+TILES = {0: (256, 256), 1: (256, 128), 2: (128, 256), 3: (128, 128), 5: (128, 64), 6: (64, 64), 7: (224, 256), 8: (256, 192)}
+
+
+def whole(n, K, seed):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.randint(-3, 4, (n, K), generator=g) * (torch.rand(n, K, generator=g) < 0.15)).to(torch.bfloat16).cuda()
+
+
+def out_of(M, N, shift=0):
+    buf = torch.full((M * N + 64,), 7.0, dtype=torch.bfloat16, device="cuda")
+    return buf, buf[shift:shift + M * N].view(M, N)
+
+
+def untouched(buf, M, N, shift=0):
+    return bool((buf[:shift] == 7).all() and (buf[shift + M * N:] == 7).all())
+
+
+@pytest.mark.parametrize("cfg", sorted(TILES))
+@pytest.mark.parametrize("stages", [1, 2, 3, 4, 5, 6, 7, 9, 13])
+def test_stages_of_every_ring(cfg, stages):
+    """One row tile (every XCD begins at its own stage and wraps) and two (all begin at the first)."""
+    bp, bq = TILES[cfg]
+    K = 64 * stages
+    for M, N, shift in ((1, 8, 0), (bq - 3, bp + 4, 0), (bq, 9 * bp - 8, 0), (bq + 1, bp + 16, 0), (bq - 1, 2 * bp - 4, 4)):
+        x, w = whole(M, K, M + K), whole(N, K, N)
+        want = x.float() @ w.float().T
+        assert want.abs().max() <= 256
+        buf, out = out_of(M, N, shift)
+        ops.native().pgemm4(out.data_ptr(), 0, x.data_ptr(), w.data_ptr(), M, N, K, ops.EPI_BF16, cfg, 1, 4, 0, 0, 0.0, -1)
+        assert torch.equal(out.float(), want) and untouched(buf, M, N, shift), (M, N, shift)
+        assert torch.equal(ops.pgemm4(x, w, ops.EPI_F32, cfg=cfg), want), (M, N)
+        if stages >= 3:
+            assert torch.equal(ops.pgemm4(x, w, ops.EPI_BF16, cfg=cfg, splits=3).float(), want), (M, N, "split")
+
+
+@pytest.mark.parametrize("cfg", [6, 7, 8])
+@pytest.mark.parametrize("K", [64, 448])
+def test_pairs_and_activations(cfg, K):
+    """Gate and up rows of a feature in one fragment (224 rows) or in two; columns that do not fill the tile, a bias, split k."""
+    bp, bq = TILES[cfg]
+    for M, N, shift in ((bq - 1, bp // 2 + 8, 0), (bq + 5, bp // 2 - 4, 0), (17, bp + 12, 4), (3, 4, 0)):
+        x, w = whole(M, K, M), whole(2 * N, K, N + 1)
+        b = torch.randint(-2, 3, (2 * N,), generator=torch.Generator().manual_seed(N)).to(torch.bfloat16).cuda()
+        y = x.float() @ w.float().T
+        for bias in (None, b):
+            z = y if bias is None else y + b.float()
+            buf, out = out_of(M, N, shift)
+            ops.native().pgemm4_act(out.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K, cfg, 4, sm.ACT_RELU, 0.0, 1.0,
+                                    0 if bias is None else b.data_ptr(), -1)
+            assert torch.equal(out, (z[:, :N].clamp(min=0) * z[:, N:]).to(torch.bfloat16)) and untouched(buf, M, N, shift), (M, N)
+        x = x + 1
+        y = (x.double() @ w.double().T) * (x.double().square().mean(1, keepdim=True) + 1e-5).rsqrt()
+        want = torch.nn.functional.silu(y[:, :N]) * y[:, N:]
+        for splits in (1, 2) if K > 64 else (1,):
+            got = ops.pgemm4(x, w, ops.EPI_SWIGLU, cfg=cfg, splits=splits, rms_eps=1e-5).double()
+            # a rounding to bf16; the gate's exponential and division, |y| <= 60: its argument's error 60 x 2^-22
+            assert ((got - want).abs() <= want.abs() * (2.0 ** -8 + 2.0 ** -14) + 1e-6).all(), (M, N, splits)
+
+
+@pytest.mark.parametrize("sizes", [(64, 65, 0, 63, 1, 128, 200, 10), tuple([40] * 7 + [0, 3])])
+@pytest.mark.parametrize("cfg", [1, 6, 7, 8])
+@pytest.mark.parametrize("kind", [None, sm.ACT_RELU])
+def test_groups_spread_over_k(sizes, cfg, kind, monkeypatch):
+    """8 and more groups of few rows: every XCD at its own stage; gathered rows."""
+    monkeypatch.setattr(sm, "_grouped_tile", lambda *a: cfg)
+    E, P, N, K = len(sizes), sum(sizes), 264, 576
+    seg = torch.tensor((0,) + sizes).cumsum(0).to(torch.int32).cuda()
+    x, w = whole(70, K, P), whole(E * N * (1 if kind is None else 2), K, cfg).view(E, -1, K)
+    rows = torch.randint(0, 70, (P,), generator=torch.Generator().manual_seed(P)).to(torch.int32).cuda()
+    tiles = torch.full((1, 3), -1, dtype=torch.int32, device="cuda")
+    kw = dict(a_rows=rows, tiles=tiles, rows=P, seg=seg)
+    assert sm._grouped_big(x, w, seg, P, N)
+    got = sm.gemm(x, w, **kw) if kind is None else sm.gemm_act(x, w, kind, 0.0, 1.0, **kw)
+    y = torch.cat([x[rows[int(seg[e]):int(seg[e + 1])].long()].float() @ w[e].float().T for e in range(E)])
+    want = y if kind is None else y[:, :N].clamp(min=0) * y[:, N:]
+    assert torch.equal(got, want.to(torch.bfloat16))
