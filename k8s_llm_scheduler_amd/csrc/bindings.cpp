@@ -116,7 +116,9 @@ int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M, int rows,
                        const int* a_rows, long ldx, int cfg, int group_m, int kind, float limit, float alpha,
                        hipStream_t stream);
 int k8s_pgemm4(void* out, float* slab, const void* x, const void* W, int M, int N_out, int K, int epi, int cfg,
-               int splits, int group_m, const void* res, int rms, float eps, hipStream_t s);
+               int splits, int group_m, const void* res, int rms, float eps, const float* scale, hipStream_t s);
+int k8s_pgemm4_scaled(int cfg);
+int k8s_row_scale(float* out, const void* x, int M, int K, float eps, hipStream_t s);
 int k8s_embed_rows(float* out, void* copy, const int* ids, const void* table, int T, int W, int vocab, float scale,
                    int f32, hipStream_t s);
 int k8s_decode_meta(int* pos, int* slots, int* ar, const int* ctx, const int* block_tables, int max_blocks, int B, int bs,
@@ -846,8 +848,15 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
   });
   m.def("pgemm4", [](uintptr_t out, uintptr_t slab, uintptr_t x, uintptr_t W, int M, int N, int K, int epi, int cfg,
                      int splits, int group_m, uintptr_t res, int rms, float eps, int64_t s) {
-    check(k8s_pgemm4(P(out), P<float>(slab), P(x), P(W), M, N, K, epi, cfg, splits, group_m, P(res), rms, eps, S(s)),
+    check(k8s_pgemm4(P(out), P<float>(slab), P(x), P(W), M, N, K, epi, cfg, splits, group_m, P(res), rms, eps, nullptr, S(s)),
           "pgemm4");
+  });
+  m.def("pgemm4_scaled_ok", [](int cfg) { return k8s_pgemm4_scaled(cfg) != 0; });
+  m.def("pgemm4_scaled", [](uintptr_t out, uintptr_t slab, uintptr_t x, uintptr_t W, int M, int N, int K, int epi, int cfg,
+                            int splits, int group_m, uintptr_t res, uintptr_t scale, float eps, int64_t s) {
+    check(k8s_row_scale(P<float>(scale), P(x), M, K, eps, S(s)), "row_scale");
+    check(k8s_pgemm4(P(out), P<float>(slab), P(x), P(W), M, N, K, epi, cfg, splits, group_m, P(res), 1, eps, P<float>(scale),
+                     S(s)), "pgemm4_scaled");
   });
   m.def("pgemm_configs", []() {
     py::list out;

@@ -50,6 +50,7 @@ namespace k8sllm {
 
 namespace {
 enum { P4_BF16 = 0, P4_F32 = 1, P4_SWIGLU = 2, P4_GLU = 3, P4_ACT = 4 };   // GLU, ACT: bf16 out, activation KIND
+enum { P4_PLAIN = 0, P4_RMS = 1, P4_SCALED = 2 };   // rows as they are; 1 / rms from a prologue in the k loop; from P4Args::scale
 typedef __attribute__((ext_vector_type(2))) uint32_t p4_u32x2;
 typedef __attribute__((ext_vector_type(2))) float p4_f32x2;
 
@@ -89,6 +90,7 @@ struct P4Args {
   int M, N_out, half_rows, wrows, K;
   int m_tiles, n_tiles, ks, splits, group_m, nwg;
   float eps;
+  const float* scale;    // P4_SCALED: 1 / rms of every token's row
   int spread;            // the XCDs start their walk over k an eighth of it apart
   int wide;              // the output's rows can be stored in 16-byte pieces
   float limit, alpha;    // P4_GLU: of the gated kind
@@ -106,13 +108,14 @@ struct P4Args {
   int groups;
 };
 
-template <int FP, int FQ, int DW, int DX, int EPI, bool RMS, bool GRP = false, int KIND = -1>
+template <int FP, int FQ, int DW, int DX, int EPI, int NORM, bool GRP = false, int KIND = -1>
 __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
+  constexpr bool RMS = NORM == P4_RMS;
   static_assert(DW == DX || DW == DX + 1, "a stage's last load is followed by whole stages of later ones");
   constexpr int BP = 32 * FP, BQ = 32 * FQ;          // weight rows, tokens per tile (2 x 2 waves)
   constexpr bool PAIR = EPI == P4_SWIGLU || EPI == P4_GLU;   // gate and up rows of one feature in one wave
   constexpr bool MIX = PAIR && FP % 2 != 0;          // ... and in one fragment: a lane's four rows are gate, gate, up, up
-  static_assert(!GRP || !RMS, "the grouped form has no prologue");
+  static_assert(!GRP || NORM == P4_PLAIN, "the grouped form has no prologue");
   constexpr int SUBW = BP * 128, SUBX = BQ * 128;    // a 64-deep stage of either operand
   constexpr int GW = BP / 32, GX = BQ / 32;          // 16-byte DMA instructions per thread and stage
   constexpr int X0 = (DW + 1) * SUBW, RING = X0 + (DX + 1) * SUBX;
@@ -426,6 +429,7 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
   constexpr int FF = MIX ? 8 : 16, LF = FF / 4;      // features of one, and of a lane in it
   auto rms = [&](int mloc) -> float {
     if constexpr (RMS) return rsqrtf(rss[mloc] / (float)a.K + a.eps);
+    else if constexpr (NORM == P4_SCALED) return a.scale[min(m0 + mloc, m_end - 1)];
     else return 1.f;
   };
   // the LF features of fragments (i, j): the sums with their scale, bias and activation
@@ -564,7 +568,7 @@ __global__ void __launch_bounds__(256) pgemm_reduce_kernel(void* __restrict__ ou
     for (int k = 0; k < splits; ++k) t += slab[(size_t)splits * stride + (size_t)k * M + m];
     sx = rsqrtf(t / (float)K + eps);
   }
-  if (FP8 && xs != nullptr) sx *= xs[m];
+  if (xs != nullptr) sx *= xs[m];   // fp8: the token's scale; bf16: 1 / rms of its row
   float v[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -603,6 +607,21 @@ __global__ void __launch_bounds__(256) pgemm_reduce_kernel(void* __restrict__ ou
   }
 }
 
+// 1 / rms of every row of x [M][K] (K a multiple of 8, rows 16-byte aligned), a workgroup per row.
+__global__ void __launch_bounds__(256) row_scale_kernel(float* __restrict__ out, const bf16_t* __restrict__ x, int K, float eps) {
+  __shared__ float red[16];
+  const u32x4* row = reinterpret_cast<const u32x4*>(x + (size_t)blockIdx.x * K);
+  float s = 0.f;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < K / 8; i += 256) {
+    const u32x4 v = row[i];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s += lo_bf(v[e]) * lo_bf(v[e]) + hi_bf(v[e]) * hi_bf(v[e]);
+  }
+  s = block_sum(s, red);
+  if (threadIdx.x == 0) out[blockIdx.x] = rsqrtf(s / (float)K + eps);
+}
+
 }  // namespace k8sllm
 
 using namespace k8sllm;
@@ -625,25 +644,32 @@ constexpr P4Cfg kP4Cfgs[] = {
 };
 constexpr int kP4NumCfgs = sizeof(kP4Cfgs) / sizeof(kP4Cfgs[0]);
 
-template <int C, int EPI, bool RMS>
+template <int C, int EPI, int NORM>
 int p4_launch(const P4Args& a, hipStream_t s) {
-  hipLaunchKernelGGL((pgemm4_kernel<kP4Cfgs[C].fp, kP4Cfgs[C].fq, kP4Cfgs[C].dw, kP4Cfgs[C].dx, EPI, RMS>), dim3(a.nwg),
+  hipLaunchKernelGGL((pgemm4_kernel<kP4Cfgs[C].fp, kP4Cfgs[C].fq, kP4Cfgs[C].dw, kP4Cfgs[C].dx, EPI, NORM>), dim3(a.nwg),
                      dim3(256), 0, s, a);
   return (int)hipGetLastError();
 }
+// row scales that are given: the tiles of large products only
+constexpr bool p4_scaled(int cfg) { return kP4Cfgs[cfg].fp * kP4Cfgs[cfg].fq >= 32; }
 template <int C>
-int p4_epi(const P4Args& a, int epi, int rms, hipStream_t s) {
-  if (rms) {
+int p4_epi(const P4Args& a, int epi, int norm, hipStream_t s) {
+  if (norm == P4_SCALED) {
+    if constexpr (p4_scaled(C)) {
+      if (epi == P4_BF16) return p4_launch<C, P4_BF16, P4_SCALED>(a, s);
+      if (epi == P4_SWIGLU) return p4_launch<C, P4_SWIGLU, P4_SCALED>(a, s);
+    }
+  } else if (norm == P4_RMS) {
     switch (epi) {
-      case P4_BF16: return p4_launch<C, P4_BF16, true>(a, s);
-      case P4_F32: return p4_launch<C, P4_F32, true>(a, s);
-      case P4_SWIGLU: return p4_launch<C, P4_SWIGLU, true>(a, s);
+      case P4_BF16: return p4_launch<C, P4_BF16, P4_RMS>(a, s);
+      case P4_F32: return p4_launch<C, P4_F32, P4_RMS>(a, s);
+      case P4_SWIGLU: return p4_launch<C, P4_SWIGLU, P4_RMS>(a, s);
     }
   } else {
     switch (epi) {
-      case P4_BF16: return p4_launch<C, P4_BF16, false>(a, s);
-      case P4_F32: return p4_launch<C, P4_F32, false>(a, s);
-      case P4_SWIGLU: return p4_launch<C, P4_SWIGLU, false>(a, s);
+      case P4_BF16: return p4_launch<C, P4_BF16, P4_PLAIN>(a, s);
+      case P4_F32: return p4_launch<C, P4_F32, P4_PLAIN>(a, s);
+      case P4_SWIGLU: return p4_launch<C, P4_SWIGLU, P4_PLAIN>(a, s);
     }
   }
   return -2;
@@ -711,7 +737,7 @@ extern "C" int k8s_pgemm_reduce(void* out, const void* res, const float* slab, i
 // The forms with an activation (gated kinds 0, 1, 5; elementwise 7) and the grouped ones.
 template <int C, int EPI, bool GRP, int KIND>
 int p4_act_launch(const P4Args& a, hipStream_t s) {
-  hipLaunchKernelGGL((pgemm4_kernel<kP4Cfgs[C].fp, kP4Cfgs[C].fq, kP4Cfgs[C].dw, kP4Cfgs[C].dx, EPI, false, GRP, KIND>), dim3(a.nwg),
+  hipLaunchKernelGGL((pgemm4_kernel<kP4Cfgs[C].fp, kP4Cfgs[C].fq, kP4Cfgs[C].dw, kP4Cfgs[C].dx, EPI, P4_PLAIN, GRP, KIND>), dim3(a.nwg),
                      dim3(256), 0, s, a);
   return (int)hipGetLastError();
 }
@@ -753,6 +779,8 @@ P4Args p4_args(void* out, const void* x, const void* W, int M, int N_out, int K,
   return a;
 }
 
+extern "C" int k8s_pgemm4_scaled(int cfg) { return cfg >= 0 && cfg < kP4NumCfgs && p4_scaled(cfg); }
+
 extern "C" int k8s_pgemm4_num_configs() { return kP4NumCfgs; }
 
 extern "C" int k8s_pgemm4_config(int cfg, int* bp, int* bq, int* lds_bytes) {
@@ -779,8 +807,17 @@ extern "C" int k8s_pgemm4_plan(int M, int N_out, int K, int epi, int cfg, int sp
   return 0;
 }
 
+extern "C" int k8s_row_scale(float* out, const void* x, int M, int K, float eps, hipStream_t stream) {
+  if (M < 0 || K <= 0 || K % 8 || ((uintptr_t)x & 15)) return -1;
+  if (M == 0) return 0;
+  hipLaunchKernelGGL(row_scale_kernel, dim3(M), dim3(256), 0, stream, out, static_cast<const bf16_t*>(x), K, eps);
+  return (int)hipGetLastError();
+}
+
+// scale [M] fp32 (optional; bf16 and SwiGLU epilogues, tiles of k8s_pgemm4_scaled): 1 / rms of the rows of x, not from a prologue.
 extern "C" int k8s_pgemm4(void* out, float* slab, const void* x, const void* W, int M, int N_out, int K, int epi,
-                          int cfg, int splits, int group_m, const void* res, int rms, float eps, hipStream_t stream) {
+                          int cfg, int splits, int group_m, const void* res, int rms, float eps, const float* scale,
+                          hipStream_t stream) {
   int nwg;
   long long nsl;
   if (k8s_pgemm4_plan(M, N_out, K, epi, cfg, splits, &nwg, &nsl) != 0) return -1;
@@ -810,11 +847,13 @@ extern "C" int k8s_pgemm4(void* out, float* slab, const void* x, const void* W, 
   a.group_m = group_m > 0 ? group_m : 1;
   a.nwg = nwg;
   a.eps = eps;
+  a.scale = scale;
   a.spread = a.m_tiles == 1;
   a.wide = res == nullptr && N_out % 8 == 0 && ((uintptr_t)out & 15) == 0;
-  int rc = p4_cfg(a, cfg, epi, rms, stream);
+  if (scale != nullptr && splits > 1) a.scale = nullptr;   // the sums of the slices are scaled by the combine
+  int rc = p4_cfg(a, cfg, epi, a.scale != nullptr ? P4_SCALED : scale == nullptr && rms ? P4_RMS : P4_PLAIN, stream);
   if (rc != 0 || splits == 1) return rc;
-  return k8s_pgemm_reduce(out, res, slab, splits, M, N_out, K, epi, rms, eps, nullptr, nullptr, nullptr, nullptr,
+  return k8s_pgemm_reduce(out, res, slab, splits, M, N_out, K, epi, scale == nullptr && rms, eps, scale, nullptr, nullptr, nullptr,
                           stream);
 }
 

@@ -941,6 +941,13 @@ def pgemm4_tiles(cfg: int, M: int, N: int, epi: int) -> int:
     return math.ceil(N / feat) * math.ceil(M / bq)
 
 
+# From this many operations on, the rows' 1 / rms is taken in a pass of its own ahead of a big-tile product: in the product every
+# column of tiles squares the same rows again, 4 - 5 % of its time (us, prologue / pass and product: 3413 x 2 x 28672 x 8192 2544 /
+# 2444, 3413 x 10240 x 8192 422 / 415 on the 256 x 192 tile, 520 / 488 on 128 x 256); shorter ones do not repay the launch (241 x 2 x
+# 28672 x 8192 202 / 201, 512 x 2 x 14336 x 4096 97 / 96, 1024 x 6144 x 4096 53.4 / 57.5).
+P4_SCALE_FLOPS = 4e11
+
+
 def pgemm4(x: torch.Tensor, w: torch.Tensor, epi: int = EPI_BF16, cfg: int = 0, splits: int = 1, group_m: int = 4,
            res: Optional[torch.Tensor] = None, rms_eps: Optional[float] = None,
            out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -956,8 +963,14 @@ def pgemm4(x: torch.Tensor, w: torch.Tensor, epi: int = EPI_BF16, cfg: int = 0, 
     slab = torch.empty(n_slab, dtype=F32, device=x.device) if n_slab > 0 else None
     rp = _chk(res, BF16, "res") if res is not None else 0
     rms, eps = (1, float(rms_eps)) if rms_eps is not None else (0, 0.0)
-    native().pgemm4(out.data_ptr(), slab.data_ptr() if slab is not None else 0, _chk(x, BF16, "x"), _chk(w, BF16, "w"),
-                    M, N, K, epi, cfg, splits, group_m, rp, rms, eps, -1)
+    sp = slab.data_ptr() if slab is not None else 0
+    if rms and 2.0 * M * w.shape[0] * K >= P4_SCALE_FLOPS and epi != EPI_F32 and native().pgemm4_scaled_ok(cfg):
+        scale = torch.empty(M, dtype=F32, device=x.device)
+        native().pgemm4_scaled(out.data_ptr(), sp, _chk(x, BF16, "x"), _chk(w, BF16, "w"), M, N, K, epi, cfg, splits, group_m,
+                               rp, scale.data_ptr(), eps, -1)
+    else:
+        native().pgemm4(out.data_ptr(), sp, _chk(x, BF16, "x"), _chk(w, BF16, "w"), M, N, K, epi, cfg, splits, group_m, rp,
+                        rms, eps, -1)
     del slab
     return out
 
