@@ -336,11 +336,15 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out_dtype=None, *, a_rows: Optional[t
     return out
 
 
-# Grouped bf16 products of at least GROUP_BIG_MIN rows per group on average (whole rows of at least 64 elements) run on the
-# big-tile kernel (pgemm4.hip).  8 groups, N = K = 2048, 8 / 16 / 32 / 96 / 192 / 512 rows per group, weights from memory: 20 /
-# 20 / 20 / 22 / 24 / 46 us, past the LDS (gemm_group_kernel) 18 / 22 / 31 us; gate / up with the activation in its epilogue
-# (N = 2 x 2048), 16 / 32 / 96 / 192 / 512 rows: 33 / 33 / 36 / 41 / 89 us, 37 / 44 us.  Fewer rows stream the weights past the LDS.
-GROUP_BIG_MIN = 16
+# Grouped bf16 products of at least GROUP_BIG_MIN rows per group on average (GROUP_BIG_MIN_FEW of up to 8 groups; whole rows of at
+# least 64 elements) run on the big-tile kernel (pgemm4.hip); fewer stream the weights past the LDS (gemm_group_kernel), whose time
+# goes with the groups that have rows.  us, weights from memory, past the LDS / big tiles: gate / up of 8 groups with the activation
+# (2 x 2048 x 2048), 0.5 / 1 / 2 / 4 / 8 / 16 rows per group 17.1 / 19.0, 23.3 / 22.6, 29.8 / 26.1, 34.7 / 28.2, 33.7 / 28.4, 41.9 /
+# 28.4; down (2048 x 2048) 8.8 / 10.8, 12.8 / 13.2, 16.7 / 15.1, 18.5 / 17.1, 19.0 / 17.2, 23.0 / 16.2; 8 of 4096 x 3584, 1 / 2 / 8 31.5 /
+# 40.7, 42.0 / 43.0, 56.3 / 47.9; 16 of 2 x 2048 x 4096, 2 / 4 / 6 / 8 91 / 103, 105 / 111, 109 / 110, 112 / 111; 16 of 2048 x 1024, 4 / 6 / 8
+# 15.6 / 17.1, 16.4 / 16.9, 17.8 / 17.1.
+GROUP_BIG_MIN = 6
+GROUP_BIG_MIN_FEW = 2
 GROUP_BIG_MAX_GROUPS = 64        # every workgroup walks the groups' offsets
 
 
@@ -348,7 +352,7 @@ def _grouped_big(a: torch.Tensor, w: torch.Tensor, seg: Optional[torch.Tensor], 
     E, _, K = w.shape
     return (not _ops.LEAN and FAST_GEMM and a.dtype == BF16 and seg is not None and seg.is_cuda and seg.dtype == I32
             and seg.is_contiguous() and seg.numel() == E + 1 and E <= GROUP_BIG_MAX_GROUPS
-            and rows >= GROUP_BIG_MIN * E and K % 64 == 0 and N % 4 == 0 and N >= 128 and a.dim() == 2 and a.stride(1) == 1
+            and rows >= (GROUP_BIG_MIN if E > 8 else GROUP_BIG_MIN_FEW) * E and K % 64 == 0 and N % 4 == 0 and N >= 128 and a.dim() == 2 and a.stride(1) == 1
             and a.stride(0) >= K and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.is_contiguous()
             and w.data_ptr() % 16 == 0 and w.shape[1] * K * 2 < 1 << 32 and a.shape[0] * a.stride(0) * 2 < 1 << 32)
 

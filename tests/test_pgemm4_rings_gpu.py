@@ -66,7 +66,7 @@ def test_pairs_and_activations(cfg, K):
             assert ((got - want).abs() <= want.abs() * (2.0 ** -8 + 2.0 ** -14) + 1e-6).all(), (M, N, splits)
 
 
-@pytest.mark.parametrize("sizes", [(64, 65, 0, 63, 1, 128, 200, 10), tuple([40] * 7 + [0, 3])])
+@pytest.mark.parametrize("sizes", [(1, 0, 3, 2, 7, 0, 5, 2), (64, 65, 0, 63, 1, 128, 200, 10), tuple([40] * 7 + [0, 3])])
 @pytest.mark.parametrize("cfg", [1, 6, 7, 8])
 @pytest.mark.parametrize("kind", [None, sm.ACT_RELU])
 def test_groups_spread_over_k(sizes, cfg, kind, monkeypatch):
