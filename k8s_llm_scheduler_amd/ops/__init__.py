@@ -1048,6 +1048,40 @@ def pgemm_heuristic(M: int, N: int, K: int, epi: int, fp8: bool, num_cus: int = 
     return _pgemm_big_tiles(M, N, K, epi, fp8, num_cus)
 
 
+# The same for 17 - 128 rows (one row tile; weights from memory, every XCD at another part of k), fitted to 19 weight shapes (3648 x
+# 2048 .. 57344 x 8192) at 12 row counts: rms error 6 - 7 %, the pick within 3 % of the best plan on average.
+_P4_FEW_COST = {1: (0.66, 3.75, 0.0, 2.1, 0.329, 0.0717, 2.56), 3: (0.477, 0.0, 0.00672, 2.34, 0.382, 0.0575, 4.07),
+                5: (0.269, 0.317, 0.127, 2.31, 0.358, 0.0746, 3.1), 6: (0.187, 0.0, 0.00361, 2.16, 0.459, 0.0779, 3.32)}
+
+
+@functools.lru_cache(maxsize=4096)
+def _few_rows_tile(M: int, rows: int, K: int, epi: int, num_cus: int = 256) -> Optional[Tuple[int, int]]:
+    """(configuration, splits) on pgemm4.hip of a bf16 product of 17 - 128 rows with ``rows`` weight rows, or None: mgemm's.  The
+    4-wave kernel streams large weights faster, since its ring holds more of them in flight and the XCDs spread over k; with small
+    ones mgemm's shorter start counts.  us, mgemm / here: 33 x 10240 x 8192 52 / 40, with the RMS prologue 70 / 38; 65 x 8192 x 8192 51 /
+    34; 128 x 14336 x 4096 42 / 34; 17 x 16384 x 2048 17.3 / 13.9; 128 x 2 x 28672 x 8192 (SwiGLU, RMS) 200 / 177.  Below the lines: 64 x
+    4096 x 2048 9.0 / 10.6, 17 x 8192 x 8192 28.1 / 29.5, 128 x 4096 x 2048 11.9 / 12.4."""
+    if M <= SGEMV_MAX_M or M >= PG_MIN_M or K % 64 or rows % 8 or rows * K * 2 >= 1 << 32:
+        return None
+    mb = rows * K * 2e-6
+    if mb < (20.0 if M > 64 else 30.0 if M > 32 else 60.0) or (M <= 32 and (rows < 12288 or epi == EPI_SWIGLU)):
+        return None
+    kt, best = K // 64, None
+    for cfg, (tile, rnd, step, sp, slab, wmb, t0) in _P4_FEW_COST.items():
+        bp, bq, _ = pgemm4_configs()[cfg]
+        if bq > 64 and M <= bq // 2:
+            continue
+        tiles = -(-rows // bp) * -(-M // bq)
+        for s in (1, 2, 3, 4, 6, 8):
+            if s > 1 and (tiles * s > 600 or kt // s < 4):
+                break
+            rounds, per = -(-tiles * s // num_cus), -(-kt // s)
+            us = t0 + rounds * (rnd + tile * per) + step * per + wmb * mb + (sp + slab * M * rows * s * 4e-6 if s > 1 else 0.0)
+            if best is None or us < best[0]:
+                best = (us, cfg, s)
+    return best[1:]
+
+
 def _pgemm_big_tiles(M: int, N: int, K: int, epi: int, fp8: bool, num_cus: int = 256) -> Tuple[str, int, int, int]:
     cfg = 0
     tiles = pgemm_tiles(cfg, M, N, epi)
@@ -1149,6 +1183,10 @@ def _gemm(x2: torch.Tensor, w, epi: int, res: Optional[torch.Tensor] = None, rms
         if y is not None:
             return y
     N = w.shape[0] // 2 if epi == EPI_SWIGLU else w.shape[0]
+    if not fp8 and act is None and GEMM_BACKEND == "auto" and M < PG_MIN_M:
+        tile = _few_rows_tile(M, w.shape[0], K, epi)
+        if tile is not None:
+            return pgemm4(x2, w, epi, cfg=tile[0], splits=tile[1], group_m=1, res=res, rms_eps=rms_eps, out=out)
     kern, plan = gemm_route(M, N, K, epi, fp8)
     if kern == "library" or (fp8 and rms_eps is not None):
         return None   # (fp8: the activations are quantized after the norm, so the caller normalises first)
