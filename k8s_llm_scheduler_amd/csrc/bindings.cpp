@@ -128,6 +128,9 @@ int k8s_resnorm(float* x, const void* branch, const void* branch2, float mult, c
 int k8s_norm_mix(void* out, const void* a, long lda, const void* wa, const void* b, const void* wb, float eps, float ca,
                  float cb, int T, int W, int groups, const void* gate, long ldg, int gkind, int in_f32, int out_f32,
                  hipStream_t s);
+int k8s_branchnorm_moe(float* x, const void* D, const int* pos, int cols, int top, float scale, const void* shared,
+                       const float* logits, int ld, const void* w, const void* nw, float gain, const void* dotw, float* dot,
+                       float eps, void* out, int T, int W, int f32, hipStream_t s);
 int k8s_branchnorm(float* x, const void* branch, const void* w, const void* bias, const void* nw, float gain,
                    const void* dotw, float* dot, float eps, void* out, int T, int W, int branch_f32, int f32,
                    hipStream_t s);
@@ -550,6 +553,15 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
                        int out_f32, int64_t s) {
     check(k8s_norm_mix(P(out), P(a), lda, P(wa), P(b), P(wb), eps, ca, cb, T, W, groups, P(gate), ldg, gkind, in_f32,
                        out_f32, S(s)), "norm_mix");
+  });
+  // false: sizes or alignments that its kernel does not take; nothing was launched
+  m.def("branchnorm_moe", [](uintptr_t x, uintptr_t D, uintptr_t pos, int cols, int top, float scale, uintptr_t shared,
+                             uintptr_t gate, uintptr_t w, uintptr_t nw, float gain, uintptr_t dotw, uintptr_t dot, float eps,
+                             uintptr_t out, int T, int W, int f32, int64_t s) {
+    const int rc = k8s_branchnorm_moe(P<float>(x), P(D), P<int>(pos), cols, top, scale, P(shared), P<float>(gate), 1, P(w), P(nw),
+                                      gain, P(dotw), P<float>(dot), eps, P(out), T, W, f32, S(s));
+    if (rc != -1) check(rc, "branchnorm_moe");
+    return rc != -1;
   });
   m.def("branchnorm", [](uintptr_t x, uintptr_t branch, uintptr_t w, uintptr_t bias, uintptr_t nw, float gain,
                          uintptr_t dotw, uintptr_t dot, float eps, uintptr_t out, int T, int W, int branch_f32, int f32,

@@ -184,15 +184,30 @@ __global__ __launch_bounds__(256) void postnorm_kernel(float* __restrict__ x, co
 // projection onto one number per token).  branch == null: nothing is added.  One workgroup per row.  NV > 0 (W % 4 == 0,
 // W <= 1024 NV): everything a thread needs is loaded as vectors ahead of the reductions and stays in registers; else the
 // row is read again after them (a thread re-reads only the elements it wrote).
-template <typename TB, typename TA, int NV>
+// MOE (NV > 0): the branch is the experts' combine of moe.hip, branch[t] = sum over `top` choices k of scale D[pos[t, k]] + gate_t s_t,
+// rounded to its type as that kernel's output is; s_t is row t of `shared` or, where that is null and pos has one column more, D's row
+// pos[t, top] (shared and pos of `top` columns null: no shared expert), gate_t = sigmoid(logits[t ld]) (logits null: 1).  It saves
+// the combine's launch and its output's way through memory: 32 rows of 2048 5.0 + 5.6 us in a step, 1534 rows 8.0 + 10.5.
+template <typename TA>
+struct MoeBranch {
+  const TA* D;
+  const int* pos;
+  const TA* shared;
+  const float* logits;
+  int cols, top, ld;
+  float scale;
+};
+template <typename TB, typename TA, int NV, bool MOE = false>
 __global__ __launch_bounds__(256) void branchnorm_kernel(float* __restrict__ x, const TB* __restrict__ branch,
                                                          const TA* __restrict__ w, const TA* __restrict__ bias,
                                                          const TA* __restrict__ nw, float gain,
                                                          const TA* __restrict__ dotw, float* __restrict__ dot, float eps,
-                                                         TA* __restrict__ out, int W) {
+                                                         TA* __restrict__ out, int W, MoeBranch<TA> moe) {
   __shared__ float red[16];
   const size_t base = (size_t)blockIdx.x * W;
   float ss = 0.f, ds = 0.f;
+  static_assert(!MOE || NV > 0, "the combine goes with whole vectors");
+  const bool add = MOE || branch != nullptr;
   if constexpr (NV > 0) {
     const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
     f32x4 v[NV], xv[NV], wv[NV], nv[NV];
@@ -200,17 +215,51 @@ __global__ __launch_bounds__(256) void branchnorm_kernel(float* __restrict__ x, 
     for (int n = 0; n < NV; ++n) {
       const int i = 4 * (threadIdx.x + 256 * n);
       const bool in = i < W;
-      v[n] = in && branch != nullptr ? ldf4(branch + base + i) : zero;
+      if constexpr (!MOE) v[n] = in && branch != nullptr ? ldf4(branch + base + i) : zero;
       xv[n] = in ? ldf4(x + base + i) : zero;
-      wv[n] = in && branch != nullptr ? ldf4(w + i) : zero;
+      wv[n] = in && add ? ldf4(w + i) : zero;
       nv[n] = in && nw != nullptr ? ldf4(nw + i) : zero;
-      if (in && bias != nullptr) {
+    }
+    if constexpr (MOE) {
+      const int* pos = moe.pos + (size_t)blockIdx.x * moe.cols;
+      const float gate = moe.logits != nullptr ? 1.f / (1.f + expf(-moe.logits[(size_t)blockIdx.x * moe.ld])) : 1.f;
+      const TA* last = moe.shared != nullptr ? moe.shared + base : moe.cols > moe.top ? moe.D + (size_t)pos[moe.top] * W : nullptr;
+#pragma unroll
+      for (int n = 0; n < NV; ++n) v[n] = zero;
+      for (int k = 0; k < moe.top; ++k) {
+        const TA* row = moe.D + (size_t)pos[k] * W;
+#pragma unroll
+        for (int n = 0; n < NV; ++n) {
+          const int i = 4 * (threadIdx.x + 256 * n);
+          const f32x4 d = i < W ? ldf4(row + i) : zero;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[n][e] = fmaf(moe.scale, d[e], v[n][e]);
+        }
+      }
+#pragma unroll
+      for (int n = 0; n < NV; ++n) {
+        const int i = 4 * (threadIdx.x + 256 * n);
+        if (last != nullptr) {
+          const f32x4 d = i < W ? ldf4(last + i) : zero;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[n][e] = fmaf(gate, d[e], v[n][e]);
+        }
+        if constexpr (sizeof(TA) == 2) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[n][e] = bf_round(v[n][e]);
+        }
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      const int i = 4 * (threadIdx.x + 256 * n);
+      if (i < W && bias != nullptr) {
         const f32x4 bv = ldf4(bias + i);
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[n][e] += bv[e];
       }
     }
-    if (branch != nullptr) {
+    if (add) {
 #pragma unroll
       for (int n = 0; n < NV; ++n)
 #pragma unroll
@@ -987,7 +1036,7 @@ extern "C" int k8s_branchnorm(float* x, const void* branch, const void* w, const
   if (dot != nullptr && (nw == nullptr || dotw == nullptr)) return -1;
 #define K8S_BN(TB, TA, NV)                                                                                               \
   branchnorm_kernel<TB, TA, NV><<<T, 256, 0, s>>>(x, (const TB*)branch, (const TA*)w, (const TA*)bias, (const TA*)nw, gain, \
-                                                  (const TA*)dotw, dot, eps, (TA*)out, W)
+                                                  (const TA*)dotw, dot, eps, (TA*)out, W, MoeBranch<TA>{})
 #define K8S_BN_T(TB, TA)                                                                                                \
   do {                                                                                                                  \
     const bool vec = W % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)branch % (4 * sizeof(TB)) == 0 &&               \
@@ -1003,6 +1052,34 @@ extern "C" int k8s_branchnorm(float* x, const void* branch, const void* w, const
   else K8S_BN_T(bf16_t, bf16_t);
 #undef K8S_BN_T
 #undef K8S_BN
+  return (int)hipGetLastError();
+}
+
+// The same behind experts: the branch is their combine (MoeBranch), W % 4 == 0 up to 8192, every pointer aligned to four elements.
+extern "C" int k8s_branchnorm_moe(float* x, const void* D, const int* pos, int cols, int top, float scale, const void* shared,
+                                  const float* logits, int ld, const void* w, const void* nw, float gain, const void* dotw,
+                                  float* dot, float eps, void* out, int T, int W, int f32, hipStream_t s) {
+  if (T <= 0) return 0;
+  if (W <= 0 || W % 4 || W > 8192 || x == nullptr || D == nullptr || pos == nullptr || w == nullptr || top <= 0) return -1;
+  if (cols != top && (cols != top + 1 || shared != nullptr)) return -1;
+  if ((nw != nullptr && out == nullptr) || (dot != nullptr && (nw == nullptr || dotw == nullptr))) return -1;
+  if ((uintptr_t)x % 16 || ((uintptr_t)D | (uintptr_t)shared | (uintptr_t)w | (uintptr_t)nw | (uintptr_t)dotw | (uintptr_t)out) % (f32 ? 16 : 8))
+    return -1;
+#define K8S_BM(TA, NV)                                                                                                      \
+  branchnorm_kernel<TA, TA, NV, true><<<T, 256, 0, s>>>(x, (const TA*)nullptr, (const TA*)w, (const TA*)nullptr, (const TA*)nw, \
+                                                        gain, (const TA*)dotw, dot, eps, (TA*)out, W,                        \
+                                                        MoeBranch<TA>{(const TA*)D, pos, (const TA*)shared, logits, cols, top, ld, scale})
+#define K8S_BM_T(TA)                                                                    \
+  do {                                                                                  \
+    if (W <= 1024) K8S_BM(TA, 1);                                                       \
+    else if (W <= 2048) K8S_BM(TA, 2);                                                  \
+    else if (W <= 4096) K8S_BM(TA, 4);                                                  \
+    else K8S_BM(TA, 8);                                                                 \
+  } while (0)
+  if (f32) K8S_BM_T(float);
+  else K8S_BM_T(bf16_t);
+#undef K8S_BM_T
+#undef K8S_BM
   return (int)hipGetLastError();
 }
 

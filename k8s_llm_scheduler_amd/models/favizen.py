@@ -522,7 +522,7 @@ class FavizenModel(StreamModel):
     def _glu(w: _Glu, h) -> torch.Tensor:
         return sm.linear(sm.linear_act(h, w.w_gu, sm.ACT_SWISH_CLAMP, w.limit, SWISH_ALPHA, bias=w.b_gu), w.w_down)
 
-    def _moe(self, w: _Moe, h, sg, b) -> torch.Tensor:
+    def _moe(self, w: _Moe, h, sg, b) -> sm.MoeBranch:
         f = w.cfg
         P = h.shape[0] * f.top
         key, l = w.route
@@ -531,7 +531,7 @@ class FavizenModel(StreamModel):
                         seg=seg)
         d = sm.gemm(g, w.experts.w_down, tiles=tiles, rows=P, seg=seg)
         shared = self._glu(w.shared, h) if w.shared is not None else None
-        return sm.moe_combine(d, pos, None, shared, sg, 0 if sg is not None else -1, top=f.top, scale=1.0 / f.top)
+        return sm.MoeBranch(d, pos, f.top, 1.0 / f.top, shared, sg if shared is not None else None, h.shape[0])
 
     def _blocks(self, ids, b, after=None):
         """The residual stream before the last layer's branch is added, and that branch: (x, branch, norm weight, bias)."""

@@ -41,9 +41,11 @@ def stack_rows(parts, align: int = 16):
     return torch.cat(rows), cols
 
 
-def pick_rows(t: Optional[torch.Tensor], rows: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
-    """The rows whose logits are wanted (None: all of them)."""
-    return t if t is None or rows is None else t.index_select(0, rows)
+def pick_rows(t, rows: Optional[torch.Tensor]):
+    """The rows (of a tensor, a branch of experts or None) whose logits are wanted (None: all of them)."""
+    if t is None or rows is None:
+        return t
+    return t.select(rows) if isinstance(t, sm.MoeBranch) else t.index_select(0, rows)
 
 
 class StreamModel:

@@ -14,7 +14,7 @@ import functools
 import math
 import os
 import sys
-from typing import Optional
+from typing import NamedTuple, Optional
 
 import torch
 
@@ -153,12 +153,22 @@ def branchnorm(x: torch.Tensor, branch: Optional[torch.Tensor], w: Optional[torc
                out_dtype=None, bias: Optional[torch.Tensor] = None, next_w: Optional[torch.Tensor] = None,
                gain: float = 1.0, dot_w: Optional[torch.Tensor] = None):
     """Norm of the sublayer's output only: ``x`` (fp32 [T, W], updated in place) += rms-norm(branch + ``bias``) * w.
-    ``branch`` is of w's type, or fp32 (None, with ``next_w``: nothing is added).  With ``out_dtype`` (the weights' type)
+    ``branch`` is of w's type, or fp32 (None, with ``next_w``: nothing is added), or a :class:`MoeBranch`.  With ``out_dtype`` (the weights' type)
     the new rows are also returned in that type, for a sublayer that reads the stream itself -- or, with ``next_w``, their
     norm rms-norm(x) * next_w * gain, for a sublayer that is normed on both sides.  ``dot_w`` [W] (with ``next_w``):
     returns (rows, the normed rows' products with it, fp32 [T, 1])."""
     if x.dtype != F32 or not x.is_contiguous():
         raise TypeError("the residual stream is contiguous fp32")
+    if isinstance(branch, MoeBranch):
+        if bias is None and w is not None and _gpu(x, branch.D, w, next_w) and branch.joins(x, w, out_dtype, next_w, dot_w):
+            T, W = x.shape
+            out = torch.empty(T, W, dtype=out_dtype, device=x.device) if out_dtype is not None else None
+            dot = torch.empty(T, 1, dtype=F32, device=x.device) if dot_w is not None else None
+            if _native().branchnorm_moe(_p(x), branch.D.data_ptr(), _p(branch.pos, I32), branch.pos.numel() // max(T, 1), branch.top,
+                                        float(branch.scale), _p(branch.shared), _p(branch.gate), _p(w), _p(next_w), float(gain),
+                                        _p(dot_w), _p(dot), float(eps), _p(out), T, W, _f32(w.dtype), -1):
+                return (out, dot) if dot_w is not None else out
+        branch = branch.combined()
     wt = (w if w is not None else next_w).dtype
     if branch is not None and (branch.shape != x.shape or branch.dtype not in (wt, F32) or w is None):
         raise TypeError("branchnorm: branch [T, W] of the weight's type or fp32, w [W]")
@@ -823,6 +833,47 @@ def moe_combine(D: torch.Tensor, pos_of_pair: torch.Tensor, topk_w: Optional[tor
                           _p(logits, F32), logits.stride(0) if logits is not None else 0, sg_col, T, W, top,
                           _f32(D.dtype), -1)
     return z
+
+
+class MoeBranch(NamedTuple):
+    """The experts' output ahead of its combine, for the norm that follows (:func:`branchnorm`): row t is
+    sum over ``top`` choices of ``scale`` D[pos[t, k]] + sigmoid(gate[t]) * shared[t] (``gate`` fp32 [T, 1] or None: 1).  With top + 1
+    columns of ``pos`` and no ``shared`` the last one names the shared expert's row of ``D``."""
+    D: torch.Tensor
+    pos: torch.Tensor                  # int32, T x top or T x (top + 1) values
+    top: int
+    scale: float
+    shared: Optional[torch.Tensor] = None
+    gate: Optional[torch.Tensor] = None
+    tokens: int = 0
+
+    def select(self, rows: torch.Tensor) -> "MoeBranch":
+        """The branch of these tokens."""
+        pick = lambda t: None if t is None else t.index_select(0, rows)
+        return self._replace(pos=self.pos.view(self.tokens, -1).index_select(0, rows), shared=pick(self.shared), gate=pick(self.gate),
+                             tokens=rows.numel())
+
+    def combined(self) -> torch.Tensor:
+        pos, shared = self.pos.view(self.tokens, -1), self.shared
+        if pos.shape[1] > self.top:
+            shared, pos = self.D.index_select(0, pos[:, self.top].long()), pos[:, :self.top].contiguous()
+        return moe_combine(self.D, pos.reshape(-1), None, shared, self.gate, 0 if self.gate is not None else -1, top=self.top,
+                           scale=self.scale)
+
+    def joins(self, x: torch.Tensor, w: torch.Tensor, out_dtype, next_w, dot_w) -> bool:
+        """Whether the combine can go with the norm: one type, the sizes that either would ask for (the kernel itself looks at the
+        alignment)."""
+        D, shared, gate, W, dt = self.D, self.shared, self.gate, x.shape[1], w.dtype
+        if D.dtype != dt or D.shape[1] != W or x.shape[0] != self.tokens or out_dtype not in (None, dt) or not D.is_contiguous():
+            return False
+        for t in (w, next_w, dot_w):
+            if t is not None and (t.numel() != W or t.dtype != dt):
+                return False
+        if (next_w is not None and out_dtype is None) or (dot_w is not None and next_w is None):
+            return False
+        if shared is not None and (shared.dtype != dt or shared.shape != x.shape or not shared.is_contiguous()):
+            return False
+        return gate is None or (gate.dtype == F32 and gate.numel() == self.tokens and gate.is_contiguous())
 
 
 # ----------------------------------------------------------------------------- windowed attention with pooled blocks
