@@ -114,7 +114,7 @@ int k8s_pgemm4_act(void* out, const void* x, const void* W, int M, int N_out, in
                    float limit, float alpha, const void* bias, hipStream_t stream);
 int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M, int rows, int N_out, int K, int groups, const int* seg,
                        const int* a_rows, long ldx, int cfg, int group_m, int kind, float limit, float alpha,
-                       hipStream_t stream);
+                       float last_limit, hipStream_t stream);
 int k8s_pgemm4(void* out, float* slab, const void* x, const void* W, int M, int N_out, int K, int epi, int cfg,
                int splits, int group_m, const void* res, int rms, float eps, const float* scale, hipStream_t s);
 int k8s_pgemm4_scaled(int cfg);
@@ -159,7 +159,8 @@ int k8s_rglru_scan(void* out, const float* u, const float* gates, const float* g
 int k8s_act(void* out, const void* x, int T, int F, int kind, float limit, float alpha, const float* row_scale,
             const int* row_map, const void* bias, int f32, hipStream_t s);
 int k8s_gemm_few_act(void* C, const void* A, const void* W, int M, int N, int K, long lda, const int* a_rows,
-                     const int* tiles, int ntiles, int kind, float limit, float alpha, hipStream_t s);
+                     const int* tiles, int ntiles, int kind, float limit, float alpha, int last, float last_limit,
+                     hipStream_t s);
 int k8s_gemv_act(void* out, void* partial, const void* x, const void* W, int M, int N_out, int K, int kind, float limit, float alpha,
                  hipStream_t stream);
 int k8s_gemv_act_plan(int M, int N_out, int K, int pair, int* ks, int* splits, int* wgs, int* per);
@@ -622,8 +623,13 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
   });
   m.def("gemm_few_act", [](uintptr_t C, uintptr_t A, uintptr_t W, int M, int N, int K, long lda, uintptr_t a_rows,
                            uintptr_t tiles, int ntiles, int kind, float limit, float alpha, int64_t s) {
-    check(k8s_gemm_few_act(P(C), P(A), P(W), M, N, K, lda, P<int>(a_rows), P<int>(tiles), ntiles, kind, limit, alpha, S(s)),
+    check(k8s_gemm_few_act(P(C), P(A), P(W), M, N, K, lda, P<int>(a_rows), P<int>(tiles), ntiles, kind, limit, alpha, -1, 0.f, S(s)),
           "gemm_few_act");
+  });
+  m.def("gemm_few_act", [](uintptr_t C, uintptr_t A, uintptr_t W, int M, int N, int K, long lda, uintptr_t a_rows, uintptr_t tiles,
+                           int ntiles, int kind, float limit, float alpha, int last, float last_limit, int64_t s) {
+    check(k8s_gemm_few_act(P(C), P(A), P(W), M, N, K, lda, P<int>(a_rows), P<int>(tiles), ntiles, kind, limit, alpha, last,
+                           last_limit, S(s)), "gemm_few_act");
   });
   m.def("gemm_f32_tiles", [](uintptr_t C, uintptr_t A, uintptr_t W, int M, int N, int K, long lda, long ldw, long ldc,
                              int batch, long sA, long sW, long sC, uintptr_t a_rows, uintptr_t tiles, int ntiles,
@@ -856,7 +862,13 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
   m.def("pgemm4_grouped", [](uintptr_t out, uintptr_t x, uintptr_t W, int M, int rows, int N, int K, int groups, uintptr_t seg,
                              uintptr_t a_rows, long ldx, int cfg, int group_m, int kind, float limit, float alpha, int64_t s) {
     check(k8s_pgemm4_grouped(P(out), P(x), P(W), M, rows, N, K, groups, P<int>(seg), P<int>(a_rows), ldx, cfg, group_m, kind,
-                             limit, alpha, S(s)), "pgemm4_grouped");
+                             limit, alpha, limit, S(s)), "pgemm4_grouped");
+  });
+  m.def("pgemm4_grouped", [](uintptr_t out, uintptr_t x, uintptr_t W, int M, int rows, int N, int K, int groups, uintptr_t seg,
+                             uintptr_t a_rows, long ldx, int cfg, int group_m, int kind, float limit, float alpha,
+                             float last_limit, int64_t s) {
+    check(k8s_pgemm4_grouped(P(out), P(x), P(W), M, rows, N, K, groups, P<int>(seg), P<int>(a_rows), ldx, cfg, group_m, kind,
+                             limit, alpha, last_limit, S(s)), "pgemm4_grouped");
   });
   m.def("pgemm4", [](uintptr_t out, uintptr_t slab, uintptr_t x, uintptr_t W, int M, int N, int K, int epi, int cfg,
                      int splits, int group_m, uintptr_t res, int rms, float eps, int64_t s) {

@@ -94,6 +94,7 @@ struct P4Args {
   int spread;            // the XCDs start their walk over k an eighth of it apart
   int wide;              // the output's rows can be stored in 16-byte pieces
   float limit, alpha;    // P4_GLU: of the gated kind
+  float last_limit;      // grouped form: the limit of the last group
   const bf16_t* bias;    // P4_GLU, optional: [gate; up] biases
   // grouped form: group g's rows are [seg[g], seg[g + 1]) of a compact row space (row r of x: a_rows[r], or r) and its
   // weights W + g wstride bytes; m_tiles bounds the groups' row tiles.  8 experts, 3068 rows, K = 2048, in a step: gate / up
@@ -151,6 +152,7 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
   // tokens of the tile: rows [m0, m_end) of the compact row space
   const uint8_t* Wb = a.W;
   int m0 = mt * BQ, m_end = a.M;
+  float limit = a.limit;
   if constexpr (GRP) {
     int gi = 0, left = mt;                           // mt < m_tiles: a group is found
     for (;; ++gi) {
@@ -161,6 +163,7 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
     m0 = first(gi) + left * BQ;
     m_end = first(gi + 1);
     Wb += (long long)gi * a.wstride;
+    if (gi == a.groups - 1) limit = a.last_limit;
   }
   auto xrow = [&](int r) -> uint32_t {               // row r of the tile, past the end its last one
     const int m = min(m0 + r, m_end - 1);
@@ -450,7 +453,7 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
 #pragma unroll
       for (int e = 0; e < LF; ++e) {
         const float up = MIX ? acc[i][j][2 + e] : acc[FP / 2 + i][j][e];
-        v[e] = epi_pair<KIND>(acc[i][j][e] + bg[e], up + bu[e], a.limit, a.alpha);
+        v[e] = epi_pair<KIND>(acc[i][j][e] + bg[e], up + bu[e], limit, a.alpha);
       }
     } else if constexpr (EPI == P4_SWIGLU) {
 #pragma unroll
@@ -887,10 +890,10 @@ extern "C" int k8s_pgemm4_act(void* out, const void* x, const void* W, int M, in
 }
 
 // Grouped product over at most `rows` compact rows (x: M rows in memory, ldx elements apart): kind < 0 plain, or a gated kind
-// with [groups][2 N_out][K] weights.
+// with [groups][2 N_out][K] weights (last_limit: the last group's).
 extern "C" int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M, int rows, int N_out, int K, int groups,
                                   const int* seg, const int* a_rows, long ldx, int cfg, int group_m, int kind, float limit,
-                                  float alpha, hipStream_t stream) {
+                                  float alpha, float last_limit, hipStream_t stream) {
   const bool pair = kind >= 0;
   if (kind < -1 || (pair && kind > 1 && kind != 5)) return -1;
   if (rows <= 0) return 0;
@@ -912,6 +915,7 @@ extern "C" int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M
   a.groups = groups;
   a.limit = limit;
   a.alpha = alpha;
+  a.last_limit = last_limit;
   switch (cfg) {
     case 1: return p4_act_kind<1, true>(a, kind, stream);
     case 2: return p4_act_kind<2, true>(a, kind, stream);

@@ -812,6 +812,8 @@ enum { FEW_NONE = 0, FEW_ELEM = 1, FEW_PAIR = 2 };
 struct FewAct {
   int kind;
   float limit, alpha;
+  int last;            // grouped: this group's limit is last_limit
+  float last_limit;
 };
 // Grouped products of few rows (decoding with experts): a workgroup takes 16 columns of one row tile (at most 64 rows).  The
 // weights go from memory straight into MFMA operands, no LDS staging; its 4 waves share the k range in 64-deep pieces (wave w
@@ -910,6 +912,7 @@ __global__ __launch_bounds__(256) void gemm_group_kernel(TO* __restrict__ C, con
   if (g < 0) return;
   const int row0 = tiles[3 * blockIdx.y + 1], rows = tiles[3 * blockIdx.y + 2];
   Wt += (size_t)g * sW;
+  if (ACT == FEW_PAIR && g == act.last) act.limit = act.last_limit;
   if (rows <= 16) gemm_group_tile<TO, 1, ACT>(C, A, Wt, N, K, lda, ldw, ldc, a_rows, row0, rows, red, act);
   else gemm_group_tile<TO, 4, ACT>(C, A, Wt, N, K, lda, ldw, ldc, a_rows, row0, rows, red, act);
 }
@@ -1130,9 +1133,10 @@ extern "C" int k8s_act(void* out, const void* x, int T, int F, int kind, float l
 }
 
 // act(A W^T) in bf16 of few rows: elementwise of a plain product (tiles == nullptr; M rows), or a gated `kind` of a grouped one
-// (tiles, W [groups, 2 N, K]).  K % 64 == 0, rows of whole 16-byte vectors.
+// (tiles, W [groups, 2 N, K]; group `last`, if there is one, with last_limit).  K % 64 == 0, rows of whole 16-byte vectors.
 extern "C" int k8s_gemm_few_act(void* C, const void* A, const void* W, int M, int N, int K, long lda, const int* a_rows,
-                                const int* tiles, int ntiles, int kind, float limit, float alpha, hipStream_t s) {
+                                const int* tiles, int ntiles, int kind, float limit, float alpha, int last, float last_limit,
+                                hipStream_t s) {
   const bool pair = kind == 0 || kind == 1 || kind == 5;
   if (N <= 0 || K <= 0 || K % 64 || lda % 8 || kind < 0 || kind > 7 || (((uintptr_t)A | (uintptr_t)W) & 15)) return -1;
   if (pair != (tiles != nullptr) || (kind == 6 && !(limit > 0.f))) return -1;
@@ -1140,7 +1144,7 @@ extern "C" int k8s_gemm_few_act(void* C, const void* A, const void* W, int M, in
   if (M <= 0 || gy <= 0) return 0;
   if (gy > 65535) return -2;
   const dim3 grid((N + 15) / 16, gy);
-  const FewAct act{kind, limit, alpha};
+  const FewAct act{kind, limit, alpha, last, last_limit};
   if (pair)
     gemm_group_kernel<bf16_t, FEW_PAIR><<<grid, 256, 0, s>>>((bf16_t*)C, (const bf16_t*)A, (const bf16_t*)W, N, K, lda, K, N,
                                                              2L * N * K, a_rows, tiles, act);

@@ -310,6 +310,7 @@ class _Moe:
     shared: Optional[_Glu]
     sg: Optional[torch.Tensor]             # [W]
     route: tuple                           # (key into the stacked tables, layer in them)
+    joint: Optional[_Glu] = None           # experts and the shared one in one stack (the two above are views of it)
 
 
 @dataclass
@@ -419,19 +420,30 @@ class FavizenModel(StreamModel):
         if not 0 < f.top <= E:
             raise ValueError(f"{where}: {f.top} of {E} experts per token")
         stack = lambda names: torch.stack([torch.cat([get(f"{p}e{e}.{n}") for n in names]) for e in range(E)])
-        experts = _Glu(f.limit, t(stack(("gate", "up"))), t(stack(("down",))))
-        shared = sg = None
+        gate_up, down = stack(("gate", "up")), stack(("down",))
+        shared = sg = joint = None
         if f.shared_ff:
             q = p + "shared."
-            shared = _Glu(f.shared_limit, t(torch.cat([get(q + "gate"), get(q + "up")])), t(get(q + "down")))
+            s_gate_up, s_down = torch.cat([get(q + "gate"), get(q + "up")]), get(q + "down")
             sg = self._maybe(get, q + "sg")
             sg = t(sg.reshape(-1)) if sg is not None else None
         table = get(p + "table").to(torch.int32).cpu()
         if table.shape != (self.cfg.vocab, f.top) or int(table.min()) < 0 or int(table.max()) >= E:
             raise ValueError(f"{where}: the experts' table must name {f.top} of {E} experts for every token id")
-        group = self._tables.setdefault((E, f.top), [])
+        if f.shared_ff == f.ff and self.dtype == torch.bfloat16 and sm.joint_experts(E, self.cfg.hidden, f.ff):
+            # a shared expert of the others' size is one more of them, which every token has
+            joint = _Glu(f.limit, t(torch.cat([gate_up, s_gate_up.unsqueeze(0)])), t(torch.cat([down, s_down.unsqueeze(0)])))
+            experts = _Glu(f.limit, joint.w_gu[:E], joint.w_down[:E])
+            shared = _Glu(f.shared_limit, joint.w_gu[E], joint.w_down[E])
+            table = torch.cat([table, torch.full((self.cfg.vocab, 1), E, dtype=torch.int32)], 1)
+        else:
+            experts = _Glu(f.limit, t(gate_up), t(down))
+            if f.shared_ff:
+                shared = _Glu(f.shared_limit, t(s_gate_up), t(s_down))
+        key = (E + (joint is not None), table.shape[1])
+        group = self._tables.setdefault(key, [])
         group.append(table)
-        return _Moe(f, experts, shared, sg, ((E, f.top), len(group) - 1))
+        return _Moe(f, experts, shared, sg, (key, len(group) - 1), joint)
 
     def _build(self, get) -> None:
         c, t = self.cfg, self._t
@@ -523,15 +535,20 @@ class FavizenModel(StreamModel):
         return sm.linear(sm.linear_act(h, w.w_gu, sm.ACT_SWISH_CLAMP, w.limit, SWISH_ALPHA, bias=w.b_gu), w.w_down)
 
     def _moe(self, w: _Moe, h, sg, b) -> sm.MoeBranch:
-        f = w.cfg
-        P = h.shape[0] * f.top
+        f, T = w.cfg, h.shape[0]
         key, l = w.route
         sorted_tok, pos, seg, tiles = b["routes"][key][l]
+        if w.joint is not None:
+            kw = dict(tiles=tiles, rows=T * (f.top + 1), seg=seg, common=T)
+            g = sm.gemm_act(h, w.joint.w_gu, sm.ACT_SWISH_CLAMP, f.limit, SWISH_ALPHA, a_rows=sorted_tok,
+                            common_limit=f.shared_limit, **kw)
+            return sm.MoeBranch(sm.gemm(g, w.joint.w_down, **kw), pos, f.top, 1.0 / f.top, None, sg, T)
+        P = T * f.top
         g = sm.gemm_act(h, w.experts.w_gu, sm.ACT_SWISH_CLAMP, f.limit, SWISH_ALPHA, a_rows=sorted_tok, tiles=tiles, rows=P,
                         seg=seg)
         d = sm.gemm(g, w.experts.w_down, tiles=tiles, rows=P, seg=seg)
         shared = self._glu(w.shared, h) if w.shared is not None else None
-        return sm.MoeBranch(d, pos, f.top, 1.0 / f.top, shared, sg if shared is not None else None, h.shape[0])
+        return sm.MoeBranch(d, pos, f.top, 1.0 / f.top, shared, sg if shared is not None else None, T)
 
     def _blocks(self, ids, b, after=None):
         """The residual stream before the last layer's branch is added, and that branch: (x, branch, norm weight, bias)."""

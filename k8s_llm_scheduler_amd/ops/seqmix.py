@@ -294,12 +294,13 @@ def linear(a: torch.Tensor, w: torch.Tensor, out_dtype=None) -> torch.Tensor:
 
 def gemm(a: torch.Tensor, w: torch.Tensor, out_dtype=None, *, a_rows: Optional[torch.Tensor] = None,
          tiles: Optional[torch.Tensor] = None, rows: Optional[int] = None,
-         seg: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+         seg: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None, common: int = 0) -> torch.Tensor:
     """The any-shape GEMM.  2-D: a [M, K] (row stride free) @ w [N, K]^T.  3-D: batched over dim 0 (a [G, M, K] with
     any strides whose last is 1, w [G, N, K]) -> [G, M, N]; ``out``: a [G, M, N] view with any batch / row strides.
     Grouped (``tiles`` [n, 3] from :func:`moe_align`, w [G, N, K]): ``rows`` compact rows, row r = a[a_rows[r]] (or
     a[r]), the rows of tile (g, r0, n) use w[g] -> [rows, N].  ``seg`` int32 [G + 1]: the groups' row offsets, the same
-    rows as ``tiles`` lists; the CPU reference and the big-tile kernel (:func:`_grouped_big`) go by them.  The order of an output's
+    rows as ``tiles`` lists; the CPU reference and the big-tile kernel (:func:`_grouped_big`) go by them.  ``common``: that many of
+    the rows are the last group's (an expert that every token has), which the choice of the tile goes by.  The order of an output's
     sums depends on the kernel, and that on the sizes: in bf16, and in fp32 from a depth of 512 on, a row's result may differ in the last
     bits with the rows beside it (fp32 of less depth or of rows that are not 16-byte aligned: not)."""
     out_dtype = out_dtype or a.dtype
@@ -314,7 +315,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out_dtype=None, *, a_rows: Optional[t
         if not _gpu(a, w):
             return ref.gemm_any(a, w, out_dtype, a_rows, tiles, seg)
         if out_dtype == BF16 and _grouped_big(a, w, seg, rows, N):
-            return _pgemm4_grouped(a, w, a_rows, rows, seg, N)
+            return _pgemm4_grouped(a, w, a_rows, rows, seg, N, common=common)
         out = torch.empty(rows, N, dtype=out_dtype, device=a.device)
         _native().gemm_any(out.data_ptr(), a.data_ptr(), _p(w), rows, N, K, a.stride(0), K, N, 1, 0, N * K, 0,
                            _p(a_rows, I32, "a_rows"), _p(tiles, I32, "tiles"), tiles.shape[0], _f32(a.dtype),
@@ -346,7 +347,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out_dtype=None, *, a_rows: Optional[t
     return out
 
 
-# Grouped bf16 products of at least GROUP_BIG_MIN rows per group on average (GROUP_BIG_MIN_FEW of up to 8 groups; whole rows of at
+# Grouped bf16 products of at least GROUP_BIG_MIN rows per group on average (GROUP_BIG_MIN_FEW of up to 12 groups; whole rows of at
 # least 64 elements) run on the big-tile kernel (pgemm4.hip); fewer stream the weights past the LDS (gemm_group_kernel), whose time
 # goes with the groups that have rows.  us, weights from memory, past the LDS / big tiles: gate / up of 8 groups with the activation
 # (2 x 2048 x 2048), 0.5 / 1 / 2 / 4 / 8 / 16 rows per group 17.1 / 19.0, 23.3 / 22.6, 29.8 / 26.1, 34.7 / 28.2, 33.7 / 28.4, 41.9 /
@@ -354,7 +355,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, out_dtype=None, *, a_rows: Optional[t
 # 40.7, 42.0 / 43.0, 56.3 / 47.9; 16 of 2 x 2048 x 4096, 2 / 4 / 6 / 8 91 / 103, 105 / 111, 109 / 110, 112 / 111; 16 of 2048 x 1024, 4 / 6 / 8
 # 15.6 / 17.1, 16.4 / 16.9, 17.8 / 17.1.
 GROUP_BIG_MIN = 6
-GROUP_BIG_MIN_FEW = 2
+GROUP_BIG_MIN_FEW = 2            # of up to 12 groups
 GROUP_BIG_MAX_GROUPS = 64        # every workgroup walks the groups' offsets
 
 
@@ -362,7 +363,7 @@ def _grouped_big(a: torch.Tensor, w: torch.Tensor, seg: Optional[torch.Tensor], 
     E, _, K = w.shape
     return (not _ops.LEAN and FAST_GEMM and a.dtype == BF16 and seg is not None and seg.is_cuda and seg.dtype == I32
             and seg.is_contiguous() and seg.numel() == E + 1 and E <= GROUP_BIG_MAX_GROUPS
-            and rows >= (GROUP_BIG_MIN if E > 8 else GROUP_BIG_MIN_FEW) * E and K % 64 == 0 and N % 4 == 0 and N >= 128 and a.dim() == 2 and a.stride(1) == 1
+            and rows >= (GROUP_BIG_MIN if E > 12 else GROUP_BIG_MIN_FEW) * E and K % 64 == 0 and N % 4 == 0 and N >= 128 and a.dim() == 2 and a.stride(1) == 1
             and a.stride(0) >= K and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.is_contiguous()
             and w.data_ptr() % 16 == 0 and w.shape[1] * K * 2 < 1 << 32 and a.shape[0] * a.stride(0) * 2 < 1 << 32)
 
@@ -380,11 +381,12 @@ _GROUP_COST = {1: (0.0, 0.632, 2.7, 0.0, 0.0957, 0.701, 3.45), 2: (1.58, 0.488, 
 
 
 @functools.lru_cache(maxsize=4096)
-def _grouped_tile(rows: int, E: int, N: int, K: int, pair: bool, even: bool = False) -> int:
+def _grouped_tile(rows: int, E: int, N: int, K: int, pair: bool, even: bool = False, common: int = 0) -> int:
     """Configuration of the grouped big-tile product: the cheapest of them all by _GROUP_COST, for groups of the same size (``even``)
-    or of about equal size drawn at random, whose tiles are expected ones: up to 5 that would begin another round most often are
+    or of about equal size drawn at random beside ``common`` rows that are the last group's, whose tiles are expected ones: up to 5 that would begin another round most often are
     not there (1700 rows of 16 experts, 2 x 2048 x 4096: 260.5 tiles expected, 136 us in one round, 152 the next best)."""
-    r, n, kt, best = rows / E, (2 * N if pair else N), K / 64, None
+    drawn = E - (common > 0)
+    r, n, kt, best = (rows - common) / max(drawn, 1), (2 * N if pair else N), K / 64, None
     for cfg, (t0, tile, rnd, step, wmb, omb, act_us) in _GROUP_COST.items():
         bp, bq = _GROUP_TILE[cfg]
         if even or E == 1:
@@ -392,7 +394,7 @@ def _grouped_tile(rows: int, E: int, N: int, K: int, pair: bool, even: bool = Fa
         else:   # a group's tiles beyond k: the chance that it has more than bq k rows, 1 up to six deviations below the mean
             d = 6.0 * math.sqrt(max(r, 1.0))
             sure = max(0, int((r - d) // bq))
-            tiles = E * (1 + sure + sum(0.5 + 0.5 * math.erf((r - bq * k) / math.sqrt(2.0 * max(r, 1.0)))
+            tiles = -(-common // bq) + drawn * (1 + sure + sum(0.5 + 0.5 * math.erf((r - bq * k) / math.sqrt(2.0 * max(r, 1.0)))
                                         for k in range(sure + 1, int((r + d) / bq) + 2)))
             spare = 0.02
         rounds = max(1, math.ceil(tiles * -(-n // bp) / 256 - spare))
@@ -403,12 +405,13 @@ def _grouped_tile(rows: int, E: int, N: int, K: int, pair: bool, even: bool = Fa
     return best[1]
 
 
-def _pgemm4_grouped(a, w, a_rows, rows: int, seg, N: int, kind: int = -1, limit: float = 0.0, alpha: float = 1.0):
+def _pgemm4_grouped(a, w, a_rows, rows: int, seg, N: int, kind: int = -1, limit: float = 0.0, alpha: float = 1.0, common: int = 0,
+                    common_limit: Optional[float] = None):
     E, _, K = w.shape
     out = torch.empty(rows, N, dtype=BF16, device=a.device)
     _native().pgemm4_grouped(out.data_ptr(), a.data_ptr(), w.data_ptr(), a.shape[0], rows, N, K, E, _p(seg, I32, "seg"),
-                             _p(a_rows, I32, "a_rows"), a.stride(0), _grouped_tile(rows, E, N, K, kind >= 0, seg is None), 4, kind,
-                             float(limit), float(alpha), -1)
+                             _p(a_rows, I32, "a_rows"), a.stride(0), _grouped_tile(rows, E, N, K, kind >= 0, seg is None, common), 4, kind,
+                             float(limit), float(alpha), float(limit if common_limit is None else common_limit), -1)
     return out
 
 
@@ -450,23 +453,30 @@ def _each_once(a: torch.Tensor, w: torch.Tensor) -> bool:
 
 def gemm_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, alpha: float = 1.0, *,
              a_rows: Optional[torch.Tensor] = None, tiles: Optional[torch.Tensor] = None, rows: int = 0,
-             seg: Optional[torch.Tensor] = None) -> torch.Tensor:
+             seg: Optional[torch.Tensor] = None, common: int = 0, common_limit: Optional[float] = None) -> torch.Tensor:
     """act(gemm(a, w)) of a grouped product and a gated kind, w [E, 2 N, K] = gate | up: in the product's epilogue where
-    it runs on the big-tile kernel (the sums are then not rounded ahead of the activation)."""
-    N = w.shape[1] // 2
+    it runs on the big-tile kernel (the sums are then not rounded ahead of the activation).  ``common``, ``seg``: as in
+    :func:`gemm`; the last group's limit is then ``common_limit``, if given."""
+    N, E = w.shape[1] // 2, w.shape[0]
+    own = common > 0 and common_limit is not None and common_limit != limit
     if a.shape[-1] == w.shape[-1] and w.shape[1] % 2 == 0 and a.dtype == w.dtype and _gpu(a, w) and \
             _grouped_big(a, w, seg, rows, N):
-        return _pgemm4_grouped(a, w, a_rows, rows, seg, N, kind, limit, alpha)
+        return _pgemm4_grouped(a, w, a_rows, rows, seg, N, kind, limit, alpha, common, common_limit if own else None)
     if tiles is not None and w.dim() == 3 and kind in (ACT_GELU_TANH, ACT_SWISH_CLAMP, ACT_RELU) and 0 < rows <= 512 and \
-            rows <= 32 * tiles.shape[0] and (rows >= 6 * w.shape[0] or w.shape[1] * w.shape[2] <= 1 << 22) and \
+            rows <= 32 * tiles.shape[0] and (rows >= 6 * E or own or w.shape[1] * w.shape[2] <= 1 << 22) and \
             w.shape[1] % 2 == 0 and a.dim() == 2 and _few_fits(a, w):
         # (16 experts of 2 x 2048 x 4096: 8 rows 53 / 56 us, 64 rows 102 / 102 us, 96 rows 109 / 105 us)
         out = torch.empty(rows, N, dtype=BF16, device=a.device)
         _native().gemm_few_act(out.data_ptr(), a.data_ptr(), w.data_ptr(), rows, N, w.shape[2], a.stride(0),
                                _p(a_rows, I32, "a_rows"), _p(tiles, I32, "tiles"), tiles.shape[0], kind, float(limit),
-                               float(alpha), -1)
+                               float(alpha), E - 1 if own else -1, float(common_limit if own else 0.0), -1)
         return out
-    return act(gemm(a, w, a_rows=a_rows, tiles=tiles, rows=rows, seg=seg), kind, limit, alpha)
+    y = gemm(a, w, a_rows=a_rows, tiles=tiles, rows=rows, seg=seg, common=common)
+    out = act(y, kind, limit, alpha)
+    if own:
+        mine = torch.arange(rows, device=y.device) >= seg[E - 1]
+        out = torch.where(mine.unsqueeze(-1), act(y, kind, common_limit, alpha), out)
+    return out
 
 
 def linear_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, alpha: float = 1.0, *,
@@ -833,6 +843,15 @@ def moe_combine(D: torch.Tensor, pos_of_pair: torch.Tensor, topk_w: Optional[tor
                           _p(logits, F32), logits.stride(0) if logits is not None else 0, sg_col, T, W, top,
                           _f32(D.dtype), -1)
     return z
+
+
+def joint_experts(E: int, W: int, F: int) -> bool:
+    """Whether a shared expert of the E others' size runs as one more group of their products: sizes that the big tiles take with
+    any number of rows.  Two launches less a layer, and its rows fill the other groups' rounds: us, apart / joined (8 experts, top
+    2; products of a layer, weights from memory): W = F = 2048, 1 token 29.9 / 25.7, 32 61.4 / 57.8, 97 66.8 / 58.7, 333 83.0 / 67.1,
+    1531 151 / 133, 2048 183 / 172; W = 4096, F = 3584, 1 66.3 / 62.3, 32 156 / 150, 97 170 / 153, 200 188 / 197, 700 252 / 263, 1024 335 /
+    289, 2048 533 / 509."""
+    return E + 1 <= GROUP_BIG_MAX_GROUPS and W % 64 == 0 and F % 64 == 0 and W >= 128 and F >= 128
 
 
 class MoeBranch(NamedTuple):
