@@ -163,6 +163,9 @@ int k8s_gemm_few_act(void* C, const void* A, const void* W, int M, int N, int K,
                      hipStream_t s);
 int k8s_gemv_act(void* out, void* partial, const void* x, const void* W, int M, int N_out, int K, int kind, float limit, float alpha,
                  hipStream_t stream);
+int k8s_norm_gemv(void* out, float* x_out, const float* x, const void* branch, long ldb, int b32, const void* w1, float mult,
+                  const void* gate, long ldg, int gate_silu, const void* nw, float offset, float gain, float eps, const void* W,
+                  int M, int N_out, int K, int kind, float limit, float alpha, hipStream_t stream);
 int k8s_gemv_act_plan(int M, int N_out, int K, int pair, int* ks, int* splits, int* wgs, int* per);
 int k8s_sgemv_act(void* out, void* partial, const void* x, const void* W, int M, int N, int K, int kind, float limit, float alpha,
                   hipStream_t stream);
@@ -361,6 +364,14 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
   m.def("pgemm_set_prio", [](int mode) { return k8s_pgemm_set_prio(mode); });
   m.def("pgemm_set_row_slabs", [](int on) { return k8s_pgemm_set_row_slabs(on); });
   m.def("gemv_set_wide", [](int on) { return k8s_gemv_set_wide(on); });
+  m.def("norm_gemv", [](uintptr_t out, uintptr_t x_out, uintptr_t x, uintptr_t branch, long ldb, int b32, uintptr_t w1, float mult,
+                        uintptr_t gate, long ldg, int gate_silu, uintptr_t nw, float offset, float gain, float eps, uintptr_t W,
+                        int M, int N, int K, int kind, float limit, float alpha, int64_t s) {
+    const int rc = k8s_norm_gemv(P(out), P<float>(x_out), P<float>(x), P(branch), ldb, b32, P(w1), mult, P(gate), ldg, gate_silu,
+                                 P(nw), offset, gain, eps, P(W), M, N, K, kind, limit, alpha, S(s));
+    if (rc != -5) check(rc, "norm_gemv");
+    return rc != -5;    // false: sizes that it does not take, nothing was launched
+  });
   m.def("gemv_act", [](uintptr_t out, uintptr_t partial, uintptr_t x, uintptr_t W, int M, int N, int K, int kind, float limit,
                        float alpha, int64_t s) {
     const int rc = k8s_gemv_act(P(out), P(partial), P(x), P(W), M, N, K, kind, limit, alpha, S(s));

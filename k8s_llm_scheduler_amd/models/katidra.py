@@ -375,50 +375,55 @@ class KatidraModel(StreamModel):
         return sum(4 * m.heads * sm.gated_scan_record(sm.SCAN_DECAY, m.dim, m.vdim) for m in self._scans)
 
     # ------------------------------------------------------------------ layers
-    def _lightning(self, w: _Lightning, cache: int, h, b) -> torch.Tensor:
-        m = w.cfg
+    def _lightning(self, w: _Lightning, cache: int, proj, b) -> torch.Tensor:
+        m = w.cfg                                                          # proj [T, q | k | v | gate]
         H, D, V = m.heads, m.dim, m.vdim
-        proj = sm.linear(h, w.w_in)                                        # [T, q | k | v | gate]
         y = sm.gated_scan(proj, sm.SCAN_DECAY, w.cols, None, self.states[cache], b["cu_q"], b["seq_slots"],
                           b["positions"], H, D, V, self.cfg.rms_eps, F32, head_params=w.decay, groups=H,
                           max_qlen=b.get("max_qlen", 0))
-        y = sm.norm_mix(y, w.norm, None, None, self.cfg.rms_eps, out_dtype=self.dtype,
-                        gate=proj[:, w.cols["g"]:w.cols["g"] + H * V])
-        return sm.linear(y, w.o)
+        return sm.norm_linear(None, y, w.norm, self.cfg.rms_eps, w.o, gate=proj[:, w.cols["g"]:w.cols["g"] + H * V])[0]
 
-    def _latent(self, w: _Latent, cache: int, h, b) -> torch.Tensor:
-        m = w.cfg
-        T = h.shape[0]
+    def _latent(self, w: _Latent, cache: int, proj, b) -> torch.Tensor:
+        m = w.cfg                                                          # proj [T, dq | dkv | gate]
         H, Dn, R, C, V = m.heads, m.dim, m.rot_dim, m.kv_rank, m.vdim
         eps, kv = self.cfg.rms_eps, self.kv_cache[cache]
-        proj = sm.linear(h, w.w_in)                                        # [T, dq | dkv | gate]
-        cq = sm.norm_mix(proj[:, w.cols["dq"]:w.cols["dq"] + m.q_rank], w.dq_norm, None, None, eps)
-        q = sm.linear(cq, w.uq)                                            # [T, H (Dn + R)]
+        q, _ = sm.norm_linear(None, proj[:, w.cols["dq"]:w.cols["dq"] + m.q_rank], w.dq_norm, eps, w.uq)     # [T, H (Dn + R)]
         sm.latent_kv_write(kv, proj[:, w.cols["dkv"]:w.cols["dkv"] + C + R], w.dkv_norm, q, w.cos_sin, b["positions"],
                            b["slot_mapping"], C, R, H, Dn, m.rot_dims, eps, interleaved=True)
         a = sm.latent_mix(q, kv, w.uk_t, w.uv, w.ukv, b, C, R, H, Dn, V, m.window, m.scale, self.block_size,
                           gate=proj[:, w.cols["g"]:w.cols["g"] + H])
         return sm.linear(a, w.o)
 
-    def _blocks(self, ids, b, after=None) -> torch.Tensor:
-        """The residual stream after the last layer."""
+    def _blocks(self, ids, b, after=None):
+        """The residual stream before the last sublayer's output is added, that output and the weight of the norm on it."""
         c, dt = self.cfg, self.dtype
-        x, h = sm.embed_rows(ids, self.embed, c.embed_scale, copy=True)    # h: the stream as the next sublayer reads it
+        x, h = sm.embed_rows(ids, self.embed, c.embed_scale, copy=True)    # h: the stream as the first sublayer reads it
+        pend = None                       # the output not yet added: the product that reads the stream next norms and adds it
         for L in self.layers:
             w = L.w
+            if pend is None:
+                proj = sm.linear(h, w.mixer.w_in)
+            else:
+                proj, x = sm.norm_linear(x, *pend, c.rms_eps, w.mixer.w_in)
             run = self._lightning if isinstance(w.mixer, _Lightning) else self._latent
-            h = sm.branchnorm(x, run(w.mixer, L.cache, h, b), w.n1, c.rms_eps, out_dtype=dt)
+            pend = (run(w.mixer, L.cache, proj, b), w.n1)
             if w.w_up is not None:
-                f = sm.linear(sm.linear_act(h, w.w_up, sm.ACT_RELU2), w.w_down)
-                h = sm.branchnorm(x, f, w.n2, c.rms_eps, out_dtype=dt)
+                f, x = sm.norm_linear(x, *pend, c.rms_eps, w.w_up, act_kind=sm.ACT_RELU2)
+                pend = (sm.linear(f, w.w_down), w.n2)
             if after is not None:
+                h = sm.branchnorm(x, *pend, c.rms_eps, out_dtype=dt)
+                pend = None
                 after.append(x.clone())
-        return x
+        return (x, *(pend or (None, None)))
 
     def _forward(self, ids, b, rows) -> torch.Tensor:
-        x = self._blocks(ids, b)
-        hf = sm.resnorm(pick_rows(x, rows), self.final_norm, self.cfg.rms_eps, out_dtype=self.dtype)
-        return sm.linear(hf, self.lm_head, out_dtype=F32).unsqueeze(0)     # [1, S, vocab]
+        x, branch, w = self._blocks(ids, b)
+        if branch is None:                # no layers
+            hf = sm.resnorm(pick_rows(x, rows), self.final_norm, self.cfg.rms_eps, out_dtype=self.dtype)
+            return sm.linear(hf, self.lm_head, out_dtype=F32).unsqueeze(0)
+        out, _ = sm.norm_linear(pick_rows(x, rows), pick_rows(branch, rows), w, self.cfg.rms_eps, self.lm_head, out_dtype=F32,
+                                next_w=self.final_norm)
+        return out.unsqueeze(0)                                            # [1, S, vocab]
 
     def residual_after_runs(self, ids, b) -> List[torch.Tensor]:
         """(debugging / tests) the fp32 residual stream after every layer."""

@@ -510,6 +510,58 @@ def linear_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, 
 
 
 # ----------------------------------------------------------------------------- recurrent mixer
+NORM_GEMV_MAX_M = 2       # rows (norm_gemv.hip)
+
+
+def norm_linear(x: Optional[torch.Tensor], branch: torch.Tensor, w: Optional[torch.Tensor], eps: float, weight: torch.Tensor, *,
+                act_kind: Optional[int] = None, limit: float = 0.0, alpha: float = 1.0, out_dtype=None, mult: float = 1.0,
+                next_w: Optional[torch.Tensor] = None, offset: float = 0.0, gain: float = 1.0, gate: Optional[torch.Tensor] = None,
+                gate_kind: int = GATE_SIGMOID):
+    """A product and the norms between it and the output ``branch`` of the sublayer before, (out, stream): with a stream x (fp32 [T,
+    W]) first x + ``mult`` * branch (``w`` None: :func:`resnorm`) or x + rms-norm(branch) * w (:func:`branchnorm`), that row itself or,
+    with ``next_w``, its rms-norm * (``offset`` + next_w) * ``gain`` -- without one rms-norm(branch) * w, times ``gate``'s sigmoid or
+    silu (:func:`norm_mix`) -- times ``weight``, with :func:`linear_act`'s activation if ``act_kind`` is given.  The stream is a new
+    tensor or x itself, updated: the caller goes on with what is returned.  One or two bf16 rows run in one launch; more, or other
+    sizes, as the norm and the product."""
+    T, W = branch.shape
+    dt = weight.dtype
+    if T <= NORM_GEMV_MAX_M and dt == BF16 and FAST_GEMM and not _ops.LEAN and _ops.GEMM_BACKEND == "auto" and _ops.GEMV_MAX_M >= T > 0 and \
+            _gpu(branch, weight, x, w, next_w, gate) and weight.is_contiguous() and branch.stride(1) == 1 and weight.shape[1] == W:
+        pair = act_kind in (ACT_GELU_TANH, ACT_SWISH_CLAMP, ACT_RELU)
+        b32, N = branch.dtype == F32, weight.shape[0] // 2 if pair else weight.shape[0]
+        ok = act_kind is None or act_kind == ACT_RELU2 or (pair and weight.shape[0] % 2 == 0)
+        ok = ok and out_dtype in (None, BF16, F32) and (act_kind is None or out_dtype != F32) and branch.dtype in (BF16, F32)
+        for t, d in ((w, branch.dtype), (next_w, BF16)):
+            ok = ok and (t is None or (t.dtype == d and t.numel() == W and t.is_contiguous()))
+        if x is not None:
+            ok = ok and x.dtype == F32 and x.shape == branch.shape and x.is_contiguous() and not b32 and gate is None
+        else:
+            ok = ok and w is not None and next_w is None and (gate is None or (gate.dtype == BF16 and gate.shape == branch.shape
+                                                                               and gate.stride(1) == 1))
+        if ok:
+            out = torch.empty(T, N, dtype=out_dtype or BF16, device=branch.device)
+            new = torch.empty_like(x) if x is not None else None
+            kind = act_kind if act_kind is not None else -2 if out_dtype == F32 else -1
+            if _native().norm_gemv(out.data_ptr(), _p(new), _p(x), branch.data_ptr(), branch.stride(0), int(b32), _p(w), float(mult),
+                                   gate.data_ptr() if gate is not None else 0, gate.stride(0) if gate is not None else 0,
+                                   int(gate_kind == GATE_SILU), _p(next_w), float(offset), float(gain), float(eps), weight.data_ptr(),
+                                   T, N, W, kind, float(limit), float(alpha), -1):
+                return out, new
+    if x is None:
+        h = norm_mix(branch, w, None, None, eps, out_dtype=dt, gate=gate, gate_kind=gate_kind)
+    elif w is not None:
+        if offset:
+            raise ValueError("norm_linear: branchnorm's second norm has no offset")
+        h = branchnorm(x, branch, w, eps, out_dtype=dt, next_w=next_w, gain=gain)
+    else:
+        if next_w is None or gain != 1.0:
+            raise ValueError("norm_linear: resnorm's row is normed, without a gain")
+        h = resnorm(x, next_w, eps, branch=branch, mult=mult, offset=offset, out_dtype=dt)
+    if act_kind is not None:
+        return linear_act(h, weight, act_kind, limit, alpha), x
+    return linear(h, weight, out_dtype), x
+
+
 def token_shift(h: torch.Tensor, mu: torch.Tensor, state: torch.Tensor, cu_q: torch.Tensor, tok_seq: torch.Tensor,
                 seq_slots: torch.Tensor, positions: torch.Tensor, save: bool = False) -> torch.Tensor:
     """[n, T, W]: h + (previous token's h - h) * mu[s]; the previous token of a portion's first token is the slot's

@@ -1,0 +1,114 @@
+"""One or two rows times a weight matrix with the norms in the prologue, against 64 bits: widths at the ends of a thread's chunks and
+of a lane's blocks, column counts at the ends of a row set, every form of norm and output; what it does not take runs as two launches."""
+import pytest
+import torch
+
+from k8s_llm_scheduler_amd import ops
+from k8s_llm_scheduler_amd.ops import seqmix as sm
+
+pytestmark = pytest.mark.gpu
+DEV, EPS = "cuda", 1e-5
+
+
+@pytest.fixture
+def entries(monkeypatch):
+    nat, seen = ops.native(), []
+
+    class Spy:
+        def __getattr__(self, name):
+            seen.append(name)
+            return getattr(nat, name)
+
+    monkeypatch.setattr(ops, "native", Spy)
+    return seen
+
+
+def rms(v):
+    return v * (v.square().mean(-1, keepdim=True) + EPS).rsqrt()
+
+
+def reference(x, b, w, nw, mult, offset, gain, gate, silu):
+    """(h, stream) in 64 bits."""
+    d = lambda t: None if t is None else t.double()
+    x, b, w, nw, gate = map(d, (x, b, w, nw, gate))
+    y = rms(b) * w if w is not None else mult * b
+    if x is not None:
+        y = x + y
+    if gate is not None:
+        y = y * (torch.nn.functional.silu(gate) if silu else torch.sigmoid(gate))
+    return (y if nw is None else rms(y) * (offset + nw) * gain), (None if x is None else y)
+
+
+FORMS = {"branch": dict(w=1), "both": dict(w=1, nw=1, gain=0.5), "sum": dict(nw=1, mult=0.7, offset=1.0), "alone": dict(x=0, w=1),
+         "gated": dict(x=0, w=1, gate=1), "silu32": dict(x=0, w=1, gate=1, silu=1, b32=1), "alone32": dict(x=0, w=1, b32=1)}
+
+
+def check(form, M, N, K, act, out_dtype, entries, fused=True):
+    f = dict(dict(x=1, w=0, nw=0, mult=1.0, offset=0.0, gain=1.0, gate=0, silu=0, b32=0), **FORMS[form])
+    g = torch.Generator().manual_seed(M + N + K)
+    r = lambda *s, dt=torch.bfloat16, m=1.0: (torch.randn(*s, generator=g) * m).to(dt).to(DEV)
+    bdt = torch.float32 if f["b32"] else torch.bfloat16
+    x = r(M, K, dt=torch.float32, m=3.0) if f["x"] else None
+    b = r(M, K + 24, dt=bdt, m=2.0)[:, 8:K + 8] if not f["x"] else r(M, K, m=2.0)
+    w, nw = (r(K, dt=bdt) if f["w"] else None), (r(K) if f["nw"] else None)
+    gate = r(M, K + 16)[:, 16:] if f["gate"] else None
+    pair = act in (sm.ACT_GELU_TANH, sm.ACT_SWISH_CLAMP, sm.ACT_RELU)
+    W = r(N * (2 if pair else 1), K, m=K ** -0.5)
+    h, y = reference(x, b, w, nw, f["mult"], f["offset"], f["gain"], gate, f["silu"])
+    kw = dict(mult=f["mult"], next_w=nw, offset=f["offset"], gain=f["gain"], gate=gate,
+              gate_kind=sm.GATE_SILU if f["silu"] else sm.GATE_SIGMOID, act_kind=act, limit=1.5, alpha=1.702, out_dtype=out_dtype)
+    x0 = None if x is None else x.clone()
+    entries.clear()
+    got, new = sm.norm_linear(x, b, w, EPS, W, **kw)
+    if fused:
+        assert entries == ["norm_gemv"]
+        assert x is None or torch.equal(x, x0)              # a new stream beside the old one
+    if y is None:
+        assert new is None
+    else:                                                    # fp32: the norm's sums, two divisions and a root
+        assert (new.double() - y).abs().max() <= 2.0 ** -20 * y.abs().max()
+    # h rounded to bf16, then sums of K products in fp32
+    e = 2.0 ** -8 * 1.01 * (h.abs() @ W.double().abs().T) + 2.0 * K * 2.0 ** -24 * (h.abs() @ W.double().abs().T)
+    z = h @ W.double().T
+    if act is None:
+        out = 2.0 ** -8 * z.abs() if out_dtype != torch.float32 else 0.0
+        assert ((got.double() - z).abs() <= e + out + 1e-30).all()
+    elif act == sm.ACT_RELU2:
+        want = z.clamp(min=0).square()
+        assert ((got.double() - want).abs() <= 2.0 * z.abs() * e + e * e + 2.0 ** -8 * want + 1e-30).all()
+    else:
+        gz, u = z.chunk(2, -1)
+        eg, eu = e.chunk(2, -1)
+        if act == sm.ACT_RELU:
+            want, slope = gz.clamp(min=0) * u, 1.0
+        elif act == sm.ACT_GELU_TANH:
+            want, slope = torch.nn.functional.gelu(gz, approximate="tanh") * u, 1.13
+        else:
+            gc, uc = gz.clamp(max=1.5), u.clamp(-1.5, 1.5)
+            want, slope, u = gc * torch.sigmoid(1.702 * gc) * (uc + 1.0), 1.1, uc + 1.0
+        assert ((got.double() - want).abs() <= slope * eg * u.abs() + gz.abs() * eu + slope * eg * eu + 2.0 ** -7 * want.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("form", sorted(FORMS))
+@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("K", [8, 512, 520, 2048, 2056, 4096])
+def test_forms_and_widths(form, M, K, entries):
+    for N in (1, 7, 2050):
+        check(form, M, N, K, None, None, entries)
+
+
+@pytest.mark.parametrize("act,out_dtype", [(None, None), (None, torch.float32), (sm.ACT_RELU2, None), (sm.ACT_GELU_TANH, None),
+                                           (sm.ACT_SWISH_CLAMP, None), (sm.ACT_RELU, None)])
+@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("N", [4, 4095, 4096, 8193, 20001])
+def test_outputs_and_row_sets(act, out_dtype, M, N, entries):
+    """Column counts around the change to two weight rows a wave and to several row sets a wave."""
+    for form in ("branch", "sum"):
+        check(form, M, N, 1024, act, out_dtype, entries)
+
+
+@pytest.mark.parametrize("M,K", [(3, 256), (1, 4104), (2, 12), (1, 4)])
+def test_other_sizes_run_as_norm_and_product(M, K, entries):
+    for form in ("branch", "both", "sum", "gated"):
+        check(form, M, 64, K, None, None, entries, fused=False)
+        assert entries[-1] != "norm_gemv" and any(n in entries for n in ("branchnorm", "resnorm", "norm_mix"))
