@@ -375,44 +375,68 @@ class KatidraModel(StreamModel):
         return sum(4 * m.heads * sm.gated_scan_record(sm.SCAN_DECAY, m.dim, m.vdim) for m in self._scans)
 
     # ------------------------------------------------------------------ layers
-    def _lightning(self, w: _Lightning, cache: int, proj, b) -> torch.Tensor:
-        m = w.cfg                                                          # proj [T, q | k | v | gate]
+    def _lightning(self, w: _Lightning, cache: int, read, b) -> torch.Tensor:
+        m = w.cfg
         H, D, V = m.heads, m.dim, m.vdim
+        proj = read(w.w_in)                                                # [T, q | k | v | gate]
         y = sm.gated_scan(proj, sm.SCAN_DECAY, w.cols, None, self.states[cache], b["cu_q"], b["seq_slots"],
                           b["positions"], H, D, V, self.cfg.rms_eps, F32, head_params=w.decay, groups=H,
                           max_qlen=b.get("max_qlen", 0))
-        return sm.norm_linear(None, y, w.norm, self.cfg.rms_eps, w.o, gate=proj[:, w.cols["g"]:w.cols["g"] + H * V])[0]
+        gate = proj[:, w.cols["g"]:w.cols["g"] + H * V]
+        if y.shape[0] <= sm.NORM_GEMV_MAX_M:
+            return sm.norm_linear(None, y, w.norm, self.cfg.rms_eps, w.o, gate=gate)[0]
+        y = sm.norm_mix(y, w.norm, None, None, self.cfg.rms_eps, out_dtype=self.dtype, gate=gate)
+        del proj, gate
+        return sm.linear(y, w.o)
 
-    def _latent(self, w: _Latent, cache: int, proj, b) -> torch.Tensor:
-        m = w.cfg                                                          # proj [T, dq | dkv | gate]
+    def _latent(self, w: _Latent, cache: int, read, b) -> torch.Tensor:
+        m = w.cfg
         H, Dn, R, C, V = m.heads, m.dim, m.rot_dim, m.kv_rank, m.vdim
         eps, kv = self.cfg.rms_eps, self.kv_cache[cache]
-        q, _ = sm.norm_linear(None, proj[:, w.cols["dq"]:w.cols["dq"] + m.q_rank], w.dq_norm, eps, w.uq)     # [T, H (Dn + R)]
+        proj = read(w.w_in)                                                # [T, dq | dkv | gate]
+        dq = proj[:, w.cols["dq"]:w.cols["dq"] + m.q_rank]
+        if dq.shape[0] <= sm.NORM_GEMV_MAX_M:
+            q, _ = sm.norm_linear(None, dq, w.dq_norm, eps, w.uq)          # [T, H (Dn + R)]
+        else:
+            q = sm.linear(sm.norm_mix(dq, w.dq_norm, None, None, eps), w.uq)
         sm.latent_kv_write(kv, proj[:, w.cols["dkv"]:w.cols["dkv"] + C + R], w.dkv_norm, q, w.cos_sin, b["positions"],
                            b["slot_mapping"], C, R, H, Dn, m.rot_dims, eps, interleaved=True)
         a = sm.latent_mix(q, kv, w.uk_t, w.uv, w.ukv, b, C, R, H, Dn, V, m.window, m.scale, self.block_size,
                           gate=proj[:, w.cols["g"]:w.cols["g"] + H])
+        del proj, dq, q
         return sm.linear(a, w.o)
 
     def _blocks(self, ids, b, after=None):
         """The residual stream before the last sublayer's output is added, that output and the weight of the norm on it."""
         c, dt = self.cfg, self.dtype
-        x, h = sm.embed_rows(ids, self.embed, c.embed_scale, copy=True)    # h: the stream as the first sublayer reads it
-        pend = None                       # the output not yet added: the product that reads the stream next norms and adds it
-        for L in self.layers:
+        x, h = sm.embed_rows(ids, self.embed, c.embed_scale, copy=True)    # h: the stream as the next sublayer reads it
+        few = ids.shape[0] <= sm.NORM_GEMV_MAX_M and after is None
+        pend, last = None, len(self.layers) - 1       # few rows: the output not yet added, which the next product norms and adds
+
+        def read(weight, act=None):
+            nonlocal x
+            if pend is not None:
+                out, x = sm.norm_linear(x, *pend, c.rms_eps, weight, act_kind=act)
+                return out
+            return sm.linear(h, weight) if act is None else sm.linear_act(h, weight, act)
+
+        for i, L in enumerate(self.layers):
             w = L.w
-            if pend is None:
-                proj = sm.linear(h, w.mixer.w_in)
-            else:
-                proj, x = sm.norm_linear(x, *pend, c.rms_eps, w.mixer.w_in)
             run = self._lightning if isinstance(w.mixer, _Lightning) else self._latent
-            pend = (run(w.mixer, L.cache, proj, b), w.n1)
+            if few:
+                pend = (run(w.mixer, L.cache, read, b), w.n1)
+                if w.w_up is not None:
+                    pend = (sm.linear(read(w.w_up, sm.ACT_RELU2), w.w_down), w.n2)
+                continue
+            # (a batch's outputs are not held past the norm: the next product's rows take their memory, still in the caches)
+            if i == last and w.w_up is None and after is None:
+                return x, run(w.mixer, L.cache, read, b), w.n1
+            h = sm.branchnorm(x, run(w.mixer, L.cache, read, b), w.n1, c.rms_eps, out_dtype=dt)
             if w.w_up is not None:
-                f, x = sm.norm_linear(x, *pend, c.rms_eps, w.w_up, act_kind=sm.ACT_RELU2)
-                pend = (sm.linear(f, w.w_down), w.n2)
+                if i == last and after is None:
+                    return x, sm.linear(read(w.w_up, sm.ACT_RELU2), w.w_down), w.n2
+                h = sm.branchnorm(x, sm.linear(read(w.w_up, sm.ACT_RELU2), w.w_down), w.n2, c.rms_eps, out_dtype=dt)
             if after is not None:
-                h = sm.branchnorm(x, *pend, c.rms_eps, out_dtype=dt)
-                pend = None
                 after.append(x.clone())
         return (x, *(pend or (None, None)))
 

@@ -443,9 +443,11 @@ class PutulornModel(StreamModel):
         mix = sm.token_shift(h, w.mu, shift, b["cu_q"], b["tok_seq"], b["seq_slots"], b["positions"], save=True)   # [5, T, W]
         r, k, v, g = sm.linear_each(mix[:4], w.w_rkvg)
         lo = sm.linear_act(mix[4], w.w1, sm.ACT_TANH)
+        del mix
         z = sm.linear(lo, w.w2, out_dtype=torch.float32)                  # decay logits stay fp32
         y = sm.wkv_scan(r, k, v, g, z, w.w0, w.u, w.lnw, S, b["cu_q"], b["seq_slots"], b["positions"], m.heads, m.dim,
                         self.cfg.rms_eps)
+        del r, k, v, g, z, lo
         return sm.linear(y, w.o)
 
     def _latent(self, w: _Latent, run: _Run, h, b) -> torch.Tensor:
@@ -458,6 +460,7 @@ class PutulornModel(StreamModel):
         sm.latent_kv_write(cache, dkv, w.dkv_norm, q, w.cos_sin, b["positions"], b["slot_mapping"], C, R, H, Dn,
                            m.rot_dims, self.cfg.rms_eps)
         a = sm.latent_mix(q, cache, w.uk_t, w.uv, w.ukv, b, C, R, H, Dn, V, m.window, m.scale, self.block_size)
+        del q, dkv
         return sm.linear(a, w.o)
 
     def _mlp(self, w: _Mlp, h) -> torch.Tensor:
