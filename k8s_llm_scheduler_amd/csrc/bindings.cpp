@@ -123,6 +123,8 @@ int k8s_embed_rows(float* out, void* copy, const int* ids, const void* table, in
                    int f32, hipStream_t s);
 int k8s_decode_meta(int* pos, int* slots, int* ar, const int* ctx, const int* block_tables, int max_blocks, int B, int bs,
                     hipStream_t s);
+int k8s_norm_shift(void* out, float* x, const void* branch, float mult, const void* rowvec, const void* w, float offset, float eps,
+                   const void* mu, void* state, const int* seq_slots, const int* positions, int n, int T, int W, int f32, hipStream_t s);
 int k8s_resnorm(float* x, const void* branch, const void* branch2, float mult, const void* rowvec, const void* w,
                 float offset, float eps, void* out, int T, int W, int groups, int f32, hipStream_t s);
 int k8s_norm_mix(void* out, const void* a, long lda, const void* wa, const void* b, const void* wb, float eps, float ca,
@@ -166,6 +168,11 @@ int k8s_gemv_act(void* out, void* partial, const void* x, const void* W, int M, 
 int k8s_norm_gemv(void* out, float* x_out, const float* x, const void* branch, long ldb, int b32, const void* w1, float mult,
                   const void* gate, long ldg, int gate_silu, const void* nw, float offset, float gain, float eps, const void* W,
                   int M, int N_out, int K, int kind, float limit, float alpha, hipStream_t stream);
+long long k8s_rows_workspace(int M, int N, int K, int pair);
+int k8s_rows_out(float* y, void* h, float* sums, const float* x, const void* nw, const void* a, const void* W, void* partial, int M, int N,
+                 int K, float mult, float offset, hipStream_t stream);
+int k8s_rows_in(void* out, void* out2, int n1, const void* h, const float* sums, int count, const void* W, void* partial, int M, int N,
+                int K, float eps, int kind, float limit, float alpha, hipStream_t stream);
 int k8s_gemv_act_plan(int M, int N_out, int K, int pair, int* ks, int* splits, int* wgs, int* per);
 int k8s_sgemv_act(void* out, void* partial, const void* x, const void* W, int M, int N, int K, int kind, float limit, float alpha,
                   hipStream_t stream);
@@ -372,6 +379,23 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
     if (rc != -5) check(rc, "norm_gemv");
     return rc != -5;    // false: sizes that it does not take, nothing was launched
   });
+  m.def("rows_workspace", [](int M, int N, int K, int pair) { return k8s_rows_workspace(M, N, K, pair); });
+  // the number of sums a row, or 0: sizes that it does not take, nothing was launched
+  m.def("rows_out", [](uintptr_t y, uintptr_t h, uintptr_t sums, uintptr_t x, uintptr_t nw, uintptr_t a, uintptr_t W, uintptr_t partial,
+                       int M, int N, int K, float mult, float offset, int64_t s) {
+    const int rc = k8s_rows_out(P<float>(y), P(h), P<float>(sums), P<float>(x), P(nw), P(a), P(W), P(partial), M, N, K, mult, offset,
+                                S(s));
+    if (rc == -5) return 0;
+    check(rc <= -100 ? -100 - rc : rc < 0 ? rc : 0, "rows_out");
+    return rc;
+  });
+  m.def("rows_in", [](uintptr_t out, uintptr_t out2, int n1, uintptr_t h, uintptr_t sums, int count, uintptr_t W, uintptr_t partial,
+                      int M, int N, int K, float eps, int kind, float limit, float alpha, int64_t s) {
+    const int rc = k8s_rows_in(P(out), P(out2), n1, P(h), P<float>(sums), count, P(W), P(partial), M, N, K, eps, kind, limit, alpha,
+                               S(s));
+    if (rc != -5) check(rc, "rows_in");
+    return rc != -5;
+  });
   m.def("gemv_act", [](uintptr_t out, uintptr_t partial, uintptr_t x, uintptr_t W, int M, int N, int K, int kind, float limit,
                        float alpha, int64_t s) {
     const int rc = k8s_gemv_act(P(out), P(partial), P(x), P(W), M, N, K, kind, limit, alpha, S(s));
@@ -559,6 +583,14 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
                       float offset, float eps, uintptr_t out, int T, int W, int groups, int f32, int64_t s) {
     check(k8s_resnorm(P<float>(x), P(branch), P(branch2), mult, P(rowvec), P(w), offset, eps, P(out), T, W, groups, f32,
                       S(s)), "resnorm");
+  });
+  m.def("norm_shift", [](uintptr_t out, uintptr_t x, uintptr_t branch, float mult, uintptr_t rowvec, uintptr_t w, float offset,
+                         float eps, uintptr_t mu, uintptr_t state, uintptr_t seq_slots, uintptr_t positions, int n, int T, int W, int f32,
+                         int64_t s) {
+    const int rc = k8s_norm_shift(P(out), P<float>(x), P(branch), mult, P(rowvec), P(w), offset, eps, P(mu), P(state),
+                                  P<int>(seq_slots), P<int>(positions), n, T, W, f32, S(s));
+    if (rc != -5) check(rc, "norm_shift");
+    return rc != -5;
   });
   m.def("norm_mix", [](uintptr_t out, uintptr_t a, long lda, uintptr_t wa, uintptr_t b, uintptr_t wb, float eps,
                        float ca, float cb, int T, int W, int groups, uintptr_t gate, long ldg, int gkind, int in_f32,

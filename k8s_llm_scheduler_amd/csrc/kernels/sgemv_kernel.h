@@ -319,12 +319,27 @@ __device__ __forceinline__ void sm_store(void* out, size_t o, float a, float u, 
 constexpr int SM_TICKET_RANGE = 256, SM_TICKET_RANGES = 256;
 __device__ unsigned sm_tickets[SM_TICKET_RANGE * SM_TICKET_RANGES];
 
-template <int MT, int JT, int EPI, bool NORM, bool RES, bool FP8>
+// Products of a normed fp32 stream (stream_gemv.hip).  ROWS 1 adds to the stream and leaves what the next product's norm needs, ROWS
+// 2 reads that: the norm is a factor of each row, which a product's sums can take as well as its input.
+struct SmRows {
+  const float* x;          // 1: y = x + mult * product -> y (another buffer), h = bf16(y (offset + nw)), and of every workgroup's
+  float* y;                //    columns the rows' sums of y^2 -> sums[m][blockIdx.x]
+  bf16_t* h;
+  const bf16_t* nw;
+  float* sums;
+  const float* sums_in;    // 2: [M][count]; the product times gain / sqrt(sum / K + eps)
+  bf16_t* out2;            //    columns from n1 on (n1 = N: none), rows of N - n1; the others: rows of n1
+  int count, n1;
+  float mult, offset;
+};
+constexpr int SM_SUMS = 256;   // most workgroups that leave sums of a row
+
+template <int MT, int JT, int EPI, bool NORM, bool RES, bool FP8, int ROWS = 0>
 __global__ void __launch_bounds__(512) smfma_kernel(void* __restrict__ out, float* __restrict__ part,
                                                      const bf16_t* __restrict__ x, const void* __restrict__ W,
                                                      const float* __restrict__ wscale, const bf16_t* res, int M,
                                                      int N, int K, float eps, int band_rows, int jw,
-                                                     unsigned* tickets, EpiAct act) {
+                                                     unsigned* tickets, EpiAct act, SmRows rows) {
   constexpr int EPC = FP8 ? 16 : 8;                // k per 16-byte weight chunk
   constexpr int XG = MT / 4;                       // x groups of 4 rows (the B operand's 4 columns)
   constexpr int KQ = EPC / 4;                      // k-quads per chunk
@@ -339,6 +354,7 @@ __global__ void __launch_bounds__(512) smfma_kernel(void* __restrict__ out, floa
   static_assert((JT & (JT - 1)) == 0 && JT <= 8 && V <= 16, "bad smfma configuration");
   __shared__ float red[SM_KW][QMAX][4][MT];
   __shared__ float ssw[SM_KW][MT];
+  __shared__ float sq[ROWS == 1 ? 4 * QMAX * MT : 1];   // ROWS 1: the squares of the workgroup's outputs
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int kw = __builtin_amdgcn_readfirstlane(tid >> 6);   // (wave-uniform: the step masks below are scalar)
@@ -366,6 +382,20 @@ __global__ void __launch_bounds__(512) smfma_kernel(void* __restrict__ out, floa
             s < jv ? (unsigned)(4 * xg + r4) * K * 2 + (unsigned)(16 * (sb + s) + cb) * EPC * 2 : OOB;
 #pragma unroll
         for (int v = 0; v < XV; ++v) xr[s][xg][v] = __builtin_amdgcn_raw_buffer_load_b128(xs, off + 16 * v, 0, 0);
+      }
+  }
+
+  // wave kw's rows' sums, ahead of the weights as the x loads are
+  float rs[ROWS == 2 ? MT / SM_KW : 1][SM_SUMS / 64];
+  if constexpr (ROWS == 2) {
+    const auto ss = sg_rsrc(rows.sums_in, (long long)M * rows.count * 4);
+#pragma unroll
+    for (int r = 0; r < MT / SM_KW; ++r)
+#pragma unroll
+      for (int i = 0; i < SM_SUMS / 64; ++i) {
+        const int m = kw + SM_KW * r, c = lane + 64 * i;
+        rs[r][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                 ss, c < rows.count && m < M ? (unsigned)(m * rows.count + c) * 4 : OOB, 0, 0));
       }
   }
 
@@ -459,14 +489,28 @@ __global__ void __launch_bounds__(512) smfma_kernel(void* __restrict__ out, floa
     }
   }
 
+  if constexpr (ROWS == 2) {
+#pragma unroll
+    for (int r = 0; r < MT / SM_KW; ++r) {
+#pragma unroll
+      for (int i = 0; i < SM_SUMS / 64; ++i) asm volatile("" : "+v"(rs[r][i]));
+      const float t = wave_sum((rs[r][0] + rs[r][1]) + (rs[r][2] + rs[r][3]));
+      if (lane == 0) ssw[0][kw + SM_KW * r] = t;
+    }
+  }
+
   // the first epilogue pass's residual and row scales are requested now, behind the first weight set (clamped, so no
   // load sits under a branch): their latency hides under the weight stream instead of ending the kernel
-  float pre_res = 0.f, pre_sa = 1.f, pre_su = 1.f;
+  float pre_res = 0.f, pre_sa = 1.f, pre_su = 1.f;   // (ROWS 1: the stream and the next norm's weight)
   asm volatile("" ::: "memory");
   {
     const int idx = min(tid, band * M - 1);
     const int m = idx / band, n = b0 + idx - m * band;
     if constexpr (RES) pre_res = bf2f(res[(size_t)m * N + n]);
+    if constexpr (ROWS == 1) {
+      pre_res = rows.x[(size_t)m * N + n];
+      pre_sa = bf2f(rows.nw[n]);
+    }
     if constexpr (FP8) {
       pre_sa = wscale[n];
       if constexpr (sg_paired(EPI)) pre_su = wscale[N + n];
@@ -514,6 +558,32 @@ __global__ void __launch_bounds__(512) smfma_kernel(void* __restrict__ out, floa
 
   // ---- combine the 8 k-slices (fixed order), scale, epilogue
   const int G = gridDim.y;
+  auto store = [&](int idx, int m, int n, float a, float u) {
+    const size_t o = (size_t)m * N + n;
+    const bool first = idx == tid;
+    if constexpr (ROWS == 1) {
+      const float y = fmaf(rows.mult, a, first ? pre_res : rows.x[o]);
+      rows.y[o] = y;
+      rows.h[o] = f2bf(y * (rows.offset + (first ? pre_sa : bf2f(rows.nw[n]))));
+      sq[idx] = y * y;
+    } else if constexpr (ROWS == 2) {
+      const bool second = n >= rows.n1;
+      sm_store<EPI, false>(second ? rows.out2 : out, second ? (size_t)m * (N - rows.n1) + (n - rows.n1) : (size_t)m * rows.n1 + n, a,
+                           u, 0.f, act);
+    } else {
+      sm_store<EPI, RES>(out, o, a, u, RES ? (first ? pre_res : bf2f(res[o])) : 0.f, act);
+    }
+  };
+  auto row_sums = [&]() {   // after the last store
+    if constexpr (ROWS == 1) {
+      __syncthreads();
+      if (tid < M) {
+        float t = 0.f;
+        for (int c = 0; c < band; ++c) t += sq[tid * band + c];
+        rows.sums[tid * gridDim.x + blockIdx.x] = t;
+      }
+    }
+  };
   for (int idx = tid; idx < band * M; idx += 512) {
     const int m = idx / band, lr = idx - m * band;
     const int n = b0 + lr, qd = lr >> 2, i = lr & 3;
@@ -531,6 +601,11 @@ __global__ void __launch_bounds__(512) smfma_kernel(void* __restrict__ out, floa
       a *= inv;
       u *= inv;
     }
+    if constexpr (ROWS == 2) {
+      const float inv = 1.0f / sqrtf(ssw[0][m] / (float)K + eps);
+      a *= inv;
+      u *= inv;
+    }
     const bool first = idx == tid;
     if constexpr (FP8) {
       a *= first ? pre_sa : wscale[n];
@@ -543,9 +618,9 @@ __global__ void __launch_bounds__(512) smfma_kernel(void* __restrict__ out, floa
       if (sg_paired(EPI)) __hip_atomic_store(slab + N + n, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       continue;
     }
-    const size_t o = (size_t)m * N + n;
-    sm_store<EPI, RES>(out, o, a, u, RES ? (first ? pre_res : bf2f(res[o])) : 0.f, act);
+    store(idx, m, n, a, u);
   }
+  if (G == 1) row_sums();
   if (G == 1 || tickets == nullptr) return;   // (no tickets: sgemv_finalize_kernel sums the slabs)
 
   // ---- k-groups: the LAST workgroup of this band to finish sums the G slabs (fixed order, as the finalize kernel
@@ -570,9 +645,9 @@ __global__ void __launch_bounds__(512) smfma_kernel(void* __restrict__ out, floa
       a += __hip_atomic_load(slab + n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (sg_paired(EPI)) u += __hip_atomic_load(slab + N + n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    const size_t o = (size_t)m * N + n;
-    sm_store<EPI, RES>(out, o, a, u, RES ? (idx == tid ? pre_res : bf2f(res[o])) : 0.f, act);
+    store(idx, m, n, a, u);
   }
+  row_sums();
   if (tid == 0)   // ready for the next launch that draws this ticket range
     __hip_atomic_store(&tickets[blockIdx.x], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -645,12 +720,13 @@ static int sm_wg_cap() {
 }
 static std::atomic<unsigned> g_sm_next_range{0};   // of this unit's ranges, for every instantiation (launches on any stream)
 
-template <int MT, int JT, int EE, bool NN, bool RR, bool F8>
+template <int MT, int JT, int EE, bool NN, bool RR, bool F8, int ROWS = 0>
 static bool sm_launch(void* out, void* partial, const bf16_t* x, const void* W, const float* wscale, const bf16_t* res,
-                      int M, int N, int K, float eps, const SmPlan& sp, hipStream_t stream, EpiAct act = {}) {
+                      int M, int N, int K, float eps, const SmPlan& sp, hipStream_t stream, EpiAct act = {},
+                      const SmRows& rows = {}, int* bands = nullptr) {
   static const int occ = [] {
     int n = 1;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void*>(&smfma_kernel<MT, JT, EE, NN, RR, F8>),
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void*>(&smfma_kernel<MT, JT, EE, NN, RR, F8, ROWS>),
                                                      512, 0) != hipSuccess)
       n = 1;
     return max(1, min(n, sm_wg_cap()));
@@ -676,9 +752,12 @@ static bool sm_launch(void* out, void* partial, const bf16_t* x, const void* W, 
     if (hipGetSymbolAddress((void**)&base, HIP_SYMBOL(sm_tickets)) == hipSuccess)
       tk = base + (size_t)(g_sm_next_range.fetch_add(1) % SM_TICKET_RANGES) * SM_TICKET_RANGE;
   }
-  smfma_kernel<MT, JT, EE, NN, RR, F8><<<grid, 512, 0, stream>>>(out, part, x, W, wscale, res, M, N, K, eps, band,
-                                                                 sp.jw, tk, act);
-  return tk != nullptr;
+  if (bands != nullptr) *bands = (int)grid.x;
+  if constexpr (ROWS != 0)   // (its sums have SM_SUMS places, the reduction by a second launch knows no rows)
+    if ((ROWS == 1 && grid.x > (unsigned)SM_SUMS) || (sp.g > 1 && tk == nullptr)) return false;
+  smfma_kernel<MT, JT, EE, NN, RR, F8, ROWS><<<grid, 512, 0, stream>>>(out, part, x, W, wscale, res, M, N, K, eps, band,
+                                                                       sp.jw, tk, act, rows);
+  return ROWS != 0 || tk != nullptr;
 }
 
 }  // namespace k8sllm

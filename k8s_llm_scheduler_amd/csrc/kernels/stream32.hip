@@ -147,6 +147,75 @@ __global__ __launch_bounds__(256) void resnorm_row_kernel(float* __restrict__ x,
   }
 }
 
+// A step of single tokens: the row's norm (resnorm_row_kernel) and the token shift that reads it in one launch, which a chain of small
+// launches pays for twice: h = the norm's row, out[k] = h + (prev - h) mu[k] with prev the slot's row of `state` (zeros at position 0),
+// which becomes h; an idle row (position < 0) gives zeros and leaves the state alone.  As resnorm_row_kernel and token_shift_row_kernel
+// in turn, bit for bit.
+constexpr int SHIFT_MIXES = 5;
+template <typename TA, int NV>
+__global__ __launch_bounds__(256) void norm_shift_kernel(TA* __restrict__ out, float* __restrict__ x, const TA* __restrict__ branch,
+                                                         float mult, const TA* __restrict__ rowvec, const TA* __restrict__ w,
+                                                         float offset, float eps, const TA* __restrict__ mu, TA* __restrict__ state,
+                                                         const int* __restrict__ seq_slots, const int* __restrict__ positions, int n,
+                                                         int T, int W) {
+  __shared__ float red[4];
+  const int t = blockIdx.x;
+  const size_t base = (size_t)t * W;
+  const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int p = positions[t];
+  TA* row = state + (size_t)(p >= 0 ? seq_slots[t] : 0) * W;
+  f32x4 xv[NV], bv[NV], rv[NV], wv[NV], pv[NV], mv[SHIFT_MIXES][NV];
+#pragma unroll
+  for (int q = 0; q < NV; ++q) {
+    const int i = 4 * (threadIdx.x + 256 * q);
+    const bool in = i < W;
+    xv[q] = in ? ldf4(x + base + i) : zero;
+    bv[q] = in && branch != nullptr ? ldf4(branch + base + i) : zero;
+    rv[q] = in && rowvec != nullptr ? ldf4(rowvec + i) : zero;
+    wv[q] = in ? ldf4(w + i) : zero;
+#pragma unroll
+    for (int k = 0; k < SHIFT_MIXES; ++k) mv[k][q] = in && k < n ? ldf4(mu + (size_t)k * W + i) : zero;
+    pv[q] = in && p > 0 ? ldf4(row + i) : zero;
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int q = 0; q < NV; ++q) {
+    const int i = 4 * (threadIdx.x + 256 * q);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float v = xv[q][e];
+      if (branch != nullptr) v += mult * bv[q][e];
+      if (rowvec != nullptr) v += rv[q][e];
+      xv[q][e] = v;
+      ss += v * v;
+    }
+    if (i < W && (branch != nullptr || rowvec != nullptr)) stf4(x + base + i, xv[q]);
+  }
+  ss = row_total(ss, red);
+  const float inv = 1.0f / sqrtf(ss / (float)W + eps);
+#pragma unroll
+  for (int q = 0; q < NV; ++q) {
+    const int i = 4 * (threadIdx.x + 256 * q);
+    if (i >= W) continue;
+    f32x4 h, d;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      h[e] = xv[q][e] * inv * (offset + wv[q][e]);
+      if constexpr (sizeof(TA) == 2) h[e] = bf2f(f2bf(h[e]));
+      d[e] = pv[q][e] - h[e];
+    }
+#pragma unroll
+    for (int k = 0; k < SHIFT_MIXES; ++k) {
+      if (k >= n) break;
+      f32x4 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = p < 0 ? 0.f : h[e] + d[e] * mv[k][q][e];
+      stf4(out + ((size_t)k * T + t) * W + i, y);
+    }
+    if (p >= 0) stf4(row + i, h);
+  }
+}
+
 // Norm after the sum: x[t] <- (alpha x[t] + c1 branch[t] + c2 branch2[t]) / sqrt(mean(.^2) + eps) * gain, stored back
 // in fp32 (the stream stays normed); `out` (optional) receives the same row in the activation type, for the sublayer
 // that reads it next.  `gain` is one number for the whole row.  One workgroup per row; the row is held in registers
@@ -979,6 +1048,31 @@ extern "C" int k8s_resnorm(float* x, const void* branch, const void* branch2, fl
   else K8S_RN_T(bf16_t);
 #undef K8S_RN_T
 #undef K8S_RN
+  return (int)hipGetLastError();
+}
+
+// -5: a size or an alignment that this form does not take; nothing was launched
+extern "C" int k8s_norm_shift(void* out, float* x, const void* branch, float mult, const void* rowvec, const void* w, float offset,
+                              float eps, const void* mu, void* state, const int* seq_slots, const int* positions, int n, int T, int W,
+                              int f32, hipStream_t s) {
+  if (T <= 0) return 0;
+  if (W <= 0 || n <= 0 || w == nullptr || out == nullptr || state == nullptr || mu == nullptr) return -1;
+  if (n > SHIFT_MIXES || W % 4 || W > 4096 || (uintptr_t)x % 16 ||
+      ((uintptr_t)branch | (uintptr_t)rowvec | (uintptr_t)w | (uintptr_t)out | (uintptr_t)mu | (uintptr_t)state) % (f32 ? 16 : 8))
+    return -5;
+#define K8S_NS(TA, NV)                                                                                                       \
+  norm_shift_kernel<TA, NV><<<T, 256, 0, s>>>((TA*)out, x, (const TA*)branch, mult, (const TA*)rowvec, (const TA*)w, offset, eps, \
+                                              (const TA*)mu, (TA*)state, seq_slots, positions, n, T, W)
+#define K8S_NS_T(TA)                   \
+  do {                                 \
+    if (W <= 1024) K8S_NS(TA, 1);      \
+    else if (W <= 2048) K8S_NS(TA, 2); \
+    else K8S_NS(TA, 4);                \
+  } while (0)
+  if (f32) K8S_NS_T(float);
+  else K8S_NS_T(bf16_t);
+#undef K8S_NS_T
+#undef K8S_NS
   return (int)hipGetLastError();
 }
 

@@ -301,6 +301,7 @@ class _Latent:
     o: torch.Tensor         # [W, H V]
     cos_sin: torch.Tensor   # [positions, rot_dims] fp32
     ukv: Optional[torch.Tensor]   # [H (Dn + V), C]: both up-projections as one product (sm.latent_expand)
+    qdkv: Optional[torch.Tensor]  # q and dkv, which then are parts of it: one product of few rows
 
 
 @dataclass
@@ -378,10 +379,14 @@ class PutulornModel(StreamModel):
                 H, Dn, C, V = m.heads, m.dim, m.kv_rank, m.vdim
                 if m.rot_dims > m.rot_dim or m.rot_dims % 2:
                     raise ValueError(f"layer {i}: rot.dims {m.rot_dims} must be even and at most rot_dim {m.rot_dim}")
-                mixer = _Latent(m, t(get(p + "q")), t(get(p + "dkv")), t(get(p + "dkv.norm")),
+                q, dkv, qdkv = t(get(p + "q")), t(get(p + "dkv")), None
+                if sm.rows_join(1, W) and self.dtype == torch.bfloat16:
+                    qdkv = torch.cat([q, dkv])
+                    q, dkv = qdkv[:q.shape[0]], qdkv[q.shape[0]:]
+                mixer = _Latent(m, q, dkv, t(get(p + "dkv.norm")),
                                 t(get(p + "uk").reshape(H, Dn, C).transpose(1, 2)), t(get(p + "uv").reshape(H, V, C)),
                                 t(get(p + "o")), self._rope_table(m.rot_dims, m.rot_base),
-                                self._expand(get, p, H, m.rot_dim))
+                                self._expand(get, p, H, m.rot_dim), qdkv)
             f, mlp, n2 = L.mlp, None, None
             if f is not None:
                 q = f"l{i}.mlp."
@@ -437,31 +442,27 @@ class PutulornModel(StreamModel):
         return sum(m.cfg.heads * m.cfg.dim * m.cfg.dim * 4 + self.cfg.hidden * eb for _, m in self._wkv_runs())
 
     # ------------------------------------------------------------------ layers
-    def _wkv(self, w: _Wkv, run: _Run, h, b) -> torch.Tensor:
+    def _wkv(self, w: _Wkv, run: _Run, mixed, b) -> torch.Tensor:
+        """``mixed``(mu, state): the token-shifted inputs."""
         m = w.cfg
         S, shift = self.states[run.cache]
-        mix = sm.token_shift(h, w.mu, shift, b["cu_q"], b["tok_seq"], b["seq_slots"], b["positions"], save=True)   # [5, T, W]
+        mix = mixed(w.mu, shift)                                          # [5, T, W]
         r, k, v, g = sm.linear_each(mix[:4], w.w_rkvg)
         lo = sm.linear_act(mix[4], w.w1, sm.ACT_TANH)
         del mix
         z = sm.linear(lo, w.w2, out_dtype=torch.float32)                  # decay logits stay fp32
-        y = sm.wkv_scan(r, k, v, g, z, w.w0, w.u, w.lnw, S, b["cu_q"], b["seq_slots"], b["positions"], m.heads, m.dim,
-                        self.cfg.rms_eps)
-        del r, k, v, g, z, lo
-        return sm.linear(y, w.o)
+        return sm.wkv_scan(r, k, v, g, z, w.w0, w.u, w.lnw, S, b["cu_q"], b["seq_slots"], b["positions"], m.heads, m.dim,
+                           self.cfg.rms_eps)
 
-    def _latent(self, w: _Latent, run: _Run, h, b) -> torch.Tensor:
+    def _latent(self, w: _Latent, run: _Run, products, b) -> torch.Tensor:
+        """``products``(): the query [T, H (Dn + R)] and the latent row [T, C + R]."""
         m = w.cfg
-        T = h.shape[0]
         H, Dn, R, C, V = m.heads, m.dim, m.rot_dim, m.kv_rank, m.vdim
         cache = self.kv_cache[run.cache]
-        q = sm.linear(h, w.q)                                              # [T, H (Dn + R)]
-        dkv = sm.linear(h, w.dkv)                                          # [T, C + R]
+        q, dkv = products()
         sm.latent_kv_write(cache, dkv, w.dkv_norm, q, w.cos_sin, b["positions"], b["slot_mapping"], C, R, H, Dn,
                            m.rot_dims, self.cfg.rms_eps)
-        a = sm.latent_mix(q, cache, w.uk_t, w.uv, w.ukv, b, C, R, H, Dn, V, m.window, m.scale, self.block_size)
-        del q, dkv
-        return sm.linear(a, w.o)
+        return sm.latent_mix(q, cache, w.uk_t, w.uv, w.ukv, b, C, R, H, Dn, V, m.window, m.scale, self.block_size)
 
     def _mlp(self, w: _Mlp, h) -> torch.Tensor:
         f = w.cfg
@@ -480,25 +481,67 @@ class PutulornModel(StreamModel):
             shared = sm.linear(sm.linear_act(h, w.s_wgu, sm.ACT_SWISH_CLAMP, f.shared_limit, SWISH_ALPHA), w.s_down)
         return sm.moe_combine(D, pos, wts, shared, logits, w.sg_col)
 
+    def _mix(self, run: _Run, b, x, branch, step, r: Optional[sm.Rows]) -> torch.Tensor:
+        """The mixer's output ahead of its last product, of the stream x (+ ``branch`` and the loop pass's vector: x is updated) or of
+        the rows ``r`` that the product before left."""
+        L, eps = self.layers[run.layer], self.cfg.rms_eps
+        w = L.mixer
+        norm = dict(branch=branch, mult=self.cfg.residual_mult, rowvec=step, offset=1.0)
+        if isinstance(w, _Wkv):
+            if r is not None and r.sums is None:
+                mixed = lambda mu, s: sm.token_shift(r.h, mu, s, b["cu_q"], b["tok_seq"], b["seq_slots"], b["positions"], save=True)
+            else:
+                mixed = lambda mu, s: sm.norm_shift(x, L.n1, eps, mu, s, b, single="max_keys" in b, **norm)
+            return self._wkv(w, run, mixed, b)
+        if r is not None:
+            return self._latent(w, run, lambda: sm.rows_linear(r, w.qdkv, eps, split=w.q.shape[0]), b)
+        h = sm.resnorm(x, L.n1, eps, out_dtype=self.dtype, **norm)
+        return self._latent(w, run, lambda: (sm.linear(h, w.q), sm.linear(h, w.dkv)), b)
+
     def _forward(self, ids, b, rows) -> torch.Tensor:
         c, dt = self.cfg, self.dtype
         eps, mult = c.rms_eps, c.residual_mult
         x = sm.embed_rows(ids, self.embed)
-        pend = None                       # the branch output not yet added: the next norm adds it in fp32
-        for run in self.runs:
+        few = dt == torch.bfloat16 and sm.rows_join(ids.shape[0], c.hidden)   # the norms go with the products on both sides
+        pend = r = None                   # the branch output not yet added: the next norm adds it in fp32; or the rows as they are then
+        for i, run in enumerate(self.runs):
             L = self.layers[run.layer]
             step = self.loop_step[run.step] if run.step is not None else None
-            h = sm.resnorm(x, L.n1, eps, branch=pend, mult=mult, rowvec=step, offset=1.0, out_dtype=dt)
-            y = self._wkv(L.mixer, run, h, b) if isinstance(L.mixer, _Wkv) else self._latent(L.mixer, run, h, b)
-            if L.mlp is not None:
+            y = self._mix(run, b, x, pend, step, r)
+            pend, r, nxt = None, None, None
+            if few:                       # the norm that reads this layer's output
+                last = i + 1 == len(self.runs)
+                nxt = (self.final_norm if rows is None else None) if last else \
+                    self.layers[self.runs[i + 1].layer].n1 if self.runs[i + 1].step is None else None
+            o = L.mixer.o
+            if L.mlp is None:
+                if nxt is not None:
+                    r = sm.linear_rows(y, o, x, nxt, eps, mult=mult, offset=1.0)
+                else:
+                    pend = sm.linear(y, o)
+            elif few and L.mlp.cfg.kind == "dense":
+                r = sm.linear_rows(y, o, x, L.n2, eps, mult=mult, offset=1.0)
+                x = r.x
+                g = sm.rows_linear(r, L.mlp.wgu, eps, act_kind=sm.ACT_GELU_TANH)
+                if nxt is not None:
+                    r = sm.linear_rows(g, L.mlp.down, x, nxt, eps, mult=mult, offset=1.0)
+                else:
+                    pend, r = sm.linear(g, L.mlp.down), None
+            else:
+                y = sm.linear(y, o)
                 h = sm.resnorm(x, L.n2, eps, branch=y, mult=mult, offset=1.0, out_dtype=dt)
                 pend = self._mlp(L.mlp, h)
-            else:
-                pend = y
+            if r is not None:
+                x = r.x
+        if r is not None:
+            return sm.rows_linear(r, self.lm_head, eps, out_dtype=torch.float32).unsqueeze(0)
         xs = pick_rows(x, rows)
-        hf = sm.resnorm(xs, self.final_norm, eps, branch=pick_rows(pend, rows),
-                        mult=mult, offset=1.0, out_dtype=dt)
-        return sm.linear(hf, self.lm_head, out_dtype=torch.float32).unsqueeze(0)      # [1, S, vocab]
+        if pend is None:                  # no layers
+            hf = sm.resnorm(xs, self.final_norm, eps, offset=1.0, out_dtype=dt)
+            return sm.linear(hf, self.lm_head, out_dtype=torch.float32).unsqueeze(0)
+        out, _ = sm.norm_linear(xs, pick_rows(pend, rows), None, eps, self.lm_head, out_dtype=torch.float32, mult=mult,
+                                next_w=self.final_norm, offset=1.0)
+        return out.unsqueeze(0)                                                       # [1, S, vocab]
 
     def residual_after_runs(self, ids, b) -> List[torch.Tensor]:
         """(debugging / tests) the fp32 residual stream after every layer run."""
@@ -508,8 +551,7 @@ class PutulornModel(StreamModel):
         for run in self.runs:
             L = self.layers[run.layer]
             step = self.loop_step[run.step] if run.step is not None else None
-            h = sm.resnorm(x, L.n1, c.rms_eps, rowvec=step, offset=1.0, out_dtype=dt)
-            y = self._wkv(L.mixer, run, h, b) if isinstance(L.mixer, _Wkv) else self._latent(L.mixer, run, h, b)
+            y = sm.linear(self._mix(run, b, x, None, step, None), L.mixer.o)
             if L.mlp is not None:
                 h = sm.resnorm(x, L.n2, c.rms_eps, branch=y, mult=c.residual_mult, offset=1.0, out_dtype=dt)
                 y = self._mlp(L.mlp, h)

@@ -562,6 +562,88 @@ def norm_linear(x: Optional[torch.Tensor], branch: torch.Tensor, w: Optional[tor
     return linear(h, weight, out_dtype), x
 
 
+class Rows(NamedTuple):
+    """A stream and its rows as the next product reads them: normed (``sums`` None), or times the norm's weight alone with what is
+    missing of the norm, sums of squares."""
+    x: torch.Tensor
+    h: torch.Tensor
+    sums: Optional[torch.Tensor]      # [T, 256] of which the first T * count are used, rows of count
+    count: int
+    w: torch.Tensor                   # the norm's weight and what is added to it
+    offset: float
+
+
+def rows_join(T: int, W: int) -> bool:
+    """Whether T rows of a stream of W columns go from product to product as :class:`Rows` with sums (bf16)."""
+    return FAST_GEMM and not _ops.LEAN and _ops.GEMM_BACKEND == "auto" and 1 <= T <= _ops.SGEMV_MAX_M and W % 128 == 0 and W <= 4096
+
+
+def linear_rows(a: torch.Tensor, weight: torch.Tensor, x: torch.Tensor, next_w: torch.Tensor, eps: float, *, mult: float = 1.0,
+                offset: float = 0.0) -> Rows:
+    """x (fp32) + ``mult`` * linear(a, weight), a new tensor or x itself, updated, and its rows for :func:`rows_linear`, normed with
+    (``offset`` + next_w).  Up to 16 bf16 rows in one launch (stream_gemv.hip), which rounds neither the branch nor -- the norm's factor
+    being the next product's -- the rows more than once; otherwise the product and :func:`resnorm`."""
+    T, K = a.shape
+    N = weight.shape[0]
+    if rows_join(T, N) and _gpu(a, weight, x, next_w) and a.dtype == weight.dtype == next_w.dtype == BF16 and x.dtype == F32 and \
+            x.shape == (T, N) and weight.shape[1] == K and all(t.is_contiguous() for t in (a, weight, x, next_w)):
+        y, h = torch.empty_like(x), torch.empty(T, N, dtype=BF16, device=x.device)
+        sums = torch.empty(T, 256, dtype=F32, device=x.device)
+        n = _native().rows_workspace(T, N, K, 0)
+        part = torch.empty(n, dtype=F32, device=x.device) if n > 0 else None
+        count = _native().rows_out(_p(y), _p(h), _p(sums), _p(x), _p(next_w), a.data_ptr(), weight.data_ptr(), _p(part), T, N, K,
+                                   float(mult), float(offset), -1)
+        if count:
+            return Rows(y, h, sums, count, next_w, offset)
+    h = resnorm(x, next_w, eps, branch=linear(a, weight), mult=mult, offset=offset, out_dtype=weight.dtype)
+    return Rows(x, h, None, 0, next_w, offset)
+
+
+def rows_linear(r: Rows, weight: torch.Tensor, eps: float, *, act_kind: Optional[int] = None, limit: float = 0.0, alpha: float = 1.0,
+                out_dtype=None, split: int = 0):
+    """linear(rms-norm(r.x) * (r.offset + r.w), weight) or, with a gated kind, :func:`linear_act`; ``split``: two tensors, of the first
+    ``split`` rows of ``weight`` and of the others."""
+    h = r.h
+    if r.sums is not None:
+        T, K = h.shape
+        pair = act_kind in (ACT_GELU_TANH, ACT_SWISH_CLAMP, ACT_RELU)
+        N = weight.shape[0] // 2 if pair else weight.shape[0]
+        if weight.dtype == BF16 and weight.is_contiguous() and weight.shape[1] == K and out_dtype in (None, BF16, F32) and \
+                (act_kind is None or (pair and weight.shape[0] % 2 == 0 and out_dtype != F32)) and \
+                (not split or (act_kind is None and out_dtype != F32 and 0 < split < N)):
+            out = torch.empty(T, split or N, dtype=out_dtype or BF16, device=h.device)
+            rest = torch.empty(T, N - split, dtype=BF16, device=h.device) if split else None
+            n = _native().rows_workspace(T, N, K, int(pair))
+            part = torch.empty(n, dtype=F32, device=h.device) if n > 0 else None
+            kind = act_kind if act_kind is not None else -2 if out_dtype == F32 else -1
+            if _native().rows_in(out.data_ptr(), _p(rest), split or N, _p(h), _p(r.sums), r.count, weight.data_ptr(), _p(part), T, N, K,
+                                 float(eps), kind, float(limit), float(alpha), -1):
+                return (out, rest) if split else out
+        h = resnorm(r.x, r.w, eps, offset=r.offset, out_dtype=BF16)
+    if act_kind is not None:
+        return linear_act(h, weight, act_kind, limit, alpha)
+    if split:
+        return linear(h, weight[:split], out_dtype), linear(h, weight[split:], out_dtype)
+    return linear(h, weight, out_dtype)
+
+
+def norm_shift(x: torch.Tensor, w: torch.Tensor, eps: float, mu: torch.Tensor, state: torch.Tensor, b: dict, *,
+               branch: Optional[torch.Tensor] = None, mult: float = 1.0, rowvec: Optional[torch.Tensor] = None, offset: float = 0.0,
+               single: bool = False) -> torch.Tensor:
+    """:func:`token_shift`, with its save, of :func:`resnorm`'s rows in the type of ``w``, ``b`` a batch description; in one launch if
+    every sequence brings a single token (``single``)."""
+    T, W = x.shape
+    if single and _gpu(x, w, mu, state, branch, rowvec) and W % 4 == 0 and W <= 4096 and mu.shape[0] <= 5 and x.dtype == F32 and \
+            all(t is None or t.dtype == w.dtype for t in (mu, state, branch, rowvec)):
+        out = torch.empty(mu.shape[0], T, W, dtype=w.dtype, device=x.device)
+        if _native().norm_shift(_p(out), _p(x), _p(branch), float(mult), _p(rowvec), _p(w), float(offset), float(eps), _p(mu), _p(state),
+                                _p(b["seq_slots"], I32, "seq_slots"), _p(b["positions"], I32, "positions"), mu.shape[0], T, W,
+                                _f32(w.dtype), -1):
+            return out
+    h = resnorm(x, w, eps, branch=branch, mult=mult, rowvec=rowvec, offset=offset, out_dtype=w.dtype)
+    return token_shift(h, mu, state, b["cu_q"], b["tok_seq"], b["seq_slots"], b["positions"], save=True)
+
+
 def token_shift(h: torch.Tensor, mu: torch.Tensor, state: torch.Tensor, cu_q: torch.Tensor, tok_seq: torch.Tensor,
                 seq_slots: torch.Tensor, positions: torch.Tensor, save: bool = False) -> torch.Tensor:
     """[n, T, W]: h + (previous token's h - h) * mu[s]; the previous token of a portion's first token is the slot's

@@ -1,0 +1,129 @@
+"""Rows of an fp32 stream between the product that adds to it and the product that reads its norm, against 64 bits: widths and depths at
+the ends of a wave's steps and in several k-groups, output counts at the ends of a band, every output form, both parts of a split; and the
+norm with the token shift behind it, bit for bit as the two launches."""
+import pytest
+import torch
+
+from k8s_llm_scheduler_amd import ops
+from k8s_llm_scheduler_amd.ops import seqmix as sm
+
+pytestmark = pytest.mark.gpu
+DEV, EPS, BF, F32 = "cuda", 1e-5, torch.bfloat16, torch.float32
+
+
+@pytest.fixture
+def entries(monkeypatch):
+    nat, seen = ops.native(), []
+
+    class Spy:
+        def __getattr__(self, name):
+            seen.append(name)
+            return getattr(nat, name)
+
+    monkeypatch.setattr(ops, "native", Spy)
+    return seen
+
+
+def data(seed):
+    g = torch.Generator().manual_seed(seed)
+    return lambda *s, dt=BF, m=1.0: (torch.randn(*s, generator=g) * m).to(dt).to(DEV)
+
+
+def stream(r, M, K, N):
+    """Inputs of linear_rows, its stream in 64 bits and a bound of that: fp32 sums of K products in any order, one addition."""
+    x, a, w, nw = r(M, N, dt=F32, m=3.0), r(M, K), r(N, K, m=K ** -0.5), r(N, m=0.3)
+    b = a.double() @ w.double().T
+    mass = a.double().abs() @ w.double().abs().T
+    y = x.double() + 0.6 * b
+    return x, a, w, nw, y, 0.6 * 2.0 * K * 2.0 ** -24 * mass + 2.0 ** -23 * (y.abs() + b.abs())
+
+
+def read(y, nw):
+    return y * (1.0 + nw.double()) * (y.square().mean(-1, keepdim=True) + EPS).rsqrt()
+
+
+def close(got, y, ey, nw, w, out_dtype, act=None):
+    """The product of the normed rows: those rounded to bf16 once (2^-9 of a row, and y's own error), its sums in fp32, its output."""
+    K = y.shape[1]
+    h, W = read(y, nw), w.double()
+    slack = (ey / y.abs().clamp(min=1e-30) * h.abs()).clamp(max=1e3) + ey.square().mean(-1, keepdim=True).sqrt() * h.abs()
+    z, mass = h @ W.T, h.abs() @ W.abs().T
+    e = (2.0 ** -8 + 2.0 * K * 2.0 ** -24) * mass + slack @ W.abs().T
+    if act is None:
+        assert ((got.double() - z).abs() <= e + (2.0 ** -8 * z.abs() if out_dtype != F32 else 0) + 1e-30).all()
+        return
+    g, u = z.chunk(2, -1)
+    eg, eu = e.chunk(2, -1)
+    if act == sm.ACT_GELU_TANH:
+        want, slope = torch.nn.functional.gelu(g, approximate="tanh") * u, 1.13
+    elif act == sm.ACT_RELU:
+        want, slope = g.clamp(min=0) * u, 1.0
+    else:
+        g, u = g.clamp(max=1.5), u.clamp(-1.5, 1.5) + 1.0
+        want, slope = g * torch.sigmoid(1.702 * g) * u, 1.1
+    assert ((got.double() - want).abs() <= slope * eg * u.abs() + slope * (g.abs() * eu + eg * eu) + 2.0 ** -7 * want.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 8, 9, 16])
+@pytest.mark.parametrize("K,N", [(128, 128), (1152, 2048), (2048, 2048), (8192, 2048), (14336, 4096), (2176, 1280), (4096, 3968)])
+def test_stream_and_rows(M, K, N, entries):
+    r = data(M + K + N)
+    x, a, w, nw, y, ey = stream(r, M, K, N)
+    x0 = x.clone()
+    rows = sm.linear_rows(a, w, x, nw, EPS, mult=0.6, offset=1.0)
+    assert rows.sums is not None and "resnorm" not in entries and torch.equal(x, x0)
+    assert ((rows.x.double() - y).abs() <= ey).all()
+    want = rows.x.double() * (1.0 + nw.double())
+    assert ((rows.h.double() - want).abs() <= 2.0 ** -8 * want.abs()).all()
+    ss = rows.sums.view(-1)[:M * rows.count].view(M, rows.count).double().sum(-1)
+    assert ((ss - rows.x.double().square().sum(-1)).abs() <= 2.0 ** -17 * ss).all()     # bands of at most 64 squares, in fp32
+    for n in (1, 5, 2050):
+        v = r(n, N, m=N ** -0.5)
+        close(sm.rows_linear(rows, v, EPS), y, ey, nw, v, BF)
+        close(sm.rows_linear(rows, v, EPS, out_dtype=F32), y, ey, nw, v, F32)
+    assert entries.count("rows_in") == 6 and "resnorm" not in entries
+
+
+@pytest.mark.parametrize("act", [sm.ACT_GELU_TANH, sm.ACT_SWISH_CLAMP, sm.ACT_RELU])
+@pytest.mark.parametrize("M,W", [(1, 2048), (3, 128), (8, 2048), (16, 2048), (8, 4096), (13, 4096)])
+@pytest.mark.parametrize("N", [1, 63, 2050, 14336])
+def test_gated(act, M, W, N, entries):
+    r = data(M + W + N)
+    x, a, w, nw, y, ey = stream(r, M, 256, W)
+    rows = sm.linear_rows(a, w, x, nw, EPS, mult=0.6, offset=1.0)
+    v = r(2 * N, W, m=W ** -0.5)
+    got = sm.rows_linear(rows, v, EPS, act_kind=act, limit=1.5, alpha=1.702)
+    assert "rows_in" in entries and "resnorm" not in entries
+    close(got, y, ey, nw, v, BF, act)
+
+
+@pytest.mark.parametrize("M,W", [(1, 2048), (8, 2048), (16, 2048), (5, 4096), (17, 2048), (3, 192)])
+@pytest.mark.parametrize("n1,n2", [(1, 1), (3072, 576), (2045, 13), (7, 4096)])
+def test_split_and_other_sizes(M, W, n1, n2, entries):
+    r = data(M + n1)
+    x, a, w, nw, y, ey = stream(r, M, 256, W)
+    rows = sm.linear_rows(a, w, x, nw, EPS, mult=0.6, offset=1.0)
+    v = r(n1 + n2, W, m=W ** -0.5)
+    first, rest = sm.rows_linear(rows, v, EPS, split=n1)
+    assert first.shape == (M, n1) and rest.shape == (M, n2)
+    if M > 16 or W % 128:
+        assert rows.sums is None and "resnorm" in entries        # the product and the norm: the branch is rounded on its way
+        ey = ey + 0.6 * 2.0 ** -8 * (a.double() @ w.double().T).abs()
+    close(torch.cat([first, rest], 1), y, ey, nw, v, BF)
+
+
+@pytest.mark.parametrize("dt", [BF, F32])
+@pytest.mark.parametrize("W", [4, 1024, 1028, 2048, 4096])
+@pytest.mark.parametrize("T,n,branch,rowvec", [(1, 5, True, False), (8, 5, False, False), (33, 4, True, True), (3, 1, False, True)])
+def test_norm_shift(dt, W, T, n, branch, rowvec, entries):
+    r = data(W + T)
+    x, w, mu, state = r(T, W, dt=F32, m=2.0), r(W, dt=dt), r(n, W, dt=dt), r(T + 2, W, dt=dt)
+    kw = dict(branch=r(T, W, dt=dt) if branch else None, mult=0.6, rowvec=r(W, dt=dt) if rowvec else None, offset=1.0)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    b = {"seq_slots": i32([T + 1 - i for i in range(T)]), "cu_q": i32(list(range(T + 1))),
+         "tok_seq": i32(list(range(T))), "positions": i32([(0, 7, -1, 3)[i % 4] for i in range(T)])}
+    x2, s2 = x.clone(), state.clone()
+    got = sm.norm_shift(x, w, EPS, mu, state, b, single=True, **kw)
+    assert entries == ["norm_shift"]
+    want = sm.norm_shift(x2, w, EPS, mu, s2, b, **kw)
+    assert torch.equal(got, want) and torch.equal(x, x2) and torch.equal(state, s2)
