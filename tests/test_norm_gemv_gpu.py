@@ -1,4 +1,4 @@
-"""One or two rows times a weight matrix with the norms in the prologue, against 64 bits: widths at the ends of a thread's chunks and
+"""One row times a weight matrix with the norms in the prologue, against 64 bits: widths at the ends of a thread's chunks and
 of a lane's blocks, column counts at the ends of a row set, every form of norm and output; what it does not take runs as two launches."""
 import pytest
 import torch
@@ -90,7 +90,7 @@ def check(form, M, N, K, act, out_dtype, entries, fused=True):
 
 
 @pytest.mark.parametrize("form", sorted(FORMS))
-@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("M", [1])
 @pytest.mark.parametrize("K", [8, 512, 520, 2048, 2056, 4096])
 def test_forms_and_widths(form, M, K, entries):
     for N in (1, 7, 2050):
@@ -99,7 +99,7 @@ def test_forms_and_widths(form, M, K, entries):
 
 @pytest.mark.parametrize("act,out_dtype", [(None, None), (None, torch.float32), (sm.ACT_RELU2, None), (sm.ACT_GELU_TANH, None),
                                            (sm.ACT_SWISH_CLAMP, None), (sm.ACT_RELU, None)])
-@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("M", [1])
 @pytest.mark.parametrize("N", [4, 4095, 4096, 8193, 20001])
 def test_outputs_and_row_sets(act, out_dtype, M, N, entries):
     """Column counts around the change to two weight rows a wave and to several row sets a wave."""
@@ -107,7 +107,7 @@ def test_outputs_and_row_sets(act, out_dtype, M, N, entries):
         check(form, M, N, 1024, act, out_dtype, entries)
 
 
-@pytest.mark.parametrize("M,K", [(3, 256), (1, 4104), (2, 12), (1, 4)])
+@pytest.mark.parametrize("M,K", [(3, 256), (1, 4104), (2, 2048), (1, 12), (1, 4)])
 def test_other_sizes_run_as_norm_and_product(M, K, entries):
     for form in ("branch", "both", "sum", "gated"):
         check(form, M, 64, K, None, None, entries, fused=False)
