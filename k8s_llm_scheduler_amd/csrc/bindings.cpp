@@ -165,9 +165,10 @@ int k8s_gemm_few_act(void* C, const void* A, const void* W, int M, int N, int K,
                      hipStream_t s);
 int k8s_gemv_act(void* out, void* partial, const void* x, const void* W, int M, int N_out, int K, int kind, float limit, float alpha,
                  hipStream_t stream);
-int k8s_norm_gemv(void* out, float* x_out, const float* x, const void* branch, long ldb, int b32, const void* w1, float mult,
-                  const void* gate, long ldg, int gate_silu, const void* nw, float offset, float gain, float eps, const void* W,
-                  int M, int N_out, int K, int kind, float limit, float alpha, hipStream_t stream);
+int k8s_norm_gemv(void* out, float* x_out, const float* x, const void* branch, int b32, const void* w1, float mult, const void* gate,
+                  int gate_silu, const void* nw, float offset, float gain, float eps, const void* W, int N_out, int K, int kind,
+                  float limit, float alpha, hipStream_t stream);
+int k8s_rows_each(void* out, void* out2, const void* x, const void* W, int groups, int n, int rest, int M, int K, hipStream_t stream);
 long long k8s_rows_workspace(int M, int N, int K, int pair);
 int k8s_rows_out(float* y, void* h, float* sums, const float* x, const void* nw, const void* a, const void* W, void* partial, int M, int N,
                  int K, float mult, float offset, hipStream_t stream);
@@ -191,6 +192,9 @@ int k8s_shift_save(void* state, const void* h, const int* cu_q, const int* seq_s
                    int W, int f32, hipStream_t s);
 int k8s_wkv_max_dim();
 long long k8s_wkv_workspace(int T, int nseq, int H, int D, int Lc);
+int k8s_wkv_step(void* out, const void* r, const void* k, const void* v, const void* g, long ld, const void* lo, const void* w2, int L,
+                 const void* w0, const void* u, const void* lnw, float* state, const int* cu_q, const int* seq_slots,
+                 const int* positions, int nseq, int H, int D, float eps, int f32, hipStream_t s);
 int k8s_wkv_scan(void* out, const void* r, const void* k, const void* v, const void* g, long ld, const float* z,
                  const void* w0, const void* u, const void* lnw, float* state, const int* cu_q, const int* seq_slots,
                  const int* positions, int nseq, int H, int D, float eps, int f32, int T, int Lc, float* ws,
@@ -371,13 +375,18 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
   m.def("pgemm_set_prio", [](int mode) { return k8s_pgemm_set_prio(mode); });
   m.def("pgemm_set_row_slabs", [](int on) { return k8s_pgemm_set_row_slabs(on); });
   m.def("gemv_set_wide", [](int on) { return k8s_gemv_set_wide(on); });
-  m.def("norm_gemv", [](uintptr_t out, uintptr_t x_out, uintptr_t x, uintptr_t branch, long ldb, int b32, uintptr_t w1, float mult,
-                        uintptr_t gate, long ldg, int gate_silu, uintptr_t nw, float offset, float gain, float eps, uintptr_t W,
-                        int M, int N, int K, int kind, float limit, float alpha, int64_t s) {
-    const int rc = k8s_norm_gemv(P(out), P<float>(x_out), P<float>(x), P(branch), ldb, b32, P(w1), mult, P(gate), ldg, gate_silu,
-                                 P(nw), offset, gain, eps, P(W), M, N, K, kind, limit, alpha, S(s));
+  m.def("norm_gemv", [](uintptr_t out, uintptr_t x_out, uintptr_t x, uintptr_t branch, int b32, uintptr_t w1, float mult, uintptr_t gate,
+                        int gate_silu, uintptr_t nw, float offset, float gain, float eps, uintptr_t W, int N, int K, int kind,
+                        float limit, float alpha, int64_t s) {
+    const int rc = k8s_norm_gemv(P(out), P<float>(x_out), P<float>(x), P(branch), b32, P(w1), mult, P(gate), gate_silu, P(nw), offset,
+                                 gain, eps, P(W), N, K, kind, limit, alpha, S(s));
     if (rc != -5) check(rc, "norm_gemv");
     return rc != -5;    // false: sizes that it does not take, nothing was launched
+  });
+  m.def("rows_each", [](uintptr_t out, uintptr_t out2, uintptr_t x, uintptr_t W, int groups, int n, int rest, int M, int K, int64_t s) {
+    const int rc = k8s_rows_each(P(out), P(out2), P(x), P(W), groups, n, rest, M, K, S(s));
+    if (rc != -5) check(rc, "rows_each");
+    return rc != -5;
   });
   m.def("rows_workspace", [](int M, int N, int K, int pair) { return k8s_rows_workspace(M, N, K, pair); });
   // the number of sums a row, or 0: sizes that it does not take, nothing was launched
@@ -705,6 +714,14 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
     check(k8s_wkv_scan(P(out), P(r), P(k), P(v), P(g), ld, P<float>(z), P(w0), P(u), P(lnw), P<float>(state),
                        P<int>(cu_q), P<int>(seq_slots), P<int>(positions), nseq, H, D, eps, f32, T, Lc, P<float>(ws),
                        S(s)), "wkv_scan");
+  });
+  m.def("wkv_step", [](uintptr_t out, uintptr_t r, uintptr_t k, uintptr_t v, uintptr_t g, long ld, uintptr_t lo, uintptr_t w2, int L,
+                       uintptr_t w0, uintptr_t u, uintptr_t lnw, uintptr_t state, uintptr_t cu_q, uintptr_t seq_slots,
+                       uintptr_t positions, int nseq, int H, int D, float eps, int f32, int64_t s) {
+    const int rc = k8s_wkv_step(P(out), P(r), P(k), P(v), P(g), ld, P(lo), P(w2), L, P(w0), P(u), P(lnw), P<float>(state),
+                                P<int>(cu_q), P<int>(seq_slots), P<int>(positions), nseq, H, D, eps, f32, S(s));
+    if (rc != -5) check(rc, "wkv_step");
+    return rc != -5;
   });
   m.def("wkv_workspace", [](int T, int nseq, int H, int D, int Lc) { return k8s_wkv_workspace(T, nseq, H, D, Lc); });
   m.def("latent_kv_write", [](uintptr_t cache, uintptr_t dkv, uintptr_t normw, uintptr_t q, uintptr_t cos_sin,

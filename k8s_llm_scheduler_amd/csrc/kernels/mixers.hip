@@ -89,6 +89,8 @@ __global__ void shift_save_kernel(TA* __restrict__ state, const TA* __restrict__
 // wkv_prefix_kernel then walks a sequence's chunks: start[c + 1] = dec[c] * start[c] + loc[c];
 // MODE 2 (heads of more than 64 channels; wkv_chunk_out_kernel for the others): a chunk from its start state with outputs;
 //         a sequence's last chunk leaves the slot's state.
+// MODE 3: MODE 0 for sequences of one token each, with the decay logits z = lo w2^T (lo [T][L], w2 [H D][L]) worked out here, a slice
+//         of L by each channel group: 2 KB a head and row against a launch of its own.
 template <typename TA, int CH, int MODE>
 __global__ __launch_bounds__(1024) void wkv_scan_kernel(TA* __restrict__ out, const TA* __restrict__ r,
                                                         const TA* __restrict__ k, const TA* __restrict__ v,
@@ -97,7 +99,8 @@ __global__ __launch_bounds__(1024) void wkv_scan_kernel(TA* __restrict__ out, co
                                                         const TA* __restrict__ lnw, float* __restrict__ state,
                                                         const int* __restrict__ cu_q, const int* __restrict__ seq_slots,
                                                         const int* __restrict__ positions, int H, int D, float eps,
-                                                        int nseq, int Lc, const float* __restrict__ cs_start) {
+                                                        int nseq, int Lc, const float* __restrict__ cs_start,
+                                                        const TA* __restrict__ lo, const TA* __restrict__ w2, int L) {
   constexpr int DMAX = 128;
   __shared__ __attribute__((aligned(16))) float sr[DMAX], sk[DMAX], sw[DMAX], su[DMAX];
   __shared__ float po[DMAX / CH][DMAX];
@@ -105,10 +108,10 @@ __global__ __launch_bounds__(1024) void wkv_scan_kernel(TA* __restrict__ out, co
   const int hd = blockIdx.y;
   int s, a, b, p0;
   bool from_zero, last = true, many = false;
-  if (MODE == 0) {
+  if (MODE == 0 || MODE == 3) {
     s = blockIdx.x;
     a = cu_q[s];
-    b = cu_q[s + 1];
+    b = MODE == 3 ? a + 1 : cu_q[s + 1];
     if (b <= a) return;
     p0 = positions[a];
     if (p0 < 0) return;
@@ -154,11 +157,28 @@ __global__ __launch_bounds__(1024) void wkv_scan_kernel(TA* __restrict__ out, co
         nr = ldf(r, base);
         ng = ldf(g, base);
         nk = ldf(k, base);
-        nz = z[(size_t)t * HD + (size_t)hd * D + j];
+        if (MODE != 3) nz = z[(size_t)t * HD + (size_t)hd * D + j];
       }
     }
   };
   fetch(a);
+  if (MODE == 3) {
+    const int n = L / NS;
+    float part = 0.f;
+    if (on) {
+      const TA* x = lo + (size_t)a * L + c * n;
+      const TA* w = w2 + ((size_t)hd * D + j) * L + c * n;
+#pragma unroll 8
+      for (int i = 0; i < n; i += 4) {
+        const f32x4 x4 = ldf4(x + i), w4 = ldf4(w + i);
+        part = fmaf(x4[3], w4[3], fmaf(x4[2], w4[2], fmaf(x4[1], w4[1], fmaf(x4[0], w4[0], part))));
+      }
+      po[c][j] = part;
+    }
+    lds_barrier();
+    if (c == 0 && on)
+      for (int x = 0; x < NS; ++x) nz += po[x][j];
+  }
   for (int t = a; t < b; ++t) {
     const float cr = nr, ck = nk, cv = nv, cg = ng, cz = nz;
     fetch(t + 1);
@@ -990,6 +1010,25 @@ extern "C" long long k8s_wkv_workspace(int T, int nseq, int H, int D, int Lc) {
   return chunks * H * ((long long)2 * D * D + D);
 }
 
+// Sequences of one token each, z = lo w2^T.  -5: a size or an alignment that this form does not take; nothing was launched.
+extern "C" int k8s_wkv_step(void* out, const void* r, const void* k, const void* v, const void* g, long ld, const void* lo,
+                            const void* w2, int L, const void* w0, const void* u, const void* lnw, float* state, const int* cu_q,
+                            const int* seq_slots, const int* positions, int nseq, int H, int D, float eps, int f32, hipStream_t s) {
+  if (nseq <= 0) return 0;
+  if (H <= 0 || D <= 0 || D > 128 || H > 65535 || L <= 0 || lo == nullptr || w2 == nullptr) return -1;
+  constexpr int CH = 16;
+  const dim3 block((D + 63) / 64 * 64, (D + CH - 1) / CH);
+  if (L % (4 * block.y) || ((uintptr_t)lo | (uintptr_t)w2) % (f32 ? 16 : 8)) return -5;
+#define K8S_WS(TA)                                                                                                                  \
+  wkv_scan_kernel<TA, CH, 3><<<dim3(nseq, H), block, 0, s>>>((TA*)out, (const TA*)r, (const TA*)k, (const TA*)v, (const TA*)g, ld, nullptr, \
+                                                             (const TA*)w0, (const TA*)u, (const TA*)lnw, state, cu_q, seq_slots,       \
+                                                             positions, H, D, eps, nseq, 0, nullptr, (const TA*)lo, (const TA*)w2, L)
+  if (f32) K8S_WS(float);
+  else K8S_WS(bf16_t);
+#undef K8S_WS
+  return (int)hipGetLastError();
+}
+
 extern "C" int k8s_wkv_scan(void* out, const void* r, const void* k, const void* v, const void* g, long ld,
                             const float* z, const void* w0, const void* u, const void* lnw, float* state,
                             const int* cu_q, const int* seq_slots, const int* positions, int nseq, int H, int D,
@@ -1002,7 +1041,7 @@ extern "C" int k8s_wkv_scan(void* out, const void* r, const void* k, const void*
   wkv_scan_kernel<TA, CH, MODE><<<dim3(GX, H), block, 0, s>>>((TA*)out, (const TA*)r, (const TA*)k, (const TA*)v,      \
                                                               (const TA*)g, ld, z, (const TA*)w0, (const TA*)u,        \
                                                               (const TA*)lnw, state, cu_q, seq_slots, positions, H, D, \
-                                                              eps, nseq, Lc, START)
+                                                              eps, nseq, Lc, START, nullptr, nullptr, 0)
   if (Lc <= 0 || ws == nullptr) {
     if (f32) K8S_WKV(float, 0, nseq, nullptr);
     else K8S_WKV(bf16_t, 0, nseq, nullptr);

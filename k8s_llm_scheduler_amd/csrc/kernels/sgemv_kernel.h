@@ -319,8 +319,9 @@ __device__ __forceinline__ void sm_store(void* out, size_t o, float a, float u, 
 constexpr int SM_TICKET_RANGE = 256, SM_TICKET_RANGES = 256;
 __device__ unsigned sm_tickets[SM_TICKET_RANGE * SM_TICKET_RANGES];
 
-// Products of a normed fp32 stream (stream_gemv.hip).  ROWS 1 adds to the stream and leaves what the next product's norm needs, ROWS
-// 2 reads that: the norm is a factor of each row, which a product's sums can take as well as its input.
+// Products of a decode step's few rows (stream_gemv.hip).  Of a normed fp32 stream: ROWS 1 adds to the stream and leaves what the next product's norm needs, ROWS
+// 2 reads that: the norm is a factor of each row, which a product's sums can take as well as its input.  ROWS 3: several inputs of M
+// rows one after the other, `count` rows of W for each and the rest, past n1, for the last, through tanh to out2.
 struct SmRows {
   const float* x;          // 1: y = x + mult * product -> y (another buffer), h = bf16(y (offset + nw)), and of every workgroup's
   float* y;                //    columns the rows' sums of y^2 -> sums[m][blockIdx.x]
@@ -373,7 +374,7 @@ __global__ void __launch_bounds__(512) smfma_kernel(void* __restrict__ out, floa
   // ---- x -> registers: xr[s][xg] = x[4 xg + r4][chunk 16 (sb + s) + cb]; rows >= M / dead steps read 0
   u32x4 xr[JT][XG][XV];
   {
-    const auto xs = sg_rsrc(x, (long long)M * K * 2);
+    const auto xs = sg_rsrc(x + (ROWS == 3 ? (size_t)(b0 / rows.count) * M * K : 0), (long long)M * K * 2);
 #pragma unroll
     for (int s = 0; s < JT; ++s)
 #pragma unroll
@@ -570,6 +571,10 @@ __global__ void __launch_bounds__(512) smfma_kernel(void* __restrict__ out, floa
       const bool second = n >= rows.n1;
       sm_store<EPI, false>(second ? rows.out2 : out, second ? (size_t)m * (N - rows.n1) + (n - rows.n1) : (size_t)m * rows.n1 + n, a,
                            u, 0.f, act);
+    } else if constexpr (ROWS == 3) {
+      const size_t g = b0 / rows.count;             // (a band lies in one input's rows)
+      if (n < rows.n1) reinterpret_cast<bf16_t*>(out)[(g * M + m) * rows.count + (n - g * rows.count)] = f2bf(a);
+      else rows.out2[(size_t)m * (N - rows.n1) + (n - rows.n1)] = f2bf(tanhf(a));
     } else {
       sm_store<EPI, RES>(out, o, a, u, RES ? (first ? pre_res : bf2f(res[o])) : 0.f, act);
     }
@@ -743,6 +748,11 @@ static bool sm_launch(void* out, void* partial, const bf16_t* x, const void* W, 
     int nb = (N + bandmax - 1) / bandmax;
     nb = (nb + per - 1) / per * per;   // whole rounds of workgroups
     band = (N + nb - 1) / nb;
+  }
+  if constexpr (ROWS == 3) {   // bands of one input each, about a workgroup per CU
+    band = 8;
+    while (2 * band <= bandmax && rows.count % (2 * band) == 0 && (N + band - 1) / band > sm_cus() + sm_cus() / 8) band *= 2;
+    if (rows.count % band != 0) return false;
   }
   const dim3 grid((N + band - 1) / band, sp.g);
   float* part = sp.g > 1 ? (float*)partial : nullptr;

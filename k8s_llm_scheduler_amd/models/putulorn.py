@@ -281,8 +281,7 @@ PRESETS = {
 class _Wkv:
     cfg: MixerConfig
     mu: torch.Tensor        # [5, W]: r, k, v, g, w
-    w_rkvg: torch.Tensor    # [4, H D, W]
-    w1: torch.Tensor        # [lora, W]
+    w_in: torch.Tensor      # [4 H D + lora, W]: r, k, v, g, the decay's first factor
     w2: torch.Tensor        # [H D, lora]
     w0: torch.Tensor        # [H D]
     u: torch.Tensor         # [H D]
@@ -370,8 +369,7 @@ class PutulornModel(StreamModel):
             p, m = f"l{i}.mix.", L.mixer
             if m.type == "wkv":
                 mixer = _Wkv(m, t(torch.stack([get(p + "mu." + s) for s in MU_ORDER])),
-                             t(torch.stack([get(p + s) for s in ("r", "k", "v", "g")])), t(get(p + "w1")),
-                             t(get(p + "w2")), t(get(p + "w0")), t(get(p + "u").reshape(-1)), t(get(p + "norm")),
+                             t(torch.cat([get(p + s) for s in ("r", "k", "v", "g", "w1")])), t(get(p + "w2")), t(get(p + "w0")), t(get(p + "u").reshape(-1)), t(get(p + "norm")),
                              t(get(p + "o")))
                 if m.dim > sm.wkv_max_dim():
                     raise ValueError(f"layer {i}: wkv head dimension {m.dim} exceeds {sm.wkv_max_dim()}")
@@ -447,12 +445,9 @@ class PutulornModel(StreamModel):
         m = w.cfg
         S, shift = self.states[run.cache]
         mix = mixed(w.mu, shift)                                          # [5, T, W]
-        r, k, v, g = sm.linear_each(mix[:4], w.w_rkvg)
-        lo = sm.linear_act(mix[4], w.w1, sm.ACT_TANH)
+        (r, k, v, g), lo = sm.linear_each_tanh(mix, w.w_in, m.heads * m.dim)
         del mix
-        z = sm.linear(lo, w.w2, out_dtype=torch.float32)                  # decay logits stay fp32
-        return sm.wkv_scan(r, k, v, g, z, w.w0, w.u, w.lnw, S, b["cu_q"], b["seq_slots"], b["positions"], m.heads, m.dim,
-                           self.cfg.rms_eps)
+        return sm.wkv_step(r, k, v, g, lo, w.w2, w.w0, w.u, w.lnw, S, b, m.heads, m.dim, self.cfg.rms_eps, "max_keys" in b)
 
     def _latent(self, w: _Latent, run: _Run, products, b) -> torch.Tensor:
         """``products``(): the query [T, H (Dn + R)] and the latent row [T, C + R]."""

@@ -444,6 +444,23 @@ def linear_each(a: torch.Tensor, w: torch.Tensor):
     return tuple(linear(a[i], w[i]) for i in range(G))
 
 
+def linear_each_tanh(a: torch.Tensor, w: torch.Tensor, N: int):
+    """(:func:`linear_each` of all inputs but the last, tanh of the last one's product): a [G + 1, M, K], w [G N + L, K] the weights one
+    after the other.  A few bf16 rows in one launch (stream_gemv.hip).  us, two launches or more / one, weights from memory: 4 weights of
+    2048 x 2048 and one of 128 x 2048, 1 row 15.4 / 12.0, 8 17.5 / 13.3, 16 19.1 / 17.5; of 4096 x 4096 and 256 x 4096, 1 39.2 / 37.0,
+    8 42.4 / 39.6, 16 44.1 / 46.4 (x in registers: 16 rows of 4096 leave room for less of the weights under way)."""
+    G, M, K = a.shape[0] - 1, a.shape[1], a.shape[2]
+    L = w.shape[0] - G * N
+    if G < 1 or L < 1 or w.shape[1] != K:
+        raise ValueError(f"linear_each_tanh: inputs {tuple(a.shape)}, weights {tuple(w.shape)} of {N} rows each")
+    if rows_join(M, K) and (M <= 8 or K <= 2048) and _gpu(a, w) and a.dtype == w.dtype == BF16 and a.is_contiguous() and w.is_contiguous() and N % 8 == 0:
+        out = torch.empty(G, M, N, dtype=BF16, device=a.device)
+        last = torch.empty(M, L, dtype=BF16, device=a.device)
+        if _native().rows_each(out.data_ptr(), last.data_ptr(), a.data_ptr(), w.data_ptr(), G, N, L, M, K, -1):
+            return out.unbind(0), last
+    return linear_each(a[:G], w[:G * N].view(G, N, K)), linear_act(a[G], w[G * N:], ACT_TANH)
+
+
 def _each_once(a: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether products of several inputs may share a launch: the routing is free, sizes and places fit the big tiles."""
     G, M, K = a.shape
@@ -510,7 +527,7 @@ def linear_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, 
 
 
 # ----------------------------------------------------------------------------- recurrent mixer
-NORM_GEMV_MAX_M = 2       # rows (norm_gemv.hip)
+NORM_GEMV_MAX_M = 1       # rows (norm_gemv.hip)
 
 
 def norm_linear(x: Optional[torch.Tensor], branch: torch.Tensor, w: Optional[torch.Tensor], eps: float, weight: torch.Tensor, *,
@@ -521,8 +538,8 @@ def norm_linear(x: Optional[torch.Tensor], branch: torch.Tensor, w: Optional[tor
     W]) first x + ``mult`` * branch (``w`` None: :func:`resnorm`) or x + rms-norm(branch) * w (:func:`branchnorm`), that row itself or,
     with ``next_w``, its rms-norm * (``offset`` + next_w) * ``gain`` -- without one rms-norm(branch) * w, times ``gate``'s sigmoid or
     silu (:func:`norm_mix`) -- times ``weight``, with :func:`linear_act`'s activation if ``act_kind`` is given.  The stream is a new
-    tensor or x itself, updated: the caller goes on with what is returned.  One or two bf16 rows run in one launch; more, or other
-    sizes, as the norm and the product."""
+    tensor or x itself, updated: the caller goes on with what is returned.  One bf16 row runs in one launch; more, or other sizes, as
+    the norm and the product."""
     T, W = branch.shape
     dt = weight.dtype
     if T <= NORM_GEMV_MAX_M and dt == BF16 and FAST_GEMM and not _ops.LEAN and _ops.GEMM_BACKEND == "auto" and _ops.GEMV_MAX_M >= T > 0 and \
@@ -542,10 +559,9 @@ def norm_linear(x: Optional[torch.Tensor], branch: torch.Tensor, w: Optional[tor
             out = torch.empty(T, N, dtype=out_dtype or BF16, device=branch.device)
             new = torch.empty_like(x) if x is not None else None
             kind = act_kind if act_kind is not None else -2 if out_dtype == F32 else -1
-            if _native().norm_gemv(out.data_ptr(), _p(new), _p(x), branch.data_ptr(), branch.stride(0), int(b32), _p(w), float(mult),
-                                   gate.data_ptr() if gate is not None else 0, gate.stride(0) if gate is not None else 0,
-                                   int(gate_kind == GATE_SILU), _p(next_w), float(offset), float(gain), float(eps), weight.data_ptr(),
-                                   T, N, W, kind, float(limit), float(alpha), -1):
+            if _native().norm_gemv(out.data_ptr(), _p(new), _p(x), branch.data_ptr(), int(b32), _p(w), float(mult),
+                                   gate.data_ptr() if gate is not None else 0, int(gate_kind == GATE_SILU), _p(next_w), float(offset),
+                                   float(gain), float(eps), weight.data_ptr(), N, W, kind, float(limit), float(alpha), -1):
                 return out, new
     if x is None:
         h = norm_mix(branch, w, None, None, eps, out_dtype=dt, gate=gate, gate_kind=gate_kind)
@@ -723,6 +739,22 @@ def wkv_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
                        _p(cu_q, I32), _p(seq_slots, I32), _p(positions, I32), nseq, H, D, float(eps),
                        _f32(r.dtype), T, Lc, _p(ws), -1)
     return out
+
+
+def wkv_step(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, lo: torch.Tensor, w2: torch.Tensor, w0: torch.Tensor,
+             u: torch.Tensor, lnw: torch.Tensor, state: torch.Tensor, b: dict, H: int, D: int, eps: float, single: bool) -> torch.Tensor:
+    """:func:`wkv_scan` with the decay logits' product z = lo @ w2.T in fp32, ``b`` a batch description; the product inside the scan's
+    launch if every sequence brings a single token (``single``)."""
+    if single and _gpu(r, state) and 0 < D <= wkv_max_dim() and lo.dtype == w2.dtype == r.dtype and state.dtype == F32 and \
+            r.shape[0] == b["cu_q"].shape[0] - 1 and all(t.stride() == r.stride() and t.dtype == r.dtype and t.stride(1) == 1 for t in (r, k, v, g)):
+        T, L = lo.shape
+        out = torch.empty(T, H * D, dtype=r.dtype, device=r.device)
+        if _native().wkv_step(out.data_ptr(), r.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), r.stride(0), _p(lo), _p(w2), L,
+                              _p(w0, r.dtype, "w0"), _p(u, r.dtype, "u"), _p(lnw, r.dtype, "lnw"), _p(state), _p(b["cu_q"], I32),
+                              _p(b["seq_slots"], I32), _p(b["positions"], I32), T, H, D, float(eps), _f32(r.dtype), -1):
+            return out
+    z = linear(lo, w2, out_dtype=F32)                                      # decay logits stay fp32
+    return wkv_scan(r, k, v, g, z, w0, u, lnw, state, b["cu_q"], b["seq_slots"], b["positions"], H, D, eps)
 
 
 # ----------------------------------------------------------------------------- latent attention

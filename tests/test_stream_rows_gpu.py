@@ -127,3 +127,44 @@ def test_norm_shift(dt, W, T, n, branch, rowvec, entries):
     assert entries == ["norm_shift"]
     want = sm.norm_shift(x2, w, EPS, mu, s2, b, **kw)
     assert torch.equal(got, want) and torch.equal(x, x2) and torch.equal(state, s2)
+
+
+@pytest.mark.parametrize("M", [1, 3, 8, 9, 16, 17])
+@pytest.mark.parametrize("N,L,K", [(2048, 128, 2048), (8, 8, 128), (24, 1, 1152), (4096, 256, 4096), (2040, 127, 1024), (20, 4, 256)])
+def test_several_inputs(M, N, L, K, entries):
+    r = data(M + N + L)
+    a, w = r(5, M, K), r(4 * N + L, K, m=K ** -0.5)
+    outs, last = sm.linear_each_tanh(a, w, N)
+    assert ("rows_each" in entries) == (M <= (16 if K <= 2048 else 8) and N % 8 == 0)
+    bound = lambda x, v, slope=1.0: slope * 2.0 * K * 2.0 ** -24 * (x.double().abs() @ v.double().abs().T)    # fp32 sums in any order
+    for i in range(4):
+        z = a[i].double() @ w[i * N:(i + 1) * N].double().T
+        assert ((outs[i].double() - z).abs() <= bound(a[i], w[i * N:(i + 1) * N]) + 2.0 ** -8 * z.abs()).all()
+    z = a[4].double() @ w[4 * N:].double().T
+    twice = 0.0 if "rows_each" in entries else 2.0 ** -8 * z.abs()     # (other routes may round the product first)
+    assert ((last.double() - z.tanh()).abs() <= bound(a[4], w[4 * N:]) + twice + 2.0 ** -8 * z.tanh().abs() + 1e-7).all()
+
+
+@pytest.mark.parametrize("dt", [BF, F32])
+@pytest.mark.parametrize("H,D,L", [(32, 64, 128), (2, 20, 24), (3, 128, 256), (1, 16, 4), (2, 48, 8)])
+@pytest.mark.parametrize("T", [1, 8, 33])
+def test_wkv_step(dt, H, D, L, T, entries):
+    r = data(H + D + L + T)
+    rkvg = r(4, T, H * D, dt=dt)
+    lo, w2 = r(T, L, dt=dt).tanh(), r(H * D, L, dt=dt, m=L ** -0.5)
+    w0, u, lnw, state = r(H * D, dt=dt), r(H * D, dt=dt), r(H * D, dt=dt), r(T + 1, H, D, D, dt=F32)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    b = {"seq_slots": i32([T - i for i in range(T)]), "cu_q": i32(list(range(T + 1))), "positions": i32([(9, 0, -1)[i % 3] for i in range(T)])}
+    s2 = state.clone()
+    got = sm.wkv_step(*rkvg, lo, w2, w0, u, lnw, state, b, H, D, 1e-6, True)
+    groups = -(-D // 16)
+    assert ("wkv_step" in entries) and ("wkv_scan" in entries) == (L % (4 * groups) != 0)
+    z = lo.double() @ w2.double().T
+    want = sm.wkv_scan(*rkvg, z.float(), w0, u, lnw, s2, b["cu_q"], b["seq_slots"], b["positions"], H, D, 1e-6)
+    live = b["positions"] >= 0
+    assert torch.equal(got[live], want[live])                        # a token's output reads the state before its own decay
+    # |d exp(-exp(z)) / dz| <= 1 / e, z in fp32 sums
+    dz = (L + 8) * 2.0 ** -24 * (lo.double().abs() @ w2.double().abs().T) + 2.0 ** -22 * (z.abs() + w0.double().abs() + 1)
+    bound = torch.zeros_like(s2, dtype=torch.float64)
+    bound[b["seq_slots"].long()] = dz.view(T, H, D, 1).expand(T, H, D, D) / 2.7
+    assert ((state.double() - s2.double()).abs() <= bound * (8.0 + s2.double().abs()) + 1e-6).all()
