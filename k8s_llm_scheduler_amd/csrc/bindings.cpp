@@ -199,6 +199,9 @@ int k8s_wkv_scan(void* out, const void* r, const void* k, const void* v, const v
                  const void* w0, const void* u, const void* lnw, float* state, const int* cu_q, const int* seq_slots,
                  const int* positions, int nseq, int H, int D, float eps, int f32, int T, int Lc, float* ws,
                  hipStream_t s);
+int k8s_latent_begin(void* q_abs, const void* uk, void* cache, const void* dkv, const void* normw, void* q, const float* cos_sin,
+                     const int* positions, const int* slot_mapping, int T, int C, int R, int H, int Dn, int dims, float eps, long ldd,
+                     int interleaved, hipStream_t s);
 int k8s_latent_kv_write(void* cache, const void* dkv, const void* normw, void* q, const float* cos_sin,
                         const int* positions, const int* slot_mapping, int T, int C, int R, int H, int Dn, int dims,
                         float eps, int f32, long ldd, int interleaved, hipStream_t s);
@@ -724,6 +727,14 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
     return rc != -5;
   });
   m.def("wkv_workspace", [](int T, int nseq, int H, int D, int Lc) { return k8s_wkv_workspace(T, nseq, H, D, Lc); });
+  m.def("latent_begin", [](uintptr_t q_abs, uintptr_t uk, uintptr_t cache, uintptr_t dkv, uintptr_t normw, uintptr_t q,
+                           uintptr_t cos_sin, uintptr_t positions, uintptr_t slots, int T, int C, int R, int H, int Dn, int dims,
+                           float eps, long ldd, int interleaved, int64_t s) {
+    const int rc = k8s_latent_begin(P(q_abs), P(uk), P(cache), P(dkv), P(normw), P(q), P<float>(cos_sin), P<int>(positions),
+                                    P<int>(slots), T, C, R, H, Dn, dims, eps, ldd, interleaved, S(s));
+    if (rc != -5) check(rc, "latent_begin");
+    return rc != -5;
+  });
   m.def("latent_kv_write", [](uintptr_t cache, uintptr_t dkv, uintptr_t normw, uintptr_t q, uintptr_t cos_sin,
                               uintptr_t positions, uintptr_t slots, int T, int C, int R, int H, int Dn, int dims,
                               float eps, int f32, long ldd, int interleaved, int64_t s) {

@@ -118,6 +118,23 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// The sum over a workgroup of 4 full waves, in every thread: 16 lanes by register moves, the rows of a wave by lane reads, the
+// waves through 4 floats of `red` (of which every call of a kernel has its own) behind a barrier that waits for LDS only.  The
+// row norms are a chain of latencies: block_sum's 12 shuffles and its waits for the stores in flight cost one row of 2048 0.3 us
+// (3.45 -> 3.16), a norm on both sides 0.65 (4.29 -> 3.64), 2048 rows 0.3 - 0.8 of 5.4 - 10.7.
+template <int CTRL>
+__device__ __forceinline__ float lane_add(float v) {
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float row_total(float v, float* red) {
+  v = lane_add<0x140>(lane_add<0x141>(lane_add<0x4E>(lane_add<0xB1>(v))));     // lanes ^ 1, ^ 2, mirrored in 8, in 16
+  const auto lane = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l)); };
+  const float w = (lane(0) + lane(16)) + (lane(32) + lane(48));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = w;
+  lds_barrier();
+  return (red[0] + red[1]) + (red[2] + red[3]);
+}
+
 // Chunk g of a varlen batch cut into chunks of Lc tokens per sequence: (sequence, chunk in the sequence, chunks of the
 // sequence), or sequence -1 when g is past the last chunk.  Idle (position < 0) and empty sequences have no chunks.
 struct WkvChunk { int s, c, n; };

@@ -26,7 +26,7 @@ __global__ __launch_bounds__(256) void latent_token_kernel(
   float* wm = reinterpret_cast<float*>(pw + 16 * (KT + 8));      // the waves' maxima, then sums: [4][16]
   const int t = blockIdx.x, hg = blockIdx.y, split = blockIdx.z, HP = gridDim.y * 16;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, g = lane >> 4;
-  const int p = positions[t], lo = window > 0 ? max(0, p - window + 1) : 0;
+  const int p = positions[t], seq = tok_seq[t], lo = window > 0 ? max(0, p - window + 1) : 0;
   const int nsteps = p < 0 ? 0 : (p - lo + KT) / KT, per = (nsteps + nsplit - 1) / nsplit;
   const int s0 = split * per, s1 = min(nsteps, s0 + per);
   const size_t rec0 = ((size_t)t * HP + hg * 16) * nsplit + split;    // the head's record: rec0 + head * nsplit
@@ -37,7 +37,7 @@ __global__ __launch_bounds__(256) void latent_token_kernel(
     }
     return;
   }
-  const int* btr = block_tables + (size_t)tok_seq[t] * max_blocks;
+  const int* btr = block_tables + (size_t)seq * max_blocks;
   const int lr = tid >> 3, lc = tid & 7;                         // loader: rows lr, lr + 32, pieces lc + 8 i
   const u32x4 zero = u32x4{0u, 0u, 0u, 0u};
   u32x4 pre[2][NLD];
@@ -170,41 +170,53 @@ __global__ __launch_bounds__(4 * V) void latent_out_kernel(bf16_t* __restrict__ 
   __shared__ __attribute__((aligned(16))) bf16_t lat[16][C + 8];
   const int hd = blockIdx.x, t0 = blockIdx.y * 4, nt = min(4, T - t0);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, g = lane >> 4;
+  // everything is requested at once, in the order of its use (loads retire in order): maxima and sums, the first splits' sums, weights
+  const int tw = t0 + min(wave, nt - 1);               // a wave per token, a lane per split
+  const size_t rec = ((size_t)tw * HP + hd) * nsplit + min(lane, nsplit - 1);
+  const float m0 = pml[2 * rec], l0 = pml[2 * rec + 1];
+  const float g0 = gate != nullptr ? bf2f(gate[(size_t)tw * ldg + hd]) : 0.f;
+  constexpr int AHEAD = 16;
+  const int k = tid >> 7, c = 4 * (tid & 127);
+  const float* pr = pacc + ((size_t)(t0 + min(k, nt - 1)) * HP + hd) * nsplit * C + c;
+  f32x4 x[AHEAD];
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u) x[u] = *reinterpret_cast<const f32x4*>(pr + (size_t)min(u, nsplit - 1) * C);
   bf16x8 wf[NKK];
   const bf16_t* wr = uv + ((size_t)hd * V + 16 * wave + li) * C + 8 * g;
 #pragma unroll
   for (int kk = 0; kk < NKK; ++kk) wf[kk] = *reinterpret_cast<const bf16x8*>(wr + 32 * kk);
-  if (wave < nt) {                   // a wave per token, a lane per split
-    const size_t rec = ((size_t)(t0 + wave) * HP + hd) * nsplit + min(lane, nsplit - 1);
-    const float m = lane < nsplit ? pml[2 * rec] : -INFINITY, l = lane < nsplit ? pml[2 * rec + 1] : 0.f;
+  asm volatile("" ::: "memory");
+  if (wave < nt) {
+    const float m = lane < nsplit ? m0 : -INFINITY, l = lane < nsplit ? l0 : 0.f;
     float M = wave_max(m);
     if (sinks != nullptr) M = fmaxf(M, sinks[hd]);
     const float e = m == -INFINITY ? 0.f : expf(m - M);
     float den = wave_sum(e * l);
     if (sinks != nullptr) den += expf(sinks[hd] - M);
-    const float gh = gate != nullptr ? 1.f / (1.f + expf(-bf2f(gate[(size_t)(t0 + wave) * ldg + hd]))) : 1.f;
+    const float gh = gate != nullptr ? 1.f / (1.f + expf(-g0)) : 1.f;
     // weight 0 is for records that were not written (maximum -inf, sum 0); a NaN or infinite score makes the sum NaN
     if (lane < 32) ws[wave][lane] = m == -INFINITY && l == 0.f ? 0.f : e / den * gh;
   }
-  __syncthreads();
-  const int k = tid >> 7, c = 4 * (tid & 127);
+  lds_barrier();
   if (k < nt) {
-    const float* pr = pacc + ((size_t)(t0 + k) * HP + hd) * nsplit * C + c;
     f32x4 y = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < nsplit; s += 8) {
-      f32x4 x[8];
+    auto add = [&](const f32x4& v, int s) {
+      const float w = s < nsplit ? ws[k][s] : 0.f;
 #pragma unroll
-      for (int u = 0; u < 8; ++u) x[u] = *reinterpret_cast<const f32x4*>(pr + (size_t)min(s + u, nsplit - 1) * C);
+      for (int i = 0; i < 4; ++i) y[i] += w != 0.f ? w * v[i] : 0.f;             // (w 0: nothing, or nothing written)
+    };
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const float w = s + u < nsplit ? ws[k][s + u] : 0.f;
+    for (int u = 0; u < AHEAD; ++u) add(x[u], u);
+    for (int s = AHEAD; s < nsplit; s += 8) {
+      f32x4 z[8];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) y[i] += w != 0.f ? w * x[u][i] : 0.f;     // (w 0: nothing, or nothing written)
-      }
+      for (int u = 0; u < 8; ++u) z[u] = *reinterpret_cast<const f32x4*>(pr + (size_t)min(s + u, nsplit - 1) * C);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) add(z[u], s + u);
     }
     stf4(&lat[k][c], y);
   }
-  __syncthreads();
+  lds_barrier();
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int kk = 0; kk < NKK; ++kk)

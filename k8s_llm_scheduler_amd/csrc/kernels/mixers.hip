@@ -6,6 +6,7 @@
 // Both run varlen batches: sequence s owns tokens cu_q[s] .. cu_q[s + 1] - 1, positions[t] is a token's position in
 // its sequence (negative: the row is idle and touches nothing), seq_slots[s] the slot of its recurrent state.
 #include "common.h"
+#include "latent_row.h"
 
 namespace k8sllm {
 
@@ -601,6 +602,12 @@ __global__ __launch_bounds__(256) void latent_kv_write_kernel(TA* __restrict__ c
   }
 }
 
+template <typename TA, bool IL>
+__global__ __launch_bounds__(256) void latent_row_kernel(LatentRows<TA> a) {
+  __shared__ float red[4];
+  latent_row<TA, IL>(a, blockIdx.x, red);
+}
+
 // One workgroup per token, one wave per head (heads beyond the wave count take further passes).  Keys come in blocks
 // of KB <= 64 cached rows staged in LDS as fp32 and shared by the heads; lane l scores key l of the block
 // ((q_abs . c + q_rot . k_rot) * scale), the block joins a running softmax, and lane l accumulates latent
@@ -1087,6 +1094,18 @@ extern "C" int k8s_latent_kv_write(void* cache, const void* dkv, const void* nor
                                    int dims, float eps, int f32, long ldd, int interleaved, hipStream_t s) {
   if (T <= 0) return 0;
   if (C <= 0 || R < 0 || dims < 0 || dims > R || (dims & 1) || H <= 0 || ldd < C + R) return -1;
+#define K8S_LR(TA)                                                                                                                    \
+  do {                                                                                                                                \
+    const LatentRows<TA> a = {(TA*)cache, (const TA*)dkv, (const TA*)normw, (TA*)q, cos_sin, positions, slot_mapping, C, R, H, Dn, dims, \
+                              eps, ldd};                                                                                              \
+    if (!latent_row_ok(a)) break;                                                                                                     \
+    if (interleaved) latent_row_kernel<TA, true><<<T, 256, 0, s>>>(a);                                                                \
+    else latent_row_kernel<TA, false><<<T, 256, 0, s>>>(a);                                                                           \
+    return (int)hipGetLastError();                                                                                                    \
+  } while (0)
+  if (f32) K8S_LR(float);
+  else K8S_LR(bf16_t);
+#undef K8S_LR
   if (f32)
     latent_kv_write_kernel<float><<<T, 256, 0, s>>>((float*)cache, (const float*)dkv, (const float*)normw, (float*)q,
                                                     cos_sin, positions, slot_mapping, C, R, H, Dn, dims, eps, ldd,

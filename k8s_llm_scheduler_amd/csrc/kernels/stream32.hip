@@ -4,26 +4,9 @@
 // mode) is added in fp32 by the norm that follows it, so the add costs no extra pass.  All kernels take the
 // activation / weight element type as a template parameter: bf16 storage or true fp32.
 #include "common.h"
+#include "latent_row.h"
 
 namespace k8sllm {
-
-// The sum over a workgroup of 4 full waves, in every thread: 16 lanes by register moves, the rows of a wave by lane reads, the
-// waves through 4 floats of `red` (of which every call of a kernel has its own) behind a barrier that waits for LDS only.  The
-// row norms are a chain of latencies: block_sum's 12 shuffles and its waits for the stores in flight cost one row of 2048 0.3 us
-// (3.45 -> 3.16), a norm on both sides 0.65 (4.29 -> 3.64), 2048 rows 0.3 - 0.8 of 5.4 - 10.7.
-template <int CTRL>
-__device__ __forceinline__ float lane_add(float v) {
-  return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
-}
-__device__ __forceinline__ float row_total(float v, float* red) {
-  v = lane_add<0x140>(lane_add<0x141>(lane_add<0x4E>(lane_add<0xB1>(v))));     // lanes ^ 1, ^ 2, mirrored in 8, in 16
-  const auto lane = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l)); };
-  const float w = (lane(0) + lane(16)) + (lane(32) + lane(48));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = w;
-  lds_barrier();
-  return (red[0] + red[1]) + (red[2] + red[3]);
-}
-
 
 // out[t, :] = float(table[ids[t], :]) * scale; copy (optional) the same in the table's type, as the first sublayer reads it
 template <typename TA>
@@ -1002,9 +985,48 @@ __global__ __launch_bounds__(256) void gemm_narrow_kernel(TO* __restrict__ C, co
   else gemm_group_tile<TO, 4, ACT>(C, A, Wt, N, K, lda, ldw, ldc, nullptr, row0, rows, red, act);
 }
 
+// A decode step's latent attention up to the attention itself, one launch for two: the tokens' cache rows and query rotation (plane 0),
+// and the queries' unrotated parts taken into the latent space, gemm_narrow_kernel's work for a head a plane.  Neither reads what the
+// other writes.
+template <bool IL>
+__global__ __launch_bounds__(256) void latent_begin_kernel(LatentRows<bf16_t> a, int T, bf16_t* __restrict__ q_abs,
+                                                           const bf16_t* __restrict__ uk) {
+  __shared__ __attribute__((aligned(16))) float red[4 * 4 * 64 * 4];
+  if (blockIdx.z == 0) {
+    for (int t = blockIdx.x; t < T; t += gridDim.x) {
+      latent_row<bf16_t, IL>(a, t, red);
+      __syncthreads();                             // the sums of the row before have been read
+    }
+    return;
+  }
+  const int h = blockIdx.z - 1;
+  const bf16_t* A = a.q + (size_t)h * (a.Dn + a.R);
+  const bf16_t* W = uk + (size_t)h * a.C * a.Dn;
+  const long lda = (long)a.H * (a.Dn + a.R), ldc = (long)a.H * a.C;
+  if (T <= 16) gemm_group_tile<bf16_t, 1, FEW_NONE>(q_abs + (size_t)h * a.C, A, W, a.C, a.Dn, lda, a.Dn, ldc, nullptr, 0, T, red, FewAct{});
+  else gemm_group_tile<bf16_t, 4, FEW_NONE>(q_abs + (size_t)h * a.C, A, W, a.C, a.Dn, lda, a.Dn, ldc, nullptr, 0, T, red, FewAct{});
+}
+
 }  // namespace k8sllm
 
 using namespace k8sllm;
+
+// q_abs [T][H][C] = q's unrotated parts times uk [H][C][Dn]^T, and latent_kv_write, of bf16.  -5: a size or an alignment that this form
+// does not take; nothing was launched.
+extern "C" int k8s_latent_begin(void* q_abs, const void* uk, void* cache, const void* dkv, const void* normw, void* q, const float* cos_sin,
+                                const int* positions, const int* slot_mapping, int T, int C, int R, int H, int Dn, int dims, float eps,
+                                long ldd, int interleaved, hipStream_t s) {
+  if (T <= 0) return 0;
+  if (C <= 0 || R < 0 || dims < 0 || dims > R || (dims & 1) || H <= 0 || Dn <= 0 || ldd < C + R || !q_abs || !uk) return -1;
+  const LatentRows<bf16_t> a = {(bf16_t*)cache, (const bf16_t*)dkv, (const bf16_t*)normw, (bf16_t*)q, cos_sin, positions, slot_mapping,
+                                C, R, H, Dn, dims, eps, ldd};
+  if (T > 64 || H >= 65535 || Dn % 64 || (Dn + R) % 8 || C % 16 || ((uintptr_t)q | (uintptr_t)uk | (uintptr_t)q_abs) % 16 || !latent_row_ok(a))
+    return -5;
+  const dim3 grid(C / 16, 1, H + 1);
+  if (interleaved) latent_begin_kernel<true><<<grid, 256, 0, s>>>(a, T, (bf16_t*)q_abs, (const bf16_t*)uk);
+  else latent_begin_kernel<false><<<grid, 256, 0, s>>>(a, T, (bf16_t*)q_abs, (const bf16_t*)uk);
+  return (int)hipGetLastError();
+}
 
 extern "C" int k8s_embed_rows(float* out, void* copy, const int* ids, const void* table, int T, int W, int vocab,
                               float scale, int f32, hipStream_t s) {

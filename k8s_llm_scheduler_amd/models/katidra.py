@@ -399,10 +399,11 @@ class KatidraModel(StreamModel):
             q, _ = sm.norm_linear(None, dq, w.dq_norm, eps, w.uq)          # [T, H (Dn + R)]
         else:
             q = sm.linear(sm.norm_mix(dq, w.dq_norm, None, None, eps), w.uq)
-        sm.latent_kv_write(kv, proj[:, w.cols["dkv"]:w.cols["dkv"] + C + R], w.dkv_norm, q, w.cos_sin, b["positions"],
-                           b["slot_mapping"], C, R, H, Dn, m.rot_dims, eps, interleaved=True)
+        q_abs = sm.latent_kv_write(kv, proj[:, w.cols["dkv"]:w.cols["dkv"] + C + R], w.dkv_norm, q, w.cos_sin, b["positions"],
+                                   b["slot_mapping"], C, R, H, Dn, m.rot_dims, eps, interleaved=True,
+                                   absorb=w.uk_t if "max_keys" in b else None)
         a = sm.latent_mix(q, kv, w.uk_t, w.uv, w.ukv, b, C, R, H, Dn, V, m.window, m.scale, self.block_size,
-                          gate=proj[:, w.cols["g"]:w.cols["g"] + H])
+                          gate=proj[:, w.cols["g"]:w.cols["g"] + H], q_abs=q_abs)
         del proj, dq, q
         return sm.linear(a, w.o)
 

@@ -455,9 +455,10 @@ class PutulornModel(StreamModel):
         H, Dn, R, C, V = m.heads, m.dim, m.rot_dim, m.kv_rank, m.vdim
         cache = self.kv_cache[run.cache]
         q, dkv = products()
-        sm.latent_kv_write(cache, dkv, w.dkv_norm, q, w.cos_sin, b["positions"], b["slot_mapping"], C, R, H, Dn,
-                           m.rot_dims, self.cfg.rms_eps)
-        return sm.latent_mix(q, cache, w.uk_t, w.uv, w.ukv, b, C, R, H, Dn, V, m.window, m.scale, self.block_size)
+        q_abs = sm.latent_kv_write(cache, dkv, w.dkv_norm, q, w.cos_sin, b["positions"], b["slot_mapping"], C, R, H, Dn,
+                                   m.rot_dims, self.cfg.rms_eps, absorb=w.uk_t if "max_keys" in b else None)
+        del dkv
+        return sm.latent_mix(q, cache, w.uk_t, w.uv, w.ukv, b, C, R, H, Dn, V, m.window, m.scale, self.block_size, q_abs=q_abs)
 
     def _mlp(self, w: _Mlp, h) -> torch.Tensor:
         f = w.cfg

@@ -480,9 +480,11 @@ class SemanexModel(StreamModel):
         proj = sm.linear(h, w.w_in)                                        # [T, dq | dkv | gate]
         cq = sm.norm_mix(proj[:, w.cols["dq"]:w.cols["dq"] + m.q_rank], w.dq_norm, None, None, eps)
         q = sm.linear(cq, w.uq)                                            # [T, H (Dn + R)]
-        sm.latent_kv_write(cache, proj[:, w.cols["dkv"]:w.cols["dkv"] + C + R], w.dkv_norm, q, w.cos_sin,
-                           b["positions"], b["slot_mapping"], C, R, H, Dn, m.rot_dims, eps, interleaved=True)
-        a = sm.latent_mix(q, cache, w.uk_t, w.uv, w.ukv, b, C, R, H, Dn, V, 0, m.scale, self.block_size, sinks=w.sinks)
+        q_abs = sm.latent_kv_write(cache, proj[:, w.cols["dkv"]:w.cols["dkv"] + C + R], w.dkv_norm, q, w.cos_sin,
+                                   b["positions"], b["slot_mapping"], C, R, H, Dn, m.rot_dims, eps, interleaved=True,
+                                   absorb=w.uk_t if "max_keys" in b else None)
+        a = sm.latent_mix(q, cache, w.uk_t, w.uv, w.ukv, b, C, R, H, Dn, V, 0, m.scale, self.block_size, sinks=w.sinks,
+                          q_abs=q_abs)
         y = sm.gate_mul(a, proj[:, w.cols["g"]:w.cols["g"] + H * V], sm.GATE_SIGMOID)
         return sm.linear(y, w.o)
 

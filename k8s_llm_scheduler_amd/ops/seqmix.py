@@ -760,11 +760,13 @@ def wkv_step(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor,
 # ----------------------------------------------------------------------------- latent attention
 def latent_kv_write(cache: torch.Tensor, dkv: torch.Tensor, normw: torch.Tensor, q: torch.Tensor,
                     cos_sin: torch.Tensor, positions: torch.Tensor, slot_mapping: torch.Tensor, C: int, R: int, H: int,
-                    Dn: int, rot_dims: int, eps: float, interleaved: bool = False) -> None:
+                    Dn: int, rot_dims: int, eps: float, interleaved: bool = False,
+                    absorb: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """cache[slot] = [rms-norm(dkv[:, :C]) * normw | rotated dkv[:, C:]]; rotates the last R of every head of q
     ([T, H (Dn + R)]) in place.  ``cos_sin`` [positions, rot_dims] = [cos | sin] fp32.  The rotation pairs dimension i
     with i + rot_dims / 2, or (``interleaved``) dimension 2i with 2i + 1.  ``dkv`` [T, C + R] may be a column slice of
-    a wider projection."""
+    a wider projection.  ``absorb``: :func:`latent_mix`'s ``uk_t``, whose product with the queries is then, for up to 64 bf16 tokens,
+    part of the launch and returned for ``q_abs`` there (None: not taken)."""
     if dkv.dim() != 2 or dkv.shape[1] != C + R:
         raise ValueError("latent_kv_write: dkv must be [T, C + R]")
     if not _gpu(cache, dkv, q):
@@ -773,6 +775,14 @@ def latent_kv_write(cache: torch.Tensor, dkv: torch.Tensor, normw: torch.Tensor,
     dt = dkv.dtype
     if dkv.stride(1) != 1:
         raise ValueError("latent_kv_write: rows must be contiguous")
+    T = dkv.shape[0]
+    if absorb is not None and dt == BF16 and 0 < T <= 64 and _gpu(absorb) and absorb.shape == (H, C, Dn) and absorb.dtype == dt and \
+            absorb.is_contiguous():
+        q_abs = torch.empty(T, H, C, dtype=dt, device=q.device)
+        if _native().latent_begin(q_abs.data_ptr(), absorb.data_ptr(), _p(cache, dt, "cache"), dkv.data_ptr(), _p(normw, dt, "normw"),
+                                  _p(q, dt, "q"), _p(cos_sin, F32, "cos_sin"), _p(positions, I32), _p(slot_mapping, I32), T, C, R, H, Dn,
+                                  rot_dims, float(eps), dkv.stride(0), int(bool(interleaved)), -1):
+            return q_abs
     _native().latent_kv_write(_p(cache, dt, "cache"), dkv.data_ptr(), _p(normw, dt, "normw"), _p(q, dt, "q"),
                               _p(cos_sin, F32, "cos_sin"), _p(positions, I32), _p(slot_mapping, I32), dkv.shape[0], C,
                               R, H, Dn, rot_dims, float(eps), _f32(dt), dkv.stride(0), int(bool(interleaved)), -1)
@@ -876,11 +886,12 @@ def _latent_keys(b: dict, window: int, block_size: int, cap: int) -> tuple:
 
 def latent_mix(q: torch.Tensor, cache: torch.Tensor, uk_t: torch.Tensor, uv: torch.Tensor, ukv: Optional[torch.Tensor],
                b: dict, C: int, R: int, H: int, Dn: int, V: int, window: int, scale: float, block_size: int, *,
-               sinks: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None) -> torch.Tensor:
+               sinks: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
+               q_abs: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Latent attention with its up-projections, [T, H V]: queries q [T, H (Dn + R)] (rotated) over the batch ``b``'s cached
     rows, ``uk_t`` [H, C, Dn], ``uv`` [H, V, C], ``ukv`` from :func:`latent_expand`; ``sinks`` and ``gate`` as for
     :func:`latent_attention`.  Decoding and short portions absorb the queries (q W_uk), attend the cache as it is stored and
-    take the result through W_uv; batches of longer portions write the visible rows' keys and values out first."""
+    take the result through W_uv (``q_abs``: the first of these, done already); batches of longer portions write the visible rows' keys and values out first."""
     T = q.shape[0]
     dt = q.dtype
     if sinks is not None and (sinks.dtype != F32 or sinks.numel() != H):
@@ -912,8 +923,9 @@ def latent_mix(q: torch.Tensor, cache: torch.Tensor, uk_t: torch.Tensor, uv: tor
                               _p(sinks), gate.data_ptr() if gate is not None else 0,
                               gate.stride(0) if gate is not None else 0, _f32(dt), -1)
             return out
-    q_abs = torch.empty(T, H, C, dtype=dt, device=q.device)
-    gemm(q.view(T, H, Dn + R)[:, :, :Dn].permute(1, 0, 2), uk_t, out=q_abs.permute(1, 0, 2))
+    if q_abs is None:
+        q_abs = torch.empty(T, H, C, dtype=dt, device=q.device)
+        gemm(q.view(T, H, Dn + R)[:, :, :Dn].permute(1, 0, 2), uk_t, out=q_abs.permute(1, 0, 2))
     if LATENT_MFMA and max_qlen == 0 and dt == BF16 and _gpu(q, cache, sinks, gate) and aligned and \
             uv.data_ptr() % 16 == 0 and _native().latent_token_ok(C, R, Dn, V):
         # decoding: key splits of at least one 64-key step for about one workgroup per CU, joined by the kernel that takes

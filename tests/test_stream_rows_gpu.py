@@ -168,3 +168,48 @@ def test_wkv_step(dt, H, D, L, T, entries):
     bound = torch.zeros_like(s2, dtype=torch.float64)
     bound[b["seq_slots"].long()] = dz.view(T, H, D, 1).expand(T, H, D, D) / 2.7
     assert ((state.double() - s2.double()).abs() <= bound * (8.0 + s2.double().abs()) + 1e-6).all()
+
+
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("C,R,H,Dn,dims", [(512, 64, 16, 128, 64), (512, 64, 16, 128, 32), (16, 8, 3, 64, 8), (1024, 64, 2, 64, 64), (64, 24, 5, 128, 16),
+                                           (512, 64, 33, 64, 0)])
+@pytest.mark.parametrize("T", [1, 16, 17, 64, 65])
+def test_latent_begin(C, R, H, Dn, dims, interleaved, T, entries):
+    """The cache rows and the queries against 64 bits, and the one launch bit for bit as the two."""
+    r = data(C + H + T)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    wide, nw, q, uk, cache = r(T, C + R + 8, m=2.0), r(C), r(T, H * (Dn + R)), r(H, C, Dn, m=Dn ** -0.5), r(T + 3, C + R)
+    dkv, cs = wide[:, 8:], r(40, max(dims, 1), dt=F32)[:, :dims].contiguous()
+    pos, slots = [(i * 7) % 40 if i % 5 != 3 else -1 for i in range(T)], [T + 2 - i if i % 4 != 2 else -1 for i in range(T)]
+    run = lambda c, qq, absorb: sm.latent_kv_write(c, dkv, nw, qq, cs, i32(pos), i32(slots), C, R, H, Dn, dims, 1e-6, interleaved, absorb)
+    c2, q2, c1, q1 = cache.clone(), q.clone(), cache.clone(), q.clone()
+    got = run(c1, q1, uk)
+    assert ("latent_begin" in entries) == (T <= 64) and (got is not None) == (T <= 64)
+    assert run(c2, q2, None) is None
+    assert torch.equal(c1, c2) and torch.equal(q1, q2)
+    if got is not None:
+        want = torch.empty(T, H, C, dtype=BF, device=DEV)
+        sm.gemm(q.view(T, H, Dn + R)[:, :, :Dn].permute(1, 0, 2), uk, out=want.permute(1, 0, 2))
+        z = torch.matmul(q.view(T, H, Dn + R)[:, :, :Dn].permute(1, 0, 2).double(), uk.double().transpose(1, 2).contiguous()).permute(1, 0, 2)
+        assert ((got.double() - z).abs() <= 2.0 ** -8 * z.abs() + 2.0 * Dn * 2.0 ** -24 * 8 * Dn ** 0.5).all()
+
+    def rotated(v, p):
+        v, half = v.double().clone(), dims // 2
+        c, s = cs[p, :half].double(), cs[p, half:].double()
+        ia, ib = (slice(0, dims, 2), slice(1, dims, 2)) if interleaved else (slice(0, half), slice(half, dims))
+        a, b = v[..., ia].clone(), v[..., ib].clone()
+        v[..., ia], v[..., ib] = a * c - b * s, b * c + a * s
+        return v
+    for t in range(T):
+        qt, qo = q1[t].view(H, Dn + R), q[t].view(H, Dn + R)
+        if pos[t] < 0:
+            assert torch.equal(qt, qo)
+            continue
+        want = torch.cat([qo[:, :Dn].double(), rotated(qo[:, Dn:], pos[t])], 1)
+        assert ((qt.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()
+        if slots[t] >= 0:
+            d = dkv[t].double()
+            row = torch.cat([d[:C] * (d[:C].square().mean() + 1e-6).rsqrt() * nw.double(), rotated(dkv[t, C:], pos[t])])
+            assert ((c1[slots[t]].double() - row).abs() <= 2.0 ** -8 * row.abs() + 1e-5).all()
+    untouched = [i for i in range(T + 3) if i not in [s for s, p in zip(slots, pos) if s >= 0 and p >= 0]]
+    assert torch.equal(c1[untouched], cache[untouched])
