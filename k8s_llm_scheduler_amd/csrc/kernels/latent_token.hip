@@ -157,19 +157,22 @@ __global__ __launch_bounds__(256) void latent_token_kernel(
 // tokens) of V / 16 waves.  lat[c] = sum_s e^(m_s - M) O_s[c] / sum_s e^(m_s - M) l_s (with a sink: one more term e^sink),
 // times the head's gate, rounded to bf16 as the product's operand; out = lat W_uv^T with the tokens as the columns of the
 // instruction's tile and the weights, loaded ahead of the merge, straight from memory as its rows.  nsplit <= 32.
-// 16 splits, 16 heads: 7.5 us at 1 and 8 rows (a merge of 11 us and a product of 8 us before).
-template <int C, int V>
+// 16 splits, 16 heads: 4.8 us at 1 and 8 rows in quarters of the value columns, 7.3 with all of a head's.
+// CB: blocks of 16 value columns of a workgroup, its waves sharing k where they are fewer than waves.
+template <int C, int V, int CB>
 __global__ __launch_bounds__(4 * V) void latent_out_kernel(bf16_t* __restrict__ out, const float* __restrict__ pacc,
                                                            const float* __restrict__ pml, const bf16_t* __restrict__ uv,
                                                            int T, int H, int HP, int nsplit,
                                                            const float* __restrict__ sinks,
                                                            const bf16_t* __restrict__ gate, long ldg) {
-  constexpr int NKK = C / 32;
+  constexpr int KS = V / 16 / CB, NKK = C / 32 / KS;   // shares of k, steps of a share
   static_assert(V == 128 && C == 512, "a thread per 4 latent columns and token");
   __shared__ float ws[4][32];
   __shared__ __attribute__((aligned(16))) bf16_t lat[16][C + 8];
-  const int hd = blockIdx.x, t0 = blockIdx.y * 4, nt = min(4, T - t0);
+  __shared__ __attribute__((aligned(16))) float part[KS > 1 ? KS : 1][CB][KS > 1 ? 64 : 1][4];
+  const int hd = blockIdx.x % H, v0 = blockIdx.x / H * (16 * CB), t0 = blockIdx.y * 4, nt = min(4, T - t0);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, g = lane >> 4;
+  const int cb = wave % CB, kk0 = wave / CB * NKK;
   // everything is requested at once, in the order of its use (loads retire in order): maxima and sums, the first splits' sums, weights
   const int tw = t0 + min(wave, nt - 1);               // a wave per token, a lane per split
   const size_t rec = ((size_t)tw * HP + hd) * nsplit + min(lane, nsplit - 1);
@@ -182,7 +185,7 @@ __global__ __launch_bounds__(4 * V) void latent_out_kernel(bf16_t* __restrict__ 
 #pragma unroll
   for (int u = 0; u < AHEAD; ++u) x[u] = *reinterpret_cast<const f32x4*>(pr + (size_t)min(u, nsplit - 1) * C);
   bf16x8 wf[NKK];
-  const bf16_t* wr = uv + ((size_t)hd * V + 16 * wave + li) * C + 8 * g;
+  const bf16_t* wr = uv + ((size_t)hd * V + v0 + 16 * cb + li) * C + 32 * kk0 + 8 * g;
 #pragma unroll
   for (int kk = 0; kk < NKK; ++kk) wf[kk] = *reinterpret_cast<const bf16x8*>(wr + 32 * kk);
   asm volatile("" ::: "memory");
@@ -220,10 +223,21 @@ __global__ __launch_bounds__(4 * V) void latent_out_kernel(bf16_t* __restrict__ 
   f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int kk = 0; kk < NKK; ++kk)
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[kk], *reinterpret_cast<const bf16x8*>(&lat[li][32 * kk + 8 * g]), acc, 0,
-                                                  0, 0);
-  // acc[i] = out[token li][value column 16 wave + 4 g + i]
-  if (li < nt) stf4(out + ((size_t)(t0 + li) * H + hd) * V + 16 * wave + 4 * g, acc);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[kk], *reinterpret_cast<const bf16x8*>(&lat[li][32 * (kk0 + kk) + 8 * g]), acc,
+                                                  0, 0, 0);
+  // acc[i] = out[token li][value column v0 + 16 cb + 4 g + i], this wave's share of k
+  if constexpr (KS > 1) {
+    *reinterpret_cast<f32x4*>(part[wave / CB][cb][lane]) = acc;
+    lds_barrier();
+    if (wave >= CB) return;
+#pragma unroll
+    for (int x = 1; x < KS; ++x) {
+      const f32x4 y = *reinterpret_cast<const f32x4*>(part[x][cb][lane]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] += y[i];
+    }
+  }
+  if (li < nt) stf4(out + ((size_t)(t0 + li) * H + hd) * V + v0 + 16 * cb + 4 * g, acc);
 }
 
 }  // namespace k8sllm
@@ -251,9 +265,14 @@ extern "C" int k8s_latent_token(void* out, float* pacc, float* pml, const void* 
   latent_token_kernel<512, 64><<<dim3(T, hg, nsplit), 256, LDS, s>>>(pacc, pml, (const bf16_t*)q_abs, (const bf16_t*)q,
                                                                      (const bf16_t*)cache, block_tables, max_blocks, tok_seq,
                                                                      positions, H, Dn, window, scale, bs, nsplit);
-  const dim3 grid(H, (T + 3) / 4);
-  if (grid.y > 65535) return -2;
-  latent_out_kernel<512, 128><<<grid, 512, 0, s>>>((bf16_t*)out, pacc, pml, (const bf16_t*)uv, T, H, hg * 16, nsplit, sinks,
-                                                   (const bf16_t*)gate, ldg);
+  // few heads and tokens: a quarter of a head's value columns a workgroup.  A compute unit takes the weights of 128 columns, rows of 64
+  // bytes to an instruction, in about 4 us whoever else is idle; the splits' sums are read four times as often, from L2
+  const int groups = (T + 3) / 4;
+#define K8S_LO(CB)                                                                                                                  \
+  latent_out_kernel<512, 128, CB><<<dim3(H * (8 / CB), groups), 512, 0, s>>>((bf16_t*)out, pacc, pml, (const bf16_t*)uv, T, H, hg * 16, \
+                                                                             nsplit, sinks, (const bf16_t*)gate, ldg)
+  if (H * groups < 128) K8S_LO(2);
+  else K8S_LO(8);
+#undef K8S_LO
   return (int)hipGetLastError();
 }
