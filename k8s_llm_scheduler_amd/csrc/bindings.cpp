@@ -123,6 +123,8 @@ int k8s_embed_rows(float* out, void* copy, const int* ids, const void* table, in
                    int f32, hipStream_t s);
 int k8s_decode_meta(int* pos, int* slots, int* ar, const int* ctx, const int* block_tables, int max_blocks, int B, int bs,
                     hipStream_t s);
+int k8s_embed_step(float* out, void* copy, const int* ids, const void* table, int W, int vocab, float scale, int f32, int* pos, int* slots,
+                   int* ar, const int* ctx, const int* block_tables, int max_blocks, int B, int bs, hipStream_t s);
 int k8s_norm_shift(void* out, float* x, const void* branch, float mult, const void* rowvec, const void* w, float offset, float eps,
                    const void* mu, void* state, const int* seq_slots, const int* positions, int n, int T, int W, int f32, hipStream_t s);
 int k8s_resnorm(float* x, const void* branch, const void* branch2, float mult, const void* rowvec, const void* w,
@@ -585,6 +587,12 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
   m.def("embed_rows", [](uintptr_t out, uintptr_t copy, uintptr_t ids, uintptr_t table, int T, int W, int vocab,
                          float scale, int f32, int64_t s) {
     check(k8s_embed_rows(P<float>(out), P(copy), P<int>(ids), P(table), T, W, vocab, scale, f32, S(s)), "embed_rows");
+  });
+  m.def("embed_step", [](uintptr_t out, uintptr_t copy, uintptr_t ids, uintptr_t table, int W, int vocab, float scale, int f32,
+                         uintptr_t pos, uintptr_t slots, uintptr_t ar, uintptr_t ctx, uintptr_t block_tables, int max_blocks, int B,
+                         int bs, int64_t s) {
+    check(k8s_embed_step(P<float>(out), P(copy), P<int>(ids), P(table), W, vocab, scale, f32, P<int>(pos), P<int>(slots), P<int>(ar),
+                         P<int>(ctx), P<int>(block_tables), max_blocks, B, bs, S(s)), "embed_step");
   });
   m.def("decode_meta", [](uintptr_t pos, uintptr_t slots, uintptr_t ar, uintptr_t ctx, uintptr_t block_tables,
                           int max_blocks, int B, int bs, int64_t s) {

@@ -109,10 +109,15 @@ __global__ __launch_bounds__(1024) void wkv_scan_kernel(TA* __restrict__ out, co
   const int hd = blockIdx.y;
   int s, a, b, p0;
   bool from_zero, last = true, many = false;
-  if (MODE == 0 || MODE == 3) {
+  if (MODE == 3) {                    // (token s; what its position decides is applied when its inputs are under way)
+    s = a = blockIdx.x;
+    b = a + 1;
+    p0 = positions[a];
+    from_zero = false;
+  } else if (MODE == 0) {
     s = blockIdx.x;
     a = cu_q[s];
-    b = MODE == 3 ? a + 1 : cu_q[s + 1];
+    b = cu_q[s + 1];
     if (b <= a) return;
     p0 = positions[a];
     if (p0 < 0) return;
@@ -131,7 +136,8 @@ __global__ __launch_bounds__(1024) void wkv_scan_kernel(TA* __restrict__ out, co
   const int j = threadIdx.x, c = threadIdx.y, NS = blockDim.y, DV = blockDim.x;
   const bool on = j < D;
   const int HD = H * D, i0 = c * CH;
-  float* st = state + ((size_t)seq_slots[s] * H + hd) * D * D;
+  const int slot = seq_slots[s];
+  float* st = state + ((size_t)(MODE == 3 && p0 < 0 ? 0 : slot) * H + hd) * D * D;
   const float* src = many ? cs_start + ((size_t)blockIdx.x * H + hd) * D * D : st;
   float S[CH];
 #pragma unroll
@@ -164,6 +170,11 @@ __global__ __launch_bounds__(1024) void wkv_scan_kernel(TA* __restrict__ out, co
   };
   fetch(a);
   if (MODE == 3) {
+    if (p0 <= 0) {
+      if (p0 < 0) return;
+#pragma unroll
+      for (int e = 0; e < CH; ++e) S[e] = 0.f;
+    }
     const int n = L / NS;
     float part = 0.f;
     if (on) {

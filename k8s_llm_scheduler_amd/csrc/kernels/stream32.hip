@@ -10,9 +10,8 @@ namespace k8sllm {
 
 // out[t, :] = float(table[ids[t], :]) * scale; copy (optional) the same in the table's type, as the first sublayer reads it
 template <typename TA>
-__global__ void embed_rows_kernel(float* __restrict__ out, TA* __restrict__ copy, const int* __restrict__ ids,
-                                  const TA* __restrict__ table, int W, int vocab, float scale) {
-  const int t = blockIdx.x;
+__device__ __forceinline__ void embed_row(float* __restrict__ out, TA* __restrict__ copy, const int* __restrict__ ids,
+                                          const TA* __restrict__ table, int W, int vocab, float scale, int t) {
   int id = ids[t];
   id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
   for (int i = threadIdx.x; i < W; i += blockDim.x) {
@@ -21,15 +20,19 @@ __global__ void embed_rows_kernel(float* __restrict__ out, TA* __restrict__ copy
     if (copy != nullptr) stf(copy, (size_t)t * W + i, v);
   }
 }
+template <typename TA>
+__global__ void embed_rows_kernel(float* __restrict__ out, TA* __restrict__ copy, const int* __restrict__ ids,
+                                  const TA* __restrict__ table, int W, int vocab, float scale) {
+  embed_row(out, copy, ids, table, W, vocab, scale, blockIdx.x);
+}
 
 // What a step of single tokens needs to know of its B slot rows, in one launch: pos = ctx - 1, the cache slot of that
 // position (-1: an idle row, ctx <= 0), ar = 0 .. B (query offsets, sequence and state slot of every row).  A context
 // beyond its row of the block table idles the row.  Launch bound: as a dozen element-wise launches this took 67 us of a
 // captured step (4.6 us a launch), as one 5 us.
-__global__ void decode_meta_kernel(int* __restrict__ pos, int* __restrict__ slots, int* __restrict__ ar,
-                                   const int* __restrict__ ctx, const int* __restrict__ block_tables, int max_blocks,
-                                   int B, int bs) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void decode_meta_row(int* __restrict__ pos, int* __restrict__ slots, int* __restrict__ ar,
+                                                const int* __restrict__ ctx, const int* __restrict__ block_tables, int max_blocks,
+                                                int B, int bs, int i) {
   if (i > B) return;
   ar[i] = i;
   if (i == B) return;
@@ -37,6 +40,21 @@ __global__ void decode_meta_kernel(int* __restrict__ pos, int* __restrict__ slot
   const bool live = p >= 0 && blk < max_blocks;
   pos[i] = live ? p : min(p, -1);
   slots[i] = live ? block_tables[(size_t)i * max_blocks + blk] * bs + (p - blk * bs) : -1;
+}
+__global__ void decode_meta_kernel(int* __restrict__ pos, int* __restrict__ slots, int* __restrict__ ar,
+                                   const int* __restrict__ ctx, const int* __restrict__ block_tables, int max_blocks,
+                                   int B, int bs) {
+  decode_meta_row(pos, slots, ar, ctx, block_tables, max_blocks, B, bs, blockIdx.x * blockDim.x + threadIdx.x);
+}
+// Both of a step of B tokens, which begin it, in one launch: workgroups of a row each, then those of the step's description.
+template <typename TA>
+__global__ void embed_step_kernel(float* __restrict__ out, TA* __restrict__ copy, const int* __restrict__ ids,
+                                  const TA* __restrict__ table, int W, int vocab, float scale, int* __restrict__ pos,
+                                  int* __restrict__ slots, int* __restrict__ ar, const int* __restrict__ ctx,
+                                  const int* __restrict__ block_tables, int max_blocks, int B, int bs) {
+  const int t = blockIdx.x;
+  if (t < B) embed_row(out, copy, ids, table, W, vocab, scale, t);
+  else decode_meta_row(pos, slots, ar, ctx, block_tables, max_blocks, B, bs, (t - B) * blockDim.x + threadIdx.x);
 }
 
 // x[t] += mult * (branch[t] + branch2[t]) + rowvec (each optional), stored back in fp32; then (w != null)
@@ -1042,6 +1060,18 @@ extern "C" int k8s_decode_meta(int* pos, int* slots, int* ar, const int* ctx, co
                                int B, int bs, hipStream_t s) {
   if (B < 0 || max_blocks < 0 || bs <= 0) return -1;
   decode_meta_kernel<<<(B + 256) / 256, 256, 0, s>>>(pos, slots, ar, ctx, block_tables, max_blocks, B, bs);
+  return (int)hipGetLastError();
+}
+
+extern "C" int k8s_embed_step(float* out, void* copy, const int* ids, const void* table, int W, int vocab, float scale, int f32, int* pos,
+                              int* slots, int* ar, const int* ctx, const int* block_tables, int max_blocks, int B, int bs,
+                              hipStream_t s) {
+  if (B <= 0 || max_blocks < 0 || bs <= 0 || W <= 0 || vocab <= 0) return -1;
+  const int grid = B + (B + 256) / 256;
+  if (f32) embed_step_kernel<float><<<grid, 256, 0, s>>>(out, (float*)copy, ids, (const float*)table, W, vocab, scale, pos, slots, ar, ctx,
+                                                         block_tables, max_blocks, B, bs);
+  else embed_step_kernel<bf16_t><<<grid, 256, 0, s>>>(out, (bf16_t*)copy, ids, (const bf16_t*)table, W, vocab, scale, pos, slots, ar, ctx,
+                                                      block_tables, max_blocks, B, bs);
   return (int)hipGetLastError();
 }
 

@@ -324,6 +324,8 @@ class _Layer:
 
 
 class FavizenModel(StreamModel):
+    embeds_step = True
+
     def __init__(self, cfg: FavizenConfig, tp: Optional[TPGroup] = None, device="cpu", dtype=torch.bfloat16,
                  seed: int = 0, weights: Optional[str] = None, tensors: Optional[Dict[str, torch.Tensor]] = None,
                  max_model_len: int = 8192, weight_dtype: str = "bf16"):
@@ -553,7 +555,7 @@ class FavizenModel(StreamModel):
     def _blocks(self, ids, b, after=None):
         """The residual stream before the last layer's branch is added, and that branch: (x, branch, norm weight, bias)."""
         c, dt = self.cfg, self.dtype
-        x = sm.embed_rows(ids, self.embed, c.embed_scale)
+        x = self._embed(ids, b, c.embed_scale)
         b["routes"] = {k: sm.moe_table_align(ids, t, k[0]) for k, t in self._tables.items()}
         pend = (None, None, None)        # branch, weight of the norm on it, its bias: not yet added
 

@@ -283,6 +283,8 @@ class _Layer:
 
 
 class KatidraModel(StreamModel):
+    embeds_step = True
+
     def __init__(self, cfg: KatidraConfig, tp: Optional[TPGroup] = None, device="cpu", dtype=torch.bfloat16,
                  seed: int = 0, weights: Optional[str] = None, tensors: Optional[Dict[str, torch.Tensor]] = None,
                  max_model_len: int = 8192, weight_dtype: str = "bf16"):
@@ -410,7 +412,7 @@ class KatidraModel(StreamModel):
     def _blocks(self, ids, b, after=None):
         """The residual stream before the last sublayer's output is added, that output and the weight of the norm on it."""
         c, dt = self.cfg, self.dtype
-        x, h = sm.embed_rows(ids, self.embed, c.embed_scale, copy=True)    # h: the stream as the next sublayer reads it
+        x, h = self._embed(ids, b, c.embed_scale, copy=True)    # h: the stream as the next sublayer reads it
         few = ids.shape[0] <= sm.NORM_GEMV_MAX_M and after is None
         pend, last = None, len(self.layers) - 1       # few rows: the output not yet added, which the next product norms and adds
 

@@ -330,6 +330,8 @@ class _Run:
 
 
 class PutulornModel(StreamModel):
+    embeds_step = True
+
     def __init__(self, cfg: PutulornConfig, tp: Optional[TPGroup] = None, device="cpu", dtype=torch.bfloat16,
                  seed: int = 0, weights: Optional[str] = None, tensors: Optional[Dict[str, torch.Tensor]] = None,
                  max_model_len: int = 8192, weight_dtype: str = "bf16"):
@@ -497,7 +499,7 @@ class PutulornModel(StreamModel):
     def _forward(self, ids, b, rows) -> torch.Tensor:
         c, dt = self.cfg, self.dtype
         eps, mult = c.rms_eps, c.residual_mult
-        x = sm.embed_rows(ids, self.embed)
+        x = self._embed(ids, b)
         few = dt == torch.bfloat16 and sm.rows_join(ids.shape[0], c.hidden)   # the norms go with the products on both sides
         pend = r = None                   # the branch output not yet added: the next norm adds it in fp32; or the rows as they are then
         for i, run in enumerate(self.runs):
@@ -543,7 +545,7 @@ class PutulornModel(StreamModel):
         """(debugging / tests) the fp32 residual stream after every layer run."""
         outs = []
         c, dt = self.cfg, self.dtype
-        x = sm.embed_rows(ids, self.embed)
+        x = self._embed(ids, b)
         for run in self.runs:
             L = self.layers[run.layer]
             step = self.loop_step[run.step] if run.step is not None else None

@@ -55,6 +55,7 @@ class StreamModel:
     prefill_overlap = False
     prefill_overlap_min = 1 << 30
     fused_decode = True
+    embeds_step = False      # _forward takes its first rows from _embed, which also works out a decode step's description
 
     def __init__(self, cfg, tp: Optional[TPGroup], device, dtype, seed: int, max_model_len: int, weight_dtype: str):
         self.cfg = cfg
@@ -150,10 +151,23 @@ class StreamModel:
         self._check_ready()
         B = tokens.shape[0]
         tables = block_tables.contiguous()
+        if self.embeds_step:
+            return self._forward(tokens, {"step": (context_lens.to(torch.int32).contiguous(), tables.to(torch.int32)),
+                                          "block_tables": tables, "max_keys": int(max_context)}, None)
         pos, slots, ar = sm.decode_meta(context_lens.to(torch.int32).contiguous(), tables.to(torch.int32), self.block_size)
         b = {"positions": pos, "slot_mapping": slots, "cu_q": ar, "tok_seq": ar[:B], "block_tables": tables,
              "seq_slots": ar[:B], "max_keys": int(max_context)}
         return self._forward(tokens, b, None)
+
+    def _embed(self, ids, b: dict, scale: float = 1.0, copy: bool = False):
+        """:func:`seqmix.embed_rows`, and with it the rest of a decode step's description."""
+        step = b.pop("step", None)
+        if step is None:
+            return sm.embed_rows(ids, self.embed, scale, copy)
+        x, (pos, slots, ar) = sm.embed_step(ids, self.embed, *step, self.block_size, scale, copy)
+        B = ids.shape[0]
+        b.update(positions=pos, slot_mapping=slots, cu_q=ar, tok_seq=ar[:B], seq_slots=ar[:B])
+        return x
 
     def warm(self) -> None:
         pass

@@ -80,20 +80,39 @@ def embed_rows(ids: torch.Tensor, table: torch.Tensor, scale: float = 1.0, copy:
     return (out, same) if copy else out
 
 
-def decode_meta(context_lens: torch.Tensor, block_tables: torch.Tensor, block_size: int):
-    """Of a step of single tokens, row i = state slot i with ``context_lens[i]`` tokens (0: idle): int32 (positions,
-    cache slots (-1: idle), 0 .. B)."""
-    if not _gpu(context_lens, block_tables):
-        return ref.decode_meta(context_lens, block_tables, block_size)
+def _step_meta(context_lens: torch.Tensor, block_tables: torch.Tensor):
     B = context_lens.shape[0]
     if block_tables.dim() != 2 or block_tables.shape[0] < B:
         raise ValueError("decode_meta: a row of the block table for every context length")
     n = (B + 4) // 4 * 4
     meta = torch.empty(3, n, dtype=I32, device=context_lens.device)      # rows 16 bytes aligned
-    pos, slots, ar = meta[0, :B], meta[1, :B], meta[2, :B + 1]
+    return meta[0, :B], meta[1, :B], meta[2, :B + 1]
+
+
+def decode_meta(context_lens: torch.Tensor, block_tables: torch.Tensor, block_size: int):
+    """Of a step of single tokens, row i = state slot i with ``context_lens[i]`` tokens (0: idle): int32 (positions,
+    cache slots (-1: idle), 0 .. B)."""
+    if not _gpu(context_lens, block_tables):
+        return ref.decode_meta(context_lens, block_tables, block_size)
+    pos, slots, ar = _step_meta(context_lens, block_tables)
     _native().decode_meta(pos.data_ptr(), slots.data_ptr(), ar.data_ptr(), _p(context_lens, I32, "context_lens"),
-                          _p(block_tables, I32, "block_tables"), block_tables.shape[1], B, int(block_size), -1)
+                          _p(block_tables, I32, "block_tables"), block_tables.shape[1], context_lens.shape[0], int(block_size), -1)
     return pos, slots, ar
+
+
+def embed_step(ids: torch.Tensor, table: torch.Tensor, context_lens: torch.Tensor, block_tables: torch.Tensor, block_size: int,
+               scale: float = 1.0, copy: bool = False):
+    """(:func:`embed_rows`, :func:`decode_meta`) of a step of single tokens in one launch."""
+    B, W = ids.shape[0], table.shape[1]
+    if B == 0 or context_lens.shape[0] != B or not _gpu(ids, table, context_lens, block_tables):
+        return embed_rows(ids, table, scale, copy), decode_meta(context_lens, block_tables, block_size)
+    pos, slots, ar = _step_meta(context_lens, block_tables)
+    out = torch.empty(B, W, dtype=F32, device=table.device)
+    same = torch.empty(B, W, dtype=table.dtype, device=table.device) if copy else None
+    _native().embed_step(out.data_ptr(), _p(same), _p(ids, I32, "ids"), _p(table), W, table.shape[0], float(scale), _f32(table.dtype),
+                         pos.data_ptr(), slots.data_ptr(), ar.data_ptr(), _p(context_lens, I32, "context_lens"),
+                         _p(block_tables, I32, "block_tables"), block_tables.shape[1], B, int(block_size), -1)
+    return ((out, same) if copy else out), (pos, slots, ar)
 
 
 def resnorm(x: torch.Tensor, w: Optional[torch.Tensor], eps: float, *, branch: Optional[torch.Tensor] = None,

@@ -213,3 +213,50 @@ def test_latent_begin(C, R, H, Dn, dims, interleaved, T, entries):
             assert ((c1[slots[t]].double() - row).abs() <= 2.0 ** -8 * row.abs() + 1e-5).all()
     untouched = [i for i in range(T + 3) if i not in [s for s, p in zip(slots, pos) if s >= 0 and p >= 0]]
     assert torch.equal(c1[untouched], cache[untouched])
+
+
+@pytest.mark.parametrize("dt", [BF, F32])
+@pytest.mark.parametrize("B,W,copy", [(1, 2048, True), (8, 48, False), (255, 64, True), (256, 4096, False), (600, 8, True)])
+def test_embed_step(dt, B, W, copy, entries):
+    r = data(B + W)
+    table, ids = r(90, W, dt=dt), torch.randint(-1, 91, (B,), dtype=torch.int32).to(DEV)
+    ctx = torch.randint(0, 70, (B,), dtype=torch.int32).to(DEV)              # (beyond the tables' 4 pages of 16: idle)
+    tables = torch.randint(0, 999, (B + 1, 4), dtype=torch.int32).to(DEV)
+    got, meta = sm.embed_step(ids, table, ctx, tables, 16, 1.7, copy)
+    assert entries == ["embed_step"]
+    want = sm.embed_rows(ids, table, 1.7, copy)
+    for a, b in zip(got if copy else (got,), want if copy else (want,)):
+        assert torch.equal(a, b)
+    for a, b in zip(meta, sm.decode_meta(ctx, tables, 16)):
+        assert torch.equal(a, b) and a.data_ptr() % 16 == 0
+
+
+@pytest.mark.parametrize("gate", [False, True])
+@pytest.mark.parametrize("T,H", [(1, 16), (5, 3), (28, 16), (32, 16), (9, 40), (13, 40), (1, 130)])
+@pytest.mark.parametrize("ctx", [40, 700, 2200])
+def test_single_tokens_value_columns(T, H, ctx, gate):
+    """A quarter of a head's value columns a workgroup, and all of them, on both sides of the change; up to 32 splits."""
+    r = data(T + H + ctx)
+    C, R, Dn, V, bs = 512, 64, 128, 128, 16
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    pages = -(-ctx // bs)
+    cache, q, q_abs, uv = r(T * pages * bs, C + R), r(T, H * (Dn + R)), r(T, H, C), r(H, V, C, m=C ** -0.5)
+    g = r(T, H) if gate else None
+    pos = [ctx - 1 - (7 * i) % 30 for i in range(T)]
+    b = {"cu_q": i32(list(range(T + 1))), "tok_seq": i32(list(range(T))), "positions": i32(pos), "max_keys": ctx,
+         "block_tables": torch.randperm(T * pages).to(torch.int32).to(DEV).view(T, pages)}
+    got = sm.latent_mix(q, cache, r(H, C, Dn), uv, None, b, C, R, H, Dn, V, 0, 0.05, bs, gate=g, q_abs=q_abs).view(T, H, V)
+    for t in {0, T // 2, T - 1}:
+        rows = (b["block_tables"][t].long()[:, None] * bs + torch.arange(bs, device=DEV)).reshape(-1)[:pos[t] + 1]
+        k = cache[rows].double()
+        qq = torch.cat([q_abs[t], q[t].view(H, Dn + R)[:, Dn:]], 1).double()
+        p = torch.softmax(0.05 * qq @ k.T, -1)
+        lat = p @ k[:, :C]
+        mass = p @ k[:, :C].abs()
+        if gate:
+            s = torch.sigmoid(g[t].double())[:, None]
+            lat, mass = lat * s, mass * s
+        want = torch.matmul(uv.double(), lat.unsqueeze(-1)).squeeze(-1)
+        # weights and the latent sum in bf16 (2^-9 each, and a score's fp32 error), sums in fp32, the output in bf16
+        bound = torch.matmul(uv.double().abs(), (2.0 ** -7 * mass).unsqueeze(-1)).squeeze(-1) + 2.0 ** -8 * want.abs()
+        assert ((got[t].double() - want).abs() <= bound).all()
