@@ -4,27 +4,28 @@
 // kernel serve plain prefill, chunked prefill and prefix-cached prompts: query i of sequence s
 // sits at absolute position ctx_s - qlen_s + i and attends keys [0, pos].
 //
-// GQA packing: one workgroup = NW waves = 16 NW (query, head) rows = QT = 16 NW / G consecutive queries x
-// the G query heads that share ONE kv head (G = nq / nkv), so every K/V tile is fetched once per
-// group instead of once per query head (8x fewer K/V bytes at Llama-3.3-70B's 8:1 GQA), and the
-// causal key range of a workgroup ends at its QT-th query instead of its 64th.  Row r of the
-// workgroup is query tile * QT + r / G, head kvh * G + r % G.
-// NW = 4, 8 or 16 (64 / 128 / 256 rows): every K/V byte a workgroup stages feeds 16 NW rows of MFMA work, so at
-// long contexts -- where every workgroup streams the whole causal K/V range through L2 -- wider workgroups cut
-// the K/V traffic per FLOP.  The host takes 8 waves when that grid still has >= 256 workgroups (16: opt-in).
+// GQA packing: a wave has 16 RB (query, head) rows, a workgroup those of NW / KS waves = QT consecutive queries x the G query
+// heads that share ONE kv head (G = nq / nkv), so every K/V tile is fetched once per group instead of once per query head, and
+// the causal key range of a workgroup ends at its last query.  Row r of the workgroup is query tile * QT + r / G, head kvh * G +
+// r % G.  KS 2: half of the waves takes every other tile of the same rows' keys; their sums meet at the end.
 //
 // Structure:
-//  * "swapped" QK^T: S^T = K . Q^T with v_mfma_f32_16x16x32_bf16, so each lane ends up holding
-//    16 scores of ONE query row (row = lane & 15): the row max/sum need 2 cross-lane steps and
-//    the probabilities feed the P.V MFMA as its A operand straight from registers (the key
-//    order inside a 32-key step is permuted identically on the V side, see below).
-//  * V tiles (64 keys x 128 d) are staged in LDS with an XOR swizzle and read with the gfx950
-//    transposing read ds_read_b64_tr_b16, which delivers 4 keys of one d column per lane --
-//    exactly the B-operand layout, so V needs no register transpose.
-//  * K and V tiles are fetched one tile AHEAD into registers by all 256 threads (the loads of tile
-//    t+1 are in flight during tile t's MFMAs), then stored into swizzled LDS images shared by the
-//    4 waves; K fragments are read back with conflict-free ds_read_b128.
-//  * online softmax in the log2 domain (scale * log2(e) folded into S).
+//  * "swapped" QK^T: S^T = K . Q^T with v_mfma_f32_16x16x32_bf16, so each lane ends up holding 16 scores of ONE query row (row =
+//    lane & 15) and the probabilities feed the P.V MFMA as its A operand straight from registers (the key order inside a 32-key
+//    step is permuted identically on the V side, see below).
+//  * V tiles (64 keys x 128 d) are staged in LDS with an XOR swizzle and read with the gfx950 transposing read
+//    ds_read_b64_tr_b16, which delivers 4 keys of one d column per lane -- exactly the B-operand layout.
+//  * K and V go through registers into two swizzled LDS images each: the tile after next is on its way, the next one is written,
+//    one barrier a tile that waits for LDS only.
+//  * 32 rows a wave (RB 2) read each K and V fragment for two products: at 16 rows a wave's LDS reads take twice the time of its
+//    products.
+//  * softmax in the log2 domain without a running maximum: the weights are 2^(score - m) with an m that is brought up to date (and
+//    the sums with it) only for a row's first tile and when the weights outgrow 2^12, so a tile costs one fma, power and addition a
+//    score; masks only where a tile crosses the wave's diagonal.
+//  * longest workgroups first, so that the last round is of short ones.
+// What bounds it now: two waves a SIMD, in step between the barriers, each with its products, LDS reads and softmax in turn; at
+// long prompts 42 % of the matrix cores' rate.  Tried: waves of a SIMD half a tile apart with two barriers a tile (251 us against
+// 230 at 3413 tokens), 128 rows of 4 waves (256 us).
 #include <cstdlib>
 
 #include "common.h"
@@ -37,162 +38,230 @@ typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
 
 __device__ __forceinline__ int v_swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
 
-template <int D, int G, int NW>
-__global__ void __launch_bounds__(64 * NW) paged_prefill_kernel(
+template <int G, int RB, int NW, int KS>
+__global__ void __launch_bounds__(64 * NW, 2) paged_prefill_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int* __restrict__ cu_q, const int* __restrict__ context_lens,
-    const int* __restrict__ block_tables, float scale_log2, int nq, int nkv, int block_size, int max_blocks) {
-  static_assert(D == 128, "head_dim 128");
-  constexpr int KT = 64;             // keys per tile
-  constexpr int NT = 64 * NW;        // threads
-  constexpr int CPT = KT * D / 8 / NT;  // 16-byte chunks of one tile per thread (K and V each)
-  __shared__ __attribute__((aligned(16))) char klds[KT * D * 2];
-  __shared__ __attribute__((aligned(16))) char vlds[KT * D * 2];
+    const int* __restrict__ block_tables, float scale_log2, int nq, int nkv, int block_size, int max_blocks, int tiles) {
+  constexpr int D = 128;
+  constexpr int KT = 64;                // keys per tile
+  constexpr int ST = KS * KT;           // keys staged at once: a tile for each share of the waves
+  constexpr int NT = 64 * NW;           // threads
+  constexpr int CPT = ST * D / 8 / NT;  // 16-byte chunks of what is staged per thread (K and V each)
+  constexpr int RW = NW / KS;           // waves of a share
+  constexpr int QT = 16 * RB * RW / G;  // queries per workgroup
+  static_assert(16 * RB % G == 0 || G % (16 * RB) == 0, "a wave's rows are whole queries or part of one");
+  __shared__ __attribute__((aligned(16))) char klds[2][ST * D * 2];
+  __shared__ __attribute__((aligned(16))) char vlds[2][ST * D * 2];
 
-  constexpr int QT = 16 * NW / G;  // queries per workgroup
-  const int s = blockIdx.z, kvh = blockIdx.y, tile = blockIdx.x;
+  // the longest workgroups first; those of a kv head follow each other at a stride of the heads
+  const int s = blockIdx.z, kvh = blockIdx.x % nkv, tile = tiles - 1 - blockIdx.x / nkv;
   const int q0 = cu_q[s], qlen = cu_q[s + 1] - q0;
   if (tile * QT >= qlen) return;
   int ctx = context_lens[s];
   K8S_CHECK_MAX(ctx, max_blocks * block_size, K8S_CHK_CTX);
   const int qstart = ctx - qlen;  // absolute position of query 0
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wid = wave % RW, share = wave / RW;   // which rows, which tile of those staged
   const int g = lane >> 4, li = lane & 15;
   const int* bt = block_tables + (size_t)s * max_blocks;
-  const size_t kv_stride = (size_t)nkv * D;
-
   const int last_row = min(tile * QT + QT - 1, qlen - 1);
   const int kv_end = qstart + last_row + 1;  // keys needed by this workgroup
-  const int ntiles = (kv_end + KT - 1) / KT;
+  const int ntiles = (kv_end + ST - 1) / ST;
 
-  // Tile staging, one tile ahead: thread tid fetches chunks idx = tid + NT c (key row idx/16,
-  // 16-byte column chunk idx%16) of K and V into registers while the current tile is computed,
-  // then stores them swizzled into LDS.  Keys past the context: K clamped (their scores are
-  // masked), V zero (P is 0 there, V must be finite).
-  // The block ids of a tile are requested one tile before its K/V (nbt): otherwise every prefetch is two dependent
-  // round trips (block id, then K/V) against one tile of math, and long contexts pay that chain once per tile.
+  // Tile staging: thread tid fetches chunks idx = tid + NT c (key row idx/16, 16-byte column chunk idx%16) of K and V into
+  // registers while tiles before are computed.  Rows past the context lie in the last key's block (finite or not: K's scores are
+  // masked), V is zeroed there (P is 0, V must be finite).  The block ids of a tile are requested a tile before its K/V: otherwise
+  // every prefetch is two dependent round trips.  Where a row is in its block is carried from tile to tile: the division by the
+  // block size was half of the loop's vector work.
   u32x4 kn[CPT], vn[CPT];
-  int nbt[CPT];
-  auto load_bt = [&](int t) {
+  int nbt[CPT], nbv[CPT], wof[CPT], wov[CPT];    // block ids of the next K and V tile's rows, rows in the blocks
+  int ib[CPT], io[CPT];                          // block table position and row in the block of the next ids
+  const int lastb = (ctx - 1) / block_size, stepb = ST / block_size, stepo = ST - stepb * block_size;
+  const unsigned row_bytes = (unsigned)nkv * D * 2;
+  const char* kp = reinterpret_cast<const char*>(k_cache) + (kvh * D + tid % (D / 8) * 8) * 2;
+  const char* vp = reinterpret_cast<const char*>(v_cache) + (kvh * D + tid % (D / 8) * 8) * 2;
 #pragma unroll
-    for (int c = 0; c < CPT; ++c) {
-      nbt[c] = bt[min(t * KT + (tid + NT * c) / (D / 8), ctx - 1) / block_size];
-      K8S_CHECK_RANGE(nbt[c], 0, K8S_CHK_BLOCK, 0);
-    }
-  };
-  auto fetch = [&](int t) {   // tile t's K/V with the ids in nbt, then tile t + 1's ids
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) {
-      const int idx = tid + NT * c;
-      const int key = t * KT + idx / (D / 8), ch = idx % (D / 8);
-      const int kc = min(key, ctx - 1);
-      const size_t off = (size_t)(nbt[c] * block_size + kc % block_size) * kv_stride + kvh * D + ch * 8;
-      kn[c] = *reinterpret_cast<const u32x4*>(k_cache + off);
-      vn[c] = key < ctx ? *reinterpret_cast<const u32x4*>(v_cache + off) : u32x4{0u, 0u, 0u, 0u};
-    }
-    load_bt(t + 1);   // (keys past the context clamp to the last one: always a valid id)
-  };
-  load_bt(0);
-  fetch(0);
-
-  // my (query, head) row (B operand columns / softmax rows)
-  const int wr = wid * 16 + li;
-  const int row = tile * QT + wr / G, head = kvh * G + wr % G;
-  const int row_c = min(row, qlen - 1);  // clamp padding rows to a valid query
-  const int qpos = qstart + row_c;
-  bf16x8 qf[D / 32];
-  {
-    const bf16_t* qp = q + ((size_t)(q0 + row_c) * nq + head) * D;
-#pragma unroll
-    for (int kk = 0; kk < D / 32; ++kk) qf[kk] = *reinterpret_cast<const bf16x8*>(qp + kk * 32 + g * 8);
+  for (int c = 0; c < CPT; ++c) {
+    const int r = (tid + NT * c) / (D / 8);
+    ib[c] = r / block_size;
+    io[c] = r - ib[c] * block_size;
   }
-
-  f32x4 o[D / 16];
-#pragma unroll
-  for (int n = 0; n < D / 16; ++n) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
-
-  for (int t = 0; t < ntiles; ++t) {
-    const int kbase = t * KT;
-    // ---- tile t: registers -> LDS (both images swizzled: 16-byte chunk ch of row r at ch ^ swz(r))
+  auto ids = [&]() {                             // of the next tile
 #pragma unroll
     for (int c = 0; c < CPT; ++c) {
-      const int idx = tid + NT * c;
-      const int kr = idx / (D / 8), ch = idx % (D / 8);
-      *reinterpret_cast<u32x4*>(klds + kr * (D * 2) + 16 * (ch ^ (kr & 15))) = kn[c];
-      *reinterpret_cast<u32x4*>(vlds + kr * (D * 2) + 16 * (ch ^ v_swz(kr))) = vn[c];
+      nbt[c] = bt[min(ib[c], lastb)];
+      K8S_CHECK_RANGE(nbt[c], 0, K8S_CHK_BLOCK, 0);
+      wof[c] = io[c];
+      ib[c] += stepb;
+      io[c] += stepo;
+      const bool wrap = io[c] >= block_size;
+      io[c] -= wrap ? block_size : 0;
+      ib[c] += wrap;
     }
-    __syncthreads();
-    if (t + 1 < ntiles) fetch(t + 1);  // in flight during this tile's math
+  };
+  auto keep = [&]() {                            // K's ids for V, a tile later
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) {
+      nbv[c] = nbt[c];
+      wov[c] = wof[c];
+    }
+  };
+  auto fetch_k = [&]() {
+#pragma unroll
+    for (int c = 0; c < CPT; ++c)
+      kn[c] = *reinterpret_cast<const u32x4*>(kp + (size_t)(unsigned)(nbt[c] * block_size + wof[c]) * row_bytes);
+  };
+  auto fetch_v = [&]() {
+#pragma unroll
+    for (int c = 0; c < CPT; ++c)
+      vn[c] = *reinterpret_cast<const u32x4*>(vp + (size_t)(unsigned)(nbv[c] * block_size + wov[c]) * row_bytes);
+  };
+  auto mask_v = [&](int t) {                     // tile t's, ahead of its staging
+    if (t * ST + ST <= ctx) return;
+#pragma unroll
+    for (int c = 0; c < CPT; ++c)
+      if (t * ST + (tid + NT * c) / (D / 8) >= ctx) vn[c] = u32x4{0u, 0u, 0u, 0u};
+  };
+  auto stage_k = [&](int buf) {   // both images swizzled: 16-byte chunk ch of row r at ch ^ swz(r)
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) {
+      const int kr = (tid + NT * c) / (D / 8), ch = (tid + NT * c) % (D / 8);
+      *reinterpret_cast<u32x4*>(klds[buf] + kr * (D * 2) + 16 * (ch ^ (kr & 15))) = kn[c];
+    }
+  };
+  auto stage_v = [&](int buf) {
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) {
+      const int kr = (tid + NT * c) / (D / 8), ch = (tid + NT * c) % (D / 8);
+      *reinterpret_cast<u32x4*>(vlds[buf] + kr * (D * 2) + 16 * (ch ^ v_swz(kr))) = vn[c];
+    }
+  };
+  ids();
+  fetch_k();
+  keep();
 
-    // ---- S^T = K . Q^T for 4 key sub-tiles of 16; lane (li, g) reads key row 16m + li, d 32kk + 8g
-    f32x4 sacc[KT / 16];
+  // my (query, head) rows (B operand columns / softmax rows)
+  bf16x8 qf[RB][D / 32];
+  int qpos[RB];
+  // (a negative scale: of the negated queries; 0, which the masked scores could not take: of zeros)
+  const uint32_t flip = scale_log2 < 0.f ? 0x80008000u : 0u, live = scale_log2 == 0.f ? 0u : ~0u;
+  const float scale = scale_log2 == 0.f ? 1.f : fabsf(scale_log2);
+#pragma unroll
+  for (int b = 0; b < RB; ++b) {
+    const int wr = (wid * RB + b) * 16 + li;
+    const int row = min(tile * QT + wr / G, qlen - 1), head = kvh * G + wr % G;   // (padding rows: a valid query)
+    qpos[b] = qstart + row;
+    const u32x4* qp = reinterpret_cast<const u32x4*>(q + ((size_t)(q0 + row) * nq + head) * D);
+#pragma unroll
+    for (int kk = 0; kk < D / 32; ++kk) {
+      u32x4 v = qp[kk * 4 + g];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = (v[e] ^ flip) & live;
+      qf[b][kk] = __builtin_bit_cast(bf16x8, v);
+    }
+  }
+  // the wave's first and last query: tiles past the last are left out, tiles up to the first need no mask
+  const int wq0 = qstart + min(tile * QT + wid * RB * 16 / G, qlen - 1);
+  const int wq1 = qstart + min(tile * QT + (wid * RB * 16 + 16 * RB - 1) / G, qlen - 1);
+
+  f32x4 o[RB][D / 16];
+#pragma unroll
+  for (int b = 0; b < RB; ++b)
+#pragma unroll
+    for (int n = 0; n < D / 16; ++n) o[b][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run[RB], l_run[RB];   // row li's maximum so far, log2 (or up to 8 less); this lane's share of its sum
+#pragma unroll
+  for (int b = 0; b < RB; ++b) m_run[b] = -INFINITY, l_run[b] = 0.f;
+
+  f32x4 sacc[RB][KT / 16];
+  bf16x8 pa[RB][KT / 32];
+  // S^T = K . Q^T for 4 key sub-tiles of 16; lane (li, g) reads key row 16m + li, d 32kk + 8g
+  auto scores = [&](const char* kl) {
 #pragma unroll
     for (int m = 0; m < KT / 16; ++m) {
       const int kr = 16 * m + li;
-      f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int b = 0; b < RB; ++b) sacc[b][m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kk = 0; kk < D / 32; ++kk) {
-        const bf16x8 ka = *reinterpret_cast<const bf16x8*>(klds + kr * (D * 2) + 16 * ((4 * kk + g) ^ (kr & 15)));
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qf[kk], acc, 0, 0, 0);
-      }
-      sacc[m] = acc;
-    }
-    // lane holds S[row li][key kbase + 16m + 4g + i]
-    float tmax = -INFINITY;
+        const bf16x8 ka = *reinterpret_cast<const bf16x8*>(kl + kr * (D * 2) + 16 * ((4 * kk + g) ^ (kr & 15)));
 #pragma unroll
-    for (int m = 0; m < KT / 16; ++m) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int key = kbase + m * 16 + g * 4 + i;
-        float v = sacc[m][i] * scale_log2;
-        v = (key <= qpos && key < ctx) ? v : -INFINITY;
-        sacc[m][i] = v;
-        tmax = fmaxf(tmax, v);
+        for (int b = 0; b < RB; ++b) sacc[b][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qf[b][kk], sacc[b][m], 0, 0, 0);
       }
     }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
-    const float m_new = fmaxf(m_run, tmax);
-    const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-    const float alpha = exp2f(m_run - m_use);
-    float rsum = 0.f;
+  };
+  // lane holds S[row li][key kbase + 16m + 4g + i]; the weights are 2^(score - m) for an m near the row's maximum: a row's first tile
+  // brings it up to date, and later ones only if the row has outgrown it (a lane's weights of a tile sum past 2^12: none is larger)
+  auto weights = [&](int kbase, bool first) {
+    if (kbase + KT - 1 > wq0) {
 #pragma unroll
-    for (int m = 0; m < KT / 16; ++m) {
+      for (int b = 0; b < RB; ++b)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float pv = exp2f(sacc[m][i] - m_use);
-        sacc[m][i] = pv;
-        rsum += pv;
+        for (int m = 0; m < KT / 16; ++m)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (kbase + m * 16 + g * 4 + i > qpos[b]) sacc[b][m][i] = -INFINITY;
+    }
+    f32x4 pw[RB][KT / 16];
+    float rs[RB];
+    auto power = [&]() {
+#pragma unroll
+      for (int b = 0; b < RB; ++b) {
+        const float m_use = m_run[b] == -INFINITY ? 0.f : m_run[b];
+        f32x4 r4 = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < KT / 16; ++m)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            pw[b][m][i] = __builtin_amdgcn_exp2f(fmaf(sacc[b][m][i], scale, -m_use));
+            r4[i] += pw[b][m][i];
+          }
+        rs[b] = (r4[0] + r4[1]) + (r4[2] + r4[3]);
       }
+    };
+    bool grow = first;
+    if (!first) {
+      power();
+#pragma unroll
+      for (int b = 0; b < RB; ++b) grow |= rs[b] > 4096.f || m_run[b] == -INFINITY;
     }
-    rsum += __shfl_xor(rsum, 16, WAVE);
-    rsum += __shfl_xor(rsum, 32, WAVE);
-    l_run = l_run * alpha + rsum;
-    m_run = m_new;
-
-    // rescale O rows (row 4g+i of O lives in lanes whose li == 4g+i for the stats)
-    float a_i[4];
+    if (__any(grow)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) a_i[i] = __shfl(alpha, g * 4 + i, WAVE);
+      for (int b = 0; b < RB; ++b) {
+        float v = -INFINITY;
 #pragma unroll
-    for (int n = 0; n < D / 16; ++n) {
+        for (int m = 0; m < KT / 16; ++m)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o[n][i] *= a_i[i];
+          for (int i = 0; i < 4; ++i) v = fmaxf(v, sacc[b][m][i] * scale);
+        v = fmaxf(v, __shfl_xor(v, 16, WAVE));
+        v = fmaxf(v, __shfl_xor(v, 32, WAVE));
+        const float m_new = fmaxf(m_run[b], v);
+        const float alpha = m_run[b] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[b] - m_new);
+        l_run[b] *= alpha;
+        m_run[b] = m_new;
+        // row 4g+i of O lives in lanes whose li == 4g+i for the stats
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float a = __shfl(alpha, g * 4 + i, WAVE);
+#pragma unroll
+          for (int n = 0; n < D / 16; ++n) o[b][n][i] *= a;
+        }
+      }
+      power();
     }
-
     // P as A operand: k-step st covers keys 32st..32st+31 in the permuted order
     // slot j<4 -> key 32st + 4g + j ; slot j>=4 -> key 32st + 16 + 4g + (j-4)
-    bf16x8 pa[KT / 32];
 #pragma unroll
-    for (int st = 0; st < KT / 32; ++st) {
+    for (int b = 0; b < RB; ++b) {
+      l_run[b] += rs[b];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        pa[st][j] = (__bf16)sacc[2 * st][j];
-        pa[st][4 + j] = (__bf16)sacc[2 * st + 1][j];
-      }
+      for (int st = 0; st < KT / 32; ++st)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) pa[b][st][j] = (__bf16)pw[b][2 * st + (j >> 2)][j & 3];
     }
-
+  };
+  auto values = [&](const char* vl) {
     const int qd = li >> 2, pd = li & 3;  // tr-read lane roles: row q, column group p
 #pragma unroll
     for (int st = 0; st < KT / 32; ++st) {
@@ -202,34 +271,103 @@ __global__ void __launch_bounds__(64 * NW) paged_prefill_kernel(
       for (int n = 0; n < D / 16; ++n) {
         const int col = 16 * n + 4 * pd;
         const int ch = col >> 3, hb = (col & 7) * 2;
-        const lds_bf16x4* a0 = (const lds_bf16x4*)(vlds + r0 * (D * 2) + 16 * (ch ^ v_swz(r0)) + hb);
-        const lds_bf16x4* a1 = (const lds_bf16x4*)(vlds + r1 * (D * 2) + 16 * (ch ^ v_swz(r1)) + hb);
+        const lds_bf16x4* a0 = (const lds_bf16x4*)(vl + r0 * (D * 2) + 16 * (ch ^ v_swz(r0)) + hb);
+        const lds_bf16x4* a1 = (const lds_bf16x4*)(vl + r1 * (D * 2) + 16 * (ch ^ v_swz(r1)) + hb);
         const bf16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)a0);
         const bf16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)a1);
         bf16x8 vb;
 #pragma unroll
         for (int j = 0; j < 4; ++j) { vb[j] = v0[j]; vb[4 + j] = v1[j]; }
-        o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa[st], vb, o[n], 0, 0, 0);
+#pragma unroll
+        for (int b = 0; b < RB; ++b) o[b][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa[b][st], vb, o[b][n], 0, 0, 0);
       }
     }
-    __syncthreads();  // before the next tile overwrites the LDS images
+  };
+  fetch_v();
+  ids();
+  stage_k(0);
+  mask_v(0);
+  stage_v(0);
+  auto ahead = [&](int t) {
+    if (t >= ntiles) return;
+    fetch_k();
+    keep();
+    fetch_v();
+    ids();
+  };
+  ahead(1);
+  lds_barrier();
+  for (int t = 0; t < ntiles; ++t) {
+    if (t + 1 < ntiles) {
+      stage_k((t + 1) & 1);          // (tile t - 1 was read before the last barrier)
+      mask_v(t + 1);
+      stage_v((t + 1) & 1);
+      ahead(t + 2);
+    }
+    const int kbase = t * ST + share * KT;
+    if (kbase <= wq1) {
+      scores(klds[t & 1] + share * (KT * D * 2));
+      weights(kbase, t == 0);
+      values(vlds[t & 1] + share * (KT * D * 2));
+    }
+    lds_barrier();                   // tile t has been read and tile t + 1 written
   }
 
-  // ---- normalise and store: o[n][i] = O[row 4g+i][d 16n + li]
-  float inv_l[4];
+  float l_row[RB];                   // row li's sum
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float lv = __shfl(l_run, g * 4 + i, WAVE);
-    inv_l[i] = lv > 0.f ? 1.f / lv : 0.f;
+  for (int b = 0; b < RB; ++b) {
+    l_row[b] = l_run[b] + __shfl_xor(l_run[b], 16, WAVE);
+    l_row[b] += __shfl_xor(l_row[b], 32, WAVE);
   }
+  if constexpr (KS == 2) {           // the second share's sums join the first one's, through the staged K
+    static_assert(RW * RB * (D / 16) * 64 * 16 <= 2 * ST * D * 2, "room for a share's sums");
+    if (share == 1 && kv_end <= KT) return;
+    f32x4* os = reinterpret_cast<f32x4*>(klds[0]);
+    float* ms = reinterpret_cast<float*>(vlds[0]);
+    if (share == 1) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int orow = wid * 16 + g * 4 + i;
-    const int r = tile * QT + orow / G, oh = kvh * G + orow % G;
-    if (r < qlen) {
-      bf16_t* op = out + ((size_t)(q0 + r) * nq + oh) * D + li;
+      for (int b = 0; b < RB; ++b) {
 #pragma unroll
-      for (int n = 0; n < D / 16; ++n) op[16 * n] = f2bf(o[n][i] * inv_l[i]);
+        for (int n = 0; n < D / 16; ++n) os[((wid * RB + b) * (D / 16) + n) * 64 + lane] = o[b][n];
+        if (g == 0) {
+          ms[((wid * RB + b) * 16 + li) * 2] = m_run[b];
+          ms[((wid * RB + b) * 16 + li) * 2 + 1] = l_row[b];
+        }
+      }
+    }
+    if (kv_end > KT) lds_barrier();
+    if (share == 1) return;
+#pragma unroll
+    for (int b = 0; b < RB && kv_end > KT; ++b) {
+      const float m1 = ms[((wid * RB + b) * 16 + li) * 2], l1 = ms[((wid * RB + b) * 16 + li) * 2 + 1];
+      const float m = fmaxf(m_run[b], m1);
+      const float a0 = m_run[b] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[b] - m);
+      const float a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - m);
+      l_row[b] = l_row[b] * a0 + l1 * a1;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float c0 = __shfl(a0, g * 4 + i, WAVE), c1 = __shfl(a1, g * 4 + i, WAVE);
+#pragma unroll
+        for (int n = 0; n < D / 16; ++n)
+          o[b][n][i] = o[b][n][i] * c0 + os[((wid * RB + b) * (D / 16) + n) * 64 + lane][i] * c1;
+      }
+    }
+  }
+
+  // ---- normalise and store: o[b][n][i] = O[row 4g+i][d 16n + li]
+#pragma unroll
+  for (int b = 0; b < RB; ++b) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float lv = __shfl(l_row[b], g * 4 + i, WAVE);
+      const float inv_l = lv > 0.f ? 1.f / lv : lv == 0.f ? 0.f : lv;   // (NaN stays one)
+      const int orow = (wid * RB + b) * 16 + g * 4 + i;
+      const int r = tile * QT + orow / G, oh = kvh * G + orow % G;
+      if (r < qlen) {
+        bf16_t* op = out + ((size_t)(q0 + r) * nq + oh) * D + li;
+#pragma unroll
+        for (int n = 0; n < D / 16; ++n) op[16 * n] = f2bf(o[b][n][i] * inv_l);
+      }
     }
   }
 }
@@ -248,30 +386,40 @@ extern "C" int k8s_paged_prefill_attention(void* out, const void* q, const void*
   if (D != 128 || nq % nkv != 0) return -1;
   const int G = nq / nkv;
   const float sl2 = scale * 1.4426950408889634f;
-  // 8 waves when that grid still covers every CU, else 4.  The 16-wave form measured no faster than 8 on the 256-node
-  // prompts (profiles/bench_r3_nodes256_attn_waves_ab.jsonl) and stays opt-in: K8S_PREFILL_ATTN_WAVES = 4 / 8 / 16.
-  static const int waves_env = [] { const char* e = getenv("K8S_PREFILL_ATTN_WAVES"); return e ? atoi(e) : 0; }();
-  auto wgs = [&](int nw) { return (long long)((max_qlen + 16 * nw / G - 1) / (16 * nw / G)) * nkv * num_seqs; };
-  const int nw = (waves_env == 4 || waves_env == 8 || waves_env == 16) ? waves_env : wgs(8) >= 256 ? 8 : 4;
-#define PF(GG, NWW)                                                                                          \
+  // Rows of a workgroup and shares of the keys.  Few workgroups: 64 rows, the keys shared by two halves of 8 waves (one workgroup a CU);
+  // up to two a CU of 4 waves, unless the prompt is long and the longest of them decides; from about one workgroup of 256 rows a CU
+  // those, which read each key and value byte a quarter as often; between, 128 rows with shared keys.  us of 64 rows, 64 shared, 128
+  // shared, 256, heads 64 / 8 unless said: 241 tokens behind 224 14.9, 12.6, 17.3,
+  // 21.5; 97 behind 1000 27.3, 20.4, 28.2, 39.6; 512 17.2, 19.0, 18.9, 22.8; 8 of 50 behind 300 16.2, 19.7, 16.3, 18.5; 900 36.0, 44.9,
+  // 34.5, 36.7; 1500 75, 89, 70, 57; 3413 329, 374, 282, 233; 2048 with heads 32 / 8 67, 74, 56, 69; 3413 with heads 8 / 1 74, 50, 68,
+  // 102.  (Before, with 16 rows a wave, a maximum a tile and two barriers: 19.9, 40.7, 24.0, 22.5, 52, 124, 427, 118, 127.)
+  // K8S_PREFILL_ATTN_WAVES 4, 8, 16: 64, 128, 256 rows
+  static const int env = [] { const char* e = getenv("K8S_PREFILL_ATTN_WAVES"); return e ? atoi(e) : 0; }();
+  auto wgs = [&](int rows) { return (long long)((max_qlen + rows / G - 1) / (rows / G)) * nkv * num_seqs; };
+  const int form = env == 4 || env == 8 || env == 16 ? env
+                   : wgs(256) > 256                        ? 16
+                   : wgs(64) > 512                         ? 8
+                   : wgs(64) > 256 && max_qlen <= 1024     ? 4
+                                                           : 5;
+#define PF(GG, RB, NW, KS)                                                                                   \
   {                                                                                                          \
-    constexpr int QT = 16 * NWW / GG;                                                                        \
-    dim3 grid((max_qlen + QT - 1) / QT, nkv, num_seqs);                                                      \
-    paged_prefill_kernel<128, GG, NWW><<<grid, 64 * NWW, 0, stream>>>(                                       \
+    constexpr int QT = 16 * RB * NW / KS / GG;                                                               \
+    const int tiles = (max_qlen + QT - 1) / QT;                                                              \
+    paged_prefill_kernel<GG, RB, NW, KS><<<dim3(tiles * nkv, 1, num_seqs), 64 * NW, 0, stream>>>(            \
         (bf16_t*)out, (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, cu_q, context_lens,  \
-        block_tables, sl2, nq, nkv, block_size, max_blocks);                                                 \
+        block_tables, sl2, nq, nkv, block_size, max_blocks, tiles);                                          \
   }
-#define PFW(GG) \
-  if (nw == 16) PF(GG, 16) else if (nw == 8) PF(GG, 8) else PF(GG, 4)
+#define PFR(GG) \
+  if (form == 16) PF(GG, 2, 8, 1) else if (form == 8) PF(GG, 2, 8, 2) else if (form == 4) PF(GG, 1, 4, 1) else PF(GG, 1, 8, 2)
   switch (G) {  // query heads per kv head (Llama-3.3-70B: 8; Llama-3-8B: 4)
-    case 1: PFW(1) break;
-    case 2: PFW(2) break;
-    case 4: PFW(4) break;
-    case 8: PFW(8) break;
-    case 16: PFW(16) break;
+    case 1: PFR(1) break;
+    case 2: PFR(2) break;
+    case 4: PFR(4) break;
+    case 8: PFR(8) break;
+    case 16: PFR(16) break;
     default: return -1;
   }
-#undef PFW
+#undef PFR
 #undef PF
   return (int)hipGetLastError();
 }
