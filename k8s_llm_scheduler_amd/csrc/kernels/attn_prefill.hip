@@ -11,21 +11,23 @@
 //
 // Structure:
 //  * "swapped" QK^T: S^T = K . Q^T with v_mfma_f32_16x16x32_bf16, so each lane ends up holding 16 scores of ONE query row (row =
-//    lane & 15) and the probabilities feed the P.V MFMA as its A operand straight from registers (the key order inside a 32-key
-//    step is permuted identically on the V side, see below).
+//    lane & 15) and the probabilities feed the P.V MFMA as its B operand straight from registers (the key order inside a 32-key
+//    step is permuted identically on the V side, see below), whose result O^T has a query row in the same lanes.
 //  * V tiles (64 keys x 128 d) are staged in LDS with an XOR swizzle and read with the gfx950 transposing read
-//    ds_read_b64_tr_b16, which delivers 4 keys of one d column per lane -- exactly the B-operand layout.
+//    ds_read_b64_tr_b16, which delivers 4 keys of one d column per lane -- exactly the A-operand layout.
 //  * K and V go through registers into two swizzled LDS images each: the tile after next is on its way, the next one is written,
 //    one barrier a tile that waits for LDS only.
 //  * 32 rows a wave (RB 2) read each K and V fragment for two products: at 16 rows a wave's LDS reads take twice the time of its
 //    products.
-//  * softmax in the log2 domain without a running maximum: the weights are 2^(score - m) with an m that is brought up to date (and
-//    the sums with it) only for a row's first tile and when the weights outgrow 2^12, so a tile costs one fma, power and addition a
-//    score; masks only where a tile crosses the wave's diagonal.
+//  * online softmax in the log2 domain: one fma (scale and maximum), maximum, power and addition a score; the lanes of a row meet,
+//    and the sums are rescaled, only in tiles where a row of the block has outgrown its maximum; masks only where a tile crosses
+//    the wave's diagonal.  (A reference up to 2^12 below the maximum would spare most of the rest; the largest weight, 1 here, would
+//    then be rounded to bf16: 3 - 8 % more error against 64 bits.)
 //  * longest workgroups first, so that the last round is of short ones.
 // What bounds it now: two waves a SIMD, in step between the barriers, each with its products, LDS reads and softmax in turn; at
-// long prompts 42 % of the matrix cores' rate.  Tried: waves of a SIMD half a tile apart with two barriers a tile (251 us against
-// 230 at 3413 tokens), 128 rows of 4 waves (256 us).
+// long prompts 35 % of the matrix cores' rate.  Tried: waves of a SIMD half a tile apart with two barriers a tile (251 us against
+// 230 at 3413 tokens, without the running maximum), 128 rows of 4 waves (256 us), one branch for both blocks of rows (272 us
+// against 266).
 #include <cstdlib>
 
 #include "common.h"
@@ -37,6 +39,23 @@ namespace k8sllm {
 typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
 
 __device__ __forceinline__ int v_swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+
+// Over the four lanes that share a column of a 16 x 16 product (l, l ^ 16, l ^ 32, l ^ 48), in all of them, by register moves: odd rows of 16 lanes of one copy against
+// even ones of the other, then halves.  (In asm with its wait states: the builtins hand back the first of the two registers twice.)
+template <typename F>
+__device__ __forceinline__ float row_join(float v, F f) {
+  float x = v, y = v;
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+  x = y = f(x, y);
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+  return f(x, y);
+}
+__device__ __forceinline__ float row_max(float v) {
+  return row_join(v, [](float a, float b) { return fmaxf(a, b); });
+}
+__device__ __forceinline__ float row_sum(float v) {
+  return row_join(v, [](float a, float b) { return a + b; });
+}
 
 template <int G, int RB, int NW, int KS>
 __global__ void __launch_bounds__(64 * NW, 2) paged_prefill_kernel(
@@ -170,7 +189,7 @@ __global__ void __launch_bounds__(64 * NW, 2) paged_prefill_kernel(
   for (int b = 0; b < RB; ++b)
 #pragma unroll
     for (int n = 0; n < D / 16; ++n) o[b][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run[RB], l_run[RB];   // row li's maximum so far, log2 (or up to 8 less); this lane's share of its sum
+  float m_run[RB], l_run[RB];   // row li's maximum so far, log2; this lane's share of its sum
 #pragma unroll
   for (int b = 0; b < RB; ++b) m_run[b] = -INFINITY, l_run[b] = 0.f;
 
@@ -191,9 +210,8 @@ __global__ void __launch_bounds__(64 * NW, 2) paged_prefill_kernel(
       }
     }
   };
-  // lane holds S[row li][key kbase + 16m + 4g + i]; the weights are 2^(score - m) for an m near the row's maximum: a row's first tile
-  // brings it up to date, and later ones only if the row has outgrown it (a lane's weights of a tile sum past 2^12: none is larger)
-  auto weights = [&](int kbase, bool first) {
+  // lane holds S[row li][key kbase + 16m + 4g + i]
+  auto weights = [&](int kbase) {
     if (kbase + KT - 1 > wq0) {
 #pragma unroll
       for (int b = 0; b < RB; ++b)
@@ -203,62 +221,47 @@ __global__ void __launch_bounds__(64 * NW, 2) paged_prefill_kernel(
           for (int i = 0; i < 4; ++i)
             if (kbase + m * 16 + g * 4 + i > qpos[b]) sacc[b][m][i] = -INFINITY;
     }
-    f32x4 pw[RB][KT / 16];
-    float rs[RB];
-    auto power = [&]() {
-#pragma unroll
-      for (int b = 0; b < RB; ++b) {
-        const float m_use = m_run[b] == -INFINITY ? 0.f : m_run[b];
-        f32x4 r4 = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int m = 0; m < KT / 16; ++m)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            pw[b][m][i] = __builtin_amdgcn_exp2f(fmaf(sacc[b][m][i], scale, -m_use));
-            r4[i] += pw[b][m][i];
-          }
-        rs[b] = (r4[0] + r4[1]) + (r4[2] + r4[3]);
-      }
-    };
-    bool grow = first;
-    if (!first) {
-      power();
-#pragma unroll
-      for (int b = 0; b < RB; ++b) grow |= rs[b] > 4096.f || m_run[b] == -INFINITY;
-    }
-    if (__any(grow)) {
-#pragma unroll
-      for (int b = 0; b < RB; ++b) {
-        float v = -INFINITY;
-#pragma unroll
-        for (int m = 0; m < KT / 16; ++m)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) v = fmaxf(v, sacc[b][m][i] * scale);
-        v = fmaxf(v, __shfl_xor(v, 16, WAVE));
-        v = fmaxf(v, __shfl_xor(v, 32, WAVE));
-        const float m_new = fmaxf(m_run[b], v);
-        const float alpha = m_run[b] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[b] - m_new);
-        l_run[b] *= alpha;
-        m_run[b] = m_new;
-        // row 4g+i of O lives in lanes whose li == 4g+i for the stats
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float a = __shfl(alpha, g * 4 + i, WAVE);
-#pragma unroll
-          for (int n = 0; n < D / 16; ++n) o[b][n][i] *= a;
-        }
-      }
-      power();
-    }
-    // P as A operand: k-step st covers keys 32st..32st+31 in the permuted order
-    // slot j<4 -> key 32st + 4g + j ; slot j>=4 -> key 32st + 16 + 4g + (j-4)
 #pragma unroll
     for (int b = 0; b < RB; ++b) {
-      l_run[b] += rs[b];
+      // the scores against the maximum so far: only if one of the rows has outgrown it do the lanes meet for the new one
+      const float base = m_run[b] == -INFINITY ? 0.f : m_run[b];
+      float top[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
-      for (int st = 0; st < KT / 32; ++st)
+      for (int m = 0; m < KT / 16; ++m)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) pa[b][st][j] = (__bf16)pw[b][2 * st + (j >> 2)][j & 3];
+        for (int i = 0; i < 4; ++i) {
+          sacc[b][m][i] = fmaf(sacc[b][m][i], scale, -base);
+          top[i] = fmaxf(top[i], sacc[b][m][i]);
+        }
+      float over = fmaxf(fmaxf(top[0], top[1]), fmaxf(top[2], top[3]));
+      if (__any(over > 0.f || m_run[b] == -INFINITY)) {
+        over = row_max(over);
+        const float m_new = fmaxf(m_run[b], base + over);
+        const float alpha = m_run[b] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[b] - m_new);
+        const float d = m_new == -INFINITY ? 0.f : m_new - base;
+        l_run[b] *= alpha;
+        m_run[b] = m_new;
+#pragma unroll
+        for (int m = 0; m < KT / 16; ++m)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sacc[b][m][i] -= d;
+#pragma unroll
+        for (int n = 0; n < D / 16; ++n)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[b][n][i] *= alpha;
+      }
+      // P as B operand: k-step st covers keys 32st..32st+31 in the permuted order
+      // slot j<4 -> key 32st + 4g + j ; slot j>=4 -> key 32st + 16 + 4g + (j-4)
+      f32x4 rs = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int m = 0; m < KT / 16; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float w = __builtin_amdgcn_exp2f(sacc[b][m][i]);
+          rs[i] += w;
+          pa[b][m >> 1][4 * (m & 1) + i] = (__bf16)w;
+        }
+      l_run[b] += (rs[0] + rs[1]) + (rs[2] + rs[3]);
     }
   };
   auto values = [&](const char* vl) {
@@ -279,7 +282,7 @@ __global__ void __launch_bounds__(64 * NW, 2) paged_prefill_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) { vb[j] = v0[j]; vb[4 + j] = v1[j]; }
 #pragma unroll
-        for (int b = 0; b < RB; ++b) o[b][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa[b][st], vb, o[b][n], 0, 0, 0);
+        for (int b = 0; b < RB; ++b) o[b][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vb, pa[b][st], o[b][n], 0, 0, 0);
       }
     }
   };
@@ -307,7 +310,7 @@ __global__ void __launch_bounds__(64 * NW, 2) paged_prefill_kernel(
     const int kbase = t * ST + share * KT;
     if (kbase <= wq1) {
       scores(klds[t & 1] + share * (KT * D * 2));
-      weights(kbase, t == 0);
+      weights(kbase);
       values(vlds[t & 1] + share * (KT * D * 2));
     }
     lds_barrier();                   // tile t has been read and tile t + 1 written
@@ -316,8 +319,7 @@ __global__ void __launch_bounds__(64 * NW, 2) paged_prefill_kernel(
   float l_row[RB];                   // row li's sum
 #pragma unroll
   for (int b = 0; b < RB; ++b) {
-    l_row[b] = l_run[b] + __shfl_xor(l_run[b], 16, WAVE);
-    l_row[b] += __shfl_xor(l_row[b], 32, WAVE);
+    l_row[b] = row_sum(l_run[b]);
   }
   if constexpr (KS == 2) {           // the second share's sums join the first one's, through the staged K
     static_assert(RW * RB * (D / 16) * 64 * 16 <= 2 * ST * D * 2, "room for a share's sums");
@@ -345,29 +347,25 @@ __global__ void __launch_bounds__(64 * NW, 2) paged_prefill_kernel(
       const float a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - m);
       l_row[b] = l_row[b] * a0 + l1 * a1;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float c0 = __shfl(a0, g * 4 + i, WAVE), c1 = __shfl(a1, g * 4 + i, WAVE);
+      for (int n = 0; n < D / 16; ++n) {
+        const f32x4 o1 = os[((wid * RB + b) * (D / 16) + n) * 64 + lane];
 #pragma unroll
-        for (int n = 0; n < D / 16; ++n)
-          o[b][n][i] = o[b][n][i] * c0 + os[((wid * RB + b) * (D / 16) + n) * 64 + lane][i] * c1;
+        for (int i = 0; i < 4; ++i) o[b][n][i] = o[b][n][i] * a0 + o1[i] * a1;
       }
     }
   }
 
-  // ---- normalise and store: o[b][n][i] = O[row 4g+i][d 16n + li]
+  // ---- normalise and store: o[b][n][i] = O[row li][d 16n + 4g + i]
 #pragma unroll
   for (int b = 0; b < RB; ++b) {
+    const float inv_l = l_row[b] > 0.f ? 1.f / l_row[b] : l_row[b] == 0.f ? 0.f : l_row[b];   // (NaN stays one)
+    const int orow = (wid * RB + b) * 16 + li;
+    const int r = tile * QT + orow / G, oh = kvh * G + orow % G;
+    if (r < qlen) {
+      bf16_t* op = out + ((size_t)(q0 + r) * nq + oh) * D + 4 * g;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float lv = __shfl(l_row[b], g * 4 + i, WAVE);
-      const float inv_l = lv > 0.f ? 1.f / lv : lv == 0.f ? 0.f : lv;   // (NaN stays one)
-      const int orow = (wid * RB + b) * 16 + g * 4 + i;
-      const int r = tile * QT + orow / G, oh = kvh * G + orow % G;
-      if (r < qlen) {
-        bf16_t* op = out + ((size_t)(q0 + r) * nq + oh) * D + li;
-#pragma unroll
-        for (int n = 0; n < D / 16; ++n) op[16 * n] = f2bf(o[b][n][i] * inv_l);
-      }
+      for (int n = 0; n < D / 16; ++n)
+        stf4(op + 16 * n, f32x4{o[b][n][0] * inv_l, o[b][n][1] * inv_l, o[b][n][2] * inv_l, o[b][n][3] * inv_l});
     }
   }
 }
@@ -383,16 +381,16 @@ extern "C" int k8s_paged_prefill_attention(void* out, const void* q, const void*
                                            float scale, int num_seqs, int max_qlen, int nq, int nkv, int D,
                                            int block_size, int max_blocks, hipStream_t stream) {
   if (num_seqs <= 0 || max_qlen <= 0) return 0;
-  if (D != 128 || nq % nkv != 0) return -1;
+  if (D != 128 || nq % nkv != 0 || (uintptr_t)out % 8) return -1;
   const int G = nq / nkv;
   const float sl2 = scale * 1.4426950408889634f;
   // Rows of a workgroup and shares of the keys.  Few workgroups: 64 rows, the keys shared by two halves of 8 waves (one workgroup a CU);
   // up to two a CU of 4 waves, unless the prompt is long and the longest of them decides; from about one workgroup of 256 rows a CU
   // those, which read each key and value byte a quarter as often; between, 128 rows with shared keys.  us of 64 rows, 64 shared, 128
-  // shared, 256, heads 64 / 8 unless said: 241 tokens behind 224 14.9, 12.6, 17.3,
-  // 21.5; 97 behind 1000 27.3, 20.4, 28.2, 39.6; 512 17.2, 19.0, 18.9, 22.8; 8 of 50 behind 300 16.2, 19.7, 16.3, 18.5; 900 36.0, 44.9,
-  // 34.5, 36.7; 1500 75, 89, 70, 57; 3413 329, 374, 282, 233; 2048 with heads 32 / 8 67, 74, 56, 69; 3413 with heads 8 / 1 74, 50, 68,
-  // 102.  (Before, with 16 rows a wave, a maximum a tile and two barriers: 19.9, 40.7, 24.0, 22.5, 52, 124, 427, 118, 127.)
+  // shared, 256, heads 64 / 8 unless said: 241 tokens behind 224 15.8, 13.2, 19.5,
+  // 24.6; 97 behind 1000 28.2, 21.5, 33.2, 47.3; 512 17.8, 19.9, 21.3, 27.7; 8 of 50 behind 300 16.8, 20.5, 17.7, 22.3; 900 38.1, 46.7,
+  // 39.7, 43.2; 1500 78, 95, 85, 68; 3413 346, 407, 335, 266; 2048 with heads 32 / 8 72, 79, 68, 81; 3413 with heads 8 / 1 76, 53, 83,
+  // 117.  (Before, with 16 rows a wave and two barriers a tile: 20.1, 41.0, 25.1, 22.6, 54, 127, 443, 120, 128.)
   // K8S_PREFILL_ATTN_WAVES 4, 8, 16: 64, 128, 256 rows
   static const int env = [] { const char* e = getenv("K8S_PREFILL_ATTN_WAVES"); return e ? atoi(e) : 0; }();
   auto wgs = [&](int rows) { return (long long)((max_qlen + rows / G - 1) / (rows / G)) * nkv * num_seqs; };
