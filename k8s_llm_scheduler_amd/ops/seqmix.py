@@ -282,7 +282,10 @@ def act(x: torch.Tensor, kind: int, limit: float = 0.0, alpha: float = 1.0, *,
 def _route_fast(a: torch.Tensor, w: torch.Tensor, out_dtype) -> bool:
     """bf16 products of production size whose shape the framework's tuned GEMV / MFMA GEMM kernels take (128-byte
     k steps, N % 16 == 0, at least 1024 x 512 weights: the sizes their plan tables and heuristics were tuned and
-    tested on).  Smaller products are launch-bound and stay on the any-shape kernel."""
+    tested on).  Smaller products are launch-bound and stay on the any-shape kernel, but of half that size those with rows enough to
+    fill it or with a depth that its few tiles walk alone: us, any-shape / tuned, M x N x K in bf16 and (N >= K) fp32: 512 x 2048 x 128
+    5.4 / 4.4, 2048 12.9 / 7.4; 512 x 512 x 512 5.2 / 4.9, 2048 9.0 / 4.7; 2048 x 256 x 1024 12.8 / 6.2; x 128 x 2048 33 rows 7.0 /
+    5.6, 64 10.0 / 5.6, 200 11.4 / 7.5, 2048 14.5 / 9.4.  200 x 1024 x 256 and x 512 x 512 in fp32 are 4 - 10 % slower there."""
     if _ops.LEAN:
         return False
     if a.dtype != BF16 or w.dtype != BF16 or out_dtype not in (BF16, F32) or a.dim() != 2 or w.dim() != 2:
@@ -290,7 +293,9 @@ def _route_fast(a: torch.Tensor, w: torch.Tensor, out_dtype) -> bool:
     if _ops.GEMM_BACKEND == "library" or not a.is_contiguous() or not w.is_contiguous():
         return False
     N, K = w.shape
-    return a.shape[1] == K and K % 64 == 0 and N % 16 == 0 and K * N >= 512 * 1024 and K >= 128 and N >= 128
+    M, size = a.shape[0], K * N
+    return a.shape[1] == K and K % 64 == 0 and N % 16 == 0 and K >= 128 and N >= 128 and \
+        (size >= 512 * 1024 or (size >= 256 * 1024 and (M >= 512 or (K >= 1024 and M > 128) or (K >= 2048 and M >= 33))))
 
 
 # route fitting bf16 shapes to ops.linear (K8S_SEQMIX_FAST_GEMM=0: every product on the any-shape kernel)
