@@ -407,10 +407,17 @@ _GROUP_COST = {1: (0.0, 0.632, 2.7, 0.0, 0.0957, 0.701, 3.45), 2: (1.58, 0.488, 
 @functools.lru_cache(maxsize=4096)
 def _grouped_tile(rows: int, E: int, N: int, K: int, pair: bool, even: bool = False, common: int = 0) -> int:
     """Configuration of the grouped big-tile product: the cheapest of them all by _GROUP_COST, for groups of the same size (``even``)
-    or of about equal size drawn at random beside ``common`` rows that are the last group's, whose tiles are expected ones: up to 5 that would begin another round most often are
-    not there (1700 rows of 16 experts, 2 x 2048 x 4096: 260.5 tiles expected, 136 us in one round, 152 the next best)."""
+    or of about equal size drawn at random beside ``common`` rows that are the last group's, whose tiles are expected ones: up to 5 that
+    would begin another round most often are not there (1700 rows of 16 experts, 2 x 2048 x 4096: 260.5 tiles expected, 136 us in one
+    round, 152 the next best).  With three rows a group or fewer there are groups without any, and what is left is a stream of weights
+    that the smallest tiles, two of them on a CU, keep up best, of wide groups the next ones: us, 64 x 64 / 128 x 64 tiles, 8 groups
+    beside a common one, 0.5 / 1 / 2 rows each: 2048 x 2048 12.2 / 19.1, 14.7 / 20.2, 16.3 / 20.8; 4096 x 3584 24.8 / 32.0, 42.3 / 43.1,
+    47.2 / 48.1; gated 2 x 2048 x 2048 15.5 / 19.0, 25.6 / 26.0, 27.7 / 29.2; 2 x 3584 x 4096 48.4 / 48.1, 86.2 / 81.3, 89.4 / 86.9 (256 x
+    128: 65.5, 82.2, 90.7)."""
     drawn = E - (common > 0)
     r, n, kt, best = (rows - common) / max(drawn, 1), (2 * N if pair else N), K / 64, None
+    if rows <= 3 * E and E > 1 and not even:
+        return 6 if n <= 4096 else 5
     for cfg, (t0, tile, rnd, step, wmb, omb, act_us) in _GROUP_COST.items():
         bp, bq = _GROUP_TILE[cfg]
         if even or E == 1:

@@ -13,3 +13,9 @@ def test_rule(M, N, K, fast):
     a, w = torch.empty(M, K, dtype=torch.bfloat16), torch.empty(N, K, dtype=torch.bfloat16)
     assert sm._route_fast(a, w, torch.bfloat16) == fast and sm._route_fast(a, w, torch.float32) == fast
     assert not sm._route_fast(a.float(), w.float(), torch.float32)
+
+
+@pytest.mark.parametrize("rows,N,pair,even,want", [(27, 2048, False, False, 6), (6, 2048, True, False, 6), (6, 2052, True, False, 5),
+                                                   (27, 4100, False, False, 5), (28, 2048, False, False, 5), (27, 2048, False, True, 5)])
+def test_grouped_tiles_of_few_rows(rows, N, pair, even, want):
+    assert sm._grouped_tile(rows, 9, N, 2048, pair, even, rows // 3) == want
