@@ -40,7 +40,8 @@
 // the clock that the power allows (1.7 - 2.0 GHz in long launches; operands all zero take 25 % less time): 89 % of a stage's
 // cycles are the matrix cores', and at K = 2048 a fifth of the launch is its start, first loads and stores.  The 256 x 256 tiles
 // take all 512 registers, and by the compiler's report spill 16 - 38 of them between the k loop and the rows in LDS (bf16 20,
-// SwiGLU 31, fp32 output 0, with the RMS prologue 28, 24 and 12; the gated kinds 31 - 38, relu^2 16), none of it inside the loop.
+// SwiGLU 31, fp32 output 0, with the RMS prologue 28, 24 and 12, with row scales 20 and 32; the gated kinds 26 - 38, relu^2 16), none
+// of it inside the loop.
 #include <type_traits>
 
 #include "act.h"
@@ -97,8 +98,9 @@ struct P4Args {
   float last_limit;      // grouped form: the limit of the last group
   const bf16_t* bias;    // P4_GLU, optional: [gate; up] biases
   // grouped form: group g's rows are [seg[g], seg[g + 1]) of a compact row space (row r of x: a_rows[r], or r) and its
-  // weights W + g wstride bytes; m_tiles bounds the groups' row tiles.  8 experts, 3068 rows, K = 2048, in a step: gate / up
-  // with its activation (N = 2 x 2048) 69 us, down (N = 2048) 34 us; 140 and 10 us, and 78 us on the 64-row tiles of stream32.hip.
+  // weights W + g wstride bytes; m_tiles bounds the groups' row tiles.  8 experts, 3068 rows, K = 2048, in a step, as it was
+  // brought here: gate / up with its activation (N = 2 x 2048) 69 us, down (N = 2048) 34 us; on the 64-row tiles of stream32.hip 140 and
+  // 10 us, and 78 us.
   // spread with 8 groups and more, an XCD's tiles then another group's, of up to 192 rows: gate / up of 8 experts, 4 - 192 rows
   // each 29.4 -> 27.8 us (64 x 64), 16 of 2 x 2048 x 4096 139 -> 108 (256 x 128); 4 groups 30.0 -> 34.0, 320 rows 70 -> 71.
   // seg == nullptr: groups of gsize rows (products of several inputs with a weight each in one launch)

@@ -1009,8 +1009,9 @@ def _pg_load_table() -> dict:
 # hide part from each other; with split-K the combine launch and the slabs it moves; the weights and the output.  Fitted to 22
 # weight shapes (576 x 2048 .. 28672 x 4096) at 12 row counts (130 .. 2048), weights cold: rms error 5 - 10 % per configuration,
 # the pick within 1 % of the best plan on average and 18 % at most, 6 % faster on average than the rule for the six tiles there
-# were (64 x 64 then two stages ahead), 7 % slower at most (256 x 6144 x 3072) but for 14 % at 256 x 2048 x 8192.  pgemm.hip's 8-wave tiles were the best plan of none of these; the tuned table names them for some of the 70B's
-# products of 256 - 8192 rows and its logits, and SwiGLU and fp8 products that it does not list take them (_pgemm_big_tiles).
+# were (64 x 64 then two stages ahead), 7 % slower at most (256 x 6144 x 3072) but for 14 % at 256 x 2048 x 8192.  pgemm.hip's
+# 8-wave tiles were the best plan of none of these; the tuned table names them for some of the 70B's products of 256 - 8192
+# rows and its logits, and SwiGLU and fp8 products that it does not list take them (_pgemm_big_tiles).
 _P4_COST = {1: (0.652, 2.2, 0.0, 5.33, 0.24, 0.066, 0.305),
             2: (0.652, 2.3, 0.0, 4.98, 0.273, 0.0316, 0.345),
             3: (0.299, 0.0, 0.148, 4.36, 0.307, 0.0852, 0.37),
