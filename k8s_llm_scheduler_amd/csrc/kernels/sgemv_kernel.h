@@ -374,7 +374,8 @@ __global__ void __launch_bounds__(512) smfma_kernel(void* __restrict__ out, floa
   // ---- x -> registers: xr[s][xg] = x[4 xg + r4][chunk 16 (sb + s) + cb]; rows >= M / dead steps read 0
   u32x4 xr[JT][XG][XV];
   {
-    const auto xs = sg_rsrc(x + (ROWS == 3 ? (size_t)(b0 / rows.count) * M * K : 0), (long long)M * K * 2);
+    // (ROWS 3: all bands past n1 are the last input's, which may have more rows of W than the others)
+    const auto xs = sg_rsrc(x + (ROWS == 3 ? (size_t)(min(b0, rows.n1) / rows.count) * M * K : 0), (long long)M * K * 2);
 #pragma unroll
     for (int s = 0; s < JT; ++s)
 #pragma unroll

@@ -130,7 +130,8 @@ def test_norm_shift(dt, W, T, n, branch, rowvec, entries):
 
 
 @pytest.mark.parametrize("M", [1, 3, 8, 9, 16, 17])
-@pytest.mark.parametrize("N,L,K", [(2048, 128, 2048), (8, 8, 128), (24, 1, 1152), (4096, 256, 4096), (2040, 127, 1024), (20, 4, 256)])
+@pytest.mark.parametrize("N,L,K", [(2048, 128, 2048), (8, 8, 128), (24, 1, 1152), (4096, 256, 4096), (2040, 127, 1024), (20, 4, 256),
+                                   (8, 9, 128), (8, 24, 128), (64, 300, 256), (16, 2048, 1024)])
 def test_several_inputs(M, N, L, K, entries):
     r = data(M + N + L)
     a, w = r(5, M, K), r(4 * N + L, K, m=K ** -0.5)
