@@ -380,7 +380,7 @@ class PutulornModel(StreamModel):
                 if m.rot_dims > m.rot_dim or m.rot_dims % 2:
                     raise ValueError(f"layer {i}: rot.dims {m.rot_dims} must be even and at most rot_dim {m.rot_dim}")
                 q, dkv, qdkv = t(get(p + "q")), t(get(p + "dkv")), None
-                if sm.rows_join(1, W) and self.dtype == torch.bfloat16:
+                if self.dtype == torch.bfloat16 and W % 128 == 0:     # (whatever the switches say now: rows_join's widths are among them)
                     qdkv = torch.cat([q, dkv])
                     q, dkv = qdkv[:q.shape[0]], qdkv[q.shape[0]:]
                 mixer = _Latent(m, q, dkv, t(get(p + "dkv.norm")),

@@ -464,3 +464,19 @@ def test_random_configurations(tmp_path, device, seed):
         ga.append(rows[:1])
     assert rel_err(torch.cat(ga), wa) < TOL["float32"], cfg
     assert rel_err(torch.cat(gb), wb) < TOL["float32"], cfg
+
+
+@pytest.mark.parametrize("device", DEVICES)
+def test_switches_set_after_the_weights_were_laid_out(tmp_path, device, monkeypatch):
+    """A model loaded while the tuned kernels were switched off decodes as one loaded with them on."""
+    from k8s_llm_scheduler_amd.ops import seqmix as sm
+
+    cfg = config([with_mlp(wkv(), dense()), with_mlp(latent(), dense())], width=128)
+    monkeypatch.setattr(sm, "FAST_GEMM", False)
+    off, _ = make(tmp_path, cfg, device, "bfloat16")
+    monkeypatch.setattr(sm, "FAST_GEMM", True)
+    on, _ = make(tmp_path, cfg, device, "bfloat16")
+    toks = tokens(12, 90, 1)
+    assert torch.equal(whole(off, "s", toks), whole(on, "s", toks))
+    for t in (5, 17, 3):                      # a prompt of one token, then decoding
+        assert torch.equal(off.replay_step([("r", [t], [0])]), on.replay_step([("r", [t], [0])]))
