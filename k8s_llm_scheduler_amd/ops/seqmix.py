@@ -279,6 +279,9 @@ def act(x: torch.Tensor, kind: int, limit: float = 0.0, alpha: float = 1.0, *,
     return out
 
 
+FAST_WEIGHTS = 512 * 1024        # weights from which on a bf16 product goes to the tuned kernels with any number of rows
+
+
 def _route_fast(a: torch.Tensor, w: torch.Tensor, out_dtype) -> bool:
     """bf16 products of production size whose shape the framework's tuned GEMV / MFMA GEMM kernels take (128-byte
     k steps, N % 16 == 0, at least 1024 x 512 weights: the sizes their plan tables and heuristics were tuned and
@@ -295,7 +298,7 @@ def _route_fast(a: torch.Tensor, w: torch.Tensor, out_dtype) -> bool:
     N, K = w.shape
     M, size = a.shape[0], K * N
     return a.shape[1] == K and K % 64 == 0 and N % 16 == 0 and K >= 128 and N >= 128 and \
-        (size >= 512 * 1024 or (size >= 256 * 1024 and (M >= 512 or (K >= 1024 and M > 128) or (K >= 2048 and M >= 33))))
+        (size >= FAST_WEIGHTS or (2 * size >= FAST_WEIGHTS and (M >= 512 or (K >= 1024 and M > 128) or (K >= 2048 and M >= 33))))
 
 
 # route fitting bf16 shapes to ops.linear (K8S_SEQMIX_FAST_GEMM=0: every product on the any-shape kernel)
@@ -547,10 +550,13 @@ def linear_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, 
             _native().pgemm4_act(out.data_ptr(), _p(a), _p(w), M, N, K, plan[0], plan[2], kind, float(limit), float(alpha),
                                  _p(bias), -1)
             return out
-    elif bias is None and not pair and kind != ACT_SOFTCAP and a.dim() == w.dim() == 2 and a.shape[0] > 0 and \
+    # few tiles: gemm() would take that kernel, or of 256 - 512 Ki weights a tuned one, whose sums an activation of its own would take
+    # rounded to bf16: of these one launch and one rounding too, faster or not (us, one launch / the tuned product and tanh, M x N x K: 64 x
+    # 128 x 2048 11.9 / 7.6, 333 11.9 / 10.9, 2048 15.0 / 12.1, 4096 25.2 / 12.7; 333 x 256 x 1024 7.7 / 8.8; 512 x 512 x 512 5.7 / 8.3)
+    if bias is None and not pair and kind != ACT_SOFTCAP and a.dim() == w.dim() == 2 and a.shape[0] > 0 and \
             -(-a.shape[0] // 64) * (-(-w.shape[0] // 64)) <= 128 and _few_fits(a, w) and \
-            not (FAST_GEMM and _route_fast(a, w, BF16)):
-        out = torch.empty(a.shape[0], w.shape[0], dtype=BF16, device=a.device)     # few tiles: gemm() would take that kernel
+            (w.numel() < FAST_WEIGHTS or not (FAST_GEMM and _route_fast(a, w, BF16))):
+        out = torch.empty(a.shape[0], w.shape[0], dtype=BF16, device=a.device)
         _native().gemm_few_act(out.data_ptr(), a.data_ptr(), w.data_ptr(), a.shape[0], w.shape[0], w.shape[1], a.stride(0), 0, 0,
                                0, kind, float(limit), float(alpha), -1)
         return out
