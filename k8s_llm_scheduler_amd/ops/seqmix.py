@@ -514,9 +514,10 @@ def gemm_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, al
             _grouped_big(a, w, seg, rows, N):
         return _pgemm4_grouped(a, w, a_rows, rows, seg, N, kind, limit, alpha, common, common_limit if own else None)
     if tiles is not None and w.dim() == 3 and kind in (ACT_GELU_TANH, ACT_SWISH_CLAMP, ACT_RELU) and 0 < rows <= 512 and \
-            rows <= 32 * tiles.shape[0] and (rows >= 6 * E or own or w.shape[1] * w.shape[2] <= 1 << 22) and \
+            rows <= 32 * tiles.shape[0] and (rows >= 6 * E or common > 0 or w.shape[1] * w.shape[2] <= 1 << 22) and \
             w.shape[1] % 2 == 0 and a.dim() == 2 and _few_fits(a, w):
-        # (16 experts of 2 x 2048 x 4096: 8 rows 53 / 56 us, 64 rows 102 / 102 us, 96 rows 109 / 105 us)
+        # (16 experts of 2 x 2048 x 4096: 8 rows 53 / 56 us, 64 rows 102 / 102 us, 96 rows 109 / 105 us; with a common expert always, whose
+        # product alone, linear_act of as many rows, does not round its sums either)
         out = torch.empty(rows, N, dtype=BF16, device=a.device)
         _native().gemm_few_act(out.data_ptr(), a.data_ptr(), w.data_ptr(), rows, N, w.shape[2], a.stride(0),
                                _p(a_rows, I32, "a_rows"), _p(tiles, I32, "tiles"), tiles.shape[0], kind, float(limit),

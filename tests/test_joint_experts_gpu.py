@@ -45,14 +45,43 @@ def test_limit_of_the_last_group(T, path, limits, E, top, monkeypatch):
     monkeypatch.setattr(ops, "native", Spy)
     got = sm.gemm_act(h, w, sm.ACT_SWISH_CLAMP, limits[0], 1.702, a_rows=tok, tiles=tiles, rows=T * (top + 1), seg=seg, common=T,
                       common_limit=limits[1])
-    if path != "plain" and (path == "big" or limits[0] != limits[1]):
+    if path != "plain":
         assert names == ["pgemm4_grouped" if path == "big" else "gemm_few_act"]
-    slack = 2.0 ** -8 if path == "big" or (path == "few" and limits[0] != limits[1]) else 2.0 ** -6
+    slack = 2.0 ** -8 if path != "plain" else 2.0 ** -6
     got = got.double()[pos.long()].view(T, top + 1, F)
     for c in range(top + 1):
         z = (h.double().unsqueeze(1) @ w.double()[idx[:, c].long()].transpose(1, 2)).squeeze(1)
         want = glu64(z, limits[1] if c == top else limits[0])
         assert ((got[:, c] - want).abs() <= slack * want.abs() + (1e-4 if slack < 2.0 ** -7 else 4e-2)).all(), c
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 2, 5])
+@pytest.mark.parametrize("limits", [(1.0, 1.0), (0.0, 0.7)])
+def test_large_weights_of_few_tokens(T, limits, monkeypatch):
+    """More than 4 Mi values an expert and fewer rows than the big tiles take: one launch, the sums not rounded ahead of the activation."""
+    W, F, E, top = 1536, 1408, 8, 2
+    g = torch.Generator().manual_seed(T)
+    h = torch.randn(T, W, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(E + 1, 2 * F, W, generator=g) * 2 / W ** 0.5).to(torch.bfloat16).to(DEV)
+    idx = torch.cat([torch.rand(T, E, generator=g).argsort(1)[:, :top], torch.full((T, 1), E)], 1).to(torch.int32).to(DEV)
+    tok, pos, seg, tiles = sm.moe_align(idx, E + 1)
+    names, nat = [], ops.native()
+
+    class Spy:
+        def __getattr__(self, name):
+            names.append(name)
+            return getattr(nat, name)
+
+    monkeypatch.setattr(ops, "native", Spy)
+    got = sm.gemm_act(h, w, sm.ACT_SWISH_CLAMP, limits[0], 1.702, a_rows=tok, tiles=tiles, rows=T * (top + 1), seg=seg, common=T,
+                      common_limit=limits[1])
+    assert names == ["gemm_few_act"]
+    got = got.double()[pos.long()].view(T, top + 1, F)
+    for c in range(top + 1):
+        z = torch.stack([h[t].double() @ w[int(idx[t, c])].double().T for t in range(T)])
+        want = glu64(z, limits[1] if c == top else limits[0])
+        assert ((got[:, c] - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all(), c
 
 
 def model(dev, dtype, shared_ff, tokens=None):
