@@ -964,7 +964,8 @@ def pgemm4(x: torch.Tensor, w: torch.Tensor, epi: int = EPI_BF16, cfg: int = 0, 
     rp = _chk(res, BF16, "res") if res is not None else 0
     rms, eps = (1, float(rms_eps)) if rms_eps is not None else (0, 0.0)
     sp = slab.data_ptr() if slab is not None else 0
-    if rms and 2.0 * M * w.shape[0] * K >= P4_SCALE_FLOPS and epi != EPI_F32 and native().pgemm4_scaled_ok(cfg):
+    if rms and 2.0 * M * w.shape[0] * K >= P4_SCALE_FLOPS and epi != EPI_F32 and x.data_ptr() % 16 == 0 and \
+            native().pgemm4_scaled_ok(cfg):
         scale = torch.empty(M, dtype=F32, device=x.device)
         native().pgemm4_scaled(out.data_ptr(), sp, _chk(x, BF16, "x"), _chk(w, BF16, "w"), M, N, K, epi, cfg, splits, group_m,
                                rp, scale.data_ptr(), eps, -1)
