@@ -35,7 +35,7 @@ int k8s_paged_decode_attention(void* out, void* part_acc, void* part_ml, const v
                                hipStream_t s);
 int k8s_paged_prefill_attention(void* out, const void* q, const void* k_cache, const void* v_cache, const int* cu_q,
                                 const int* context_lens, const int* block_tables, float scale, int num_seqs,
-                                int max_qlen, int nq, int nkv, int D, int block_size, int max_blocks, hipStream_t s);
+                                int max_qlen, int nq, int nkv, int D, int block_size, int max_blocks, int form, hipStream_t s);
 void k8s_gemv_plan(int M, int N_out, int K, int epi, int mode, int* ks_out, int* splits_out);
 int k8s_sgemv(void* out, void* partial, const void* x, const void* W, const float* wscale, const void* res, int M,
               int N, int K, int epi, int norm, float eps, hipStream_t s);
@@ -353,9 +353,9 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
   });
   m.def("paged_prefill_attention", [](uintptr_t out, uintptr_t q, uintptr_t kc, uintptr_t vc, uintptr_t cu_q,
                                       uintptr_t ctx, uintptr_t bt, float scale, int nseq, int max_qlen, int nq,
-                                      int nkv, int D, int bs, int max_blocks, int64_t s) {
+                                      int nkv, int D, int bs, int max_blocks, int form, int64_t s) {
     check(k8s_paged_prefill_attention(P(out), P(q), P(kc), P(vc), P<int>(cu_q), P<int>(ctx), P<int>(bt), scale, nseq,
-                                      max_qlen, nq, nkv, D, bs, max_blocks, S(s)),
+                                      max_qlen, nq, nkv, D, bs, max_blocks, form, S(s)),
           "paged_prefill_attention");
   });
 #endif

@@ -28,8 +28,6 @@
 // long prompts 35 % of the matrix cores' rate.  Tried: waves of a SIMD half a tile apart with two barriers a tile (251 us against
 // 230 at 3413 tokens, without the running maximum), 128 rows of 4 waves (256 us), one branch for both blocks of rows (272 us
 // against 266).
-#include <cstdlib>
-
 #include "common.h"
 
 #define K8S_CHK_THIS_UNIT 5
@@ -376,29 +374,15 @@ using namespace k8sllm;
 
 K8S_CHECK_UNIT(attn_prefill)
 
+// form 4: 64 rows a workgroup; 5: 64, the keys shared by two halves of 8 waves; 8: 128, shared; 16: 256 (which when: ops/__init__.py _prefill_form)
 extern "C" int k8s_paged_prefill_attention(void* out, const void* q, const void* k_cache, const void* v_cache,
                                            const int* cu_q, const int* context_lens, const int* block_tables,
                                            float scale, int num_seqs, int max_qlen, int nq, int nkv, int D,
-                                           int block_size, int max_blocks, hipStream_t stream) {
+                                           int block_size, int max_blocks, int form, hipStream_t stream) {
   if (num_seqs <= 0 || max_qlen <= 0) return 0;
-  if (D != 128 || nq % nkv != 0 || (uintptr_t)out % 8) return -1;
+  if (D != 128 || nq % nkv != 0 || (uintptr_t)out % 8 || (form != 4 && form != 5 && form != 8 && form != 16)) return -1;
   const int G = nq / nkv;
   const float sl2 = scale * 1.4426950408889634f;
-  // Rows of a workgroup and shares of the keys.  Few workgroups: 64 rows, the keys shared by two halves of 8 waves (one workgroup a CU);
-  // up to two a CU of 4 waves, unless the prompt is long and the longest of them decides; from about one workgroup of 256 rows a CU
-  // those, which read each key and value byte a quarter as often; between, 128 rows with shared keys.  us of 64 rows, 64 shared, 128
-  // shared, 256, heads 64 / 8 unless said: 241 tokens behind 224 15.8, 13.2, 19.5,
-  // 24.6; 97 behind 1000 28.2, 21.5, 33.2, 47.3; 512 17.8, 19.9, 21.3, 27.7; 8 of 50 behind 300 16.8, 20.5, 17.7, 22.3; 900 38.1, 46.7,
-  // 39.7, 43.2; 1500 78, 95, 85, 68; 3413 346, 407, 335, 266; 2048 with heads 32 / 8 72, 79, 68, 81; 3413 with heads 8 / 1 76, 53, 83,
-  // 117.  (Before, with 16 rows a wave and two barriers a tile: 20.1, 41.0, 25.1, 22.6, 54, 127, 443, 120, 128.)
-  // K8S_PREFILL_ATTN_WAVES 4, 8, 16: 64, 128, 256 rows
-  static const int env = [] { const char* e = getenv("K8S_PREFILL_ATTN_WAVES"); return e ? atoi(e) : 0; }();
-  auto wgs = [&](int rows) { return (long long)((max_qlen + rows / G - 1) / (rows / G)) * nkv * num_seqs; };
-  const int form = env == 4 || env == 8 || env == 16 ? env
-                   : wgs(256) > 256                        ? 16
-                   : wgs(64) > 512                         ? 8
-                   : wgs(64) > 256 && max_qlen <= 1024     ? 4
-                                                           : 5;
 #define PF(GG, RB, NW, KS)                                                                                   \
   {                                                                                                          \
     constexpr int QT = 16 * RB * NW / KS / GG;                                                               \

@@ -383,6 +383,41 @@ def paged_decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
     return out
 
 
+# K8S_PREFILL_ATTN_WAVES = 4, 8, 16: always 64, 128 (keys shared), 256 rows a workgroup
+PREFILL_ATTN_FORM = {"4": 4, "8": 8, "16": 16}.get(os.environ.get("K8S_PREFILL_ATTN_WAVES", "").strip(), 0)
+
+
+@functools.lru_cache(maxsize=4096)
+def _prefill_form(T: int, max_qlen: int, num_seqs: int, nq: int, nkv: int) -> int:
+    """Rows of a workgroup of the paged prompt attention and shares of its keys (attn_prefill.hip): 4: 64 rows, 5: 64 with the keys shared
+    by two halves of 8 waves (one workgroup a CU), 8: 128 shared, 16: 256, which read each key and value byte a quarter as often.  By
+    the workgroups that find a query of the batch, of T tokens: a sequence has at most one that is not full, and those past a sequence's end
+    return at once, but hold a place on a CU for a moment.  256 rows from about one workgroup a CU on, single tokens (which leave
+    theirs idle) counted half; up to one of 64 rows a CU the shared form, beyond it two of 4 waves, unless the prompt is long and the
+    longest decides; one long prompt between them 128.
+    us of 4, 5, 8, 16 (and of the kernel with 16 rows a wave and two barriers a tile that this one replaced), heads 64 / 8 unless said: 241
+    tokens behind 224 17.5, 14.8, 21.1, 25.9 (22.3), with 8 single tokens of up to 500 keys 19.8, 23.7, 32.2, 35.6 (58.9); 97 behind 1000 29.3,
+    23.0, 34.3, 47.4 (42.6), with 8 of 1500 44.2, 30.0, 41.9, 92.4 (82.0); 512 18.7, 21.1, 22.2, 28.5 (25.3), with 8 of 500 28.3, 37.5, 36.2, 38.6
+    (98.9); 300 + 40 + 50 + 60 + 70 13.8, 19.2, 19.4, 21.4 (18.8); 900 39.7, 48.6, 40.7, 42.9 (56.3), with 8 of 500 46.6, 58.8, 54.5, 41.9; 1500 76.4,
+    93.8, 81.7, 64.0 (125); 2000 + 3 x 100 with 8 of 500 139, 185, 152, 116 (180); heads 32 / 8: 2048 72, 79, 68, 81 (120), 1500 with 8 of 500
+    53.1, 64.9, 58.0, 60.1 (78.6); heads 8 / 1: 900 with 8 of 1500 37.9, 27.7, 39.7, 52.7 (64.9), 3000 71.1, 51.5, 75.7, 106 (114).  Over 180 such
+    batches the pick is 1 % behind the best on average (17 % with every sequence taken for as long as the longest).  Short contexts lose a
+    microsecond: 24 tokens alone 6.8, 7.6, 10.1, 11.0 (6.2); behind 1000 keys, which the host does not see, the shared form is the best."""
+    if PREFILL_ATTN_FORM:
+        return PREFILL_ATTN_FORM
+
+    def bound(rows, partial):
+        tile = max(1, rows * nkv // nq)
+        return min(num_seqs * -(-max_qlen // tile), T // tile + partial) * nkv
+    if bound(256, (num_seqs + 1) // 2) > (256 if num_seqs == 1 else 239):
+        return 16
+    few = bound(64, num_seqs)
+    if num_seqs == 1 and max_qlen > 1024 and few > 512:
+        return 8
+    exact = few == bound(64, num_seqs * max_qlen)
+    return 4 if few > (256 if exact else 248) and (max_qlen <= 1024 or few > 512) else 5
+
+
 def paged_prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, cu_q: torch.Tensor,
                             context_lens: torch.Tensor, block_tables: torch.Tensor, scale: float, block_size: int,
                             max_qlen: int) -> torch.Tensor:
@@ -396,7 +431,7 @@ def paged_prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
                                      _chk(v_cache, BF16, "v_cache"), _chk(cu_q, I32, "cu_q"),
                                      _chk(context_lens, I32, "context_lens"), _chk(block_tables, I32, "block_tables"),
                                      float(scale), context_lens.shape[0], int(max_qlen), nq, nkv, D, block_size,
-                                     block_tables.shape[1], -1)
+                                     block_tables.shape[1], _prefill_form(T, int(max_qlen), context_lens.shape[0], nq, nkv), -1)
     return out
 
 
