@@ -704,6 +704,7 @@ def mgemm_heuristic(M: int, N: int, K: int, epi: int, fp8: bool, num_cus: int = 
 # "M_bucket,N,K,epi,fp8".  A row count between tuned buckets uses the plan of the nearest bucket
 # above it (the largest one beyond the table).
 _MG_TABLE: Optional[dict] = None
+_MG_NAMED: set = set()      # rows that K8S_MGEMM_OVERRIDE names: (N, K, epi, fp8, row bucket)
 MG_TABLE_PATH = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "engine", "assets",
                              "mgemm_gfx950.json")
 
@@ -731,6 +732,8 @@ def _mg_load_table() -> dict:
             for item in filter(None, os.environ.get("K8S_MGEMM_OVERRIDE", "").split(";")):
                 key, val = item.split("=")
                 plans[key.strip()] = [int(t) for t in val.split(":")] + [0.0, 0.0]
+                mb, n, kk, epi, fp8 = (int(t) for t in key.split(","))
+                _MG_NAMED.add((n, kk, epi, fp8, mb))
             for k, v in plans.items():
                 mb, n, kk, epi, fp8 = (int(t) for t in k.split(","))
                 mg_us, lib_us = (float(v[2]), float(v[3])) if len(v) >= 4 else (0.0, 0.0)
@@ -1097,11 +1100,18 @@ def _few_rows_tile(M: int, rows: int, K: int, epi: int, num_cus: int = 256) -> O
     4-wave kernel streams large weights faster, since its ring holds more of them in flight and the XCDs spread over k; with small
     ones mgemm's shorter start counts.  us, mgemm / here: 33 x 10240 x 8192 52 / 40, with the RMS prologue 70 / 38; 65 x 8192 x 8192 51 /
     34; 128 x 14336 x 4096 42 / 34; 17 x 16384 x 2048 17.3 / 13.9; 128 x 2 x 28672 x 8192 (SwiGLU, RMS) 200 / 177.  Below the lines: 64 x
-    4096 x 2048 9.0 / 10.6, 17 x 8192 x 8192 28.1 / 29.5, 128 x 4096 x 2048 11.9 / 12.4."""
+    4096 x 2048 9.0 / 10.6, 17 x 8192 x 8192 28.1 / 29.5, 128 x 4096 x 2048 11.9 / 12.4.  Over mgemm's tuned shapes (1280 .. 128256 x 1024 .. 28672, 17 -
+    128 rows, with the norm or the residual that they have in use) 15 % less time on average; a tuned plan of twice as deep as wide stays
+    up to 64 rows (8192 x 28672 33 93 / 93, 48 94 / 95, 64 96 / 99; untuned 4096 x 14336 30 / 28), and one that K8S_MGEMM_OVERRIDE names
+    always."""
     if M <= SGEMV_MAX_M or M >= PG_MIN_M or K % 64 or rows % 8 or rows * K * 2 >= 1 << 32:
         return None
     mb = rows * K * 2e-6
     if mb < (20.0 if M > 64 else 30.0 if M > 32 else 60.0) or (M <= 32 and (rows < 12288 or epi == EPI_SWIGLU)):
+        return None
+    n = rows // 2 if epi == EPI_SWIGLU else rows
+    tuned = _mg_table_row(M, n, K, epi, False)
+    if tuned is not None and ((n, K, epi, 0, tuned[0]) in _MG_NAMED or (M <= 64 and K > 2 * rows)):
         return None
     kt, best = K // 64, None
     for cfg, (tile, rnd, step, sp, slab, wmb, t0) in _P4_FEW_COST.items():
