@@ -341,11 +341,17 @@ __global__ __launch_bounds__(256, 1) void gemm_f32_kwave_kernel(F32Args a) {
 
 using namespace k8sllm;
 
-// The tile for a product, and whether it is expected to beat gemm_f32_kernel's tiles (0: it is not): us per 32 k, a part per round
-// of tiles over the CUs, one for an odd round (its tiles are alone on their CUs) and one a product.  16 more: k shared by the
-// waves, one workgroup on a CU always.  The tile's parts are fitted to 8 shapes of 2048 x 2048 .. 28672 x 4096 at M 24 - 512, rms
-// error 4 and 6 %: with a fit to N <= 16384 alone the pick was up to 14 % behind, 40 x 28672 x 4096 133 -> 117, 64 157 -> 141, 241 x
-// 6144 x 4096 129 -> 116, 384 x 4096 x 4096 115 -> 109.  K < 512: shares of K / 8 leave the smaller error.
+// The tile for a product (0: gemm_f32_kernel's are expected to be as good); 16 more: k shared by the waves.  Whether, and which of the
+// two, in us per 32 k, one constant part and one per round of tiles over the CUs, fitted to M 24 - 512, N 128 - 16384, K 512 - 8192 (where
+// the two models are within 5 % of each other, so are the kernels); a round of one workgroup per CU with k shared also pays its start and
+// its sum (4.5 us, of which nothing overlaps), so that is the choice for one or two rounds.  Where columns are faster there all the same
+// (28672 x 4096, 24 - 64 rows, 116 / 95 and 156 / 149 us; 384 x 4096 x 4096 117 / 112) the shares keep the smaller error, 2-norm against 64
+// bits: K = 4096 2.15e-7 / 2.29e-7, 14336 2.3e-7 / 2.8e-7.
+// How many rows a tile of columns has goes by a fit of 8 shapes of 2048 x 2048 .. 28672 x 4096, rms error 4 %: a part per round, one for
+// an odd round of up to three (its tiles are alone on their CUs) and one a product; from eight rounds on one that is partly filled costs that
+// part.  By the first fit / this one: 457 x 6720 x 4096 276 / 255, 441 x 3072 x 1536 50 / 47, 384 x 3648 x 2048 58.0 / 56.8, 393 x 14336 x
+// 4096 429 / 417; without the two exceptions 401 x 6144 x 4096 195 / 182, 352 x 7168 x 4096 195 / 183.  K < 512: shares of K / 8 leave the
+// smaller error.
 extern "C" int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles) {
   if (K < 512 || K % 32 || M <= 0 || N <= 0) return 0;
   // Listed tiles: most of the list is short of 64 rows or empty, and where its blocks meet on a CU is left to chance, so the parts
@@ -370,26 +376,31 @@ extern "C" int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles) {
   // 20.8 / 19.8, 70.1 / 68.7.
   const long cols = (long)N * batch;
   if (r1 == 1.0 && M <= 32 && (M <= 4 ? cols > 256 : M <= 16 || M > 24 || cols > 2048)) return 0;
-  // whether at all, by one fit (M 24 - 512, N 128 - 16384, K 512 - 8192), and with which tile, by the other
-  const double other = 2.0 * r2 < 1.1 * r1 ? 0.365 * r2 + 0.03 : 0.16 * r1 + 0.1;
-  bool ahead = false;
-  double best = 1e30;
+  double best = 2.0 * r2 < 1.1 * r1 ? 0.365 * r2 + 0.03 : 0.16 * r1 + 0.1;
   int pick = 0;
   for (int fq = 8; fq >= 1; --fq) {
     const double r = rounds((M + 16 * fq - 1) / (16 * fq), (N + 63) / 64);
-    ahead |= r * (0.125 * fq + 0.04) + 0.1 < other || (fq <= 4 && r * (0.12 * fq + 0.03 + 4.5 * 32 / K) < 0.96 * other);
-    const double t = r * (0.1157 * fq + 0.056) + ((long)r & 1 ? 0.002 * fq + 0.0666 : 0.0) + 5.24 * 32 / K;
+    const double t = r * (0.125 * fq + 0.04) + 0.1;
     if (t < best) {
       best = t;
       pick = fq;
     }
-    const double tk = r * (0.1164 * fq + 0.0773 + 0.445 * 32 / K) + 4.27 * 32 / K;
+    const double tk = r * (0.12 * fq + 0.03 + 4.5 * 32 / K);
     if (fq <= 4 && tk < 0.96 * best) {
       best = tk;
       pick = 16 + fq;
     }
   }
-  if (!ahead) pick = 0;
+  if (pick == 0 || pick > 16) return pick;
+  best = 1e30;
+  for (int fq = 8; fq >= 1; --fq) {
+    const double tiles = (double)((M + 16 * fq - 1) / (16 * fq)) * ((N + 63) / 64) * batch / 256.0, r = ceil(tiles);
+    const double t = (r >= 8.0 ? tiles : r) * (0.1157 * fq + 0.056) + (r == 1.0 || r == 3.0 ? 0.002 * fq + 0.0666 : 0.0);
+    if (t < best) {
+      best = t;
+      pick = fq;
+    }
+  }
   return pick;
 }
 
