@@ -1064,9 +1064,10 @@ def moe_combine(D: torch.Tensor, pos_of_pair: torch.Tensor, topk_w: Optional[tor
 def joint_experts(E: int, W: int, F: int) -> bool:
     """Whether a shared expert of the E others' size runs as one more group of their products: sizes that the big tiles take with
     any number of rows.  Two launches less a layer, and its rows fill the other groups' rounds: us, apart / joined (8 experts, top
-    2; products of a layer, weights from memory): W = F = 2048, 1 token 29.9 / 25.7, 32 61.4 / 57.8, 97 66.8 / 58.7, 333 83.0 / 67.1,
-    1531 151 / 133, 2048 183 / 172; W = 4096, F = 3584, 1 66.3 / 62.3, 32 156 / 150, 97 170 / 153, 200 188 / 197, 700 252 / 263, 1024 335 /
-    289, 2048 533 / 509."""
+    2; products of a layer, weights from memory): W = F = 2048, 1 token 30.4 / 25.1, 12 58.6 / 57.0, 32 61.2 / 58.8, 97 66.5 / 58.2, 333 83.7 /
+    68.0, 1531 154 / 134, 2048 188 / 177; W = 4096, F = 3584, 1 65.5 / 62.6, 4 108.5 / 110.5, 32 155 / 151, 97 168 / 151, 200 187 / 180, 333 216 /
+    194, 700 251 / 256, 1024 332 / 296, 1531 406 / 409, 2048 522 / 499: at most 3 % behind, where the rows of both end in part of a round, so
+    not a choice of the step's."""
     return E + 1 <= GROUP_BIG_MAX_GROUPS and W % 64 == 0 and F % 64 == 0 and W >= 128 and F >= 128
 
 

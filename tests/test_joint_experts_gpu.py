@@ -111,15 +111,15 @@ def test_stacks_hold_every_weight_once():
         assert sum(own.values()) == moe and m.weight_bytes() >= e * moe
 
 
-@pytest.mark.gpu
+@pytest.mark.parametrize("dev", ["cpu", pytest.param(DEV, marks=pytest.mark.gpu)])
 @pytest.mark.parametrize("T", [1, 7, 40])
-def test_layer_with_the_shared_expert_joined_and_apart(T):
+def test_layer_with_the_shared_expert_joined_and_apart(T, dev):
     """The same layer by one product of six experts and by five and one: sums of another order, a rounding of each output."""
-    _, _, m = model(DEV, torch.bfloat16, 128)
+    _, _, m = model(dev, torch.bfloat16, 128)
     L = m.layers[0].mlp
-    ids = torch.randint(0, 96, (T,), generator=torch.Generator().manual_seed(T)).to(torch.int32).to(DEV)
-    h = torch.randn(T, 128, generator=torch.Generator().manual_seed(T)).to(torch.bfloat16).to(DEV)
-    sg = torch.randn(T, 1, generator=torch.Generator().manual_seed(T)).to(DEV)
+    ids = torch.randint(0, 96, (T,), generator=torch.Generator().manual_seed(T)).to(torch.int32).to(dev)
+    h = torch.randn(T, 128, generator=torch.Generator().manual_seed(T)).to(torch.bfloat16).to(dev)
+    sg = torch.randn(T, 1, generator=torch.Generator().manual_seed(T)).to(dev)
     table = m._tables[(6, 3)]
     joined = m._moe(L, h, sg, {"routes": {(6, 3): sm.moe_table_align(ids, table, 6)}}).combined().double()
     apart = type(L)(L.cfg, L.experts, L.shared, L.sg, ((5, 2), 0))
