@@ -1062,10 +1062,9 @@ _P4_COST = {1: (0.652, 2.2, 0.0, 5.33, 0.24, 0.066, 0.305),
 _P4_COST_T0 = {1: 2.16, 2: 1.46, 3: 2.25, 4: 0.0, 5: 0.34, 6: 2.9, 7: 0.298, 8: 1.16}
 
 
-@functools.lru_cache(maxsize=4096)
-def _pgemm_cheapest(M: int, N: int, K: int, num_cus: int) -> Tuple[str, int, int]:
-    """(kernel, configuration, splits) of the cheapest bf16 plan by _P4_COST."""
-    kt, best = K // 64, None
+def _pgemm_costs(M: int, N: int, K: int, num_cus: int):
+    """(us, configuration, splits) of the bf16 plans by _P4_COST."""
+    kt = K // 64
     for cfg, (tile, rnd, step, sp, slab, wmb, omb) in _P4_COST.items():
         bp, bq, _ = pgemm4_configs()[cfg]
         tiles = -(-N // bp) * -(-M // bq)
@@ -1074,10 +1073,28 @@ def _pgemm_cheapest(M: int, N: int, K: int, num_cus: int) -> Tuple[str, int, int
             if s > 1 and (tiles * s > 2 * num_cus or kt // s < 4):
                 break
             rounds, per = -(-tiles * s // num_cus), -(-kt // s)
-            us = base + rounds * (rnd + tile * per) + step * per + (sp + slab * M * N * s * 4e-6 if s > 1 else 0.0)
-            if best is None or us < best[0]:
-                best = (us, cfg, s)
-    return ("pgemm4",) + best[1:]
+            yield base + rounds * (rnd + tile * per) + step * per + (sp + slab * M * N * s * 4e-6 if s > 1 else 0.0), cfg, s
+
+
+@functools.lru_cache(maxsize=4096)
+def _pgemm_cheapest(M: int, N: int, K: int, num_cus: int) -> Tuple[str, int, int]:
+    """(kernel, configuration, splits) of the cheapest bf16 plan by _P4_COST."""
+    return ("pgemm4",) + min(_pgemm_costs(M, N, K, num_cus), key=lambda p: p[0])[1:]
+
+
+# An activation is part of an unsplit product's epilogue, on sums that nothing has rounded, and behind a split one a launch on rounded
+# sums: so a split plan within P4_ACT_SLACK of an unsplit one gives way to it.  us, gated, split and activation / unsplit: 192 x 14336 x 4096
+# 47.9 / 44.0, 130 x 16384 x 4096 47.1 / 44.5, 900 x 5120 x 5120 66.2 / 62.4.  Beyond it, or deeper than P4_ACT_MAX_K, where the fit flatters
+# a lone walk over k, the split stays: 384 x 5120 x 5120 39.3 / 43.6, 448 x 2048 x 8192 32.2 / 35.8.
+P4_ACT_SLACK, P4_ACT_MAX_K = 1.065, 5120
+
+
+@functools.lru_cache(maxsize=4096)
+def _pgemm_unsplit(M: int, N: int, K: int, num_cus: int = 256) -> Optional[int]:
+    """Configuration of the cheapest unsplit bf16 plan if a split one gives way to it."""
+    plans = list(_pgemm_costs(M, N, K, num_cus))
+    us, cfg, _ = min((p for p in plans if p[2] == 1), key=lambda p: p[0])
+    return cfg if K <= P4_ACT_MAX_K and us <= P4_ACT_SLACK * min(p[0] for p in plans) else None
 
 
 def pgemm_heuristic(M: int, N: int, K: int, epi: int, fp8: bool, num_cus: int = 256) -> Tuple[str, int, int, int]:
@@ -1173,6 +1190,17 @@ def gemm_route(M: int, N: int, K: int, epi: int, fp8: bool) -> Tuple[str, Option
     if M < PG_MIN_M or plan[0] == "mgemm":   # (the tuner records "mgemm" where its tuned plan was faster)
         return "mgemm", None
     return plan[0], plan[1:]
+
+
+def gemm_act_route(M: int, N: int, K: int) -> Tuple[str, Optional[tuple]]:
+    """:func:`gemm_route` of a bf16 product with an activation behind it: unsplit where that costs little (_pgemm_unsplit; plans of
+    the table stand)."""
+    kern, plan = gemm_route(M, N, K, EPI_BF16, False)
+    if kern == "pgemm4" and plan[1] > 1 and GEMM_BACKEND == "auto" and (N, K, EPI_BF16, 0) not in _pg_load_table():
+        cfg = _pgemm_unsplit(-(-M // 64) * 64, N, K)
+        if cfg is not None:
+            plan = (cfg, 1, plan[2])
+    return kern, plan
 
 
 def mx_rows(M: int, w) -> bool:

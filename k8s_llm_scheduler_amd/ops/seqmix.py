@@ -543,7 +543,7 @@ def linear_act(a: torch.Tensor, w: torch.Tensor, kind: int, limit: float = 0.0, 
             out = _ops.linear_act_rows(a, w, pair, kind, float(limit), float(alpha))
             if out is not None:
                 return out
-        kern, plan = _ops.gemm_route(M, w.shape[0], K, _ops.EPI_BF16, False) if M >= 129 else ("", None)
+        kern, plan = _ops.gemm_act_route(M, w.shape[0], K) if M >= 129 else ("", None)
         if kern == "pgemm4" and plan[1] == 1 and a.data_ptr() % 16 == 0 and \
                 (bias is None or (pair and bias.dtype == BF16 and bias.numel() == w.shape[0] and bias.data_ptr() % 8 == 0)):
             N = w.shape[0] // 2 if pair else w.shape[0]

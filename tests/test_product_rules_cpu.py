@@ -143,6 +143,15 @@ def test_activations_join_every_unsplit_product_of_big_tiles(M, N, K, kind, laun
     assert launches.names() == (["pgemm4_act"] if plan[1] == 1 else ["pgemm4", "act"]) and (plan[1] > 1) == (K == 4096)
 
 
+@pytest.mark.parametrize("M,N,K,joins", [(192, 14336, 4096, True), (130, 16384, 4096, True), (900, 5120, 5120, True), (256, 7168, 4096, True),
+                                         (333, 6720, 4096, True), (384, 5120, 5120, False), (448, 2048, 8192, False)])
+def test_activations_keep_split_products_from_rounding_ahead_of_them(M, N, K, joins, launches):
+    """A product whose split plan is a little cheaper takes the unsplit one with its activation, one rounding; the product alone does not."""
+    assert ops.gemm_route(M, N, K, ops.EPI_BF16, False)[1][1] > 1
+    sm.linear_act(torch.zeros(M, K, dtype=BF16), torch.zeros(N, K, dtype=BF16), sm.ACT_GELU_TANH)
+    assert launches.names() == (["pgemm4_act"] if joins else ["pgemm4", "act"])
+
+
 def test_activations_follow_the_switches_of_the_gemv(launches, monkeypatch):
     """K8S_GEMV_MAX_M moves 3 - 8 rows to the GEMV, whose form with an activation takes two: then the product and the activation."""
     for rows, kind in ((4096, sm.ACT_GELU_TANH), (2048, sm.ACT_RELU2)):
