@@ -282,6 +282,7 @@ class _Wkv:
     cfg: MixerConfig
     mu: torch.Tensor        # [5, W]: r, k, v, g, w
     w_in: torch.Tensor      # [4 H D + lora, W]: r, k, v, g, the decay's first factor
+    w_parts: tuple          # views of it, [4, H D, W] and [lora, W]
     w2: torch.Tensor        # [H D, lora]
     w0: torch.Tensor        # [H D]
     u: torch.Tensor         # [H D]
@@ -370,9 +371,9 @@ class PutulornModel(StreamModel):
         for i, L in enumerate(c.layers):
             p, m = f"l{i}.mix.", L.mixer
             if m.type == "wkv":
-                mixer = _Wkv(m, t(torch.stack([get(p + "mu." + s) for s in MU_ORDER])),
-                             t(torch.cat([get(p + s) for s in ("r", "k", "v", "g", "w1")])), t(get(p + "w2")), t(get(p + "w0")), t(get(p + "u").reshape(-1)), t(get(p + "norm")),
-                             t(get(p + "o")))
+                w_in = t(torch.cat([get(p + s) for s in ("r", "k", "v", "g", "w1")]))
+                mixer = _Wkv(m, t(torch.stack([get(p + "mu." + s) for s in MU_ORDER])), w_in, sm.each_parts(w_in, 4, m.heads * m.dim),
+                             t(get(p + "w2")), t(get(p + "w0")), t(get(p + "u").reshape(-1)), t(get(p + "norm")), t(get(p + "o")))
                 if m.dim > sm.wkv_max_dim():
                     raise ValueError(f"layer {i}: wkv head dimension {m.dim} exceeds {sm.wkv_max_dim()}")
             else:
@@ -447,7 +448,7 @@ class PutulornModel(StreamModel):
         m = w.cfg
         S, shift = self.states[run.cache]
         mix = mixed(w.mu, shift)                                          # [5, T, W]
-        (r, k, v, g), lo = sm.linear_each_tanh(mix, w.w_in, m.heads * m.dim)
+        (r, k, v, g), lo = sm.linear_each_tanh(mix, w.w_in, m.heads * m.dim, w.w_parts)
         del mix
         return sm.wkv_step(r, k, v, g, lo, w.w2, w.w0, w.u, w.lnw, S, b, m.heads, m.dim, self.cfg.rms_eps, "max_keys" in b)
 

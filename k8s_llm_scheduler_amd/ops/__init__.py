@@ -1182,12 +1182,14 @@ def gemm_route(M: int, N: int, K: int, epi: int, fp8: bool) -> Tuple[str, Option
         return ("mgemm", None) if mg_ok else ("library", None)
     if not pg_ok:
         return "library", None
+    if M < PG_MIN_M and GEMM_BACKEND == "auto":
+        return "mgemm", None
     plan, pg_us = pgemm_plan_for(M, N, K, epi, fp8)
     if GEMM_BACKEND == "pgemm":
         if plan[0] == "mgemm":
             plan = _pgemm_big_tiles(M, N, K, epi, fp8)
         return plan[0], plan[1:]
-    if M < PG_MIN_M or plan[0] == "mgemm":   # (the tuner records "mgemm" where its tuned plan was faster)
+    if plan[0] == "mgemm":   # (the tuner records it where its tuned plan was faster)
         return "mgemm", None
     return plan[0], plan[1:]
 

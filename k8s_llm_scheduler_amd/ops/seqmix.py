@@ -478,9 +478,14 @@ def linear_each(a: torch.Tensor, w: torch.Tensor):
     return tuple(linear(a[i], w[i]) for i in range(G))
 
 
-def linear_each_tanh(a: torch.Tensor, w: torch.Tensor, N: int):
+def each_parts(w: torch.Tensor, G: int, N: int):
+    """The weights of :func:`linear_each_tanh` apart, for its ``parts``: [G, N, K] and [L, K]."""
+    return w[:G * N].view(G, N, w.shape[1]), w[G * N:]
+
+
+def linear_each_tanh(a: torch.Tensor, w: torch.Tensor, N: int, parts: Optional[tuple] = None):
     """(:func:`linear_each` of all inputs but the last, tanh of the last one's product): a [G + 1, M, K], w [G N + L, K] the weights one
-    after the other.  A few bf16 rows in one launch (stream_gemv.hip).  us, two launches or more / one, weights from memory: 4 weights of
+    after the other (``parts``: views of them, :func:`each_parts`, where a caller keeps them).  A few bf16 rows in one launch (stream_gemv.hip).  us, two launches or more / one, weights from memory: 4 weights of
     2048 x 2048 and one of 128 x 2048, 1 row 15.4 / 12.0, 8 17.5 / 13.3, 16 19.1 / 17.5; of 4096 x 4096 and 256 x 4096, 1 39.2 / 37.0,
     8 42.4 / 39.6, 16 44.1 / 46.4 (x in registers: 16 rows of 4096 leave room for less of the weights under way)."""
     G, M, K = a.shape[0] - 1, a.shape[1], a.shape[2]
@@ -492,7 +497,8 @@ def linear_each_tanh(a: torch.Tensor, w: torch.Tensor, N: int):
         last = torch.empty(M, L, dtype=BF16, device=a.device)
         if _native().rows_each(out.data_ptr(), last.data_ptr(), a.data_ptr(), w.data_ptr(), G, N, L, M, K, -1):
             return out.unbind(0), last
-    return linear_each(a[:G], w[:G * N].view(G, N, K)), linear_act(a[G], w[G * N:], ACT_TANH)
+    each, last = parts or each_parts(w, G, N)
+    return linear_each(a[:G], each), linear_act(a[G], last, ACT_TANH)
 
 
 def _each_once(a: torch.Tensor, w: torch.Tensor) -> bool:
