@@ -33,7 +33,7 @@ CSRC = PKG / "csrc"
 BUILD = PKG.parent / "build" / "native"
 ARCH = os.environ.get("K8S_HIP_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-# Kernels added since the packed-fp32 rule, and pgemm4.hip with its activation epilogues, are built without the packed fp32
+# Kernels added since the packed-fp32 rule, pgemm4.hip with its activation epilogues and the rewritten attn_prefill.hip are built without the packed fp32
 # instructions (v_pk_add/mul/fma_f32), which -O3 otherwise forms from ordinary float code.  The other kernel files keep the
 # flags they were validated with: with the option on every file, the two-rank fused GEMV all-reduce check of tests/test_multigpu.py reported a wrong sum.
 NO_PACKED_FP32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

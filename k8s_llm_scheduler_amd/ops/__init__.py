@@ -1048,7 +1048,7 @@ def _pg_load_table() -> dict:
 # hide part from each other; with split-K the combine launch and the slabs it moves; the weights and the output.  Fitted to 22
 # weight shapes (576 x 2048 .. 28672 x 4096) at 12 row counts (130 .. 2048), weights cold: rms error 5 - 10 % per configuration,
 # the pick within 1 % of the best plan on average and 18 % at most, 6 % faster on average than the rule for the six tiles there
-# were (64 x 64 then two stages ahead), 7 % slower at most (256 x 6144 x 3072) but for 14 % at 256 x 2048 x 8192.  pgemm.hip's
+# were (64 x 64 then two stages ahead), 9 % slower at most (256 x 2048 x 8192; 256 x 6144 x 3072 8 %).  pgemm.hip's
 # 8-wave tiles were the best plan of none of these; the tuned table names them for some of the 70B's products of 256 - 8192
 # rows and its logits, and SwiGLU and fp8 products that it does not list take them (_pgemm_big_tiles).
 _P4_COST = {1: (0.652, 2.2, 0.0, 5.33, 0.24, 0.066, 0.305),
@@ -1084,7 +1084,7 @@ def _pgemm_cheapest(M: int, N: int, K: int, num_cus: int) -> Tuple[str, int, int
 
 # An activation is part of an unsplit product's epilogue, on sums that nothing has rounded, and behind a split one a launch on rounded
 # sums: so a split plan within P4_ACT_SLACK of an unsplit one gives way to it.  us, gated, split and activation / unsplit: 192 x 14336 x 4096
-# 47.9 / 44.0, 130 x 16384 x 4096 47.1 / 44.5, 900 x 5120 x 5120 66.2 / 62.4.  Beyond it, or deeper than P4_ACT_MAX_K, where the fit flatters
+# 47.8 / 41.8, 130 x 16384 x 4096 46.7 / 43.8, 900 x 5120 x 5120 66.5 / 62.2.  Beyond it, or deeper than P4_ACT_MAX_K, where the fit flatters
 # a lone walk over k, the split stays: 384 x 5120 x 5120 39.3 / 43.6, 448 x 2048 x 8192 32.2 / 35.8.
 P4_ACT_SLACK, P4_ACT_MAX_K = 1.065, 5120
 
