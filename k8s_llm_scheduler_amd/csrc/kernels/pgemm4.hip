@@ -20,7 +20,14 @@
 //    all of them ask for the same bytes of every row, whose strides of 16 KB meet on a part of the memory's channels, and for the
 //    same lines of x (loads alone, 32768 rows of 16 KB: 4.1 -> 6 TB/s).  241 x 57344 x 8192 251 -> 230 us, 8192 x 28672 136 -> 131,
 //    8192 x 8192 50 -> 47.  With more row tiles the walk in step is the better one (2048 x 16384 x 2048 106 -> 111): so not there; the
-//    grouped form by its rows (P4Args::spread).
+//    grouped form by its rows (P4Args::spread); but deep ones, whose rows' strides put whole columns of tiles on the same channels, from
+//    16384 columns on up to 8 row tiles (x 8192 x 28672, 333 rows 171 -> 151 us, 512 204 -> 192, 1024 363 -> 348, 2048 675 -> 654; 3413
+//    1265 -> 1279; of 14336 columns and fewer 1 % slower on average).
+//  * rows of 4 KB and less (K up to 2048) on tiles of at most 128 x 128 and on those of 32 tokens: every column of tiles starts its walk
+//    an eighth of it after the one before (P4Args::fine): at one k the rows' bytes lie in a few of the memory's channels, and short
+//    tiles have no time to drift apart.  us: 2048 x 2048 x 2048 21.1 -> 19.0, 1024 x 3072 x 2048 19.1 -> 16.3, 512 x 3648 x 2048 16.4 ->
+//    13.2, gated 130 x 2 x 8192 x 2048 26.6 -> 25.3; over 65 products of 128 - 3413 rows 3 - 5 % less on average, none more than 1.8 % slower.  Of
+//    larger tiles, which read x from L2 in step, 2 - 12 % slower; of K = 4096 at 128 x 128 0.89 - 1.20 of the time.
 //  * tiles of 224 rows (a fragment then holds 8 gate and 8 up rows, a pair in a lane) and of 192 tokens, where they fill the last
 //    round: 241 x 57344 x 8192 on 256 CUs 230 -> 207 us, 3413 x 10240 x 8192 484 -> 412.
 //  * register double buffer: the fragments of the next 32 k are read (ds_read_b128) under the MFMAs of the current ones, in
@@ -93,6 +100,7 @@ struct P4Args {
   float eps;
   const float* scale;    // P4_SCALED: 1 / rms of every token's row
   int spread;            // the XCDs start their walk over k an eighth of it apart
+  int fine;              // ... and the tile columns fine / 32 of it, on top of that
   int wide;              // the output's rows can be stored in 16-byte pieces
   float limit, alpha;    // P4_GLU: of the gated kind
   float last_limit;      // grouped form: the limit of the last group
@@ -202,7 +210,7 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
   // this wave's 1 KB of the first 4 KB of LDS
   const uint32_t lds0 = (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)lds) + wid * 1024;
   // the walk over k starts at stage `rot` and wraps: stage u reads bytes k0(u) .. k0(u) + 127 of the slice's rows
-  const int rot = a.spread ? (int)(((long long)xcd * n2) >> 3) : 0;
+  const int rot = a.spread ? (int)((((uint32_t)(4 * xcd + a.fine * nt) & 31u) * (uint32_t)n2) >> 5) : 0;
   const uint32_t kend = (uint32_t)n2 * 128u;
   auto next_k = [&](uint32_t k) -> uint32_t { return k + 128u == kend ? 0u : k + 128u; };
   // instruction d of a stage's weights (k offset, byte offset of its slot), of its x
@@ -501,8 +509,9 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
       __builtin_amdgcn_wave_barrier();
       const int c = lane % NC;
 #pragma unroll
-      for (int p = 0; p < 16 * FQ * NC / 64; ++p) {
+      for (int p = 0; p < (16 * FQ * NC + 63) / 64; ++p) {
         const int row = p * (64 / NC) + lane / NC, m = m0 + wc * (BQ / 2) + row, n0 = nw + c * 8;
+        if (16 * FQ * NC < 64 && row >= 16 * FQ) break;
         const u32x4 o = *reinterpret_cast<const u32x4*>(mine + row * ROW + ((c ^ ((row >> SH) & (NC - 1))) << 4));
         if (m < m_end && n0 < a.N_out && (CH == NC || c < CH))
           *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(a.out) + (size_t)m * a.N_out + n0) = o;
@@ -648,6 +657,28 @@ constexpr P4Cfg kP4Cfgs[] = {
     {8, 6, 2, 1},   // 8: 256 x 192
 };
 constexpr int kP4NumCfgs = sizeof(kP4Cfgs) / sizeof(kP4Cfgs[0]);
+// tiles of 32 tokens, of the grouped form only (configurations kP4NumCfgs and up), two workgroups on a CU: groups of a few rows are a
+// stream of weights, at which the CUs are equally busy only if the tiles fill a whole number of rounds, so several widths.  Which one:
+// ops/seqmix.py _grouped_few.  us, tiles of 64 and 128 rows / these, 8 groups and a common one, weights from memory: gated 2 x 2048 x 2048, 32
+// tokens 36.1 / 31.3 (160 x 32), 8 27.6 / 26.6; 2048 x 2048, 32 21.8 / 18.1 (96 x 32); 4096 x 3584, 16 55.8 / 49.2.
+constexpr P4Cfg kP4Few[] = {
+    {2, 1, 4, 4},   //  9:  64 x 32
+    {3, 1, 3, 3},   // 10:  96 x 32
+    {4, 1, 3, 3},   // 11: 128 x 32
+    {5, 1, 2, 2},   // 12: 160 x 32
+};
+constexpr int kP4Grouped = kP4NumCfgs + sizeof(kP4Few) / sizeof(kP4Few[0]);
+constexpr P4Cfg p4_tile(int c) { return c < kP4NumCfgs ? kP4Cfgs[c] : kP4Few[c - kP4NumCfgs]; }
+// the walks of P4Args::spread and fine
+void p4_walk(P4Args& a, int cfg) {
+  const P4Cfg t = p4_tile(cfg);
+  if (a.K <= 2048 && (t.fq == 1 || (t.fp <= 4 && t.fq <= 4))) {
+    a.spread = 1;
+    a.fine = 4;
+  } else if (a.K >= 16384 && a.m_tiles <= 8 && a.groups == 0) {
+    a.spread = 1;
+  }
+}
 
 template <int C, int EPI, int NORM>
 int p4_launch(const P4Args& a, hipStream_t s) {
@@ -742,8 +773,8 @@ extern "C" int k8s_pgemm_reduce(void* out, const void* res, const float* slab, i
 // The forms with an activation (gated kinds 0, 1, 5; elementwise 7) and the grouped ones.
 template <int C, int EPI, bool GRP, int KIND>
 int p4_act_launch(const P4Args& a, hipStream_t s) {
-  hipLaunchKernelGGL((pgemm4_kernel<kP4Cfgs[C].fp, kP4Cfgs[C].fq, kP4Cfgs[C].dw, kP4Cfgs[C].dx, EPI, P4_PLAIN, GRP, KIND>), dim3(a.nwg),
-                     dim3(256), 0, s, a);
+  constexpr P4Cfg T = p4_tile(C);
+  hipLaunchKernelGGL((pgemm4_kernel<T.fp, T.fq, T.dw, T.dx, EPI, P4_PLAIN, GRP, KIND>), dim3(a.nwg), dim3(256), 0, s, a);
   return (int)hipGetLastError();
 }
 template <int C, bool GRP>
@@ -762,7 +793,7 @@ int p4_act_kind(const P4Args& a, int kind, hipStream_t s) {
   return -1;
 }
 P4Args p4_args(void* out, const void* x, const void* W, int M, int N_out, int K, bool pair, int cfg, int group_m) {
-  const int bp = 32 * kP4Cfgs[cfg].fp, bq = 32 * kP4Cfgs[cfg].fq, feat = pair ? bp / 2 : bp;
+  const int bp = 32 * p4_tile(cfg).fp, bq = 32 * p4_tile(cfg).fq, feat = pair ? bp / 2 : bp;
   P4Args a = {};
   a.out = out;
   a.x = static_cast<const uint8_t*>(x);
@@ -780,6 +811,7 @@ P4Args p4_args(void* out, const void* x, const void* W, int M, int N_out, int K,
   a.group_m = group_m > 0 ? group_m : 1;
   a.nwg = a.m_tiles * a.n_tiles;
   a.spread = a.m_tiles == 1;
+  p4_walk(a, cfg);
   a.wide = N_out % 8 == 0 && ((uintptr_t)out & 15) == 0;
   return a;
 }
@@ -854,6 +886,7 @@ extern "C" int k8s_pgemm4(void* out, float* slab, const void* x, const void* W, 
   a.eps = eps;
   a.scale = scale;
   a.spread = a.m_tiles == 1;
+  p4_walk(a, cfg);
   a.wide = res == nullptr && N_out % 8 == 0 && ((uintptr_t)out & 15) == 0;
   if (scale != nullptr && splits > 1) a.scale = nullptr;   // the sums of the slices are scaled by the combine
   int rc = p4_cfg(a, cfg, epi, a.scale != nullptr ? P4_SCALED : scale == nullptr && rms ? P4_RMS : P4_PLAIN, stream);
@@ -899,14 +932,17 @@ extern "C" int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M
   const bool pair = kind >= 0;
   if (kind < -1 || (pair && kind > 1 && kind != 5)) return -1;
   if (rows <= 0) return 0;
-  if (M <= 0 || N_out <= 0 || N_out % 4 || K <= 0 || K % 64 || groups <= 0 || (seg == nullptr && rows % groups) || cfg < 0 || cfg >= kP4NumCfgs) return -1;
+  if (M <= 0 || N_out <= 0 || N_out % 4 || K <= 0 || K % 64 || groups <= 0 || (seg == nullptr && rows % groups) || cfg < 0 || cfg >= kP4Grouped) return -1;
   if (ldx < K || ldx % 8 || (((uintptr_t)x | (uintptr_t)W) & 15) || ((uintptr_t)out & 7)) return -1;
   const long long kbytes = (long long)K * 2, wrows = (pair ? 2LL : 1LL) * N_out;
   if (wrows * kbytes >= (1LL << 32) || (long long)M * ldx * 2 >= (1LL << 32)) return -5;   // 32-bit DMA offsets
   P4Args a = p4_args(out, x, W, rows, N_out, K, pair, cfg, group_m);
-  const int bq = 32 * kP4Cfgs[cfg].fq;
+  const int bq = 32 * p4_tile(cfg).fq;
   a.m_tiles = rows / bq + groups;        // whole tiles, and a partial one per group
+  a.groups = groups;
   a.spread = groups >= 8 && rows <= 192LL * groups;
+  a.fine = 0;
+  p4_walk(a, cfg);
   if ((long long)a.m_tiles * a.n_tiles > (1LL << 30)) return -1;
   a.nwg = a.m_tiles * a.n_tiles;
   a.xbytes = (uint32_t)(ldx * 2);
@@ -914,7 +950,6 @@ extern "C" int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M
   a.gsize = rows / groups;
   a.a_rows = a_rows;
   a.wstride = wrows * kbytes;
-  a.groups = groups;
   a.limit = limit;
   a.alpha = alpha;
   a.last_limit = last_limit;
@@ -926,6 +961,10 @@ extern "C" int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M
     case 6: return p4_act_kind<6, true>(a, kind, stream);
     case 7: return p4_act_kind<7, true>(a, kind, stream);
     case 8: return p4_act_kind<8, true>(a, kind, stream);
+    case 9: return p4_act_kind<9, true>(a, kind, stream);
+    case 10: return p4_act_kind<10, true>(a, kind, stream);
+    case 11: return p4_act_kind<11, true>(a, kind, stream);
+    case 12: return p4_act_kind<12, true>(a, kind, stream);
   }
   return p4_act_kind<4, true>(a, kind, stream);
 }

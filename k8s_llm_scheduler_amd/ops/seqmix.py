@@ -439,12 +439,70 @@ def _grouped_tile(rows: int, E: int, N: int, K: int, pair: bool, even: bool = Fa
     return best[1]
 
 
+# The same for groups of GROUP_FEW_ROWS drawn rows each on average and fewer, of GROUP_FEW_WEIGHTS weights (least, most), which are a stream
+# of weights at which the CUs have to be equally busy: configuration -> (fixed, per MB of the weights that are read, per 64-deep
+# k-step of a CU's first tile, of its other ones, per tile, per tile and 65536 outputs of a gated activation); the stream and the
+# busiest CU's tiles hide each other but for where they are about as long (the root of their fourth powers' sum).  Fitted to 312
+# products of 4 - 33 groups, 2048 x 1024 .. 2 x 3584 x 4096, 1 - 160 tokens, weights cold: rms error 9 %.  8 groups and a common one of 1 - 80
+# tokens, by the rule above and its tiles / here: 2 x 2048 x 2048 8 33.2 / 32.6, 32 36.7 / 33.2, 64 40.3 / 35.9; 2048 x 2048 32 22.0 / 18.5;
+# 4096 x 3584 2 28.4 / 28.5, 32 59.6 / 50.3; over 60 such products 10 % less on average, 1 % more at most.  Larger weights have tiles for
+# many rounds whatever their width: 2 x 3584 x 4096, 64 tokens 94.9 / 108.5.
+GROUP_FEW_ROWS, GROUP_FEW_WEIGHTS = 20, (1 << 21, 1 << 24)
+_GROUP_FEW_TILE = {3: (128, 128), 5: (128, 64), 6: (64, 64), 9: (64, 32), 10: (96, 32), 11: (128, 32), 12: (160, 32)}
+_GROUP_FEW_COST = {3: (5.43, 0.186, 0.434, 0.537, 0.0, 8.03), 5: (4.93, 0.187, 0.346, 0.517, 0.0, 17.0),
+                   6: (3.10, 0.169, 0.210, 0.293, 1.30, 5.90), 9: (3.29, 0.185, 0.170, 0.228, 1.0, 6.11),
+                   10: (3.97, 0.187, 0.185, 0.356, 0.66, 15.3), 11: (4.75, 0.182, 0.203, 0.529, 0.0, 20.7),
+                   12: (5.38, 0.187, 0.256, 0.552, 0.0, 40.0)}
+
+
+def _grouped_few(rows: int, drawn: int, N: int, K: int, pair: bool, common: int) -> int:
+    """Configuration of the grouped product of ``drawn`` groups, of few rows each, and ``common`` rows of one more, by _GROUP_FEW_COST:
+    the mean over the tiles that are expected and 1.2 deviations on both sides of them (the groups' sizes as Poisson's).  Below 1.5 rows a
+    group too many of them have none for whole rounds to go by: the smallest tile, 0 - 7 % faster than 64 x 64 (2048 x 2048, 5 tokens 15.1 /
+    14.9, on 96 x 32 16.0, on 128 x 32 17.7)."""
+    r, n, kt, best = (rows - common) / drawn, (2 * N if pair else N), K / 64, None
+    if r < 1.5:
+        return 9
+    more, p, left = [], math.exp(-r), 1.0            # the chances of more than 0, 32, 64, ... rows
+    for k in range(1 + int(r + 8.0 * math.sqrt(r) + 8.0)):
+        left -= p
+        if k % 32 == 0:
+            more.append(max(left, 0.0))
+        p *= r / (k + 1)
+    stream = (drawn * more[0] + (common > 0)) * n * K * 2e-6
+    dist = {}                                        # tokens of a tile: tiles of the groups, the deviation of their number
+    for bq in (32, 64, 128):
+        m1, m2 = sum(more[::bq // 32]), sum((2 * t + 1) * c for t, c in enumerate(more[::bq // 32]))
+        dist[bq] = drawn * m1 + -(-common // bq), math.sqrt(max(0.0, m2 - m1 * m1) * drawn)
+    for cfg, (t0, wmb, first, other, tile, act_us) in _GROUP_FEW_COST.items():
+        bp, bq = _GROUP_FEW_TILE[cfg]
+        tiles, dev = dist[bq]
+        us = 0.0
+        for z in (-1.2, 0.0, 1.2):
+            q = max(1, math.ceil(max(tiles + z * dev, 0.0) * -(-n // bp) / 256 - 0.01))
+            busy = kt * (first + other * (q - 1)) + q * (tile + (act_us * bp * bq / 65536 if pair else 0.0))
+            us += t0 + ((stream * wmb) ** 4 + busy ** 4) ** 0.25
+        if best is None or us < best[0]:
+            best = (us, cfg)
+    return best[1]
+
+
+@functools.lru_cache(maxsize=4096)
+def _grouped_plan(rows: int, E: int, N: int, K: int, pair: bool, even: bool, common: int) -> int:
+    """Configuration of the grouped big-tile product: :func:`_grouped_few`'s or :func:`_grouped_tile`'s."""
+    drawn = E - (common > 0)
+    least, most = GROUP_FEW_WEIGHTS
+    if not even and E > 1 and 0 < rows - common <= GROUP_FEW_ROWS * drawn and least <= (2 * N if pair else N) * K <= most:
+        return _grouped_few(rows, drawn, N, K, pair, common)
+    return _grouped_tile(rows, E, N, K, pair, even, common)
+
+
 def _pgemm4_grouped(a, w, a_rows, rows: int, seg, N: int, kind: int = -1, limit: float = 0.0, alpha: float = 1.0, common: int = 0,
                     common_limit: Optional[float] = None):
     E, _, K = w.shape
     out = torch.empty(rows, N, dtype=BF16, device=a.device)
     _native().pgemm4_grouped(out.data_ptr(), a.data_ptr(), w.data_ptr(), a.shape[0], rows, N, K, E, _p(seg, I32, "seg"),
-                             _p(a_rows, I32, "a_rows"), a.stride(0), _grouped_tile(rows, E, N, K, kind >= 0, seg is None, common), 4, kind,
+                             _p(a_rows, I32, "a_rows"), a.stride(0), _grouped_plan(rows, E, N, K, kind >= 0, seg is None, common), 4, kind,
                              float(limit), float(alpha), float(limit if common_limit is None else common_limit), -1)
     return out
 

@@ -83,3 +83,38 @@ def test_groups_spread_over_k(sizes, cfg, kind, monkeypatch):
     y = torch.cat([x[rows[int(seg[e]):int(seg[e + 1])].long()].float() @ w[e].float().T for e in range(E)])
     want = y if kind is None else y[:, :N].clamp(min=0) * y[:, N:]
     assert torch.equal(got, want.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("cfg,bp", [(9, 64), (10, 96), (11, 128), (12, 160)])
+@pytest.mark.parametrize("stages", [1, 2, 3, 5, 7, 32, 33])
+@pytest.mark.parametrize("kind", [None, sm.ACT_RELU])
+def test_groups_of_few_rows(cfg, bp, stages, kind):
+    """The tiles of 32 tokens: groups at their edges, empty ones, columns that do not fill the last tile, one stage to more than the ring
+    holds, k walked from every column's own stage (up to 32) and in step or an XCD's; rows stored whole and piecewise."""
+    K = 64 * stages
+    for sizes, N, shift in (((1, 0, 31, 32, 33, 0, 65, 2), bp + 16, 0), ((3, 32), 2 * bp, 0), ((0, 7, 64), bp - 4, 4), ((1, 2, 0, 1, 5, 0, 0, 2, 9), 3 * bp + 4, 0)):
+        E, P = len(sizes), sum(sizes)
+        seg = torch.tensor((0,) + sizes).cumsum(0).to(torch.int32).cuda()
+        x, w = whole(70, K, P + stages), whole(E * N * (1 if kind is None else 2), K, cfg + N).view(E, -1, K)
+        rows = torch.randint(0, 70, (P,), generator=torch.Generator().manual_seed(P)).to(torch.int32).cuda()
+        y = torch.cat([x[rows[int(seg[e]):int(seg[e + 1])].long()].float() @ w[e].float().T for e in range(E)])
+        want = y if kind is None else y[:, :N].clamp(min=0) * y[:, N:]
+        buf, out = out_of(P, N, shift)
+        ops.native().pgemm4_grouped(out.data_ptr(), x.data_ptr(), w.data_ptr(), 70, P, N, K, E, seg.data_ptr(), rows.data_ptr(),
+                                    K, cfg, 4, -1 if kind is None else kind, 0.0, 1.0, 0.0, -1)
+        assert torch.equal(out, want.to(torch.bfloat16)) and untouched(buf, P, N, shift), (sizes, N)
+
+
+@pytest.mark.parametrize("cfg", [0, 1, 3, 5, 6, 8])
+@pytest.mark.parametrize("K", [2048, 2112, 16384])
+def test_walks_over_k(cfg, K):
+    """Columns of tiles that start apart (up to 2048), XCDs of deep rows with several row tiles (from 16384): whole, split and gated."""
+    bp, bq = TILES[cfg]
+    M, N = 2 * bq + 5, 3 * bp + 8
+    x, w = whole(M, K, K), whole(N, K, N)
+    y = x.float() @ w.float().T                       # whole numbers below 2^24
+    assert torch.equal(ops.pgemm4(x, w, ops.EPI_F32, cfg=cfg), y)
+    assert torch.equal(ops.pgemm4(x, w, ops.EPI_F32, cfg=cfg, splits=4), y)
+    out = torch.empty(M, N // 2, dtype=torch.bfloat16, device="cuda")
+    ops.native().pgemm4_act(out.data_ptr(), x.data_ptr(), w.data_ptr(), M, N // 2, K, cfg, 4, sm.ACT_RELU, 0.0, 1.0, 0, -1)
+    assert torch.equal(out, (y[:, :N // 2].clamp(min=0) * y[:, N // 2:]).to(torch.bfloat16))
