@@ -7,7 +7,8 @@ from k8s_llm_scheduler_amd import ops
 from k8s_llm_scheduler_amd.ops import seqmix as sm
 
 pytestmark = pytest.mark.gpu
-TILES = {0: (256, 256), 1: (256, 128), 2: (128, 256), 3: (128, 128), 5: (128, 64), 6: (64, 64), 7: (224, 256), 8: (256, 192)}
+TILES = {0: (256, 256), 1: (256, 128), 2: (128, 256), 3: (128, 128), 5: (128, 64), 6: (64, 64), 7: (224, 256), 8: (256, 192), 9: (128, 96),
+         10: (192, 96), 11: (192, 128), 12: (128, 192), 13: (192, 192), 14: (224, 192), 15: (192, 224), 16: (224, 224), 17: (256, 224)}
 
 
 def whole(n, K, seed):
@@ -42,7 +43,7 @@ def test_stages_of_every_ring(cfg, stages):
             assert torch.equal(ops.pgemm4(x, w, ops.EPI_BF16, cfg=cfg, splits=3).float(), want), (M, N, "split")
 
 
-@pytest.mark.parametrize("cfg", [6, 7, 8])
+@pytest.mark.parametrize("cfg", [6, 7, 8, 9, 10, 13, 14, 16, 17])
 @pytest.mark.parametrize("K", [64, 448])
 def test_pairs_and_activations(cfg, K):
     """Gate and up rows of a feature in one fragment (224 rows) or in two; columns that do not fill the tile, a bias, split k."""
@@ -67,7 +68,7 @@ def test_pairs_and_activations(cfg, K):
 
 
 @pytest.mark.parametrize("sizes", [(1, 0, 3, 2, 7, 0, 5, 2), (64, 65, 0, 63, 1, 128, 200, 10), tuple([40] * 7 + [0, 3])])
-@pytest.mark.parametrize("cfg", [1, 6, 7, 8])
+@pytest.mark.parametrize("cfg", [1, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17])
 @pytest.mark.parametrize("kind", [None, sm.ACT_RELU])
 def test_groups_spread_over_k(sizes, cfg, kind, monkeypatch):
     """8 and more groups of few rows: every XCD at its own stage; gathered rows."""
@@ -85,7 +86,7 @@ def test_groups_spread_over_k(sizes, cfg, kind, monkeypatch):
     assert torch.equal(got, want.to(torch.bfloat16))
 
 
-@pytest.mark.parametrize("cfg,bp", [(9, 64), (10, 96), (11, 128), (12, 160)])
+@pytest.mark.parametrize("cfg,bp", [(18, 64), (19, 96), (20, 128), (21, 160)])
 @pytest.mark.parametrize("stages", [1, 2, 3, 5, 7, 32, 33])
 @pytest.mark.parametrize("kind", [None, sm.ACT_RELU])
 def test_groups_of_few_rows(cfg, bp, stages, kind):
@@ -105,7 +106,7 @@ def test_groups_of_few_rows(cfg, bp, stages, kind):
         assert torch.equal(out, want.to(torch.bfloat16)) and untouched(buf, P, N, shift), (sizes, N)
 
 
-@pytest.mark.parametrize("cfg", [0, 1, 3, 5, 6, 8])
+@pytest.mark.parametrize("cfg", [0, 1, 3, 5, 6, 8, 9, 10, 14])
 @pytest.mark.parametrize("K", [2048, 2112, 16384])
 def test_walks_over_k(cfg, K):
     """Columns of tiles that start apart (up to 2048), XCDs of deep rows with several row tiles (from 16384): whole, split and gated."""
