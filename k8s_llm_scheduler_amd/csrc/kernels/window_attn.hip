@@ -1036,11 +1036,15 @@ __global__ __launch_bounds__(512, 4) void window_prompt_kernel(
 // workgroup barrier: keys go from the cache straight into MFMA operands (a lane loads 8 dimensions of one key), values
 // through the wave's LDS rows for the transposing read; the 16 columns of the products are the group's heads (padded).  The
 // waves merge in LDS; one split writes the result, several leave (max, sum, unnormalised sum) for window_merge_kernel.
+// AHEAD: a tile's loads go out ahead of the softmax and the second product of the one before, at a sixth more registers; for few tokens,
+// whose workgroups have a CU each (16 heads over 4 of 128, 32 tokens behind up to 545 keys 15.7 -> 14.1 us, 1500 26.0 -> 24.9, 4 in splits
+// 10.2 -> 9.7; 32 over 8, 16 tokens 15.3 -> 13.6; 32 behind 1500 30.7 / 32.3 with it, 31.4 without).  Keys past the last repeat it, where skipping
+// them took a branch a load.
 // A tile is a chain of loads and LDS of 2.5 us, the merge's launch 4 us: 8 waves take the tiles of 512 keys in two rounds and
 // need no splits.  16 heads over 4 of 128, us, 4 waves with splits and their merge -> 8 waves: 32 tokens behind up to 545 keys
 // 17.5 -> 13.9, behind 100 10.0 -> 6.2, 64 behind 545 20.4 -> 14.8; with half the splits one token behind 1024 14.6 -> 12.5, 8
 // behind 1500 without a window 21.3 -> 15.3.  16 waves (no splits at all) do not fit 128 registers at 128 dimensions: 19.1.
-template <int DK, int NW>
+template <int DK, int NW, bool AHEAD>
 __global__ __launch_bounds__(64 * NW) void window_token_kernel(
     bf16_t* __restrict__ out, float* __restrict__ pacc, float* __restrict__ pml, const bf16_t* __restrict__ q, long ldq,
     const bf16_t* __restrict__ gate, long ldg, const bf16_t* __restrict__ kcache, const bf16_t* __restrict__ vcache,
@@ -1079,28 +1083,44 @@ __global__ __launch_bounds__(64 * NW) void window_token_kernel(
   for (int n = 0; n < NVB; ++n) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
   char* vl = vrows[wave];
   const int qd = li >> 2, pd = li & 3;
-  for (int tile = tile0 + wave; tile < tile1; tile += NW) {
-    const int j0 = lo + tile * 32;
-    int slot[2];                                  // cache slots of keys j0 + li and j0 + 16 + li
+  // keys past the last (the tile's rest) repeat it: their scores are masked, their values zeroed on the way to LDS
+  int slot[2];                                    // cache slots of keys 16 m + li of the tile that is loaded next
+  bf16x8 kf[2][NKK];
+  u32x4 vv[NV];
+  auto slots_of = [&](int tile) {
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
-      const int j = j0 + 16 * m + li;
-      slot[m] = j <= p ? (btr[j >> bshift] << bshift) + (j & bmask) : -1;
+      const int j = min(lo + tile * 32 + 16 * m + li, p);
+      slot[m] = (btr[j >> bshift] << bshift) + (j & bmask);
     }
-    bf16x8 kf[2][NKK];
+  };
+  auto load_k = [&]() {
 #pragma unroll
     for (int m = 0; m < 2; ++m)
 #pragma unroll
       for (int kk = 0; kk < NKK; ++kk)
-        kf[m][kk] = __builtin_bit_cast(
-            bf16x8, slot[m] >= 0 ? *reinterpret_cast<const u32x4*>(kcache + (size_t)slot[m] * GD + (size_t)g * DK + 32 * kk + 8 * g4)
-                                 : zero);
-    u32x4 vv[NV];
+        kf[m][kk] = *reinterpret_cast<const bf16x8*>(kcache + (size_t)slot[m] * GD + (size_t)g * DK + 32 * kk + 8 * g4);
+  };
+  auto load_v = [&]() {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int idx = lane + 64 * i, r = idx / C8, c = idx - r * C8;
       const int s0 = __shfl(slot[0], r & 15, WAVE), s1 = __shfl(slot[1], r & 15, WAVE), sv = r < 16 ? s0 : s1;
-      vv[i] = sv >= 0 ? *reinterpret_cast<const u32x4*>(vcache + (size_t)sv * GD + (size_t)g * DK + 8 * c) : zero;
+      vv[i] = *reinterpret_cast<const u32x4*>(vcache + (size_t)sv * GD + (size_t)g * DK + 8 * c);
+    }
+  };
+  if (AHEAD && tile0 + wave < tile1) {
+    slots_of(tile0 + wave);
+    load_k();
+    load_v();
+    slots_of(tile0 + wave + NW);
+  }
+  for (int tile = tile0 + wave; tile < tile1; tile += NW) {
+    const int j0 = lo + tile * 32;
+    if constexpr (!AHEAD) {
+      slots_of(tile);
+      load_k();
+      load_v();
     }
     f32x4 sacc[2];
 #pragma unroll
@@ -1113,7 +1133,12 @@ __global__ __launch_bounds__(64 * NW) void window_token_kernel(
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int idx = lane + 64 * i, r = idx / C8, c = idx - r * C8;
-      *reinterpret_cast<u32x4*>(vl + r * ROWV + 16 * c) = vv[i];
+      *reinterpret_cast<u32x4*>(vl + r * ROWV + 16 * c) = j0 + r <= p ? vv[i] : zero;
+    }
+    if (AHEAD && tile + NW < tile1) {             // the next tile is under way while this one is weighed and summed
+      load_k();
+      load_v();
+      slots_of(tile + 2 * NW);
     }
     float tmax = -INFINITY;
 #pragma unroll
@@ -1341,22 +1366,23 @@ extern "C" int k8s_window_token(void* out, float* pacc, float* pml, const void* 
   if (nsplit < 1 || nsplit > 64 || (nsplit > 1 && (pacc == nullptr || pml == nullptr))) return -1;
   int bshift = 0;
   while ((1 << bshift) < bs) ++bshift;
-#define K8S_WT(DK, NW)                                                                                                    \
-  window_token_kernel<DK, NW><<<dim3(T, G, nsplit), 64 * NW, 0, s>>>(                                                     \
+#define K8S_WT(DK, NW, AHEAD)                                                                                             \
+  window_token_kernel<DK, NW, AHEAD><<<dim3(T, G, nsplit), 64 * NW, 0, s>>>(                                              \
       (bf16_t*)out, pacc, pml, (const bf16_t*)q, ldq, (const bf16_t*)gate, ldg, (const bf16_t*)kcache,                    \
       (const bf16_t*)vcache, block_tables, max_blocks, tok_seq, positions, H, G, window, scale, sink, bshift, nsplit, chunk, \
       softcap, sinkv, gate_ph, slopes)
-#define K8S_WT_D(NW)                \
-  do {                              \
-    if (D == 64) K8S_WT(64, NW);    \
-    else if (D == 96) K8S_WT(96, NW); \
-    else K8S_WT(128, NW);           \
+#define K8S_WT_D(NW, AHEAD)                  \
+  do {                                       \
+    if (D == 64) K8S_WT(64, NW, AHEAD);      \
+    else if (D == 96) K8S_WT(96, NW, AHEAD); \
+    else K8S_WT(128, NW, AHEAD);             \
   } while (0)
   // 8 waves while every workgroup runs at once (two on a CU at 64 dimensions, one at more), else 4, of which two to four share a
   // CU.  16 heads over 4 of 128, us, 8 / 4 waves: 64 tokens behind 40 6.2 / 6.6, behind 1000 29 / 36; 66 9.6 / 7.1, 39 / 40; 128 10.4 /
   // 7.9, 53 / 50; of 64, 128 tokens 6.5 / 5.9, 28 / 31, 144 6.7 / 6.5, 35 / 34.  (T x G alone decides: the splits are made for it.)
-  if ((long)T * G <= (D == 64 ? 512 : 256)) K8S_WT_D(8);
-  else K8S_WT_D(4);
+  if ((long)T * G <= (nsplit > 1 ? 64 : 128)) K8S_WT_D(8, true);
+  else if ((long)T * G <= (D == 64 ? 512 : 256)) K8S_WT_D(8, false);
+  else K8S_WT_D(4, false);
 #undef K8S_WT_D
 #undef K8S_WT
   if (nsplit > 1)
