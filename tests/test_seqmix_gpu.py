@@ -788,6 +788,30 @@ def test_decay_scan(dt, H, G, D, V):
         close(s2, sc, 1e-5)
 
 
+@pytest.mark.parametrize("lens", [(64, 63, 1, 0), (33, 32, 17, 16), (15, 48, 49, 64), (65, 130, 2, 64)])
+@pytest.mark.parametrize("H,G,D,V", [(4, 2, 16, 24), (2, 1, 128, 128), (2, 2, 8, 248), (3, 3, 72, 80), (1, 1, 128, 64)])
+def test_decay_scan_of_one_launch(H, G, D, V, lens):
+    """Portions said to be of at most 64 tokens are walked by one kernel, longer ones by three: the same products of the
+    same terms, so equal outputs within the first chunk; the new states differ by the order of fp32 sums (64 terms), and what
+    follows from them by that and their two bf16 terms (16 bits).  A portion longer than said is walked to its end."""
+    torch.manual_seed(63)
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32)
+    pos = torch.cat([torch.arange(p, p + n) for p, n in zip((0, 5, 0, 130), lens)]).int()
+    slots = torch.tensor([2, 0, 1, 3], dtype=torch.int32)
+    proj, cols, decay, state = _decay_case(torch.bfloat16, H, G, D, V, cu, pos)
+    out, new = {}, {}
+    for most in (64, max(65, *lens)):
+        new[most] = state.to(DEV).clone()
+        out[most] = sm.gated_scan(proj.to(DEV), sm.SCAN_DECAY, cols, None, new[most], cu.to(DEV), slots.to(DEV), pos.to(DEV),
+                                  H, D, V, 1e-6, torch.float32, head_params=decay.to(DEV), groups=G, max_qlen=most)
+    (a, b), (s, t) = out.values(), new.values()
+    for i, n in enumerate(lens):
+        r = slice(int(cu[i]), int(cu[i]) + min(n, 64))
+        assert torch.equal(a[r], b[r])
+    assert (a - b).abs().max() <= 2 ** -14 * b.abs().max()
+    assert (s - t).abs().max() <= 64 * 2 ** -24 * t.abs().max()
+
+
 @pytest.mark.parametrize("lens", [(9, 1, 0, 27), (64, 65, 63, 1), (200, 0, 128, 7), (2, 2, 2, 2), (600, 1, 1, 0)])
 @pytest.mark.parametrize("H,G,D,V", [(4, 2, 16, 24), (3, 3, 40, 56), (2, 1, 128, 128), (6, 3, 64, 8), (2, 2, 8, 248),
                                      (1, 1, 96, 160), (5, 5, 32, 64), (3, 3, 72, 80)])
