@@ -242,8 +242,8 @@ __global__ void __launch_bounds__(NW * 64) decode_fused_kernel(
       m = fmaxf(m, v);
     }
   }
-  m = fmaxf(m, __shfl_xor(m, 16, WAVE));
-  m = fmaxf(m, __shfl_xor(m, 32, WAVE));
+  m = lane_max<16>(m);
+  m = lane_max<32>(m);
   if (g4 == 0) wm[wid][li] = m;
   __syncthreads();
   float M = -INFINITY;
@@ -259,8 +259,8 @@ __global__ void __launch_bounds__(NW * 64) decode_fused_kernel(
       l += e;
     }
   }
-  l += __shfl_xor(l, 16, WAVE);
-  l += __shfl_xor(l, 32, WAVE);
+  l = lane_sum<16>(l);
+  l = lane_sum<32>(l);
   if (g4 == 0) wl[wid][li] = l;
 
   // ---- O = P . V over 32-key steps; V staged per wave in LDS (swizzled 16-byte chunks)
@@ -529,8 +529,8 @@ __global__ void __launch_bounds__(512) decode_prefix_kernel(
         sacc[t][i] *= qscale;
         mloc = fmaxf(mloc, sacc[t][i]);
       }
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 16, WAVE));
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 32, WAVE));
+    mloc = lane_max<16>(mloc);
+    mloc = lane_max<32>(mloc);
     const float m_new = fmaxf(m_run, mloc);
     const float alpha = exp2f(m_run - m_new);   // (0 on the first span: m_run = -inf)
     float lsum = 0.f;
@@ -542,8 +542,8 @@ __global__ void __launch_bounds__(512) decode_prefix_kernel(
         sacc[t][i] = e;
         lsum += e;
       }
-    lsum += __shfl_xor(lsum, 16, WAVE);
-    lsum += __shfl_xor(lsum, 32, WAVE);
+    lsum = lane_sum<16>(lsum);
+    lsum = lane_sum<32>(lsum);
     l_run = l_run * alpha + lsum;
     m_run = m_new;
     // o[nn][i] holds column 4 g4 + i: its rescale factor lives in lane 4 g4 + i (g4 = 0 there, li = the column)

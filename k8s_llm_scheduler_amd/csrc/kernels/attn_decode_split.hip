@@ -209,8 +209,8 @@ __device__ __forceinline__ void split_body(
       m = fmaxf(m, v);
     }
   }
-  m = fmaxf(m, __shfl_xor(m, 16, WAVE));
-  m = fmaxf(m, __shfl_xor(m, 32, WAVE));  // max of head li over the chunk (n >= 1: finite)
+  m = lane_max<16>(m);
+  m = lane_max<32>(m);  // max of head li over the chunk (n >= 1: finite)
   float l = 0.f;
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
@@ -221,8 +221,8 @@ __device__ __forceinline__ void split_body(
       l += e;
     }
   }
-  l += __shfl_xor(l, 16, WAVE);
-  l += __shfl_xor(l, 32, WAVE);
+  l = lane_sum<16>(l);
+  l = lane_sum<32>(l);
   TR(3);
 
   // ---- O = P . V over two 32-key steps.  The V image has landed (the K wait above drained the

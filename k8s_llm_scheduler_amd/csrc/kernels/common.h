@@ -2,6 +2,7 @@
 // Wave = 64 lanes everywhere; bf16 tensors are moved as 16-byte vectors (8 x bf16).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <type_traits>
 #include <stdint.h>
 
 namespace k8sllm {
@@ -35,17 +36,56 @@ template <typename T> __device__ __forceinline__ void stf(T* p, size_t i, float 
 template <> __device__ __forceinline__ void stf<float>(float* p, size_t i, float v) { p[i] = v; }
 template <> __device__ __forceinline__ void stf<bf16_t>(bf16_t* p, size_t i, float v) { p[i] = f2bf(v); }
 
-template <typename T>
-__device__ __forceinline__ T wave_sum(T v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-  return v;
+// The value of lane ^ O, and sums and maxima over the two, by register moves: a shuffle goes through LDS and its address
+// (a wave sum in a chain of them 187 -> 55 ns).  Every lane of the wave takes part.  Same operands as by shuffles, so the same results.
+template <int O>
+__device__ __forceinline__ float lane_xor(float v) {
+  static_assert(O == 1 || O == 2 || O == 4 || O == 8, "within rows of 16 lanes");
+  const auto move = [](float x, auto ctrl) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), decltype(ctrl)::value, 0xF, 0xF, true));
+  };
+  if constexpr (O == 1) return move(v, std::integral_constant<int, 0xB1>{});          // quad_perm 1 0 3 2
+  else if constexpr (O == 2) return move(v, std::integral_constant<int, 0x4E>{});     // quad_perm 2 3 0 1
+  else if constexpr (O == 8) return move(v, std::integral_constant<int, 0x128>{});    // row_ror 8
+  else return move(move(v, std::integral_constant<int, 0x141>{}), std::integral_constant<int, 0x1B>{});  // mirrored in 8, then in 4
 }
-template <typename T>
-__device__ __forceinline__ T wave_max(T v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, WAVE));
-  return v;
+// (a of the lanes without bit O, b of those with it) and the same of lane ^ O: the two halves exchange the other's operand
+template <int O>
+__device__ __forceinline__ void lane_swap(float a, float b, float& x, float& y) {
+  static_assert(O == 16 || O == 32, "rows of 16 lanes");
+  if constexpr (O == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    x = __uint_as_float(r[0]), y = __uint_as_float(r[1]);
+  } else {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    x = __uint_as_float(r[0]), y = __uint_as_float(r[1]);
+  }
+}
+template <int O>
+__device__ __forceinline__ float lane_sum(float v) {
+  if constexpr (O >= 16) {
+    float x, y;
+    lane_swap<O>(v, v, x, y);
+    return x + y;
+  } else {
+    return v + lane_xor<O>(v);
+  }
+}
+template <int O>
+__device__ __forceinline__ float lane_max(float v) {
+  if constexpr (O >= 16) {
+    float x, y;
+    lane_swap<O>(v, v, x, y);
+    return fmaxf(x, y);
+  } else {
+    return fmaxf(v, lane_xor<O>(v));
+  }
+}
+__device__ __forceinline__ float wave_sum(float v) {
+  return lane_sum<1>(lane_sum<2>(lane_sum<4>(lane_sum<8>(lane_sum<16>(lane_sum<32>(v))))));
+}
+__device__ __forceinline__ float wave_max(float v) {
+  return lane_max<1>(lane_max<2>(lane_max<4>(lane_max<8>(lane_max<16>(lane_max<32>(v))))));
 }
 
 // OCP MX e4m3 (K16 block-scaled activations; fp8.hip has the format): one E8M0 byte per 32 values, the smallest
@@ -76,9 +116,7 @@ __device__ __forceinline__ size_t mx_scale_off(size_t m, int kb, int M) {
 // MX store of one value per lane, the 32 lanes of an aligned half-wave holding one block (row m, columns col..,
 // col of the half-wave's first lane a multiple of 32): shuffle max, then one e4m3 byte per lane and the block's E8M0.
 __device__ __forceinline__ void mx_store_lane(uint8_t* oq, uint8_t* oe, size_t m, int col, int K, int M, float v) {
-  float amax = fabsf(v);
-#pragma unroll
-  for (int o = 1; o < 32; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+  const float amax = lane_max<16>(lane_max<8>(lane_max<4>(lane_max<2>(lane_max<1>(fabsf(v))))));
   const uint32_t e = mx_e8m0(amax);
   oq[m * (size_t)K + col] = (uint8_t)(mx_pack4(v, 0.f, 0.f, 0.f, mx_inv_scale(e)) & 0xffu);
   if ((col & 31) == 0) oe[mx_scale_off(m, col >> 5, M)] = (uint8_t)e;

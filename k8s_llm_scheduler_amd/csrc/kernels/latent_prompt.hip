@@ -223,8 +223,8 @@ __global__ __launch_bounds__(512) void latent_prompt_kernel(
         }
         float tmax = fmaxf(fmaxf(fmaxf(sacc[cb][0][0], sacc[cb][0][1]), fmaxf(sacc[cb][0][2], sacc[cb][0][3])),
                            fmaxf(fmaxf(sacc[cb][1][0], sacc[cb][1][1]), fmaxf(sacc[cb][1][2], sacc[cb][1][3])));
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
+        tmax = lane_max<16>(tmax);
+        tmax = lane_max<32>(tmax);
         if (__any(tmax > m_run[cb])) {
           const float m_new = fmaxf(m_run[cb], tmax);
           const float alpha = m_run[cb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[cb] - m_new);
@@ -271,8 +271,8 @@ __global__ __launch_bounds__(512) void latent_prompt_kernel(
   // o[cb][n][i] = O[column 4 g4 + i][d 16 n + li]; m_run, l_run belong to column li.  Group 1 leaves its part in LDS.
 #pragma unroll
   for (int cb = 0; cb < NCB; ++cb) {
-    l_run[cb] += __shfl_xor(l_run[cb], 16, WAVE);
-    l_run[cb] += __shfl_xor(l_run[cb], 32, WAVE);
+    l_run[cb] = lane_sum<16>(l_run[cb]);
+    l_run[cb] = lane_sum<32>(l_run[cb]);
   }
   float* mo = reinterpret_cast<float*>(smem_p) + (size_t)wave * 64 * NCB * (4 * NVB + 2);   // [NCB (4 NVB + 2)][64 lanes]
   if (grp == 1) {
@@ -404,8 +404,8 @@ __global__ __launch_bounds__(256) void latent_prompt_f32_kernel(
         s[m][i] = key <= p && key >= lo ? s[m][i] * scale : -INFINITY;
         tmax = fmaxf(tmax, s[m][i]);
       }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
+    tmax = lane_max<16>(tmax);
+    tmax = lane_max<32>(tmax);
     const float m_new = fmaxf(m_run, tmax);
     const float alpha = m_run == -INFINITY ? 0.f : expf(m_run - m_new);
     const float m_ref = m_new == -INFINITY ? 0.f : m_new;      // a token that has seen nothing yet
@@ -430,8 +430,8 @@ __global__ __launch_bounds__(256) void latent_prompt_f32_kernel(
     }
   }
   if (!ok) return;
-  l_run += __shfl_xor(l_run, 16, WAVE);
-  l_run += __shfl_xor(l_run, 32, WAVE);
+  l_run = lane_sum<16>(l_run);
+  l_run = lane_sum<32>(l_run);
   float f = 1.f / l_run;
   if (gate != nullptr) f /= 1.f + expf(-gate[(size_t)(tq0 + toff) * ldg + hd]);
 #pragma unroll

@@ -90,8 +90,8 @@ __global__ __launch_bounds__(256) void latent_token_kernel(
       s[i] = j0 + i <= p ? s[i] * scale : -INFINITY;
       tmax = fmaxf(tmax, s[i]);
     }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
+    tmax = lane_max<16>(tmax);
+    tmax = lane_max<32>(tmax);
     if (g == 0) wm[16 * wave + li] = tmax;
     lds_barrier();
     const float m_new = fmaxf(fmaxf(fmaxf(wm[li], wm[16 + li]), fmaxf(wm[32 + li], wm[48 + li])), m_run);   // finite
@@ -142,8 +142,8 @@ __global__ __launch_bounds__(256) void latent_token_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       pacc[(rec0 + (size_t)(4 * g + i) * nsplit) * C + (C / 4) * wave + 16 * n + li] = o[n][i];
-  l_run += __shfl_xor(l_run, 16, WAVE);
-  l_run += __shfl_xor(l_run, 32, WAVE);
+  l_run = lane_sum<16>(l_run);
+  l_run = lane_sum<32>(l_run);
   __syncthreads();
   if (g == 0) wm[16 * wave + li] = l_run;
   __syncthreads();

@@ -374,8 +374,8 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) mgemm_kernel(MgArgs a) {
     if (do_rms) {
 #pragma unroll
       for (int j = 0; j < FM; ++j) {
-        ss[j] += __shfl_xor(ss[j], 16, WAVE);
-        ss[j] += __shfl_xor(ss[j], 32, WAVE);
+        ss[j] = lane_sum<16>(ss[j]);
+        ss[j] = lane_sum<32>(ss[j]);
       }
       if (g == 0) {
 #pragma unroll
@@ -524,8 +524,8 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) mgemm_kernel(MgArgs a) {
           }
           am[j] = fmaxf(am[j], fabsf(v[j][i]));
         }
-        am[j] = fmaxf(am[j], __shfl_xor(am[j], 16, WAVE));
-        am[j] = fmaxf(am[j], __shfl_xor(am[j], 32, WAVE));
+        am[j] = lane_max<16>(am[j]);
+        am[j] = lane_max<32>(am[j]);
         xpair[wn * BM + wm * (BM / WM) + j * 16 + li] = am[j];
       }
       mg_barrier();
@@ -567,8 +567,8 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) mgemm_kernel(MgArgs a) {
           float amax = 0.f;
 #pragma unroll
           for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
-          amax = fmaxf(amax, __shfl_xor(amax, 16, WAVE));
-          amax = fmaxf(amax, __shfl_xor(amax, 32, WAVE));
+          amax = lane_max<16>(amax);
+          amax = lane_max<32>(amax);
           const uint32_t e = mx_e8m0(amax);
           const float inv = mx_inv_scale(e);
           uint8_t* orow = a.oq + (long long)m * a.N_out;
@@ -605,8 +605,8 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) mgemm_kernel(MgArgs a) {
           float amax = 0.f;
 #pragma unroll
           for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
-          amax = fmaxf(amax, __shfl_xor(amax, 16, WAVE));
-          amax = fmaxf(amax, __shfl_xor(amax, 32, WAVE));
+          amax = lane_max<16>(amax);
+          amax = lane_max<32>(amax);
           const uint32_t e = mx_e8m0(amax);
           const float inv = mx_inv_scale(e);
           uint8_t* orow = a.oq + (long long)m * a.N_out;

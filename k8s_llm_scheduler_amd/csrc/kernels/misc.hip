@@ -27,8 +27,8 @@ __global__ void embedding_kernel(bf16_t* __restrict__ out, const int* __restrict
         f[2 * j + 1] = hi_bf(v[j]);
         amax = fmaxf(amax, fmaxf(fabsf(f[2 * j]), fabsf(f[2 * j + 1])));
       }
-      amax = fmaxf(amax, __shfl_xor(amax, 1, WAVE));
-      amax = fmaxf(amax, __shfl_xor(amax, 2, WAVE));
+      amax = lane_max<1>(amax);
+      amax = lane_max<2>(amax);
       const uint32_t e = mx_e8m0(amax);
       const float inv = mx_inv_scale(e);
       uint32_t* q = reinterpret_cast<uint32_t*>(oq + (size_t)t * H + (size_t)i * 8);

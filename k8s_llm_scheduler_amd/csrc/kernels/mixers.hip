@@ -419,9 +419,7 @@ __global__ __launch_bounds__(256, 4) void wkv_chunk_out_kernel(TA* __restrict__ 
 #pragma unroll
     for (int x = 0; x < TW; ++x) own[x] = row_sum(rx[x] * (ui * kx[x]));
 #pragma unroll
-    for (int m = 32; m > 8; m >>= 1)
-#pragma unroll
-      for (int x = 0; x < TW; ++x) own[x] += __shfl_xor(own[x], m, WAVE);
+    for (int x = 0; x < TW; ++x) own[x] = lane_sum<16>(lane_sum<32>(own[x]));
     const bool all = __all(fin);
     if (lane == 0) odd[wave] = !all;
     if (t0 + TB < b) fetch(t0 + TB);
@@ -876,8 +874,8 @@ __global__ __launch_bounds__(64 * NWV) void latent_attention_mfma_kernel(
         sacc[m][i] = v;
         tmax = fmaxf(tmax, v);
       }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
+    tmax = lane_max<16>(tmax);
+    tmax = lane_max<32>(tmax);
     const float m_new = fmaxf(m_run, tmax);       // finite: the step holds a visible key
     const float alpha = m_run == -INFINITY ? 0.f : __expf(m_run - m_new);
     float rsum = 0.f;
@@ -889,8 +887,8 @@ __global__ __launch_bounds__(64 * NWV) void latent_attention_mfma_kernel(
         sacc[m][i] = pv;
         rsum += pv;
       }
-    rsum += __shfl_xor(rsum, 16, WAVE);
-    rsum += __shfl_xor(rsum, 32, WAVE);
+    rsum = lane_sum<16>(rsum);
+    rsum = lane_sum<32>(rsum);
     l_run = l_run * alpha + rsum;
     m_run = m_new;
     // the running maxima settle after the first steps: the accumulators are rescaled only when some head's moved

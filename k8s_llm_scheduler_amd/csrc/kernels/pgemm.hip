@@ -427,8 +427,8 @@ __global__ void __launch_bounds__(512) pgemm_kernel(PgArgs a) {
   if constexpr (RMS) {
 #pragma unroll
     for (int f = 0; f < FQ; ++f) {
-      ss[f] += __shfl_xor(ss[f], 16, WAVE);
-      ss[f] += __shfl_xor(ss[f], 32, WAVE);
+      ss[f] = lane_sum<16>(ss[f]);
+      ss[f] = lane_sum<32>(ss[f]);
     }
     if (g == 0) {
 #pragma unroll
@@ -548,8 +548,8 @@ __global__ void __launch_bounds__(512) pgemm_kernel(PgArgs a) {
         float amax = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
-        amax = fmaxf(amax, __shfl_xor(amax, 16, WAVE));
-        amax = fmaxf(amax, __shfl_xor(amax, 32, WAVE));
+        amax = lane_max<16>(amax);
+        amax = lane_max<32>(amax);
         const uint32_t e = mx_e8m0(amax);
         const float inv = mx_inv_scale(e);
         uint8_t* orow = a.oq + (size_t)m * a.N_out;

@@ -50,9 +50,9 @@ __global__ void __launch_bounds__(256) pgemm_reduce_kernel(void* __restrict__ ou
   }
   if constexpr (MXO) {
     float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-    amax = fmaxf(amax, __shfl_xor(amax, 1, WAVE));
-    amax = fmaxf(amax, __shfl_xor(amax, 2, WAVE));
-    amax = fmaxf(amax, __shfl_xor(amax, 4, WAVE));
+    amax = lane_max<1>(amax);
+    amax = lane_max<2>(amax);
+    amax = lane_max<4>(amax);
     const uint32_t e = mx_e8m0(amax);
     *reinterpret_cast<uint32_t*>(oq + (size_t)m * N_out + n0) = mx_pack4(v[0], v[1], v[2], v[3], mx_inv_scale(e));
     if ((n0 & 31) == 0) oe[mx_scale_off(m, n0 >> 5, M)] = (uint8_t)e;

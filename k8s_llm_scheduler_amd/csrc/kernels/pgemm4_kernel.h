@@ -397,8 +397,8 @@ __global__ void __launch_bounds__(256, 1) pgemm4_kernel(P4Args a) {
     __syncthreads();                                     // rss lies in the last stage's memory
 #pragma unroll
     for (int f = 0; f < FQ; ++f) {
-      ss[f] += __shfl_xor(ss[f], 16, WAVE);
-      ss[f] += __shfl_xor(ss[f], 32, WAVE);
+      ss[f] = lane_sum<16>(ss[f]);
+      ss[f] = lane_sum<32>(ss[f]);
     }
     if (g == 0) {
 #pragma unroll

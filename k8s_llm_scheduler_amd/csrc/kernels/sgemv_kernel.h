@@ -32,20 +32,26 @@ __device__ __forceinline__ float sg_dot8(const u32x4& w, const u32x4& x, float a
 // (the lower half if bit O of its lane id is clear) and adds the partner's copy of that half.  Once one value is
 // left, the remaining offsets are plain xor sums.  Afterwards value index (lane >> (6 - log2 V)) & (V - 1) of the
 // ORIGINAL V values is the wave total in v[0] of every lane (all lanes of a group agree).
+template <int O>
+__device__ __forceinline__ float sg_keep(float a, float b, int lane) {   // lanes without bit O: a, the others: b, of both lanes
+  if constexpr (O >= 16) {
+    float x, y;
+    lane_swap<O>(a, b, x, y);
+    return x + y;
+  } else {
+    const bool up = (lane & O) != 0;
+    return (up ? b : a) + lane_xor<O>(up ? a : b);
+  }
+}
 template <int CNT, int O>
 __device__ __forceinline__ void sg_halve(float* v, int lane) {
   if constexpr (O >= 1) {
     if constexpr (CNT > 1) {
-      const bool up = (lane & O) != 0;
 #pragma unroll
-      for (int i = 0; i < CNT / 2; ++i) {
-        const float give = up ? v[i] : v[i + CNT / 2];
-        const float keep = up ? v[i + CNT / 2] : v[i];
-        v[i] = keep + __shfl_xor(give, O, WAVE);
-      }
+      for (int i = 0; i < CNT / 2; ++i) v[i] = sg_keep<O>(v[i], v[i + CNT / 2], lane);
       sg_halve<CNT / 2, O / 2>(v, lane);
     } else {
-      v[0] += __shfl_xor(v[0], O, WAVE);
+      v[0] = lane_sum<O>(v[0]);
       sg_halve<1, O / 2>(v, lane);
     }
   }
@@ -282,16 +288,11 @@ template <int CNT, int O>
 __device__ __forceinline__ void sm_halve(float* v, int lane) {   // sg_halve that stops at offset 4 (j = lane & 3)
   if constexpr (O >= 4) {
     if constexpr (CNT > 1) {
-      const bool up = (lane & O) != 0;
 #pragma unroll
-      for (int i = 0; i < CNT / 2; ++i) {
-        const float give = up ? v[i] : v[i + CNT / 2];
-        const float keep = up ? v[i + CNT / 2] : v[i];
-        v[i] = keep + __shfl_xor(give, O, WAVE);
-      }
+      for (int i = 0; i < CNT / 2; ++i) v[i] = sg_keep<O>(v[i], v[i + CNT / 2], lane);
       sm_halve<CNT / 2, O / 2>(v, lane);
     } else {
-      v[0] += __shfl_xor(v[0], O, WAVE);
+      v[0] = lane_sum<O>(v[0]);
       sm_halve<1, O / 2>(v, lane);
     }
   }
@@ -481,9 +482,7 @@ __global__ void __launch_bounds__(512) smfma_kernel(void* __restrict__ out, floa
             const float lo = lo_bf(xr[s][xg][v][e]), hi = hi_bf(xr[s][xg][v][e]);
             t += lo * lo + hi * hi;
           }
-#pragma unroll
-      for (int o = 4; o < 64; o <<= 1) t += __shfl_xor(t, o, WAVE);
-      ss[xg] = t;
+      ss[xg] = lane_sum<32>(lane_sum<16>(lane_sum<8>(lane_sum<4>(t))));
     }
     if (lane < 4) {
 #pragma unroll

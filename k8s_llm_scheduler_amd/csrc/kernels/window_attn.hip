@@ -653,8 +653,8 @@ __global__ __launch_bounds__(256) void window_attention_mfma_kernel(
           sacc[cb][m][i] = v;
           tmax = fmaxf(tmax, v);
         }
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
+      tmax = lane_max<16>(tmax);
+      tmax = lane_max<32>(tmax);
       const float m_new = fmaxf(m_run[cb], tmax);
       const float m_ref = m_new == -INFINITY ? 0.f : m_new;      // a column that has seen nothing yet
       const float alpha = m_run[cb] == -INFINITY ? 0.f : expf(m_run[cb] - m_ref);
@@ -667,8 +667,8 @@ __global__ __launch_bounds__(256) void window_attention_mfma_kernel(
           sacc[cb][m][i] = pv;
           rsum += pv;
         }
-      rsum += __shfl_xor(rsum, 16, WAVE);
-      rsum += __shfl_xor(rsum, 32, WAVE);
+      rsum = lane_sum<16>(rsum);
+      rsum = lane_sum<32>(rsum);
       l_run[cb] = l_run[cb] * alpha + rsum;
       m_run[cb] = m_new;
 #pragma unroll
@@ -921,8 +921,8 @@ __global__ __launch_bounds__(512, 4) void window_prompt_kernel(
         }
         float tmax = fmaxf(fmaxf(fmaxf(sacc[cb][0][0], sacc[cb][0][1]), fmaxf(sacc[cb][0][2], sacc[cb][0][3])),
                            fmaxf(fmaxf(sacc[cb][1][0], sacc[cb][1][1]), fmaxf(sacc[cb][1][2], sacc[cb][1][3])));
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
+        tmax = lane_max<16>(tmax);
+        tmax = lane_max<32>(tmax);
         if (__any(tmax > m_run[cb])) {
           const float m_new = fmaxf(m_run[cb], tmax);
           const float alpha = m_run[cb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[cb] - m_new);
@@ -974,8 +974,8 @@ __global__ __launch_bounds__(512, 4) void window_prompt_kernel(
   // o[cb][n][i] = O[column 4 g4 + i][d 16 n + li]; m_run, l_run belong to column li.  Group 1 leaves its part in LDS.
 #pragma unroll
   for (int cb = 0; cb < NCB; ++cb) {
-    l_run[cb] += __shfl_xor(l_run[cb], 16, WAVE);
-    l_run[cb] += __shfl_xor(l_run[cb], 32, WAVE);
+    l_run[cb] = lane_sum<16>(l_run[cb]);
+    l_run[cb] = lane_sum<32>(l_run[cb]);
   }
   float* mo = reinterpret_cast<float*>(smem_p) + (size_t)wave * 64 * NCB * (4 * NVB + 2);   // [NCB (4 NVB + 2)][64 lanes]
   if (grp == 1) {
@@ -1151,8 +1151,8 @@ __global__ __launch_bounds__(64 * NW) void window_token_kernel(
         sacc[m][i] = v;
         tmax = fmaxf(tmax, v);
       }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
+    tmax = lane_max<16>(tmax);
+    tmax = lane_max<32>(tmax);
     const float m_new = fmaxf(m_run, tmax);       // finite: the tile's first key is seen
     const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
     m_run = m_new;
@@ -1186,8 +1186,8 @@ __global__ __launch_bounds__(64 * NW) void window_token_kernel(
       o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl, vb, o[n], 0, 0, 0);
     }
   }
-  l_run += __shfl_xor(l_run, 16, WAVE);
-  l_run += __shfl_xor(l_run, 32, WAVE);
+  l_run = lane_sum<16>(l_run);
+  l_run = lane_sum<32>(l_run);
   if (g4 == 0) {
     ml[wave][li][0] = m_run;
     ml[wave][li][1] = l_run;
