@@ -185,6 +185,9 @@ int k8s_gemm_f32_tiles(void* C, const float* A, const float* W, int M, int N, in
                        long sA, long sW, long sC, const int* a_rows, const int* tiles, int ntiles, int out_f32, int fq,
                        hipStream_t s);
 int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles);
+int k8s_gemm_f32_parts(float* C, const float* A, const float* W, int M, int N, int K, long lda, long ldw, long ldc, int batch,
+                       long sA, long sW, long sC, const int* a_rows, const int* tiles, int ntiles, int tile, hipStream_t s);
+int k8s_gemm_f32_parts_rule(int M, int N, int K, int batch, int ntiles);
 int k8s_gemm_any(void* C, const void* A, const void* W, int M, int N, int K, long lda, long ldw, long ldc, int batch,
                  long sA, long sW, long sC, const int* a_rows, const int* tiles, int ntiles, int in_f32, int out_f32,
                  hipStream_t s);
@@ -700,6 +703,12 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
     check(k8s_gemm_f32_tiles(P(C), P<float>(A), P<float>(W), M, N, K, lda, ldw, ldc, batch, sA, sW, sC, P<int>(a_rows),
                              P<int>(tiles), ntiles, out_f32, fq, S(s)), "gemm_f32_tiles");
   });
+  m.def("gemm_f32_parts", [](uintptr_t C, uintptr_t A, uintptr_t W, int M, int N, int K, long lda, long ldw, long ldc,
+                             int batch, long sA, long sW, long sC, uintptr_t a_rows, uintptr_t tiles, int ntiles, int tile, intptr_t s) {
+    check(k8s_gemm_f32_parts(P<float>(C), P<float>(A), P<float>(W), M, N, K, lda, ldw, ldc, batch, sA, sW, sC, P<int>(a_rows),
+                             P<int>(tiles), ntiles, tile, S(s)), "gemm_f32_parts");
+  });
+  m.def("gemm_f32_parts_rule", [](int M, int N, int K, int batch, int ntiles) { return k8s_gemm_f32_parts_rule(M, N, K, batch, ntiles); });
   m.def("gemm_f32_rule", [](int M, int N, int K, int batch, int ntiles) { return k8s_gemm_f32_rule(M, N, K, batch, ntiles); });
   m.def("gemm_any", [](uintptr_t C, uintptr_t A, uintptr_t W, int M, int N, int K, long lda, long ldw, long ldc,
                        int batch, long sA, long sW, long sC, uintptr_t a_rows, uintptr_t tiles, int ntiles, int in_f32,

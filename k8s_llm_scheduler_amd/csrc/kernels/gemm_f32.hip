@@ -352,7 +352,8 @@ using namespace k8sllm;
 // part.  By the first fit / this one: 457 x 6720 x 4096 276 / 255, 441 x 3072 x 1536 50 / 47, 384 x 3648 x 2048 58.0 / 56.8, 393 x 14336 x
 // 4096 429 / 417; without the two exceptions 401 x 6144 x 4096 195 / 182, 352 x 7168 x 4096 195 / 183.  K < 512: shares of K / 8 leave the
 // smaller error.
-extern "C" int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles) {
+static int f32_rule(int M, int N, int K, int batch, int ntiles, double* cost) {
+  *cost = 0.0;
   if (K < 512 || K % 32 || M <= 0 || N <= 0) return 0;
   // Listed tiles: most of the list is short of 64 rows or empty, and where its blocks meet on a CU is left to chance, so the parts
   // below do not hold.  From 32 rows a group on (the list has one tile a group more than the rows fill) 32-row tiles, where the
@@ -375,7 +376,12 @@ extern "C" int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles) {
   // 17 rows 18.5 / 19.6, 2048 x 8192 61.5 / 68.7, 4096 x 14336 124 / 120; 24 rows 20.0 / 19.7, 67.1 / 68.7, 129 / 121; 32 rows
   // 20.8 / 19.8, 70.1 / 68.7.
   const long cols = (long)N * batch;
-  if (r1 == 1.0 && M <= 32 && (M <= 4 ? cols > 256 : M <= 16 || M > 24 || cols > 2048)) return 0;
+  // us, from the fitted parts: a constant, so much of the parts, and a share of what the weights take
+  const auto us = [&](double c, double parts, double weights) { *cost = c + parts * K / 32.0 + weights * 4e-6 * cols * (double)K; };
+  if (r1 == 1.0 && M <= 32 && (M <= 4 ? cols > 256 : M <= 16 || M > 24 || cols > 2048)) {
+    us(3.0, 0.787 * 0.26, 0.101);
+    return 0;
+  }
   double best = 2.0 * r2 < 1.1 * r1 ? 0.365 * r2 + 0.03 : 0.16 * r1 + 0.1;
   int pick = 0;
   for (int fq = 8; fq >= 1; --fq) {
@@ -391,6 +397,8 @@ extern "C" int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles) {
       pick = 16 + fq;
     }
   }
+  if (pick == 0) us(2.1, 1.052 * best, 0.156);
+  else if (pick > 16) us(0.0, 1.044 * best, 0.078);
   if (pick == 0 || pick > 16) return pick;
   best = 1e30;
   for (int fq = 8; fq >= 1; --fq) {
@@ -401,7 +409,20 @@ extern "C" int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles) {
       pick = fq;
     }
   }
+  us(4.1, 1.108 * best, 0.039);
   return pick;
+}
+
+extern "C" int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles) {
+  double cost;
+  return f32_rule(M, N, K, batch, ntiles, &cost);
+}
+
+// What a product of K >= 512 takes on the fp32 pipes by that choice, us (fitted to M 1 - 512, N 128 - 32768, K 512 - 14336; rms error 3 - 8 %)
+extern "C" double k8s_gemm_f32_cost(int M, int N, int K, int batch) {
+  double cost;
+  f32_rule(M, N, K, batch, 0, &cost);
+  return cost;
 }
 
 // fq: rows of a tile / 16 (1 - 8; listed tiles of at most 64 rows: 1, 2, 4), or 16 + that (1 - 4): k shared by the waves.

@@ -688,7 +688,7 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(TO* __restrict__ C, const
 // give every SIMD two waves.  A lane reads 4 consecutive k of its row and spends one on each of 4 instructions.  PF steps'
 // loads are in flight.  The waves' sums meet in LDS in wave order: an output's accumulation order depends on K alone, not on
 // the tile or the rows that share it.  Same three forms.
-// It takes what k8s_gemm_f32_rule leaves it: few rows, few tiles, short listed groups, depths below 512 or no multiple of 32; the rest
+// It takes what k8s_gemm_f32_parts_rule and k8s_gemm_f32_rule leave it: few rows, few tiles, short listed groups, depths below 512 or no multiple of 32; the rest
 // runs on gemm_f32.hip's tiles.  Bound by the loads of weights that no other workgroup reads (16 rows, from memory: 2048 x 2048
 // (N x K) 19.6 us, 4096 x 14336 120 us), and with many rows by the fp32 matrix rate (157 TFLOP/s; a 32 x 32 x 2048 tile is 7 us of
 // a CU's four pipes).
@@ -1305,6 +1305,10 @@ extern "C" int k8s_gemm_f32_rule(int M, int N, int K, int batch, int ntiles);
 extern "C" int k8s_gemm_f32_tiles(void* C, const float* A, const float* W, int M, int N, int K, long lda, long ldw, long ldc,
                                   int batch, long sA, long sW, long sC, const int* a_rows, const int* tiles, int ntiles,
                                   int out_f32, int fq, hipStream_t s);
+extern "C" int k8s_gemm_f32_parts_rule(int M, int N, int K, int batch, int ntiles);
+extern "C" int k8s_gemm_f32_parts(float* C, const float* A, const float* W, int M, int N, int K, long lda, long ldw, long ldc,
+                                  int batch, long sA, long sW, long sC, const int* a_rows, const int* tiles, int ntiles, int tile,
+                                  hipStream_t s);
 
 extern "C" int k8s_gemm_any(void* C, const void* A, const void* W, int M, int N, int K, long lda, long ldw, long ldc,
                             int batch, long sA, long sW, long sC, const int* a_rows, const int* tiles, int ntiles,
@@ -1320,8 +1324,8 @@ extern "C" int k8s_gemm_any(void* C, const void* A, const void* W, int M, int N,
     gy = (M + 63) / 64;
   }
   if (gy > 65535 || batch > 65535) return -2;
-  // bf16 rows that can be moved as 16-byte vectors: the bf16 MFMA kernels; fp32 ones: gemm_f32.hip's tiles or gemm_f32_kernel, by
-  // k8s_gemm_f32_rule; anything else: plain FMAs
+  // bf16 rows that can be moved as 16-byte vectors: the bf16 MFMA kernels; fp32 ones: gemm_f32_parts.hip's tiles by its rule (fp32
+  // outputs), else gemm_f32.hip's tiles or gemm_f32_kernel, by k8s_gemm_f32_rule; anything else: plain FMAs
   const bool vec = !in_f32 && K % 8 == 0 && lda % 8 == 0 && ldw % 8 == 0 && sA % 8 == 0 && sW % 8 == 0 &&
                    ((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0;
   if (vec && tiles != nullptr && K % 64 == 0 && M <= 32 * ntiles && M <= 512) {   // few rows per group
@@ -1357,6 +1361,12 @@ extern "C" int k8s_gemm_any(void* C, const void* A, const void* W, int M, int N,
   const int gm = tiles != nullptr ? gy * 2 : (M + 31) / 32;     // fp32 tiles are 32 rows high
   if (in_f32 && K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && sA % 4 == 0 && sW % 4 == 0 && ((uintptr_t)A & 15) == 0 &&
       ((uintptr_t)W & 15) == 0 && gm <= 65535) {
+    const int tile = out_f32 ? k8s_gemm_f32_parts_rule(M, N, K, batch, tiles != nullptr ? ntiles : 0) : 0;
+    if (tile > 0) {
+      const int rc = k8s_gemm_f32_parts((float*)C, (const float*)A, (const float*)W, M, N, K, lda, ldw, ldc, batch, sA, sW, sC, a_rows,
+                                        tiles, ntiles, tile, s);
+      if (rc != -2) return rc;
+    }
     const int fq = k8s_gemm_f32_rule(M, N, K, batch, tiles != nullptr ? ntiles : 0);
     if (fq > 0) {
       const int rc = k8s_gemm_f32_tiles(C, (const float*)A, (const float*)W, M, N, K, lda, ldw, ldc, batch, sA, sW, sC, a_rows,
