@@ -1126,6 +1126,11 @@ extern "C" int k8s_latent_kv_write(void* cache, const void* dkv, const void* nor
   return (int)hipGetLastError();
 }
 
+extern "C" int k8s_latent_f32(float* out, const float* q_abs, const float* q, const float* cache, const int* block_tables, int max_blocks,
+                              const int* tok_seq, const int* positions, int T, int C, int R, int H, int Dn, int window, float scale,
+                              int bs, const float* sinks, const float* gate, long ldg, hipStream_t s);
+
+// f32: 0 bf16, 1 fp32, 2 fp32 on the matrix cores where the sizes are ones that k8s_latent_f32 takes
 extern "C" int k8s_latent_attention(void* out, const void* q_abs, const void* q, const void* cache,
                                     const int* block_tables, int max_blocks, const int* tok_seq, const int* positions,
                                     int T, int C, int R, int H, int Dn, int window, float scale, int bs, int f32,
@@ -1133,6 +1138,11 @@ extern "C" int k8s_latent_attention(void* out, const void* q_abs, const void* q,
   if (T <= 0) return 0;
   if (gate != nullptr && ldg < H) return -1;
   if (C <= 0 || C > 512 || R < 0 || H <= 0 || bs <= 0) return -1;
+  if (f32 == 2) {
+    const int rc = k8s_latent_f32((float*)out, (const float*)q_abs, (const float*)q, (const float*)cache, block_tables, max_blocks, tok_seq,
+                                  positions, T, C, R, H, Dn, window, scale, bs, sinks, (const float*)gate, ldg, s);
+    if (rc != -2) return rc;
+  }
   const int L = C + R;
   const int nw = H < 8 ? H : 8;
   // LDS floats: KB (L + 1) key tile + nw L queries, within 60 KB

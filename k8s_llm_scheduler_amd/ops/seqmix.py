@@ -956,7 +956,7 @@ def latent_attention(q_abs: torch.Tensor, q: torch.Tensor, cache: torch.Tensor, 
     ``sinks`` [H] fp32: the softmax denominator of head h holds one more term e^sinks[h] (no key, no value).
     ``gate`` [T, H] of q's type (row stride free): head h's result is multiplied by sigmoid(gate[t, h]), which commutes
     with the value up-projection that follows.
-    bf16 with 16-byte-aligned parts runs on the matrix cores; fp32 and other sizes on the plain-FMA kernel."""
+    bf16 with 16-byte-aligned parts and fp32 of the usual sizes run on the matrix cores; other sizes on the plain-FMA kernel."""
     if sinks is not None and (sinks.dtype != F32 or sinks.numel() != H):
         raise ValueError("latent_attention: sinks are fp32 [H]")
     if gate is not None and (gate.shape != (q.shape[0], H) or gate.dtype != q.dtype or gate.stride(1) != 1):
@@ -985,7 +985,7 @@ def latent_attention(q_abs: torch.Tensor, q: torch.Tensor, cache: torch.Tensor, 
         nat.latent_attention_mfma(out.data_ptr(), _p(pacc), _p(pml), *args, ns, _p(cu_q, I32, "cu_q"), nseq,
                                   int(max_qlen), _p(sinks), gp, ldg, -1)
     else:
-        nat.latent_attention(out.data_ptr(), *args, _f32(dt), _p(sinks), gp, ldg, -1)
+        nat.latent_attention(out.data_ptr(), *args, 2 if LATENT_MFMA and dt == F32 else _f32(dt), _p(sinks), gp, ldg, -1)
     return out
 
 
