@@ -745,8 +745,9 @@ __global__ __launch_bounds__(64 * NWV) void latent_attention_mfma_kernel(
     p_first = p_last = positions[t];
     valid = true;
   } else {
-    seq = blockIdx.z;
-    split = 0;
+    const int nseq = gridDim.z / nsplit;
+    seq = blockIdx.z % nseq;
+    split = blockIdx.z / nseq;
     const int tq0 = cu_q[seq] + blockIdx.x * NWV, tend = cu_q[seq + 1];
     if (tq0 >= tend) return;
     const int nval = min(NWV, tend - tq0);
@@ -767,7 +768,13 @@ __global__ __launch_bounds__(64 * NWV) void latent_attention_mfma_kernel(
   const int lo_min = window > 0 ? max(0, p_first - window + 1) : 0;
   const int lo = window > 0 ? max(0, p - window + 1) : 0;
   const int ntiles = (p_last + 1 - lo_min + 31) / 32;
-  const int tps = (ntiles + nsplit - 1) / nsplit;
+  // The host splits by the keys that there may be.  Four tokens that see at most 192 are one split after all, which writes their
+  // result itself, and no split has fewer than 96.  16 heads over 512 + 64, window 1024, us, one split or (up to 127 tokens) a wave a token
+  // with splits / as it is: 97 tokens behind 1000 191 / 39, 8 x 12 behind 1000 265 / 38, 128 behind 472 81 / 38, 200 behind 400 81 / 40,
+  // 97 fresh ones 35 / 23, 24 fresh 19 / 15, 4 behind 600 28 / 23; 32 heads, 97 behind 1000 134 / 54, 200 behind 400 83 / 67.
+  const int tps = NWV == 4 && ntiles <= 6 ? ntiles : max(NWV == 4 && nsplit > 1 ? 3 : 1, (ntiles + nsplit - 1) / nsplit);
+  const bool whole = nsplit == 1 || (NWV == 4 && ntiles <= tps);
+  if (NWV == 4 && whole && split > 0) return;
   const int t0 = split * tps, t1 = min(ntiles, t0 + tps);
   const int* btr = block_tables + (size_t)seq * max_blocks;
   const int cpr = EX ? 4 * NKK : L / 8;   // 16-byte chunks per row
@@ -933,7 +940,8 @@ __global__ __launch_bounds__(64 * NWV) void latent_attention_mfma_kernel(
   for (int i = 0; i < 4; ++i) {
     const int hd = hg * 16 + 4 * g + i;
     if (hd >= H) continue;
-    if (nsplit == 1) {
+    if (nsplit > 1 && whole && li == 0) pml[((size_t)t * HP + hd) * nsplit * 2 + 1] = -1.f;        // nothing to join
+    if (whole) {
       float inv = 1.f / l_i[i];
       if (sinks != nullptr) {
         const float sk = sinks[hd], mx = fmaxf(m_i[i], sk), am = expf(m_i[i] - mx);
@@ -945,9 +953,11 @@ __global__ __launch_bounds__(64 * NWV) void latent_attention_mfma_kernel(
         if (n < ndb) out[((size_t)t * H + hd) * C + 16 * n + li] = f2bf(o[n][i] * inv);
     } else {
       const size_t rec = ((size_t)t * HP + hg * 16 + 4 * g + i) * nsplit + split;
+      if (m_i[i] != -INFINITY) {        // a record without keys is not read
 #pragma unroll
-      for (int n = 0; n < NDB; ++n)
-        if (n < ndb) pacc[rec * C + 16 * n + li] = o[n][i];
+        for (int n = 0; n < NDB; ++n)
+          if (n < ndb) pacc[rec * C + 16 * n + li] = o[n][i];
+      }
       if (li == 0) {
         pml[rec * 2] = m_i[i];      // -inf and 0 for a split without tiles
         pml[rec * 2 + 1] = l_i[i];
@@ -956,35 +966,43 @@ __global__ __launch_bounds__(64 * NWV) void latent_attention_mfma_kernel(
   }
 }
 
-// out[t][head] = sum_s e^(m_s - M) O_s / sum_s e^(m_s - M) l_s over the key splits; workgroups (token, head, slice of
-// the latent columns)
-__global__ void latent_merge_kernel(bf16_t* __restrict__ out, const float* __restrict__ pacc,
-                                    const float* __restrict__ pml, const int* __restrict__ positions, int C, int H,
-                                    int HP, int nsplit, const float* __restrict__ sinks,
-                                    const bf16_t* __restrict__ gate, long ldg) {
-  const int t = blockIdx.x, hd = blockIdx.y;
-  const int d0 = blockIdx.z * blockDim.x + threadIdx.x, dstep = blockDim.x * gridDim.z;
+// out[t][head] = sum_s e^(m_s - M) O_s / sum_s e^(m_s - M) l_s over the key splits (at most 64; lane s has split s); a workgroup is a
+// token and a head, a thread 4 latent columns, four records' loads in flight.  Records past the last with keys are not read.
+__global__ __launch_bounds__(128) void latent_merge_kernel(bf16_t* __restrict__ out, const float* __restrict__ pacc,
+                                                           const float* __restrict__ pml, const int* __restrict__ positions, int C,
+                                                           int H, int HP, int nsplit, const float* __restrict__ sinks,
+                                                           const bf16_t* __restrict__ gate, long ldg) {
+  const int t = blockIdx.x, hd = blockIdx.y, d = 4 * threadIdx.x, lane = threadIdx.x & 63;
+  bf16_t* o = out + ((size_t)t * H + hd) * C;
   if (positions[t] < 0) {
-    for (int d = d0; d < C; d += dstep) out[((size_t)t * H + hd) * C + d] = 0;
+    for (int i = threadIdx.x; i < C; i += 128) o[i] = 0;
     return;
   }
   const size_t rec0 = ((size_t)t * HP + hd) * nsplit;
-  float M = sinks != nullptr ? sinks[hd] : -INFINITY;
-  for (int s = 0; s < nsplit; ++s) M = fmaxf(M, pml[(rec0 + s) * 2]);
-  float den = sinks != nullptr ? expf(sinks[hd] - M) : 0.f;
-  for (int s = 0; s < nsplit; ++s) {
-    const float ms = pml[(rec0 + s) * 2];
-    if (ms != -INFINITY) den += expf(ms - M) * pml[(rec0 + s) * 2 + 1];
+  float ms = -INFINITY, ls = 0.f;
+  if (lane < nsplit) {
+    ms = pml[(rec0 + lane) * 2];
+    ls = pml[(rec0 + lane) * 2 + 1];
   }
+  if (__uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(ls))) < 0.f) return;        // written already
+  const int used = 64 - __builtin_clzll(__ballot(ms != -INFINITY) | 1);
+  const float M = fmaxf(wave_max(ms), sinks != nullptr ? sinks[hd] : -INFINITY);
+  const float w = ms == -INFINITY ? 0.f : expf(ms - M);
+  const float den = wave_sum(w * ls) + (sinks != nullptr ? expf(sinks[hd] - M) : 0.f);
+  if (d >= C) return;
   const float gh = head_gate(gate, ldg, t, hd);
-  for (int d = d0; d < C; d += dstep) {
-    float a = 0.f;
-    for (int s = 0; s < nsplit; ++s) {
-      const float ms = pml[(rec0 + s) * 2];
-      if (ms != -INFINITY) a += expf(ms - M) * pacc[(rec0 + s) * C + d];
+  f32x4 a = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < used; s0 += 4) {
+    f32x4 x[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) x[k] = *reinterpret_cast<const f32x4*>(pacc + (rec0 + min(s0 + k, used - 1)) * C + d);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float ws = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), min(s0 + k, 63)));
+      if (s0 + k < used && ws != 0.f) a += ws * x[k];          // (a record without keys holds nothing)
     }
-    out[((size_t)t * H + hd) * C + d] = f2bf(a / den * gh);
   }
+  for (int e = 0; e < 4; ++e) o[d + e] = f2bf(a[e] / den * gh);
 }
 
 }  // namespace k8sllm
@@ -1175,8 +1193,8 @@ extern "C" int k8s_latent_mfma_ok(int C, int R, int Dn) {
   return C % 16 == 0 && R % 8 == 0 && Dn % 8 == 0 && C <= 512 && L <= 640;
 }
 
-// nsplit == 1 and cu_q given (nseq sequences of at most max_qlen tokens): 4 consecutive tokens of a sequence per
-// workgroup; else one wave per (token, head group, key split).
+// cu_q given (nseq sequences of at most max_qlen tokens): 4 consecutive tokens of a sequence per workgroup (and key split);
+// else one wave per (token, head group, key split).
 extern "C" int k8s_latent_attention_mfma(void* out, float* pacc, float* pml, const void* q_abs, const void* q,
                                          const void* cache, const int* block_tables, int max_blocks,
                                          const int* tok_seq, const int* positions, int T, int C, int R, int H, int Dn,
@@ -1185,15 +1203,15 @@ extern "C" int k8s_latent_attention_mfma(void* out, float* pacc, float* pml, con
                                          hipStream_t s) {
   if (T <= 0) return 0;
   if (gate != nullptr && ldg < H) return -1;
-  if (!k8s_latent_mfma_ok(C, R, Dn) || H <= 0 || bs <= 0 || nsplit < 1 || (nsplit > 1 && (!pacc || !pml))) return -1;
+  if (!k8s_latent_mfma_ok(C, R, Dn) || H <= 0 || bs <= 0 || nsplit < 1 || nsplit > 64 || (nsplit > 1 && (!pacc || !pml))) return -1;
   const int L = C + R, HG = (H + 15) / 16;
   const size_t lds = (size_t)32 * (L + 8) * 2;
   // the block table of one sequence beside the key tile, within the 64 KB a launch gets without asking for more
   const int bt_lds = lds + (size_t)max_blocks * sizeof(int) <= 65536;
   const size_t bt_bytes = bt_lds ? (size_t)max_blocks * sizeof(int) : 0;
-  const bool tiles = nsplit == 1 && cu_q != nullptr && nseq > 0 && max_qlen > 1;
-  if (tiles && nseq > 65535) return -2;
-  const dim3 grid = tiles ? dim3((max_qlen + 3) / 4, HG, nseq) : dim3(T, HG, nsplit);
+  const bool tiles = cu_q != nullptr && nseq > 0 && max_qlen > 1;
+  if (tiles && (long)nseq * nsplit > 65535) return -2;
+  const dim3 grid = tiles ? dim3((max_qlen + 3) / 4, HG, nseq * nsplit) : dim3(T, HG, nsplit);
 #define K8S_LM(NDB, NKK, EX)                                                                                            \
   do {                                                                                                                \
     if (tiles)                                                                                                        \
@@ -1218,7 +1236,7 @@ extern "C" int k8s_latent_attention_mfma(void* out, float* pacc, float* pml, con
   else K8S_LM(32, 20, false);
 #undef K8S_LM
   if (nsplit > 1)
-    latent_merge_kernel<<<dim3(T, H, (C + 127) / 128), 128, 0, s>>>((bf16_t*)out, pacc, pml, positions, C, H, HG * 16,
+    latent_merge_kernel<<<dim3(T, H), 128, 0, s>>>((bf16_t*)out, pacc, pml, positions, C, H, HG * 16,
                                                                     nsplit, sinks, (const bf16_t*)gate, ldg);
   return (int)hipGetLastError();
 }

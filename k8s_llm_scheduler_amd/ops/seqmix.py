@@ -944,6 +944,12 @@ def latent_splits(T: int, H: int, max_keys: int) -> int:
     return max(1, min(256 // groups, (max(1, max_keys) + 31) // 32, 32))
 
 
+def latent_quad_splits(T: int, nseq: int, H: int, max_keys: int) -> int:
+    """Key splits of portions of ``nseq`` sequences, ``T`` tokens in all, whose workgroups are four consecutive tokens."""
+    groups = min(T, T // 4 + nseq) * ((H + 15) // 16)
+    return max(1, min(256 // groups, (max(1, max_keys) + 63) // 64, 32))
+
+
 def latent_attention(q_abs: torch.Tensor, q: torch.Tensor, cache: torch.Tensor, block_tables: torch.Tensor,
                      tok_seq: torch.Tensor, positions: torch.Tensor, C: int, R: int, H: int, Dn: int, window: int,
                      scale: float, block_size: int, max_keys: int = 0, cu_q: Optional[torch.Tensor] = None,
@@ -975,13 +981,13 @@ def latent_attention(q_abs: torch.Tensor, q: torch.Tensor, cache: torch.Tensor, 
     if LATENT_MFMA and dt == BF16 and nat.latent_mfma_ok(C, R, Dn):
         cap = block_tables.shape[1] * block_size
         bound = min(max_keys or cap, window or cap, cap)
-        ns = latent_splits(T, H, bound)
+        nseq = cu_q.shape[0] - 1 if cu_q is not None else 0
+        ns = latent_quad_splits(T, nseq, H, bound) if nseq and max_qlen > 1 else latent_splits(T, H, bound)
         pacc = pml = None
         if ns > 1:
             HP = (H + 15) // 16 * 16
             pacc = torch.empty(T * HP * ns * C, dtype=F32, device=q.device)
             pml = torch.empty(T * HP * ns * 2, dtype=F32, device=q.device)
-        nseq = cu_q.shape[0] - 1 if cu_q is not None else 0
         nat.latent_attention_mfma(out.data_ptr(), _p(pacc), _p(pml), *args, ns, _p(cu_q, I32, "cu_q"), nseq,
                                   int(max_qlen), _p(sinks), gp, ldg, -1)
     else:

@@ -1,4 +1,5 @@
-"""Latent attention in true fp32 on the matrix cores (latent_f32.hip) against 64 bits, and beside the plain-FMA kernel."""
+"""Latent attention over cached rows against 64 bits: true fp32 on the matrix cores (latent_f32.hip) beside the plain-FMA kernel, and the
+key splits of portions of prompts in bf16."""
 import pytest
 import torch
 
@@ -50,3 +51,28 @@ def test_against_64_bits(C, R, H, window, bs, extra, monkeypatch):
         assert (y[pos < 0] == 0).all()
         err.append(float((y - want).norm() / want.norm()))
     assert err[0] <= 2e-6 and err[0] <= 1.25 * err[1], err        # scores of up to 10: a part in 2^22 of them, and no more than plain FMAs give
+
+
+@pytest.mark.parametrize("H,lens,past,window", [(16, (4, 9), 600, 0), (16, (97, 1, 1), 300, 1024), (20, (30, 3), 1000, 70), (32, (60, 5), 130, 0),
+                                                (16, (5, 2), 189, 0), (3, (8,), 2000, 0)])
+def test_key_splits_of_portions_in_bf16(H, lens, past, window):
+    """Four tokens a workgroup, their keys split: fewer keys than a split, around the fewest that are split, splits that stay empty; idle
+    rows at a batch's end; sinks and gates through the kernel that joins and through the one that has nothing to join."""
+    C, R, Dn, bs = 512, 64, 16, 16
+    g = torch.Generator().manual_seed(past + H)
+    n, T = len(lens), sum(lens)
+    pos = torch.cat([torch.arange(k) + (past if i != 1 else 0) for i, k in enumerate(lens)]).int()
+    seq = torch.cat([torch.full((k,), i) for i, k in enumerate(lens)]).int()
+    nb = (past + max(lens)) // bs + 1
+    bt = torch.randperm(n * nb, generator=g).view(n, nb).int()
+    cu = torch.tensor([0, *lens]).cumsum(0).int()
+    cache = torch.randn(n * nb * bs, C + R, generator=g).bfloat16()
+    qa, q = torch.randn(T, H, C, generator=g).bfloat16(), torch.randn(T, H * (Dn + R), generator=g).bfloat16()
+    sinks, gate = torch.randn(H, generator=g), torch.randn(T, H, generator=g).bfloat16()
+    scale = (C + R)**-0.5
+    assert sm.latent_quad_splits(T, n, H, nb * bs) > 1
+    want = exact(qa, q, cache, bt, seq, pos, C, R, H, Dn, window, scale, bs, sinks, gate)
+    y = sm.latent_attention(qa.cuda(), q.cuda(), cache.cuda(), bt.cuda(), seq.cuda(), pos.cuda(), C, R, H, Dn, window, scale, bs, 0, cu.cuda(),
+                            max(lens), sinks=sinks.cuda(), gate=gate.cuda()).cpu().double()
+    for t in range(T):          # weights and result rounded to bf16: 2^-9 of each, 2-norm below 2^-8 a row
+        assert float((y[t] - want[t]).norm()) <= 2.0**-7 * float(want[t].norm()), t
