@@ -37,7 +37,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # instructions (v_pk_add/mul/fma_f32), which -O3 otherwise forms from ordinary float code.  The other kernel files keep the
 # flags they were validated with: with the option on every file, the two-rank fused GEMV all-reduce check of tests/test_multigpu.py reported a wrong sum.
 NO_PACKED_FP32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
-NO_PACKED_FP32_FILES = {"stream32.hip", "mixers.hip", "latent_prompt.hip", "latent_token.hip", "latent_f32.hip", "moe.hip",
+NO_PACKED_FP32_FILES = {"stream32.hip", "mixers.hip", "latent_prompt.hip", "latent_token.hip", "latent_f32.hip", "window_f32.hip", "moe.hip",
                         "window_attn.hip", "gemm_f32.hip", "gemm_f32_parts.hip", "gated_scan.hip", "delta_scan.hip", "decay_scan.hip", "pgemm4.hip", "pgemm4_tiles.hip", "pgemm4_wide.hip",
                         "gemv_act.hip", "sgemv_act.hip", "mgemm_act.hip", "norm_gemv.hip", "stream_gemv.hip", "attn_prefill.hip"}
 # the lean module: kernels of the fp32-stream designs, the sampler, the small shared kernels; the block allocator

@@ -7,7 +7,9 @@
 // A workgroup is a token and 16 heads; its 4 waves take the tiles of 16 keys in turn, each with a maximum and sums of its own and no
 // barrier, and meet at the end.  The next tile's rows are under way while the second product runs.  A wave holds queries, rows and
 // sums of 512 + 64 dimensions in registers (one wave a SIMD), which is why a workgroup has no more tokens.
-// Bound by the fp32 matrix rate: a tile is 272 products of 32 cycles a wave.
+// Bound by the fp32 matrix rate: a tile is 272 products of 32 cycles a wave.  us, plain FMAs (a workgroup a token, a wave a head, keys in LDS)
+// / here, 16 heads over 512 + 64, window 1024: 125 tokens behind 940 3305 / 112, 64 behind 600 2110 / 77, 1 behind 600 2097 / 75, 512 behind 1500 3786 /
+// 238, 24 fresh 126 / 18; 32 heads, 125 behind 940 6582 / 122.
 #include "common.h"
 
 namespace k8sllm {
@@ -71,6 +73,7 @@ __global__ __launch_bounds__(256, 1) void latent_f32_kernel(
     }
 #pragma unroll
     for (int s = 0; s < NC; ++s) *reinterpret_cast<f32x4*>(&mine[li][16 * s + 4 * g]) = kf[s];
+    asm volatile("" ::: "memory");                 // other lanes read what this one wrote
     if (tile + 4 < tiles) load(row_of(tile + 4));
     f32x4 w = (sc[0] + sc[1]) + (sc[2] + sc[3]);   // key 4 g + i, head li
     float top = -INFINITY;

@@ -1361,8 +1361,8 @@ def window_attention(q: torch.Tensor, gate: Optional[torch.Tensor], kcache: torc
     is taken off the score of the token at position j (not off the sink's; not with pooled blocks).
     ``cu_q`` / ``max_qlen`` (the sequences' query offsets and longest portion): bf16 portions of prompts whose sizes
     fit run on the matrix cores, tiles of consecutive tokens sharing the staged keys; so do bf16 tokens one by one
-    (decoding, or query groups that make no tile) without pooled blocks; anything else (fp32, other sizes) on the plain-FMA
-    kernel.  The keys of few tokens are split over several workgroups
+    (decoding, or query groups that make no tile) without pooled blocks, and fp32 portions of the usual sizes without them; anything
+    else on the plain-FMA kernel.  The keys of few tokens are split over several workgroups
     (``max_keys``: an upper bound of the positions any token sees, 0: the block tables' capacity)."""
     G, D, V = kcache.shape[1], kcache.shape[2], vcache.shape[2]
     if H % G:
@@ -1404,6 +1404,14 @@ def window_attention(q: torch.Tensor, gate: Optional[torch.Tensor], kcache: torc
                                   _p(positions, I32), cu_q.shape[0] - 1, int(max_qlen), T, H, G, D, V, int(window), int(P),
                                   float(scale), int(bool(sink)), block_size, ns, int(chunk), float(softcap), _p(sinks),
                                   int(bool(gate_per_head)), _p(slopes), -1)
+        return out
+    if (WINDOW_MFMA and dt == F32 and P <= 0 and cu_q is not None and max_qlen > 1 and nat.window_f32_ok(H, G, D, V)
+            and q.stride(0) % 4 == 0 and (q.data_ptr() | kcache.data_ptr() | vcache.data_ptr()) % 16 == 0):
+        nat.window_f32(out.data_ptr(), q.data_ptr(), q.stride(0), gate.data_ptr() if gate is not None else 0,
+                       gate.stride(0) if gate is not None else 0, _p(kcache, dt, "kcache"), _p(vcache, dt, "vcache"),
+                       _p(block_tables, I32, "block_tables"), block_tables.shape[1], _p(cu_q, I32, "cu_q"), _p(positions, I32),
+                       cu_q.shape[0] - 1, int(max_qlen), H, G, D, V, int(window), float(scale), int(bool(sink)), block_size, int(chunk),
+                       float(softcap), _p(sinks), int(bool(gate_per_head)), _p(slopes), -1)
         return out
     max_pos = max_keys or block_tables.shape[1] * block_size
     if (WINDOW_MFMA and dt == BF16 and P <= 0 and nat.window_token_ok(H, G, D, V, block_size) and q.stride(0) % 8 == 0
