@@ -314,8 +314,9 @@ __global__ __launch_bounds__(512) void latent_prompt_kernel(
 // fp32, every product and sum in fp32 (v_mfma_f32_16x16x4_f32).  A workgroup takes 64 tokens of one head, a wave 16 of them;
 // 32-key steps staged through LDS.  S^T = K Q^T leaves a lane the scores of the keys 16 m + 4 g + i of its token; O^T = V^T P
 // takes them as the B operand of the instruction (m, i) where they are, so nothing is exchanged but the maxima and sums.
-// DK = DN + R and DV multiples of 16.  333 tokens, 16 heads: 45 us (absorbed, on
-// plain FMAs: 1235 us); six token tiles of 16 heads leave most of the chip idle.
+// DK = DN + R and DV multiples of 16.  A score is four sums of every fourth dimension: in one, 48 instructions long, it was the largest
+// part of the result's error (2-norm against 64 bits 4.0 - 4.9e-7, so 2.7 - 3.5e-7; 45 -> 47 us).  333 tokens, 16 heads: 47 us (absorbed 104
+// in latent_f32.hip); six token tiles of 16 heads leave most of the chip idle.
 template <int DN, int R, int DV>
 __global__ __launch_bounds__(256) void latent_prompt_f32_kernel(
     float* __restrict__ out, const float* __restrict__ kv, const int* __restrict__ rows, const int* __restrict__ kbase,
@@ -386,15 +387,18 @@ __global__ __launch_bounds__(256) void latent_prompt_f32_kernel(
     if (step + 1 < nsteps) stage_load(step + 1);
     const int j0 = lo_min + step * KT;
     if (!w_any || j0 > w_last || j0 + KT - 1 < w_lo) continue;
-    f32x4 s[2] = {zero, zero};     // s[m][i] = score of key j0 + 16 m + 4 g + i for token li
+    f32x4 s[2];                    // s[m][i] = score of key j0 + 16 m + 4 g + i for token li
 #pragma unroll
-    for (int m = 0; m < 2; ++m)
+    for (int m = 0; m < 2; ++m) {
+      f32x4 part[4] = {zero, zero, zero, zero};
 #pragma unroll
       for (int j = 0; j < NK4; ++j) {
         const f32x4 kf = *reinterpret_cast<const f32x4*>(&ks[16 * m + li][16 * j + 4 * g]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i], qf[j][i], s[m], 0, 0, 0);
+        for (int i = 0; i < 4; ++i) part[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i], qf[j][i], part[i], 0, 0, 0);
       }
+      s[m] = (part[0] + part[1]) + (part[2] + part[3]);
+    }
     float tmax = -INFINITY;
 #pragma unroll
     for (int m = 0; m < 2; ++m)
