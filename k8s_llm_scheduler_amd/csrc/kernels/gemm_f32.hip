@@ -1,4 +1,5 @@
 // fp32 products of many tiles: C[M, N] = A[M, K] W[N, K]^T on v_mfma_f32_16x16x4_f32 (fp32 products and sums), K % 32 == 0.
+// They take what gemm_f32_parts.hip's rule leaves them: bf16 outputs, and sizes at which they are within a tenth of its tiles.
 //
 // A workgroup of 4 waves owns 64 columns x 16 FQ rows (swapped orientation C^T = W A^T; a wave 16 columns x all rows), so the
 // row count is padded to 16 and FQ is chosen for the tiles to fill the CUs' last round.  k in 32-deep stages of 128-byte rows
