@@ -512,6 +512,11 @@ def _grouped_more(rows: int, E: int, N: int, K: int, pair: bool, even: bool, com
     for cfg in [base] + [c for c in _GROUP_MORE_COST if c not in _GROUP_TILE]:
         t0, tile, rnd, step, wmb, omb, act_us = _GROUP_MORE_COST[cfg]
         bp, bq = _GROUP_MORE_TILE[cfg]
+        # Tiles of 96 tokens that every group, the common rows too, fills at most once are one round of which a quarter is empty, and
+        # the fit has them cheaper than they are; with a second one for the common rows they are.  8 groups and a common one, gated 2 x 2048 x
+        # 2048, the tile between / _grouped_tile's: 83 tokens 35.8 / 34.5, 96 36.1 / 34.8, 97 34.0 / 34.9, 160 34.4 / 36.9; 4096 x 3584, 81 - 96 55.5 - 56.4 / 56.1 - 57.2.
+        if cfg == 10 and base != 10 and 0 < common <= bq and r + 3.0 * sd <= bq:
+            continue
         if even:
             tiles, dev = E * -(-rows // E // bq), 0.0
         else:
