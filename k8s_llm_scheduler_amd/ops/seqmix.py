@@ -501,6 +501,12 @@ _GROUP_MORE_COST = {1: (0.0, 0.613, 3.47, 0.0, 0.104, 0.44, 5.08), 2: (0.497, 0.
                     12: (1.04, 0.501, 2.48, 0.0, 0.0826, 0.535, 7.01), 13: (0.0, 0.632, 4.95, 0.0, 0.0749, 0.429, 5.13),
                     15: (0.0, 0.686, 6.1, 0.0, 0.0699, 0.416, 4.79), 16: (0.0, 0.777, 6.37, 0.0, 0.0695, 0.43, 4.81),
                     17: (0.0, 0.853, 6.61, 0.0, 0.0756, 0.441, 3.83)}
+# ... and per MB of weights where the common rows are one row of tiles, each of which reads weights of its own; with two of them, pairs
+# share theirs.  8 groups and a common one, 96 / 97 tokens, us: on 192 x 96 gated 2 x 2048 x 2048 36.9 / 34.4 (64 x 64 35.1 / 35.0), 4096 x 3584 56.1 /
+# 50.1 (56.3 / 56.5), 2048 x 2048 27.0 / 24.8; 128 / 130 on 192 x 128 38.1 / 34.9, 57.5 / 52.0, 28.8 / 26.1; none on the tiles of _GROUP_TILE that are
+# picked there.  Over 936 products of 4 - 17 groups, 17 weights, 41 - 2900 tokens the picks take 2.2 % less than _grouped_tile's, 20 of them 2 %
+# more and over, up to 25 % (4096 x 2048 of 4 groups, 214 tokens 20.4 -> 25.6); with twice or half the term they are the same.
+_GROUP_MORE_ALONE = {10: 0.008, 11: 0.008, 12: 0.002, 13: 0.002}
 
 
 @functools.lru_cache(maxsize=4096)
@@ -512,11 +518,6 @@ def _grouped_more(rows: int, E: int, N: int, K: int, pair: bool, even: bool, com
     for cfg in [base] + [c for c in _GROUP_MORE_COST if c not in _GROUP_TILE]:
         t0, tile, rnd, step, wmb, omb, act_us = _GROUP_MORE_COST[cfg]
         bp, bq = _GROUP_MORE_TILE[cfg]
-        # Tiles of 96 tokens that every group, the common rows too, fills at most once are one round of which a quarter is empty, and
-        # the fit has them cheaper than they are; with a second one for the common rows they are.  8 groups and a common one, gated 2 x 2048 x
-        # 2048, the tile between / _grouped_tile's: 83 tokens 35.8 / 34.5, 96 36.1 / 34.8, 97 34.0 / 34.9, 160 34.4 / 36.9; 4096 x 3584, 81 - 96 55.5 - 56.4 / 56.1 - 57.2.
-        if cfg == 10 and base != 10 and 0 < common <= bq and r + 3.0 * sd <= bq:
-            continue
         if even:
             tiles, dev = E * -(-rows // E // bq), 0.0
         else:
@@ -526,6 +527,8 @@ def _grouped_more(rows: int, E: int, N: int, K: int, pair: bool, even: bool, com
         rounds = sum(max(1, math.ceil((tiles + z * dev) * -(-n // bp) / 256 - 0.01)) for z in (-1.2, 0.0, 1.2)) / 3.0
         us = t0 + rounds * (tile * kt + rnd + (act_us * bp * bq / 65536 if pair else 0.0)) + step * kt + wmb * E * n * K * 2e-6 + \
             omb * rows * N * 2e-6
+        if 0 < common <= bq:
+            us += _GROUP_MORE_ALONE.get(cfg, 0.0) * E * n * K * 2e-6
         if best is None or us < best[0]:
             best = (us if best is not None else 0.96 * us, cfg)
     return best[1]

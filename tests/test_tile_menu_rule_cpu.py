@@ -34,7 +34,8 @@ def test_tuned_plans_stay_at_their_row_count(monkeypatch):
 @pytest.mark.parametrize("rows,E,N,K,pair,even,common,want", [
     (4602, 9, 2048, 2048, True, False, 1534, 15), (2800, 4, 2048, 2048, False, True, 0, 12), (8192, 4, 2048, 2048, False, True, 0, 4),
     (2800, 4, 512, 2048, False, True, 0, None), (249, 9, 2048, 2048, True, False, 83, None), (288, 9, 2048, 2048, True, False, 96, None),
-    (291, 9, 2048, 2048, True, False, 97, 10)])
+    (291, 9, 2048, 2048, True, False, 97, 10), (243, 9, 4096, 3584, False, False, 81, 10), (288, 9, 4096, 3584, False, False, 96, 10),
+    (243, 9, 2560, 2048, True, False, 81, 10), (288, 9, 2560, 2048, True, False, 96, 10), (396, 6, 2560, 2048, True, False, 132, 10)])
 def test_grouped_picks(rows, E, N, K, pair, even, common, want):
     got = sm._grouped_plan(rows, E, N, K, pair, even, common)
     assert got == (want if want is not None else sm._grouped_tile(rows, E, N, K, pair, even, common))
