@@ -6,18 +6,23 @@
 // PFLOP/s over 157 TFLOP/s, over 6).  Registers sum chains of 64 k (128 from 128 steps on), and a second set the chains, so the
 // error against 64 bits is below the fp32 pipes' (2-norm, here / there: K = 1024 1.2e-7 / 1.6 - 2.1e-7, 2048 1.2 - 1.5e-7 / 2.1 -
 // 2.9e-7, 8192 1.5 - 1.6e-7 / 2.2 - 5.7e-7, 14336 1.7 - 2.25e-7 / 2.3 - 7.7e-7; one chain for all of K = 2048: 2.4 - 7e-7).
-// Parts of infinities are NaN, those of values below 2^-108 lose bits: an output that is NaN or below 2^-80 is computed again with plain fp32 FMAs.
+// Parts of infinities are NaN, a high part may round to infinity, and parts and products below 2^-126 may be lost: of a product at
+// most 2^-126 times the other side's value, and six times 2^-126.  So an output is computed again with plain fp32 FMAs where it is not
+// finite, where it is smaller than K 2^-97 times the largest value of its row and column (or 1: above that what may be lost is 2^-25
+// of it and less), and where it is zero though both have values.  The largest values are met on the way to the parts, one
+// instruction for two of them.  A lane computes its 4 columns again, so a row or a column of such outputs costs a walk over k at the
+// speed of loads: with one NaN in a row 333 x 2048 x 8192 takes 470 us instead of 101, with an infinity in a column 430.
 //
 // A workgroup of 8 waves owns 16 CW WC columns x 16 FQ rows: WC waves side by side, each with CW x 16 columns and all rows, and
 // 8 / WC shares of k (steps of 32 k in turn).  A wave loads its weights itself and cuts them in registers; with WC > 1 the rows are
 // cut once a workgroup and pass through LDS, with WC = 1 a wave cuts its own.  Both for the step after the current one, two
 // values between every CW products (the barriers of the compiler's schedule keep them there: left alone it cuts everything first).
-// Bound by the matrix cores on the large tiles (333 x 16384 x 2048, 131 us: 1.18 PFLOP/s of bf16 products with the padding, where
+// Bound by the matrix cores on the large tiles (333 x 16384 x 2048, 142 us: 1.09 PFLOP/s of bf16 products with the padding, where
 // large bf16 products reach 1.35), on the small ones by the loads of rows 64 bytes at a time and the cutting (60 x 2048 x 8192, 47 us: 27
 // without the loads, 17 without both; loads two and four steps ahead, and tiles that start at different k, change nothing).
-// us, fp32 pipes / here, weights from memory: 333 x 16384 x 2048 208 / 123, x 2048 x 8192 107 / 96, x 3072 x 2048 57 / 36, 512 x
-// 16384 x 2048 309 / 154, 457 x 4096 x 14336 550 / 314, 150 x 28672 x 4096 376 / 243, 64 x 16384 x 2048 46 / 34, 17 x 2048 x 2048
-// 14.8 / 11.3, 1 x 2048 x 8192 67 / 27, 16 x 3072 x 2048 18.5 / 11.2.
+// us, fp32 pipes / here, weights from memory: 333 x 16384 x 2048 195 / 142, x 2048 x 8192 110 / 104, x 3072 x 2048 51 / 39, 512 x
+// 16384 x 2048 257 / 168, 457 x 4096 x 14336 472 / 347, 150 x 28672 x 4096 338 / 253, 64 x 16384 x 2048 44 / 40, 17 x 2048 x 2048
+// 14.8 / 11.1, 1 x 2048 x 8192 64 / 27, 16 x 3072 x 2048 18.6 / 11.1.  The largest values cost 1 - 3 % of that.
 #include <math.h>
 
 #include "common.h"
@@ -32,17 +37,18 @@ struct PartsArgs {
   const int *a_rows, *tiles;        // listed tiles of at most 64 rows: 64 / Q blocks for each
   int vec;                          // 4 consecutive columns can be stored as one vector
   int chain;                        // steps of a chain - 1 (a power of two less one)
+  float least;                      // of an output, over the larger side's largest value (or 1): below it parts may be missing
 };
 
 struct Three {                      // the parts of 8 values, two in a word
   u32x4 h, m, l;
 };
 
-// values 2 q and 2 q + 1 of the eight (a, b)
-__device__ __forceinline__ void cut2(Three& t, const f32x4 (&r)[2], int q) {
+// values 2 q and 2 q + 1 of the eight (a, b); top: the largest magnitude met so far
+__device__ __forceinline__ void cut2(Three& t, const f32x4 (&r)[2], int q, float& top) {
   typedef __attribute__((ext_vector_type(2))) float f32x2;
   float a = r[q >> 1][2 * q & 3], b = r[q >> 1][(2 * q & 3) + 1];
-  asm volatile("" : "+v"(a), "+v"(b));
+  asm volatile("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top), "+v"(a), "+v"(b));
   f32x2 x = {a, b};
   uint32_t p[3];
 #pragma unroll
@@ -54,10 +60,10 @@ __device__ __forceinline__ void cut2(Three& t, const f32x4 (&r)[2], int q) {
   asm volatile("" : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]));
   t.h[q] = p[0], t.m[q] = p[1], t.l[q] = p[2];
 }
-__device__ __forceinline__ Three cut(const f32x4 (&r)[2]) {
+__device__ __forceinline__ Three cut(const f32x4 (&r)[2], float& top) {
   Three t;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) cut2(t, r, q);
+  for (int q = 0; q < 4; ++q) cut2(t, r, q, top);
   return t;
 }
 
@@ -65,7 +71,7 @@ template <int WC, int CW, int FQ>
 __global__ __launch_bounds__(512, 2) void gemm_f32_parts_kernel(PartsArgs a) {
   constexpr int WK = 8 / WC, P = 16 * CW * WC, Q = 16 * FQ, NX = (FQ + WC - 1) / WC;
   constexpr int GS = Q * 16 + 32, BUF = WK * 12 * GS, RED = 8 * CW * FQ * 1024;
-  constexpr int STAGES = WC > 1 ? 2 * BUF : 0, LDS = STAGES > RED ? STAGES : RED;
+  constexpr int STAGES = WC > 1 ? 2 * BUF : 0, TOPS = WK * (P + Q) * 4 + 32, LDS = STAGES > RED + TOPS ? STAGES : RED + TOPS;
   __shared__ __attribute__((aligned(16))) char lds[LDS];
   const int tot = a.mt * a.nt * a.batch, q8 = tot >> 3, r8 = tot & 7, xcd = blockIdx.x & 7;
   int t = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (int)(blockIdx.x >> 3);
@@ -136,6 +142,11 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_parts_kernel(PartsArgs a) {
 #pragma unroll
     for (int j = 0; j < FQ; ++j) acc[c][j] = sum[c][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   Three wa[CW], wb[CW], xf[2], xs;
+  float wtop[CW], xtop[NR];         // the largest magnitudes of this lane's share of a column, of a row
+#pragma unroll
+  for (int c = 0; c < CW; ++c) wtop[c] = 0.f;
+#pragma unroll
+  for (int n = 0; n < NR; ++n) xtop[n] = 0.f;
   const auto read_x = [&](int s, int j) {
     const char* xb = lds + (s & 1) * BUF + wk * 12 * GS + g * GS + li * 16 + j * 256;
     return Three{*reinterpret_cast<const u32x4*>(xb), *reinterpret_cast<const u32x4*>(xb + 4 * GS),
@@ -147,18 +158,18 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_parts_kernel(PartsArgs a) {
   for (int n = 0; n < NR; ++n) load_x(0, n);
 #pragma unroll
   for (int c = 0; c < CW; ++c) {
-    wa[c] = cut(wr[c]);
+    wa[c] = cut(wr[c], wtop[c]);
     load_w(1, c);
   }
   if constexpr (WC > 1) {
 #pragma unroll
     for (int n = 0; n < NR; ++n) {
-      store_x(0, n, cut(xr[n]));
+      store_x(0, n, cut(xr[n], xtop[n]));
       load_x(1, n);
     }
     meet();
   } else {
-    xf[0] = cut(xr[0]);
+    xf[0] = cut(xr[0], xtop[0]);
     load_x(1, 0);
   }
   // One step's products.  `more`: between them the next step's weights and rows are cut into parts, two values at a time, and the
@@ -186,7 +197,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_parts_kernel(PartsArgs a) {
 #pragma unroll
           for (int n = 0; n < WP; ++n)
             if (n * GROUPS / WP == q) {
-              cut2(wn[n >> 2], wr[n >> 2], n & 3);
+              cut2(wn[n >> 2], wr[n >> 2], n & 3, wtop[n >> 2]);
               if ((n & 3) == 3) load_w(s + 2, n >> 2);
             }
         }
@@ -194,7 +205,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_parts_kernel(PartsArgs a) {
 #pragma unroll
           for (int n = 0; n < XP; ++n)
             if (n * GROUPS / XP == q) {
-              cut2(xs, xr[n >> 2], n & 3);
+              cut2(xs, xr[n >> 2], n & 3, xtop[n >> 2]);
               if ((n & 3) == 3) {
                 store_x(s + 1, n >> 2, xs);
                 load_x(s + 2, n >> 2);
@@ -204,7 +215,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_parts_kernel(PartsArgs a) {
         if constexpr (WC == 1) {
           const int n = j + 1 < FQ ? j + 1 : 0;
           if (p < 4 && (MORE || n)) {
-            cut2(xn, xr[n], p);
+            cut2(xn, xr[n], p, xtop[n]);
             if (p == 3 && MORE) load_x(n ? s + 1 : s + 2, n);
           }
         }
@@ -247,7 +258,34 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_parts_kernel(PartsArgs a) {
   for (int c = 0; c < CW; ++c)
 #pragma unroll
     for (int j = 0; j < FQ; ++j) *reinterpret_cast<f32x4*>(red + (((wid * CW + c) * FQ + j) * 64 + lane) * 4) = sum[c][j];
+  // [wave]: its largest of all; [share of k][column], [row]
+  float *tops = red + RED / 4, *wtops = tops + 8, *xtops = wtops + WK * P;
+  float most = 0.f;
+#pragma unroll
+  for (int c = 0; c < CW; ++c) {
+    const float m = lane_max<16>(lane_max<32>(wtop[c]));
+    most = fmaxf(most, wtop[c]);
+    if (g == 0) wtops[wk * P + 16 * (wc * CW + c) + li] = m;
+  }
+#pragma unroll
+  for (int n = 0; n < NR; ++n) {
+    most = fmaxf(most, xtop[n]);
+    if constexpr (WC > 1) {
+      const float m = lane_max<1>(lane_max<2>(xtop[n]));      // a row's four chunks
+      const int q = (tid + 512 * n) >> 2;                     // (its rows in turn: a share of k has Q of them)
+      if ((tid & 3) == 0 && q < WK * Q) xtops[q] = m;
+    } else {
+      const float m = lane_max<16>(lane_max<32>(xtop[n]));
+      if (g == 0) xtops[wk * Q + 16 * n + li] = m;
+    }
+  }
+  most = wave_max(most);
+  if (lane == 0) tops[wid] = most;
   __syncthreads();
+  // most outputs are large enough for any value of the workgroup
+  const f32x4 t0 = *reinterpret_cast<const f32x4*>(tops), t1 = *reinterpret_cast<const f32x4*>(tops + 4);
+  most = fmaxf(fmaxf(fmaxf(t0[0], t0[1]), fmaxf(t0[2], t0[3])), fmaxf(fmaxf(t1[0], t1[1]), fmaxf(t1[2], t1[3])));
+  const float enough = a.least * fmaxf(most, 1.f);
 #pragma unroll 1
   for (int f = wk; f < CW * FQ; f += WK) {
     f32x4 y = *reinterpret_cast<const f32x4*>(red + ((wc * CW * FQ + f) * 64 + lane) * 4);
@@ -257,17 +295,37 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_parts_kernel(PartsArgs a) {
     if (r >= rows || n >= a.N) continue;
     bool again = false;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) again |= y[e] != 0.f && !(fabsf(y[e]) >= 0x1p-80f);
+    for (int e = 0; e < 4; ++e) again |= !(fabsf(y[e]) >= enough && fabsf(y[e]) < INFINITY);
+    if (again) {
+      float mx = 0.f;
+      f32x4 mw = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < WK; ++k) {
+        mx = fmaxf(mx, xtops[k * Q + r]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mw[e] = fmaxf(mw[e], wtops[k * P + n - col0 + e]);
+      }
+      again = false;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        again |= y[e] == 0.f ? mx > 0.f && mw[e] > 0.f : !(fabsf(y[e]) >= a.least * fmaxf(fmaxf(mx, mw[e]), 1.f) && fabsf(y[e]) < INFINITY);
+    }
     if (again) {
       const float* x = row(r);
       y = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
       for (int k0 = 0; k0 < a.K; k0 += 32) {
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-        for (int k = k0; k < k0 + 32; ++k)
+#pragma unroll 2
+        for (int k = k0; k < k0 + 32; k += 4) {
+          const f32x4 xk = *reinterpret_cast<const f32x4*>(x + k);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = fmaf(x[k], W[(size_t)min(n + e, a.N - 1) * a.ldw + k], v[e]);
+          for (int e = 0; e < 4; ++e) {
+            const f32x4 wk4 = *reinterpret_cast<const f32x4*>(W + (size_t)min(n + e, a.N - 1) * a.ldw + k);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[e] = fmaf(xk[i], wk4[i], v[e]);
+          }
+        }
         y += v;
       }
     }
@@ -334,7 +392,7 @@ extern "C" int k8s_gemm_f32_parts(float* C, const float* A, const float* W, int 
       (((uintptr_t)A | (uintptr_t)W) & 15))
     return -1;
   if (tiles != nullptr && (64 % (16 * fq) || ntiles <= 0)) return -1;
-  PartsArgs a = {C, A, W, M, N, K, 0, 0, 0, lda, ldw, ldc, sA, sW, sC, a_rows, tiles, 0, 0};
+  PartsArgs a = {C, A, W, M, N, K, 0, 0, 0, lda, ldw, ldc, sA, sW, sC, a_rows, tiles, 0, 0, (float)K * 0x1p-97f};
   a.mt = tiles != nullptr ? ntiles * (4 / fq) : (M + 16 * fq - 1) / (16 * fq);
   a.nt = (N + 16 * cw * wc - 1) / (16 * cw * wc);
   a.batch = tiles != nullptr ? 1 : batch;

@@ -57,6 +57,46 @@ def test_values_without_parts(tile):
     assert ((call(a, w, tile).double() - ref).norm()) <= NORM * ref.norm()
 
 
+@pytest.mark.parametrize("tile", MENU)
+@pytest.mark.parametrize("small,large", [(-116, 60), (-120, 100), (-125, 60), (-136, 100), (-140, 120)])
+def test_small_values_against_large_ones(tile, small, large):
+    """Operands that lose parts to their size, or all of them, where the other side's size makes ordinary outputs of theirs."""
+    M, N, K = 40, 70, 544
+    g = torch.Generator().manual_seed(tile - small)
+    a, w = torch.randn(M, K, generator=g) * 2.0**small, torch.randn(N, K, generator=g) * 2.0**large
+    a[7] = 0.0
+    for x, y in ((a.cuda(), w.cuda()), (w.cuda(), a.cuda())):
+        ref = x.double() @ y.double().T
+        got = call(x, y, tile).double()
+        assert (got - ref).norm() <= NORM * ref.norm()
+        assert (got[ref == 0] == 0).all()
+
+
+@pytest.mark.parametrize("tile", MENU)
+def test_rows_and_columns_of_every_size(tile):
+    """Each output by the sizes of its own row and column, whatever lies beside them; rows and columns that do not fill the tiles."""
+    M, N, K = 16 * (tile % 10) + 5, 16 * (tile // 10 % 10) * (tile // 100) + 6, 288
+    g = torch.Generator().manual_seed(tile)
+    a = torch.randn(M, K, generator=g) * 2.0**torch.tensor([-120.0, 0.0, 20.0, -60.0])[torch.arange(M) % 4, None]
+    w = torch.randn(N, K, generator=g) * 2.0**torch.tensor([100.0, -20.0, 0.0])[torch.arange(N) % 3, None]
+    a, w = a.cuda(), w.cuda()
+    ref, most = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    assert ((call(a, w, tile).double() - ref).abs() <= 2.0**-20 * most + 2.0**-120).all()
+
+
+@pytest.mark.parametrize("tile", [111, 224, 826])
+def test_results_next_to_the_largest(tile):
+    """High parts whose product rounds to infinity where the values' own does not; sums that are infinite stay so."""
+    M, N, K = 20, 40, 96
+    a, w = torch.zeros(M, K, device="cuda"), torch.ones(N, K, device="cuda")
+    most = 2.0 - 2.0**-23
+    a[:, 5], w[:, 5] = most * 2.0**63, most * 2.0**63
+    a[3, 5] = -a[3, 5]
+    a[4, 6] = 3e38
+    y, ref = call(a, w, tile), (a.double() @ w.double().T).float()
+    assert torch.equal(y, ref) and ref[4].isinf().all() and ref[:3].isfinite().all()
+
+
 @pytest.mark.parametrize("fq,tile", [(1, 111), (2, 222), (4, 224), (4, 424)])
 def test_listed_tiles(fq, tile):
     g = torch.Generator().manual_seed(tile)
