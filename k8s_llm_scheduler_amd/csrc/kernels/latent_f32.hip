@@ -84,12 +84,13 @@ __global__ __launch_bounds__(256, 1) void latent_f32_kernel(
     }
     top = lane_max<16>(top);
     top = lane_max<32>(top);
-    const float mn = fmaxf(m, top), alpha = m == -INFINITY ? 0.f : expf(m - mn);
+    const float mn = fmaxf(m, top), ref = mn == -INFINITY ? 0.f : mn;            // scores of -infinity so far: they weigh nothing
+    const float alpha = m == -INFINITY ? 0.f : expf(m - ref);
     m = mn;
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      w[i] = expf(w[i] - mn);
+      w[i] = expf(w[i] - ref);
       sum += w[i];
     }
     l = l * alpha + sum;

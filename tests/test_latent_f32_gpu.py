@@ -53,6 +53,22 @@ def test_against_64_bits(C, R, H, window, bs, extra, monkeypatch):
     assert err[0] <= 2e-6 and err[0] <= 1.25 * err[1], err        # scores of up to 10: a part in 2^22 of them, and no more than plain FMAs give
 
 
+@pytest.mark.parametrize("first,last", [(0, 16), (16, 32), (0, 64), (48, 101)])
+def test_scores_of_minus_infinity(first, last):
+    """Keys whose scores overflow to -infinity weigh nothing, wherever a wave meets them."""
+    C, R, H, Dn, bs, p = 64, 32, 4, 8, 16, 100
+    g = torch.Generator().manual_seed(first + last)
+    cache = torch.randn(7 * bs, C + R, generator=g)
+    cache[:, C] = 0.0
+    cache[first:last, C] = -1e20
+    qa, q = torch.randn(1, H, C, generator=g), torch.randn(1, H * (Dn + R), generator=g)
+    q.view(H, Dn + R)[:, Dn] = 1e20
+    bt, seq, pos = torch.arange(7, dtype=torch.int32)[None], torch.zeros(1, dtype=torch.int32), torch.tensor([p], dtype=torch.int32)
+    want = exact(qa, q, cache, bt, seq, pos, C, R, H, Dn, 0, 0.1, bs, None, None)
+    y = sm.latent_attention(qa.cuda(), q.cuda(), cache.cuda(), bt.cuda(), seq.cuda(), pos.cuda(), C, R, H, Dn, 0, 0.1, bs).cpu().double()
+    assert float((y - want).norm()) <= 2e-6 * float(want.norm())
+
+
 @pytest.mark.parametrize("H,lens,past,window", [(16, (4, 9), 600, 0), (16, (97, 1, 1), 300, 1024), (20, (30, 3), 1000, 70), (32, (60, 5), 130, 0),
                                                 (16, (5, 2), 189, 0), (3, (8,), 2000, 0)])
 def test_key_splits_of_portions_in_bf16(H, lens, past, window):
