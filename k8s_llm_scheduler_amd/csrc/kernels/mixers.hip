@@ -883,14 +883,15 @@ __global__ __launch_bounds__(64 * NWV) void latent_attention_mfma_kernel(
       }
     tmax = lane_max<16>(tmax);
     tmax = lane_max<32>(tmax);
-    const float m_new = fmaxf(m_run, tmax);       // finite: the step holds a visible key
-    const float alpha = m_run == -INFINITY ? 0.f : __expf(m_run - m_new);
+    const float m_new = fmaxf(m_run, tmax);
+    const float m_ref = m_new == -INFINITY ? 0.f : m_new;   // visible keys' scores of -infinity so far: they weigh nothing
+    const float alpha = m_run == -INFINITY ? 0.f : __expf(m_run - m_ref);
     float rsum = 0.f;
 #pragma unroll
     for (int m = 0; m < 2; ++m)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float pv = __expf(sacc[m][i] - m_new);     // the weights are rounded to bf16 for the product
+        const float pv = __expf(sacc[m][i] - m_ref);     // the weights are rounded to bf16 for the product
         sacc[m][i] = pv;
         rsum += pv;
       }

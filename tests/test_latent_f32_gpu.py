@@ -69,6 +69,26 @@ def test_scores_of_minus_infinity(first, last):
     assert float((y - want).norm()) <= 2e-6 * float(want.norm())
 
 
+@pytest.mark.parametrize("first,last", [(0, 32), (128, 160), (256, 512)])
+def test_scores_of_minus_infinity_in_bf16_splits(first, last):
+    """The same for four tokens a workgroup, where those keys are the first of a split, or a whole one."""
+    C, R, H, Dn, bs, T, past = 512, 64, 16, 16, 16, 200, 400
+    g = torch.Generator().manual_seed(first)
+    pos, seq = torch.arange(past, past + T, dtype=torch.int32), torch.zeros(T, dtype=torch.int32)
+    nb = (past + T) // bs + 1
+    bt, cu = torch.arange(nb, dtype=torch.int32)[None], torch.tensor([0, T], dtype=torch.int32)
+    cache = torch.randn(nb * bs, C + R, generator=g).bfloat16()
+    cache[:, C] = 0.0
+    cache[first:last, C] = -1e30
+    qa, q = torch.randn(T, H, C, generator=g).bfloat16(), torch.randn(T, H * (Dn + R), generator=g).bfloat16()
+    q.view(T, H, Dn + R)[:, :, Dn] = 1e30
+    assert sm.latent_quad_splits(T, 1, H, nb * bs) > 1
+    want = exact(qa, q, cache, bt, seq, pos, C, R, H, Dn, 0, 0.04, bs, None, None)
+    y = sm.latent_attention(qa.cuda(), q.cuda(), cache.cuda(), bt.cuda(), seq.cuda(), pos.cuda(), C, R, H, Dn, 0, 0.04, bs, 0, cu.cuda(),
+                            T).cpu().double()
+    assert float((y - want).norm()) <= 2.0**-7 * float(want.norm())          # (weights and result rounded to bf16)
+
+
 @pytest.mark.parametrize("H,lens,past,window", [(16, (4, 9), 600, 0), (16, (97, 1, 1), 300, 1024), (20, (30, 3), 1000, 70), (32, (60, 5), 130, 0),
                                                 (16, (5, 2), 189, 0), (3, (8,), 2000, 0)])
 def test_key_splits_of_portions_in_bf16(H, lens, past, window):
