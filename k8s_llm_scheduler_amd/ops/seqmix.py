@@ -955,7 +955,7 @@ def latent_splits(T: int, H: int, max_keys: int) -> int:
 def latent_quad_splits(T: int, nseq: int, H: int, max_keys: int) -> int:
     """Key splits of portions of ``nseq`` sequences, ``T`` tokens in all, whose workgroups are four consecutive tokens."""
     groups = min(T, T // 4 + nseq) * ((H + 15) // 16)
-    return max(1, min(256 // groups, (max(1, max_keys) + 63) // 64, 32))
+    return max(1, min(256 // groups, (max(1, max_keys) + 63) // 64, 32, 65535 // nseq))       # (the grid's third side)
 
 
 def latent_attention(q_abs: torch.Tensor, q: torch.Tensor, cache: torch.Tensor, block_tables: torch.Tensor,
