@@ -8,8 +8,9 @@
 // token's keys run the second product token by token, with the values that it does not see as zeros.
 // Bound by the fp32 matrix rate (a tile is 64 products of 32 cycles at 128 dimensions) and the loads' way where there are few tiles.
 // us, plain FMAs (a workgroup a token, keys in LDS) / here, 16 heads over 4 of 128, window 1024: 300 tokens 144 / 28, 2 x 100 behind 400
-// 221 / 29, 512 behind 500 861 / 73, 97 behind 1000 251 / 50, 24 fresh 17 / 11, 24 behind 1000 66 / 44 (splits of the keys would help there);
-// 32 over 8, 300 tokens 239 / 38; 2 tokens behind 3000 102 / 104.
+// 221 / 29, 512 behind 500 861 / 73, 97 behind 1000 251 / 50, 24 fresh 17 / 11, 24 behind 1000 66 / 44; 32 over 8, 300 tokens 239 / 38.  Few
+// tokens behind many keys, which a workgroup walks by itself, are left to that kernel's key splits (2 behind 3000 59 / 104) by
+// ops/seqmix.py window_f32_plain.
 #include "common.h"
 
 namespace k8sllm {

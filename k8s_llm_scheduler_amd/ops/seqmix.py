@@ -1352,6 +1352,30 @@ def prompt_splits(groups: int, keys: int) -> int:
     return max(1, min(most // max(1, groups), -(-max(1, keys) // 128), 6))
 
 
+# fp32 portions: us of the plain-FMA kernel (a workgroup a token, key head and key split), head size and heads a key head -> (the splits'
+# merge, per key of a split, whole tiles of them, and round of 512 workgroups, 1024 at 64 dimensions); of window_f32.hip, which has no
+# splits, head size -> (fixed, per token of a workgroup, whose last keys it weighs token by token, per key).  Fitted to 901 batches of 2 - 97
+# tokens behind 30 - 30000 (1 - 8 sequences, 1 - 16 heads a key head): rms error 12 - 26 % and 6 - 8 %.
+_WINDOW_PLAIN_COST = {(64, 1): (3.1, 0.22), (64, 2): (3.3, 0.189), (64, 4): (4.1, 0.171), (64, 8): (2.8, 0.201), (64, 16): (6.2, 0.267),
+                      (128, 1): (1.1, 0.386), (128, 2): (3.9, 0.302), (128, 4): (4.4, 0.272), (128, 8): (5.9, 0.259), (128, 16): (5.5, 0.471)}
+_WINDOW_F32_COST = {64: (5.4, 0.536, 0.0202), 128: (6.9, 0.868, 0.0354)}
+
+
+@functools.lru_cache(maxsize=4096)
+def window_f32_plain(T: int, longest: int, H: int, G: int, D: int, keys: int, splits: int, tile_rows: int) -> bool:
+    """Whether fp32 portions of ``T`` tokens, ``longest`` of one sequence, that see up to ``keys`` keys stay on the plain-FMA kernel and
+    its ``splits``: few tokens behind many keys, since a workgroup of the other walks all of them.  Plain / window_f32.hip, us, 16 heads
+    over 4 of 128: 2 tokens behind 250 19.8 / 17.3, 1000 33 / 41, 3000 59 / 104, 30000 471 / 1093; 8 behind 3000 70 / 106; 16 128.8 / 121.5; 24
+    180 / 122; of 64, 8 behind 1000 15.6 / 26.5, 24 27.0 / 26.7; 8 heads over 8 of 64, 16 fresh tokens 12.2 / 14.7.  Within 5 % of each other
+    the plain one: of the 901 two are more than 3 % slower than on it, 48 than on the other, 1.2 % from the faster one on average.  ``keys`` is
+    what the launch knows; where there are fewer than it says, this is the time there was (2 behind 30 13.2 / 9.1)."""
+    merge, key = _WINDOW_PLAIN_COST[D, H // G]
+    fixed, token, each = _WINDOW_F32_COST[D]
+    chain = -(-(-(-keys // splits)) // tile_rows) * tile_rows
+    plain = (merge if splits > 1 else 0.0) + key * chain * max(1.0, T * G * splits / (1024 if D == 64 else 512))
+    return plain < 1.05 * (fixed + token * min(longest, 16 * G // H) + each * keys)
+
+
 def window_attention(q: torch.Tensor, gate: Optional[torch.Tensor], kcache: torch.Tensor, vcache: torch.Tensor,
                      kpool: Optional[torch.Tensor], vpool: Optional[torch.Tensor], block_tables: torch.Tensor,
                      tok_seq: torch.Tensor, positions: torch.Tensor, H: int, window: int, P: int, scale: float,
@@ -1369,8 +1393,9 @@ def window_attention(q: torch.Tensor, gate: Optional[torch.Tensor], kcache: torc
     is taken off the score of the token at position j (not off the sink's; not with pooled blocks).
     ``cu_q`` / ``max_qlen`` (the sequences' query offsets and longest portion): bf16 portions of prompts whose sizes
     fit run on the matrix cores, tiles of consecutive tokens sharing the staged keys; so do bf16 tokens one by one
-    (decoding, or query groups that make no tile) without pooled blocks, and fp32 portions of the usual sizes without them; anything
-    else on the plain-FMA kernel.  The keys of few tokens are split over several workgroups
+    (decoding, or query groups that make no tile) without pooled blocks, and fp32 portions of the usual sizes without them but few
+    tokens behind many keys (:func:`window_f32_plain`); anything else on the plain-FMA kernel.  The keys of few tokens are split over
+    several workgroups, but for those fp32 portions
     (``max_keys``: an upper bound of the positions any token sees, 0: the block tables' capacity)."""
     G, D, V = kcache.shape[1], kcache.shape[2], vcache.shape[2]
     if H % G:
@@ -1413,15 +1438,20 @@ def window_attention(q: torch.Tensor, gate: Optional[torch.Tensor], kcache: torc
                                   float(scale), int(bool(sink)), block_size, ns, int(chunk), float(softcap), _p(sinks),
                                   int(bool(gate_per_head)), _p(slopes), -1)
         return out
-    if (WINDOW_MFMA and dt == F32 and P <= 0 and cu_q is not None and max_qlen > 1 and nat.window_f32_ok(H, G, D, V)
-            and q.stride(0) % 4 == 0 and (q.data_ptr() | kcache.data_ptr() | vcache.data_ptr()) % 16 == 0):
-        nat.window_f32(out.data_ptr(), q.data_ptr(), q.stride(0), gate.data_ptr() if gate is not None else 0,
-                       gate.stride(0) if gate is not None else 0, _p(kcache, dt, "kcache"), _p(vcache, dt, "vcache"),
-                       _p(block_tables, I32, "block_tables"), block_tables.shape[1], _p(cu_q, I32, "cu_q"), _p(positions, I32),
-                       cu_q.shape[0] - 1, int(max_qlen), H, G, D, V, int(window), float(scale), int(bool(sink)), block_size, int(chunk),
-                       float(softcap), _p(sinks), int(bool(gate_per_head)), _p(slopes), -1)
-        return out
     max_pos = max_keys or block_tables.shape[1] * block_size
+    span = chunk if chunk > 0 else window
+    if (WINDOW_MFMA and dt == F32 and P <= 0 and cu_q is not None and max_qlen > 1 and nat.window_f32_ok(H, G, D, V)
+            and q.stride(0) % 4 == 0 and (q.data_ptr() | kcache.data_ptr() | vcache.data_ptr()) % 16 == 0 and cu_q.shape[0] <= 65536):
+        rows = nat.window_tile_rows(H, G, D, V)
+        plain = rows > 0 and window_f32_plain(T, int(max_qlen), H, G, D, min(max_pos, span) if span > 0 else max_pos,
+                                              window_splits(T, G, span, 0, max_pos, rows), rows)
+        if not plain:
+            nat.window_f32(out.data_ptr(), q.data_ptr(), q.stride(0), gate.data_ptr() if gate is not None else 0,
+                           gate.stride(0) if gate is not None else 0, _p(kcache, dt, "kcache"), _p(vcache, dt, "vcache"),
+                           _p(block_tables, I32, "block_tables"), block_tables.shape[1], _p(cu_q, I32, "cu_q"), _p(positions, I32),
+                           cu_q.shape[0] - 1, int(max_qlen), H, G, D, V, int(window), float(scale), int(bool(sink)), block_size,
+                           int(chunk), float(softcap), _p(sinks), int(bool(gate_per_head)), _p(slopes), -1)
+            return out
     if (WINDOW_MFMA and dt == BF16 and P <= 0 and nat.window_token_ok(H, G, D, V, block_size) and q.stride(0) % 8 == 0
             and q.data_ptr() % 16 == 0):
         ns = token_splits(T, G, min(max_pos, chunk or window or max_pos), D, max_keys > 0)
@@ -1436,7 +1466,7 @@ def window_attention(q: torch.Tensor, gate: Optional[torch.Tensor], kcache: torc
                          int(bool(sink)), block_size, ns, int(chunk), float(softcap), _p(sinks), int(bool(gate_per_head)),
                          _p(slopes), -1)
         return out
-    ns = window_splits(T, G, window if chunk <= 0 else chunk, P, max_pos, nat.window_tile_rows(H, G, D, V))
+    ns = window_splits(T, G, span, P, max_pos, nat.window_tile_rows(H, G, D, V))
     pacc = pml = None
     if ns > 1:
         pacc = torch.empty(T * H * ns * V, dtype=F32, device=q.device)
