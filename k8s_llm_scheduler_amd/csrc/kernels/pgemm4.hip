@@ -153,7 +153,7 @@ int p4_act(const P4Args& a, int cfg, int kind, bool grouped, hipStream_t s) {
   return grouped ? p4_act_cfg<true, 1, P4_TILES>(a, cfg, kind, s) : p4_act_cfg<false, 1, P4_TILES>(a, cfg, kind, s);
 }
 }  // namespace
-P4Args p4_args(void* out, const void* x, const void* W, int M, int N_out, int K, bool pair, int cfg, int group_m) {
+P4Args p4_args(void* out, const void* x, const void* W, int M, int N_out, int K, bool pair, int cfg, int group_m, int groups = 0) {
   const int bp = 32 * p4_tile(cfg).fp, bq = 32 * p4_tile(cfg).fq, feat = pair ? bp / 2 : bp;
   P4Args a = {};
   a.out = out;
@@ -171,6 +171,7 @@ P4Args p4_args(void* out, const void* x, const void* W, int M, int N_out, int K,
   a.splits = 1;
   a.group_m = group_m > 0 ? group_m : 1;
   a.nwg = a.m_tiles * a.n_tiles;
+  a.groups = groups;
   a.spread = a.m_tiles == 1;
   p4_walk(a, cfg);
   a.wide = N_out % 8 == 0 && ((uintptr_t)out & 15) == 0;
@@ -286,10 +287,9 @@ extern "C" int k8s_pgemm4_grouped(void* out, const void* x, const void* W, int M
   if (ldx < K || ldx % 8 || (((uintptr_t)x | (uintptr_t)W) & 15) || ((uintptr_t)out & 7)) return -1;
   const long long kbytes = (long long)K * 2, wrows = (pair ? 2LL : 1LL) * N_out;
   if (wrows * kbytes >= (1LL << 32) || (long long)M * ldx * 2 >= (1LL << 32)) return -5;   // 32-bit DMA offsets
-  P4Args a = p4_args(out, x, W, rows, N_out, K, pair, cfg, group_m);
+  P4Args a = p4_args(out, x, W, rows, N_out, K, pair, cfg, group_m, groups);
   const int bq = 32 * p4_tile(cfg).fq;
   a.m_tiles = rows / bq + groups;        // whole tiles, and a partial one per group
-  a.groups = groups;
   a.spread = groups >= 8 && rows <= 192LL * groups;
   a.fine = 0;
   p4_walk(a, cfg);

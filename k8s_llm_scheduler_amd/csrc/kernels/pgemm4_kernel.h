@@ -24,8 +24,10 @@
 //    same lines of x (loads alone, 32768 rows of 16 KB: 4.1 -> 6 TB/s).  241 x 57344 x 8192 251 -> 230 us, 8192 x 28672 136 -> 131,
 //    8192 x 8192 50 -> 47.  With more row tiles the walk in step is the better one (2048 x 16384 x 2048 106 -> 111): so not there; the
 //    grouped form by its rows (P4Args::spread); but deep ones, whose rows' strides put whole columns of tiles on the same channels, from
-//    16384 columns on up to 8 row tiles (x 8192 x 28672, 333 rows 171 -> 151 us, 512 204 -> 192, 1024 363 -> 348, 2048 675 -> 654; 3413
-//    1265 -> 1279; of 14336 columns and fewer 1 % slower on average).
+//    16384 columns on up to 8 row tiles, which then follow each other (group_m): 7 weights of 4096 - 16384 x 16384 - 28672, 333 - 2048 rows,
+//    12 % less time with 2 row tiles, 5 - 8 % with 3 - 7, 3 % with 8 (at most 5 % more, on 5120 x 20480 with 8); 8192 x 28672, 333 rows 164 ->
+//    152 us, 1536 525 -> 490; 12288 x 24576, 333 237 -> 192.  In groups of 4, 6 and 8 row tiles were 1 % slower than in step, in groups of 2 1 - 4 %
+//    whatever their number.  3413 rows of 8192 x 28672 1265 -> 1279; of 14336 columns and fewer 1 % slower on average.
 //  * rows of 4 KB and less (K up to 2048) on tiles of at most 128 x 128 and on those of 32 tokens: every column of tiles starts its walk
 //    an eighth of it after the one before (P4Args::fine): at one k the rows' bytes lie in a few of the memory's channels, and short
 //    tiles have no time to drift apart.  us: 2048 x 2048 x 2048 21.1 -> 19.0, 1024 x 3072 x 2048 19.1 -> 16.3, 512 x 3648 x 2048 16.4 ->
@@ -600,7 +602,7 @@ constexpr P4Cfg kP4Few[] = {
 };
 constexpr int kP4Grouped = kP4NumCfgs + sizeof(kP4Few) / sizeof(kP4Few[0]);
 constexpr P4Cfg p4_tile(int c) { return c < kP4NumCfgs ? kP4Cfgs[c] : kP4Few[c - kP4NumCfgs]; }
-// the walks of P4Args::spread and fine
+// the walks of P4Args::spread and fine, and what goes with them
 inline void p4_walk(P4Args& a, int cfg) {
   const P4Cfg t = p4_tile(cfg);
   if (a.K <= 2048 && (t.fq == 1 || (t.fp <= 4 && t.fq <= 4))) {
@@ -608,6 +610,7 @@ inline void p4_walk(P4Args& a, int cfg) {
     a.fine = 4;
   } else if (a.K >= 16384 && a.m_tiles <= 8 && a.groups == 0) {
     a.spread = 1;
+    if (a.group_m < a.m_tiles) a.group_m = a.m_tiles;
   }
 }
 

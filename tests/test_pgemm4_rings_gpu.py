@@ -119,3 +119,16 @@ def test_walks_over_k(cfg, K):
     out = torch.empty(M, N // 2, dtype=torch.bfloat16, device="cuda")
     ops.native().pgemm4_act(out.data_ptr(), x.data_ptr(), w.data_ptr(), M, N // 2, K, cfg, 4, sm.ACT_RELU, 0.0, 1.0, 0, -1)
     assert torch.equal(out, (y[:, :N // 2].clamp(min=0) * y[:, N // 2:]).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("cfg", [3, 8, 13])
+@pytest.mark.parametrize("tiles", [5, 8, 9])
+@pytest.mark.parametrize("group_m", [1, 4])
+def test_deep_weights_in_one_group_of_row_tiles(cfg, tiles, group_m):
+    """From 16384 columns on up to 8 row tiles follow each other whatever group they are asked for in; 9 do not."""
+    bp, bq = TILES[cfg]
+    M, N, K = tiles * bq - 3, 2 * bp + 8, 16384
+    x, w = whole(M, K, tiles), whole(N, K, cfg)
+    y = x.float() @ w.float().T                       # whole numbers below 2^24
+    assert torch.equal(ops.pgemm4(x, w, ops.EPI_F32, cfg=cfg, group_m=group_m), y)
+    assert torch.equal(ops.pgemm4(x, w, ops.EPI_F32, cfg=cfg, group_m=group_m, splits=3), y)
