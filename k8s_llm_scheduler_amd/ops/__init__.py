@@ -1017,11 +1017,12 @@ def pgemm4(x: torch.Tensor, w: torch.Tensor, epi: int = EPI_BF16, cfg: int = 0, 
 # ----------------------------------------------------------------------------- GEMM routing (M > GEMV_MAX_M)
 # Tuned big-tile plans: engine/assets/pgemm_gfx950.json, written by tools/pgemm_tune.py, keyed "M,N,K,epi,fp8" ->
 # [kernel, cfg, splits, group_m, us, library us].  A row count between tuned buckets takes the plan of the nearest
-# bucket at or above it; past the largest tuned bucket, the largest one's (big tiles, no split-K: it only gets
-# better with more rows).
+# bucket at or above it (in bf16 on a tile that suits its rows better, gemm_route; a table that K8S_PGEMM_TABLE_PATH names is
+# followed as it is); past the largest tuned bucket, the largest one's (big tiles, no split-K: it only gets better with more rows).
 _PG_TABLE: Optional[dict] = None
 PG_TABLE_PATH = os.environ.get("K8S_PGEMM_TABLE_PATH") or os.path.join(   # (override: in-situ table A/B runs)
     os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "engine", "assets", "pgemm_gfx950.json")
+PG_TABLE_NAMED = bool(os.environ.get("K8S_PGEMM_TABLE_PATH"))
 PG_MIN_M = 129      # below: mgemm's streaming tiles (batched decode, short prefill chunks)
 
 
@@ -1237,7 +1238,7 @@ def gemm_route(M: int, N: int, K: int, epi: int, fp8: bool) -> Tuple[str, Option
         return plan[0], plan[1:]
     if plan[0] == "mgemm":   # (the tuner records it where its tuned plan was faster)
         return "mgemm", None
-    if plan[0] == "pgemm4" and not fp8 and pg_us is not None and (N, K, epi, 0) in _pg_load_table() and \
+    if plan[0] == "pgemm4" and not fp8 and pg_us is not None and not PG_TABLE_NAMED and (N, K, epi, 0) in _pg_load_table() and \
             all(r[0] != M for r in _PG_TABLE[N, K, epi, 0]):
         # tuned for more rows than these: 60 products of 161 - 2089 rows 5 % less time on average, up to 28 %, none slower (1169 x 6144 x 4096
         # 73 -> 53 us, 535 x 4096 x 14336 81 -> 65)

@@ -31,6 +31,12 @@ def test_tuned_plans_stay_at_their_row_count(monkeypatch):
     assert ops.gemm_route(850, 8192, 512, 0, False) == ("pgemm", (0, 1, 4))
 
 
+def test_plans_of_a_table_that_is_named_stand(monkeypatch):
+    monkeypatch.setattr(ops, "_PG_TABLE", {(10240, 8192, 0, 0): [(1024, "pgemm4", 8, 1, 4, 137.0), (1536, "pgemm4", 0, 1, 8, 175.0)]})
+    monkeypatch.setattr(ops, "PG_TABLE_NAMED", True)
+    assert ops.gemm_route(1300, 10240, 8192, 0, False) == ("pgemm4", (0, 1, 8)) == ops.gemm_route(1536, 10240, 8192, 0, False)
+
+
 @pytest.mark.parametrize("rows,E,N,K,pair,even,common,want", [
     (4602, 9, 2048, 2048, True, False, 1534, 15), (2800, 4, 2048, 2048, False, True, 0, 12), (8192, 4, 2048, 2048, False, True, 0, 4),
     (2800, 4, 512, 2048, False, True, 0, None), (249, 9, 2048, 2048, True, False, 83, None), (288, 9, 2048, 2048, True, False, 96, None),
