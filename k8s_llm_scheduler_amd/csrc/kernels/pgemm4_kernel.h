@@ -585,7 +585,7 @@ constexpr P4Cfg kP4Cfgs[] = {
     {4, 6, 2, 1},   // 12: 128 x 192
     {6, 6, 2, 1},   // 13: 192 x 192
     {7, 6, 2, 1},   // 14: 224 x 192
-    {6, 7, 2, 1},   // 15: 192 x 224
+    {6, 7, 2, 1},   // 15: 192 x 224 (ungrouped for tuned plans alone: ops/__init__.py has no figures for it off the table)
     {7, 7, 2, 1},   // 16: 224 x 224
     {8, 7, 2, 1},   // 17: 256 x 224
 };
@@ -676,10 +676,14 @@ int p4_act_kind(const P4Args& a, int kind, hipStream_t s) {
   }
   return -1;
 }
+// the grouped form is built on the tiles that ops/seqmix.py's rules take
+constexpr bool p4_grouped(int cfg) { return cfg != 9 && cfg != 14; }
 template <bool GRP, int C, int END>
 int p4_act_cfg(const P4Args& a, int cfg, int kind, hipStream_t s) {
   if constexpr (C < END) {
-    if (cfg == C) return p4_act_kind<C, GRP>(a, kind, s);
+    if constexpr (!GRP || p4_grouped(C)) {
+      if (cfg == C) return p4_act_kind<C, GRP>(a, kind, s);
+    }
     return p4_act_cfg<GRP, C + 1, END>(a, cfg, kind, s);
   } else {
     return -4;

@@ -45,3 +45,8 @@ def test_plans_of_a_table_that_is_named_stand(monkeypatch):
 def test_grouped_picks(rows, E, N, K, pair, even, common, want):
     got = sm._grouped_plan(rows, E, N, K, pair, even, common)
     assert got == (want if want is not None else sm._grouped_tile(rows, E, N, K, pair, even, common))
+
+
+def test_rules_of_grouped_products_take_every_tile_that_is_built():
+    """... and no other: 128 x 96 (9) and 224 x 192 (14) are not."""
+    assert set(sm._GROUP_MORE_COST) | set(sm._GROUP_FEW_TILE) | {4} == set(range(1, len(ops.pgemm4_configs()) + 4)) - {9, 14}
