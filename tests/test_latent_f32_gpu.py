@@ -92,12 +92,15 @@ def test_scores_of_minus_infinity_in_bf16_splits(first, last):
 @pytest.mark.parametrize("H,lens,past,window", [(16, (4, 9), 600, 0), (16, (97, 1, 1), 300, 1024), (20, (30, 3), 1000, 70), (32, (60, 5), 130, 0),
                                                 (16, (5, 2), 189, 0), (3, (8,), 2000, 0)])
 def test_key_splits_of_portions_in_bf16(H, lens, past, window):
-    """Four tokens a workgroup, their keys split: fewer keys than a split, around the fewest that are split, splits that stay empty; idle
-    rows at a batch's end; sinks and gates through the kernel that joins and through the one that has nothing to join."""
-    C, R, Dn, bs = 512, 64, 16, 16
+    """Four tokens a workgroup, their keys split: fewer keys than a split, around the fewest that are split, splits that stay empty; an
+    idle sequence at the batch's end, whose workgroups leave no records; sinks and gates through the kernel that joins and through the
+    one that has nothing to join."""
+    C, R, Dn, bs, idle = 512, 64, 16, 16, 5
     g = torch.Generator().manual_seed(past + H)
-    n, T = len(lens), sum(lens)
+    n, lens = len(lens) + 1, (*lens, idle)
+    T = sum(lens)
     pos = torch.cat([torch.arange(k) + (past if i != 1 else 0) for i, k in enumerate(lens)]).int()
+    pos[-idle:] = -1
     seq = torch.cat([torch.full((k,), i) for i, k in enumerate(lens)]).int()
     nb = (past + max(lens)) // bs + 1
     bt = torch.randperm(n * nb, generator=g).view(n, nb).int()
@@ -106,9 +109,17 @@ def test_key_splits_of_portions_in_bf16(H, lens, past, window):
     qa, q = torch.randn(T, H, C, generator=g).bfloat16(), torch.randn(T, H * (Dn + R), generator=g).bfloat16()
     sinks, gate = torch.randn(H, generator=g), torch.randn(T, H, generator=g).bfloat16()
     scale = (C + R)**-0.5
-    assert sm.latent_quad_splits(T, n, H, nb * bs) > 1
+    ns = sm.latent_quad_splits(T, n, H, min(window or nb * bs, nb * bs))
+    assert ns > 1
     want = exact(qa, q, cache, bt, seq, pos, C, R, H, Dn, window, scale, bs, sinks, gate)
-    y = sm.latent_attention(qa.cuda(), q.cuda(), cache.cuda(), bt.cuda(), seq.cuda(), pos.cuda(), C, R, H, Dn, window, scale, bs, 0, cu.cuda(),
-                            max(lens), sinks=sinks.cuda(), gate=gate.cuda()).cpu().double()
+    args = [x.cuda() for x in (qa, q, cache, bt, seq, pos)]
+    kw = dict(sinks=sinks.cuda(), gate=gate.cuda())
+    cu = cu.cuda()
+    HP = (H + 15) // 16 * 16
+    stale = [torch.full((k,), float("nan"), device="cuda") for k in (T * HP * ns * C, T * HP * ns * 2, (T * H * C + 1) // 2)]
+    del stale                  # what the result and the records are given: one that is read without being written shows
+    y = sm.latent_attention(*args, C, R, H, Dn, window, scale, bs, 0, cu, max(lens), **kw).cpu().double()
+    assert (y[-idle:] == 0).all()
+    T -= idle
     for t in range(T):          # weights and result rounded to bf16: 2^-9 of each, 2-norm below 2^-8 a row
         assert float((y[t] - want[t]).norm()) <= 2.0**-7 * float(want[t].norm()), t
