@@ -273,6 +273,7 @@ int k8s_gated_scan(void* out, const void* proj, long ld, int kind, int cq, int c
 long long k8s_gated_scan_workspace(int T, int nseq, int H, int D, int V, int Lc);
 int k8s_decay_scan_ok(int D, int V);
 long long k8s_decay_scan_workspace(int T, int nseq, int H, int D, int V);
+int k8s_decay_scan_once(int nseq, int H, int V, int max_qlen);
 int k8s_decay_scan(float* out, const void* proj, long ld, int cq, int ck, int cv, const float* decay, float* state,
                    const int* cu_q, const int* seq_slots, const int* positions, int nseq, int H, int D, int V, int R,
                    int T, int max_qlen, void* ws, hipStream_t s);
@@ -890,6 +891,7 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
   m.def("decay_scan_workspace", [](int T, int nseq, int H, int D, int V) {
     return k8s_decay_scan_workspace(T, nseq, H, D, V);
   });
+  m.def("decay_scan_once", [](int nseq, int H, int V, int max_qlen) { return k8s_decay_scan_once(nseq, H, V, max_qlen) != 0; });
   m.def("decay_scan", [](uintptr_t out, uintptr_t proj, long ld, int cq, int ck, int cv, uintptr_t decay, uintptr_t state,
                          uintptr_t cu_q, uintptr_t seq_slots, uintptr_t positions, int nseq, int H, int D, int V, int R,
                          int T, int max_qlen, uintptr_t ws, int64_t s) {

@@ -9,7 +9,7 @@
 //   decay_prefix_kernel  per (sequence, head, state elements): walks the sequence's chunks from the slot's state, leaves
 //                        every chunk's S0 in the place of its sum and, at the end, the slot's new state;
 //   decay_out_kernel     per (chunk, head, slice of value columns): the outputs, fp32.
-// Where no portion is longer than one chunk the last does it all.
+// Where no portion is longer than one chunk, or two of them and there are more than 16 workgroups, the last does it all.
 // Exactness: q, k, v enter the products as bf16 (activations); the decay weights, the scores and the state are fp32 and
 // enter a product as two bf16 terms (hi + lo, 16 bits of mantissa together); sums are fp32.
 //
@@ -224,8 +224,10 @@ __global__ __launch_bounds__(256) void decay_prefix_kernel(float* __restrict__ r
 // addresses), not by memory or the matrix cores.  Hence 8 waves of 16 value columns (4 of 32 before), every load under way
 // before the first use, powers by a table, the queries staged beside the keys, states handed on as one fp32 record.  All three
 // kernels, 128 channels, before and after, us: 2048 tokens of 16 heads 61.6 -> 50, of 32 96.4 -> 79; 512 of 32 41.7 -> 34;
-// 100 of 16 26.0 -> 19.5; 60 of 16 24.9 -> 11.6, 100 by ONCE 20.2.  Segments of two chunks a workgroup (half the records) were
-// slower below a thousand workgroups: 2048 tokens of 16 heads 54.9 against 50.1.
+// 100 of 16 26.0 -> 19.5; 60 of 16 24.9 -> 11.6.  ONCE takes 12 us and 8 for a second chunk, the three kernels 19 and more with every
+// workgroup, us, three / ONCE: 128 tokens of 16 heads 20.4 / 20.4, of 8 19.3 / 20.3, of 32 23.3 / 20.8, 3 x 128 of 4 (2 slices) 19.8 / 19.4,
+// 4 x 100 of 32 40 / 22, 16 x 128 of 32 109 / 51.  Segments of two chunks a workgroup (half the records) were slower below a
+// thousand workgroups: 2048 tokens of 16 heads 54.9 against 50.1.
 template <int KK, int NTHR, bool ONCE>
 __global__ __launch_bounds__(NTHR, ONCE ? 1 : NTHR / 128) void decay_out_kernel(float* __restrict__ out, const float* __restrict__ rec, float* __restrict__ state,
                                                            DecayArgs A) {
@@ -421,13 +423,18 @@ extern "C" long long k8s_decay_scan_workspace(int T, int nseq, int H, int D, int
   return chunks * H * rec * 4;
 }
 
+// Whether portions of at most max_qlen tokens run in one launch, which needs no workspace (figures at decay_out_kernel).
+extern "C" int k8s_decay_scan_once(int nseq, int H, int V, int max_qlen) {
+  return max_qlen > 0 && (max_qlen <= DSC_L || (max_qlen <= 2 * DSC_L && (long long)nseq * H * ((V + DSC_VS - 1) / DSC_VS) > 16));
+}
+
 // proj bf16 [T, ld] (16-byte aligned rows and parts); out fp32 [T, H V]; state [slots, H, D V] fp32, updated in place.  max_qlen: no portion
-// is longer; up to 64 tokens no workspace is needed.
+// is longer.
 extern "C" int k8s_decay_scan(float* out, const void* proj, long ld, int cq, int ck, int cv, const float* decay,
                               float* state, const int* cu_q, const int* seq_slots, const int* positions, int nseq, int H,
                               int D, int V, int R, int T, int max_qlen, void* ws, hipStream_t s) {
   if (T <= 0 || nseq <= 0) return 0;
-  const bool once = max_qlen > 0 && max_qlen <= DSC_L;
+  const bool once = k8s_decay_scan_once(nseq, H, V, max_qlen) != 0;
   if (!k8s_decay_scan_ok(D, V) || H <= 0 || H > 65535 || R <= 0 || H % R || (ws == nullptr && !once) || decay == nullptr) return -1;
   if (ld % 8 || cq % 8 || ck % 8 || cv % 8 || ((uintptr_t)proj & 15)) return -1;
   const DecayArgs A{(const bf16_t*)proj, ld, cq, ck, cv, decay, cu_q, seq_slots, positions, nseq, H, D, V, R};

@@ -1497,7 +1497,6 @@ SCAN_CHUNK = int(os.environ.get("K8S_SCAN_CHUNK", "64"))
 SCAN_CHUNK_MIN = int(os.environ.get("K8S_SCAN_CHUNK_MIN", "256"))
 # SCAN_DECAY in bf16 with a portion of at least this many tokens runs on the matrix cores (0: never)
 DECAY_MFMA_MIN = int(os.environ.get("K8S_DECAY_MFMA_MIN", "32"))
-DECAY_CHUNK = 64         # tokens of its chunks: portions of one chunk need no workspace
 
 
 def gated_scan(proj: torch.Tensor, kind: int, cols: dict, normw: torch.Tensor, state: torch.Tensor, cu_q: torch.Tensor,
@@ -1564,7 +1563,7 @@ def gated_scan(proj: torch.Tensor, kind: int, cols: dict, normw: torch.Tensor, s
             and _native().decay_scan_ok(D, V) and proj.data_ptr() % 16 == 0
             and not any(n % 8 for n in (proj.stride(0), c("q"), c("k"), c("v")))):
         ws = torch.empty(_native().decay_scan_workspace(T, nseq, H, D, V), dtype=torch.uint8, device=proj.device) \
-            if max_qlen > DECAY_CHUNK else None
+            if not _native().decay_scan_once(nseq, H, V, int(max_qlen)) else None
         _native().decay_scan(out.data_ptr(), proj.data_ptr(), proj.stride(0), c("q"), c("k"), c("v"), _p(head_params),
                              _p(state), _p(cu_q, I32), _p(seq_slots, I32), _p(positions, I32), nseq, H, D, V, H // G, T,
                              int(max_qlen), _p(ws), -1)

@@ -812,6 +812,30 @@ def test_decay_scan_of_one_launch(H, G, D, V, lens):
     assert (s - t).abs().max() <= 64 * 2 ** -24 * t.abs().max()
 
 
+@pytest.mark.parametrize("lens", [(128, 65, 127, 100), (96, 1, 0, 128), (66, 64, 112, 113)])
+@pytest.mark.parametrize("H,G,D,V", [(8, 4, 128, 128), (6, 3, 40, 56), (5, 5, 96, 160)])
+def test_decay_scan_of_two_chunks_in_one_launch(H, G, D, V, lens):
+    """Two chunks by one kernel beside the three (one token more than one launch takes): equal outputs within the first chunk, the rest and
+    the new states to the order of fp32 sums, as above."""
+    torch.manual_seed(64)
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32)
+    pos = torch.cat([torch.arange(p, p + n) for p, n in zip((0, 5, 0, 130), lens)]).int()
+    slots = torch.tensor([2, 0, 1, 3], dtype=torch.int32)
+    proj, cols, decay, state = _decay_case(torch.bfloat16, H, G, D, V, cu, pos)
+    assert sm._native().decay_scan_once(4, H, V, 128) and not sm._native().decay_scan_once(4, H, V, 129)
+    res = []
+    for most in (128, 129):
+        new = state.to(DEV).clone()
+        res.append((sm.gated_scan(proj.to(DEV), sm.SCAN_DECAY, cols, None, new, cu.to(DEV), slots.to(DEV), pos.to(DEV), H, D, V, 1e-6,
+                                  torch.float32, head_params=decay.to(DEV), groups=G, max_qlen=most), new))
+    (a, s), (b, t) = res
+    for i, n in enumerate(lens):
+        r = slice(int(cu[i]), int(cu[i]) + min(n, 64))
+        assert torch.equal(a[r], b[r])
+    assert (a - b).abs().max() <= 2 ** -14 * b.abs().max()
+    assert (s - t).abs().max() <= 128 * 2 ** -24 * t.abs().max()
+
+
 @pytest.mark.parametrize("lens", [(9, 1, 0, 27), (64, 65, 63, 1), (200, 0, 128, 7), (2, 2, 2, 2), (600, 1, 1, 0)])
 @pytest.mark.parametrize("H,G,D,V", [(4, 2, 16, 24), (3, 3, 40, 56), (2, 1, 128, 128), (6, 3, 64, 8), (2, 2, 8, 248),
                                      (1, 1, 96, 160), (5, 5, 32, 64), (3, 3, 72, 80)])
