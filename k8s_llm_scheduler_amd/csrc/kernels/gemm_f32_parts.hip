@@ -10,8 +10,9 @@
 // most 2^-126 times the other side's value, and six times 2^-126.  So an output is computed again with plain fp32 FMAs where it is not
 // finite, where it is smaller than K 2^-97 times the largest value of its row and column (or 1: above that what may be lost is 2^-25
 // of it and less), and where it is zero though both have values.  The largest values are met on the way to the parts, one
-// instruction for two of them.  A lane computes its 4 columns again, so a row or a column of such outputs costs a walk over k at the
-// speed of loads: with one NaN in a row 333 x 2048 x 8192 takes 470 us instead of 101, with an infinity in a column 430.
+// instruction for two of them.  A wave computes such an output together: one does not show (a sum may happen to be zero, one in 10^7 or
+// 10^8), 333 x 2048 x 8192 with a NaN in one row takes 161 us instead of 105, with an infinity in a column 145, and 1.8 ms where all
+// outputs are zero.
 //
 // A workgroup of 8 waves owns 16 CW WC columns x 16 FQ rows: WC waves side by side, each with CW x 16 columns and all rows, and
 // 8 / WC shares of k (steps of 32 k in turn).  A wave loads its weights itself and cuts them in registers; with WC > 1 the rows are
@@ -292,43 +293,47 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_parts_kernel(PartsArgs a) {
 #pragma unroll
     for (int k = 1; k < WK; ++k) y += *reinterpret_cast<const f32x4*>(red + (((k * WC + wc) * CW * FQ + f) * 64 + lane) * 4);
     const int r = 16 * (f % FQ) + li, n = col0 + 16 * (wc * CW + f / FQ) + 4 * g;
-    if (r >= rows || n >= a.N) continue;
-    bool again = false;
+    const bool mine = r < rows && n < a.N;
+    uint32_t again = 0;             // bit e: this lane's output n + e
 #pragma unroll
-    for (int e = 0; e < 4; ++e) again |= !(fabsf(y[e]) >= enough && fabsf(y[e]) < INFINITY);
-    if (again) {
-      float mx = 0.f;
-      f32x4 mw = {0.f, 0.f, 0.f, 0.f};
+    for (int e = 0; e < 4; ++e) again |= (mine && n + e < a.N && !(fabsf(y[e]) >= enough && fabsf(y[e]) < INFINITY)) << e;
+    if (__any(again != 0)) {
+      if (again != 0) {
+        float mx = 0.f;
+        f32x4 mw = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int k = 0; k < WK; ++k) {
-        mx = fmaxf(mx, xtops[k * Q + r]);
+        for (int k = 0; k < WK; ++k) {
+          mx = fmaxf(mx, xtops[k * Q + r]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) mw[e] = fmaxf(mw[e], wtops[k * P + n - col0 + e]);
-      }
-      again = false;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        again |= y[e] == 0.f ? mx > 0.f && mw[e] > 0.f : !(fabsf(y[e]) >= a.least * fmaxf(fmaxf(mx, mw[e]), 1.f) && fabsf(y[e]) < INFINITY);
-    }
-    if (again) {
-      const float* x = row(r);
-      y = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-      for (int k0 = 0; k0 < a.K; k0 += 32) {
-        f32x4 v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-        for (int k = k0; k < k0 + 32; k += 4) {
-          const f32x4 xk = *reinterpret_cast<const f32x4*>(x + k);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const f32x4 wk4 = *reinterpret_cast<const f32x4*>(W + (size_t)min(n + e, a.N - 1) * a.ldw + k);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[e] = fmaf(xk[i], wk4[i], v[e]);
-          }
+          for (int e = 0; e < 4; ++e) mw[e] = fmaxf(mw[e], wtops[k * P + n - col0 + e]);
         }
-        y += v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (y[e] == 0.f ? !(mx > 0.f && mw[e] > 0.f) : fabsf(y[e]) >= a.least * fmaxf(fmaxf(mx, mw[e]), 1.f) && fabsf(y[e]) < INFINITY)
+            again &= ~(1u << e);
       }
+      // the wave takes one output after the other, 256 of k at a time
+#pragma unroll 1
+      for (int e = 0; e < 4; ++e)
+#pragma unroll 1
+        for (uint64_t left = __ballot(again >> e & 1); left != 0; left &= left - 1) {
+          const int src = __builtin_ctzll(left);
+          const float* x = row(16 * (f % FQ) + (src & 15));
+          const float* w = W + (size_t)(col0 + 16 * (wc * CW + f / FQ) + 4 * (src >> 4) + e) * a.ldw;
+          float v = 0.f;
+#pragma unroll 4
+          for (int k = 4 * lane; k < a.K; k += 256) {
+            const f32x4 xk = *reinterpret_cast<const f32x4*>(x + k), wv = *reinterpret_cast<const f32x4*>(w + k);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v = fmaf(xk[i], wv[i], v);
+          }
+          v = wave_sum(v);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (lane == src && i == e) y[i] = v;
+        }
     }
+    if (!mine) continue;
     const size_t at = (size_t)(row0 + r) * a.ldc + n;
     if (a.vec) {
       *reinterpret_cast<f32x4*>(C + at) = y;

@@ -84,6 +84,21 @@ def test_rows_and_columns_of_every_size(tile):
     assert ((call(a, w, tile).double() - ref).abs() <= 2.0**-20 * most + 2.0**-120).all()
 
 
+@pytest.mark.parametrize("tile", MENU)
+@pytest.mark.parametrize("K", [32, 288, 2208])
+def test_outputs_that_are_computed_again(tile, K):
+    """Sums that cancel to zero beside others, in every place of a tile, and k that does not fill the wave."""
+    M, N = 16 * (tile % 10) + 3, 16 * (tile // 10 % 10) * (tile // 100) + 5
+    g = torch.Generator().manual_seed(tile + K)
+    a, w = torch.randint(-9, 10, (M, K), generator=g).float(), torch.randint(-9, 10, (N, K), generator=g).float()
+    a[::3, 2:], w[::5, 2:] = 0.0, 0.0
+    a[::3, :2], w[::5, 0], w[::5, 1] = 1.0, 7.0, -7.0
+    a[1, 5] = 2.0**-130                                 # a row of small values with an ordinary one
+    a, w = a.cuda(), w.cuda()
+    ref = a.double() @ w.double().T
+    assert (ref[::3, ::5] == 0).all() and torch.equal(call(a, w, tile).double(), ref.float().double())
+
+
 @pytest.mark.parametrize("tile", [111, 224, 826])
 def test_results_next_to_the_largest(tile):
     """High parts whose product rounds to infinity where the values' own does not; sums that are infinite stay so."""
