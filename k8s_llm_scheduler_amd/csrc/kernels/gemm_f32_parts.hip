@@ -355,7 +355,7 @@ extern "C" double k8s_gemm_f32_cost(int M, int N, int K, int batch);
 // steps and start for every round of workgroups over the CUs (from three on two of the small ones share one), and a share of what the weights
 // take; fitted to M 1 - 512, N 128 - 32768, K 512 - 14336 (rms error 4 - 7 % of the larger ones, 10 - 17 % of those of one column of waves), as are the fp32
 // pipes' times.  A tenth is left to these: of 300 sizes none is slower by more than 3 %, and all take 23 % less on average, 0.8 % more than
-// with the best of both for each.  They keep 33 - 100 rows of 1024 - 4096 columns in one round (56 x 3072 x 2048 16.1 / 19.3, 40 x 4096 x 14336 88 / 108), short weights (24 x 1024 x 512 6.5 / 7.3) and
+// with the best of both for each (with the largest values met, of 169 more that it takes one by 2 %, 31 % less on average).  They keep 33 - 100 rows of 1024 - 4096 columns in one round (56 x 3072 x 2048 16.1 / 19.3, 40 x 4096 x 14336 88 / 108), short weights (24 x 1024 x 512 6.5 / 7.3) and
 // few rows of wide ones, which both read at the memory's rate (3 x 32768 x 2048 40 / 42).
 // Listed tiles: from 32 rows a group on, where the groups' tiles of 32 or 64 rows of 64 columns fill one round, else 64 x 128.  Groups x columns x k, rows
 // a group: 8 x 4096 x 2048, 40 90 / 66, 250 287 / 226; 8 x 2048 x 2048, 40 58 / 37; 16 x 1024 x 2048, 40 45 / 38; 4 x 2048 x 2048, 40 32
