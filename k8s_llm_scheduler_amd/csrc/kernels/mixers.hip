@@ -745,11 +745,11 @@ __global__ __launch_bounds__(64 * NWV) void latent_attention_mfma_kernel(
     p_first = p_last = positions[t];
     valid = true;
   } else {
-    const int nseq = gridDim.z / nsplit;
-    seq = blockIdx.z % nseq;
+    const int nseq = gridDim.z / nsplit, portion = blockIdx.z % nseq;
     split = blockIdx.z / nseq;
-    const int tq0 = cu_q[seq] + blockIdx.x * NWV, tend = cu_q[seq + 1];
+    const int tq0 = cu_q[portion] + blockIdx.x * NWV, tend = cu_q[portion + 1];
     if (tq0 >= tend) return;
+    seq = tok_seq[tq0];
     const int nval = min(NWV, tend - tq0);
     t = tq0 + wave;
     valid = wave < nval;

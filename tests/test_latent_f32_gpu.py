@@ -101,7 +101,7 @@ def test_key_splits_of_portions_in_bf16(H, lens, past, window):
     T = sum(lens)
     pos = torch.cat([torch.arange(k) + (past if i != 1 else 0) for i, k in enumerate(lens)]).int()
     pos[-idle:] = -1
-    seq = torch.cat([torch.full((k,), i) for i, k in enumerate(lens)]).int()
+    seq = torch.cat([torch.full((k,), n - 1 - i) for i, k in enumerate(lens)]).int()      # the block table's rows, as they are named
     nb = (past + max(lens)) // bs + 1
     bt = torch.randperm(n * nb, generator=g).view(n, nb).int()
     cu = torch.tensor([0, *lens]).cumsum(0).int()
