@@ -249,9 +249,9 @@ int k8s_window_attention(void* out, float* pacc, float* pml, const void* q, long
 int k8s_window_mfma_ok(int H, int G, int D, int V);
 int k8s_window_f32_ok(int H, int G, int D, int V);
 int k8s_window_f32(float* out, const float* q, long ldq, const float* gate, long ldg, const float* kcache, const float* vcache,
-                   const int* block_tables, int max_blocks, const int* cu_q, const int* positions, int nseq, int max_qlen, int H, int G,
-                   int D, int V, int window, float scale, int sink, int bs, int chunk, float softcap, const float* sinkv, int gate_ph,
-                   const float* slopes, hipStream_t s);
+                   const int* block_tables, int max_blocks, const int* cu_q, const int* tok_seq, const int* positions, int T, int nseq,
+                   int max_qlen, int H, int G, int D, int V, int window, float scale, int sink, int bs, int chunk, float softcap,
+                   const float* sinkv, int gate_ph, const float* slopes, hipStream_t s);
 int k8s_window_token_ok(int H, int G, int D, int V, int bs);
 int k8s_window_token(void* out, float* pacc, float* pml, const void* q, long ldq, const void* gate, long ldg,
                      const void* kcache, const void* vcache, const int* block_tables, int max_blocks, const int* tok_seq,
@@ -842,11 +842,11 @@ PYBIND11_MODULE(K8S_MODULE_NAME, m) {
   });
   m.def("window_f32_ok", [](int H, int G, int D, int V) { return k8s_window_f32_ok(H, G, D, V) != 0; });
   m.def("window_f32", [](uintptr_t out, uintptr_t q, long ldq, uintptr_t gate, long ldg, uintptr_t kcache, uintptr_t vcache, uintptr_t bt,
-                         int max_blocks, uintptr_t cu_q, uintptr_t positions, int nseq, int max_qlen, int H, int G, int D, int V,
-                         int window, float scale, int sink, int bs, int chunk, float softcap, uintptr_t sinkv, int gate_ph,
+                         int max_blocks, uintptr_t cu_q, uintptr_t tok_seq, uintptr_t positions, int T, int nseq, int max_qlen, int H, int G,
+                         int D, int V, int window, float scale, int sink, int bs, int chunk, float softcap, uintptr_t sinkv, int gate_ph,
                          uintptr_t slopes, int64_t s) {
     check(k8s_window_f32(P<float>(out), P<float>(q), ldq, P<float>(gate), ldg, P<float>(kcache), P<float>(vcache), P<int>(bt), max_blocks,
-                         P<int>(cu_q), P<int>(positions), nseq, max_qlen, H, G, D, V, window, scale, sink, bs, chunk, softcap,
+                         P<int>(cu_q), P<int>(tok_seq), P<int>(positions), T, nseq, max_qlen, H, G, D, V, window, scale, sink, bs, chunk, softcap,
                          P<float>(sinkv), gate_ph, P<float>(slopes), S(s)), "window_f32");
   });
   m.def("window_token_ok", [](int H, int G, int D, int V, int bs) { return k8s_window_token_ok(H, G, D, V, bs) != 0; });

@@ -19,13 +19,16 @@ template <int D>
 __global__ __launch_bounds__(256, 2) void window_f32_kernel(
     float* __restrict__ out, const float* __restrict__ q, long ldq, const float* __restrict__ gate, long ldg,
     const float* __restrict__ kcache, const float* __restrict__ vcache, const int* __restrict__ block_tables, int max_blocks,
-    const int* __restrict__ cu_q, const int* __restrict__ positions, int H, int G, int window, float scale, int sink, int bs, int chunk,
+    const int* __restrict__ cu_q, const int* __restrict__ tok_seq, const int* __restrict__ positions, int T, int H, int G, int window, float scale, int sink, int bs, int chunk,
     float softcap, const float* __restrict__ sinkv, int gate_ph, const float* __restrict__ slopes) {
   constexpr int NS = D / 16, NT = D / 64, LD = D + 4;
   __shared__ __attribute__((aligned(16))) float rows[4][16][LD];       // a wave's tile of values; at the end its sums
   __shared__ float ml[4][16][2];
   const int R = H / G, NTK = 16 / R, kh = blockIdx.y, seq = blockIdx.z;
-  const int tq0 = cu_q[seq] + blockIdx.x * NTK, n = min(NTK, cu_q[seq + 1] - tq0);
+  const int tq0 = cu_q[seq] + blockIdx.x * NTK, end = cu_q[seq + 1], n = min(NTK, end - tq0);
+  if (seq + 1 == (int)gridDim.z && blockIdx.x == 0)     // rows behind the last sequence: as idle ones
+    for (int i = threadIdx.x; i < (T - end) * R * D; i += 256)
+      out[((size_t)(end + i / (R * D)) * H + kh * R) * D + i % (R * D)] = 0.f;
   if (n <= 0) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, g = lane >> 4;
   const int pf = positions[tq0], pl = pf + n - 1;
@@ -37,7 +40,7 @@ __global__ __launch_bounds__(256, 2) void window_f32_kernel(
   const int lo = first(pf), tiles = (pl - lo) / 16 + 1;              // first() does not fall with p
   const int tok = min(li / R, n - 1), hd = kh * R + li % R, p = pf + tok, lp = first(p);     // this lane's column (past the last: repeats)
   const int edge_lo = first(pl);     // keys from here to pf are seen by every token
-  const int* btr = block_tables + (size_t)seq * max_blocks;
+  const int* btr = block_tables + (size_t)tok_seq[tq0] * max_blocks;
   const auto row_of = [&](int tile) {
     const int j = min(lo + tile * 16 + li, pl);
     return ((size_t)btr[j / bs] * bs + j % bs) * G * D + (size_t)kh * D + 4 * g;
@@ -185,10 +188,11 @@ extern "C" int k8s_window_f32_ok(int H, int G, int D, int V) {
   return G > 0 && H > 0 && H % G == 0 && 16 % (H / G) == 0 && D == V && (D == 64 || D == 128) && G <= 65535;
 }
 
-// cu_q: the query offsets of nseq sequences (the rows of the block tables) of at most max_qlen tokens at consecutive positions.
+// cu_q: the query offsets of nseq sequences of at most max_qlen tokens at consecutive positions; tok_seq [T]: a token's row of the block
+// tables (a sequence's first token's is read).
 extern "C" int k8s_window_f32(float* out, const float* q, long ldq, const float* gate, long ldg, const float* kcache, const float* vcache,
-                              const int* block_tables, int max_blocks, const int* cu_q, const int* positions, int nseq, int max_qlen,
-                              int H, int G, int D, int V, int window, float scale, int sink, int bs, int chunk, float softcap,
+                              const int* block_tables, int max_blocks, const int* cu_q, const int* tok_seq, const int* positions, int T,
+                              int nseq, int max_qlen, int H, int G, int D, int V, int window, float scale, int sink, int bs, int chunk, float softcap,
                               const float* sinkv, int gate_ph, const float* slopes, hipStream_t s) {
   if (!k8s_window_f32_ok(H, G, D, V) || bs <= 0 || ldq % 4 || (((uintptr_t)out | (uintptr_t)q | (uintptr_t)kcache | (uintptr_t)vcache) & 15))
     return -1;
@@ -197,7 +201,8 @@ extern "C" int k8s_window_f32(float* out, const float* q, long ldq, const float*
   const int ntk = 16 / (H / G);
   const dim3 grid((max_qlen + ntk - 1) / ntk, G, nseq);
 #define K8S_WF(DD)                                                                                                                \
-  window_f32_kernel<DD><<<grid, 256, 0, s>>>(out, q, ldq, gate, ldg, kcache, vcache, block_tables, max_blocks, cu_q, positions, H, G, \
+  window_f32_kernel<DD><<<grid, 256, 0, s>>>(out, q, ldq, gate, ldg, kcache, vcache, block_tables, max_blocks, cu_q, tok_seq, \
+                                             positions, T, H, G, \
                                              window, scale, sink, bs, chunk, softcap, sinkv, gate_ph, slopes)
   if (D == 64) K8S_WF(64);
   else K8S_WF(128);

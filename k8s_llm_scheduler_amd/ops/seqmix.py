@@ -1441,16 +1441,16 @@ def window_attention(q: torch.Tensor, gate: Optional[torch.Tensor], kcache: torc
     max_pos = max_keys or block_tables.shape[1] * block_size
     span = chunk if chunk > 0 else window
     if (WINDOW_MFMA and dt == F32 and P <= 0 and cu_q is not None and max_qlen > 1 and nat.window_f32_ok(H, G, D, V)
-            and q.stride(0) % 4 == 0 and (q.data_ptr() | kcache.data_ptr() | vcache.data_ptr()) % 16 == 0 and cu_q.shape[0] <= 65536):
+            and q.stride(0) % 4 == 0 and (q.data_ptr() | kcache.data_ptr() | vcache.data_ptr()) % 16 == 0 and 1 < cu_q.shape[0] <= 65536):
         rows = nat.window_tile_rows(H, G, D, V)
         plain = rows > 0 and window_f32_plain(T, int(max_qlen), H, G, D, min(max_pos, span) if span > 0 else max_pos,
                                               window_splits(T, G, span, 0, max_pos, rows), rows)
         if not plain:
             nat.window_f32(out.data_ptr(), q.data_ptr(), q.stride(0), gate.data_ptr() if gate is not None else 0,
                            gate.stride(0) if gate is not None else 0, _p(kcache, dt, "kcache"), _p(vcache, dt, "vcache"),
-                           _p(block_tables, I32, "block_tables"), block_tables.shape[1], _p(cu_q, I32, "cu_q"), _p(positions, I32),
-                           cu_q.shape[0] - 1, int(max_qlen), H, G, D, V, int(window), float(scale), int(bool(sink)), block_size,
-                           int(chunk), float(softcap), _p(sinks), int(bool(gate_per_head)), _p(slopes), -1)
+                           _p(block_tables, I32, "block_tables"), block_tables.shape[1], _p(cu_q, I32, "cu_q"), _p(tok_seq, I32),
+                           _p(positions, I32), T, cu_q.shape[0] - 1, int(max_qlen), H, G, D, V, int(window), float(scale),
+                           int(bool(sink)), block_size, int(chunk), float(softcap), _p(sinks), int(bool(gate_per_head)), _p(slopes), -1)
             return out
     if (WINDOW_MFMA and dt == BF16 and P <= 0 and nat.window_token_ok(H, G, D, V, block_size) and q.stride(0) % 8 == 0
             and q.data_ptr() % 16 == 0):

@@ -39,8 +39,8 @@ def test_against_64_bits(D, H, G, window, chunk, bs, extra, monkeypatch):
     lens, past = [1, 17, 40, 3, 130], [0, 60, 25, 0, 300]
     T, nb = sum(lens), -(-430 // bs)
     pos = torch.cat([torch.arange(a, a + n) for a, n in zip(past, lens)]).int()
-    seq = torch.cat([torch.full((n,), i) for i, n in enumerate(lens)]).int()
-    pos[seq == 3] = -1
+    seq = torch.cat([torch.full((n,), (2 * i) % 5) for i, n in enumerate(lens)]).int()     # the block table's rows, as they are named
+    pos[seq == 1] = -1
     cu = torch.tensor([0, *lens]).cumsum(0).int()
     bt = torch.randperm(5 * nb, generator=g).view(5, nb).int()
     kc, vc = (torch.randn(5 * nb * bs, G, D, generator=g) for _ in range(2))
@@ -69,6 +69,20 @@ def test_against_64_bits(D, H, G, window, chunk, bs, extra, monkeypatch):
     # a value reaches the tokens that see it and no other, whatever it is
     bad = vc.clone()
     for p, v in ((302, float("nan")), (331, float("inf")), (50, float("inf"))):
-        bad[int(bt[4, p // bs]) * bs + p % bs] = v
+        bad[int(bt[3, p // bs]) * bs + p % bs] = v
     a, b = run(True, bad), run(False, bad)
     assert torch.equal(a.isfinite(), b.isfinite()) and torch.equal(a.isnan(), b.isnan())
+
+
+def test_rows_behind_the_last_sequence(monkeypatch):
+    """Idle rows that no sequence has (a batch filled up to its size) are zeros."""
+    g = torch.Generator().manual_seed(5)
+    T, H, G, D, bs = 40, 8, 2, 64, 16
+    pos, seq = torch.cat([torch.arange(29), torch.full((11,), -1)]).int().cuda(), torch.zeros(T, dtype=torch.int32, device="cuda")
+    kc, vc, q = (torch.randn(*n, generator=g).cuda() for n in ((32, G, D), (32, G, D), (T, H * D)))
+    bt, cu = torch.tensor([[1, 0]], dtype=torch.int32).cuda(), torch.tensor([0, 29], dtype=torch.int32).cuda()
+    monkeypatch.setattr(sm, "window_f32_plain", lambda *sizes: False)
+    stale = torch.full((T, H * D), float("nan"), device="cuda")
+    del stale
+    y = sm.window_attention(q, None, kc, vc, None, None, bt, seq, pos, H, 0, 0, D**-0.5, False, bs, cu, 29)
+    assert (y[29:] == 0).all() and y[:29].isfinite().all()
